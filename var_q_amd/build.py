@@ -30,6 +30,7 @@ FLAGS = {
     'dequant.hip': ['-ffp-contract=off'],
     'qkv_prepare.hip': ['-ffp-contract=off'],
     'fused_attn.hip': [],
+    'wide_attn.hip': [],
 }
 
 

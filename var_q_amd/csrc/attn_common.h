@@ -1,0 +1,100 @@
+// What the attention kernels share: launch parameters, operand types, conversions to the attention's
+// 16-bit type, the matrix instruction, the key order of its rows.
+#pragma once
+#include "varq_common.h"
+
+namespace varq_attn {
+
+typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 bf16x8_t;
+typedef __attribute__((__vector_size__(16 * sizeof(float)))) float floatx16_t;
+typedef __attribute__((__vector_size__(4 * sizeof(u32)))) u32 u32x4_t;
+
+constexpr float kLog2e = 1.4426950408889634f;
+constexpr int BN = 64;   // keys per tile
+
+constexpr int kMaxSegments = 16;
+constexpr int kMaxSplits_v = 8;        // shares of a query block's keys in the general kernel
+constexpr int kMaxKeyShares_v = 64;    // ... and in the kernel for few queries
+constexpr int kChanTableRows = 4;   // LDS rows per segment of the per-channel tables
+
+struct AttnParams {
+  const __bf16 *q;
+  __bf16 *out;
+  const u32 *k_words, *v_words;
+  const float *k_scale, *k_zp, *v_scale, *v_zp;
+  // per-(head, channel) quantization (CHAN kernels): fp32 [Hkv, D] tables shared by all
+  // tokens and batch entries; the per-key pointers above are unused then
+  const float *k_chan_scale, *k_chan_zp, *v_chan_scale, *v_chan_zp;
+  // the tables may change along the keys: keys [seg_end[s-1], seg_end[s]) use table s
+  // (fp32 [nseg, Hkv, D]); this is a cache that was quantized step by step
+  int nseg;
+  int seg_end[kMaxSegments];
+  const int32_t *head_map;
+  const int32_t *kv_limit;
+  int B, Hq, Hkv, Lq, Lk, Lstride;
+  int q_tiles, bh_total;
+  float scale_log2e;
+  // the keys of a query block may be shared out over nsplit workgroups; each leaves its
+  // normalized output (fp32 [nsplit][B*Hkv*Lq][D]) and softmax statistics (reference,
+  // denominator: fp32 [nsplit][B*Hkv*Lq][2]) for the combining kernel.  nsplit = 1: no
+  // workspace, the output is written directly.
+  int nsplit;
+  float *ws_o, *ws_ml;
+  // the caller asked for exact codes in the MFMA operands where such a kernel exists (host side only)
+  int exact_codes;
+  int f16;   // q, out and the MFMA operands are fp16 (host side only: it selects the instantiation)
+  int fq_share_blocks;   // few-queries kernel: 32-key blocks per share of the keys
+  // memory layout, in rows (a row = the D values of one token of one head):
+  // q row = b*q_bs + h*q_hs + i*q_ts, out row likewise with o_*, key row = b*kv_bs + slot*kv_hs + j*kv_ts.
+  // BHLc: (H*L, L, 1); BLHc (the layout of the flash-attention call): (L*H, 1, H).
+  int64_t q_bs, q_hs, q_ts, o_bs, o_hs, o_ts, kv_bs, kv_hs, kv_ts;
+};
+
+__device__ __forceinline__ u32 pack_bf16_rne(float lo, float hi) {
+  typedef __bf16 bf2 __attribute__((ext_vector_type(2)));
+  typedef float f2 __attribute__((ext_vector_type(2)));
+  f2 v = {lo, hi};
+  bf2 b = __builtin_convertvector(v, bf2);
+  return __builtin_bit_cast(u32, b);
+}
+__device__ __forceinline__ u32 pack_f16_rne(float lo, float hi) {
+  typedef _Float16 h2 __attribute__((ext_vector_type(2)));
+  typedef float f2 __attribute__((ext_vector_type(2)));
+  f2 v = {lo, hi};
+  h2 b = __builtin_convertvector(v, h2);
+  return __builtin_bit_cast(u32, b);
+}
+// two fp32 values rounded to nearest-even into a pair of the attention's 16-bit type
+template <bool F16> __device__ __forceinline__ u32 pack_io_rne(float lo, float hi) {
+  if constexpr (F16) return pack_f16_rne(lo, hi);
+  else return pack_bf16_rne(lo, hi);
+}
+// D (32x32 fp32) += A (32x16) B (16x32), operands in the attention's 16-bit type
+template <bool F16> __device__ __forceinline__ floatx16_t mfma_32x32x16(u32x4_t a, u32x4_t b, floatx16_t c) {
+  if constexpr (F16) {
+    typedef _Float16 f16x8_t __attribute__((ext_vector_type(8)));
+    return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8_t, a), __builtin_bit_cast(f16x8_t, b), c, 0, 0, 0);
+  } else {
+    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, a), __builtin_bit_cast(bf16x8_t, b), c, 0, 0, 0);
+  }
+}
+// MFMA row r (0..31) of the S^T block carries key kperm(r) of the 32-key block
+// (bits 2 and 3 of r swapped), so accumulator register i of a lane in half h
+// holds key 16*(i/8) + 8*h + i%8.
+__device__ __forceinline__ int kperm(int r) { return (r & 0x13) | ((r & 4) << 1) | ((r & 8) >> 1); }
+
+
+// ---- the wide path (wide_attn.hip): K and V expanded once, then attended by many query blocks ----
+struct WidePlan {
+  int n_wgs, rounds;    // workgroups of the attention kernel; blocks that each of them takes whole
+  size_t tile_bytes;    // the expanded tiles, at the start of the workspace
+  size_t ws_bytes;      // ... and the partial results behind them
+};
+WidePlan plan_wide(int64_t bh, int Lq, int Lk, int D, int cus);
+// Expands the packed cache of p (per-key groups of k_group / v_group channels, or the per-channel
+// tables) into `tiles`, pair after pair.
+void launch_expand(const AttnParams &p, int D, int bits, int k_group, int v_group, bool chan, char *tiles, hipStream_t st);
+// Attends the expanded tiles at the start of `ws`; p.q_tiles counts blocks of 256 queries.
+void launch_wide(const AttnParams &p, int D, const WidePlan &plan, char *ws, hipStream_t st);
+
+}  // namespace varq_attn

@@ -50,60 +50,18 @@
 //      goes through an fp32 correction term on tiles that have one.
 #include <type_traits>
 
-#include "varq_common.h"
+#include "attn_common.h"
+
+using namespace varq_attn;
 
 namespace {
-
-typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 bf16x8_t;
-typedef __attribute__((__vector_size__(16 * sizeof(float)))) float floatx16_t;
-typedef __attribute__((__vector_size__(4 * sizeof(u32)))) u32 u32x4_t;
 
 constexpr int NW = 8;          // wavefronts per workgroup
 constexpr int BM = NW * 32;    // queries per workgroup (32 per wavefront)
 // (The D=64 kernels also exist with four wavefronts per workgroup, for launches of many (batch,
 // head) pairs with at most 128 queries each -- the first steps of a scale schedule at a large
 // batch -- see launch().)
-constexpr int BN = 64;   // keys per tile
-constexpr float kLog2e = 1.4426950408889634f;
 constexpr float kHeadroom = 15.f;   // exact-code kernels: octaves between a fresh softmax reference and the row maximum
-
-constexpr int kMaxSegments = 16;
-constexpr int kMaxSplits_v = 8;        // shares of a query block's keys in the general kernel
-constexpr int kMaxKeyShares_v = 64;    // ... and in the kernel for few queries
-constexpr int kChanTableRows = 4;   // LDS rows per segment of the per-channel tables
-
-struct AttnParams {
-  const __bf16 *q;
-  __bf16 *out;
-  const u32 *k_words, *v_words;
-  const float *k_scale, *k_zp, *v_scale, *v_zp;
-  // per-(head, channel) quantization (CHAN kernels): fp32 [Hkv, D] tables shared by all
-  // tokens and batch entries; the per-key pointers above are unused then
-  const float *k_chan_scale, *k_chan_zp, *v_chan_scale, *v_chan_zp;
-  // the tables may change along the keys: keys [seg_end[s-1], seg_end[s]) use table s
-  // (fp32 [nseg, Hkv, D]); this is a cache that was quantized step by step
-  int nseg;
-  int seg_end[kMaxSegments];
-  const int32_t *head_map;
-  const int32_t *kv_limit;
-  int B, Hq, Hkv, Lq, Lk, Lstride;
-  int q_tiles, bh_total;
-  float scale_log2e;
-  // the keys of a query block may be shared out over nsplit workgroups; each leaves its
-  // normalized output (fp32 [nsplit][B*Hkv*Lq][D]) and softmax statistics (reference,
-  // denominator: fp32 [nsplit][B*Hkv*Lq][2]) for the combining kernel.  nsplit = 1: no
-  // workspace, the output is written directly.
-  int nsplit;
-  float *ws_o, *ws_ml;
-  // the caller asked for exact codes in the MFMA operands where such a kernel exists (host side only)
-  int exact_codes;
-  int f16;   // q, out and the MFMA operands are fp16 (host side only: it selects the instantiation)
-  int fq_share_blocks;   // few-queries kernel: 32-key blocks per share of the keys
-  // memory layout, in rows (a row = the D values of one token of one head):
-  // q row = b*q_bs + h*q_hs + i*q_ts, out row likewise with o_*, key row = b*kv_bs + slot*kv_hs + j*kv_ts.
-  // BHLc: (H*L, L, 1); BLHc (the layout of the flash-attention call): (L*H, 1, H).
-  int64_t q_bs, q_hs, q_ts, o_bs, o_hs, o_ts, kv_bs, kv_hs, kv_ts;
-};
 
 __device__ __forceinline__ u32 pack_bf16_hi(float lo, float hi) {  // exact for values with <= 8 significant bits
   return __builtin_amdgcn_perm(f2u(hi), f2u(lo), 0x07060302u);   // {hi[31:16], lo[31:16]} in one v_perm_b32
@@ -186,34 +144,6 @@ __device__ __forceinline__ void v_pair_values(const u32 *row0, const u32 *row1, 
   }
 }
 
-__device__ __forceinline__ u32 pack_bf16_rne(float lo, float hi) {
-  typedef __bf16 bf2 __attribute__((ext_vector_type(2)));
-  typedef float f2 __attribute__((ext_vector_type(2)));
-  f2 v = {lo, hi};
-  bf2 b = __builtin_convertvector(v, bf2);
-  return __builtin_bit_cast(u32, b);
-}
-__device__ __forceinline__ u32 pack_f16_rne(float lo, float hi) {
-  typedef _Float16 h2 __attribute__((ext_vector_type(2)));
-  typedef float f2 __attribute__((ext_vector_type(2)));
-  f2 v = {lo, hi};
-  h2 b = __builtin_convertvector(v, h2);
-  return __builtin_bit_cast(u32, b);
-}
-// two fp32 values rounded to nearest-even into a pair of the attention's 16-bit type
-template <bool F16> __device__ __forceinline__ u32 pack_io_rne(float lo, float hi) {
-  if constexpr (F16) return pack_f16_rne(lo, hi);
-  else return pack_bf16_rne(lo, hi);
-}
-// D (32x32 fp32) += A (32x16) B (16x32), operands in the attention's 16-bit type
-template <bool F16> __device__ __forceinline__ floatx16_t mfma_32x32x16(u32x4_t a, u32x4_t b, floatx16_t c) {
-  if constexpr (F16) {
-    typedef _Float16 f16x8_t __attribute__((ext_vector_type(8)));
-    return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8_t, a), __builtin_bit_cast(f16x8_t, b), c, 0, 0, 0);
-  } else {
-    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, a), __builtin_bit_cast(bf16x8_t, b), c, 0, 0, 0);
-  }
-}
 // x = h0 + h1 + h2 exactly, each piece a bf16 (returned as its 16 bits): three
 // 8-bit slices of the 24-bit significand
 __device__ __forceinline__ void split3_bf16(float x, u32 &h0, u32 &h1, u32 &h2) {
@@ -223,11 +153,6 @@ __device__ __forceinline__ void split3_bf16(float x, u32 &h0, u32 &h1, u32 &h2) 
   const float x2 = r1 - x1;
   h0 = f2u(x0) >> 16; h1 = f2u(x1) >> 16; h2 = f2u(x2) >> 16;
 }
-
-// MFMA row r (0..31) of the S^T block carries key kperm(r) of the 32-key block
-// (bits 2 and 3 of r swapped), so accumulator register i of a lane in half h
-// holds key 16*(i/8) + 8*h + i%8.
-__device__ __forceinline__ int kperm(int r) { return (r & 0x13) | ((r & 4) << 1) | ((r & 8) >> 1); }
 
 // ---- code widening ---------------------------------------------------------
 // K side: 8 codes of one octet -> 8 bf16 (4 dwords) holding code*kMul'+const,
@@ -1284,6 +1209,11 @@ __global__ __launch_bounds__(256) void combine_splits_kernel(AttnParams p) {
   *reinterpret_cast<uint2 *>(optr) = make_uint2(pack_io_rne<F16>(acc[0] * inv, acc[1] * inv), pack_io_rne<F16>(acc[2] * inv, acc[3] * inv));
 }
 
+template <int D, bool F16> void launch_combine(const AttnParams &p, hipStream_t st) {
+  const int64_t rows = (int64_t)p.bh_total * p.Lq;
+  hipLaunchKernelGGL((combine_splits_kernel<D, F16>), dim3((unsigned)((rows + 1) / 2)), dim3(256), 0, st, p);
+}
+
 int device_cus();
 
 template <int D, int BITS, int GK, int GV, bool CHAN, int NWV, int WPS = 2, bool EXACT = false, bool F16 = false>
@@ -1305,10 +1235,7 @@ void launch_shape(const AttnParams &p, hipStream_t st) {
   const int bh_pad = (p.bh_total + 7) / 8 * 8;
   dim3 grid((unsigned)(bh_pad * p.q_tiles * p.nsplit));
   hipLaunchKernelGGL((fused_attn_kernel<D, BITS, GK, GV, CHAN, NWV, WPS, EXACT, F16>), grid, dim3(NWV * 64), lds_bytes, st, p);
-  if (p.nsplit > 1) {
-    const int64_t rows = (int64_t)p.bh_total * p.Lq;
-    hipLaunchKernelGGL((combine_splits_kernel<D, F16>), dim3((unsigned)((rows + 1) / 2)), dim3(256), 0, st, p);
-  }
+  if (p.nsplit > 1) launch_combine<D, F16>(p, st);
 }
 
 template <int D, int BITS, int GK, int GV, bool CHAN = false>
@@ -1904,10 +1831,28 @@ template <int BITS> void launch_fewq(const AttnParams &p, hipStream_t st) {
   const int bh_pad = (p.bh_total + 7) / 8 * 8;
   dim3 grid(8, (unsigned)p.nsplit, (unsigned)(bh_pad / 8 * p.q_tiles));
   hipLaunchKernelGGL((fused_attn_fewq_kernel<BITS>), grid, dim3(FQ_NW * 64), FewQLds::kBytes, st, p);
-  if (p.nsplit > 1) {
-    const int64_t rows = (int64_t)p.bh_total * p.Lq;
-    hipLaunchKernelGGL((combine_splits_kernel<FQ_D, false>), dim3((unsigned)((rows + 1) / 2)), dim3(256), 0, st, p);
-  }
+  if (p.nsplit > 1) launch_combine<FQ_D, false>(p, st);
+}
+
+// ---- many queries: K and V expanded once, then a plain flash attention (wide_attn.hip) ----------
+// Worth it from five (D = 128) or six blocks of 256 queries per (batch, head) on: expanding costs what
+// widening costs the kernel above in a block or two, and then its way through memory; and on a device
+// that is not nearly full the three launches cost more than they save.  Measured (us, 4-bit codes, the
+// kernel above / this): D=128 B=2 H=16 1024 x 2521 69 / 75, 1300 x 3000 109 / 104, 1600 x 4121 146 / 134,
+// 2304 x 6425 339 / 250; B=8 1024 x 2521 198 / 208, 1300 x 3000 325 / 311, 2304 x 6425 1116 / 953; B=1 H=8
+// 1600 x 4121 59 / 69; D=64 B=2 1600 x 4121 105 / 95, B=8 1300 x 3000 181 / 191, 2304 x 6425 609 / 578.
+bool wide_eligible(int64_t bh, int Lq, int Lk, int D) {
+  return Lq >= (D == 128 ? 1280 : 1536) && Lk >= 2048 && bh * ((Lq + 255) / 256) >= 160 && bh <= 65535;
+}
+// The launches of the wide path, or false when the workspace does not hold what they need.
+bool run_wide(const AttnParams &p, int D, int bits, int k_group, int v_group, bool chan, void *workspace, size_t workspace_bytes,
+              hipStream_t st) {
+  const WidePlan plan = plan_wide(p.bh_total, p.Lq, p.Lk, D, device_cus());
+  if (!workspace || ((uintptr_t)workspace & 15) || workspace_bytes < plan.ws_bytes) return false;
+  char *const ws = reinterpret_cast<char *>(workspace);
+  launch_expand(p, D, bits, k_group, v_group, chan, ws, st);
+  launch_wide(p, D, plan, ws, st);
+  return true;
 }
 
 }  // namespace
@@ -1921,7 +1866,10 @@ extern "C" size_t varq_fused_attn_workspace_bytes(int B, int Hkv, int Lq, int Lk
   // (the group sizes are not known here: room for the few-queries kernel's shares whenever the
   // other sizes would admit it)
   if (splits == 0 && fewq_eligible(B, Hkv, Lq, Lk, D, D, D)) n = max(n, fewq_shares(B * Hkv, Lq, Lk));
-  return split_workspace_bytes(n, rows, D);
+  const size_t shared = split_workspace_bytes(n, rows, D);
+  if (splits != 0 || !wide_eligible((int64_t)B * Hkv, Lq, Lk, D)) return shared;
+  const size_t wide = plan_wide((int64_t)B * Hkv, Lq, Lk, D, device_cus()).ws_bytes;
+  return wide > shared ? wide : shared;
 }
 
 extern "C" int varq_fused_attn_key_shares(int B, int Hkv, int Lq, int Lk, int D, int k_group, int v_group) {
@@ -1991,6 +1939,11 @@ extern "C" int varq_fused_attn(const void *q, void *out,
     if (k_bits == 4) launch_fewq<4>(p, st);
     else if (k_bits == 8) launch_fewq<8>(p, st);
     else launch_fewq<2>(p, st);
+    VARQ_CHECK_LAUNCH("fused_attn");
+    return VARQ_OK;
+  }
+  if (splits == 0 && !p.exact_codes && wide_eligible(p.bh_total, Lq, Lk, D) &&
+      run_wide(p, D, k_bits, k_group, v_group, false, workspace, workspace_bytes, st)) {
     VARQ_CHECK_LAUNCH("fused_attn");
     return VARQ_OK;
   }
@@ -2069,9 +2022,13 @@ extern "C" int varq_fused_attn_channel(const void *q, void *out,
   p.f16 = io_dtype == VARQ_F16;
   p.exact_codes = 0;
   if (int e = set_layout(p, layout, "fused_attn_channel")) return e;
+  hipStream_t st = (hipStream_t)stream;
+  if (splits == 0 && wide_eligible(p.bh_total, Lq, Lk, D) && run_wide(p, D, bits, D, D, true, workspace, workspace_bytes, st)) {
+    VARQ_CHECK_LAUNCH("fused_attn_channel");
+    return VARQ_OK;
+  }
   if (int e = set_splits(p, D, (Lk + BN - 1) / BN, splits, workspace, workspace_bytes, "fused_attn_channel"))
     return e;
-  hipStream_t st = (hipStream_t)stream;
   if (D == 128) {
     if (bits == 4) launch<128, 4, 128, 128, true>(p, st);
     else if (bits == 8) launch<128, 8, 128, 128, true>(p, st);

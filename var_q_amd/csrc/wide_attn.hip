@@ -1,0 +1,588 @@
+// Attention of many queries over a packed cache in two launches: the packed K and V of every
+// (batch, head) are dequantized ONCE into the operands of the matrix instructions, and a plain flash
+// attention then streams those.
+//
+// fused_attn.hip widens a key tile in every workgroup, i.e. once per 256 queries; behind that it
+// computes with the very same operands, (code - zp) * scale in fp32 rounded to the attention's
+// 16-bit type.  With several blocks of 256 queries per (batch, head) the widening is the same
+// work over and over, it takes a fifth to a quarter of that kernel's time, and its registers and
+// instructions keep the rest from overlapping.
+#include <type_traits>
+
+#include "attn_common.h"
+
+using namespace varq_attn;
+
+namespace {
+
+// A tile holds 64 keys of one (batch, head): first K, then V, 64 * D * 2 bytes each, as 1 KiB
+// fragments that are operands of v_mfma_f32_16x16x32 for a wavefront, 16 bytes per lane (r = lane % 16,
+// g = lane / 16):
+//   K fragment [kb][ch][t] (half t of the 32 keys kb, 32 channels ch): lane holds key kb*32 + 8*(r/4) + 4*t + r%4,
+//                          channels ch*32 + g*8 + 0..7
+//   V fragment [kb][d]     (16 channels d, the 32 keys kb): lane holds channel d*16 + r, keys kb*32 + g*8 + 0..7
+// so that the attention kernel copies tiles to LDS as they are and reads every operand with one
+// conflict-free ds_read_b128.  The order of the keys in the two K fragments of a block is the one
+// that leaves the logits of 8 consecutive keys in a lane of S^T = K Q^T, which is what the lane
+// holds of P^T in O^T = V^T P^T.  Keys past Lk hold zeros.
+template <int D> constexpr int kHalfTile = BN * D * 2;
+
+struct ExpandParams {
+  AttnParams a;
+  char *tiles;
+  int n_tiles, kg_shift, vg_shift;   // log2 of the channels per scale group
+};
+
+template <int BITS> __device__ __forceinline__ void load_codes(const u32 *row, int oct, float (&f)[8]) {
+  if constexpr (BITS == 8) {
+    const uint2 w = *reinterpret_cast<const uint2 *>(row + 2 * oct);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      f[j] = (float)(int)__builtin_amdgcn_sbfe((int)w.x, 8 * j, 8);
+      f[4 + j] = (float)(int)__builtin_amdgcn_sbfe((int)w.y, 8 * j, 8);
+    }
+  } else if constexpr (BITS == 4) {
+    const int w = (int)row[oct];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) f[j] = (float)(int)__builtin_amdgcn_sbfe(w, 4 * j, 4);
+  } else {
+    const int w = (int)(row[oct >> 1] >> ((oct & 1) * 16));
+#pragma unroll
+    for (int j = 0; j < 8; ++j) f[j] = (float)(int)__builtin_amdgcn_sbfe(w, 2 * j, 2);
+  }
+}
+
+// One workgroup = one tile of one (batch, head).  HBM-bound by its writes.
+template <int D, int BITS, bool CHAN, bool F16>
+__global__ __launch_bounds__(256) void expand_tiles_kernel(ExpandParams e) {
+  constexpr int WPR = D * BITS / 32, NF = D / 16, OCT = D / 8;   // NF: fragments per 32 keys
+  constexpr int VTS = BN + 8;
+  __shared__ uint16_t vt[D * VTS];
+  __shared__ int seg_end[kMaxSegments];
+  const AttnParams &p = e.a;
+  const int tile = blockIdx.x, bh = blockIdx.y, tid = threadIdx.x;
+  const int b = bh / p.Hkv, hs = bh - b * p.Hkv;
+  const int64_t kv_row0 = b * p.kv_bs + hs * p.kv_hs;
+  char *const out = e.tiles + ((int64_t)bh * e.n_tiles + tile) * (2 * kHalfTile<D>);
+  if constexpr (CHAN) {
+    if (tid < kMaxSegments) seg_end[tid] = p.seg_end[tid];
+    __syncthreads();
+  }
+  auto segment = [&](int key) {
+    int s = 0;
+    if constexpr (CHAN) while (s + 1 < p.nseg && key >= seg_end[s]) ++s;
+    return s;
+  };
+  // values of octet `oct` of one key
+  auto values = [&](const u32 *words, const float *scale, const float *zp, const float *cscale, const float *czp, int g_shift,
+                    int key, int oct, float (&f)[8]) {
+    if (key >= p.Lk) {
+#pragma unroll
+      for (int j = 0; j < 8; ++j) f[j] = 0.f;
+      return;
+    }
+    const int64_t row = kv_row0 + key * p.kv_ts;
+    load_codes<BITS>(words + row * WPR, oct, f);
+    if constexpr (CHAN) {
+      const int64_t t = ((int64_t)segment(key) * p.Hkv + hs) * D + oct * 8;
+      const float4 sa = *reinterpret_cast<const float4 *>(cscale + t), sb = *reinterpret_cast<const float4 *>(cscale + t + 4);
+      const float s[8] = {sa.x, sa.y, sa.z, sa.w, sb.x, sb.y, sb.z, sb.w};
+      if (czp) {
+        const float4 za = *reinterpret_cast<const float4 *>(czp + t), zb = *reinterpret_cast<const float4 *>(czp + t + 4);
+        const float z[8] = {za.x, za.y, za.z, za.w, zb.x, zb.y, zb.z, zb.w};
+#pragma unroll
+        for (int j = 0; j < 8; ++j) f[j] = (f[j] - z[j]) * s[j];
+      } else {
+#pragma unroll
+        for (int j = 0; j < 8; ++j) f[j] = f[j] * s[j];
+      }
+    } else {
+      const int64_t g = row * (D >> g_shift) + (oct * 8 >> g_shift);
+      const float s = scale[g], z = zp ? zp[g] : 0.f;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) f[j] = (f[j] - z) * s;
+    }
+  };
+  // V: two adjacent keys x 8 channels -> the transposed tile in LDS
+#pragma unroll
+  for (int i = 0; i < BN / 2 * OCT / 256; ++i) {
+    const int item = tid + i * 256, oct = item % OCT, kp = item / OCT;
+    float f0[8], f1[8];
+    values(p.v_words, p.v_scale, p.v_zp, p.v_chan_scale, p.v_chan_zp, e.vg_shift, tile * BN + 2 * kp, oct, f0);
+    values(p.v_words, p.v_scale, p.v_zp, p.v_chan_scale, p.v_chan_zp, e.vg_shift, tile * BN + 2 * kp + 1, oct, f1);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) *reinterpret_cast<u32 *>(&vt[(oct * 8 + j) * VTS + 2 * kp]) = pack_io_rne<F16>(f0[j], f1[j]);
+  }
+  // K: one octet of one key is one lane's 16 bytes
+#pragma unroll
+  for (int i = 0; i < BN * OCT / 256; ++i) {
+    const int item = tid + i * 256, r = item & 15, g = (item >> 4) & 3, frag = item >> 6;
+    const int t = frag & 1, ch = (frag % NF) >> 1, kb = frag / NF;
+    float f[8];
+    values(p.k_words, p.k_scale, p.k_zp, p.k_chan_scale, p.k_chan_zp, e.kg_shift, tile * BN + kb * 32 + 8 * (r >> 2) + 4 * t + (r & 3),
+           ch * 4 + g, f);
+    u32x4_t w;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) w[j] = pack_io_rne<F16>(f[2 * j], f[2 * j + 1]);
+    *reinterpret_cast<u32x4_t *>(out + item * 16) = w;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < BN * OCT / 256; ++i) {
+    const int item = tid + i * 256, r = item & 15, g = (item >> 4) & 3, frag = item >> 6;
+    *reinterpret_cast<u32x4_t *>(out + kHalfTile<D> + item * 16) =
+        *reinterpret_cast<const u32x4_t *>(&vt[((frag % NF) * 16 + r) * VTS + (frag / NF) * 32 + g * 8]);
+  }
+}
+
+typedef __attribute__((__vector_size__(4 * sizeof(float)))) float floatx4_t;
+// D (16x16 fp32) += A (16x32) B (32x16), operands in the attention's 16-bit type
+template <bool F16> __device__ __forceinline__ floatx4_t mfma_16x16x32(u32x4_t a, u32x4_t b, floatx4_t c) {
+  if constexpr (F16) {
+    typedef _Float16 f16x8_t __attribute__((ext_vector_type(8)));
+    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8_t, a), __builtin_bit_cast(f16x8_t, b), c, 0, 0, 0);
+  } else {
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, a), __builtin_bit_cast(bf16x8_t, b), c, 0, 0, 0);
+  }
+}
+
+// Work comes in blocks of 256 queries of one (batch, head), block bh * q_tiles + qt, and is dealt out to
+// n workgroups in rounds: in each of the first `rounds` rounds workgroup w takes block round * n + w
+// whole; the blocks left over are shared out by the key tile, workgroup w taking units [T w / n, T (w + 1) / n)
+// of their T = blocks * tiles units, and a block that falls on several workgroups is put together
+// from their partial results.  With n = the number of compute units all of them finish together.
+// Whole rounds first, because the workgroups of an XCD then read the same few tile streams at a time
+// through their L2.  (Consecutive w sit on one XCD: ids congruent mod 8 share an L2.)
+struct WideParams {
+  AttnParams a;
+  const char *tiles;
+  int all_tiles, rounds;
+  float *ws_o, *ws_ml;   // partial results: slot 2w the first shared block of workgroup w, slot 2w + 1 its last; [slot][256][D], [slot][256][2]
+};
+struct SharedUnits {
+  int64_t first, total;   // the first unit that is shared out, and how many are
+  int n;
+  __device__ __forceinline__ SharedUnits(const WideParams &e, int n_wgs) : n(n_wgs) {
+    first = (int64_t)e.rounds * n_wgs * e.all_tiles;
+    total = (int64_t)e.a.bh_total * e.a.q_tiles * e.all_tiles - first;
+  }
+  __device__ __forceinline__ int64_t begin(int w) const { return first + total * w / n; }
+  __device__ __forceinline__ int owner(int64_t unit) const { return (int)(((unit - first + 1) * n - 1) / total); }   // the last w with begin(w) <= unit
+};
+
+// One workgroup = 8 wavefronts = 256 queries of one (batch, head) at a time; a wavefront owns 32 queries
+// (two columns of 16) and walks blocks of 32 keys, transposed: S^T = K Q^T, O^T = V^T P^T.
+template <int D, bool F16>
+__global__ __launch_bounds__(512, 2) void wide_attn_kernel(WideParams e) {
+  constexpr int NT = 512, NF = D / 16, HT = kHalfTile<D>, PIECES = HT / (NT * 16);
+  extern __shared__ __attribute__((aligned(16))) char lds[];   // K slots [3][HT], V slots [3][HT]
+  __shared__ int lds_maxlim;
+  const AttnParams &p = e.a;
+  const int all_tiles = e.all_tiles, n_wgs = gridDim.x;
+  const int w = (blockIdx.x & 7) * (n_wgs >> 3) + min(blockIdx.x & 7, n_wgs & 7) + (blockIdx.x >> 3);
+  const SharedUnits shared(e, n_wgs);
+  int64_t unit = shared.begin(w);
+  const int64_t unit_end = shared.begin(w + 1);
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int r16 = lane & 15, quarter = lane >> 4;
+  const float scale = p.scale_log2e;
+  const char *const frag0 = lds + lane * 16;
+  const u32 my16 = tid * 16;
+
+  for (int round = 0; round < e.rounds || unit < unit_end; ++round) {
+  int qblock = round * n_wgs + w, tbase = 0, tlast = all_tiles;
+  if (round >= e.rounds) {
+    qblock = (int)(unit / all_tiles);
+    tbase = (int)(unit - (int64_t)qblock * all_tiles);
+    tlast = (int)min((int64_t)all_tiles, tbase + (unit_end - unit));
+    unit += tlast - tbase;
+  }
+  const bool partial = tlast - tbase < all_tiles;
+  if (round > 0) __syncthreads();   // (the block before is done with the LDS)
+
+  const int bh = qblock / p.q_tiles, qt = qblock - bh * p.q_tiles;
+  const int b = bh / p.Hkv, hs = bh - b * p.Hkv;
+  const int hq = p.head_map ? p.head_map[hs] : hs;
+  const int qrow0 = qt * 256 + wave * 32;
+  const bool wave_live = qrow0 < p.Lq;   // wave-uniform
+  int limit[2], qrow_c[2];
+  int maxlim = 0, minlim = p.Lk;
+#pragma unroll
+  for (int n = 0; n < 2; ++n) {
+    const int row = qrow0 + n * 16 + r16;
+    qrow_c[n] = min(row, p.Lq - 1);
+    limit[n] = p.kv_limit ? max(min(p.kv_limit[qrow_c[n]], p.Lk), 0) : p.Lk;
+    if (row < p.Lq) { maxlim = max(maxlim, limit[n]); minlim = min(minlim, limit[n]); }
+  }
+  int kv_end = p.Lk;
+  if (p.kv_limit) {
+    if (tid == 0) lds_maxlim = 0;
+    __syncthreads();
+    atomicMax(&lds_maxlim, maxlim);
+    __syncthreads();
+    kv_end = lds_maxlim;
+  }
+  const int n_tiles = __builtin_amdgcn_readfirstlane(max(min((kv_end + BN - 1) / BN, tlast) - tbase, 0));
+  for (int off = 1; off < 64; off <<= 1) minlim = min(minlim, __shfl_xor(minlim, off, 64));
+  // tiles that no query of the wavefront has to mask
+  const int n_full = __builtin_amdgcn_readfirstlane(min(max(minlim / BN - tbase, 0), n_tiles));
+
+  const char *const src = e.tiles + ((int64_t)bh * all_tiles + tbase) * (2 * HT);
+  u32x4_t kreg[PIECES], vreg[PIECES];
+  auto load_k = [&](int t) __attribute__((always_inline)) {   // (past the end: the last tile again, never used)
+    const char *s = src + (int64_t)min(t, n_tiles - 1) * (2 * HT);
+#pragma unroll
+    for (int i = 0; i < PIECES; ++i) kreg[i] = *reinterpret_cast<const u32x4_t *>(s + i * (NT * 16) + my16);
+  };
+  auto load_v = [&](int t) __attribute__((always_inline)) {
+    const char *s = src + (int64_t)min(t, n_tiles - 1) * (2 * HT) + HT;
+#pragma unroll
+    for (int i = 0; i < PIECES; ++i) vreg[i] = *reinterpret_cast<const u32x4_t *>(s + i * (NT * 16) + my16);
+  };
+  auto put_k = [&](int sl) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < PIECES; ++i) *reinterpret_cast<u32x4_t *>(lds + sl * HT + i * (NT * 16) + my16) = kreg[i];
+  };
+  auto put_v = [&](int sl) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < PIECES; ++i) *reinterpret_cast<u32x4_t *>(lds + (3 + sl) * HT + i * (NT * 16) + my16) = vreg[i];
+  };
+
+  // ---- prologue: K of tiles 0 and 1 and V of tile 0 in LDS, K of tile 2 and V of tile 1 in registers;
+  //      the V slot of "tile -1" holds zeros ----
+  u32x4_t qb[2][NF / 2];
+  if (n_tiles > 0) {
+    load_k(0); load_v(0);
+#pragma unroll
+    for (int n = 0; n < 2; ++n) {
+      const __bf16 *qptr = p.q + (b * p.q_bs + hq * p.q_hs + qrow_c[n] * p.q_ts) * D + quarter * 8;
+#pragma unroll
+      for (int ch = 0; ch < NF / 2; ++ch) qb[n][ch] = *reinterpret_cast<const u32x4_t *>(qptr + ch * 32);
+    }
+    put_k(0); put_v(0);
+    load_k(1);
+#pragma unroll
+    for (int i = 0; i < PIECES; ++i) *reinterpret_cast<u32x4_t *>(lds + 5 * HT + i * (NT * 16) + my16) = u32x4_t{0, 0, 0, 0};
+    put_k(1);
+    load_k(2); load_v(1);
+  }
+  __syncthreads();
+
+  if (!wave_live) {
+    for (int t = 0, s0 = 0, s1 = 1, s2 = 2; t < n_tiles; ++t) {
+      put_k(s2); put_v(s1);
+      load_k(t + 3); load_v(t + 2);
+      __syncthreads();
+      const int x = s0; s0 = s1; s1 = s2; s2 = x;
+    }
+    continue;
+  }
+
+  floatx4_t oacc[NF][2];                // [16 channels][16 queries]
+  floatx4_t sacc[2][2][2];              // [block parity][half of the keys][16 queries]
+  u32x4_t pop[2][2];                    // [block parity][16 queries]: weights of 8 keys
+  float l_part[2], m_ref[2];
+#pragma unroll
+  for (int n = 0; n < 2; ++n) {
+    l_part[n] = 0.f; m_ref[n] = 0.f;
+    pop[0][n] = pop[1][n] = u32x4_t{0, 0, 0, 0};
+#pragma unroll
+    for (int d = 0; d < NF; ++d) oacc[d][n] = floatx4_t{0.f, 0.f, 0.f, 0.f};
+  }
+
+  // logit of key 8*quarter + i of the block, query column n
+  auto logit = [&](const floatx4_t (&s)[2][2], int n, int i, int key0, auto mask_tag) __attribute__((always_inline)) {
+    const float z = __builtin_fmaf(scale, s[i >> 2][n][i & 3], -m_ref[n]);
+    if constexpr (decltype(mask_tag)::value) return key0 + 8 * quarter + i >= limit[n] ? -INFINITY : z;
+    else return z;
+  };
+  // largest of a query's logits over the block: four lanes hold them
+  auto row_max = [&](const floatx4_t (&s)[2][2], int n, int key0, auto mask_tag) __attribute__((always_inline)) {
+    float zmax = -INFINITY;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) zmax = fmaxf(zmax, logit(s, n, i, key0, mask_tag));
+    zmax = fmaxf(zmax, __shfl_xor(zmax, 16, 64));
+    return fmaxf(zmax, __shfl_xor(zmax, 32, 64));
+  };
+  // the sum grows by a pair of weights as rounded for the matrix product
+  auto add_pair = [&](u32 w, float blk) __attribute__((always_inline)) {
+    if constexpr (F16) {
+      typedef _Float16 f16x2_t __attribute__((ext_vector_type(2)));
+      return __builtin_amdgcn_fdot2(__builtin_bit_cast(f16x2_t, w), __builtin_bit_cast(f16x2_t, 0x3c003c00u), blk, false);
+    } else {
+      typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
+      return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2_t, w), __builtin_bit_cast(bf16x2_t, 0x3f803f80u), blk, false);
+    }
+  };
+
+  // operands of the next matrix instructions, requested ahead: K and V fragments i sit in slot i % 4
+  u32x4_t kf[4], vf[4];
+  auto frag = [&](const char *base, int i) __attribute__((always_inline)) { return *reinterpret_cast<const u32x4_t *>(base + i * 1024); };
+
+  // One pipeline step: S^T of the next block (K fragments at kp), the weights of this block
+  // (s_in -> p_out), O^T of the block before (V fragments at vp, p_in): three independent streams.
+  // kn, vn: the fragments of the step after.
+  auto step = [&](const char *kp, const char *vp, const char *kn, const char *vn, const floatx4_t (&s_in)[2][2], floatx4_t (&s_out)[2][2],
+                  const u32x4_t (&p_in)[2], u32x4_t (&p_out)[2], int key0, auto mask_tag) __attribute__((always_inline)) {
+    constexpr int HALVES = 16 / (2 * NF);   // exponentials per fragment
+    float blk[2] = {0.f, 0.f}, z[16], e[16];   // element h: query column h / 8, key h % 8
+    auto form = [&](int j) __attribute__((always_inline)) {   // the logits of pair j
+      z[2 * j] = logit(s_in, j >> 2, (2 * j) & 7, key0, mask_tag);
+      z[2 * j + 1] = logit(s_in, j >> 2, (2 * j + 1) & 7, key0, mask_tag);
+    };
+    auto pack = [&](int j) __attribute__((always_inline)) {   // the weights of pair j are rounded, kept and summed
+      const u32 w = pack_io_rne<F16>(e[2 * j], e[2 * j + 1]);
+      p_out[j >> 2][j & 3] = w;
+      blk[j >> 2] = add_pair(w, blk[j >> 2]);
+    };
+    form(0);
+    floatx4_t acc[2][2];
+#pragma unroll
+    for (int t = 0; t < 2; ++t) acc[t][0] = acc[t][1] = floatx4_t{0.f, 0.f, 0.f, 0.f};
+    int nk = 0, nv = 0;
+#pragma unroll
+    for (int o = 0; o < 2 * NF; ++o) {
+      // K K V K K V ...: S^T is done a few instructions before the step ends, where the next one reads it
+      if (nk < NF && o % 3 != 2) {
+#pragma unroll
+        for (int n = 0; n < 2; ++n) acc[nk & 1][n] = mfma_16x16x32<F16>(kf[nk % 4], qb[n][nk >> 1], acc[nk & 1][n]);
+        kf[nk % 4] = nk + 4 < NF ? frag(kp, nk + 4) : frag(kn, nk + 4 - NF);
+        ++nk;
+      } else {
+#pragma unroll
+        for (int n = 0; n < 2; ++n) oacc[nv][n] = mfma_16x16x32<F16>(vf[nv % 4], p_in[n], oacc[nv][n]);
+        vf[nv % 4] = nv + 4 < NF ? frag(vp, nv + 4) : frag(vn, nv + 4 - NF);
+        ++nv;
+      }
+      // exponential h: its pair's logits were formed a pair ahead, its pair is packed a pair behind
+#pragma unroll
+      for (int h = o * HALVES; h < (o + 1) * HALVES; ++h) {
+        const int j = h / 2;
+        if (h % 2 == 0 && j + 1 < 8) form(j + 1);
+        e[h] = __builtin_amdgcn_exp2f(z[h]);
+        if (h % 2 == 1 && j > 0) pack(j - 1);
+      }
+    }
+    pack(7);
+#pragma unroll
+    for (int t = 0; t < 2; ++t) { s_out[t][0] = acc[t][0]; s_out[t][1] = acc[t][1]; }
+    // The softmax reference moves only when a weight would pass 2^16 (2^15 in fp16, whose weights
+    // end at 65504); the block's sum of weights shows it, and the block is redone.
+    constexpr float kMoveAt = F16 ? 32768.f : 65536.f;
+    if (__any(!(blk[0] <= kMoveAt) || !(blk[1] <= kMoveAt))) {
+#pragma unroll
+      for (int n = 0; n < 2; ++n) {
+        const float delta = fmaxf(row_max(s_in, n, key0, mask_tag), 0.f);
+        const float alpha = __builtin_amdgcn_exp2f(-delta);
+        m_ref[n] += delta;
+#pragma unroll
+        for (int d = 0; d < NF; ++d) oacc[d][n] *= alpha;
+        l_part[n] *= alpha;
+        blk[n] = 0.f;
+      }
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        form(j);
+        e[2 * j] = __builtin_amdgcn_exp2f(z[2 * j]);
+        e[2 * j + 1] = __builtin_amdgcn_exp2f(z[2 * j + 1]);
+        pack(j);
+      }
+    }
+    l_part[0] += blk[0];
+    l_part[1] += blk[1];
+  };
+
+  int s0 = 0, s1 = 1, s2 = 2;   // slots of tiles t, t+1, t+2 (= t-1)
+  if (n_tiles > 0) {
+#pragma unroll
+    for (int t = 0; t < 2; ++t) sacc[0][t][0] = sacc[0][t][1] = floatx4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int i = 0; i < NF; ++i)
+#pragma unroll
+      for (int n = 0; n < 2; ++n) sacc[0][i & 1][n] = mfma_16x16x32<F16>(frag(frag0, i), qb[n][i >> 1], sacc[0][i & 1][n]);
+#pragma unroll
+    for (int n = 0; n < 2; ++n) {
+      const float zmax = row_max(sacc[0], n, tbase * BN, std::true_type{});
+      m_ref[n] = zmax == -INFINITY ? 0.f : zmax;
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) { kf[i] = frag(frag0 + NF * 1024, i); vf[i] = frag(frag0 + 5 * HT + NF * 1024, i); }
+  }
+  auto tile_step = [&](int t, auto mask_tag) __attribute__((always_inline)) {
+    put_k(s2); put_v(s1);
+    load_k(t + 3); load_v(t + 2);
+    const int key0 = (tbase + t) * BN;
+    const char *const ka = frag0 + s0 * HT + NF * 1024, *const va = frag0 + (3 + s2) * HT + NF * 1024;
+    const char *const kb = frag0 + s1 * HT, *const vb = frag0 + (3 + s0) * HT;
+    step(ka, va, kb, vb, sacc[0], sacc[1], pop[1], pop[0], key0, mask_tag);
+    step(kb, vb, kb + NF * 1024, vb + NF * 1024, sacc[1], sacc[0], pop[0], pop[1], key0 + 32, mask_tag);
+    __syncthreads();
+    const int x = s0; s0 = s1; s1 = s2; s2 = x;
+  };
+  int t = 0;
+  for (; t < n_full; ++t) tile_step(t, std::false_type{});
+  for (; t < n_tiles; ++t) tile_step(t, std::true_type{});
+  if (n_tiles > 0) {
+    // (the slots have been rotated: the last tile's is s2)
+    const char *vp = frag0 + (3 + s2) * HT + NF * 1024;
+#pragma unroll
+    for (int i = 0; i < NF; ++i)
+#pragma unroll
+      for (int n = 0; n < 2; ++n) oacc[i][n] = mfma_16x16x32<F16>(frag(vp, i), pop[1][n], oacc[i][n]);
+  }
+
+#pragma unroll
+  for (int n = 0; n < 2; ++n) {
+    float l_sum = l_part[n] + __shfl_xor(l_part[n], 16, 64);
+    l_sum += __shfl_xor(l_sum, 32, 64);
+    const float inv = l_sum > 0.f ? 1.0f / l_sum : 0.f;
+    const int qrow = qrow0 + n * 16 + r16;
+    if (qrow >= p.Lq) continue;
+    // register i of tile d is channel 16*d + 4*quarter + i
+    if (partial) {
+      const int64_t prow = (int64_t)(2 * w + (round == e.rounds ? 0 : 1)) * 256 + wave * 32 + n * 16 + r16;
+      if (quarter == 0) *reinterpret_cast<float2 *>(e.ws_ml + prow * 2) = make_float2(m_ref[n], l_sum);
+      float *wptr = e.ws_o + prow * D + 4 * quarter;
+#pragma unroll
+      for (int d = 0; d < NF; ++d)
+        *reinterpret_cast<float4 *>(wptr + d * 16) = make_float4(oacc[d][n][0] * inv, oacc[d][n][1] * inv, oacc[d][n][2] * inv, oacc[d][n][3] * inv);
+    } else {
+      __bf16 *optr = p.out + (b * p.o_bs + hq * p.o_hs + qrow * p.o_ts) * D + 4 * quarter;
+#pragma unroll
+      for (int d = 0; d < NF; ++d)
+        *reinterpret_cast<uint2 *>(optr + d * 16) =
+            make_uint2(pack_io_rne<F16>(oacc[d][n][0] * inv, oacc[d][n][1] * inv), pack_io_rne<F16>(oacc[d][n][2] * inv, oacc[d][n][3] * inv));
+    }
+  }
+  }
+}
+
+// The query blocks that fell on several workgroups: the partial outputs weighted by their softmax
+// mass l * 2^(m - M).  A workgroup serves 1024 / D rows of one block, a thread four channels of a row.
+template <int D, bool F16>
+__global__ __launch_bounds__(256) void wide_combine_kernel(WideParams e, int n_wgs) {
+  const AttnParams &p = e.a;
+  const SharedUnits shared(e, n_wgs);
+  const int qblock = e.rounds * n_wgs + blockIdx.y, tid = threadIdx.x;
+  const int row = blockIdx.x * (1024 / D) + tid / (D / 4), c0 = tid % (D / 4) * 4;
+  const int64_t u0 = (int64_t)qblock * e.all_tiles;
+  const int w0 = shared.owner(u0), w1 = shared.owner(u0 + e.all_tiles - 1);
+  const int bh = qblock / p.q_tiles, qrow = (qblock - bh * p.q_tiles) * 256 + row;
+  if (w0 == w1 || qrow >= p.Lq) return;
+  // (a workgroup whose units start inside the block or with it has it as its first, any other as its last)
+  auto slot_row = [&](int w) { return (int64_t)(2 * w + (shared.begin(w) >= u0 ? 0 : 1)) * 256 + row; };
+  float M = -INFINITY;
+  for (int w = w0; w <= w1; ++w) {
+    const float2 ml = *reinterpret_cast<const float2 *>(e.ws_ml + slot_row(w) * 2);
+    if (ml.y > 0.f) M = fmaxf(M, ml.x);
+  }
+  float acc[4] = {0.f, 0.f, 0.f, 0.f}, sum = 0.f;
+  for (int w = w0; w <= w1; ++w) {
+    const int64_t r = slot_row(w);
+    const float2 ml = *reinterpret_cast<const float2 *>(e.ws_ml + r * 2);
+    const float4 o = *reinterpret_cast<const float4 *>(e.ws_o + r * D + c0);
+    if (ml.y > 0.f) {
+      const float wt = ml.y * __builtin_amdgcn_exp2f(ml.x - M);
+      acc[0] = __builtin_fmaf(wt, o.x, acc[0]); acc[1] = __builtin_fmaf(wt, o.y, acc[1]);
+      acc[2] = __builtin_fmaf(wt, o.z, acc[2]); acc[3] = __builtin_fmaf(wt, o.w, acc[3]);
+      sum += wt;
+    }
+  }
+  const float inv = sum > 0.f ? 1.0f / sum : 0.f;
+  const int b = bh / p.Hkv, hs = bh - b * p.Hkv;
+  const int hq = p.head_map ? p.head_map[hs] : hs;
+  *reinterpret_cast<uint2 *>(p.out + (b * p.o_bs + hq * p.o_hs + qrow * p.o_ts) * D + c0) =
+      make_uint2(pack_io_rne<F16>(acc[0] * inv, acc[1] * inv), pack_io_rne<F16>(acc[2] * inv, acc[3] * inv));
+}
+
+template <int D, int BITS> void expand_bits(const ExpandParams &e, bool chan, dim3 grid, hipStream_t st) {
+  if constexpr (D == 64) {
+    if (e.a.f16) {
+      if (chan) hipLaunchKernelGGL((expand_tiles_kernel<D, BITS, true, true>), grid, dim3(256), 0, st, e);
+      else hipLaunchKernelGGL((expand_tiles_kernel<D, BITS, false, true>), grid, dim3(256), 0, st, e);
+      return;
+    }
+  }
+  if (chan) hipLaunchKernelGGL((expand_tiles_kernel<D, BITS, true, false>), grid, dim3(256), 0, st, e);
+  else hipLaunchKernelGGL((expand_tiles_kernel<D, BITS, false, false>), grid, dim3(256), 0, st, e);
+}
+
+template <int D, bool F16> void launch_wide_shape(const WideParams &e, int n_wgs, hipStream_t st) {
+  constexpr int lds_bytes = 6 * kHalfTile<D>;
+  // above 64 KiB the limit has to be raised, once per device the process launches on
+  static bool configured[64] = {false};
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) dev = -1;
+  if (dev < 0 || !configured[dev]) {
+    (void)hipFuncSetAttribute(reinterpret_cast<const void *>(&wide_attn_kernel<D, F16>), hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes);
+    if (dev >= 0) configured[dev] = true;
+  }
+  hipLaunchKernelGGL((wide_attn_kernel<D, F16>), dim3((unsigned)n_wgs), dim3(512), lds_bytes, st, e);
+  const int64_t left = (int64_t)e.a.bh_total * e.a.q_tiles - (int64_t)e.rounds * n_wgs;
+  if (left > 0)
+    hipLaunchKernelGGL((wide_combine_kernel<D, F16>), dim3(256 / (1024 / D), (unsigned)left), dim3(256), 0, st, e, n_wgs);
+}
+
+}  // namespace
+
+namespace varq_attn {
+
+WidePlan plan_wide(int64_t bh, int Lq, int Lk, int D, int cus) {
+  WidePlan w;
+  const int64_t blocks = bh * ((Lq + 255) / 256), tiles = (Lk + BN - 1) / BN;
+  w.tile_bytes = (size_t)bh * (size_t)tiles * (size_t)(2 * BN * D * 2);
+  w.n_wgs = (int)blocks;
+  w.rounds = 1;
+  w.ws_bytes = w.tile_bytes;
+  // One workgroup runs on a compute unit.  Whole blocks take ceil(blocks / cus) rounds; sharing the
+  // last, unfilled round out evenly takes its fraction of a round, and the way of the partial results
+  // through memory.
+  const double tile_us = D == 128 ? 1.9 : 1.2, fixed_us = 6.0;
+  const int64_t rounds = blocks / cus, left = (blocks - rounds * cus) * tiles;
+  int64_t n = rounds ? cus : left / 4 < cus ? left / 4 : cus;
+  if (n > 1 && left) {
+    const double whole = (double)tiles * tile_us + fixed_us;
+    const double pieces = (double)(n + blocks - rounds * cus);   // at most this many partial results, written and read at 5 TB/s
+    const double shared = (double)left / (double)n * tile_us + 2.0 * fixed_us + 5.0 + 2.0 * pieces * 256.0 * D * 4.0 / 5.0e6;
+    if (shared < whole) {
+      w.n_wgs = (int)n;
+      w.rounds = (int)rounds;
+      w.ws_bytes += (size_t)(2 * n) * 256 * (size_t)(D + 2) * sizeof(float);
+    }
+  }
+  return w;
+}
+
+void launch_expand(const AttnParams &p, int D, int bits, int k_group, int v_group, bool chan, char *tiles, hipStream_t st) {
+  ExpandParams e;
+  e.a = p;
+  e.tiles = tiles;
+  e.n_tiles = (p.Lk + BN - 1) / BN;
+  e.kg_shift = varq_log2_exact(k_group);
+  e.vg_shift = varq_log2_exact(v_group);
+  dim3 grid((unsigned)e.n_tiles, (unsigned)p.bh_total);
+#define VARQ_EXPAND(D_)                                        \
+  do {                                                         \
+    if (bits == 4) expand_bits<D_, 4>(e, chan, grid, st);      \
+    else if (bits == 8) expand_bits<D_, 8>(e, chan, grid, st); \
+    else expand_bits<D_, 2>(e, chan, grid, st);                \
+  } while (0)
+  if (D == 128) VARQ_EXPAND(128);
+  else VARQ_EXPAND(64);
+#undef VARQ_EXPAND
+}
+
+void launch_wide(const AttnParams &p, int D, const WidePlan &plan, char *ws, hipStream_t st) {
+  WideParams e;
+  e.a = p;
+  e.tiles = ws;
+  e.all_tiles = (p.Lk + BN - 1) / BN;
+  e.rounds = plan.rounds;
+  e.ws_o = reinterpret_cast<float *>(ws + plan.tile_bytes);
+  e.ws_ml = e.ws_o + (size_t)(2 * plan.n_wgs) * 256 * (size_t)D;
+  if (D == 128) launch_wide_shape<128, false>(e, plan.n_wgs, st);
+  else if (p.f16) launch_wide_shape<64, true>(e, plan.n_wgs, st);
+  else launch_wide_shape<64, false>(e, plan.n_wgs, st);
+}
+
+}  // namespace varq_attn
