@@ -37,6 +37,7 @@ SYMBOLS = {
                                 c_int, c_int, c_int, c_int,
                                 c_void_p, c_float, c_int, c_int, c_int, c_void_p, c_size_t, c_int, c_void_p]),
     'varq_fused_attn_workspace_bytes': (c_size_t, [c_int, c_int, c_int, c_int, c_int, c_int, c_int]),
+    'varq_fused_attn_expand_bytes': (c_size_t, [c_int, c_int, c_int, c_int, c_int]),
     'varq_fused_attn_key_shares': (c_int, [c_int, c_int, c_int, c_int, c_int, c_int, c_int]),
     'varq_fused_attn_channel': (c_int, [c_void_p, c_void_p,
                                         c_void_p, c_void_p, c_void_p,
@@ -54,6 +55,7 @@ SYMBOLS = {
 }
 
 _lib = None
+_host = None
 
 
 class VarqError(RuntimeError):
@@ -79,6 +81,20 @@ def load():
         raise VarqError(f'libvarq_hip.so ABI {got} != expected {ABI_VERSION}; rebuild')
     _lib = lib
     return lib
+
+
+def host():
+    """The native host layer (csrc/host.cpp), loaded once."""
+    global _host
+    if _host is None:
+        load()
+        try:
+            from . import _host as mod
+        except ImportError as e:
+            raise VarqError(f'the native host layer is missing or does not load ({e}): build it with `python -m var_q_amd.build`') from e
+        mod.set_error(VarqError)
+        _host = mod
+    return _host
 
 
 def check(rc, what):

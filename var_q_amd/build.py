@@ -1,7 +1,8 @@
-"""Builds libvarq_hip.so (the C-ABI library of include/varq.h) in-tree with hipcc.
+"""Builds libvarq_hip.so (the C-ABI library of include/varq.h) in-tree with hipcc, and _host.so
+(the native host layer of the Python package, csrc/host.cpp) on top of it.
 
 Run as `python -m var_q_amd.build`.  hipcc cross-compiles for gfx950 without a
-GPU.  The library has no torch or Python dependency.
+GPU.  The library has no torch or Python dependency; the host layer has both.
 """
 import os
 import shutil
@@ -12,6 +13,7 @@ from concurrent.futures import ThreadPoolExecutor
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, 'csrc')
 LIB = os.path.join(HERE, 'libvarq_hip.so')
+HOST = os.path.join(HERE, '_host.so')
 
 # Bit-exactness of the quantizer rests on these: IEEE fp32 division, no FMA
 # contraction across the oracle's separately rounded operations, denormals kept.
@@ -69,7 +71,25 @@ def build(verbose=True, jobs=6):
     os.replace(tmp, LIB)
     if verbose:
         print('[varq build] linked', LIB, flush=True)
+    build_host(verbose)
     return LIB
+
+
+def build_host(verbose=True):
+    """csrc/host.cpp against torch's C++ headers; finds libvarq_hip.so beside itself."""
+    import sysconfig
+    import torch
+    t = os.path.dirname(torch.__file__)
+    tmp = HOST + '.tmp'
+    _run([shutil.which('g++') or 'g++', '-O2', '-std=c++17', '-fPIC', '-shared', '-Wall', '-D__HIP_PLATFORM_AMD__', '-DUSE_ROCM',
+          '-D_GLIBCXX_USE_CXX11_ABI=%d' % int(torch._C._GLIBCXX_USE_CXX11_ABI),
+          '-I' + os.path.join(t, 'include'), '-I' + os.path.join(t, 'include', 'torch', 'csrc', 'api', 'include'),
+          '-I' + os.path.join(os.path.dirname(os.path.dirname(os.path.realpath(_hipcc()))), 'include'), '-I/opt/rocm/include',
+          '-I' + sysconfig.get_paths()['include'], os.path.join(CSRC, 'host.cpp'), '-o', tmp,
+          '-L' + HERE, '-lvarq_hip', '-L' + os.path.join(t, 'lib'), '-lc10', '-lc10_hip', '-ltorch_cpu', '-ltorch_python', '-Wl,-rpath,$ORIGIN'])
+    os.replace(tmp, HOST)
+    if verbose:
+        print('[varq build] linked', HOST, flush=True)
 
 
 if __name__ == '__main__':

@@ -1910,10 +1910,12 @@ extern "C" size_t varq_fused_attn_workspace_bytes(int B, int Hkv, int Lq, int Lk
   // (the group sizes are not known here: room for the few-queries kernel's shares whenever the
   // other sizes would admit it)
   if (splits == 0 && fewq_eligible(B, Hkv, Lq, Lk, D, D, D)) n = max(n, fewq_shares(B * Hkv, Lq, Lk));
-  const size_t shared = split_workspace_bytes(n, rows, D);
-  if (splits != 0 || !wide_eligible((int64_t)B * Hkv, Lq, Lk, D)) return shared;
-  const size_t wide = plan_wide((int64_t)B * Hkv, Lq, Lk, D, device_cus()).ws_bytes;
-  return wide > shared ? wide : shared;
+  return split_workspace_bytes(n, rows, D);
+}
+
+extern "C" size_t varq_fused_attn_expand_bytes(int B, int Hkv, int Lq, int Lk, int D) {
+  if (B <= 0 || Hkv <= 0 || Lq <= 0 || Lk <= 0 || (D != 64 && D != 128) || !wide_eligible((int64_t)B * Hkv, Lq, Lk, D)) return 0;
+  return plan_wide((int64_t)B * Hkv, Lq, Lk, D, device_cus()).ws_bytes;
 }
 
 extern "C" int varq_fused_attn_key_shares(int B, int Hkv, int Lq, int Lk, int D, int k_group, int v_group) {

@@ -1,0 +1,533 @@
+// The host side of a call in native code: tensor checks, output and workspace allocation and the call
+// of the C ABI, for the entry points of ops.py, pack_unpack.py, kv_cache.py and quant.py.
+//
+// A step of a few tokens is bound by its host work, not by its kernels: attributes of a dozen
+// tensors, assertions, allocations and thirty ctypes conversions took 14-20 us per call from Python
+// where the launch itself takes 3.  Functions take positional arguments only (METH_FASTCALL); the
+// Python wrappers above them carry the names, the defaults and the documentation.
+// Exceptions are those of the Python layer: AssertionError for arguments that do not fit together,
+// VarqError for tensors off the GPU and for statuses of the library.
+#include <Python.h>
+
+#include <ATen/core/Tensor.h>
+#include <ATen/ops/empty.h>
+#include <c10/core/DeviceGuard.h>
+#include <c10/hip/HIPStream.h>
+#include <torch/csrc/Exceptions.h>
+#include <torch/csrc/autograd/python_variable.h>
+
+#include "../../include/varq.h"
+
+namespace {
+
+PyObject *g_varq_error = nullptr;
+
+[[noreturn]] void raise(PyObject *type, const char *fmt, ...) {
+  va_list ap;
+  va_start(ap, fmt);
+  PyErr_FormatV(type, fmt, ap);
+  va_end(ap);
+  throw python_error();
+}
+#define ASSERT(cond, ...)                                  \
+  do {                                                     \
+    if (!(cond)) raise(PyExc_AssertionError, __VA_ARGS__); \
+  } while (0)
+
+void check(int rc, const char *what) {
+  if (rc != VARQ_OK) raise(g_varq_error, "%s failed (status %d): %s", what, rc, varq_last_error());
+}
+
+// ---- arguments ------------------------------------------------------------------------------
+const at::Tensor &gpu(PyObject *o, const char *name) {
+  if (!THPVariable_Check(o)) raise(g_varq_error, "%s must be a GPU tensor (got %s); the VAR-Q HIP path has no CPU fallback", name, Py_TYPE(o)->tp_name);
+  const at::Tensor &t = THPVariable_Unpack(o);
+  if (!t.is_cuda())
+    raise(g_varq_error, "%s must be a GPU tensor (got %s); the VAR-Q HIP path has no CPU fallback", name, t.device().str().c_str());
+  return t;
+}
+// None or a GPU tensor
+const at::Tensor *maybe(PyObject *o, const char *name) { return o == Py_None ? nullptr : &gpu(o, name); }
+
+int64_t integer(PyObject *o) {
+  const long long v = PyLong_AsLongLong(o);
+  if (v == -1 && PyErr_Occurred()) {
+    // (numpy integers and the like)
+    PyErr_Clear();
+    PyObject *i = PyNumber_Index(o);
+    if (!i) throw python_error();
+    const long long w = PyLong_AsLongLong(i);
+    Py_DECREF(i);
+    if (w == -1 && PyErr_Occurred()) throw python_error();
+    return w;
+  }
+  return v;
+}
+double real(PyObject *o) {
+  const double v = PyFloat_AsDouble(o);
+  if (v == -1.0 && PyErr_Occurred()) throw python_error();
+  return v;
+}
+bool truth(PyObject *o) { return PyObject_IsTrue(o) == 1; }
+
+int dtype_code(const at::Tensor &t) {
+  switch (t.scalar_type()) {
+    case at::kFloat: return VARQ_F32;
+    case at::kBFloat16: return VARQ_BF16;
+    case at::kHalf: return VARQ_F16;
+    default: raise(g_varq_error, "unsupported dtype %s; expected float32, bfloat16 or float16", toString(t.scalar_type()));
+  }
+}
+at::ScalarType dtype_of(int code) { return code == VARQ_F32 ? at::kFloat : code == VARQ_BF16 ? at::kBFloat16 : at::kHalf; }
+
+template <typename T> T *ptr(const at::Tensor &t) { return reinterpret_cast<T *>(t.data_ptr()); }
+template <typename T> T *ptr(const at::Tensor *t) { return t ? reinterpret_cast<T *>(t->data_ptr()) : nullptr; }
+
+void *stream_of(const at::Tensor &t) { return (void *)c10::hip::getCurrentHIPStream(t.device().index()).stream(); }
+
+at::Tensor empty(at::IntArrayRef shape, at::ScalarType dt, const at::Tensor &like) { return at::empty(shape, like.options().dtype(dt)); }
+
+PyObject *wrap(const at::Tensor &t) { return THPVariable_Wrap(t); }
+PyObject *triple(const at::Tensor &a, const at::Tensor &b, const at::Tensor &c) {
+  PyObject *t = PyTuple_New(3);
+  PyTuple_SET_ITEM(t, 0, wrap(a));
+  PyTuple_SET_ITEM(t, 1, wrap(b));
+  if (c.defined()) PyTuple_SET_ITEM(t, 2, wrap(c));
+  else { Py_INCREF(Py_None); PyTuple_SET_ITEM(t, 2, Py_None); }
+  return t;
+}
+
+void need_args(Py_ssize_t n, Py_ssize_t want, const char *name) {
+  if (n != want) raise(PyExc_TypeError, "%s takes %zd arguments (%zd given)", name, want, n);
+}
+
+// ---- quantize + pack --------------------------------------------------------------------------
+// quant_rows(x, group, bits, asym, eps) -> (words, scale, zp | None)
+PyObject *quant_rows(PyObject *const *a) {
+  const at::Tensor x = gpu(a[0], "x").contiguous();
+  const int64_t group = integer(a[1]), bits = integer(a[2]);
+  const bool asym = truth(a[3]);
+  const int64_t c = x.dim() ? x.size(-1) : 0, rows = c ? x.numel() / c : 0;
+  ASSERT(x.dim() >= 1 && group != 0, "quant_pack_rows: a tensor of rows and a group size are needed");
+  c10::DimVector shape(x.sizes().begin(), x.sizes().end());
+  shape.back() = c * bits / 32;
+  const c10::DeviceGuard guard(x.device());
+  const at::Tensor words = empty(shape, at::kInt, x);
+  shape.back() = c / group;
+  const at::Tensor scale = empty(shape, at::kFloat, x);
+  at::Tensor zp;
+  if (asym) zp = empty(shape, at::kFloat, x);
+  check(varq_quant_pack_rows(x.data_ptr(), dtype_code(x), rows, (int)c, (int)group, (int)bits, asym, (float)real(a[4]), nullptr, nullptr,
+                             ptr<int32_t>(words), ptr<float>(scale), asym ? ptr<float>(zp) : nullptr, stream_of(x)), "varq_quant_pack_rows");
+  return triple(words, scale, zp);
+}
+
+struct Shared {   // shapes of a quantization with groups that span rows
+  int64_t sh[4], sshape[4], last;
+  Shared(const at::Tensor &x, int mask, int64_t bits, bool pack) {
+    for (int d = 0; d < 4; ++d) {
+      sh[d] = x.size(d);
+      sshape[d] = mask >> d & 1 ? 1 : sh[d];
+    }
+    const int64_t vals = 32 / bits;
+    last = pack ? (sh[3] + vals - 1) / vals : sh[3];
+  }
+};
+
+// quant_shared(x, mask, bits, asym, eps, pack) -> (words | codes, scale, zp | None)
+PyObject *quant_shared(PyObject *const *a) {
+  const at::Tensor &x0 = gpu(a[0], "x");
+  ASSERT(x0.dim() == 4, "expected a 4-D [B,L,H,c] / [B,H,L,c] tensor");
+  const at::Tensor x = x0.contiguous();
+  const int mask = (int)integer(a[1]);
+  const int64_t bits = integer(a[2]);
+  const bool asym = truth(a[3]), pack = truth(a[5]);
+  ASSERT(bits > 0 && bits <= 32, "bits must be in 2..8");
+  const Shared s(x, mask, bits, pack);
+  const c10::DeviceGuard guard(x.device());
+  const at::Tensor q = empty({s.sh[0], s.sh[1], s.sh[2], s.last}, pack ? at::kInt : at::kChar, x);
+  const at::Tensor scale = empty(at::IntArrayRef(s.sshape, 4), at::kFloat, x);
+  at::Tensor zp;
+  if (asym) zp = empty(at::IntArrayRef(s.sshape, 4), at::kFloat, x);
+  const size_t ws_bytes = std::max<size_t>(varq_quant_workspace_bytes(s.sh, mask), 8);
+  const at::Tensor ws = empty({(int64_t)ws_bytes}, at::kByte, x);
+  check(varq_quant_pack(x.data_ptr(), dtype_code(x), s.sh, mask, (int)bits, asym, (float)real(a[4]), pack ? ptr<int32_t>(q) : nullptr,
+                        pack ? nullptr : ptr<int8_t>(q), ptr<float>(scale), asym ? ptr<float>(zp) : nullptr, nullptr, ws.data_ptr(), ws_bytes,
+                        stream_of(x)), "varq_quant_pack");
+  return triple(q, scale, zp);
+}
+
+// One step of a quantizer with a scale per (head, channel): codes into tokens start.. of the cache
+// buffer, scale and zero-point into row k of the step tables.
+// quant_step(mask, bits, asym, eps, token_dim, start, k, x, buf, tab, ztab | None [, x1, buf1, tab1, ztab1])
+// -> None; the second tensor (K and V of a step) goes through the same launches.
+PyObject *quant_step(PyObject *const *a, Py_ssize_t n_args) {
+  if (n_args != 11 && n_args != 15) need_args(n_args, 11, "quant_step");
+  const bool two = n_args == 15;
+  const int mask = (int)integer(a[0]);
+  const int64_t bits = integer(a[1]), d = integer(a[4]), start = integer(a[5]), k = integer(a[6]);
+  const bool asym = truth(a[2]);
+  const at::Tensor *x[2], *buf[2], *tab[2], *ztab[2];
+  for (int i = 0; i < (two ? 2 : 1); ++i) {
+    x[i] = &gpu(a[7 + 4 * i], "x");
+    buf[i] = &gpu(a[8 + 4 * i], "buffer");
+    tab[i] = &gpu(a[9 + 4 * i], "scale table");
+    ztab[i] = maybe(a[10 + 4 * i], "zero-point table");
+    const at::Tensor &t = *x[i], &b = *buf[i];
+    ASSERT(t.dim() == 4 && t.is_contiguous() && b.dim() == 4 && b.is_contiguous() && b.scalar_type() == at::kInt && tab[i]->is_contiguous() &&
+               t.sizes() == x[0]->sizes() && t.scalar_type() == x[0]->scalar_type() && b.sizes() == buf[0]->sizes(), "quant_step: operands");
+    ASSERT((!asym || ztab[i]) && b.size(3) * 32 == t.size(3) * bits && start >= 0 && start + t.size(d) <= b.size(d) &&
+               b.size(0) == t.size(0) && b.size(3 - d) == t.size(3 - d), "quant_step: buffers");
+    const int64_t row = t.size(d == 1 ? 2 : 1) * t.size(3);
+    ASSERT(k >= 0 && (k + 1) * row <= tab[i]->numel() && tab[i]->scalar_type() == at::kFloat, "quant_step: tables");
+  }
+  const at::Tensor &t = *x[0];
+  const int64_t sh[4] = {t.size(0), t.size(1), t.size(2), t.size(3)};
+  const int64_t per_tok = d == 1 ? sh[2] : 1, row = sh[d == 1 ? 2 : 1] * sh[3];
+  const int64_t map[3] = {sh[d] * per_tok, (buf[0]->size(d) - sh[d]) * per_tok, start * per_tok};
+  const c10::DeviceGuard guard(t.device());
+  const size_t one = std::max<size_t>(varq_quant_workspace_bytes(sh, mask), 8), ws_bytes = two ? 2 * one : one;
+  const at::Tensor ws = empty({(int64_t)ws_bytes}, at::kByte, t);
+  const float eps = (float)real(a[3]);
+  float *s[2], *z[2];
+  for (int i = 0; i < (two ? 2 : 1); ++i) {
+    s[i] = ptr<float>(tab[i]) + k * row;
+    z[i] = asym ? ptr<float>(ztab[i]) + k * row : nullptr;
+  }
+  if (two)
+    check(varq_quant_pack2(x[0]->data_ptr(), x[1]->data_ptr(), dtype_code(t), sh, mask, (int)bits, asym, eps, ptr<int32_t>(buf[0]), nullptr, s[0], z[0],
+                           ptr<int32_t>(buf[1]), nullptr, s[1], z[1], map, ws.data_ptr(), ws_bytes, stream_of(t)), "varq_quant_pack2");
+  else
+    check(varq_quant_pack(x[0]->data_ptr(), dtype_code(t), sh, mask, (int)bits, asym, eps, ptr<int32_t>(buf[0]), nullptr, s[0], z[0], map,
+                          ws.data_ptr(), ws_bytes, stream_of(t)), "varq_quant_pack");
+  Py_RETURN_NONE;
+}
+
+// ---- pack / unpack of int8 codes ----------------------------------------------------------------
+// pack(codes, bits) -> words
+PyObject *pack(PyObject *const *a) {
+  const at::Tensor codes = gpu(a[0], "q_int8").contiguous();
+  const int64_t bits = integer(a[1]), c = codes.size(-1), vals = 32 / bits, rows = c ? codes.numel() / c : 0;
+  c10::DimVector shape(codes.sizes().begin(), codes.sizes().end());
+  shape.back() = (c + vals - 1) / vals;
+  const c10::DeviceGuard guard(codes.device());
+  const at::Tensor words = empty(shape, at::kInt, codes);
+  check(varq_pack(ptr<int8_t>(codes), rows, (int)c, (int)bits, ptr<int32_t>(words), stream_of(codes)), "varq_pack");
+  return wrap(words);
+}
+// unpack(words, c, bits) -> codes
+PyObject *unpack(PyObject *const *a) {
+  const at::Tensor words = gpu(a[0], "packed").contiguous();
+  const int64_t c = integer(a[1]), bits = integer(a[2]), w = words.size(-1), rows = w ? words.numel() / w : 0;
+  c10::DimVector shape(words.sizes().begin(), words.sizes().end());
+  shape.back() = c;
+  const c10::DeviceGuard guard(words.device());
+  const at::Tensor codes = empty(shape, at::kChar, words);
+  check(varq_unpack(ptr<int32_t>(words), rows, (int)c, (int)bits, ptr<int8_t>(codes), stream_of(words)), "varq_unpack");
+  return wrap(codes);
+}
+
+// ---- dequantize ---------------------------------------------------------------------------------
+// One scale per (i2, channel) whatever i0 and i1, the n2 rows of an (i0, i1) pair next to each other: the
+// same bytes read as [1, n0, n1, n2 * c] (see ops._rows_as_channels, which states when and why).
+void rows_as_channels(bool packed, int64_t (&sh)[4], int64_t (&ss)[4], int64_t group, int64_t bits, int64_t *map) {
+  const int64_t n0 = sh[0], n1 = sh[1], n2 = sh[2], c = sh[3], c8 = n2 * c / 8;
+  if (!packed || group != 1 || n2 <= 1 || c % 8 || c * bits % 32 || ss[0] || ss[1] || ss[2] != c || ss[3] != 1 || c8 > 256 || (c8 & (c8 - 1))) return;
+  if (map) {
+    if (map[5] != 1 || map[7] >= 0 || map[3] % n2 || map[4] % n2 || map[6] % n2) return;
+    const int64_t m[8] = {1, n0, n1, 0, map[3] / n2, map[4] / n2, map[6] / n2, -1};
+    std::copy(m, m + 8, map);
+  }
+  sh[0] = 1; sh[1] = n0; sh[2] = n1; sh[3] = n2 * c;
+  ss[0] = ss[1] = ss[2] = 0;
+}
+
+// dequant(q, scale, zp | None, c, bits, out dtype code) -> [n0,n1,n2,c].  q: rows of words or codes, dense
+// inside (a window of a cache buffer is read where it lies).
+PyObject *dequant(PyObject *const *a) {
+  at::Tensor q = gpu(a[0], "q"), scale = gpu(a[1], "scale"), zp;
+  if (a[2] != Py_None) zp = gpu(a[2], "zp");
+  const int64_t c = integer(a[3]), bits = integer(a[4]), code = integer(a[5]);
+  ASSERT(q.dim() == 4 && scale.dim() == 4, "dequant: 4-D codes and scale");
+  const bool packed = q.scalar_type() == at::kInt;
+  ASSERT(packed || q.scalar_type() == at::kChar, "dequant: int32 words or int8 codes");
+  const int64_t wq = q.size(3);
+  const bool dense = q.is_contiguous();
+  if (!dense && (q.stride(3) != 1 || !wq || q.stride(0) % wq || q.stride(1) % wq || q.stride(2) % wq)) q = q.contiguous();
+  if (zp.defined() && (zp.sizes() != scale.sizes() || zp.strides() != scale.strides())) {
+    zp = zp.expand_as(scale).contiguous();
+    scale = scale.contiguous();
+  }
+  const int64_t s3 = scale.size(3);
+  ASSERT(s3 > 0 && c % s3 == 0, "scale last dim %lld does not divide c=%lld", (long long)s3, (long long)c);
+  int64_t sh[4] = {q.size(0), q.size(1), q.size(2), c}, ss[4], map[8];
+  for (int d = 0; d < 4; ++d) {
+    ASSERT(d == 3 || scale.size(d) == 1 || scale.size(d) == q.size(d), "scale dim %d = %lld vs %lld", d, (long long)scale.size(d), (long long)q.size(d));
+    ss[d] = scale.size(d) == 1 ? 0 : scale.stride(d);
+  }
+  const c10::DeviceGuard guard(q.device());
+  const at::Tensor out = empty(at::IntArrayRef(sh, 4), dtype_of((int)code), q);
+  bool mapped = false;
+  if (q.is_contiguous()) {
+    // (leading dims that the scale does not depend on collapse: fuller blocks)
+    if (!ss[0] && !ss[1] && !ss[2]) { sh[2] = sh[0] * sh[1] * sh[2]; sh[0] = sh[1] = 1; }
+  } else {
+    const int64_t m[8] = {sh[0], sh[1], sh[2], q.stride(0) / wq, q.stride(1) / wq, q.stride(2) / wq, 0, -1};
+    std::copy(m, m + 8, map);
+    mapped = true;
+  }
+  rows_as_channels(packed, sh, ss, c / s3, bits, mapped ? map : nullptr);
+  check(varq_dequant(packed ? ptr<int32_t>(q) : nullptr, packed ? nullptr : ptr<int8_t>(q), ptr<float>(scale), zp.defined() ? ptr<float>(zp) : nullptr,
+                     sh, ss, (int)(c / s3), (int)bits, mapped ? map : nullptr, out.data_ptr(), (int)code, stream_of(q)), "varq_dequant");
+  return wrap(out);
+}
+
+// ---- attention ----------------------------------------------------------------------------------
+struct AttnShape {
+  int64_t B, Hq, Lq, D, Hkv, Lstride;
+  int layout;   // of the call, out included
+  at::Tensor out;
+};
+
+int layout_code(PyObject *o) {
+  const char *s = PyUnicode_Check(o) ? PyUnicode_AsUTF8(o) : "";
+  if (!strcmp(s, "BHLc")) return VARQ_LAYOUT_BHLC;
+  ASSERT(!strcmp(s, "BLHc"), "layout must be one of ['BHLc', 'BLHc']");
+  return VARQ_LAYOUT_BLHC;
+}
+
+// (the checks that both attention calls share; a: q, k_words, out, layout, out_layout)
+AttnShape attn_shape(const at::Tensor &q, const at::Tensor &kw, PyObject *out, PyObject *layout, PyObject *out_layout) {
+  AttnShape s;
+  ASSERT((q.scalar_type() == at::kBFloat16 || q.scalar_type() == at::kHalf) && q.dim() == 4, "q must be bf16 or fp16");
+  ASSERT(kw.dim() == 4, "k_words must be 4-D");
+  const int lay = layout_code(layout), h = lay == VARQ_LAYOUT_BHLC ? 1 : 2, t = 3 - h;
+  s.B = q.size(0); s.Hq = q.size(h); s.Lq = q.size(t); s.D = q.size(3);
+  s.Hkv = kw.size(h); s.Lstride = kw.size(t);
+  ASSERT(kw.size(0) == s.B, "batch sizes of q and the cache differ");
+  s.layout = lay;
+  const int olay = out_layout == Py_None ? lay : layout_code(out_layout);
+  if (olay != lay) {
+    ASSERT(lay == VARQ_LAYOUT_BHLC, "out_layout: only tokens-first out of a heads-first call");
+    s.layout = VARQ_LAYOUT_BHLC_OUT_BLHC;
+  }
+  const int64_t n[4] = {s.B, olay == VARQ_LAYOUT_BHLC ? s.Hq : s.Lq, olay == VARQ_LAYOUT_BHLC ? s.Lq : s.Hq, s.D};
+  if (out == Py_None) {
+    s.out = empty(at::IntArrayRef(n, 4), q.scalar_type(), q);
+  } else {
+    s.out = gpu(out, "out");
+    ASSERT(s.out.scalar_type() == q.scalar_type() && s.out.sizes() == at::IntArrayRef(n, 4) && s.out.is_contiguous(),
+           "out must be contiguous, of the dtype of q and of the shape its layout implies");
+  }
+  return s;
+}
+const at::Tensor &dense(PyObject *o, const char *name) {
+  const at::Tensor &t = gpu(o, name);
+  ASSERT(t.is_contiguous(), "%s must be contiguous", name);
+  return t;
+}
+void check_limit_and_map(const at::Tensor *limit, const at::Tensor *map, const AttnShape &s) {
+  if (limit) ASSERT(limit->scalar_type() == at::kInt && limit->numel() == s.Lq && limit->is_contiguous(), "kv_limit must be contiguous int32 [Lq]");
+  if (map) ASSERT(map->scalar_type() == at::kInt && map->numel() == s.Hkv && map->is_contiguous(), "head_map must be int32 [Hkv]");
+  else ASSERT(s.Hkv == s.Hq, "Hkv != Hq needs a head map");
+}
+int io_code(const at::Tensor &q) { return q.scalar_type() == at::kHalf ? VARQ_F16 : VARQ_BF16; }
+
+// device memory for a launch that shares keys out or expands them (0: neither)
+size_t workspace_bytes(const AttnShape &s, int64_t Lk, int nseg, int64_t splits) {
+  const size_t shared = varq_fused_attn_workspace_bytes((int)s.B, (int)s.Hkv, (int)s.Lq, (int)Lk, (int)s.D, nseg, (int)splits);
+  return splits ? shared : std::max(shared, varq_fused_attn_expand_bytes((int)s.B, (int)s.Hkv, (int)s.Lq, (int)Lk, (int)s.D));
+}
+
+// attn(q, k_words, k_scale, k_zp, v_words, v_scale, v_zp, k_bits, v_bits, Lk, softmax_scale, kv_limit, head_map, out, splits,
+//      layout, exact_codes, out_layout) -> out
+PyObject *attn(PyObject *const *a) {
+  const at::Tensor &q = dense(a[0], "q"), &kw = dense(a[1], "k_words"), &ks = dense(a[2], "k_scale"), &vw = dense(a[4], "v_words"), &vs = dense(a[5], "v_scale");
+  const at::Tensor *kz = maybe(a[3], "k_zp"), *vz = maybe(a[6], "v_zp"), *limit = maybe(a[11], "kv_limit"), *map = maybe(a[12], "head_map");
+  const int64_t k_bits = integer(a[7]), v_bits = integer(a[8]), Lk = integer(a[9]), splits = integer(a[14]);
+  const c10::DeviceGuard guard(q.device());
+  const AttnShape s = attn_shape(q, kw, a[13], a[15], a[17]);
+  ASSERT(vw.dim() == 4 && ks.dim() == 4 && vs.dim() == 4, "4-D cache tensors");
+  for (int d = 0; d < 3; ++d)
+    ASSERT(vw.size(d) == kw.size(d) && ks.size(d) == kw.size(d) && vs.size(d) == kw.size(d), "words and scales must agree in batch, heads and tokens");
+  ASSERT(kw.size(3) * 32 == s.D * k_bits && vw.size(3) * 32 == s.D * v_bits, "words per row do not match the head dim and the bit-width");
+  ASSERT(ks.size(3) > 0 && vs.size(3) > 0, "empty scales");
+  for (const auto &[z, sc, n] : {std::tuple(kz, &ks, "k_zp"), std::tuple(vz, &vs, "v_zp")})
+    ASSERT(!z || (z->sizes() == sc->sizes() && z->scalar_type() == at::kFloat && z->is_contiguous()), "%s must look like its scale", n);
+  ASSERT(ks.scalar_type() == at::kFloat && vs.scalar_type() == at::kFloat && kw.scalar_type() == at::kInt && vw.scalar_type() == at::kInt,
+         "scales must be fp32 and words int32");
+  ASSERT(0 <= Lk && Lk <= s.Lstride, "Lk=%lld outside the cache of %lld tokens", (long long)Lk, (long long)s.Lstride);
+  check_limit_and_map(limit, map, s);
+  const size_t ws_bytes = workspace_bytes(s, Lk, 1, splits);
+  at::Tensor ws;
+  if (ws_bytes) ws = empty({(int64_t)ws_bytes}, at::kByte, q);
+  check(varq_fused_attn(q.data_ptr(), s.out.data_ptr(), ptr<int32_t>(kw), ptr<float>(ks), ptr<float>(kz), (int)k_bits, (int)(s.D / ks.size(3)),
+                        ptr<int32_t>(vw), ptr<float>(vs), ptr<float>(vz), (int)v_bits, (int)(s.D / vs.size(3)), (int)s.B, (int)s.Hq, (int)s.Hkv,
+                        ptr<int32_t>(map), (int)s.Lq, (int)Lk, (int)s.Lstride, (int)s.D, ptr<int32_t>(limit), (float)real(a[10]), s.layout, io_code(q),
+                        truth(a[16]), ws_bytes ? ws.data_ptr() : nullptr, ws_bytes, (int)splits, stream_of(q)), "varq_fused_attn");
+  return wrap(s.out);
+}
+
+// attn_channel(q, k_words, k_scale, k_zp, v_words, v_scale, v_zp, bits, Lk, softmax_scale, kv_limit, head_map, out, seg_ends, splits,
+//              layout, out_layout) -> out
+PyObject *attn_channel(PyObject *const *a) {
+  const at::Tensor &q = dense(a[0], "q"), &kw = dense(a[1], "k_words"), &ks = dense(a[2], "k_chan_scale"), &vw = dense(a[4], "v_words"), &vs = dense(a[5], "v_chan_scale");
+  const at::Tensor *kz = maybe(a[3], "k_chan_zp"), *vz = maybe(a[6], "v_chan_zp"), *limit = maybe(a[10], "kv_limit"), *map = maybe(a[11], "head_map");
+  const int64_t bits = integer(a[7]), Lk = integer(a[8]), splits = integer(a[14]);
+  const c10::DeviceGuard guard(q.device());
+  const AttnShape s = attn_shape(q, kw, a[12], a[15], a[16]);
+  ASSERT(vw.sizes() == kw.sizes() && kw.size(3) * 32 == s.D * bits, "K and V words must agree and match the head dim and the bit-width");
+  int32_t ends[16];
+  int nseg = 1;
+  const bool seg = a[13] != Py_None;
+  if (seg) {
+    PyObject *f = PySequence_Fast(a[13], "seg_ends must be a sequence");
+    if (!f) throw python_error();
+    const Py_ssize_t n = PySequence_Fast_GET_SIZE(f);
+    bool fine = n >= 1 && n <= 16;
+    if (fine) {
+      nseg = (int)n;
+      for (int i = 0; i < nseg; ++i) ends[i] = (int32_t)integer(PySequence_Fast_GET_ITEM(f, i));
+      fine = ends[nseg - 1] == Lk;
+    }
+    Py_DECREF(f);
+    ASSERT(fine, "seg_ends: 1..16 entries, the last one equal to Lk");
+  }
+  for (const auto &[t, n] : {std::pair(&ks, "k_chan_scale"), std::pair(kz, "k_chan_zp"), std::pair(&vs, "v_chan_scale"), std::pair(vz, "v_chan_zp")})
+    ASSERT(!t || (t->scalar_type() == at::kFloat && t->numel() >= nseg * s.Hkv * s.D && t->is_contiguous()),
+           "%s must be fp32 [nseg, Hkv, D] (more tables than segments are allowed)", n);
+  ASSERT(kw.scalar_type() == at::kInt && vw.scalar_type() == at::kInt, "words must be int32");
+  ASSERT(0 <= Lk && Lk <= s.Lstride, "Lk=%lld outside the cache of %lld tokens", (long long)Lk, (long long)s.Lstride);
+  check_limit_and_map(limit, map, s);
+  const size_t ws_bytes = workspace_bytes(s, Lk, nseg, splits);
+  at::Tensor ws;
+  if (ws_bytes) ws = empty({(int64_t)ws_bytes}, at::kByte, q);
+  check(varq_fused_attn_channel(q.data_ptr(), s.out.data_ptr(), ptr<int32_t>(kw), ptr<float>(ks), ptr<float>(kz), ptr<int32_t>(vw), ptr<float>(vs),
+                                ptr<float>(vz), nseg, seg ? ends : nullptr, (int)bits, (int)s.B, (int)s.Hq, (int)s.Hkv, ptr<int32_t>(map), (int)s.Lq,
+                                (int)Lk, (int)s.Lstride, (int)s.D, ptr<int32_t>(limit), (float)real(a[9]), s.layout, io_code(q),
+                                ws_bytes ? ws.data_ptr() : nullptr, ws_bytes, (int)splits, stream_of(q)), "varq_fused_attn_channel");
+  return wrap(s.out);
+}
+
+// ---- packed cache -------------------------------------------------------------------------------
+// The cache hands its buffers over as one tuple of constants, built once:
+// (B, H, Lmax, D, group, asym, eps, ((bits, heads, k_words, k_scale, k_zp, v_words, v_scale, v_zp, slot, head_map), ...))
+struct Cache {
+  int64_t B, H, Lmax, D, group;
+  bool asym;
+  float eps;
+  PyObject *classes;
+  explicit Cache(PyObject *t) {
+    auto at_ = [&](int i) { return PyTuple_GET_ITEM(t, i); };
+    ASSERT(PyTuple_Check(t) && PyTuple_GET_SIZE(t) == 8, "cache tuple");
+    B = integer(at_(0)); H = integer(at_(1)); Lmax = integer(at_(2)); D = integer(at_(3)); group = integer(at_(4));
+    asym = truth(at_(5)); eps = (float)real(at_(6)); classes = at_(7);
+  }
+  Py_ssize_t size() const { return PyTuple_GET_SIZE(classes); }
+};
+struct CacheClass {
+  int64_t bits, heads;
+  at::Tensor k_words, k_scale, k_zp, v_words, v_scale, v_zp, slot, head_map;
+  explicit CacheClass(PyObject *t) {
+    auto g = [&](int i) -> const at::Tensor & { return THPVariable_Unpack(PyTuple_GET_ITEM(t, i)); };
+    bits = integer(PyTuple_GET_ITEM(t, 0)); heads = integer(PyTuple_GET_ITEM(t, 1));
+    k_words = g(2); k_scale = g(3); k_zp = g(4); v_words = g(5); v_scale = g(6); v_zp = g(7); slot = g(8); head_map = g(9);
+  }
+};
+
+// cache_append(cache, len, k, v, layout) -> tokens appended
+PyObject *cache_append(PyObject *const *a) {
+  const Cache c(a[0]);
+  const int64_t len = integer(a[1]);
+  ASSERT(THPVariable_Check(a[2]) && THPVariable_Check(a[3]), "append: tensors");
+  at::Tensor k = THPVariable_Unpack(a[2]), v = THPVariable_Unpack(a[3]);
+  const int lay = layout_code(a[4]), h = lay == VARQ_LAYOUT_BHLC ? 1 : 2;
+  ASSERT(k.dim() == 4 && k.size(0) == c.B && k.size(h) == c.H && k.size(3) == c.D && v.sizes() == k.sizes(), "append: the step does not fit the cache");
+  const int64_t n = k.size(3 - h);
+  ASSERT(len + n <= c.Lmax, "cache overflow");
+  gpu(a[2], "k"); gpu(a[3], "v");
+  k = k.contiguous(); v = v.contiguous();
+  const c10::DeviceGuard guard(k.device());
+  void *const st = stream_of(k);
+  const int kd = dtype_code(k), vd = dtype_code(v);
+  const int64_t rows = c.B * c.H * n;
+  for (Py_ssize_t i = 0; i < c.size(); ++i) {
+    const CacheClass cl(PyTuple_GET_ITEM(c.classes, i));
+    // input rows in memory order -> output row b*hc*Lmax + slot(h)*Lmax + len + l
+    const int64_t bs = cl.heads * c.Lmax;
+    const int64_t bhlc[8] = {c.B, c.H, n, bs, c.Lmax, 1, len, 1}, blhc[8] = {c.B, n, c.H, bs, 1, c.Lmax, len, 2};
+    const int64_t *map = lay == VARQ_LAYOUT_BHLC ? bhlc : blhc;
+    float *kz = c.asym ? ptr<float>(cl.k_zp) : nullptr, *vz = c.asym ? ptr<float>(cl.v_zp) : nullptr;
+    if (kd == vd && 2 * c.B <= 65535) {
+      check(varq_quant_pack_rows2(k.data_ptr(), v.data_ptr(), kd, rows, (int)c.D, (int)c.group, (int)cl.bits, c.asym, c.eps, map, ptr<int32_t>(cl.slot),
+                                  ptr<int32_t>(cl.k_words), ptr<float>(cl.k_scale), kz, ptr<int32_t>(cl.v_words), ptr<float>(cl.v_scale), vz, st),
+            "varq_quant_pack_rows2");
+    } else {   // K and V of different dtypes (Infinity: fp32 K after cos-norm, bf16 V)
+      check(varq_quant_pack_rows(k.data_ptr(), kd, rows, (int)c.D, (int)c.group, (int)cl.bits, c.asym, c.eps, map, ptr<int32_t>(cl.slot),
+                                 ptr<int32_t>(cl.k_words), ptr<float>(cl.k_scale), kz, st), "varq_quant_pack_rows");
+      check(varq_quant_pack_rows(v.data_ptr(), vd, rows, (int)c.D, (int)c.group, (int)cl.bits, c.asym, c.eps, map, ptr<int32_t>(cl.slot),
+                                 ptr<int32_t>(cl.v_words), ptr<float>(cl.v_scale), vz, st), "varq_quant_pack_rows");
+    }
+  }
+  return PyLong_FromLongLong(n);
+}
+
+// cache_prepare(cache, len, qkv, q_scale_mul | None, l2norm, norm_eps, cos | None, sin | None, token_start) -> q
+PyObject *cache_prepare(PyObject *const *a) {
+  const Cache c(a[0]);
+  const int64_t len = integer(a[1]), start = integer(a[8]);
+  const at::Tensor qkv = gpu(a[2], "qkv").contiguous();
+  ASSERT(qkv.dim() == 5 && qkv.size(2) == 3 && qkv.size(0) == c.B && qkv.size(3) == c.H && qkv.size(4) == c.D, "append_from_qkv: qkv [B,n,3,H,D] of the cache's sizes");
+  const int64_t n = qkv.size(1);
+  ASSERT(len + n <= c.Lmax, "cache overflow");
+  const at::Tensor *mul = maybe(a[3], "q_scale_mul"), *cs = maybe(a[6], "rope cos"), *sn = maybe(a[7], "rope sin");
+  if (cs || sn) {
+    ASSERT(cs && sn && cs->dim() == 2 && cs->scalar_type() == at::kFloat && sn->scalar_type() == at::kFloat && cs->is_contiguous() && sn->is_contiguous(), "rope tables must be contiguous fp32");
+    ASSERT(cs->sizes() == sn->sizes() && cs->size(1) == c.D / 2 && cs->size(0) >= start + n, "rope tables are too small");
+  }
+  if (mul) ASSERT(mul->scalar_type() == at::kFloat && mul->numel() == c.H && mul->is_contiguous(), "q_scale_mul must be contiguous fp32 [H]");
+  const c10::DeviceGuard guard(qkv.device());
+  const at::Tensor q = empty({c.B, c.H, n, c.D}, at::kBFloat16, qkv);
+  for (Py_ssize_t i = 0; i < c.size(); ++i) {
+    const CacheClass cl(PyTuple_GET_ITEM(c.classes, i));
+    const int64_t map[8] = {c.B, n, c.H, cl.heads * c.Lmax, 1, c.Lmax, len, 2};
+    check(varq_qkv_prepare_append(qkv.data_ptr(), dtype_code(qkv), (int)c.B, (int)n, (int)c.H, (int)c.D, ptr<float>(mul), truth(a[4]), (float)real(a[5]),
+                                  ptr<float>(cs), ptr<float>(sn), (int)start, q.data_ptr(), (int)c.group, (int)cl.bits, c.asym, c.eps, map,
+                                  ptr<int32_t>(cl.slot), ptr<int32_t>(cl.k_words), ptr<float>(cl.k_scale), c.asym ? ptr<float>(cl.k_zp) : nullptr,
+                                  ptr<int32_t>(cl.v_words), ptr<float>(cl.v_scale), c.asym ? ptr<float>(cl.v_zp) : nullptr, stream_of(qkv)),
+          "varq_qkv_prepare_append");
+  }
+  return wrap(q);
+}
+
+// ---- module -------------------------------------------------------------------------------------
+template <PyObject *(*F)(PyObject *const *), int N> PyObject *fixed(PyObject *, PyObject *const *a, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  need_args(n, N, "native call");
+  return F(a);
+  END_HANDLE_TH_ERRORS
+}
+template <PyObject *(*F)(PyObject *const *, Py_ssize_t)> PyObject *varying(PyObject *, PyObject *const *a, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  return F(a, n);
+  END_HANDLE_TH_ERRORS
+}
+PyObject *set_error(PyObject *, PyObject *e) {
+  Py_INCREF(e);
+  Py_XDECREF(g_varq_error);
+  g_varq_error = e;
+  Py_RETURN_NONE;
+}
+
+#define FIXED(name, n) {#name, (PyCFunction)(void (*)(void))fixed<name, n>, METH_FASTCALL, nullptr}
+PyMethodDef g_methods[] = {
+    FIXED(quant_rows, 5), FIXED(quant_shared, 6), FIXED(pack, 2), FIXED(unpack, 3), FIXED(dequant, 6), FIXED(attn, 18), FIXED(attn_channel, 17),
+    FIXED(cache_append, 5), FIXED(cache_prepare, 9),
+    {"quant_step", (PyCFunction)(void (*)(void))varying<quant_step>, METH_FASTCALL, nullptr},
+    {"set_error", set_error, METH_O, nullptr},
+    {nullptr, nullptr, 0, nullptr}};
+PyModuleDef g_module = {PyModuleDef_HEAD_INIT, "_host", nullptr, -1, g_methods, nullptr, nullptr, nullptr, nullptr};
+
+}  // namespace
+
+PyMODINIT_FUNC PyInit__host(void) { return PyModule_Create(&g_module); }

@@ -12,7 +12,7 @@ from typing import Any, Dict, List, Optional, Sequence, Union
 
 import torch
 
-from . import ops
+from . import _lib, ops
 
 
 class _BitClass:
@@ -49,6 +49,10 @@ class PackedKVCache:
         self.classes: List[_BitClass] = [
             _BitClass(b, [h for h in range(H) if per_head[h] == b], B, H, Lmax, D, group_size, device)
             for b in sorted(set(per_head))]
+        # what the native host layer reads, built once: sizes and the buffers of every class
+        self._native = (B, H, Lmax, D, group_size, not symmetric, eps,
+                        tuple((c.bits, len(c.heads), c.k_words, c.k_scale, c.k_zp, c.v_words, c.v_scale, c.v_zp, c.slot, c.head_map)
+                              for c in self.classes))
 
     def reset(self):
         self.len = 0
@@ -123,32 +127,7 @@ class PackedKVCache:
         """Quantize + pack one step into tokens len..len+n of the cache.  The step is
         [B,H,n,D] (layout 'BHLc') or [B,n,H,D] ('BLHc', the flash-attention layout of
         VAR/models/basic_var.py:127-131); either is read where it lies."""
-        assert layout in ('BHLc', 'BLHc')
-        if layout == 'BHLc':
-            B, H, n, D = k.shape
-        else:
-            B, n, H, D = k.shape
-        assert (B, H, D) == (self.B, self.H, self.D) and v.shape == k.shape
-        assert self.len + n <= self.Lmax, 'cache overflow'
-        k, v = k.contiguous(), v.contiguous()
-        for c in self.classes:
-            hc = len(c.heads)
-            # input rows in memory order -> output row b*hc*Lmax + slot(h)*Lmax + len + l
-            if layout == 'BHLc':
-                rowmap = [B, H, n, hc * self.Lmax, self.Lmax, 1, self.len, 1]
-            else:
-                rowmap = [B, n, H, hc * self.Lmax, 1, self.Lmax, self.len, 2]
-            asym = not self.symmetric
-            if k.dtype == v.dtype and 2 * rowmap[0] <= 65535:
-                ops.quant_pack_rows_pair_into(k, v, self.group, c.bits, asym, self.eps,
-                                              (c.k_words, c.k_scale, c.k_zp if asym else None),
-                                              (c.v_words, c.v_scale, c.v_zp if asym else None), rowmap, c.slot)
-            else:   # K and V of different dtypes (Infinity: fp32 K after cos-norm, bf16 V)
-                ops.quant_pack_rows_into(k, self.group, c.bits, asym, self.eps, c.k_words, c.k_scale,
-                                         c.k_zp if asym else None, rowmap, c.slot)
-                ops.quant_pack_rows_into(v, self.group, c.bits, asym, self.eps, c.v_words, c.v_scale,
-                                         c.v_zp if asym else None, rowmap, c.slot)
-        self.len += n
+        self.len += _lib.host().cache_append(self._native, self.len, k, v, layout)
 
     def append_from_qkv(self, qkv: torch.Tensor, q_scale_mul: Optional[torch.Tensor] = None, l2norm: bool = False,
                         norm_eps: float = 1e-12, rope=None, token_start: Optional[int] = None) -> torch.Tensor:
@@ -156,21 +135,11 @@ class PackedKVCache:
         rotated if asked) and v are quantized into tokens len..len+n, the prepared q comes back
         as bf16 [B,H,n,D] (Infinity/infinity/models/basic.py:316-330 in one kernel).
         token_start (default: the cache length) selects the rotary table rows."""
-        B, n, three, H, D = qkv.shape
-        assert three == 3 and (B, H, D) == (self.B, self.H, self.D)
-        assert self.len + n <= self.Lmax, 'cache overflow'
-        qkv = qkv.contiguous()
-        q_out = torch.empty((B, H, n, D), dtype=torch.bfloat16, device=qkv.device)
-        asym = not self.symmetric
-        start = self.len if token_start is None else token_start
-        for c in self.classes:
-            hc = len(c.heads)
-            rowmap = [B, n, H, hc * self.Lmax, 1, self.Lmax, self.len, 2]
-            ops.qkv_prepare_append(qkv, q_out, self.group, c.bits, asym, self.eps, c.k_words, c.k_scale,
-                                   c.k_zp if asym else None, c.v_words, c.v_scale, c.v_zp if asym else None,
-                                   rowmap, c.slot, q_scale_mul, l2norm, norm_eps, rope, start)
-        self.len += n
-        return q_out
+        cos, sin = (None, None) if rope is None else rope
+        q = _lib.host().cache_prepare(self._native, self.len, qkv, q_scale_mul, l2norm, norm_eps, cos, sin,
+                                      self.len if token_start is None else token_start)
+        self.len += q.shape[2]
+        return q
 
     def attend(self, q: torch.Tensor, softmax_scale: float, kv_limit: Optional[torch.Tensor] = None,
                out: Optional[torch.Tensor] = None, exact_codes: bool = False, out_layout: str = 'BHLc') -> torch.Tensor:
@@ -181,6 +150,11 @@ class PackedKVCache:
         [B,Lq,C] for its output projection (no transposing copy)."""
         assert self.len > 0, 'attend on an empty cache: append keys and values first'
         assert out_layout in ('BHLc', 'BLHc')
+        if len(self.classes) == 1:
+            c, asym = self.classes[0], not self.symmetric
+            return _lib.host().attn(q, c.k_words, c.k_scale, c.k_zp if asym else None, c.v_words, c.v_scale, c.v_zp if asym else None,
+                                    c.bits, c.bits, self.len, softmax_scale, kv_limit, None, out, self.splits, 'BHLc', exact_codes,
+                                    out_layout)
         if out is None:
             B_, H_, Lq_, D_ = q.shape
             out = torch.empty((B_, Lq_, H_, D_) if out_layout == 'BLHc' else q.shape, dtype=q.dtype, device=q.device)

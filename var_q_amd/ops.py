@@ -8,8 +8,6 @@ from __future__ import annotations
 
 from typing import Optional, Sequence, Tuple
 
-import ctypes
-
 import torch
 
 from . import _lib
@@ -90,18 +88,7 @@ def quant_pack_rows(x: torch.Tensor, group: int, bits: int, asym: bool = True, e
     """One-pass quantize+pack with one (scale[, zp]) per `group` contiguous
     channels of each row.  x [..., c] -> (words [..., c*bits/32] int32,
     scale [..., c/group] fp32, zp like scale or None)."""
-    _gpu(x, 'x')
-    x = x.contiguous()
-    *lead, c = x.shape
-    n_rows = x.numel() // c if c else 0
-    words = torch.empty((*lead, c * bits // 32), dtype=torch.int32, device=x.device)
-    scale = torch.empty((*lead, c // group), dtype=torch.float32, device=x.device)
-    zp = torch.empty_like(scale) if asym else None
-    lib = _lib.load()
-    with _on_device(x.device):
-        check(lib.varq_quant_pack_rows(x.data_ptr(), _dt(x), n_rows, c, group, bits, int(asym), eps, None, None,
-                                       words.data_ptr(), scale.data_ptr(), _ptr(zp), _stream(x)), 'varq_quant_pack_rows')
-    return words, scale, zp
+    return _lib.host().quant_rows(x, group, bits, asym, eps)
 
 
 def quant_pack_rows_into(x: torch.Tensor, group: int, bits: int, asym: bool, eps: float,
@@ -161,6 +148,11 @@ def quant_pack(x: torch.Tensor, reduce_dims: Sequence[int], bits: int, asym: boo
     contiguous buffer that has the shape of the result except for more room along
     out_token_dim (1 or 2); the returned codes are that window of `out`.  scale_out, zp_out:
     contiguous fp32 buffers of n_groups elements that receive the scale and zero-point."""
+    if out is None and scale_out is None and zp_out is None:
+        mask = 0
+        for d in reduce_dims:
+            mask |= 1 << (d % 4)
+        return _lib.host().quant_shared(x, mask, bits, asym, eps, pack)
     _gpu(x, 'x')
     assert x.dim() == 4, 'expected a 4-D [B,L,H,c] / [B,H,L,c] tensor'
     x = x.contiguous()
@@ -251,28 +243,11 @@ def quant_pack_pair(x0: torch.Tensor, x1: torch.Tensor, reduce_dims: Sequence[in
 # pack / unpack of int8 codes
 # ---------------------------------------------------------------------------
 def pack(codes: torch.Tensor, bits: int) -> torch.Tensor:
-    _gpu(codes, 'q_int8')
-    codes = codes.contiguous()
-    *lead, c = codes.shape
-    vals = 32 // bits
-    rows = codes.numel() // c if c else 0
-    words = torch.empty((*lead, (c + vals - 1) // vals), dtype=torch.int32, device=codes.device)
-    lib = _lib.load()
-    with _on_device(codes.device):
-        check(lib.varq_pack(codes.data_ptr(), rows, c, bits, words.data_ptr(), _stream(codes)), 'varq_pack')
-    return words
+    return _lib.host().pack(codes, bits)
 
 
 def unpack(words: torch.Tensor, c: int, bits: int) -> torch.Tensor:
-    _gpu(words, 'packed')
-    words = words.contiguous()
-    *lead, w = words.shape
-    rows = words.numel() // w if w else 0
-    codes = torch.empty((*lead, c), dtype=torch.int8, device=words.device)
-    lib = _lib.load()
-    with _on_device(words.device):
-        check(lib.varq_unpack(words.data_ptr(), rows, c, bits, codes.data_ptr(), _stream(words)), 'varq_unpack')
-    return codes
+    return _lib.host().unpack(words, c, bits)
 
 
 # ---------------------------------------------------------------------------
@@ -283,40 +258,9 @@ def dequant(q: torch.Tensor, scale: torch.Tensor, zp: Optional[torch.Tensor], c:
     """q: packed int32 words [n0,n1,n2,W] or int8 codes [n0,n1,n2,c].  scale
     (and zp) broadcast against [n0,n1,n2,c] in the first three dims and hold
     1, c/g or c entries in the last (per-row, group-wise, per-channel); any
-    strides, including stride-0 expands, are used as they are."""
-    _gpu(q, 'q'); _gpu(scale, 'scale')
-    assert q.dim() == 4 and scale.dim() == 4
-    q = q.contiguous()
-    n0, n1, n2 = q.shape[:3]
-    packed = q.dtype == torch.int32
-    assert packed or q.dtype == torch.int8
-    if zp is not None and (zp.shape != scale.shape or zp.stride() != scale.stride()):
-        zp = zp.expand_as(scale).contiguous()
-        scale = scale.contiguous()
-    s3 = scale.shape[3]
-    assert c % s3 == 0, f'scale last dim {s3} does not divide c={c}'
-    group = c // s3
-    strides = []
-    for d in range(4):
-        if scale.shape[d] == 1:
-            strides.append(0)
-        else:
-            assert d == 3 or scale.shape[d] == q.shape[d], f'scale dim {d} = {scale.shape[d]} vs {q.shape[d]}'
-            strides.append(scale.stride(d))
-    out = torch.empty((n0, n1, n2, c), dtype=out_dtype, device=q.device)
-    lib = _lib.load()
-    # collapse the leading dims when the scale does not depend on them: fuller blocks
-    shape = [n0, n1, n2, c]
-    if strides[0] == 0 and strides[1] == 0 and strides[2] == 0:
-        shape = [1, 1, n0 * n1 * n2, c]
-    elif strides[0] == 0 and strides[1] == 0:
-        pass
-    shape, strides, _ = _rows_as_channels(packed, shape, strides, group, bits, None)
-    with _on_device(q.device):
-        check(lib.varq_dequant(q.data_ptr() if packed else None, None if packed else q.data_ptr(),
-                               scale.data_ptr(), _ptr(zp), i64arr(shape), i64arr(strides), group, bits, None,
-                               out.data_ptr(), _DT[out_dtype], _stream(q)), 'varq_dequant')
-    return out
+    strides, including stride-0 expands, are used as they are, and so is a q whose rows are
+    dense (a window of a cache buffer)."""
+    return _lib.host().dequant(q, scale, zp, c, bits, _DT[out_dtype])
 
 
 def dequant_window(words: torch.Tensor, scale: torch.Tensor, zp: Optional[torch.Tensor], shape4: Sequence[int],
@@ -400,49 +344,6 @@ def qkv_prepare_append(qkv: torch.Tensor, q_out: torch.Tensor, group: int, bits:
 # ---------------------------------------------------------------------------
 # fused dequant flash-attention
 # ---------------------------------------------------------------------------
-_LAYOUTS = {'BHLc': 0, 'BLHc': 1}
-# dtypes of q / out (the library's dtype codes): bf16 everywhere, fp16 for head dim 64 (the VAR path)
-_ATTN_DT = {torch.bfloat16: 1, torch.float16: 2}
-
-
-def _attn_dims(q, k_words, layout):
-    """(B, Hq, Lq, D, Hkv, Lstride, W) of the attention operands in either layout."""
-    assert layout in _LAYOUTS, f'layout must be one of {sorted(_LAYOUTS)}'
-    if layout == 'BHLc':
-        B, Hq, Lq, D = q.shape
-        Bk, Hkv, Lstride, W = k_words.shape
-    else:
-        B, Lq, Hq, D = q.shape
-        Bk, Lstride, Hkv, W = k_words.shape
-    assert Bk == B, 'batch sizes of q and the cache differ'
-    return B, Hq, Lq, D, Hkv, Lstride, W
-
-
-def _attn_out(q, out, layout, out_layout, dims):
-    """(layout code of the call, output tensor): out looks like q unless out_layout says
-    tokens first for a heads-first call."""
-    B, Hq, Lq, D = dims
-    if out_layout is None or out_layout == layout:
-        code, shape = _LAYOUTS[layout], q.shape
-    else:
-        assert layout == 'BHLc' and out_layout == 'BLHc', 'out_layout: only tokens-first out of a heads-first call'
-        code, shape = 2, (B, Lq, Hq, D)
-    if out is None:
-        out = torch.empty(shape, dtype=q.dtype, device=q.device)
-    assert out.dtype == q.dtype and tuple(out.shape) == tuple(shape) and out.is_contiguous(), \
-        'out must be contiguous, of the dtype of q and of the shape its layout implies'
-    return code, out
-
-
-def _attn_workspace(lib, B, Hkv, Lq, Lk, D, nseg, splits, device):
-    """Device memory for the partial results of a launch that shares keys out (None if the
-    library would not); allocated on the current stream, so its reuse after the call is ordered."""
-    n = int(lib.varq_fused_attn_workspace_bytes(B, Hkv, Lq, Lk, D, nseg, int(splits)))
-    if n == 0:
-        return None, 0
-    return torch.empty(n, dtype=torch.uint8, device=device), n
-
-
 def fused_attn(q: torch.Tensor, k_words: torch.Tensor, k_scale: torch.Tensor, k_zp: Optional[torch.Tensor],
                v_words: torch.Tensor, v_scale: torch.Tensor, v_zp: Optional[torch.Tensor],
                k_bits: int, v_bits: int, Lk: int, softmax_scale: float,
@@ -463,42 +364,8 @@ def fused_attn(q: torch.Tensor, k_words: torch.Tensor, k_scale: torch.Tensor, k_
     first -- what an attention module hands to its output projection, without a transposing copy.
     splits: over how many workgroups the keys of a query block are shared out (0: the
     library decides from the shape, 1: never, 2..8: exactly)."""
-    for t, n in ((q, 'q'), (k_words, 'k_words'), (v_words, 'v_words'), (k_scale, 'k_scale'), (v_scale, 'v_scale')):
-        _gpu(t, n)
-        assert t.is_contiguous(), f'{n} must be contiguous'
-    assert q.dtype in _ATTN_DT and q.dim() == 4, 'q must be bf16 or fp16'
-    B, Hq, Lq, D, Hkv, Lstride, Wk = _attn_dims(q, k_words, layout)
-    assert v_words.shape[:3] == k_words.shape[:3]
-    assert Wk * 32 == D * k_bits and v_words.shape[3] * 32 == D * v_bits
-    assert k_scale.shape[:3] == k_words.shape[:3] and v_scale.shape[:3] == k_words.shape[:3]
-    k_group, v_group = D // k_scale.shape[3], D // v_scale.shape[3]
-    for z, sc, n in ((k_zp, k_scale, 'k_zp'), (v_zp, v_scale, 'v_zp')):
-        if z is not None:
-            _gpu(z, n)
-            assert z.shape == sc.shape and z.dtype == torch.float32 and z.is_contiguous(), f'{n} must look like its scale'
-    assert k_scale.dtype == torch.float32 and v_scale.dtype == torch.float32 and k_words.dtype == torch.int32 \
-        and v_words.dtype == torch.int32
-    assert 0 <= Lk <= Lstride, f'Lk={Lk} outside the cache of {Lstride} tokens'
-    code, out = _attn_out(q, out, layout, out_layout, (B, Hq, Lq, D))
-    if kv_limit is not None:
-        _gpu(kv_limit, 'kv_limit')
-        assert kv_limit.dtype == torch.int32 and kv_limit.numel() == Lq and kv_limit.is_contiguous()
-    if head_map is not None:
-        _gpu(head_map, 'head_map')
-        assert head_map.dtype == torch.int32 and head_map.numel() == Hkv
-    else:
-        assert Hkv == Hq
-    lib = _lib.load()
-    with _on_device(q.device):
-        ws, ws_bytes = _attn_workspace(lib, B, Hkv, Lq, Lk, D, 1, splits, q.device)
-        check(lib.varq_fused_attn(q.data_ptr(), out.data_ptr(),
-                                  k_words.data_ptr(), k_scale.data_ptr(), _ptr(k_zp), k_bits, k_group,
-                                  v_words.data_ptr(), v_scale.data_ptr(), _ptr(v_zp), v_bits, v_group,
-                                  B, Hq, Hkv, _ptr(head_map), Lq, Lk, Lstride, D,
-                                  _ptr(kv_limit), float(softmax_scale), code, _ATTN_DT[q.dtype],
-                                  int(bool(exact_codes)), _ptr(ws), ws_bytes,
-                                  int(splits), _stream(q)), 'varq_fused_attn')
-    return out
+    return _lib.host().attn(q, k_words, k_scale, k_zp, v_words, v_scale, v_zp, k_bits, v_bits, Lk, softmax_scale, kv_limit,
+                            head_map, out, splits, layout, exact_codes, out_layout)
 
 
 def fused_attn_channel(q: torch.Tensor, k_words: torch.Tensor, k_chan_scale: torch.Tensor,
@@ -518,42 +385,5 @@ def fused_attn_channel(q: torch.Tensor, k_words: torch.Tensor, k_chan_scale: tor
     append methods has one table per step (VAR_Q/quant.py:196-201).
     With a single table the zero-point of K may be None even for an affine K: it shifts all
     logits of a query alike.  splits, layout and out_layout as in fused_attn."""
-    for t, n in ((q, 'q'), (k_words, 'k_words'), (v_words, 'v_words'), (k_chan_scale, 'k_chan_scale'),
-                 (v_chan_scale, 'v_chan_scale')):
-        _gpu(t, n)
-        assert t.is_contiguous(), f'{n} must be contiguous'
-    assert q.dtype in _ATTN_DT and q.dim() == 4, 'q must be bf16 or fp16'
-    B, Hq, Lq, D, Hkv, Lstride, W = _attn_dims(q, k_words, layout)
-    assert v_words.shape == k_words.shape and W * 32 == D * bits
-    nseg = 1 if seg_ends is None else len(seg_ends)
-    ends = None
-    if seg_ends is not None:
-        assert 1 <= nseg <= 16 and int(seg_ends[-1]) == Lk, 'seg_ends: 1..16 entries, the last one equal to Lk'
-        ends = (ctypes.c_int32 * nseg)(*[int(e) for e in seg_ends])
-    for t, n in ((k_chan_scale, 'k_chan_scale'), (k_chan_zp, 'k_chan_zp'), (v_chan_scale, 'v_chan_scale'),
-                 (v_chan_zp, 'v_chan_zp')):
-        if t is not None:
-            _gpu(t, n)
-            assert t.dtype == torch.float32 and t.numel() >= nseg * Hkv * D and t.is_contiguous(), \
-                f'{n} must be fp32 [nseg, Hkv, D] (more tables than segments are allowed)'
-    assert k_words.dtype == torch.int32 and v_words.dtype == torch.int32
-    assert 0 <= Lk <= Lstride, f'Lk={Lk} outside the cache of {Lstride} tokens'
-    code, out = _attn_out(q, out, layout, out_layout, (B, Hq, Lq, D))
-    if kv_limit is not None:
-        _gpu(kv_limit, 'kv_limit')
-        assert kv_limit.dtype == torch.int32 and kv_limit.numel() == Lq and kv_limit.is_contiguous()
-    if head_map is not None:
-        _gpu(head_map, 'head_map')
-        assert head_map.dtype == torch.int32 and head_map.numel() == Hkv
-    else:
-        assert Hkv == Hq
-    lib = _lib.load()
-    with _on_device(q.device):
-        ws, ws_bytes = _attn_workspace(lib, B, Hkv, Lq, Lk, D, nseg, splits, q.device)
-        check(lib.varq_fused_attn_channel(q.data_ptr(), out.data_ptr(),
-                                          k_words.data_ptr(), k_chan_scale.data_ptr(), _ptr(k_chan_zp),
-                                          v_words.data_ptr(), v_chan_scale.data_ptr(), _ptr(v_chan_zp),
-                                          nseg, ends, bits, B, Hq, Hkv, _ptr(head_map), Lq, Lk, Lstride, D,
-                                          _ptr(kv_limit), float(softmax_scale), code, _ATTN_DT[q.dtype],
-                                          _ptr(ws), ws_bytes, int(splits), _stream(q)), 'varq_fused_attn_channel')
-    return out
+    return _lib.host().attn_channel(q, k_words, k_chan_scale, k_chan_zp, v_words, v_chan_scale, v_chan_zp, bits, Lk, softmax_scale,
+                                    kv_limit, head_map, out, seg_ends, splits, layout, out_layout)

@@ -7,7 +7,7 @@ changes underneath:
 
 * scale + codes + packing is one kernel chain (ops.quant_pack /
   ops.quant_pack_rows) instead of ~15 torch launches with fp32 temporaries;
-* unpack + dequant is one kernel (ops.dequant_window);
+* unpack + dequant is one kernel;
 * the cache lives in pre-allocated buffers that grow geometrically; a step is
   written in place instead of re-copying the whole cache with torch.cat
   (VAR_Q/quant.py:200-201).  `cached_item` / `cached_scale` are views of the
@@ -33,7 +33,7 @@ from typing import Dict, List, Optional, Tuple
 import torch
 
 from . import _lib, ops
-from ._lib import VarqError, check, i64arr
+from ._lib import VarqError
 
 _REF_METHODS = ('G_TENSOR', 'G_SCALE_HEAD_DIM', 'G_HEAD_DIM', 'G_SCALE', 'G_TOKEN', 'G_TOKEN_HEAD')
 _EXT_METHODS = ('G_GROUP', 'G_HEAD')
@@ -132,12 +132,10 @@ class VAR_Q:
         self.bound_min = -(2 ** (quant_bits - 1))
         self.bound_max = (2 ** (quant_bits - 1)) - 1
 
-        self.quantized_item: Optional[torch.Tensor] = None
-        self.scale: Optional[torch.Tensor] = None
-        self.zp: Optional[torch.Tensor] = None
+        self._current: List[Optional[torch.Tensor]] = [None, None, None]   # quantized_item, scale, zp
+        self._window = None              # ... or where they lie, until someone looks (see _step_fast)
         self._pack_meta: Optional[Dict[str, int]] = None
         self._staged = None
-        self._fast_plans: Dict[Tuple[int, int, int, int], tuple] = {}
         self._reset_cache()
 
     # The reference derives dim_cat/dim_map once in __init__ and callers later
@@ -153,6 +151,39 @@ class VAR_Q:
         self._qkv_format = fmt
         self.dim_cat = 1 if fmt == 'BLHc' else 2
         self.dim_map = _dim_map(fmt)
+
+    # ---------------- the current step ----------------
+    def _look(self) -> List[Optional[torch.Tensor]]:
+        w = self._window
+        if w is not None:
+            self._window = None
+            buf, dim, start, n, srow, zrow, sshape = w
+            self._current = [buf.narrow(dim, start, n), srow.view(sshape), None if zrow is None else zrow.view(sshape)]
+        return self._current
+
+    @property
+    def quantized_item(self) -> Optional[torch.Tensor]:
+        return self._look()[0]
+
+    @quantized_item.setter
+    def quantized_item(self, t):
+        self._look()[0] = t
+
+    @property
+    def scale(self) -> Optional[torch.Tensor]:
+        return self._look()[1]
+
+    @scale.setter
+    def scale(self, t):
+        self._look()[1] = t
+
+    @property
+    def zp(self) -> Optional[torch.Tensor]:
+        return self._look()[2]
+
+    @zp.setter
+    def zp(self, t):
+        self._look()[2] = t
 
     # ---------------- cache views ----------------
     def _reset_cache(self):
@@ -256,107 +287,85 @@ class VAR_Q:
                 assert meta['orig_c'] == self._pack_meta['orig_c']
                 assert meta['pad_len'] == self._pack_meta['pad_len']
             self._pack_meta = meta
-        self.quantized_item, self.scale, self.zp = q, s, z
+        self._window, self._current = None, [q, s, z]
 
-    def _fast_prepare(self, x: torch.Tensor):
-        """First half of the one-call step (see `_step_fast`): room in the cache buffer and the
-        table row for a step of the shipped rule, nothing launched, no state changed.  None
-        when the quantizer or the item is of another kind."""
+    def _fast_place(self, x: torch.Tensor):
+        """Where the one-call step (see `_step_fast`) puts a step of the shipped rule: (tokens, heads,
+        channels, table row, first token), room in the cache buffer and the tables made; nothing
+        launched, no step added.  None when the quantizer or the item is of another kind."""
         bits = self.quant_bits
-        if isinstance(x, torch.Tensor) and x.numel() == 0:
-            return None                       # (quant() says why an empty step is refused)
         if self.quant_method != 'G_SCALE_HEAD_DIM' or not self.pack_to_int32 or bits not in (2, 4, 8):
             return None
-        if not isinstance(x, torch.Tensor) or x.dim() != 4 or not x.is_cuda or not x.is_contiguous() \
-                or x.dtype not in ops._DT or self._c_item.dim != self.dim_cat:
+        if not isinstance(x, torch.Tensor) or x.dim() != 4 or not x.is_cuda or not x.is_contiguous() or x.dtype not in ops._DT:
             return None
-        k = len(self._seg_ends)
+        item, d, k = self._c_item, self.dim_cat, len(self._seg_ends)
         s0, s1, s2, c = x.shape
         vals = 32 // bits
-        if k >= MAX_TABLE_STEPS or c % vals or s0 * s1 * s2 == 0:
-            return None
-        bhl = self._qkv_format == 'BHLc'
-        H, n = (s1, s2) if bhl else (s2, s1)
-        buf = self._c_item.reserve([s0, s1, s2, c // vals], torch.int32, x.device)
-        if buf is None:
-            return None
-        meta = {'orig_c': int(c), 'vals_per_word': int(vals), 'pad_len': 0, 'bits': int(bits)}
-        if self._pack_meta is not None and self._pack_meta != meta:
+        if item.dim != d or k >= MAX_TABLE_STEPS or c % vals or s0 * s1 * s2 == 0:
+            return None                       # (quant() says why an empty step is refused)
+        n, H = (s1, s2) if d == 1 else (s2, s1)
+        meta = self._pack_meta
+        if meta is None:
+            self._pack_meta = {'orig_c': c, 'vals_per_word': vals, 'pad_len': 0, 'bits': bits}
+        elif meta['orig_c'] != c or meta['bits'] != bits:
             return None                       # (quant() raises the reference's assertion for this)
-        self._table_rows(H, c, x.device)
-        plan = self._fast_plans.get((s0, s1, s2, c))
-        if plan is None:
-            sh = i64arr([s0, s1, s2, c])
-            mask = 0b0101 if bhl else 0b0011                      # reduce batch and tokens
-            ws_bytes = max(int(_lib.load().varq_quant_workspace_bytes(sh, mask)), 8)
-            plan = self._fast_plans[(s0, s1, s2, c)] = (sh, mask, ws_bytes)
-        start, cap, per_tok = self._c_item.len, buf.shape[self.dim_cat], (1 if bhl else H)
-        out_map = (n * per_tok, (cap - n) * per_tok, start * per_tok)
-        srow = self._tab_scale[k]
-        zrow = None if self.symmetric else self._tab_zp[k]
-        return (x, buf, srow, zrow, plan, out_map, meta, bhl, H, n, c, start)
+        buf, start = item.buf, item.len
+        if buf is None or start + n > buf.shape[d] or buf.shape[0] != s0 or buf.shape[3 - d] != H:
+            if item.reserve([s0, s1, s2, c // vals], torch.int32, x.device) is None:
+                return None
+        if self._tab_scale is None or self._tab_scale.shape[1] != H or self._tab_scale.shape[2] != c:
+            self._table_rows(H, c, x.device)
+        return n, H, c, k, start
 
-    def _fast_commit(self, prep):
-        """Second half: the state that quant() followed by cache() leaves, the kernels having
-        written the codes and the table row in place."""
-        x, buf, srow, zrow, plan, out_map, meta, bhl, H, n, c, start = prep
-        sshape = (1, H, 1, c) if bhl else (1, 1, H, c)
-        self.quantized_item = buf.narrow(self.dim_cat, start, n)
-        self.scale = srow.view(sshape)
-        self.zp = None if zrow is None else zrow.view(sshape)
-        self._pack_meta = meta
+    def _fast_commit(self, place):
+        """The state that quant() followed by cache() leaves, the kernels having written the codes
+        and the table row in place."""
+        n, H, c, k, start = place
+        item, d = self._c_item, self.dim_cat
+        srow, zrow = self._tab_scale[k], None if self.symmetric else self._tab_zp[k]
+        sshape = (1, H, 1, c) if d == 2 else (1, 1, H, c)
+        self._window = (item.buf, d, start, n, srow, zrow, sshape)
         self._staged = None
-        self._c_item.len = start + n
-        eshape = (-1, -1, n, -1) if bhl else (-1, n, -1, -1)
-        scale, zp = self.scale, self.zp
-        self._c_scale.append_later(lambda: scale.expand(*eshape))
-        if zp is not None:
-            self._c_zp.append_later(lambda: zp.expand(*eshape))
-        self._seg_ends.append((self._seg_ends[-1] if self._seg_ends else 0) + n)
+        item.len = start + n
+        eshape = (-1, -1, n, -1) if d == 2 else (-1, n, -1, -1)
+        self._c_scale.append_later(lambda: srow.view(sshape).expand(*eshape))
+        if zrow is not None:
+            self._c_zp.append_later(lambda: zrow.view(sshape).expand(*eshape))
+        ends = self._seg_ends
+        ends.append(ends[-1] + n if ends else n)
 
     def _step_fast(self, x: torch.Tensor) -> bool:
         """quant(x) followed by cache() for the shipped rule (G_SCALE_HEAD_DIM, packed codes)
         with the host work of a generation step cut to one library call: same kernels, same
         state afterwards.  False (nothing done) when the quantizer or the item is of another
         kind; the caller then takes the two general calls."""
-        prep = self._fast_prepare(x)
-        if prep is None:
+        place = self._fast_place(x)
+        if place is None:
             return False
-        _, buf, srow, zrow, (sh, mask, ws_bytes), out_map, *_ = prep
-        ws = torch.empty(ws_bytes, dtype=torch.uint8, device=x.device)
-        with ops._on_device(x.device):
-            check(_lib.load().varq_quant_pack(x.data_ptr(), ops._DT[x.dtype], sh, mask, self.quant_bits,
-                                              int(not self.symmetric), self.eps, buf.data_ptr(), None, srow.data_ptr(),
-                                              None if zrow is None else zrow.data_ptr(), i64arr(out_map),
-                                              ws.data_ptr(), ws_bytes, ops._stream(x)), 'varq_quant_pack')
-        self._fast_commit(prep)
+        d = self.dim_cat
+        _lib.host().quant_step(0b0011 if d == 1 else 0b0101, self.quant_bits, not self.symmetric, self.eps, d, place[4], place[3],
+                               x, self._c_item.buf, self._tab_scale, self._tab_zp)
+        self._fast_commit(place)
         return True
 
     @staticmethod
     def _step_fast_pair(kq: 'VAR_Q', vq: 'VAR_Q', k: torch.Tensor, v: torch.Tensor) -> bool:
-        """`_step_fast` for K and V of a step in the same three launches, when the two
-        quantizers are configured alike and their caches stand at the same place."""
+        """`_step_fast` for K and V of a step in the same launches, when the two quantizers are
+        configured alike and their caches stand at the same place."""
         if not (isinstance(k, torch.Tensor) and isinstance(v, torch.Tensor)):
             return False
         if kq is vq or kq.quant_bits != vq.quant_bits or kq.symmetric != vq.symmetric or kq.eps != vq.eps \
                 or kq._qkv_format != vq._qkv_format or k.shape != v.shape or k.dtype != v.dtype or k.device != v.device:
             return False
-        pk = kq._fast_prepare(k)
+        pk = kq._fast_place(k)
         if pk is None:
             return False
-        pv = vq._fast_prepare(v)
-        if pv is None or pk[5] != pv[5]:          # (same window of the two cache buffers)
+        pv = vq._fast_place(v)
+        d = kq.dim_cat
+        if pv is None or pk[3:] != pv[3:] or kq._c_item.buf.shape[d] != vq._c_item.buf.shape[d]:   # (same window of the two cache buffers)
             return False
-        sh, mask, ws_bytes = pk[4]
-        ws = torch.empty(2 * ws_bytes, dtype=torch.uint8, device=k.device)
-        zk, zv = pk[3], pv[3]
-        with ops._on_device(k.device):
-            check(_lib.load().varq_quant_pack2(k.data_ptr(), v.data_ptr(), ops._DT[k.dtype], sh, mask, kq.quant_bits,
-                                               int(not kq.symmetric), kq.eps,
-                                               pk[1].data_ptr(), None, pk[2].data_ptr(), None if zk is None else zk.data_ptr(),
-                                               pv[1].data_ptr(), None, pv[2].data_ptr(), None if zv is None else zv.data_ptr(),
-                                               i64arr(pk[5]), ws.data_ptr(), 2 * ws_bytes, ops._stream(k)),
-                  'varq_quant_pack2')
+        _lib.host().quant_step(0b0011 if d == 1 else 0b0101, kq.quant_bits, not kq.symmetric, kq.eps, d, pk[4], pk[3],
+                               k, kq._c_item.buf, kq._tab_scale, kq._tab_zp, v, vq._c_item.buf, vq._tab_scale, vq._tab_zp)
         kq._fast_commit(pk)
         vq._fast_commit(pv)
         return True
@@ -429,9 +438,9 @@ class VAR_Q:
         else:
             ng = self.scale.shape[3]
             shape = (B, H, n, ng) if bhl else (B, n, H, ng)
-            self._tok_scale.append(self.scale.expand(*shape))
+            self._tok_scale.append_later(self.scale.expand(*shape))
             if self.zp is not None:
-                self._tok_zp.append(self.zp.expand(*shape))
+                self._tok_zp.append_later(self.zp.expand(*shape))
 
     # ---------------- dequantize ----------------
     def _dequant(self, q: torch.Tensor, scale: torch.Tensor, zp: Optional[torch.Tensor],
@@ -450,7 +459,7 @@ class VAR_Q:
         """The whole cache dequantized (VAR_Q/quant.py:216-224: fp32).  out_dtype bfloat16 / float16
         gives the fp32 product rounded once to that type -- bit for bit what `.to(out_dtype)` of the
         fp32 result is, without writing and re-reading the fp32 tensor."""
-        if self.cached_item is None:
+        if self._c_item.len == 0:
             return self.dequant_current(out_dtype)
         return self._dequant(self.cached_item, self.cached_scale, self.cached_zp, out_dtype)
 
@@ -469,8 +478,9 @@ class VAR_Q:
         price is memory: 4 bytes per cached element (up to 8 while the buffer has doubled), i.e.
         two to four times an unquantized bf16 cache, resident until the quantizer is deleted --
         172 MB per tensor at [2,16,10521,128].  `dequant_all()` itself always recomputes everything."""
-        self.quant(item)
-        self.cache()
+        if not self._step_fast(item):
+            self.quant(item)
+            self.cache()
         if not self.keep_dequantized:
             return self.dequant_all(out_dtype or torch.float32)
         d, n = self._c_deq, self.quantized_item.size(self.dim_cat)
@@ -490,19 +500,7 @@ def _dequant_views(q: torch.Tensor, scale: torch.Tensor, zp: Optional[torch.Tens
                    out_dtype: torch.dtype = torch.float32) -> torch.Tensor:
     """Dequantize codes given as a (possibly strided) 4-D view of a cache buffer
     whose rows are dense, with a scale that is any broadcastable strided view."""
-    assert q.dim() == 4 and scale.dim() == 4
-    n0, n1, n2, wq = q.shape
-    assert q.stride(3) == 1 and all(st % wq == 0 for st in q.stride()[:3]), 'rows of the code tensor must be dense'
-    rowmap = [n0, n1, n2, q.stride(0) // wq, q.stride(1) // wq, q.stride(2) // wq, 0, -1]
-    if zp is not None and (zp.shape != scale.shape or zp.stride() != scale.stride()):
-        scale, zp = scale.contiguous(), zp.expand_as(scale).contiguous()
-    s3 = scale.shape[3]
-    assert c % s3 == 0
-    group = c // s3
-    strides = [0 if scale.shape[d] == 1 else scale.stride(d) for d in range(4)]
-    for d in range(3):
-        assert scale.shape[d] in (1, q.shape[d]), f'scale dim {d}: {scale.shape[d]} vs {q.shape[d]}'
-    return ops.dequant_window(q, scale, zp, (n0, n1, n2, c), strides, group, bits, rowmap, out_dtype)
+    return _lib.host().dequant(q, scale, zp, c, bits, ops._DT[out_dtype])
 
 
 # methods whose scale does not depend on the token: one table per cached step
@@ -532,11 +530,11 @@ def fused_attention(q: torch.Tensor, k_quant: VAR_Q, v_quant: VAR_Q, softmax_sca
     kernels read is kept current by `cache()`, so a call launches the attention and nothing
     else.  kv_limit: int32 [Lq], query i sees keys j < kv_limit[i].  Returns a tensor of the
     attention's dtype in the shape of q."""
-    layout = k_quant.qkv_format
-    if v_quant.qkv_format != layout:
+    layout = k_quant._qkv_format
+    if v_quant._qkv_format != layout:
         raise ValueError(f'fused_attention: K is cached in layout {layout}, V in {v_quant.qkv_format}')
     for qz, n in ((k_quant, 'k_quant'), (v_quant, 'v_quant')):
-        if not qz.pack_to_int32 or qz.cached_item is None:
+        if not qz.pack_to_int32 or qz._c_item.buf is None:
             raise ValueError(f'fused_attention: {n} needs a packed cache (pack_to_int32=True, after cache())')
     bits = k_quant.quant_bits
     if v_quant.quant_bits != bits:
@@ -564,6 +562,8 @@ def fused_attention(q: torch.Tensor, k_quant: VAR_Q, v_quant: VAR_Q, softmax_sca
                                       v_quant._tab_zp, bits, Lk, softmax_scale, kv_limit=kv_limit, out=out,
                                       seg_ends=ends, layout=layout)
     if km in _TOKEN_METHODS and vm in _TOKEN_METHODS:
+        for qz in (k_quant, v_quant):
+            qz._tok_scale.view(), qz._tok_zp.view()      # (the steps appended since the last call)
         ks, kz, vs, vz = k_quant._tok_scale.buf, k_quant._tok_zp.buf, v_quant._tok_scale.buf, v_quant._tok_zp.buf
         if ks.shape[:3] != kbuf.shape[:3] or vs.shape[:3] != kbuf.shape[:3]:
             raise ValueError('fused_attention: scale buffers and code buffers differ in capacity')
