@@ -195,6 +195,19 @@ int varq_dequant(const int32_t *words, const int8_t *codes_i8, const float *scal
                  const int64_t *host_in_rowmap, void *out, int out_dtype, void *stream);
 
 /*
+ * The whole cache of a stepwise quantizer with a scale per (head, channel), dequantized: tokens
+ * [host_seg_end[s-1], host_seg_end[s]) use table s, (code - zp) * scale as above.  What
+ * VAR_Q/quant.py:216-224 does with the per-step scales expanded over their tokens and concatenated
+ * (196-201): one fp32 scale per code to write, to read again and to keep.
+ *   words        packed codes of a cache buffer of `capacity` tokens, of which host_seg_end[nseg-1] are read
+ *   tokens_first 1: words [B, capacity, H, W], out [B, tokens, H, c]; 0: heads before tokens in both
+ *   scale, zp    fp32 [nseg, H, c] (zp NULL = symmetric)
+ * Requires c % 8 == 0, rows of whole words, nseg in 1..16.
+ */
+int varq_dequant_steps(const int32_t *words, const float *scale, const float *zp, int nseg, const int32_t *host_seg_end,
+                       int B, int H, int64_t capacity, int c, int bits, int tokens_first, void *out, int out_dtype, void *stream);
+
+/*
  * Fused dequant flash-attention (no counterpart in the reference, which
  * dequantizes the whole cache to fp32 and calls an external attention backend:
  * VAR_Q/quant.py:216-230, VAR/models/basic_var.py:156-162,

@@ -30,6 +30,8 @@ SYMBOLS = {
     'varq_unpack': (c_int, [c_void_p, c_int64, c_int, c_int, c_void_p, c_void_p]),
     'varq_dequant': (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, POINTER(c_int64), POINTER(c_int64),
                              c_int, c_int, POINTER(c_int64), c_void_p, c_int, c_void_p]),
+    'varq_dequant_steps': (c_int, [c_void_p, c_void_p, c_void_p, c_int, POINTER(c_int32), c_int, c_int, c_int64, c_int, c_int, c_int,
+                                   c_void_p, c_int, c_void_p]),
     'varq_fused_attn': (c_int, [c_void_p, c_void_p,
                                 c_void_p, c_void_p, c_void_p, c_int, c_int,
                                 c_void_p, c_void_p, c_void_p, c_int, c_int,

@@ -282,6 +282,25 @@ PyObject *dequant(PyObject *const *a) {
   return wrap(out);
 }
 
+// dequant_steps(buf, seg_ends, tab, ztab | None, c, bits, out dtype code, token_dim) -> the tokens cached so far
+PyObject *dequant_steps(PyObject *const *a) {
+  const at::Tensor &buf = gpu(a[0], "buffer"), &tab = gpu(a[2], "scale table");
+  const at::Tensor *ztab = maybe(a[3], "zero-point table");
+  const int64_t c = integer(a[4]), bits = integer(a[5]), code = integer(a[6]), d = integer(a[7]);
+  int32_t ends[16];
+  ASSERT(PyList_Check(a[1]) && PyList_GET_SIZE(a[1]) >= 1 && PyList_GET_SIZE(a[1]) <= 16, "dequant_steps: 1..16 segments");
+  const int nseg = (int)PyList_GET_SIZE(a[1]);
+  for (int i = 0; i < nseg; ++i) ends[i] = (int32_t)integer(PyList_GET_ITEM(a[1], i));
+  ASSERT(buf.dim() == 4 && buf.is_contiguous() && buf.scalar_type() == at::kInt && buf.size(3) * 32 == c * bits && (d == 1 || d == 2), "dequant_steps: buffer");
+  const int64_t B = buf.size(0), H = buf.size(3 - d);
+  ASSERT(tab.is_contiguous() && tab.scalar_type() == at::kFloat && tab.numel() >= nseg * H * c && (!ztab || ztab->sizes() == tab.sizes()), "dequant_steps: tables");
+  const c10::DeviceGuard guard(buf.device());
+  const at::Tensor out = d == 1 ? empty({B, ends[nseg - 1], H, c}, dtype_of((int)code), buf) : empty({B, H, ends[nseg - 1], c}, dtype_of((int)code), buf);
+  check(varq_dequant_steps(ptr<int32_t>(buf), ptr<float>(tab), ptr<float>(ztab), nseg, ends, (int)B, (int)H, buf.size(d), (int)c, (int)bits, d == 1,
+                           out.data_ptr(), (int)code, stream_of(buf)), "varq_dequant_steps");
+  return wrap(out);
+}
+
 // ---- attention ----------------------------------------------------------------------------------
 struct AttnShape {
   int64_t B, Hq, Lq, D, Hkv, Lstride;
@@ -521,7 +540,7 @@ PyObject *set_error(PyObject *, PyObject *e) {
 
 #define FIXED(name, n) {#name, (PyCFunction)(void (*)(void))fixed<name, n>, METH_FASTCALL, nullptr}
 PyMethodDef g_methods[] = {
-    FIXED(quant_rows, 5), FIXED(quant_shared, 6), FIXED(pack, 2), FIXED(unpack, 3), FIXED(dequant, 6), FIXED(attn, 18), FIXED(attn_channel, 17),
+    FIXED(quant_rows, 5), FIXED(quant_shared, 6), FIXED(pack, 2), FIXED(unpack, 3), FIXED(dequant, 6), FIXED(dequant_steps, 8), FIXED(attn, 18), FIXED(attn_channel, 17),
     FIXED(cache_append, 5), FIXED(cache_prepare, 9),
     {"quant_step", (PyCFunction)(void (*)(void))varying<quant_step>, METH_FASTCALL, nullptr},
     {"set_error", set_error, METH_O, nullptr},

@@ -7,7 +7,8 @@ changes underneath:
 
 * scale + codes + packing is one kernel chain (ops.quant_pack /
   ops.quant_pack_rows) instead of ~15 torch launches with fp32 temporaries;
-* unpack + dequant is one kernel;
+* unpack + dequant is one kernel, which takes the scales of a stepwise cache from one table per
+  step instead of reading them expanded over the tokens;
 * the cache lives in pre-allocated buffers that grow geometrically; a step is
   written in place instead of re-copying the whole cache with torch.cat
   (VAR_Q/quant.py:200-201).  `cached_item` / `cached_scale` are views of the
@@ -459,8 +460,16 @@ class VAR_Q:
         """The whole cache dequantized (VAR_Q/quant.py:216-224: fp32).  out_dtype bfloat16 / float16
         gives the fp32 product rounded once to that type -- bit for bit what `.to(out_dtype)` of the
         fp32 result is, without writing and re-reading the fp32 tensor."""
-        if self._c_item.len == 0:
+        item, ends = self._c_item, self._seg_ends
+        if item.len == 0:
             return self.dequant_current(out_dtype)
+        if self.pack_to_int32 and ends and len(ends) <= MAX_TABLE_STEPS and ends[-1] == item.len and item.dim == self.dim_cat:
+            c = self._pack_meta['orig_c']
+            if c % 8 == 0 and (c * self.quant_bits) % 32 == 0 and self._tab_scale.shape[2] == c:
+                # one scale table per step (the methods of _TABLE_METHODS): the expanded scales of
+                # cached_scale are neither made nor read
+                return _lib.host().dequant_steps(item.buf, ends, self._tab_scale, self._tab_zp, c, self.quant_bits,
+                                                 ops._DT[out_dtype], self.dim_cat)
         return self._dequant(self.cached_item, self.cached_scale, self.cached_zp, out_dtype)
 
     def use_var_q(self, item: torch.Tensor, out_dtype: Optional[torch.dtype] = None) -> torch.Tensor:
