@@ -1,0 +1,46 @@
+"""The quantizer's one-launch kernel at the edges of its plans: one row per group, row counts around a
+workgroup's row lanes and its 16 (fp32: 8) register steps, the row count from which the three launches
+take over, column slices with a remainder (an octet count that is no power of two), kept inner indices
+that do not fill the last tile.  Bit-exact against the CPU oracle."""
+import pytest
+import torch
+
+import varq_oracle as O
+from gpu_util import note
+from var_q_amd import ops
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize('shape,dims,dtype', [
+    ((3, 1, 5, 64), (1,), torch.bfloat16),            # every row its own group, channel by channel
+    ((2, 16, 1, 128), (0, 2), torch.float16),         # two rows per group
+    ((2, 1, 33, 16), (2,), torch.bfloat16),           # one octet pair, 33 rows
+    ((1, 3, 511, 8), (2,), torch.float32),            # one octet
+    ((1, 3, 513, 72), (2,), torch.bfloat16),          # nine octets: a slice with one live lane
+    ((2, 4, 1025, 128), (0, 2), torch.bfloat16),
+    ((64, 3, 16, 64), (0, 1), torch.float16),         # strided rows, inner index kept
+    ((64, 33, 3, 48), (0, 1), torch.float32),
+    ((1, 4096, 2, 64), (0, 1), torch.bfloat16),
+    ((1, 8192, 2, 32), (0, 1), torch.float16),        # the most rows of a group
+    ((1, 8193, 2, 32), (0, 1), torch.float16),        # one row more
+    ((1, 4, 2047, 512), (2,), torch.float32),
+    ((7, 5, 3, 64), (0, 3), torch.bfloat16),          # channel dim reduced: one scale per kept index
+    ((2, 40, 65, 80), (0, 1, 3), torch.float32),
+    ((2, 3, 129, 520), (0, 2), torch.bfloat16),       # 65 octets: past the column lanes
+])
+def test_one_launch_edges(dev, shape, dims, dtype):
+    g = torch.Generator().manual_seed(sum(shape))
+    x = (torch.randn(*shape, generator=g) * 2).to(dtype)
+    x[..., 3] *= 15
+    x[0, 0, 0] = 0
+    for bits, asym, pack in ((8, False, True), (4, True, True), (2, True, True), (5, False, False)):
+        if pack and (shape[-1] * bits) % 32:
+            continue
+        note('quant one', shape, dims, dtype, bits, asym, pack)
+        q, s, z = O.quant_reduce(x, dims, bits, asym)
+        gq, gs, gz = ops.quant_pack(x.to(dev), dims, bits, asym=asym, pack=pack)
+        torch.cuda.synchronize()
+        assert torch.equal(gs.cpu(), s)
+        assert not asym or torch.equal(gz.cpu(), z)
+        assert torch.equal(gq.cpu(), O.pack_last_dim(q, bits)[0] if pack else q)

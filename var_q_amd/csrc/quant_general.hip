@@ -307,7 +307,48 @@ __global__ __launch_bounds__(256) void finalize_tiled_kernel(GenParams p, int Z,
   plain[g] = (s > 0x1p-96f && s < 0x1p96f && (f2u(s) & 0x7fffffu) != 0x7fffffu) ? 1u : 0u;
 }
 
-template <int DT, bool KEEPC>
+// Quantizes and stores one octet (column `col`) of row `row`: s, r, z the scale, RN(1 / scale) and the
+// zero-point of the octet's groups (one per channel or one), plain whether all scales allow the exact
+// quotient shortcut.
+template <int NV>
+__device__ __forceinline__ void store_octet(const GenParams &p, int64_t row, int col, const float (&v)[8], const float (&s)[NV], const float (&r)[NV],
+                                            const float (&z)[NV], bool plain) {
+  const float qmin = (float)p.qmin, qmax = (float)p.qmax;
+  const u32 mask = (1u << p.bits) - 1u;
+  int q[8];
+  if (plain) {
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const float sj = s[j % NV], rj = r[j % NV];
+      const float q0 = v[j] * rj;
+      const float t = __builtin_fmaf(__builtin_fmaf(-q0, sj, v[j]), rj, q0);
+      q[j] = (int)__builtin_amdgcn_fmed3f(rintf(t) + z[j % NV], qmin, qmax);
+    }
+  } else {
+#pragma unroll
+    for (int j = 0; j < 8; ++j) q[j] = (int)__builtin_amdgcn_fmed3f(rintf(v[j] / s[j % NV]) + z[j % NV], qmin, qmax);
+  }
+  const int64_t orow = out_row32(p, row);
+  if (p.codes || p.bits == 8) {
+    const u32 lo = (q[0] & 0xff) | ((q[1] & 0xff) << 8) | ((q[2] & 0xff) << 16) | ((u32)q[3] << 24);
+    const u32 hi = (q[4] & 0xff) | ((q[5] & 0xff) << 8) | ((q[6] & 0xff) << 16) | ((u32)q[7] << 24);
+    if (p.codes) *reinterpret_cast<uint2 *>(p.codes + (orow * p.c8 + col) * 8) = make_uint2(lo, hi);
+    if (p.words && p.bits == 8) *reinterpret_cast<uint2 *>(p.words + orow * p.wpr + col * 2) = make_uint2(lo, hi);
+  }
+  if (p.words && p.bits != 8) {
+    u32 w = 0;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) w |= ((u32)q[j] & mask) << (j * p.bits);
+    if (p.bits == 4) {
+      p.words[orow * p.wpr + col] = (int32_t)w;
+    } else {  // 2 bits: 16 codes per word = two adjacent octets (c % 16 == 0 on this path)
+      const u32 other = __shfl_xor(w, 1, 64);
+      if ((col & 1) == 0) p.words[orow * p.wpr + (col >> 1)] = (int32_t)(w | (other << 16));
+    }
+  }
+}
+
+template <int DT, bool ASYM, bool KEEPC>
 __global__ __launch_bounds__(256) void quant_tiled_kernel(GenParams p, Plan pl, const float *rinv, const u32 *plain) {
   constexpr int NV = KEEPC ? 8 : 1;
   if (take_second(p)) { rinv += p.ws1; plain += p.ws1; }
@@ -315,7 +356,7 @@ __global__ __launch_bounds__(256) void quant_tiled_kernel(GenParams p, Plan pl, 
   // 2-bit words are assembled from two adjacent column lanes: idle lanes must still reach the shuffle
   const bool live = l.live;
   const int64_t g = (int64_t)l.ko * pl.ko_gs + (int64_t)(live ? l.q : 0) * pl.q_gs + (KEEPC ? (live ? l.col : 0) * 8 : 0);
-  float s[NV], r[NV], z[NV];
+  float s[NV], r[NV], z[NV] = {};
   bool all_plain = true;
   if constexpr (KEEPC) {
     // the lane's eight groups are adjacent and start at a multiple of 8: 16-byte loads (the
@@ -326,61 +367,147 @@ __global__ __launch_bounds__(256) void quant_tiled_kernel(GenParams p, Plan pl, 
     };
     ld8(p.scale, s);
     ld8(rinv, r);
-    if (p.asym) ld8(p.zp, z);
-    else {
-#pragma unroll
-      for (int j = 0; j < NV; ++j) z[j] = 0.f;
-    }
+    if constexpr (ASYM) ld8(p.zp, z);
     const uint4 pa = reinterpret_cast<const uint4 *>(plain + g)[0], pb = reinterpret_cast<const uint4 *>(plain + g)[1];
     all_plain = (pa.x & pa.y & pa.z & pa.w & pb.x & pb.y & pb.z & pb.w) != 0u;
   } else {
     s[0] = p.scale[g];
     r[0] = rinv[g];
-    z[0] = p.asym ? p.zp[g] : 0.f;
+    if (ASYM) z[0] = p.zp[g];
     all_plain = plain[g] != 0u;
   }
-  const float qmin = (float)p.qmin, qmax = (float)p.qmax;
-  const u32 mask = (1u << p.bits) - 1u;
   if (!live) return;   // (only the 2-bit path shuffles, and there c8 is even: partners are live together)
-  for_rows<DT>(p, pl, l, [&](int64_t row, const float (&v)[8]) {
-    int q[8];
-    if (all_plain) {
+  for_rows<DT>(p, pl, l, [&](int64_t row, const float (&v)[8]) { store_octet<NV>(p, row, l.col, v, s, r, z, all_plain); });
+}
+
+// ---- one launch: a workgroup holds all rows of its groups -----------------------------------------
+// Where the rows of a group fit the registers of a workgroup (16 rows of an octet per thread, 8 in fp32) the
+// three launches become one, and the input is read once: load, fold, derive the parameters, quantize what
+// the registers hold.  The steps of a schedule are bound by the number of their launches and by latency, not
+// by bytes.  K and V of a step, 8-bit, one scale per channel and head, fp16 [64,n,16,64] / bf16 [2,16,n,128],
+// three launches -> one: n = 1 12.7 -> 4.4 us / 9.9 -> 4.7, n = 16 11.8 -> 8.6 / 9.9 -> 4.6, n = 64 22.7 ->
+// 14.7, n = 400 14.3 -> 9.9, n = 1024 22.6 -> 16.5.
+// A workgroup owns, for one ko, 2^lq_shift kept inner indices x c8s column lanes; thread
+// ((lq * sub + f) * c8s + col) takes the reduced rows f, f + sub, ... of its q.  With the channel dim kept
+// the columns are cut into slices of c8s octets, one workgroup each, until there are workgroups enough: the
+// steps of one batch have few groups, and narrow slices (64, 32, then 16 bytes of a row, whose cache lines
+// the slices of one XCD share) still read faster than few workgroups do.
+struct OnePlan {
+  int64_t ko_rs, ro_rs, ko_gs, q_gs;
+  int nko, Q, RR, RI;           // kept outer, kept inner; reduced rows, of which RI are contiguous
+  int c8s_shift, sub_shift, lq_shift;
+  int slices, tilesQ, steps;
+  int blocks;                   // nko * tilesQ
+};
+
+template <int DT, bool ASYM, bool KEEPC, int NT, int NI>
+__global__ __launch_bounds__(NT) void quant_one_kernel(GenParams p, OnePlan pl) {
+  constexpr int NV = KEEPC ? 8 : 1, MAXG = 2048;
+  __shared__ float lds_mx[MAXG];
+  __shared__ float lds_mn[ASYM ? MAXG : 1];
+  __shared__ float par_s[MAXG], par_r[MAXG];
+  __shared__ float par_z[ASYM ? MAXG : 1];
+  take_second(p);
+  // the slices of a block on one XCD (ids congruent mod 8 share an L2): they share the rows' cache lines
+  const int bid = blockIdx.x, slice = (bid >> 3) % pl.slices, blk = (bid >> 3) / pl.slices * 8 + (bid & 7);
+  if (blk >= pl.blocks) return;
+  const int tq = blk % pl.tilesQ, ko = blk / pl.tilesQ;
+  const int tid = threadIdx.x, c8s = 1 << pl.c8s_shift, sub = 1 << pl.sub_shift;
+  const int lcol = tid & (c8s - 1), col = slice * c8s + lcol, f = (tid >> pl.c8s_shift) & (sub - 1), lq = tid >> (pl.c8s_shift + pl.sub_shift);
+  const int q = (tq << pl.lq_shift) + lq;
+  const bool live = col < p.c8 && q < pl.Q && lq < (1 << pl.lq_shift);
+  const int64_t row0 = (int64_t)ko * pl.ko_rs + (live ? q : 0);
+  auto row_of = [&](int j) { return pl.RI == 1 ? row0 + j * pl.ro_rs : row0 + (j / pl.RI) * pl.ro_rs + j % pl.RI; };
+
+  Raw8<DT> raw[NI];
 #pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        const float sj = s[j % NV], rj = r[j % NV];
-        const float q0 = v[j] * rj;
-        const float t = __builtin_fmaf(__builtin_fmaf(-q0, sj, v[j]), rj, q0);
-        q[j] = (int)__builtin_amdgcn_fmed3f(rintf(t) + z[j % NV], qmin, qmax);
-      }
+  for (int s = 0; s < NI; ++s) {
+    const int j = (s << pl.sub_shift) + f;
+    if (s < pl.steps && live && j < pl.RR)
+      raw[s] = *reinterpret_cast<const Raw8<DT> *>(reinterpret_cast<const char *>(p.x) + (row_of(j) * p.c + col * 8) * In8<DT>::kBytes);
+  }
+  float mx[NV], mn[NV];
+#pragma unroll
+  for (int j = 0; j < NV; ++j) { mx[j] = ASYM ? -INFINITY : 0.f; mn[j] = INFINITY; }
+#pragma unroll
+  for (int s = 0; s < NI; ++s) {
+    if (s >= pl.steps || !live || (s << pl.sub_shift) + f >= pl.RR) continue;
+    float v[8];
+    raw[s].widen(v);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      if (ASYM) { mx[j % NV] = fmaxf(mx[j % NV], v[j]); mn[j % NV] = fminf(mn[j % NV], v[j]); }
+      else mx[j % NV] = fmaxf(mx[j % NV], fabsf(v[j]));
+    }
+  }
+  // fold over f (and, with the channel dim reduced, over the columns), inside the wavefront first;
+  // what is left is one value per wavefront and column, or per q where a q has less than a wavefront
+  const int q_lanes = sub << pl.c8s_shift;         // threads of a q
+  for (int off = KEEPC ? c8s : 1; off < 64 && off < q_lanes; off <<= 1) {
+#pragma unroll
+    for (int j = 0; j < NV; ++j) {
+      mx[j] = fmaxf(mx[j], __shfl_xor(mx[j], off, 64));
+      if (ASYM) mn[j] = fminf(mn[j], __shfl_xor(mn[j], off, 64));
+    }
+  }
+  const int gcols = KEEPC ? c8s * 8 : 1;           // groups of a q in this workgroup
+  const int parts = q_lanes > 64 ? q_lanes >> 6 : 1, lane_in_part = q_lanes > 64 ? tid & 63 : tid & (q_lanes - 1);
+  const int part = q_lanes > 64 ? tid >> 6 : tid / q_lanes;      // = lq * parts + wavefront of the q
+  if (lane_in_part < (KEEPC ? c8s : 1)) {
+#pragma unroll
+    for (int j = 0; j < NV; ++j) {
+      lds_mx[part * gcols + lcol * NV + j] = mx[j];
+      if (ASYM) lds_mn[part * gcols + lcol * NV + j] = mn[j];
+    }
+  }
+  __syncthreads();
+  // one thread per group
+  const int n_par = gcols << pl.lq_shift;
+  for (int t = tid; t < n_par; t += NT) {
+    const int tl = t / gcols, g8 = t - tl * gcols, tqi = (tq << pl.lq_shift) + tl;
+    float m = ASYM ? -INFINITY : 0.f, n = INFINITY;
+    for (int w = 0; w < parts; ++w) {
+      m = fmaxf(m, lds_mx[(tl * parts + w) * gcols + g8]);
+      if (ASYM) n = fminf(n, lds_mn[(tl * parts + w) * gcols + g8]);
+    }
+    const bool mine = tqi < pl.Q && (!KEEPC || slice * c8s * 8 + g8 < p.c);
+    float s, zp = 0.f;
+    if (ASYM) {
+      s = fmaxf((m - n) / (float)((1 << p.bits) - 1), p.eps);
+      zp = (float)p.qmin - rintf(n / s);
+      par_z[t] = zp;
     } else {
+      s = fmaxf(m / (float)p.qmax, p.eps);
+    }
+    par_s[t] = s;
+    // (the exact-quotient shortcut, see finalize_tiled_kernel; 0: this group takes the division)
+    par_r[t] = (s > 0x1p-96f && s < 0x1p96f && (f2u(s) & 0x7fffffu) != 0x7fffffu) ? 1.0f / s : 0.f;
+    if (mine) {
+      const int64_t g = (int64_t)ko * pl.ko_gs + (int64_t)tqi * pl.q_gs + (KEEPC ? slice * c8s * 8 + g8 : 0);
+      p.scale[g] = s;
+      if (ASYM) p.zp[g] = zp;
+    }
+  }
+  __syncthreads();
+  if (!live) return;   // (2-bit words take two adjacent columns, which are live together: c is a multiple of 16 there)
+  const int t0 = lq * gcols + lcol * (KEEPC ? 8 : 0);
+  float s[NV], r[NV], z[NV] = {};
+  bool plain = true;
 #pragma unroll
-      for (int j = 0; j < 8; ++j) q[j] = (int)__builtin_amdgcn_fmed3f(rintf(v[j] / s[j % NV]) + z[j % NV], qmin, qmax);
-    }
-    const int64_t orow = out_row32(p, row);
-    const int64_t o = orow * p.c8 + l.col;
-    if (p.codes) {
-      u32 lo = (q[0] & 0xff) | ((q[1] & 0xff) << 8) | ((q[2] & 0xff) << 16) | ((u32)q[3] << 24);
-      u32 hi = (q[4] & 0xff) | ((q[5] & 0xff) << 8) | ((q[6] & 0xff) << 16) | ((u32)q[7] << 24);
-      *reinterpret_cast<uint2 *>(p.codes + o * 8) = make_uint2(lo, hi);
-    }
-    if (p.words) {
-      if (p.bits == 8) {
-        u32 lo = (q[0] & 0xff) | ((q[1] & 0xff) << 8) | ((q[2] & 0xff) << 16) | ((u32)q[3] << 24);
-        u32 hi = (q[4] & 0xff) | ((q[5] & 0xff) << 8) | ((q[6] & 0xff) << 16) | ((u32)q[7] << 24);
-        *reinterpret_cast<uint2 *>(p.words + orow * p.wpr + l.col * 2) = make_uint2(lo, hi);
-      } else {
-        u32 w = 0;
+  for (int j = 0; j < NV; ++j) {
+    s[j] = par_s[t0 + j];
+    r[j] = par_r[t0 + j];
+    if (ASYM) z[j] = par_z[t0 + j];
+    plain = plain && r[j] != 0.f;
+  }
 #pragma unroll
-        for (int j = 0; j < 8; ++j) w |= ((u32)q[j] & mask) << (j * p.bits);
-        if (p.bits == 4) {
-          p.words[orow * p.wpr + l.col] = (int32_t)w;
-        } else {  // 2 bits: 16 codes per word = two adjacent octets (c % 16 == 0 on this path)
-          u32 other = __shfl_xor(w, 1, 64);
-          if ((l.col & 1) == 0) p.words[orow * p.wpr + (l.col >> 1)] = (int32_t)(w | (other << 16));
-        }
-      }
-    }
-  });
+  for (int i = 0; i < NI; ++i) {
+    const int j = (i << pl.sub_shift) + f;
+    if (i >= pl.steps || j >= pl.RR) continue;
+    float v[8];
+    raw[i].widen(v);
+    store_octet<NV>(p, row_of(j), col, v, s, r, z, plain);
+  }
 }
 
 // ---- phase A, any c: one thread per element --------------------------------
@@ -449,41 +576,49 @@ __global__ void quant_scalar_kernel(GenParams p) {
   if (p.words) p.words[out_row(p, r) * wpr + wi] = (int32_t)w;
 }
 
-// Host side of the tiled path: canonical form of the leading dims and the launch shape.
-// Returns false when the shape needs the scalar kernels.
+// The leading dims in canonical form (see Plan).
+struct Canonical { int64_t nko, nro, Q, RI, ko_rs, ro_rs, ko_gs, q_gs; };
+Canonical canonical(const int64_t *sh, int reduce_mask) {
+  const int64_t n0 = sh[0], n1 = sh[1], n2 = sh[2], c = sh[3], rows = n0 * n1 * n2;
+  const bool k0 = !(reduce_mask & 1), k1 = !(reduce_mask & 2), k2 = !(reduce_mask & 4), kc = !(reduce_mask & 8);
+  int64_t stride = kc ? c : 1;
+  const int64_t gs2 = k2 ? stride : 0; if (k2) stride *= n2;
+  const int64_t gs1 = k1 ? stride : 0; if (k1) stride *= n1;
+  const int64_t gs0 = k0 ? stride : 0;
+  Canonical k = {1, 1, 1, 1, 0, 0, 0, 0};
+  if (k2) {
+    k.Q = n2; k.q_gs = gs2;
+    if (k1) {
+      k.Q = n1 * n2;                                   // gs1 == gs2 * n2: q runs over (i1, i2)
+      if (k0) k.Q = rows;                              // every row its own group
+      else { k.nro = n0; k.ro_rs = n1 * n2; }
+    } else if (k0) { k.nko = n0; k.ko_rs = n1 * n2; k.ko_gs = gs0; k.nro = n1; k.ro_rs = n2; }
+    else { k.nro = n0 * n1; k.ro_rs = n2; }
+  } else {
+    k.RI = n2;
+    if (!k1) {
+      k.RI = n1 * n2;
+      if (!k0) k.RI = rows;
+      else { k.nko = n0; k.ko_rs = n1 * n2; k.ko_gs = gs0; }
+    } else if (k0) { k.nko = n0 * n1; k.ko_rs = n2; k.ko_gs = gs1; }     // gs0 == gs1 * n1
+    else { k.nko = n1; k.ko_rs = n2; k.ko_gs = gs1; k.nro = n0; k.ro_rs = n1 * n2; }
+  }
+  return k;
+}
+
+// Host side of the tiled path: the launch shape.  Returns false when the shape needs the scalar kernels.
 bool make_plan(const int64_t *sh, int reduce_mask, int64_t n_groups, Plan &pl) {
-  const int64_t n0 = sh[0], n1 = sh[1], n2 = sh[2], c = sh[3];
-  const int64_t rows = n0 * n1 * n2;
+  const int64_t c = sh[3];
+  const int64_t rows = sh[0] * sh[1] * sh[2];
   if (c % 8 != 0 || rows <= 0 || rows >= (1ll << 31) - 512) return false;
   pl.c8 = (int)(c / 8);
   int c8p = 1, shl = 0;
   while (c8p < pl.c8) { c8p <<= 1; ++shl; }
   if (c8p > 64) return false;
   pl.c8p = c8p; pl.shift = shl; pl.R = 256 / c8p;
-  const bool k0 = !(reduce_mask & 1), k1 = !(reduce_mask & 2), k2 = !(reduce_mask & 4), kc = !(reduce_mask & 8);
-  int64_t stride = kc ? c : 1;
-  const int64_t gs2 = k2 ? stride : 0; if (k2) stride *= n2;
-  const int64_t gs1 = k1 ? stride : 0; if (k1) stride *= n1;
-  const int64_t gs0 = k0 ? stride : 0;
-  int64_t nko = 1, nro = 1, Q = 1, RI = 1;
-  pl.ko_rs = pl.ro_rs = pl.ko_gs = pl.q_gs = 0;
-  if (k2) {
-    Q = n2; pl.q_gs = gs2;
-    if (k1) {
-      Q = n1 * n2;                                   // gs1 == gs2 * n2: q runs over (i1, i2)
-      if (k0) Q = rows;                              // every row its own group
-      else { nro = n0; pl.ro_rs = n1 * n2; }
-    } else if (k0) { nko = n0; pl.ko_rs = n1 * n2; pl.ko_gs = gs0; nro = n1; pl.ro_rs = n2; }
-    else { nro = n0 * n1; pl.ro_rs = n2; }
-  } else {
-    RI = n2;
-    if (!k1) {
-      RI = n1 * n2;
-      if (!k0) RI = rows;
-      else { nko = n0; pl.ko_rs = n1 * n2; pl.ko_gs = gs0; }
-    } else if (k0) { nko = n0 * n1; pl.ko_rs = n2; pl.ko_gs = gs1; }     // gs0 == gs1 * n1
-    else { nko = n1; pl.ko_rs = n2; pl.ko_gs = gs1; nro = n0; pl.ro_rs = n1 * n2; }
-  }
+  const Canonical k = canonical(sh, reduce_mask);
+  const int64_t nko = k.nko, nro = k.nro, Q = k.Q, RI = k.RI;
+  pl.ko_rs = k.ko_rs; pl.ro_rs = k.ro_rs; pl.ko_gs = k.ko_gs; pl.q_gs = k.q_gs;
   pl.nko = (int)nko; pl.nro = (int)nro; pl.Q = (int)Q; pl.RI = (int)RI;
   pl.lanesQ = (int)(Q < pl.R ? Q : pl.R);
   if (RI == 1 && nro >= VARQ_GEN_NRO_MIN) {
@@ -519,6 +654,58 @@ bool make_plan(const int64_t *sh, int reduce_mask, int64_t n_groups, Plan &pl) {
   return true;
 }
 
+// The one-launch plan, or false when a group has too many rows for a workgroup's registers.
+bool make_one_plan(const int64_t *sh, int reduce_mask, int row_steps, int tensors, OnePlan &pl, int &threads) {
+  const int64_t c = sh[3], rows = sh[0] * sh[1] * sh[2];
+  if (c % 8 != 0 || c > 512 || rows <= 0 || rows >= (1ll << 31) - 512) return false;
+  const Canonical k = canonical(sh, reduce_mask);
+  const int64_t rr = k.nro * k.RI;
+  // above 16 MiB the three launches, with 2048 workgroups on either side of the fold, are the faster way
+  // through memory ([32,30,680,64], one scale per (token, head): 38 against 55 us)
+  if (rr > 8192 || rows * c * (row_steps == 8 ? 4 : 2) * tensors > (16ll << 20)) return false;
+  const bool keepc = !(reduce_mask & 8);
+  const int c8 = (int)(c / 8);
+  int c8p_shift = 0;
+  while ((1 << c8p_shift) < c8) ++c8p_shift;
+  pl.ko_rs = k.ko_rs; pl.ro_rs = k.ro_rs; pl.ko_gs = k.ko_gs; pl.q_gs = k.q_gs;
+  pl.nko = (int)k.nko; pl.Q = (int)k.Q; pl.RR = (int)rr; pl.RI = (int)k.RI;
+  int rr_shift = 0;
+  while ((1 << rr_shift) < rr) ++rr_shift;
+  // column slices (channel dim kept): whole rows while that makes workgroups enough, 64 bytes of a row at least
+  pl.c8s_shift = keepc && c8p_shift > 4 ? 4 : c8p_shift;
+  for (;; --pl.c8s_shift) {
+    pl.slices = keepc ? (c8 + (1 << pl.c8s_shift) - 1) >> pl.c8s_shift : 1;
+    // 256 threads where their rows suffice, 1024 otherwise; the row lanes of a q no more than its rows
+    for (threads = 256; ; threads = 1024) {
+      const int shift = (threads == 256 ? 8 : 10) - pl.c8s_shift;
+      pl.sub_shift = rr_shift < shift ? rr_shift : shift;
+      // (few rows: a step or two more per thread and fewer lanes per q would only make fewer workgroups)
+      pl.lq_shift = shift - pl.sub_shift;
+      while (pl.lq_shift > 0 && (1ll << (pl.lq_shift - 1)) >= k.Q) --pl.lq_shift;
+      pl.steps = (int)((rr + (1 << pl.sub_shift) - 1) >> pl.sub_shift);
+      if (pl.steps <= 4 || threads == 1024) break;
+    }
+    pl.tilesQ = (int)((k.Q + (1 << pl.lq_shift) - 1) >> pl.lq_shift);
+    pl.blocks = pl.nko * pl.tilesQ;
+    const bool fits = pl.steps <= row_steps;
+    if (fits && ((int64_t)pl.blocks * pl.slices * tensors >= 128 || !keepc || pl.c8s_shift <= 1)) return true;
+    if (!keepc || pl.c8s_shift <= 1) return false;
+  }
+}
+
+template <int DT, bool ASYM, bool KEEPC>
+void launch_one(const GenParams &p, const OnePlan &pl, int threads, hipStream_t st) {
+  constexpr int NI = DT == VARQ_F32 ? 8 : 16;
+  dim3 grid((unsigned)((pl.blocks + 7) / 8 * 8 * pl.slices), p.x1 ? 2u : 1u);
+  if (threads == 1024) hipLaunchKernelGGL((quant_one_kernel<DT, ASYM, KEEPC, 1024, NI>), grid, dim3(1024), 0, st, p, pl);
+  else if (pl.steps <= 2) hipLaunchKernelGGL((quant_one_kernel<DT, ASYM, KEEPC, 256, 2>), grid, dim3(256), 0, st, p, pl);
+  else hipLaunchKernelGGL((quant_one_kernel<DT, ASYM, KEEPC, 256, NI>), grid, dim3(256), 0, st, p, pl);
+}
+template <int DT> void run_one(const GenParams &p, const OnePlan &pl, int threads, hipStream_t st) {
+  if (p.asym) { if (p.keepc) launch_one<DT, true, true>(p, pl, threads, st); else launch_one<DT, true, false>(p, pl, threads, st); }
+  else { if (p.keepc) launch_one<DT, false, true>(p, pl, threads, st); else launch_one<DT, false, false>(p, pl, threads, st); }
+}
+
 size_t plan_workspace_bytes(const Plan &pl, int64_t n_groups) {
   return (size_t)n_groups * (2 + 2 * (size_t)pl.Z) * sizeof(float);
 }
@@ -552,8 +739,13 @@ int run_tiled(GenParams &p, const Plan &pl, void *workspace, hipStream_t st) {
   // per thread measured alike, longer ones slower)
   const Plan &pb = pl;
   dim3 bgrid((unsigned)((int64_t)pb.nko * pb.tilesQ * pb.Z), nt);
-  if (p.keepc) hipLaunchKernelGGL((quant_tiled_kernel<DT, true>), bgrid, dim3(256), 0, st, p, pb, rinv, plain);
-  else hipLaunchKernelGGL((quant_tiled_kernel<DT, false>), bgrid, dim3(256), 0, st, p, pb, rinv, plain);
+  if (p.asym) {
+    if (p.keepc) hipLaunchKernelGGL((quant_tiled_kernel<DT, true, true>), bgrid, dim3(256), 0, st, p, pb, rinv, plain);
+    else hipLaunchKernelGGL((quant_tiled_kernel<DT, true, false>), bgrid, dim3(256), 0, st, p, pb, rinv, plain);
+  } else {
+    if (p.keepc) hipLaunchKernelGGL((quant_tiled_kernel<DT, false, true>), bgrid, dim3(256), 0, st, p, pb, rinv, plain);
+    else hipLaunchKernelGGL((quant_tiled_kernel<DT, false, false>), bgrid, dim3(256), 0, st, p, pb, rinv, plain);
+  }
   return 0;
 }
 
@@ -670,7 +862,14 @@ int quant_pack_impl(const void *x, const void *x1, int x_dtype, const int64_t *h
   p.asym = asym ? 1 : 0;
   p.eps = eps;
   hipStream_t st = (hipStream_t)stream;
-  if (tiled) {
+  OnePlan one;
+  int threads;
+  if (tiled && make_one_plan(s, reduce_mask, x_dtype == VARQ_F32 ? 8 : 16, x1 ? 2 : 1, one, threads)) {
+    if (x1) { p.x1 = x1; p.scale1 = scale1; p.zp1 = zp1; p.words1 = words1; p.codes1 = codes1; }
+    if (x_dtype == VARQ_F32) run_one<VARQ_F32>(p, one, threads, st);
+    else if (x_dtype == VARQ_BF16) run_one<VARQ_BF16>(p, one, threads, st);
+    else run_one<VARQ_F16>(p, one, threads, st);
+  } else if (tiled) {
     if (x1) { p.x1 = x1; p.scale1 = scale1; p.zp1 = zp1; p.words1 = words1; p.codes1 = codes1; }
     if (x_dtype == VARQ_F32) run_tiled<VARQ_F32>(p, pl, workspace, st);
     else if (x_dtype == VARQ_BF16) run_tiled<VARQ_BF16>(p, pl, workspace, st);
