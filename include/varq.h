@@ -109,6 +109,26 @@ int varq_quant_pack_rows2(const void *x0, const void *x1, int x_dtype, int64_t n
                           float *zp1, void *stream);
 
 /*
+ * A cache whose heads have several bit-widths keeps the heads of a width together, as a "class" with
+ * dense buffers of its own.  The calls that take an array of classes (of distinct widths, together
+ * the H heads of the cache) serve all of them in one launch; each has the results of one call per class
+ * of its single-width counterpart (no counterpart in the reference).
+ */
+typedef struct varq_kv_class {
+  int bits, heads;                 /* width of the codes; heads of the class */
+  const int32_t *head_map;         /* device [heads]: the head that packed head s serves */
+  const int32_t *slot;             /* device [H]: packed head of a head, -1: of another class */
+  int32_t *k_words, *v_words;      /* [B, heads, Lk_stride, D*bits/32] */
+  float *k_scale, *k_zp, *v_scale, *v_zp;   /* [B, heads, Lk_stride, D/group]; zp NULL: symmetric */
+} varq_kv_class;
+/* K and V [B, H, n, c] (VARQ_LAYOUT_BHLC) or [B, n, H, c] (VARQ_LAYOUT_BLHC) into tokens start .. start+n of a
+ * cache of Lk_stride = Lmax tokens; either input may be NULL (K and V of different dtypes: one
+ * call each).  group must be 32, 64 or 128: VARQ_ERR_UNSUPPORTED otherwise. */
+int varq_quant_pack_classes(const void *k, const void *v, int x_dtype, int layout, int B, int H, int64_t n, int c, int group,
+                            int asym, float eps, const varq_kv_class *host_classes, int n_classes, int64_t Lmax, int64_t start,
+                            void *stream);
+
+/*
  * General quantizer for the six grouping methods of VAR_Q/quant.py:75-95 and
  * any other reduce set: a group is every element sharing the indices of the
  * dims NOT in reduce_mask (bit d set = dim d reduced).  Two phases: group
@@ -263,7 +283,7 @@ int varq_dequant_steps(const int32_t *words, const float *scale, const float *zp
  */
 size_t varq_fused_attn_workspace_bytes(int B, int Hkv, int Lq, int Lk, int D, int nseg, int splits);
 /* Many queries over a long cache (five or more blocks of 256 per (batch, head)): given a workspace of
- * this many bytes and splits = 0, both attention entry points dequantize K and V once into matrix
+ * this many bytes and splits = 0 or 1, the attention entry points dequantize K and V once into matrix
  * operands kept there and stream those, instead of dequantizing every key tile again for each block of
  * queries.  Same operands, same result to rounding.  0: not worth it for this shape.  (A caller that
  * leaves the choice to the library passes a workspace of the larger of the two sizes.) */
@@ -279,6 +299,16 @@ int varq_fused_attn(const void *q, void *out,
                     int Lq, int Lk, int Lk_stride, int D,
                     const int32_t *kv_limit, float softmax_scale, int layout, int io_dtype, int operand_form,
                     void *workspace, size_t workspace_bytes, int splits, void *stream);
+
+/*
+ * The same attention over a mixed-width cache (see varq_kv_class), every class in one call and, below
+ * the sizes of varq_fused_attn_expand_bytes, in one launch.  Layouts VARQ_LAYOUT_BHLC and VARQ_LAYOUT_BHLC_OUT_BLHC, dequantized
+ * operands; workspace sizes as for varq_fused_attn with Hkv = H.
+ */
+int varq_fused_attn_classes(const void *q, void *out, const varq_kv_class *host_classes, int n_classes, int group,
+                            int B, int H, int Lq, int Lk, int Lk_stride, int D,
+                            const int32_t *kv_limit, float softmax_scale, int layout, int io_dtype,
+                            void *workspace, size_t workspace_bytes, int splits, void *stream);
 
 /*
  * The same attention over a cache quantized per (head, channel), the layout of the
@@ -336,6 +366,12 @@ int varq_qkv_prepare_append(const void *qkv, int x_dtype, int B, int L, int H, i
                             const int64_t *host_rowmap, const int32_t *slot,
                             int32_t *k_words, float *k_scale, float *k_zp,
                             int32_t *v_words, float *v_scale, float *v_zp, void *stream);
+/* The same for all classes of a mixed-width cache (see varq_kv_class), tokens start .. start+L of a cache of
+ * Lmax tokens; c 64 or 128, group >= 32 (VARQ_ERR_UNSUPPORTED otherwise). */
+int varq_qkv_prepare_classes(const void *qkv, int x_dtype, int B, int L, int H, int c, const float *q_scale_mul, int l2norm,
+                             float norm_eps, const float *rope_cos, const float *rope_sin, int token_start, void *q_out,
+                             int group, int asym, float eps, const varq_kv_class *host_classes, int n_classes, int64_t Lmax,
+                             int64_t start, void *stream);
 
 #ifdef __cplusplus
 }

@@ -17,6 +17,8 @@ SYMBOLS = {
     'varq_quant_pack_rows2': (c_int, [c_void_p, c_void_p, c_int, c_int64, c_int, c_int, c_int, c_int, c_float,
                                       POINTER(c_int64), c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p,
                                       c_void_p, c_void_p]),
+    'varq_quant_pack_classes': (c_int, [c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int64, c_int, c_int, c_int, c_float,
+                                        c_void_p, c_int, c_int64, c_int64, c_void_p]),
     'varq_quant_workspace_bytes': (c_size_t, [POINTER(c_int64), c_int]),
     'varq_quant_pack': (c_int, [c_void_p, c_int, POINTER(c_int64), c_int, c_int, c_int, c_float,
                                 c_void_p, c_void_p, c_void_p, c_void_p, POINTER(c_int64), c_void_p, c_size_t, c_void_p]),
@@ -41,6 +43,9 @@ SYMBOLS = {
     'varq_fused_attn_workspace_bytes': (c_size_t, [c_int, c_int, c_int, c_int, c_int, c_int, c_int]),
     'varq_fused_attn_expand_bytes': (c_size_t, [c_int, c_int, c_int, c_int, c_int]),
     'varq_fused_attn_key_shares': (c_int, [c_int, c_int, c_int, c_int, c_int, c_int, c_int]),
+    'varq_fused_attn_classes': (c_int, [c_void_p, c_void_p, c_void_p, c_int, c_int,
+                                        c_int, c_int, c_int, c_int, c_int, c_int,
+                                        c_void_p, c_float, c_int, c_int, c_void_p, c_size_t, c_int, c_void_p]),
     'varq_fused_attn_channel': (c_int, [c_void_p, c_void_p,
                                         c_void_p, c_void_p, c_void_p,
                                         c_void_p, c_void_p, c_void_p,
@@ -54,6 +59,11 @@ SYMBOLS = {
                                         c_void_p, c_int, c_int, c_int, c_float,
                                         POINTER(c_int64), c_void_p,
                                         c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p]),
+    'varq_qkv_prepare_classes': (c_int, [c_void_p, c_int, c_int, c_int, c_int, c_int,
+                                         c_void_p, c_int, c_float,
+                                         c_void_p, c_void_p, c_int,
+                                         c_void_p, c_int, c_int, c_float,
+                                         c_void_p, c_int, c_int64, c_int64, c_void_p]),
 }
 
 _lib = None

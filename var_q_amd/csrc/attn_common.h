@@ -90,10 +90,11 @@ struct WidePlan {
   size_t tile_bytes;    // the expanded tiles, at the start of the workspace
   size_t ws_bytes;      // ... and the partial results behind them
 };
-WidePlan plan_wide(int64_t bh, int Lq, int Lk, int D, int cus);
+WidePlan plan_wide(int64_t bh, int Lq, int Lk, int D, int cus, bool share);   // share: whether blocks may be shared out
 // Expands the packed cache of p (per-key groups of k_group / v_group channels, or the per-channel
-// tables) into `tiles`, pair after pair.
-void launch_expand(const AttnParams &p, int D, int bits, int k_group, int v_group, bool chan, char *tiles, hipStream_t st);
+// tables) into `tiles`, pair after pair; with `place`, the pairs of a bit-width class to the places of
+// their heads (p.head_map) among the p.Hq heads of the cache.
+void launch_expand(const AttnParams &p, int D, int bits, int k_group, int v_group, bool chan, char *tiles, hipStream_t st, bool place = false);
 // Attends the expanded tiles at the start of `ws`; p.q_tiles counts blocks of 256 queries.
 void launch_wide(const AttnParams &p, int D, const WidePlan &plan, char *ws, hipStream_t st);
 

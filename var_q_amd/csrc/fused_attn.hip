@@ -48,6 +48,7 @@
 //      then use the same rounded weights.  V zero-points beyond +-kZmax (data offset by hundreds
 //      of quantization steps) or with a fractional part are split zp = zp_c + zp_r; the remainder
 //      goes through an fp32 correction term on tiles that have one.
+#include <algorithm>
 #include <type_traits>
 
 #include "attn_common.h"
@@ -303,8 +304,10 @@ template <int D, int BITS, int GK, int GV, bool CHAN, bool EXACT = false> struct
 // F16: q, out and the MFMA operands are fp16 instead of bf16 (dequantized K and V are rounded to
 // fp16, as the reference's fp16 attention call sees them: VAR/models/basic_var.py:157-158 under the
 // fp16 autocast of scripts/inference_multi_VAR.py:123); dequantizing kernels only.
-template <int D, int BITS, int GK, int GV, bool CHAN, int NWV = 8, int WPS = 2, bool EXACT = false, bool F16 = false>
-__global__ __launch_bounds__(NWV * 64, WPS) void fused_attn_kernel(AttnParams p) {
+// One workgroup's work: query tile qt of packed pair bh (= batch * p.Hkv + packed head), share `split` of its
+// keys; partial results go to the rows of pair `out_pair`.
+template <int D, int BITS, int GK, int GV, bool CHAN, int NWV, bool EXACT, bool F16>
+__device__ __forceinline__ void attend_block(const AttnParams &p, int bh, int out_pair, int qt, int split) {
   static_assert(!(F16 && EXACT), "the exact-code form builds bf16 images of the codes");
   static_assert(!CHAN || (GK == D && GV == D), "per-channel tables go with the single-group kernels");
   constexpr int NW = NWV, NT = NWV * 64, BM = NWV * 32;   // (shadow the defaults of the file)
@@ -362,20 +365,6 @@ __global__ __launch_bounds__(NWV * 64, WPS) void fused_attn_kernel(AttnParams p)
   constexpr int P_CK = 0, P_VR = NSK * BN, P_SV = P_VR + NSV * BN;
   constexpr int P_VZ = P_VR;   // DEQ: per (V group, key) the zero-point image; P_SV holds the scale image
 
-  // XCD-aware decode: consecutive workgroup ids go to different XCDs (8 of
-  // them), so ids congruent mod 8 share an L2.  All query tiles of one
-  // (batch, head) are given ids of one residue class to keep its packed K/V in
-  // that XCD's L2.
-  const int wg = blockIdx.x;
-  const int xcd = wg & 7, slot_s = wg >> 3;
-  const int split = p.nsplit > 1 ? slot_s % p.nsplit : 0;
-  const int slot = p.nsplit > 1 ? slot_s / p.nsplit : slot_s;
-  // (a token-major cache: the key rows of neighbouring heads share cache lines, so an XCD takes a
-  // run of consecutive (batch, head) pairs there instead of every eighth)
-  const int grp = slot / p.q_tiles;
-  const int bh = p.kv_hs == 1 && p.kv_ts > 1 ? xcd * ((p.bh_total + 7) >> 3) + grp : grp * 8 + xcd;
-  const int qt = slot % p.q_tiles;
-  if (bh >= p.bh_total) return;
   const int b = bh / p.Hkv, hs = bh % p.Hkv;
   const int hq = p.head_map ? p.head_map[hs] : hs;
 
@@ -1119,7 +1108,7 @@ __global__ __launch_bounds__(NWV * 64, WPS) void fused_attn_kernel(AttnParams p)
     // with the keys shared out: the normalized fp32 output and (reference, denominator) of
     // this share, for the combining kernel
     const bool shared_out = p.nsplit > 1;
-    const int64_t prow = ((int64_t)split * p.bh_total + bh) * p.Lq + qrow;
+    const int64_t prow = ((int64_t)split * p.bh_total + out_pair) * p.Lq + qrow;
     float *wptr = p.ws_o + prow * D;
     if (shared_out && half == 0) *reinterpret_cast<float2 *>(p.ws_ml + prow * 2) = make_float2(m_ref, l_sum);
 #pragma unroll
@@ -1141,6 +1130,73 @@ __global__ __launch_bounds__(NWV * 64, WPS) void fused_attn_kernel(AttnParams p)
       }
     }
   }
+}
+
+// Workgroup -> (pair, query tile, share of the keys).  XCD-aware: consecutive workgroup ids go to different
+// XCDs (8 of them), so ids congruent mod 8 share an L2.  All query tiles of one (batch, head) are given ids
+// of one residue class to keep its packed K/V in that XCD's L2.
+struct BlockOf {
+  int pair, qt, split;
+  __device__ __forceinline__ explicit BlockOf(const AttnParams &p) {
+    const int xcd = blockIdx.x & 7, slot_s = blockIdx.x >> 3;
+    split = p.nsplit > 1 ? slot_s % p.nsplit : 0;
+    const int slot = p.nsplit > 1 ? slot_s / p.nsplit : slot_s;
+    // (a token-major cache: the key rows of neighbouring heads share cache lines, so an XCD takes a
+    // run of consecutive (batch, head) pairs there instead of every eighth)
+    const int grp = slot / p.q_tiles;
+    pair = p.kv_hs == 1 && p.kv_ts > 1 ? xcd * ((p.bh_total + 7) >> 3) + grp : grp * 8 + xcd;
+    qt = slot % p.q_tiles;
+  }
+};
+
+template <int D, int BITS, int GK, int GV, bool CHAN, int NWV = 8, int WPS = 2, bool EXACT = false, bool F16 = false>
+__global__ __launch_bounds__(NWV * 64, WPS) void fused_attn_kernel(AttnParams p) {
+  const BlockOf k(p);
+  if (k.pair >= p.bh_total) return;
+  attend_block<D, BITS, GK, GV, CHAN, NWV, EXACT, F16>(p, k.pair, k.pair, k.qt, k.split);
+}
+
+// A cache whose heads have several bit-widths, all classes in one launch: pair k of the launch belongs to the
+// class that its range falls in (8-bit codes first: the longest workgroups start first), and the workgroup
+// runs that class's code.  The registers and the LDS are those of the most demanding class, which is no
+// more than each class takes alone (see launch_shape); what is gained are the launches -- and that the
+// classes, which have a few heads each, fill the device together.  Three widths, one launch per class ->
+// one launch, us: [2,16,128] 100 queries x 600 keys 66 -> 18, [8,16,128] 256 x 500 78 -> 28, 576 x 1497 140 ->
+// 117, 1024 x 2521 230 -> 200 (the last two with a stream for each class).
+struct ClassParams {
+  const u32 *k_words, *v_words;
+  const float *k_scale, *k_zp, *v_scale, *v_zp;
+  const int32_t *head_map;
+  int heads, first;   // packed heads of the class; its first pair of the launch
+};
+struct ClassTable { ClassParams c[3]; };   // of 8, 4 and 2 bits; a width that the cache does not have has no heads
+__device__ __forceinline__ void enter_class(AttnParams &p, const ClassParams &c) {
+  p.k_words = c.k_words; p.v_words = c.v_words;
+  p.k_scale = c.k_scale; p.k_zp = c.k_zp; p.v_scale = c.v_scale; p.v_zp = c.v_zp;
+  p.head_map = c.head_map;
+  p.Hkv = c.heads;
+  p.kv_bs = (int64_t)c.heads * p.Lstride;
+}
+// F(bits, pair within the class, pair of the output) for the class of pair k
+template <class F> __device__ __forceinline__ void in_class(AttnParams &p, const ClassTable &t, int k, F &&f) {
+  const int H = p.Hq;
+  auto run = [&](auto bits, const ClassParams &c) __attribute__((always_inline)) {
+    enter_class(p, c);
+    const int bh = k - c.first;
+    f(bits, bh, bh / c.heads * H + c.head_map[bh % c.heads]);
+  };
+  if (k < t.c[1].first) run(std::integral_constant<int, 8>{}, t.c[0]);
+  else if (k < t.c[2].first) run(std::integral_constant<int, 4>{}, t.c[1]);
+  else run(std::integral_constant<int, 2>{}, t.c[2]);
+}
+
+template <int D, int G, int NWV, int WPS, bool F16>
+__global__ __launch_bounds__(NWV * 64, WPS) void fused_attn_classes_kernel(AttnParams p, ClassTable t) {
+  const BlockOf k(p);
+  if (k.pair >= p.bh_total) return;
+  in_class(p, t, k.pair, [&](auto bits, int bh, int out_pair) __attribute__((always_inline)) {
+    attend_block<D, decltype(bits)::value, G, G, false, NWV, false, F16>(p, bh, out_pair, k.qt, k.split);
+  });
 }
 
 // The shares' outputs weighted by their softmax mass l * 2^(m - M), M the largest reference among
@@ -1260,6 +1316,15 @@ template <int D, bool F16> void launch_combine(const AttnParams &p, hipStream_t 
 
 int device_cus();
 
+// above 64 KiB of LDS the limit has to be raised, once per device the process launches on
+void allow_lds(const void *kernel, int bytes, bool (&configured)[64]) {
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) dev = -1;
+  if (dev >= 0 && configured[dev]) return;
+  (void)hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
+  if (dev >= 0) configured[dev] = true;
+}
+
 template <int D, int BITS, int GK, int GV, bool CHAN, int NWV, int WPS = 2, bool EXACT = false, bool F16 = false>
 void launch_shape(const AttnParams &p, hipStream_t st) {
   // (the per-channel tables take LDS by the number of segments of the launch)
@@ -1267,15 +1332,8 @@ void launch_shape(const AttnParams &p, hipStream_t st) {
   constexpr int lds_max = lds_base + kMaxSegments * lds_seg;
   static_assert(lds_max <= 160 * 1024, "LDS budget");
   const int lds_bytes = lds_base + p.nseg * lds_seg;
-  // above 64 KiB the limit has to be raised, once per device the process launches on
   static bool configured[64] = {false};
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) dev = -1;
-  if (dev < 0 || !configured[dev]) {
-    (void)hipFuncSetAttribute(reinterpret_cast<const void *>(&fused_attn_kernel<D, BITS, GK, GV, CHAN, NWV, WPS, EXACT, F16>),
-                              hipFuncAttributeMaxDynamicSharedMemorySize, lds_max);
-    if (dev >= 0) configured[dev] = true;
-  }
+  allow_lds(reinterpret_cast<const void *>(&fused_attn_kernel<D, BITS, GK, GV, CHAN, NWV, WPS, EXACT, F16>), lds_max, configured);
   const int bh_pad = (p.bh_total + 7) / 8 * 8;
   dim3 grid((unsigned)(bh_pad * p.q_tiles * p.nsplit));
   hipLaunchKernelGGL((fused_attn_kernel<D, BITS, GK, GV, CHAN, NWV, WPS, EXACT, F16>), grid, dim3(NWV * 64), lds_bytes, st, p);
@@ -1331,6 +1389,26 @@ int dispatch_groups(const AttnParams &p, int gk, int gv, hipStream_t st) {
   VARQ_G(128, 128) VARQ_G(64, 64) VARQ_G(32, 32) VARQ_G(32, 64)
 #undef VARQ_G
   return -1;
+}
+
+template <int D, int G, int NWV, int WPS, bool F16>
+void launch_classes_shape(const AttnParams &p, const ClassTable &t, hipStream_t st) {
+  constexpr int lds = std::max({AttnLds<D, 8, G, G, false>::kBytes, AttnLds<D, 4, G, G, false>::kBytes, AttnLds<D, 2, G, G, false>::kBytes});
+  static bool configured[64] = {false};
+  allow_lds(reinterpret_cast<const void *>(&fused_attn_classes_kernel<D, G, NWV, WPS, F16>), lds, configured);
+  dim3 grid((unsigned)((p.bh_total + 7) / 8 * 8 * p.q_tiles * p.nsplit));
+  hipLaunchKernelGGL((fused_attn_classes_kernel<D, G, NWV, WPS, F16>), grid, dim3(NWV * 64), lds, st, p, t);
+  if (p.nsplit > 1) launch_combine<D, F16>(p, st);
+}
+// (the workgroup sizes by the rules of launch())
+template <int D, int G> void launch_classes(const AttnParams &p, const ClassTable &t, hipStream_t st) {
+  if constexpr (D == 64) {
+    const bool four = p.Lq <= 128 && p.bh_total > device_cus();
+    if (p.f16) { if (four) launch_classes_shape<D, G, 4, 2, true>(p, t, st); else launch_classes_shape<D, G, 8, 4, true>(p, t, st); }
+    else { if (four) launch_classes_shape<D, G, 4, 2, false>(p, t, st); else launch_classes_shape<D, G, 8, 4, false>(p, t, st); }
+  } else {
+    launch_classes_shape<D, G, 8, 2, false>(p, t, st);
+  }
 }
 
 int set_layout(AttnParams &p, int layout, const char *who) {
@@ -1449,7 +1527,7 @@ struct FewQLds {
 };
 
 template <int BITS>
-__global__ __launch_bounds__(FQ_NW * 64, 2) void fused_attn_fewq_kernel(AttnParams p) {
+__device__ __forceinline__ void attend_few(const AttnParams &p, int bh, int out_pair, int qt, int split) {
   constexpr int D = FQ_D, WPR = D * BITS / 32, NCH = D / 16, NDB = D / 32;
   constexpr int HW = WPR / 2;                 // packed words of half a key row
   constexpr int KP = HW / 4;                  // 16-byte pieces of it
@@ -1465,15 +1543,6 @@ __global__ __launch_bounds__(FQ_NW * 64, 2) void fused_attn_fewq_kernel(AttnPara
   uint16_t *const vt = reinterpret_cast<uint16_t *>(lds_raw + FewQLds::kVt) + wave * D * FQ_VTS;
   float *const lds_ml = reinterpret_cast<float *>(lds_raw + FewQLds::kMl);
 
-  // workgroup -> (batch * head, query tile, share) without a division: the grid is (8, shares,
-  // groups of eight (batch, head) x query tiles); x runs fastest in the dispatch order, so the
-  // workgroups of one (batch, head) sit on one XCD (one L2), as in the kernel above.
-  static_assert(kFewQueries <= 64, "at most two query tiles");
-  const int xcd = blockIdx.x, split = blockIdx.y, slot = blockIdx.z;
-  const int qt = p.q_tiles == 2 ? (slot & 1) : 0;
-  const int grp = p.q_tiles == 2 ? (slot >> 1) : slot;
-  const int bh = p.kv_hs == 1 && p.kv_ts > 1 ? xcd * ((p.bh_total + 7) >> 3) + grp : grp * 8 + xcd;   // (as in the kernel above)
-  if (bh >= p.bh_total) return;
   const int b = bh / p.Hkv, hs = bh % p.Hkv;
   const int hq = p.head_map ? p.head_map[hs] : hs;
 
@@ -1837,7 +1906,7 @@ __global__ __launch_bounds__(FQ_NW * 64, 2) void fused_attn_fewq_kernel(AttnPara
   const float inv = l_sum > 0.f ? 1.0f / l_sum : 0.f;
   // registers 4*g4 .. 4*g4+3 are rows 32*wave + 8*g4 + 4*half + 0..3 of O^T
   if (p.nsplit > 1) {
-    const int64_t prow = ((int64_t)split * p.bh_total + bh) * p.Lq + qrow;
+    const int64_t prow = ((int64_t)split * p.bh_total + out_pair) * p.Lq + qrow;
     float *wptr = p.ws_o + prow * D + wave * 32 + 4 * half;
     if (wave == 0 && half == 0) *reinterpret_cast<float2 *>(p.ws_ml + prow * 2) = make_float2(M, l_sum);
 #pragma unroll
@@ -1850,6 +1919,34 @@ __global__ __launch_bounds__(FQ_NW * 64, 2) void fused_attn_fewq_kernel(AttnPara
       *reinterpret_cast<uint2 *>(optr + 8 * g4) =
           make_uint2(pack_bf16_rne(mine[4 * g4] * inv, mine[4 * g4 + 1] * inv), pack_bf16_rne(mine[4 * g4 + 2] * inv, mine[4 * g4 + 3] * inv));
   }
+}
+
+// Workgroup -> (pair, query tile, share) without a division: the grid is (8, shares, groups of eight
+// (batch, head) x query tiles); x runs fastest in the dispatch order, so the workgroups of one (batch,
+// head) sit on one XCD (one L2), as in the kernel above.
+struct FewBlockOf {
+  int pair, qt, split;
+  __device__ __forceinline__ explicit FewBlockOf(const AttnParams &p) {
+    static_assert(kFewQueries <= 64, "at most two query tiles");
+    const int xcd = blockIdx.x, slot = blockIdx.z;
+    split = blockIdx.y;
+    qt = p.q_tiles == 2 ? (slot & 1) : 0;
+    const int grp = p.q_tiles == 2 ? (slot >> 1) : slot;
+    pair = p.kv_hs == 1 && p.kv_ts > 1 ? xcd * ((p.bh_total + 7) >> 3) + grp : grp * 8 + xcd;   // (as in BlockOf)
+  }
+};
+template <int BITS>
+__global__ __launch_bounds__(FQ_NW * 64, 2) void fused_attn_fewq_kernel(AttnParams p) {
+  const FewBlockOf k(p);
+  if (k.pair >= p.bh_total) return;
+  attend_few<BITS>(p, k.pair, k.pair, k.qt, k.split);
+}
+__global__ __launch_bounds__(FQ_NW * 64, 2) void fused_attn_fewq_classes_kernel(AttnParams p, ClassTable t) {
+  const FewBlockOf k(p);
+  if (k.pair >= p.bh_total) return;
+  in_class(p, t, k.pair, [&](auto bits, int bh, int out_pair) __attribute__((always_inline)) {
+    attend_few<decltype(bits)::value>(p, bh, out_pair, k.qt, k.split);
+  });
 }
 
 // Whether a launch takes the few-queries kernel, and over how many workgroups the keys of a
@@ -1871,10 +1968,21 @@ int fewq_shares(int bh_total, int Lq, int Lk) {
   return s < 1 ? 1 : (int)s;
 }
 
+// The split fields of a launch of the few-queries kernel: no more shares than the workspace holds.
+void set_few(AttnParams &p, void *workspace, size_t workspace_bytes) {
+  const int64_t rows = (int64_t)p.bh_total * p.Lq;
+  int n = fewq_shares(p.bh_total, p.Lq, p.Lk);
+  while (n > 1 && (!workspace || ((uintptr_t)workspace & 15) || workspace_bytes < split_workspace_bytes(n, rows, FQ_D))) --n;
+  p.q_tiles = (p.Lq + 31) / 32;
+  p.nsplit = n;
+  p.fq_share_blocks = ((p.Lk + FQ_BK - 1) / FQ_BK + n - 1) / n;
+  p.ws_o = n > 1 ? reinterpret_cast<float *>(workspace) : nullptr;
+  p.ws_ml = n > 1 ? p.ws_o + (size_t)n * (size_t)rows * (size_t)FQ_D : nullptr;
+}
+
+dim3 few_grid(const AttnParams &p) { return dim3(8, (unsigned)p.nsplit, (unsigned)((p.bh_total + 7) / 8 * p.q_tiles)); }
 template <int BITS> void launch_fewq(const AttnParams &p, hipStream_t st) {
-  const int bh_pad = (p.bh_total + 7) / 8 * 8;
-  dim3 grid(8, (unsigned)p.nsplit, (unsigned)(bh_pad / 8 * p.q_tiles));
-  hipLaunchKernelGGL((fused_attn_fewq_kernel<BITS>), grid, dim3(FQ_NW * 64), FewQLds::kBytes, st, p);
+  hipLaunchKernelGGL((fused_attn_fewq_kernel<BITS>), few_grid(p), dim3(FQ_NW * 64), FewQLds::kBytes, st, p);
   if (p.nsplit > 1) launch_combine<FQ_D, false>(p, st);
 }
 
@@ -1889,12 +1997,12 @@ bool wide_eligible(int64_t bh, int Lq, int Lk, int D) {
   return Lq >= (D == 128 ? 1280 : 1536) && Lk >= 2048 && bh * ((Lq + 255) / 256) >= 160 && bh <= 65535;
 }
 // The launches of the wide path, or false when the workspace does not hold what they need.
-bool run_wide(const AttnParams &p, int D, int bits, int k_group, int v_group, bool chan, void *workspace, size_t workspace_bytes,
-              hipStream_t st) {
-  const WidePlan plan = plan_wide(p.bh_total, p.Lq, p.Lk, D, device_cus());
+template <class Expand>
+bool run_wide(const AttnParams &p, int D, int splits, void *workspace, size_t workspace_bytes, hipStream_t st, Expand &&expand) {
+  const WidePlan plan = plan_wide(p.bh_total, p.Lq, p.Lk, D, device_cus(), splits == 0);
   if (!workspace || ((uintptr_t)workspace & 15) || workspace_bytes < plan.ws_bytes) return false;
   char *const ws = reinterpret_cast<char *>(workspace);
-  launch_expand(p, D, bits, k_group, v_group, chan, ws, st);
+  expand(ws);
   launch_wide(p, D, plan, ws, st);
   return true;
 }
@@ -1915,7 +2023,7 @@ extern "C" size_t varq_fused_attn_workspace_bytes(int B, int Hkv, int Lq, int Lk
 
 extern "C" size_t varq_fused_attn_expand_bytes(int B, int Hkv, int Lq, int Lk, int D) {
   if (B <= 0 || Hkv <= 0 || Lq <= 0 || Lk <= 0 || (D != 64 && D != 128) || !wide_eligible((int64_t)B * Hkv, Lq, Lk, D)) return 0;
-  return plan_wide((int64_t)B * Hkv, Lq, Lk, D, device_cus()).ws_bytes;
+  return plan_wide((int64_t)B * Hkv, Lq, Lk, D, device_cus(), true).ws_bytes;
 }
 
 extern "C" int varq_fused_attn_key_shares(int B, int Hkv, int Lq, int Lk, int D, int k_group, int v_group) {
@@ -1974,22 +2082,15 @@ extern "C" int varq_fused_attn(const void *q, void *out,
   hipStream_t st = (hipStream_t)stream;
   // few queries over a long cache, left to the library: the kernel whose wavefronts share the keys
   if (splits == 0 && !p.f16 && !p.exact_codes && fewq_eligible(B, Hkv, Lq, Lk, D, k_group, v_group)) {
-    const int64_t rows = (int64_t)p.bh_total * Lq;
-    int n = fewq_shares(p.bh_total, Lq, Lk);
-    while (n > 1 && (!workspace || ((uintptr_t)workspace & 15) || workspace_bytes < split_workspace_bytes(n, rows, D))) --n;
-    p.q_tiles = (Lq + 31) / 32;
-    p.nsplit = n;
-    p.fq_share_blocks = ((Lk + FQ_BK - 1) / FQ_BK + n - 1) / n;
-    p.ws_o = n > 1 ? reinterpret_cast<float *>(workspace) : nullptr;
-    p.ws_ml = n > 1 ? p.ws_o + (size_t)n * (size_t)rows * (size_t)D : nullptr;
+    set_few(p, workspace, workspace_bytes);
     if (k_bits == 4) launch_fewq<4>(p, st);
     else if (k_bits == 8) launch_fewq<8>(p, st);
     else launch_fewq<2>(p, st);
     VARQ_CHECK_LAUNCH("fused_attn");
     return VARQ_OK;
   }
-  if (splits == 0 && !p.exact_codes && wide_eligible(p.bh_total, Lq, Lk, D) &&
-      run_wide(p, D, k_bits, k_group, v_group, false, workspace, workspace_bytes, st)) {
+  if ((splits == 0 || splits == 1) && !p.exact_codes && wide_eligible(p.bh_total, Lq, Lk, D) &&
+      run_wide(p, D, splits, workspace, workspace_bytes, st, [&](char *ws) { launch_expand(p, D, k_bits, k_group, v_group, false, ws, st); })) {
     VARQ_CHECK_LAUNCH("fused_attn");
     return VARQ_OK;
   }
@@ -2069,7 +2170,8 @@ extern "C" int varq_fused_attn_channel(const void *q, void *out,
   p.exact_codes = 0;
   if (int e = set_layout(p, layout, "fused_attn_channel")) return e;
   hipStream_t st = (hipStream_t)stream;
-  if (splits == 0 && wide_eligible(p.bh_total, Lq, Lk, D) && run_wide(p, D, bits, D, D, true, workspace, workspace_bytes, st)) {
+  if ((splits == 0 || splits == 1) && wide_eligible(p.bh_total, Lq, Lk, D) &&
+      run_wide(p, D, splits, workspace, workspace_bytes, st, [&](char *ws) { launch_expand(p, D, bits, D, D, true, ws, st); })) {
     VARQ_CHECK_LAUNCH("fused_attn_channel");
     return VARQ_OK;
   }
@@ -2085,5 +2187,85 @@ extern "C" int varq_fused_attn_channel(const void *q, void *out,
     else launch<64, 2, 64, 64, true>(p, st);
   }
   VARQ_CHECK_LAUNCH("fused_attn_channel");
+  return VARQ_OK;
+}
+
+// One call for all bit-width classes of a cache: see ClassTable.
+extern "C" int varq_fused_attn_classes(const void *q, void *out, const varq_kv_class *host_classes, int n_classes, int group,
+                                       int B, int H, int Lq, int Lk, int Lk_stride, int D,
+                                       const int32_t *kv_limit, float softmax_scale, int layout, int io_dtype,
+                                       void *workspace, size_t workspace_bytes, int splits, void *stream) {
+  VARQ_CHECK_ARG(B > 0 && H > 0 && Lq >= 0 && Lk >= 0 && Lk_stride >= Lk, "fused_attn_classes: bad sizes");
+  VARQ_CHECK_ARG(io_dtype == VARQ_BF16 || io_dtype == VARQ_F16, "fused_attn_classes: io_dtype must be VARQ_BF16 (1) or VARQ_F16 (2), got %d", io_dtype);
+  VARQ_CHECK_ARG(D == 64 || D == 128, "fused_attn_classes: D must be 64 or 128 (got %d)", D);
+  if (io_dtype == VARQ_F16 && D != 64)
+    return varq_set_error(VARQ_ERR_UNSUPPORTED, "fused_attn_classes: fp16 queries need D = 64 (got %d); D = 128 is served in bf16", D);
+  VARQ_CHECK_ARG(layout == VARQ_LAYOUT_BHLC || layout == VARQ_LAYOUT_BHLC_OUT_BLHC, "fused_attn_classes: a heads-first cache is needed (layout %d)", layout);
+  VARQ_CHECK_ARG(host_classes && n_classes >= 1 && n_classes <= 3, "fused_attn_classes: 1..3 classes (got %d)", n_classes);
+  VARQ_CHECK_ARG(group == 32 || group == 64 || (group == 128 && D == 128), "fused_attn_classes: no kernel for D=%d group=%d", D, group);
+  VARQ_CHECK_ARG(Lq == 0 || (q && out), "fused_attn_classes: null pointer");
+  VARQ_CHECK_ARG((int64_t)B * H * Lk_stride * D < (1ll << 40) && (int64_t)B * H < (1 << 24), "fused_attn_classes: cache too large");
+  VARQ_CHECK_ARG(((uintptr_t)q & 15) == 0 && ((uintptr_t)out & 7) == 0, "fused_attn_classes: q must be 16-byte and out 8-byte aligned");
+  if (Lq == 0) return VARQ_OK;
+  VARQ_CHECK_ARG(Lk > 0, "fused_attn_classes: no keys to attend");
+  ClassTable t = {};
+  int heads = 0;
+  for (int i = 0; i < n_classes; ++i) {
+    const varq_kv_class &c = host_classes[i];
+    VARQ_CHECK_ARG(c.bits == 2 || c.bits == 4 || c.bits == 8, "fused_attn_classes: bits must be 2, 4 or 8 (got %d)", c.bits);
+    VARQ_CHECK_ARG(c.heads > 0 && c.head_map && c.k_words && c.v_words && c.k_scale && c.v_scale, "fused_attn_classes: incomplete class %d", i);
+    ClassParams &d = t.c[c.bits == 8 ? 0 : c.bits == 4 ? 1 : 2];
+    VARQ_CHECK_ARG(!d.heads, "fused_attn_classes: two classes of %d bits", c.bits);
+    d = {reinterpret_cast<const u32 *>(c.k_words), reinterpret_cast<const u32 *>(c.v_words), c.k_scale, c.k_zp, c.v_scale, c.v_zp, c.head_map, c.heads, 0};
+    heads += c.heads;
+  }
+  VARQ_CHECK_ARG(heads == H, "fused_attn_classes: the classes have %d heads, not %d", heads, H);
+  t.c[1].first = B * t.c[0].heads;
+  t.c[2].first = t.c[1].first + B * t.c[1].heads;
+
+  AttnParams p = {};
+  p.q = reinterpret_cast<const __bf16 *>(q);
+  p.out = reinterpret_cast<__bf16 *>(out);
+  p.nseg = 1;
+  for (int s = 0; s < kMaxSegments; ++s) p.seg_end[s] = Lk;
+  p.kv_limit = kv_limit;
+  p.B = B; p.Hq = H; p.Hkv = H; p.Lq = Lq; p.Lk = Lk; p.Lstride = Lk_stride;
+  p.q_tiles = (Lq + BM - 1) / BM;
+  p.bh_total = B * H;
+  p.scale_log2e = softmax_scale * kLog2e;
+  p.f16 = io_dtype == VARQ_F16;
+  if (int e = set_layout(p, layout, "fused_attn_classes")) return e;
+  hipStream_t st = (hipStream_t)stream;
+  if (splits == 0 && !p.f16 && fewq_eligible(B, H, Lq, Lk, D, group, group)) {
+    set_few(p, workspace, workspace_bytes);
+    hipLaunchKernelGGL(fused_attn_fewq_classes_kernel, few_grid(p), dim3(FQ_NW * 64), FewQLds::kBytes, st, p, t);
+    if (p.nsplit > 1) launch_combine<FQ_D, false>(p, st);
+  } else if ((splits == 0 || splits == 1) && wide_eligible(p.bh_total, Lq, Lk, D) &&
+             run_wide(p, D, splits, workspace, workspace_bytes, st, [&](char *ws) {
+               // (one expanding launch per class, into the places of its heads)
+               for (int i = 0; i < 3; ++i) {
+                 if (!t.c[i].heads) continue;
+                 AttnParams c = p;
+                 c.k_words = t.c[i].k_words; c.v_words = t.c[i].v_words;
+                 c.k_scale = t.c[i].k_scale; c.k_zp = t.c[i].k_zp; c.v_scale = t.c[i].v_scale; c.v_zp = t.c[i].v_zp;
+                 c.head_map = t.c[i].head_map;
+                 c.Hkv = t.c[i].heads;
+                 c.bh_total = B * c.Hkv;
+                 c.kv_bs = (int64_t)c.Hkv * Lk_stride;
+                 launch_expand(c, D, 8 >> i, group, group, false, ws, st, true);
+               }
+             })) {
+  } else {
+    if (int e = set_splits(p, D, (Lk + BN - 1) / BN, splits, workspace, workspace_bytes, "fused_attn_classes")) return e;
+    if (D == 128) {
+      if (group == 128) launch_classes<128, 128>(p, t, st);
+      else if (group == 64) launch_classes<128, 64>(p, t, st);
+      else launch_classes<128, 32>(p, t, st);
+    } else {
+      if (group == 64) launch_classes<64, 64>(p, t, st);
+      else launch_classes<64, 32>(p, t, st);
+    }
+  }
+  VARQ_CHECK_LAUNCH("fused_attn_classes");
   return VARQ_OK;
 }

@@ -315,17 +315,9 @@ int layout_code(PyObject *o) {
   return VARQ_LAYOUT_BLHC;
 }
 
-// (the checks that both attention calls share; a: q, k_words, out, layout, out_layout)
-AttnShape attn_shape(const at::Tensor &q, const at::Tensor &kw, PyObject *out, PyObject *layout, PyObject *out_layout) {
-  AttnShape s;
-  ASSERT((q.scalar_type() == at::kBFloat16 || q.scalar_type() == at::kHalf) && q.dim() == 4, "q must be bf16 or fp16");
-  ASSERT(kw.dim() == 4, "k_words must be 4-D");
-  const int lay = layout_code(layout), h = lay == VARQ_LAYOUT_BHLC ? 1 : 2, t = 3 - h;
-  s.B = q.size(0); s.Hq = q.size(h); s.Lq = q.size(t); s.D = q.size(3);
-  s.Hkv = kw.size(h); s.Lstride = kw.size(t);
-  ASSERT(kw.size(0) == s.B, "batch sizes of q and the cache differ");
+// the layout of the call and its result tensor
+void make_out(AttnShape &s, const at::Tensor &q, PyObject *out, int lay, int olay) {
   s.layout = lay;
-  const int olay = out_layout == Py_None ? lay : layout_code(out_layout);
   if (olay != lay) {
     ASSERT(lay == VARQ_LAYOUT_BHLC, "out_layout: only tokens-first out of a heads-first call");
     s.layout = VARQ_LAYOUT_BHLC_OUT_BLHC;
@@ -338,6 +330,18 @@ AttnShape attn_shape(const at::Tensor &q, const at::Tensor &kw, PyObject *out, P
     ASSERT(s.out.scalar_type() == q.scalar_type() && s.out.sizes() == at::IntArrayRef(n, 4) && s.out.is_contiguous(),
            "out must be contiguous, of the dtype of q and of the shape its layout implies");
   }
+}
+
+// (the checks that both attention calls share; a: q, k_words, out, layout, out_layout)
+AttnShape attn_shape(const at::Tensor &q, const at::Tensor &kw, PyObject *out, PyObject *layout, PyObject *out_layout) {
+  AttnShape s;
+  ASSERT((q.scalar_type() == at::kBFloat16 || q.scalar_type() == at::kHalf) && q.dim() == 4, "q must be bf16 or fp16");
+  ASSERT(kw.dim() == 4, "k_words must be 4-D");
+  const int lay = layout_code(layout), h = lay == VARQ_LAYOUT_BHLC ? 1 : 2, t = 3 - h;
+  s.B = q.size(0); s.Hq = q.size(h); s.Lq = q.size(t); s.D = q.size(3);
+  s.Hkv = kw.size(h); s.Lstride = kw.size(t);
+  ASSERT(kw.size(0) == s.B, "batch sizes of q and the cache differ");
+  make_out(s, q, out, lay, out_layout == Py_None ? lay : layout_code(out_layout));
   return s;
 }
 const at::Tensor &dense(PyObject *o, const char *name) {
@@ -355,7 +359,7 @@ int io_code(const at::Tensor &q) { return q.scalar_type() == at::kHalf ? VARQ_F1
 // device memory for a launch that shares keys out or expands them (0: neither)
 size_t workspace_bytes(const AttnShape &s, int64_t Lk, int nseg, int64_t splits) {
   const size_t shared = varq_fused_attn_workspace_bytes((int)s.B, (int)s.Hkv, (int)s.Lq, (int)Lk, (int)s.D, nseg, (int)splits);
-  return splits ? shared : std::max(shared, varq_fused_attn_expand_bytes((int)s.B, (int)s.Hkv, (int)s.Lq, (int)Lk, (int)s.D));
+  return splits > 1 ? shared : std::max(shared, varq_fused_attn_expand_bytes((int)s.B, (int)s.Hkv, (int)s.Lq, (int)Lk, (int)s.D));
 }
 
 // attn(q, k_words, k_scale, k_zp, v_words, v_scale, v_zp, k_bits, v_bits, Lk, softmax_scale, kv_limit, head_map, out, splits,
@@ -454,6 +458,43 @@ struct CacheClass {
   }
 };
 
+// the classes of a cache as the C ABI takes them
+int class_table(const Cache &c, varq_kv_class (&t)[3]) {
+  const Py_ssize_t n = c.size();
+  ASSERT(n >= 1 && n <= 3, "a cache has 1..3 bit-width classes");
+  for (Py_ssize_t i = 0; i < n; ++i) {
+    const CacheClass k(PyTuple_GET_ITEM(c.classes, i));
+    t[i] = {(int)k.bits, (int)k.heads, ptr<int32_t>(k.head_map), ptr<int32_t>(k.slot), ptr<int32_t>(k.k_words), ptr<int32_t>(k.v_words),
+            ptr<float>(k.k_scale), c.asym ? ptr<float>(k.k_zp) : nullptr, ptr<float>(k.v_scale), c.asym ? ptr<float>(k.v_zp) : nullptr};
+  }
+  return (int)n;
+}
+
+// cache_attend(cache, len, q, softmax_scale, kv_limit, out, splits, out_layout) -> out: all classes of a mixed-width cache
+PyObject *cache_attend(PyObject *const *a) {
+  const Cache c(a[0]);
+  const int64_t len = integer(a[1]), splits = integer(a[6]);
+  const at::Tensor &q = dense(a[2], "q");
+  const at::Tensor *limit = maybe(a[4], "kv_limit");
+  ASSERT((q.scalar_type() == at::kBFloat16 || q.scalar_type() == at::kHalf) && q.dim() == 4, "q must be bf16 or fp16");
+  ASSERT(q.size(0) == c.B && q.size(1) == c.H && q.size(3) == c.D, "attend: q does not fit the cache");
+  ASSERT(0 < len && len <= c.Lmax, "attend: the cache holds no such token");
+  const c10::DeviceGuard guard(q.device());
+  AttnShape s;
+  s.B = c.B; s.Hq = s.Hkv = c.H; s.Lq = q.size(2); s.D = c.D; s.Lstride = c.Lmax;
+  make_out(s, q, a[5], VARQ_LAYOUT_BHLC, layout_code(a[7]));
+  check_limit_and_map(limit, nullptr, s);
+  varq_kv_class t[3];
+  const int n = class_table(c, t);
+  const size_t ws_bytes = workspace_bytes(s, len, 1, splits);
+  at::Tensor ws;
+  if (ws_bytes) ws = empty({(int64_t)ws_bytes}, at::kByte, q);
+  check(varq_fused_attn_classes(q.data_ptr(), s.out.data_ptr(), t, n, (int)c.group, (int)c.B, (int)c.H, (int)s.Lq, (int)len, (int)c.Lmax, (int)c.D,
+                                ptr<int32_t>(limit), (float)real(a[3]), s.layout, io_code(q), ws_bytes ? ws.data_ptr() : nullptr, ws_bytes, (int)splits,
+                                stream_of(q)), "varq_fused_attn_classes");
+  return wrap(s.out);
+}
+
 // cache_append(cache, len, k, v, layout) -> tokens appended
 PyObject *cache_append(PyObject *const *a) {
   const Cache c(a[0]);
@@ -470,6 +511,17 @@ PyObject *cache_append(PyObject *const *a) {
   void *const st = stream_of(k);
   const int kd = dtype_code(k), vd = dtype_code(v);
   const int64_t rows = c.B * c.H * n;
+  if (c.size() > 1) {   // (one launch for all classes, where the sizes allow it)
+    varq_kv_class t[3];
+    const int nc = class_table(c, t);
+    auto classes = [&](const void *kp, const void *vp, int dt) {
+      return varq_quant_pack_classes(kp, vp, dt, lay, (int)c.B, (int)c.H, n, (int)c.D, (int)c.group, c.asym, c.eps, t, nc, c.Lmax, len, st);
+    };
+    int rc = kd == vd ? classes(k.data_ptr(), v.data_ptr(), kd) : classes(k.data_ptr(), nullptr, kd);
+    if (kd != vd && rc == VARQ_OK) rc = classes(nullptr, v.data_ptr(), vd);
+    if (rc == VARQ_OK) return PyLong_FromLongLong(n);
+    if (rc != VARQ_ERR_UNSUPPORTED) check(rc, "varq_quant_pack_classes");
+  }
   for (Py_ssize_t i = 0; i < c.size(); ++i) {
     const CacheClass cl(PyTuple_GET_ITEM(c.classes, i));
     // input rows in memory order -> output row b*hc*Lmax + slot(h)*Lmax + len + l
@@ -507,6 +559,15 @@ PyObject *cache_prepare(PyObject *const *a) {
   if (mul) ASSERT(mul->scalar_type() == at::kFloat && mul->numel() == c.H && mul->is_contiguous(), "q_scale_mul must be contiguous fp32 [H]");
   const c10::DeviceGuard guard(qkv.device());
   const at::Tensor q = empty({c.B, c.H, n, c.D}, at::kBFloat16, qkv);
+  if (c.size() > 1) {
+    varq_kv_class t[3];
+    const int nc = class_table(c, t);
+    const int rc = varq_qkv_prepare_classes(qkv.data_ptr(), dtype_code(qkv), (int)c.B, (int)n, (int)c.H, (int)c.D, ptr<float>(mul), truth(a[4]),
+                                            (float)real(a[5]), ptr<float>(cs), ptr<float>(sn), (int)start, q.data_ptr(), (int)c.group, c.asym,
+                                            c.eps, t, nc, c.Lmax, len, stream_of(qkv));
+    if (rc == VARQ_OK) return wrap(q);
+    if (rc != VARQ_ERR_UNSUPPORTED) check(rc, "varq_qkv_prepare_classes");
+  }
   for (Py_ssize_t i = 0; i < c.size(); ++i) {
     const CacheClass cl(PyTuple_GET_ITEM(c.classes, i));
     const int64_t map[8] = {c.B, n, c.H, cl.heads * c.Lmax, 1, c.Lmax, len, 2};
@@ -541,7 +602,7 @@ PyObject *set_error(PyObject *, PyObject *e) {
 #define FIXED(name, n) {#name, (PyCFunction)(void (*)(void))fixed<name, n>, METH_FASTCALL, nullptr}
 PyMethodDef g_methods[] = {
     FIXED(quant_rows, 5), FIXED(quant_shared, 6), FIXED(pack, 2), FIXED(unpack, 3), FIXED(dequant, 6), FIXED(dequant_steps, 8), FIXED(attn, 18), FIXED(attn_channel, 17),
-    FIXED(cache_append, 5), FIXED(cache_prepare, 9),
+    FIXED(cache_attend, 8), FIXED(cache_append, 5), FIXED(cache_prepare, 9),
     {"quant_step", (PyCFunction)(void (*)(void))varying<quant_step>, METH_FASTCALL, nullptr},
     {"set_error", set_error, METH_O, nullptr},
     {nullptr, nullptr, 0, nullptr}};

@@ -148,29 +148,31 @@ __device__ __forceinline__ void octet_minmax(const float (&v)[8], float &mx, flo
 __device__ __forceinline__ float pair_swap(float v) { return dpp_f<0xB1>(v); }
 
 // One lane = 8 channels of one (b, l, h); LR = c/8 lanes form the row, LG = group/8 a group.
-template <int DT, int BITS, bool ASYM, int LR, int LG>
-__global__ __launch_bounds__(256) void qkv_prepare_kernel(PrepParams p) {
-  // One workgroup = one tile of 256/LR tokens of one (b, h): lanes walk the (b, h, l) order of the
-  // outputs, so the prepared q, the packed words and the scales of a wavefront are contiguous; the
-  // reads are whole 16*LR-byte rows either way.  (b, h) is uniform for the workgroup: no vector
-  // divisions.  Order of the workgroups (1-D grid; consecutive ids go to consecutive XCDs):
-  // id = ((tile / 8) * B*H + bh) * 8 + tile % 8.  The workgroups in flight together then read all
-  // heads of the same few tokens, whole 6*H*c-byte stretches of the input between them, instead
-  // of one 2*c-byte piece out of every token row (8 % of the kernel's time at H=16, c=128), and
-  // the B*H workgroups of one tile run on one XCD, whose L2 fetches that tile's rotary factors once.
-  const u32 id = blockIdx.x, j = id >> 3;
-  const u32 BH = (u32)(p.B * p.H);
-  const u32 tile8 = j / BH;                           // (uniform: scalar arithmetic)
-  const int bh = (int)(j - tile8 * BH);
-  const int h = bh % p.H, b = bh / p.H;
-  // a slot table over the heads (one launch per bit-width class of a mixed cache): the heads of
-  // the other classes are theirs altogether, q included, so that the launches share out the work
-  int head_slot = h;
-  if (p.map.slot_dim == 2) {
-    head_slot = p.slot[h];
-    if (head_slot < 0) return;                        // (uniform for the workgroup)
+//
+// One workgroup = one tile of 256/LR tokens of one (b, h): lanes walk the (b, h, l) order of the
+// outputs, so the prepared q, the packed words and the scales of a wavefront are contiguous; the
+// reads are whole 16*LR-byte rows either way.  (b, h) is uniform for the workgroup: no vector
+// divisions.  Order of the workgroups (1-D grid; consecutive ids go to consecutive XCDs):
+// id = ((tile / 8) * B*H + bh) * 8 + tile % 8.  The workgroups in flight together then read all
+// heads of the same few tokens, whole 6*H*c-byte stretches of the input between them, instead
+// of one 2*c-byte piece out of every token row (8 % of the kernel's time at H=16, c=128), and
+// the B*H workgroups of one tile run on one XCD, whose L2 fetches that tile's rotary factors once.
+struct TileOf {
+  u32 tile;
+  int bh, h, b;
+  __device__ __forceinline__ explicit TileOf(const PrepParams &p) {
+    const u32 id = blockIdx.x, j = id >> 3;
+    const u32 BH = (u32)(p.B * p.H);
+    const u32 tile8 = j / BH;                         // (uniform: scalar arithmetic)
+    bh = (int)(j - tile8 * BH);
+    h = bh % p.H; b = bh / p.H;
+    tile = tile8 * 8u + (id & 7u);
   }
-  const int o = (int)(tile8 * 8u + (id & 7u)) * 256 + threadIdx.x;
+};
+template <int DT, int BITS, bool ASYM, int LR, int LG>
+__device__ __forceinline__ void prepare_tile(const PrepParams &p, const TileOf &w, int head_slot) {
+  const int bh = w.bh, h = w.h, b = w.b;
+  const int o = (int)w.tile * 256 + threadIdx.x;
   const int lt = o / LR;                              // (LR is a power of two)
   const int col = o - lt * LR;
   const bool live = lt < p.L;
@@ -310,6 +312,42 @@ __global__ __launch_bounds__(256) void qkv_prepare_kernel(PrepParams p) {
   }
 }
 
+template <int DT, int BITS, bool ASYM, int LR, int LG>
+__global__ __launch_bounds__(256) void qkv_prepare_kernel(PrepParams p) {
+  const TileOf w(p);
+  // a slot table over the heads (one launch per bit-width class of a mixed cache): the heads of
+  // the other classes are theirs altogether, q included, so that the launches share out the work
+  int head_slot = w.h;
+  if (p.map.slot_dim == 2) {
+    head_slot = p.slot[w.h];
+    if (head_slot < 0) return;                        // (uniform for the workgroup)
+  }
+  prepare_tile<DT, BITS, ASYM, LR, LG>(p, w, head_slot);
+}
+
+// All heads of a mixed-width cache in one launch: a workgroup runs the code of its head's class.
+template <int DT, bool ASYM, int LR, int LG>
+__global__ __launch_bounds__(256) void qkv_prepare_classes_kernel(PrepParams p, ClassOuts t) {
+  const TileOf w(p);
+  in_class_of_head(t, w.h, [&](auto bits, const ClassOut &c, int slot) __attribute__((always_inline)) {
+    p.k_words = c.k_words; p.v_words = c.v_words;
+    p.k_scale = c.k_scale; p.k_zp = c.k_zp; p.v_scale = c.v_scale; p.v_zp = c.v_zp;
+    p.map.os0 = c.heads * p.map.os2;
+    prepare_tile<DT, decltype(bits)::value, ASYM, LR, LG>(p, w, slot);
+  });
+}
+
+template <int DT, bool ASYM> int launch_classes(const PrepParams &p, const ClassOuts &t, int group, dim3 grid, hipStream_t st) {
+#define VARQ_LR(C, R, G)                                                                                       \
+  if (p.c == C && group == 8 * G) {                                                                            \
+    hipLaunchKernelGGL((qkv_prepare_classes_kernel<DT, ASYM, R, G>), grid, dim3(256), 0, st, p, t);            \
+    return 0;                                                                                                  \
+  }
+  VARQ_LR(128, 16, 16) VARQ_LR(128, 16, 8) VARQ_LR(128, 16, 4) VARQ_LR(64, 8, 8) VARQ_LR(64, 8, 4)
+#undef VARQ_LR
+  return -1;
+}
+
 template <int DT, int BITS, bool ASYM, int LR>
 int launch_lg(const PrepParams &p, int lg, dim3 grid, hipStream_t st) {
   switch (lg) {
@@ -343,6 +381,37 @@ int launch_dt(const PrepParams &p, int bits, int asym, int lr, int lg, dim3 grid
 
 }  // namespace
 
+namespace {
+
+// What both entry points check and fill in alike; 0: nothing to do, 1: launch, negative: an error is set
+int prepare_params(PrepParams &p, dim3 &grid, const void *qkv, int x_dtype, int B, int L, int H, int c, const float *q_scale_mul, int l2norm,
+                   float norm_eps, const float *rope_cos, const float *rope_sin, int token_start, void *q_out, int group, float eps) {
+  auto refuse = [](const char *why) { varq_set_error(VARQ_ERR_INVALID, "qkv_prepare: %s", why); return -1; };
+  if (!(B >= 0 && L >= 0 && H > 0)) return refuse("bad sizes");
+  if (x_dtype < 0 || x_dtype > 2) return refuse("bad dtype");
+  if ((rope_cos == nullptr) != (rope_sin == nullptr)) return refuse("give both rotary tables or neither");
+  if (token_start < 0) return refuse("bad token_start");
+  const int64_t rows = (int64_t)B * L * H;
+  if (rows == 0) return 0;
+  if (!qkv || !q_out) return refuse("null pointer");
+  if (((uintptr_t)qkv & 15) || ((uintptr_t)q_out & 15)) return refuse("qkv and q_out must be 16-byte aligned");
+  const int64_t tiles = ((int64_t)L * (c / 8) + 255) / 256;
+  // (tiles are dealt out in eights; those past the last token find no live lane and store nothing)
+  const int64_t wgs = (tiles + 7) / 8 * 8 * ((int64_t)B * H);
+  if (!(rows * (c / 8) < (1ll << 31) - 256 && (int64_t)L * 3 * H * c < (1ll << 31) && ((int64_t)token_start + L) * (c / 2) < (1ll << 31)) ||
+      wgs >= (1ll << 31))
+    return refuse("tensor too large");
+  p.qkv = qkv; p.scale_mul = q_scale_mul; p.cos = rope_cos; p.sin = rope_sin; p.q_out = q_out;
+  p.B = B; p.L = L; p.H = H; p.c = c; p.c8 = c / 8; p.c8_shift = 0;
+  p.token_start = token_start; p.l2norm = l2norm ? 1 : 0; p.nseg = c / group;
+  p.norm_eps = norm_eps; p.eps = eps; p.rows = rows;
+  p.slow_levels = !(eps >= 0x1p-80f);
+  grid = dim3((unsigned)wgs);
+  return 1;
+}
+
+}  // namespace
+
 extern "C" int varq_qkv_prepare_append(const void *qkv, int x_dtype, int B, int L, int H, int c,
                                        const float *q_scale_mul, int l2norm, float norm_eps,
                                        const float *rope_cos, const float *rope_sin, int token_start,
@@ -350,39 +419,21 @@ extern "C" int varq_qkv_prepare_append(const void *qkv, int x_dtype, int B, int 
                                        const int64_t *host_rowmap, const int32_t *slot,
                                        int32_t *k_words, float *k_scale, float *k_zp,
                                        int32_t *v_words, float *v_scale, float *v_zp, void *stream) {
-  VARQ_CHECK_ARG(B >= 0 && L >= 0 && H > 0, "qkv_prepare: bad sizes");
   VARQ_CHECK_ARG(c == 32 || c == 64 || c == 128, "qkv_prepare: head dim must be 32, 64 or 128 (got %d)", c);
-  VARQ_CHECK_ARG(x_dtype >= 0 && x_dtype <= 2, "qkv_prepare: bad dtype %d", x_dtype);
   VARQ_CHECK_ARG(bits == 2 || bits == 4 || bits == 8, "qkv_prepare: bits must be 2, 4 or 8 (got %d)", bits);
   VARQ_CHECK_ARG(group >= 8 && group <= c && c % group == 0 && (group & (group - 1)) == 0,
                  "qkv_prepare: group must be a power of two in [8, c] (got %d)", group);
   VARQ_CHECK_ARG(bits != 2 || group >= 16, "qkv_prepare: 2-bit codes need groups of at least 16 channels");
-  VARQ_CHECK_ARG((rope_cos == nullptr) == (rope_sin == nullptr), "qkv_prepare: give both rotary tables or neither");
-  VARQ_CHECK_ARG(token_start >= 0, "qkv_prepare: bad token_start");
-  const int64_t rows = (int64_t)B * L * H;
-  if (rows == 0) return VARQ_OK;
-  VARQ_CHECK_ARG(qkv && q_out && k_words && v_words && k_scale && v_scale && (!asym || (k_zp && v_zp)) && host_rowmap,
-                 "qkv_prepare: null pointer");
-  VARQ_CHECK_ARG(((uintptr_t)qkv & 15) == 0 && ((uintptr_t)q_out & 15) == 0, "qkv_prepare: qkv and q_out must be 16-byte aligned");
-  VARQ_CHECK_ARG(rows * (c / 8) < (1ll << 31) - 256 && (int64_t)L * 3 * H * c < (1ll << 31) &&
-                     ((int64_t)token_start + L) * (c / 2) < (1ll << 31), "qkv_prepare: tensor too large");
-
   PrepParams p;
-  p.qkv = qkv; p.scale_mul = q_scale_mul; p.cos = rope_cos; p.sin = rope_sin; p.q_out = q_out;
+  dim3 grid;
+  const int todo = prepare_params(p, grid, qkv, x_dtype, B, L, H, c, q_scale_mul, l2norm, norm_eps, rope_cos, rope_sin, token_start, q_out, group, eps);
+  if (todo <= 0) return todo ? VARQ_ERR_INVALID : VARQ_OK;
+  VARQ_CHECK_ARG(k_words && v_words && k_scale && v_scale && (!asym || (k_zp && v_zp)) && host_rowmap, "qkv_prepare: null pointer");
   p.k_words = k_words; p.v_words = v_words; p.k_scale = k_scale; p.k_zp = k_zp; p.v_scale = v_scale; p.v_zp = v_zp;
   p.slot = slot;
-  p.map = varq_rowmap_from_host(host_rowmap, rows);
+  p.map = varq_rowmap_from_host(host_rowmap, p.rows);
   VARQ_CHECK_ARG(p.map.n0 == B && p.map.n1 == L && p.map.n2 == H, "qkv_prepare: row map dims must be (B, L, H)");
   VARQ_CHECK_ARG(p.map.slot_dim < 0 || slot, "qkv_prepare: slot table missing");
-  p.B = B; p.L = L; p.H = H; p.c = c; p.c8 = c / 8; p.c8_shift = 0;
-  p.token_start = token_start; p.l2norm = l2norm ? 1 : 0; p.nseg = c / group;
-  p.norm_eps = norm_eps; p.eps = eps; p.rows = rows;
-  p.slow_levels = !(eps >= 0x1p-80f);
-  const int64_t tiles = ((int64_t)L * p.c8 + 255) / 256;
-  // (tiles are dealt out in eights; those past the last token find no live lane and store nothing)
-  const int64_t wgs = (tiles + 7) / 8 * 8 * ((int64_t)B * H);
-  VARQ_CHECK_ARG(wgs < (1ll << 31), "qkv_prepare: tensor too large");
-  dim3 grid((unsigned)wgs);
   hipStream_t st = (hipStream_t)stream;
   int rc;
   if (x_dtype == VARQ_F32) rc = launch_dt<VARQ_F32>(p, bits, asym, p.c8, group / 8, grid, st);
@@ -390,5 +441,28 @@ extern "C" int varq_qkv_prepare_append(const void *qkv, int x_dtype, int B, int 
   else rc = launch_dt<VARQ_F16>(p, bits, asym, p.c8, group / 8, grid, st);
   if (rc) return varq_set_error(VARQ_ERR_UNSUPPORTED, "qkv_prepare: no kernel for c=%d group=%d", c, group);
   VARQ_CHECK_LAUNCH("qkv_prepare");
+  return VARQ_OK;
+}
+
+extern "C" int varq_qkv_prepare_classes(const void *qkv, int x_dtype, int B, int L, int H, int c, const float *q_scale_mul, int l2norm,
+                                        float norm_eps, const float *rope_cos, const float *rope_sin, int token_start, void *q_out, int group,
+                                        int asym, float eps, const varq_kv_class *host_classes, int n_classes, int64_t Lmax, int64_t start,
+                                        void *stream) {
+  VARQ_CHECK_ARG(c > 0 && group > 0 && c % group == 0 && start >= 0 && start + L <= Lmax, "qkv_prepare_classes: bad sizes");
+  PrepParams p;
+  dim3 grid;
+  const int todo = prepare_params(p, grid, qkv, x_dtype, B, L, H, c, q_scale_mul, l2norm, norm_eps, rope_cos, rope_sin, token_start, q_out, group, eps);
+  if (todo <= 0) return todo ? VARQ_ERR_INVALID : VARQ_OK;
+  ClassOuts t;
+  VARQ_CHECK_ARG(varq_class_outs(host_classes, n_classes, asym != 0, t), "qkv_prepare_classes: incomplete or repeated classes");
+  p.slot = nullptr;
+  p.map.n0 = B; p.map.n1 = L; p.map.n2 = H; p.map.os0 = 0; p.map.os1 = 1; p.map.os2 = Lmax; p.map.off = start; p.map.slot_dim = -1;
+  hipStream_t st = (hipStream_t)stream;
+  int rc;
+  if (x_dtype == VARQ_F32) rc = asym ? launch_classes<VARQ_F32, true>(p, t, group, grid, st) : launch_classes<VARQ_F32, false>(p, t, group, grid, st);
+  else if (x_dtype == VARQ_BF16) rc = asym ? launch_classes<VARQ_BF16, true>(p, t, group, grid, st) : launch_classes<VARQ_BF16, false>(p, t, group, grid, st);
+  else rc = asym ? launch_classes<VARQ_F16, true>(p, t, group, grid, st) : launch_classes<VARQ_F16, false>(p, t, group, grid, st);
+  if (rc) return varq_set_error(VARQ_ERR_UNSUPPORTED, "qkv_prepare_classes: no kernel for c=%d group=%d", c, group);
+  VARQ_CHECK_LAUNCH("qkv_prepare_classes");
   return VARQ_OK;
 }

@@ -193,27 +193,14 @@ __global__ __launch_bounds__(256) void quant_pack_rows_kernel(RowsParams p) {
 //
 // Rounding: x/s is needed exactly as an IEEE fp32 division rounds it; see the
 // two routes (fp32 correction step, fp64 product) in the kernel body.
+// Window `tile` of pair (i0, i1) of one tensor; stage: a wavefront-private window of 256 octets (in, then packed words out).
 template <int DT, int BITS, bool ASYM, int LPG4, bool DENSE>
-__global__ __launch_bounds__(256) void quant_pack_rows32_kernel(RowsParams p) {
-  __shared__ Raw8<DT> lds_stage[4][256];   // per wave: 256 octets in, then packed words out
-
-  const bool second = blockIdx.z >= (unsigned)p.map.n0;   // block-uniform
-  const void *px = second ? p.x1 : p.x;
-  int32_t *pwords = second ? p.words1 : p.words;
-  float *pscale = second ? p.scale1 : p.scale;
-  float *pzp = second ? p.zp1 : p.zp;
-  const int64_t i0 = blockIdx.z - (second ? (unsigned)p.map.n0 : 0u), i1 = p.strided ? blockIdx.x : blockIdx.y;
-  const int tile = p.strided ? blockIdx.y : blockIdx.x;
-  int64_t s0 = i0, s1 = i1;
-  if (p.map.slot_dim == 0) s0 = p.slot[i0];
-  if (p.map.slot_dim == 1) s1 = p.slot[i1];
-  if (s0 < 0 || s1 < 0) return;
-  const int64_t out_base = s0 * p.map.os0 + s1 * p.map.os1 + p.map.off;
+__device__ __forceinline__ void quant_window(const RowsParams &p, const void *px, int32_t *pwords, float *pscale, float *pzp, int64_t i0,
+                                             int64_t i1, int tile, int64_t out_base, Raw8<DT> *stage) {
   const int64_t pair_elem0 = i0 * p.in_s0 + i1 * p.in_s1;
 
   const int n_oct = (int)p.octets_per_pair;
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-  Raw8<DT> *stage = lds_stage[wv];
   constexpr float kMin = (float)QRange<BITS>::kMin, kMax = (float)QRange<BITS>::kMax;
   const int w0 = tile * 1024 + wv * 256;             // first octet of this wave's window, inside the pair
 
@@ -418,6 +405,45 @@ __global__ __launch_bounds__(256) void quant_pack_rows32_kernel(RowsParams p) {
   }
 }
 
+template <int DT, int BITS, bool ASYM, int LPG4, bool DENSE>
+__global__ __launch_bounds__(256) void quant_pack_rows32_kernel(RowsParams p) {
+  __shared__ Raw8<DT> lds_stage[4][256];
+  const bool second = blockIdx.z >= (unsigned)p.map.n0;   // block-uniform
+  const int64_t i0 = blockIdx.z - (second ? (unsigned)p.map.n0 : 0u), i1 = p.strided ? blockIdx.x : blockIdx.y;
+  int64_t s0 = i0, s1 = i1;
+  if (p.map.slot_dim == 0) s0 = p.slot[i0];
+  if (p.map.slot_dim == 1) s1 = p.slot[i1];
+  if (s0 < 0 || s1 < 0) return;
+  const int64_t out_base = s0 * p.map.os0 + s1 * p.map.os1 + p.map.off;
+  quant_window<DT, BITS, ASYM, LPG4, DENSE>(p, second ? p.x1 : p.x, second ? p.words1 : p.words, second ? p.scale1 : p.scale,
+                                            second ? p.zp1 : p.zp, i0, i1, p.strided ? blockIdx.y : blockIdx.x, out_base, lds_stage[threadIdx.x >> 6]);
+}
+
+// A step into a cache with several bit-widths, all heads in one launch: the head (i1) is uniform for the
+// workgroup, which runs the code of its class.  (One launch per class reads nothing twice either -- the
+// heads of the other classes return at once -- but a small step is bound by its launches, and a large one
+// by the device standing half empty at the end of each: K and V, three widths, bf16 [2,16,16,128] 11.7 ->
+// 4.3 us, [8,16,1024,128] 28.4 -> 20.1, [8,16,4096,128] 79 -> 64.)
+template <int DT, bool ASYM, int LPG4>
+__global__ __launch_bounds__(256) void quant_pack_classes_kernel(RowsParams p, ClassOuts t) {
+  __shared__ Raw8<DT> lds_stage[4][256];
+  const bool second = blockIdx.z >= (unsigned)p.map.n0;   // block-uniform
+  const int64_t i0 = blockIdx.z - (second ? (unsigned)p.map.n0 : 0u), i1 = p.strided ? blockIdx.x : blockIdx.y;
+  const bool is_v = second || !p.x;
+  in_class_of_head(t, (int)i1, [&](auto bits, const ClassOut &c, int slot) __attribute__((always_inline)) {
+    const int64_t out_base = (i0 * c.heads + slot) * p.map.os1 + p.map.off;
+    quant_window<DT, decltype(bits)::value, ASYM, LPG4, true>(p, is_v ? p.x1 : p.x, is_v ? c.v_words : c.k_words, is_v ? c.v_scale : c.k_scale,
+                                                              is_v ? c.v_zp : c.k_zp, i0, i1, p.strided ? blockIdx.y : blockIdx.x, out_base,
+                                                              lds_stage[threadIdx.x >> 6]);
+  });
+}
+
+template <int DT, bool ASYM> void launch_classes(const RowsParams &p, const ClassOuts &t, int lpg4, dim3 grid, hipStream_t st) {
+  if (lpg4 == 1) hipLaunchKernelGGL((quant_pack_classes_kernel<DT, ASYM, 1>), grid, dim3(256), 0, st, p, t);
+  else if (lpg4 == 2) hipLaunchKernelGGL((quant_pack_classes_kernel<DT, ASYM, 2>), grid, dim3(256), 0, st, p, t);
+  else hipLaunchKernelGGL((quant_pack_classes_kernel<DT, ASYM, 4>), grid, dim3(256), 0, st, p, t);
+}
+
 template <int DT, int BITS, bool ASYM>
 int launch_lpg(const RowsParams &p, int lpg, dim3 grid, hipStream_t st) {
   if (lpg >= 4) {   // groups of >= 32 channels: 4 octets per lane, 1024 octets per workgroup
@@ -530,4 +556,46 @@ extern "C" int varq_quant_pack_rows2(const void *x0, const void *x1, int x_dtype
   VARQ_CHECK_ARG(n_rows == 0 || x1, "quant_pack_rows2: null pointer");
   return quant_pack_rows_launch("quant_pack_rows2", x0, x1, x_dtype, n_rows, c, group, bits, asym, eps, host_rowmap, slot,
                                 words0, scale0, zp0, words1, scale1, zp1, stream);
+}
+
+extern "C" int varq_quant_pack_classes(const void *k, const void *v, int x_dtype, int layout, int B, int H, int64_t n, int c, int group, int asym,
+                                       float eps, const varq_kv_class *host_classes, int n_classes, int64_t Lmax, int64_t start, void *stream) {
+  VARQ_CHECK_ARG(x_dtype >= 0 && x_dtype <= 2, "quant_pack_classes: bad dtype %d", x_dtype);
+  VARQ_CHECK_ARG(layout == VARQ_LAYOUT_BHLC || layout == VARQ_LAYOUT_BLHC, "quant_pack_classes: layout must be VARQ_LAYOUT_BHLC (0) or VARQ_LAYOUT_BLHC (1), got %d", layout);
+  VARQ_CHECK_ARG(B >= 0 && H > 0 && n >= 0 && start >= 0 && start + n <= Lmax && c > 0, "quant_pack_classes: bad sizes");
+  if ((int64_t)B * n == 0) return VARQ_OK;
+  ClassOuts t;
+  VARQ_CHECK_ARG((k || v) && varq_class_outs(host_classes, n_classes, asym != 0, t), "quant_pack_classes: incomplete or repeated classes, or no input");
+  const int c8 = c / 8;
+  const bool two = k && v, strided = layout == VARQ_LAYOUT_BLHC && H > 1;
+  const int64_t tiles = (n * c8 + 1023) / 1024;
+  if ((group != 32 && group != 64 && group != 128) || c % group || (strided && varq_log2_exact(c8) < 0) || n * H * c >= (1ll << 31) || H > 65535 ||
+      (int64_t)B * 2 > 65535 || tiles > 65535)
+    return varq_set_error(VARQ_ERR_UNSUPPORTED, "quant_pack_classes: no kernel for c=%d group=%d or a tensor of this size", c, group);
+  RowsParams p = {};
+  p.x = k; p.x1 = v;
+  p.c8 = c8; p.c8_shift = varq_log2_exact(c8);
+  p.strided = strided;
+  p.in_s0 = (int64_t)H * n * c;
+  p.in_s1 = strided ? c : n * c;
+  p.in_s2 = strided ? (int64_t)H * c : c;
+  p.map.n0 = B; p.map.n1 = H; p.map.n2 = n; p.map.os1 = Lmax; p.map.os2 = 1; p.map.off = start; p.map.slot_dim = 1;
+  p.nseg = c / group;
+  p.eps = eps;
+  p.octets_per_pair = n * c8;
+  dim3 grid((unsigned)tiles, (unsigned)H, (unsigned)(two ? 2 * B : B));
+  if (strided) grid = dim3((unsigned)H, (unsigned)tiles, grid.z);
+  hipStream_t st = (hipStream_t)stream;
+  const int lpg4 = group / 32;
+#define VARQ_DT(T)                                                    \
+  do {                                                                \
+    if (asym) launch_classes<T, true>(p, t, lpg4, grid, st);          \
+    else launch_classes<T, false>(p, t, lpg4, grid, st);              \
+  } while (0)
+  if (x_dtype == VARQ_F32) VARQ_DT(VARQ_F32);
+  else if (x_dtype == VARQ_BF16) VARQ_DT(VARQ_BF16);
+  else VARQ_DT(VARQ_F16);
+#undef VARQ_DT
+  VARQ_CHECK_LAUNCH("quant_pack_classes");
+  return VARQ_OK;
 }

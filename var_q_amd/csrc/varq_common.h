@@ -4,6 +4,7 @@
 #include <stdint.h>
 #include <stdio.h>
 #include <stdarg.h>
+#include <type_traits>
 #include "../../include/varq.h"
 
 #define VARQ_WAVE 64
@@ -29,6 +30,37 @@ struct RowMap {
   int64_t os0, os1, os2, off;
   int slot_dim;
 };
+
+// The bit-width classes of a mixed cache, 8, 4 and 2 bits: where the tokens of their heads go.  A width that the
+// cache does not have has no slot table.
+struct ClassOut {
+  int32_t *k_words, *v_words;
+  float *k_scale, *k_zp, *v_scale, *v_zp;
+  const int32_t *slot;       // [H]: packed head of a head, -1: not of this class
+  int64_t heads;
+};
+struct ClassOuts { ClassOut c[3]; };
+// f(bits, class, packed head) for the class of head h (uniform for the workgroup)
+template <class F> __device__ __forceinline__ void in_class_of_head(const ClassOuts &t, int h, F &&f) {
+  const int s8 = t.c[0].slot ? t.c[0].slot[h] : -1, s4 = t.c[1].slot ? t.c[1].slot[h] : -1, s2 = t.c[2].slot ? t.c[2].slot[h] : -1;
+  if (s8 >= 0) f(std::integral_constant<int, 8>{}, t.c[0], s8);
+  else if (s4 >= 0) f(std::integral_constant<int, 4>{}, t.c[1], s4);
+  else if (s2 >= 0) f(std::integral_constant<int, 2>{}, t.c[2], s2);
+}
+// The table from the caller's classes; false where they are incomplete.
+static inline bool varq_class_outs(const varq_kv_class *host, int n, bool asym, ClassOuts &t) {
+  t = {};
+  if (!host || n < 1 || n > 3) return false;
+  for (int i = 0; i < n; ++i) {
+    const varq_kv_class &c = host[i];
+    if ((c.bits != 2 && c.bits != 4 && c.bits != 8) || c.heads <= 0 || !c.slot || !c.k_words || !c.v_words || !c.k_scale || !c.v_scale) return false;
+    if (asym && (!c.k_zp || !c.v_zp)) return false;
+    ClassOut &o = t.c[c.bits == 8 ? 0 : c.bits == 4 ? 1 : 2];
+    if (o.slot) return false;
+    o = {c.k_words, c.v_words, c.k_scale, c.k_zp, c.v_scale, c.v_zp, c.slot, c.heads};
+  }
+  return true;
+}
 
 static inline RowMap varq_dense_rowmap(int64_t n_rows) {
   RowMap m;

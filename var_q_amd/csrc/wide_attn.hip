@@ -31,6 +31,7 @@ struct ExpandParams {
   AttnParams a;
   char *tiles;
   int n_tiles, kg_shift, vg_shift;   // log2 of the channels per scale group
+  int places;                        // heads of the tile buffer per batch entry where head_map places them there (0: see the kernel)
 };
 
 template <int BITS> __device__ __forceinline__ void load_codes(const u32 *row, int oct, float (&f)[8]) {
@@ -63,7 +64,10 @@ __global__ __launch_bounds__(256) void expand_tiles_kernel(ExpandParams e) {
   const int tile = blockIdx.x, bh = blockIdx.y, tid = threadIdx.x;
   const int b = bh / p.Hkv, hs = bh - b * p.Hkv;
   const int64_t kv_row0 = b * p.kv_bs + hs * p.kv_hs;
-  char *const out = e.tiles + ((int64_t)bh * e.n_tiles + tile) * (2 * kHalfTile<D>);
+  // (the place of the head that a packed head of a mixed-width cache serves; the others attend what they hold in
+  // the order that it is packed)
+  const int place = e.places ? b * e.places + p.head_map[hs] : bh;
+  char *const out = e.tiles + ((int64_t)place * e.n_tiles + tile) * (2 * kHalfTile<D>);
   if constexpr (CHAN) {
     if (tid < kMaxSegments) seg_end[tid] = p.seg_end[tid];
     __syncthreads();
@@ -527,7 +531,7 @@ template <int D, bool F16> void launch_wide_shape(const WideParams &e, int n_wgs
 
 namespace varq_attn {
 
-WidePlan plan_wide(int64_t bh, int Lq, int Lk, int D, int cus) {
+WidePlan plan_wide(int64_t bh, int Lq, int Lk, int D, int cus, bool share) {
   WidePlan w;
   const int64_t blocks = bh * ((Lq + 255) / 256), tiles = (Lk + BN - 1) / BN;
   w.tile_bytes = (size_t)bh * (size_t)tiles * (size_t)(2 * BN * D * 2);
@@ -540,7 +544,7 @@ WidePlan plan_wide(int64_t bh, int Lq, int Lk, int D, int cus) {
   const double tile_us = D == 128 ? 1.9 : 1.2, fixed_us = 6.0;
   const int64_t rounds = blocks / cus, left = (blocks - rounds * cus) * tiles;
   int64_t n = rounds ? cus : left / 4 < cus ? left / 4 : cus;
-  if (n > 1 && left) {
+  if (share && n > 1 && left) {
     const double whole = (double)tiles * tile_us + fixed_us;
     const double pieces = (double)(n + blocks - rounds * cus);   // at most this many partial results, written and read at 5 TB/s
     const double shared = (double)left / (double)n * tile_us + 2.0 * fixed_us + 5.0 + 2.0 * pieces * 256.0 * D * 4.0 / 5.0e6;
@@ -553,8 +557,9 @@ WidePlan plan_wide(int64_t bh, int Lq, int Lk, int D, int cus) {
   return w;
 }
 
-void launch_expand(const AttnParams &p, int D, int bits, int k_group, int v_group, bool chan, char *tiles, hipStream_t st) {
+void launch_expand(const AttnParams &p, int D, int bits, int k_group, int v_group, bool chan, char *tiles, hipStream_t st, bool place) {
   ExpandParams e;
+  e.places = place ? p.Hq : 0;
   e.a = p;
   e.tiles = tiles;
   e.n_tiles = (p.Lk + BN - 1) / BN;

@@ -38,13 +38,14 @@ class PackedKVCache:
         self.B, self.H, self.Lmax, self.D, self.group = B, H, Lmax, D, group_size
         self.per_head_bits, self.symmetric, self.eps = per_head, symmetric, eps
         self.len = 0
-        self.concurrent_classes = True   # attend(): one stream per bit-width class ...
-        # ... once the call is large enough: forking and joining the streams costs the host about
-        # 50 us, more than the classes of a small step gain by running side by side (measured on
-        # the 13-scale schedule at B=8, H=16: side streams win from 576 queries over 1 497 keys
-        # on).  While a graph is being recorded there is no such cost and the streams are always used.
+        self.concurrent_classes = True   # attend(): all bit-width classes in one launch (False: one after the other).
+        # Exact codes have no such launch; there the classes run on one stream each, once the call is
+        # large enough: forking and joining the streams costs the host about 50 us, more than the
+        # classes of a small step gain by running side by side (measured on the 13-scale schedule at
+        # B=8, H=16: side streams win from 576 queries over 1 497 keys on).  While a graph is being
+        # recorded there is no such cost and the streams are always used.
         self.concurrent_min_flops = 4e10
-        self.splits = 0                  # attend() on one stream: shares of a query block's keys (0 = library's choice)
+        self.splits = 0                  # attend(): shares of a query block's keys (0 = library's choice)
         self._side = self._fork = self._join = None
         self.classes: List[_BitClass] = [
             _BitClass(b, [h for h in range(H) if per_head[h] == b], B, H, Lmax, D, group_size, device)
@@ -155,28 +156,29 @@ class PackedKVCache:
             return _lib.host().attn(q, c.k_words, c.k_scale, c.k_zp if asym else None, c.v_words, c.v_scale, c.v_zp if asym else None,
                                     c.bits, c.bits, self.len, softmax_scale, kv_limit, None, out, self.splits, 'BHLc', exact_codes,
                                     out_layout)
+        if self.concurrent_classes and not exact_codes:
+            return _lib.host().cache_attend(self._native, self.len, q, softmax_scale, kv_limit, out, self.splits, out_layout)
         if out is None:
             B_, H_, Lq_, D_ = q.shape
             out = torch.empty((B_, Lq_, H_, D_) if out_layout == 'BLHc' else q.shape, dtype=q.dtype, device=q.device)
         asym = not self.symmetric
-        many = len(self.classes) > 1
         # side streams for the bit-width classes only where the call is large enough to gain from
         # them (or a graph is being recorded); small calls stay on the caller's stream and skip
         # every stream lookup
         side = None
-        if many and self.concurrent_classes and (
+        if self.concurrent_classes and (
                 4.0 * q.shape[0] * q.shape[1] * q.shape[2] * self.len * self.D >= self.concurrent_min_flops
                 or torch.cuda.is_current_stream_capturing()):
             side = self._side_streams(q.device)
             main = torch.cuda.current_stream(q.device)
             self._fork.record(main)
-        splits = 1 if many and self.concurrent_classes else self.splits   # classes side by side fill the device already;
-        for i, c in enumerate(self.classes):                              # the same rule on one stream, so both ways add up alike
+        splits = 1 if self.concurrent_classes else self.splits   # classes side by side fill the device already;
+        for i, c in enumerate(self.classes):                     # the same rule on one stream, so both ways add up alike
             # classes cover disjoint heads and disjoint rows of `out`: with side streams their
             # launches share the GPU instead of queueing behind each other half-empty
             args = (q, c.k_words, c.k_scale, c.k_zp if asym else None, c.v_words, c.v_scale, c.v_zp if asym else None,
                     c.bits, c.bits, self.len, softmax_scale)
-            kw = dict(kv_limit=kv_limit, head_map=c.head_map if many else None, out=out, splits=splits, exact_codes=exact_codes,
+            kw = dict(kv_limit=kv_limit, head_map=c.head_map, out=out, splits=splits, exact_codes=exact_codes,
                       out_layout=out_layout)
             if side and i:
                 stream = side[i - 1]
