@@ -1092,14 +1092,6 @@ __device__ __forceinline__ void attend_block(const AttnParams &p, int bh, int ou
     }
     __syncthreads();   // the one barrier per tile
   }
-
-  // ---- epilogue -------------------------------------------------------------------
-#pragma unroll
-  for (int s = 0; s < NSVA; ++s) r_run[s] += __shfl_xor(r_run[s], 32, 64);
-  // rows 4..6 of racc are registers 0..2 of the upper lane half, rows 0..3 registers 0..3 of the lower
-  // (DEQ: the denominator is row 0, the sum of the weights against the row of ones)
-  const float l_sum = DEQ ? l_part + __shfl_xor(l_part, 32, 64) : __shfl(racc[0] + racc[1] + racc[2], col + 32, 64);
-  const float inv = l_sum > 0.f ? 1.0f / l_sum : 0.f;
   // from there on (a wavefront without queries: from the start) the wavefront only helps with staging and
   // widening, at the same barrier count as the others
   for (; tile < n_tiles; ++tile) {
@@ -1109,6 +1101,14 @@ __device__ __forceinline__ void attend_block(const AttnParams &p, int bh, int ou
     __syncthreads();
   }
   if (!wave_live) return;
+
+  // ---- epilogue -------------------------------------------------------------------
+#pragma unroll
+  for (int s = 0; s < NSVA; ++s) r_run[s] += __shfl_xor(r_run[s], 32, 64);
+  // rows 4..6 of racc are registers 0..2 of the upper lane half, rows 0..3 registers 0..3 of the lower
+  // (DEQ: the denominator is row 0, the sum of the weights against the row of ones)
+  const float l_sum = DEQ ? l_part + __shfl_xor(l_part, 32, 64) : __shfl(racc[0] + racc[1] + racc[2], col + 32, 64);
+  const float inv = l_sum > 0.f ? 1.0f / l_sum : 0.f;
   float rq[NSVA];
 #pragma unroll
   for (int s = 0; s < NSVA; ++s) rq[s] = DEQ ? 0.f : __shfl(racc[s], col, 64) + r_run[s];
@@ -1155,14 +1155,6 @@ struct BlockOf {
     const int groups = (p.bh_total + 7) >> 3;   // pairs of an XCD
     int grp = slot / p.q_tiles;
     qt = slot % p.q_tiles;
-  }
-};
-
-template <int D, int BITS, int GK, int GV, bool CHAN, int NWV = 8, int WPS = 2, bool EXACT = false, bool F16 = false>
-__global__ __launch_bounds__(NWV * 64, WPS) void fused_attn_kernel(AttnParams p) {
-  const BlockOf k(p);
-  if (k.pair >= p.bh_total) return;
-  attend_block<D, BITS, GK, GV, CHAN, NWV, EXACT, F16>(p, k.pair, k.pair, k.qt, k.split);
     if (p.kv_limit && p.q_tiles > 1) {
       // Under a key limit that grows with the query (the block-causal rule) the query tiles of a pair differ in
       // length: the pairs whose workgroups are resident together (64 on an XCD at two per compute unit) start
@@ -1173,6 +1165,14 @@ __global__ __launch_bounds__(NWV * 64, WPS) void fused_attn_kernel(AttnParams p)
       grp = first + r % n;
     }
     pair = p.kv_hs == 1 && p.kv_ts > 1 ? xcd * groups + grp : grp * 8 + xcd;
+  }
+};
+
+template <int D, int BITS, int GK, int GV, bool CHAN, int NWV = 8, int WPS = 2, bool EXACT = false, bool F16 = false>
+__global__ __launch_bounds__(NWV * 64, WPS) void fused_attn_kernel(AttnParams p) {
+  const BlockOf k(p);
+  if (k.pair >= p.bh_total) return;
+  attend_block<D, BITS, GK, GV, CHAN, NWV, EXACT, F16>(p, k.pair, k.pair, k.qt, k.split);
 }
 
 // A cache whose heads have several bit-widths, all classes in one launch: pair k of the launch belongs to the
