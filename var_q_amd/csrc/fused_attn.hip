@@ -272,22 +272,26 @@ template <int G> __device__ __forceinline__ int k_octet(int ch, int h) {
 template <int D, int BITS, int GK, int GV, bool CHAN> struct AttnForms {
   static constexpr bool kHasExact = !CHAN && D / GK == 1 && D / GV == 1 && D == 128 && BITS != 8;
 };
-template <int D, int BITS, int GK, int GV, bool CHAN, bool EXACT = false> struct AttnLds {
+// ONE: no launch of the kernel has more than one tile of keys (Lk <= 64), so there is one of each buffer.
+template <int D, int BITS, int GK, int GV, bool CHAN, bool EXACT = false, bool ONE = false> struct AttnLds {
   static_assert(!EXACT || AttnForms<D, BITS, GK, GV, CHAN>::kHasExact, "no exact-code form of this kernel");
   static constexpr bool kDeq = !EXACT;
   static constexpr int WPR = D * BITS / 32;
   static constexpr int RSV = WPR + 1;       // packed V row stride (words): odd, bank spread
   static constexpr bool kFoldSv = !kDeq && (D / GV == 1);   // one V group: its scale rides inside the logits
-  static constexpr int kParFloats = ((D / GK) + (kFoldSv ? 1 : 2) * (D / GV)) * 64;
+  static constexpr int kParFloats = CHAN ? 0 : ((kDeq ? 0 : D / GK) + (kFoldSv ? 1 : 2) * (D / GV)) * 64;
+  // Widened tiles and what only the widening reads (packed V and, where the kernel dequantizes, the per-key
+  // parameters) have two buffers, what the exact-code form reads while it attends three.
+  static constexpr int kBufs = ONE ? 1 : 2, kParBufs = kDeq ? kBufs : 3;
   static constexpr int RSR = 64 + 8;        // stride (bf16) of the rows feeding the extra PV MFMA
   static constexpr int KXS = D + 8;         // stride (bf16) of a widened K row: 16-byte rows, bank spread
-  static constexpr int kKx = 0;             // widened K, two tiles
-  static constexpr int kVp = kKx + 2 * 64 * KXS * 2;
-  static constexpr int kVt = (kVp + 3 * 64 * RSV * 4 + 15) / 16 * 16;
-  static constexpr int kKz = kVt + 2 * D * (64 + 8) * 2;          // rank-1 operands of S^T, 2 x 16 bytes per key and group
+  static constexpr int kKx = 0;             // widened K
+  static constexpr int kVp = kKx + kBufs * 64 * KXS * 2;
+  static constexpr int kVt = (kVp + kBufs * 64 * RSV * 4 + 15) / 16 * 16;
+  static constexpr int kKz = kVt + kBufs * D * (64 + 8) * 2;          // rank-1 operands of S^T, 2 x 16 bytes per key and group
   static constexpr int kWz = kKz + (kDeq ? 0 : 3 * (D / GK) * 64 * 32);   // 8 rows per slot for the extra PV MFMA
-  static constexpr int kPar = kWz + 3 * 8 * RSR * 2;
-  static constexpr int kFlag = kPar + 3 * kParFloats * 4;
+  static constexpr int kPar = kWz + (kDeq ? 0 : 3 * 8 * RSR * 2);
+  static constexpr int kFlag = kPar + kParBufs * kParFloats * 4;
   static constexpr int kBytes = kFlag + 16;
 };
 
@@ -306,7 +310,7 @@ template <int D, int BITS, int GK, int GV, bool CHAN, bool EXACT = false> struct
 // fp16 autocast of scripts/inference_multi_VAR.py:123); dequantizing kernels only.
 // One workgroup's work: query tile qt of packed pair bh (= batch * p.Hkv + packed head), share `split` of its
 // keys; partial results go to the rows of pair `out_pair`.
-template <int D, int BITS, int GK, int GV, bool CHAN, int NWV, bool EXACT, bool F16>
+template <int D, int BITS, int GK, int GV, bool CHAN, int NWV, bool EXACT, bool F16, bool ONE = false>
 __device__ __forceinline__ void attend_block(const AttnParams &p, int bh, int out_pair, int qt, int split) {
   static_assert(!(F16 && EXACT), "the exact-code form builds bf16 images of the codes");
   static_assert(!CHAN || (GK == D && GV == D), "per-channel tables go with the single-group kernels");
@@ -332,24 +336,27 @@ __device__ __forceinline__ void attend_block(const AttnParams &p, int bh, int ou
   constexpr int NCH = D / 16;               // contraction chunks of QK^T
   constexpr int NDB = D / 32;               // 32-row blocks of O^T
   constexpr int VTS = BN + 8;               // V^T row stride (bf16 elements)
-  using L = AttnLds<D, BITS, GK, GV, CHAN, EXACT>;
+  using L = AttnLds<D, BITS, GK, GV, CHAN, EXACT, ONE>;
+  constexpr int NB = L::kBufs, NPB = L::kParBufs;
 
   // Pipelined LDS buffers (one workgroup barrier per tile):
-  //   packed V and the per-key parameters of tile t live in slot t % 3, the
-  //   widened K and the widened V^T of tile t in slot t % 2.
+  //   packed V, the widened K and the widened V^T of tile t live in slot t % 2 (packed V is
+  //   read one iteration before its tile is attended, so tile t+2 may take its slot then), like
+  //   the per-key parameters where only the widening reads them; in the exact-code form those
+  //   live in slot t % 3.
   // While tile t is being attended, K and V of tile t+1 are widened (K straight
   // from the registers it was loaded into one iteration earlier, once per
   // workgroup, so the eight wavefronts share the work) and packed V of tile t+2 is
   // written from its registers.
   extern __shared__ __attribute__((aligned(16))) unsigned char lds_raw[];
-  uint16_t *const lds_kx = reinterpret_cast<uint16_t *>(lds_raw + L::kKx);  // [2][BN][KXS] widened K codes (MFMA A operands)
-  u32 *const lds_vp = reinterpret_cast<u32 *>(lds_raw + L::kVp);          // [3][BN][RSV]
-  uint16_t *const lds_vt = reinterpret_cast<uint16_t *>(lds_raw + L::kVt);  // [2][D][VTS]  raw V codes, transposed
+  uint16_t *const lds_kx = reinterpret_cast<uint16_t *>(lds_raw + L::kKx);  // [NB][BN][KXS] widened K codes (MFMA A operands)
+  u32 *const lds_vp = reinterpret_cast<u32 *>(lds_raw + L::kVp);          // [NB][BN][RSV]
+  uint16_t *const lds_vt = reinterpret_cast<uint16_t *>(lds_raw + L::kVt);  // [NB][D][VTS]  raw V codes, transposed
   u32x4_t *const lds_kz = reinterpret_cast<u32x4_t *>(lds_raw + L::kKz);  // [3][NSK][BN][2] rank-1 A operands (per lane half)
   // [3][8][RSR] bf16 rows of the extra PV MFMA: row s < NSV = vzp_c + kOff of group s,
   // rows 4..6 = the three bf16 pieces of 1/vs of group 0, row 7 = zeros
   uint16_t *const lds_wz = reinterpret_cast<uint16_t *>(lds_raw + L::kWz);
-  float *const lds_par = reinterpret_cast<float *>(lds_raw + L::kPar);    // [3][L::kParFloats]
+  float *const lds_par = reinterpret_cast<float *>(lds_raw + L::kPar);    // [NPB][L::kParFloats]
   int *const lds_flag = reinterpret_cast<int *>(lds_raw + L::kFlag);      // [3] tile+1 if that tile has a zero-point remainder
   // CHAN: the tables of this head for every segment, [nseg][4][D] fp32, filled once in the
   // prologue, as the widening steps use them: row 0 = kMul * sk and row 1 = (zk + kOff) / kMul in
@@ -362,7 +369,7 @@ __device__ __forceinline__ void attend_block(const AttnParams &p, int bh, int ou
   // parameter block of one tile: ck [NSK][BN]; vr [NSV][BN]; sv [NSV][BN] unless folded
   constexpr bool FOLD_SV = L::kFoldSv;
   constexpr int RSR = L::RSR;
-  constexpr int P_CK = 0, P_VR = NSK * BN, P_SV = P_VR + NSV * BN;
+  constexpr int P_CK = 0, P_VR = (DEQ ? 0 : NSK) * BN, P_SV = P_VR + NSV * BN;
   constexpr int P_VZ = P_VR;   // DEQ: per (V group, key) the zero-point image; P_SV holds the scale image
 
   const int b = bh / p.Hkv, hs = bh % p.Hkv;
@@ -432,6 +439,7 @@ __device__ __forceinline__ void attend_block(const AttnParams &p, int bh, int ou
     kv_end = lds_maxlim;
   }
   int n_tiles = (kv_end + BN - 1) / BN;
+  if constexpr (ONE) n_tiles = min(n_tiles, 1);
   // segment ends in LDS: indexing the kernel arguments with a run-time index would move
   // the whole argument block to scratch memory (literal indices only, for the same reason)
   __shared__ int lds_seg_end[kMaxSegments];
@@ -572,7 +580,7 @@ __device__ __forceinline__ void attend_block(const AttnParams &p, int bh, int ou
   // registers -> LDS slot of `tile` (packed words as they are, parameters precombined)
   auto stage = [&](int tile) {
     const int sl = tile % 3;
-    u32 *vp = lds_vp + sl * BN * RSV;
+    u32 *vp = lds_vp + tile % NB * BN * RSV;
 #pragma unroll
     for (int i = 0; i < LPT; ++i) {
       const int piece = tid + i * NT;
@@ -584,7 +592,7 @@ __device__ __forceinline__ void attend_block(const AttnParams &p, int bh, int ou
         for (int j = 0; j < 4; ++j) vp[key * RSV + w4 + j] = vreg[i][j] ^ VX;
       }
     }
-    float *par = lds_par + sl * L::kParFloats;
+    float *par = lds_par + tile % NPB * L::kParFloats;
     const int key = tid & 63, seg = tid >> 6, vseg = NW - 1 - seg;
     // |ck| is kept away from zero so that log2(vs)/ck stays finite for a constant group
     auto ck_of = [&](float ks) {
@@ -664,8 +672,8 @@ __device__ __forceinline__ void attend_block(const AttnParams &p, int bh, int ou
   // packed V of `tile` -> V^T bf16: a work item is 2 adjacent keys x 8 channels (one
   // packed word of each key), written as 8 dwords of the transposed tile
   auto widen_v = [&](int tile) {
-    const u32 *vp = lds_vp + (tile % 3) * BN * RSV;
-    uint16_t *vt = lds_vt + (tile & 1) * D * VTS;
+    const u32 *vp = lds_vp + (tile % NB) * BN * RSV;
+    uint16_t *vt = lds_vt + (tile % NB) * D * VTS;
     widen_cursor(tile);
     const bool one_seg = !CHAN || tile_in_one_segment(tile);
     // (where the tile has fewer items than the workgroup has threads, the upper wavefronts take
@@ -702,7 +710,7 @@ __device__ __forceinline__ void attend_block(const AttnParams &p, int bh, int ou
         }
       } else if constexpr (DEQ) {
         // code images -> values of the two keys, (raw - z') * s' in fp32, rounded to bf16
-        const float *pt = lds_par + (tile % 3) * L::kParFloats + (oct * 8 / GV) * BN + kp2 * 2;
+        const float *pt = lds_par + (tile % NPB) * L::kParFloats + (oct * 8 / GV) * BN + kp2 * 2;
         const float2 z2 = *reinterpret_cast<const float2 *>(pt + P_VZ), s2 = *reinterpret_cast<const float2 *>(pt + P_SV);
 #pragma unroll
         for (int j = 0; j < 8; ++j) pr[j] = pack_io_rne<F16>((f0[j] - z2.x) * s2.x, (f1[j] - z2.y) * s2.y);
@@ -715,7 +723,7 @@ __device__ __forceinline__ void attend_block(const AttnParams &p, int bh, int ou
   // packed K of `tile` (in kreg) -> widened bf16 rows: each piece holds OPQ octets
   // of one key, every octet becomes one 16-byte MFMA A operand
   auto widen_k = [&](int tile) {
-    uint16_t *kx = lds_kx + (tile & 1) * BN * KXS;
+    uint16_t *kx = lds_kx + (tile % NB) * BN * KXS;
     constexpr int OPQ = KPW * 4 / BITS;       // octets per piece
     widen_cursor(tile);
     const bool one_seg = !CHAN || tile_in_one_segment(tile);
@@ -766,7 +774,7 @@ __device__ __forceinline__ void attend_block(const AttnParams &p, int bh, int ou
   // ---- prologue: V tiles 0 and 1 staged, K and V of tile 0 widened, K of tile 1 and V
   //      of tile 2 in registers ------------------------------------------------------------
   if (tid < 3) lds_flag[tid] = 0;
-  for (int i = tid; i < 3 * RSR; i += NT) lds_wz[((i / RSR) * 8 + 7) * RSR + i % RSR] = 0;   // the all-zero row of each slot
+  for (int i = tid; i < (DEQ ? 0 : 3 * RSR); i += NT) lds_wz[((i / RSR) * 8 + 7) * RSR + i % RSR] = 0;   // the all-zero row of each slot
   if (n_tiles > 0) { prefetch_k(0); prefetch(0); }
   // the query values, behind the first tile's requests and ahead of the table loads: one
   // round trip for all three
@@ -817,9 +825,9 @@ __device__ __forceinline__ void attend_block(const AttnParams &p, int bh, int ou
 
   auto begin_tile = [&](int tile) {
     t0 = tile_base + tile * BN;
-    kx = lds_kx + (tile & 1) * BN * KXS;
-    par = lds_par + (tile % 3) * L::kParFloats;
-    vt = lds_vt + (tile & 1) * D * VTS;
+    kx = lds_kx + (tile % NB) * BN * KXS;
+    par = lds_par + (tile % NPB) * L::kParFloats;
+    vt = lds_vt + (tile % NB) * D * VTS;
     kz = lds_kz + (tile % 3) * NSK * BN * 2;
     wz = lds_wz + (tile % 3) * 8 * RSR;
     tile_rem = lds_flag[tile % 3] == tile + 1;   // tagged with the tile, so stale tags never match
@@ -1168,11 +1176,11 @@ struct BlockOf {
   }
 };
 
-template <int D, int BITS, int GK, int GV, bool CHAN, int NWV = 8, int WPS = 2, bool EXACT = false, bool F16 = false>
+template <int D, int BITS, int GK, int GV, bool CHAN, int NWV = 8, int WPS = 2, bool EXACT = false, bool F16 = false, bool ONE = false>
 __global__ __launch_bounds__(NWV * 64, WPS) void fused_attn_kernel(AttnParams p) {
   const BlockOf k(p);
   if (k.pair >= p.bh_total) return;
-  attend_block<D, BITS, GK, GV, CHAN, NWV, EXACT, F16>(p, k.pair, k.pair, k.qt, k.split);
+  attend_block<D, BITS, GK, GV, CHAN, NWV, EXACT, F16, ONE>(p, k.pair, k.pair, k.qt, k.split);
 }
 
 // A cache whose heads have several bit-widths, all classes in one launch: pair k of the launch belongs to the
@@ -1344,47 +1352,49 @@ void allow_lds(const void *kernel, int bytes, bool (&configured)[64]) {
   if (dev >= 0) configured[dev] = true;
 }
 
-template <int D, int BITS, int GK, int GV, bool CHAN, int NWV, int WPS = 2, bool EXACT = false, bool F16 = false>
+template <int D, int BITS, int GK, int GV, bool CHAN, int NWV, int WPS = 2, bool EXACT = false, bool F16 = false, bool ONE = false>
 void launch_shape(const AttnParams &p, hipStream_t st) {
   // (the per-channel tables take LDS by the number of segments of the launch)
-  constexpr int lds_base = (AttnLds<D, BITS, GK, GV, CHAN, EXACT>::kBytes + 15) / 16 * 16, lds_seg = CHAN ? kChanTableRows * D * 4 : 0;
+  constexpr int lds_base = (AttnLds<D, BITS, GK, GV, CHAN, EXACT, ONE>::kBytes + 15) / 16 * 16, lds_seg = CHAN ? kChanTableRows * D * 4 : 0;
   constexpr int lds_max = lds_base + kMaxSegments * lds_seg;
   static_assert(lds_max <= 160 * 1024, "LDS budget");
   const int lds_bytes = lds_base + p.nseg * lds_seg;
   static bool configured[64] = {false};
-  allow_lds(reinterpret_cast<const void *>(&fused_attn_kernel<D, BITS, GK, GV, CHAN, NWV, WPS, EXACT, F16>), lds_max, configured);
+  allow_lds(reinterpret_cast<const void *>(&fused_attn_kernel<D, BITS, GK, GV, CHAN, NWV, WPS, EXACT, F16, ONE>), lds_max, configured);
   const int bh_pad = (p.bh_total + 7) / 8 * 8;
   dim3 grid((unsigned)(bh_pad * p.q_tiles * p.nsplit));
-  hipLaunchKernelGGL((fused_attn_kernel<D, BITS, GK, GV, CHAN, NWV, WPS, EXACT, F16>), grid, dim3(NWV * 64), lds_bytes, st, p);
+  hipLaunchKernelGGL((fused_attn_kernel<D, BITS, GK, GV, CHAN, NWV, WPS, EXACT, F16, ONE>), grid, dim3(NWV * 64), lds_bytes, st, p);
   if (p.nsplit > 1) launch_combine<D, F16>(p, st);
+}
+
+// The workgroups at D=64, F16 or not.
+template <int BITS, int GK, int GV, bool CHAN, bool F16> void launch_d64(const AttnParams &p, hipStream_t st) {
+  // More (batch, head) pairs than compute units, at most four wavefronts of queries each:
+  // workgroups of four wavefronts (same arithmetic, same results).  Also for one or two
+  // wavefronts of queries: the wavefronts without queries share the staging and the widening
+  // of the tiles, which is what such a workgroup spends its time on (workgroups of two
+  // wavefronts, also two to a compute unit by their LDS, took 20-35 % longer on 16-64 queries).
+  // Such a workgroup is a chain of loads, barriers and short computations, so what counts is how many
+  // are resident: three to a compute unit, and with a single tile of keys and one of each buffer
+  // four or more.  [64,n,16,64] fp16, 8-bit codes with per-channel tables, us, two resident -> now: n=1 of 1 key
+  // 9.4 -> 7.2, 9 x 14 12.4 -> 8.8, 25 x 55 15.4 -> 11.4, 64 x 155 27.4 -> 26.3.
+  if (p.Lq <= 128 && p.bh_total > device_cus()) {
+    if (p.Lk <= BN && p.nsplit == 1) launch_shape<64, BITS, GK, GV, CHAN, 4, 4, false, F16, true>(p, st);
+    else launch_shape<64, BITS, GK, GV, CHAN, 4, 3, false, F16>(p, st);
+    return;
+  }
+  // The kernels at D=64 fit 128 registers at the price of 24-48 bytes of spills,
+  // and two resident workgroups per compute unit hide each other's prologue and barriers
+  // (8-15 % faster than one workgroup at 140 registers).
+  launch_shape<64, BITS, GK, GV, CHAN, 8, 4, false, F16>(p, st);
 }
 
 template <int D, int BITS, int GK, int GV, bool CHAN = false>
 void launch(const AttnParams &p, hipStream_t st) {
   if constexpr (D == 64) {
-    // fp16 operands (the VAR path; every VAR model has head dim 64)
-    if (p.f16) {
-      if (p.Lq <= 128 && p.bh_total > device_cus()) launch_shape<D, BITS, GK, GV, CHAN, 4, 2, false, true>(p, st);
-      else launch_shape<D, BITS, GK, GV, CHAN, 8, 4, false, true>(p, st);
-      return;
-    }
-  }
-  if constexpr (D == 64) {
-    // more (batch, head) pairs than compute units, at most four wavefronts of queries each:
-    // workgroups of four wavefronts (same arithmetic, same results).  Also for one or two
-    // wavefronts of queries: the wavefronts without queries share the staging and the widening
-    // of the tiles, which is what such a workgroup spends its time on (workgroups of two
-    // wavefronts, also two to a compute unit by their LDS, took 20-35 % longer on 16-64 queries).
-    if (p.Lq <= 128 && p.bh_total > device_cus()) {
-      launch_shape<D, BITS, GK, GV, CHAN, 4>(p, st);
-      return;
-    }
-  }
-  if constexpr (D == 64) {
-    // The kernels at D=64 fit 128 registers at the price of 24-48 bytes of spills,
-    // and two resident workgroups per compute unit hide each other's prologue and barriers
-    // (8-15 % faster than one workgroup at 140 registers).
-    launch_shape<D, BITS, GK, GV, CHAN, 8, 4>(p, st);
+    // fp16 operands (the VAR path; every VAR model has head dim 64) or bf16 ones
+    if (p.f16) launch_d64<BITS, GK, GV, CHAN, true>(p, st);
+    else launch_d64<BITS, GK, GV, CHAN, false>(p, st);
   } else {
     if constexpr (AttnForms<D, BITS, GK, GV, CHAN>::kHasExact) {
       if (p.exact_codes) {
@@ -1423,8 +1433,8 @@ void launch_classes_shape(const AttnParams &p, const ClassTable &t, hipStream_t 
 template <int D, int G> void launch_classes(const AttnParams &p, const ClassTable &t, hipStream_t st) {
   if constexpr (D == 64) {
     const bool four = p.Lq <= 128 && p.bh_total > device_cus();
-    if (p.f16) { if (four) launch_classes_shape<D, G, 4, 2, true>(p, t, st); else launch_classes_shape<D, G, 8, 4, true>(p, t, st); }
-    else { if (four) launch_classes_shape<D, G, 4, 2, false>(p, t, st); else launch_classes_shape<D, G, 8, 4, false>(p, t, st); }
+    if (p.f16) { if (four) launch_classes_shape<D, G, 4, 3, true>(p, t, st); else launch_classes_shape<D, G, 8, 4, true>(p, t, st); }
+    else { if (four) launch_classes_shape<D, G, 4, 3, false>(p, t, st); else launch_classes_shape<D, G, 8, 4, false>(p, t, st); }
   } else {
     launch_classes_shape<D, G, 8, 2, false>(p, t, st);
   }
