@@ -228,6 +228,17 @@ int varq_dequant_steps(const int32_t *words, const float *scale, const float *zp
                        int B, int H, int64_t capacity, int c, int bits, int tokens_first, void *out, int out_dtype, void *stream);
 
 /*
+ * One step of such a quantizer and the whole cache dequantized behind it (VAR_Q/quant.py:226-230: quant,
+ * cache, dequant_all), in one launch where the sizes allow: varq_quant_pack of x ([B, H, n, c], or
+ * [B, n, H, c] with tokens_first) into tokens host_seg_end[nseg-2].. of `words` and row nseg-1 of the
+ * tables, then varq_dequant_steps over all nseg steps.  The step's tokens are the last segment's.
+ * Workspace: varq_quant_workspace_bytes of the step.  x, scale, zp, out: 16-byte aligned.
+ */
+int varq_quant_step_dequant(const void *x, int x_dtype, int B, int H, int n, int c, int tokens_first, int bits, int asym, float eps,
+                            int32_t *words, int64_t capacity, float *scale, float *zp, int nseg, const int32_t *host_seg_end,
+                            void *out, int out_dtype, void *workspace, size_t workspace_bytes, void *stream);
+
+/*
  * Fused dequant flash-attention (no counterpart in the reference, which
  * dequantizes the whole cache to fp32 and calls an external attention backend:
  * VAR_Q/quant.py:216-230, VAR/models/basic_var.py:156-162,

@@ -34,6 +34,9 @@ SYMBOLS = {
                              c_int, c_int, POINTER(c_int64), c_void_p, c_int, c_void_p]),
     'varq_dequant_steps': (c_int, [c_void_p, c_void_p, c_void_p, c_int, POINTER(c_int32), c_int, c_int, c_int64, c_int, c_int, c_int,
                                    c_void_p, c_int, c_void_p]),
+    'varq_quant_step_dequant': (c_int, [c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_float,
+                                        c_void_p, c_int64, c_void_p, c_void_p, c_int, POINTER(c_int32),
+                                        c_void_p, c_int, c_void_p, c_size_t, c_void_p]),
     'varq_fused_attn': (c_int, [c_void_p, c_void_p,
                                 c_void_p, c_void_p, c_void_p, c_int, c_int,
                                 c_void_p, c_void_p, c_void_p, c_int, c_int,

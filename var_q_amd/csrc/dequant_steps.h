@@ -1,0 +1,123 @@
+// Dequantizing the cache of a stepwise quantizer: shared by the launch that does only that (dequant.hip) and the
+// one that quantizes a step as well (quant_general.hip).
+#pragma once
+#include "varq_common.h"
+
+namespace varq_deq {
+
+template <int ODT> __device__ __forceinline__ void store8(void *out, int64_t elem, const float (&f)[8], int n_valid) {
+  if (ODT == VARQ_F32) {
+    float *o = reinterpret_cast<float *>(out) + elem;
+    if (n_valid == 8) {
+      reinterpret_cast<float4 *>(o)[0] = make_float4(f[0], f[1], f[2], f[3]);
+      reinterpret_cast<float4 *>(o)[1] = make_float4(f[4], f[5], f[6], f[7]);
+    } else {
+      for (int j = 0; j < n_valid; ++j) o[j] = f[j];
+    }
+  } else {
+    uint16_t *o = reinterpret_cast<uint16_t *>(out) + elem;
+    if (ODT == VARQ_BF16 && n_valid == 8) {
+      // hardware round-to-nearest-even conversion, two values per instruction
+      typedef __bf16 bf2 __attribute__((ext_vector_type(2)));
+      typedef float f2 __attribute__((ext_vector_type(2)));
+      u32 w[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const f2 v = {f[2 * j], f[2 * j + 1]};
+        w[j] = __builtin_bit_cast(u32, __builtin_convertvector(v, bf2));
+      }
+      *reinterpret_cast<uint4 *>(o) = make_uint4(w[0], w[1], w[2], w[3]);
+      return;
+    }
+    uint16_t h[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) h[j] = (ODT == VARQ_BF16) ? f32_to_bf16_rne(f[j]) : f32_to_f16_rne(f[j]);
+    if (n_valid == 8) {
+      *reinterpret_cast<uint4 *>(o) = make_uint4(h[0] | ((u32)h[1] << 16), h[2] | ((u32)h[3] << 16),
+                                                 h[4] | ((u32)h[5] << 16), h[6] | ((u32)h[7] << 16));
+    } else {
+      for (int j = 0; j < n_valid; ++j) o[j] = h[j];
+    }
+  }
+}
+
+// The cache of a stepwise quantizer, one table of scales per step.  A pair is a (batch, head) (heads first)
+// or a batch entry (tokens first); its tokens lie one after the other in words and output, `octs` octets each,
+// so an octet's place is its number and only its table depends on the token.  HBM-bound by its output: per
+// element 4 bytes (or 2) written and bits/8 read; the tables stay in the caches.  (Reading the scales
+// expanded over the tokens instead, four more bytes per element, took 8.9 against 5.9 us at [8,680,30,64],
+// and the expansion had to be written first.)
+struct StepParams {
+  const u32 *words;
+  const float *scale, *zp;
+  void *out;
+  int64_t pair_words, pair_octs;   // words of a pair in the buffer, octets of a pair that are read
+  int64_t out_pair_octs;           // octets of a pair in the output
+  int octs, H, c, nseg;
+  int head_in_pair;                // 1: heads first, the pair's head is pair % H
+  int64_t row;                     // H * c: floats of a table
+  int seg_oct[16];                 // first octet of a pair that is past segment s
+};
+
+// Block `block` of pair `pair`: NT threads, U octets each.
+template <int ODT, int BITS, int NT, int U>
+__device__ __forceinline__ void dequant_steps_block(const StepParams &p, int64_t pair, int block) {
+  __shared__ int seg_oct[16];
+  if (threadIdx.x < 16) seg_oct[threadIdx.x] = p.seg_oct[threadIdx.x];
+  __syncthreads();
+  const u32 *words = p.words + pair * p.pair_words;
+  const float *scale = p.scale + (p.head_in_pair ? (pair % p.H) * p.c : 0);
+  const float *zp = p.zp ? p.zp + (p.head_in_pair ? (pair % p.H) * p.c : 0) : nullptr;
+  const int o0 = block * (NT * U) + threadIdx.x;
+  u32 w0[U], w1[U];
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    const int o = min(o0 + u * NT, (int)p.pair_octs - 1);
+    w1[u] = 0;
+    if (BITS == 8) { const uint2 t = *reinterpret_cast<const uint2 *>(words + 2 * (int64_t)o); w0[u] = t.x; w1[u] = t.y; }
+    else if (BITS == 4) w0[u] = words[o];
+    else w0[u] = words[o >> 1] >> ((o & 1) * 16);
+  }
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    const int o = o0 + u * NT;
+    if (o >= (int)p.pair_octs) return;
+    int seg = 0;
+    while (seg + 1 < p.nseg && o >= seg_oct[seg]) ++seg;
+    const int64_t t = seg * p.row + (int)((u32)o % (u32)p.octs) * 8;
+    const float4 sa = *reinterpret_cast<const float4 *>(scale + t), sb = *reinterpret_cast<const float4 *>(scale + t + 4);
+    const float s[8] = {sa.x, sa.y, sa.z, sa.w, sb.x, sb.y, sb.z, sb.w};
+    float f[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j)
+      f[j] = (float)(int)(BITS == 8 ? __builtin_amdgcn_sbfe((int)(j < 4 ? w0[u] : w1[u]), 8 * (j & 3), 8) : __builtin_amdgcn_sbfe((int)w0[u], BITS * j, BITS));
+    if (zp) {
+      const float4 za = *reinterpret_cast<const float4 *>(zp + t), zb = *reinterpret_cast<const float4 *>(zp + t + 4);
+      const float z[8] = {za.x, za.y, za.z, za.w, zb.x, zb.y, zb.z, zb.w};
+#pragma unroll
+      for (int j = 0; j < 8; ++j) f[j] = (f[j] - z[j]) * s[j];
+    } else {
+#pragma unroll
+      for (int j = 0; j < 8; ++j) f[j] = f[j] * s[j];
+    }
+    store8<ODT>(p.out, (pair * p.out_pair_octs + o) * 8, f, 8);
+  }
+}
+
+// The launch parameters for `nseg` steps that end at host_seg_end[..]; false where the octets of a pair exceed
+// 31 bits.  p.out_pair_octs is that of an output which holds these tokens and no others.
+inline bool set_steps(StepParams &p, const int32_t *words, const float *scale, const float *zp, int nseg, const int32_t *host_seg_end, int H,
+                      int64_t capacity, int c, int bits, bool tokens_first, void *out) {
+  const int64_t tokens = nseg ? host_seg_end[nseg - 1] : 0;
+  p.words = reinterpret_cast<const u32 *>(words); p.scale = scale; p.zp = zp; p.out = out;
+  p.H = H; p.c = c; p.nseg = nseg; p.row = (int64_t)H * c;
+  p.head_in_pair = tokens_first ? 0 : 1;
+  p.octs = (tokens_first ? H * c : c) / 8;
+  if (tokens * p.octs >= (1ll << 31) - 2048) return false;
+  for (int s = 0; s < 16; ++s) p.seg_oct[s] = (s < nseg ? host_seg_end[s] : (int)tokens) * p.octs;
+  p.pair_octs = p.out_pair_octs = tokens * p.octs;
+  p.pair_words = capacity * p.octs * 8 * bits / 32;
+  return true;
+}
+
+}  // namespace varq_deq

@@ -203,6 +203,33 @@ PyObject *quant_step(PyObject *const *a, Py_ssize_t n_args) {
   Py_RETURN_NONE;
 }
 
+// quant_step_dequant(asym, bits, eps, token_dim, x, buf, tab, ztab | None, earlier seg_ends, out dtype code)
+// -> the dequantized cache; the step goes behind the earlier ones, its scales into the next row of the tables.
+PyObject *quant_step_dequant(PyObject *const *a) {
+  const bool asym = truth(a[0]);
+  const int64_t bits = integer(a[1]), d = integer(a[3]), code = integer(a[9]);
+  const at::Tensor &x = gpu(a[4], "x"), &buf = gpu(a[5], "buffer"), &tab = gpu(a[6], "scale table");
+  const at::Tensor *ztab = maybe(a[7], "zero-point table");
+  ASSERT(PyList_Check(a[8]) && PyList_GET_SIZE(a[8]) < 16 && (d == 1 || d == 2), "quant_step_dequant: 1..16 steps");
+  const int k = (int)PyList_GET_SIZE(a[8]);
+  int32_t ends[16];
+  for (int i = 0; i < k; ++i) ends[i] = (int32_t)integer(PyList_GET_ITEM(a[8], i));
+  ASSERT(x.dim() == 4 && x.is_contiguous() && buf.dim() == 4 && buf.is_contiguous() && buf.scalar_type() == at::kInt && tab.is_contiguous(), "quant_step_dequant: operands");
+  const int64_t B = x.size(0), H = x.size(3 - d), n = x.size(d), c = x.size(3), start = k ? ends[k - 1] : 0;
+  ends[k] = (int32_t)(start + n);
+  ASSERT((!asym || ztab) && buf.size(3) * 32 == c * bits && start + n <= buf.size(d) && buf.size(0) == B && buf.size(3 - d) == H, "quant_step_dequant: buffers");
+  ASSERT((k + 1) * H * c <= tab.numel() && tab.scalar_type() == at::kFloat && (!ztab || ztab->sizes() == tab.sizes()), "quant_step_dequant: tables");
+  const int64_t sh[4] = {B, x.size(1), x.size(2), c};
+  const c10::DeviceGuard guard(x.device());
+  const size_t ws_bytes = std::max<size_t>(varq_quant_workspace_bytes(sh, d == 1 ? 0b0011 : 0b0101), 8);
+  const at::Tensor ws = empty({(int64_t)ws_bytes}, at::kByte, x);
+  const at::Tensor out = d == 1 ? empty({B, start + n, H, c}, dtype_of((int)code), x) : empty({B, H, start + n, c}, dtype_of((int)code), x);
+  check(varq_quant_step_dequant(x.data_ptr(), dtype_code(x), (int)B, (int)H, (int)n, (int)c, d == 1, (int)bits, asym, (float)real(a[2]), ptr<int32_t>(buf), buf.size(d),
+                                ptr<float>(tab), asym ? ptr<float>(ztab) : nullptr, k + 1, ends, out.data_ptr(), (int)code, ws.data_ptr(), ws_bytes, stream_of(x)),
+        "varq_quant_step_dequant");
+  return wrap(out);
+}
+
 // ---- pack / unpack of int8 codes ----------------------------------------------------------------
 // pack(codes, bits) -> words
 PyObject *pack(PyObject *const *a) {
@@ -601,7 +628,7 @@ PyObject *set_error(PyObject *, PyObject *e) {
 
 #define FIXED(name, n) {#name, (PyCFunction)(void (*)(void))fixed<name, n>, METH_FASTCALL, nullptr}
 PyMethodDef g_methods[] = {
-    FIXED(quant_rows, 5), FIXED(quant_shared, 6), FIXED(pack, 2), FIXED(unpack, 3), FIXED(dequant, 6), FIXED(dequant_steps, 8), FIXED(attn, 18), FIXED(attn_channel, 17),
+    FIXED(quant_rows, 5), FIXED(quant_shared, 6), FIXED(pack, 2), FIXED(unpack, 3), FIXED(dequant, 6), FIXED(dequant_steps, 8), FIXED(quant_step_dequant, 10), FIXED(attn, 18), FIXED(attn_channel, 17),
     FIXED(cache_attend, 8), FIXED(cache_append, 5), FIXED(cache_prepare, 9),
     {"quant_step", (PyCFunction)(void (*)(void))varying<quant_step>, METH_FASTCALL, nullptr},
     {"set_error", set_error, METH_O, nullptr},

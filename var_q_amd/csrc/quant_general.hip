@@ -10,8 +10,9 @@
 // min/max are exactly associative, so the result does not depend on the order
 // in which partial results meet.  Channel counts that are not a multiple of 8 and
 // rows wider than 512 channels take scalar kernels with ordered-integer atomics.
-#include "varq_common.h"
+#include "dequant_steps.h"
 #include <mutex>
+#include <type_traits>
 
 #ifndef VARQ_GEN_NRO_MIN
 #define VARQ_GEN_NRO_MIN 256
@@ -23,7 +24,16 @@
 #define VARQ_GEN_BLOCKS 2048
 #endif
 
+using namespace varq_deq;
+
 namespace {
+
+// Octets of earlier tokens up to which they share the step's launch (see quant_one_step_kernel): beyond, a launch of
+// their own with all of a compute unit's wavefronts and registers is the better way through memory.  Symmetric /
+// affine (whose quantizing workgroups' LDS leaves fewer of them resident), two launches -> one, us: 0.8 million 24.5 ->
+// 18.5 / 1.0 million 24.4 -> 20.8; 2.0 20.3 -> 17.1 / 1.9 25.7 -> 27.3; 3.8 40.2 -> 42.3 / 8.2 33 -> 42; 5.1 42.5 -> 52.6.
+constexpr int64_t kStepMostSym = 3ll << 20, kStepMostAsym = 3ll << 19;
+constexpr int kStepOctets = 1024;   // octets of earlier tokens that a workgroup dequantizes
 
 // Order-preserving float <-> uint map so that integer atomicMin/Max implement
 // float min/max.
@@ -310,9 +320,11 @@ __global__ __launch_bounds__(256) void finalize_tiled_kernel(GenParams p, int Z,
 // Quantizes and stores one octet (column `col`) of row `row`: s, r, z the scale, RN(1 / scale) and the
 // zero-point of the octet's groups (one per channel or one), plain whether all scales allow the exact
 // quotient shortcut.
-template <int NV>
+// also(codes): what else the caller wants from them.
+struct Nothing { __device__ __forceinline__ void operator()(const int (&)[8]) const {} };
+template <int NV, class F = Nothing>
 __device__ __forceinline__ void store_octet(const GenParams &p, int64_t row, int col, const float (&v)[8], const float (&s)[NV], const float (&r)[NV],
-                                            const float (&z)[NV], bool plain) {
+                                            const float (&z)[NV], bool plain, F &&also = F()) {
   const float qmin = (float)p.qmin, qmax = (float)p.qmax;
   const u32 mask = (1u << p.bits) - 1u;
   int q[8];
@@ -328,6 +340,7 @@ __device__ __forceinline__ void store_octet(const GenParams &p, int64_t row, int
 #pragma unroll
     for (int j = 0; j < 8; ++j) q[j] = (int)__builtin_amdgcn_fmed3f(rintf(v[j] / s[j % NV]) + z[j % NV], qmin, qmax);
   }
+  also(q);
   const int64_t orow = out_row32(p, row);
   if (p.codes || p.bits == 8) {
     const u32 lo = (q[0] & 0xff) | ((q[1] & 0xff) << 8) | ((q[2] & 0xff) << 16) | ((u32)q[3] << 24);
@@ -400,14 +413,14 @@ struct OnePlan {
   int blocks;                   // nko * tilesQ
 };
 
-template <int DT, bool ASYM, bool KEEPC, int NT, int NI>
-__global__ __launch_bounds__(NT) void quant_one_kernel(GenParams p, OnePlan pl) {
+// also(row, col, codes, scales, zero-points): what else is made of an octet once it is quantized
+template <int DT, bool ASYM, bool KEEPC, int NT, int NI, class F>
+__device__ __forceinline__ void quant_one_block(const GenParams &p, const OnePlan &pl, F &&also) {
   constexpr int NV = KEEPC ? 8 : 1, MAXG = 2048;
   __shared__ float lds_mx[MAXG];
   __shared__ float lds_mn[ASYM ? MAXG : 1];
   __shared__ float par_s[MAXG], par_r[MAXG];
   __shared__ float par_z[ASYM ? MAXG : 1];
-  take_second(p);
   // the slices of a block on one XCD (ids congruent mod 8 share an L2): they share the rows' cache lines
   const int bid = blockIdx.x, slice = (bid >> 3) % pl.slices, blk = (bid >> 3) / pl.slices * 8 + (bid & 7);
   if (blk >= pl.blocks) return;
@@ -506,8 +519,50 @@ __global__ __launch_bounds__(NT) void quant_one_kernel(GenParams p, OnePlan pl) 
     if (i >= pl.steps || j >= pl.RR) continue;
     float v[8];
     raw[i].widen(v);
-    store_octet<NV>(p, row_of(j), col, v, s, r, z, plain);
+    const int64_t row = row_of(j);
+    store_octet<NV>(p, row, col, v, s, r, z, plain, [&](const int (&codes)[8]) { also(row, col, codes, s, z); });
   }
+}
+template <int DT, bool ASYM, bool KEEPC, int NT, int NI>
+__global__ __launch_bounds__(NT) void quant_one_kernel(GenParams p, OnePlan pl) {
+  take_second(p);
+  quant_one_block<DT, ASYM, KEEPC, NT, NI>(p, pl, [](int64_t, int, const auto &, const auto &, const auto &) {});
+}
+
+// A step of a quantizer with a scale per (head, channel), and the whole cache dequantized behind it, in one launch:
+// the first workgroups quantize the step and write its dequantized values from the codes in their registers, the
+// others dequantize the earlier tokens.  The values are those of the two launches.  Bound by launches and by
+// the chain of loads and barriers in the quantizing workgroups, under which the others now work.  8 bits, fp16 to fp32,
+// two launches -> one, us: [8,n,30,64] 1 token behind none 8.3 -> 6.0, 36 behind 55 11.0 -> 8.6, 256 behind 424 24.5 -> 18.5.
+struct StepOut {
+  StepParams earlier;             // the tokens before this step (none: nseg = 0)
+  int64_t inner, delta, off;      // input row r is output row r + r / inner * delta + off
+  int odt, q_blocks, pair_blocks; // workgroups that quantize; workgroups of a pair of `earlier`
+};
+template <int DT, bool ASYM, int NT, int NI>
+__global__ __launch_bounds__(NT) void quant_one_step_kernel(GenParams p, OnePlan pl, StepOut o) {
+  auto typed = [&](auto &&f) __attribute__((always_inline)) {
+    if (o.odt == VARQ_F32) f(std::integral_constant<int, VARQ_F32>{});
+    else if (o.odt == VARQ_BF16) f(std::integral_constant<int, VARQ_BF16>{});
+    else f(std::integral_constant<int, VARQ_F16>{});
+  };
+  if ((int)blockIdx.x >= o.q_blocks) {
+    const int b = blockIdx.x - o.q_blocks, pair = b / o.pair_blocks, block = b - pair * o.pair_blocks;
+    typed([&](auto t) __attribute__((always_inline)) {
+      constexpr int ODT = decltype(t)::value, U = kStepOctets / NT;
+      if (p.bits == 8) dequant_steps_block<ODT, 8, NT, U>(o.earlier, pair, block);
+      else if (p.bits == 4) dequant_steps_block<ODT, 4, NT, U>(o.earlier, pair, block);
+      else dequant_steps_block<ODT, 2, NT, U>(o.earlier, pair, block);
+    });
+    return;
+  }
+  quant_one_block<DT, ASYM, true, NT, NI>(p, pl, [&](int64_t row, int col, const auto &q, const auto &s, const auto &z) __attribute__((always_inline)) {
+    float f[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) f[j] = ASYM ? ((float)q[j] - z[j]) * s[j] : (float)q[j] * s[j];
+    const int64_t orow = row + (int64_t)((u32)row / (u32)o.inner) * o.delta + o.off;
+    typed([&](auto t) __attribute__((always_inline)) { store8<decltype(t)::value>(o.earlier.out, orow * p.c + col * 8, f, 8); });
+  });
 }
 
 // ---- phase A, any c: one thread per element --------------------------------
@@ -706,6 +761,13 @@ template <int DT> void run_one(const GenParams &p, const OnePlan &pl, int thread
   else { if (p.keepc) launch_one<DT, false, true>(p, pl, threads, st); else launch_one<DT, false, false>(p, pl, threads, st); }
 }
 
+template <int DT, bool ASYM> void launch_one_step(const GenParams &p, const OnePlan &pl, int threads, const StepOut &o, unsigned blocks, hipStream_t st) {
+  constexpr int NI = DT == VARQ_F32 ? 8 : 16;
+  if (threads == 1024) hipLaunchKernelGGL((quant_one_step_kernel<DT, ASYM, 1024, NI>), dim3(blocks), dim3(1024), 0, st, p, pl, o);
+  else if (pl.steps <= 2) hipLaunchKernelGGL((quant_one_step_kernel<DT, ASYM, 256, 2>), dim3(blocks), dim3(256), 0, st, p, pl, o);
+  else hipLaunchKernelGGL((quant_one_step_kernel<DT, ASYM, 256, NI>), dim3(blocks), dim3(256), 0, st, p, pl, o);
+}
+
 size_t plan_workspace_bytes(const Plan &pl, int64_t n_groups) {
   return (size_t)n_groups * (2 + 2 * (size_t)pl.Z) * sizeof(float);
 }
@@ -798,7 +860,8 @@ namespace {
 int quant_pack_impl(const void *x, const void *x1, int x_dtype, const int64_t *host_shape4, int reduce_mask, int bits,
                     int asym, float eps, int32_t *words, int8_t *codes, float *scale, float *zp,
                     int32_t *words1, int8_t *codes1, float *scale1, float *zp1,
-                    const int64_t *host_out_map, void *workspace, size_t workspace_bytes, void *stream) {
+                    const int64_t *host_out_map, void *workspace, size_t workspace_bytes, void *stream,
+                    StepOut *step = nullptr, int64_t step_pairs = 0) {
   VARQ_CHECK_ARG(host_shape4, "quant_pack: null shape");
   const int64_t *s = host_shape4;
   VARQ_CHECK_ARG(s[0] >= 0 && s[1] >= 0 && s[2] >= 0 && s[3] > 0 && s[3] <= (1 << 20), "quant_pack: bad shape");
@@ -865,6 +928,20 @@ int quant_pack_impl(const void *x, const void *x1, int x_dtype, const int64_t *h
   OnePlan one;
   int threads;
   if (tiled && make_one_plan(s, reduce_mask, x_dtype == VARQ_F32 ? 8 : 16, x1 ? 2 : 1, one, threads)) {
+    if (step) {
+      step->q_blocks = (one.blocks + 7) / 8 * 8 * one.slices;
+      step->pair_blocks = (int)((step->earlier.pair_octs + kStepOctets - 1) / kStepOctets);
+      const int64_t blocks = step->q_blocks + step_pairs * step->pair_blocks;
+      if (blocks < (1ll << 31)) {
+        const unsigned n = (unsigned)blocks;
+        if (x_dtype == VARQ_F32) { if (asym) launch_one_step<VARQ_F32, true>(p, one, threads, *step, n, st); else launch_one_step<VARQ_F32, false>(p, one, threads, *step, n, st); }
+        else if (x_dtype == VARQ_BF16) { if (asym) launch_one_step<VARQ_BF16, true>(p, one, threads, *step, n, st); else launch_one_step<VARQ_BF16, false>(p, one, threads, *step, n, st); }
+        else { if (asym) launch_one_step<VARQ_F16, true>(p, one, threads, *step, n, st); else launch_one_step<VARQ_F16, false>(p, one, threads, *step, n, st); }
+        VARQ_CHECK_LAUNCH("quant_step_dequant");
+        step->q_blocks = -1;   // done
+        return VARQ_OK;
+      }
+    }
     if (x1) { p.x1 = x1; p.scale1 = scale1; p.zp1 = zp1; p.words1 = words1; p.codes1 = codes1; }
     if (x_dtype == VARQ_F32) run_one<VARQ_F32>(p, one, threads, st);
     else if (x_dtype == VARQ_BF16) run_one<VARQ_BF16>(p, one, threads, st);
@@ -905,6 +982,37 @@ extern "C" int varq_quant_pack2(const void *x0, const void *x1, int x_dtype, con
   VARQ_CHECK_ARG(x1, "quant_pack2: null second tensor");
   return quant_pack_impl(x0, x1, x_dtype, host_shape4, reduce_mask, bits, asym, eps, words0, codes0, scale0, zp0,
                          words1, codes1, scale1, zp1, host_out_map, workspace, workspace_bytes, stream);
+}
+
+// Quantizes a step into its tokens of the cache buffer and dequantizes the whole cache: in one launch where the step
+// takes one by itself and the cache is not much more work than it (see kStepMostSym), in the launches of the two calls otherwise.
+extern "C" int varq_quant_step_dequant(const void *x, int x_dtype, int B, int H, int n, int c, int tokens_first, int bits, int asym, float eps,
+                                       int32_t *words, int64_t capacity, float *scale, float *zp, int nseg, const int32_t *host_seg_end,
+                                       void *out, int out_dtype, void *workspace, size_t workspace_bytes, void *stream) {
+  VARQ_CHECK_ARG(x && words && scale && out && host_seg_end && (!asym || zp), "quant_step_dequant: null pointer");
+  VARQ_CHECK_ARG(nseg >= 1 && nseg <= 16 && B > 0 && H > 0 && n > 0 && c > 0 && c % 8 == 0 && c <= (1 << 20),
+                 "quant_step_dequant: bad sizes (1..16 steps, whole octets of channels)");
+  VARQ_CHECK_ARG((bits == 2 || bits == 4 || bits == 8) && (c * bits) % 32 == 0, "quant_step_dequant: bits must be 2, 4 or 8 and rows whole words");
+  VARQ_CHECK_ARG(out_dtype >= 0 && out_dtype <= 2, "quant_step_dequant: bad output dtype %d", out_dtype);
+  VARQ_CHECK_ARG((((uintptr_t)x | (uintptr_t)scale | (uintptr_t)zp | (uintptr_t)out) & 15) == 0 && ((uintptr_t)words & 7) == 0, "quant_step_dequant: misaligned operand");
+  for (int s = 0, prev = 0; s < nseg; prev = host_seg_end[s++])
+    VARQ_CHECK_ARG(host_seg_end[s] >= prev, "quant_step_dequant: segment ends must increase");
+  const int64_t start = nseg > 1 ? host_seg_end[nseg - 2] : 0, tokens = host_seg_end[nseg - 1], per = tokens_first ? H : 1, row = (int64_t)H * c;
+  VARQ_CHECK_ARG(tokens - start == n && tokens <= capacity, "quant_step_dequant: the last step has %d tokens and the buffer room for %lld", n, (long long)capacity);
+  const int64_t shape[4] = {B, tokens_first ? n : H, tokens_first ? H : n, c}, map[3] = {n * per, (capacity - n) * per, start * per};
+  StepOut o;
+  const int64_t pairs = tokens_first ? B : (int64_t)B * H;
+  const bool fits = set_steps(o.earlier, words, scale, asym ? zp : nullptr, nseg - 1, host_seg_end, H, capacity, c, bits, tokens_first, out) &&
+                    pairs * start * o.earlier.octs <= (asym ? kStepMostAsym : kStepMostSym);
+  o.earlier.out_pair_octs = tokens * o.earlier.octs;
+  o.inner = map[0]; o.delta = (tokens - n) * per; o.off = map[2];
+  o.odt = out_dtype; o.q_blocks = 0; o.pair_blocks = 0;
+  float *const s = scale + (nseg - 1) * row, *const z = asym ? zp + (nseg - 1) * row : nullptr;
+  if (const int e = quant_pack_impl(x, nullptr, x_dtype, shape, tokens_first ? 0b0011 : 0b0101, bits, asym, eps, words, nullptr, s, z, nullptr, nullptr,
+                                    nullptr, nullptr, map, workspace, workspace_bytes, stream, fits ? &o : nullptr, pairs))
+    return e;
+  if (o.q_blocks < 0) return VARQ_OK;
+  return varq_dequant_steps(words, scale, asym ? zp : nullptr, nseg, host_seg_end, B, H, capacity, c, bits, tokens_first, out, out_dtype, stream);
 }
 
 // ---- the entry point that allocates nothing ------------------------------------------

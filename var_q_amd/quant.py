@@ -487,6 +487,14 @@ class VAR_Q:
         price is memory: 4 bytes per cached element (up to 8 while the buffer has doubled), i.e.
         two to four times an unquantized bf16 cache, resident until the quantizer is deleted --
         172 MB per tensor at [2,16,10521,128].  `dequant_all()` itself always recomputes everything."""
+        if not self.keep_dequantized:
+            place = self._fast_place(item)
+            if place is not None and place[2] % 8 == 0 and (self._seg_ends[-1] if self._seg_ends else 0) == place[4] and item.data_ptr() % 16 == 0:
+                # the shipped rule: step and dequantized cache from one library call (and where the sizes allow, one launch)
+                out = _lib.host().quant_step_dequant(not self.symmetric, self.quant_bits, self.eps, self.dim_cat, item, self._c_item.buf,
+                                                     self._tab_scale, self._tab_zp, self._seg_ends, ops._DT[out_dtype or torch.float32])
+                self._fast_commit(place)
+                return out
         if not self._step_fast(item):
             self.quant(item)
             self.cache()
