@@ -7,7 +7,7 @@ import torch
 
 import varq_oracle as O
 from gpu_util import note
-from var_q_amd import ops
+from var_q_amd import _lib, ops
 
 pytestmark = pytest.mark.gpu
 
@@ -44,3 +44,29 @@ def test_one_launch_edges(dev, shape, dims, dtype):
         assert torch.equal(gs.cpu(), s)
         assert not asym or torch.equal(gz.cpu(), z)
         assert torch.equal(gq.cpu(), O.pack_last_dim(q, bits)[0] if pack else q)
+
+
+@pytest.mark.parametrize('shape,dims,dtype', [
+    ((3, 700, 5, 64), (0, 1), torch.float16),         # 2100 rows per group, few heads: slices of one octet
+    ((3, 700, 5, 72), (0, 1), torch.bfloat16),        # nine octets
+    ((1, 3, 4097, 24), (0, 2), torch.float32),
+    ((2, 2, 2500, 8), (0, 2), torch.bfloat16),        # nothing to slice
+    ((64, 30, 4, 128), (0, 1), torch.float16),
+])
+def test_narrow_slices(dev, shape, dims, dtype):
+    """Few workgroups' worth of columns: 8- and 4-bit codes in slices of one octet, 2-bit codes (two octets to a word)
+    in slices of two, and K and V of a step together, which are enough for wider slices."""
+    test_one_launch_edges(dev, shape, dims, dtype)
+    g = torch.Generator().manual_seed(1)
+    xs = [torch.randn(*shape, generator=g).to(dtype) for _ in range(2)]
+    tok = 1 if dims == (0, 1) else 2
+    H, c = shape[3 - tok], shape[3]
+    for bits in (8, 4, 2):
+        if c * bits % 32:
+            continue
+        pair = [[x.to(dev), torch.zeros(*shape[:3], c * bits // 32, dtype=torch.int32, device=dev), torch.zeros(16, H, c, device=dev), None] for x in xs]
+        note('quant one, two tensors', shape, dims, dtype, bits)
+        _lib.host().quant_step(0b0011 if tok == 1 else 0b0101, bits, False, 1e-12, tok, 0, 2, *pair[0], *pair[1])
+        for x, (_, words, tab, _) in zip(xs, pair):
+            q, s, _ = O.quant_reduce(x, dims, bits, False)
+            assert torch.equal(words.cpu(), O.pack_last_dim(q, bits)[0]) and torch.equal(tab[2].cpu(), s.reshape(H, c))

@@ -710,7 +710,7 @@ bool make_plan(const int64_t *sh, int reduce_mask, int64_t n_groups, Plan &pl) {
 }
 
 // The one-launch plan, or false when a group has too many rows for a workgroup's registers.
-bool make_one_plan(const int64_t *sh, int reduce_mask, int row_steps, int tensors, OnePlan &pl, int &threads) {
+bool make_one_plan(const int64_t *sh, int reduce_mask, int row_steps, int tensors, int bits, bool with_values, OnePlan &pl, int &threads) {
   const int64_t c = sh[3], rows = sh[0] * sh[1] * sh[2];
   if (c % 8 != 0 || c > 512 || rows <= 0 || rows >= (1ll << 31) - 512) return false;
   const Canonical k = canonical(sh, reduce_mask);
@@ -728,6 +728,13 @@ bool make_one_plan(const int64_t *sh, int reduce_mask, int row_steps, int tensor
   while ((1 << rr_shift) < rr) ++rr_shift;
   // column slices (channel dim kept): whole rows while that makes workgroups enough, 64 bytes of a row at least
   pl.c8s_shift = keepc && c8p_shift > 4 ? 4 : c8p_shift;
+  // Narrower slices mean more workgroups and smaller pieces of each row.  32 bytes where that leaves no more than
+  // half of the compute units without one; 16 (a word of 2-bit codes takes 32) where it does not and codes are all
+  // that is stored: K and V [64,n,16,64] fp16, 8 bits, 128 -> 256 workgroups, n = 64 24.9 -> 19.6 us, n = 16 9.9 ->
+  // 8.5; [4,400,24,128] one tensor, 192 -> 384 workgroups 13.5 -> 19.4.  The dequantized values of a step in 32-byte
+  // pieces from as many workgroups take a schedule of [8,n,30,64] from 208 to 227 us.
+  const int narrowest = bits == 2 || with_values ? 1 : 0;
+  const int enough = with_values ? 128 : 160;
   for (;; --pl.c8s_shift) {
     pl.slices = keepc ? (c8 + (1 << pl.c8s_shift) - 1) >> pl.c8s_shift : 1;
     // 256 threads where their rows suffice, 1024 otherwise; the row lanes of a q no more than its rows
@@ -743,8 +750,8 @@ bool make_one_plan(const int64_t *sh, int reduce_mask, int row_steps, int tensor
     pl.tilesQ = (int)((k.Q + (1 << pl.lq_shift) - 1) >> pl.lq_shift);
     pl.blocks = pl.nko * pl.tilesQ;
     const bool fits = pl.steps <= row_steps;
-    if (fits && ((int64_t)pl.blocks * pl.slices * tensors >= 128 || !keepc || pl.c8s_shift <= 1)) return true;
-    if (!keepc || pl.c8s_shift <= 1) return false;
+    if (fits && ((int64_t)pl.blocks * pl.slices * tensors >= enough || !keepc || pl.c8s_shift <= narrowest)) return true;
+    if (!keepc || pl.c8s_shift <= narrowest) return false;
   }
 }
 
@@ -927,7 +934,7 @@ int quant_pack_impl(const void *x, const void *x1, int x_dtype, const int64_t *h
   hipStream_t st = (hipStream_t)stream;
   OnePlan one;
   int threads;
-  if (tiled && make_one_plan(s, reduce_mask, x_dtype == VARQ_F32 ? 8 : 16, x1 ? 2 : 1, one, threads)) {
+  if (tiled && make_one_plan(s, reduce_mask, x_dtype == VARQ_F32 ? 8 : 16, x1 ? 2 : 1, words ? bits : 8, step != nullptr, one, threads)) {
     if (step) {
       step->q_blocks = (one.blocks + 7) / 8 * 8 * one.slices;
       step->pair_blocks = (int)((step->earlier.pair_octs + kStepOctets - 1) / kStepOctets);
