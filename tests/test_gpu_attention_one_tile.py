@@ -1,6 +1,6 @@
-"""Launches of many (batch, head) pairs with at most 128 queries and at most 64 keys (the first steps of a schedule
-at a large batch) run a kernel with one of each buffer; one key more, or more queries, take the pipelined ones.
-The arithmetic is the same, so every pair's output equals bit for bit what the same pair gives in a launch too
+"""Launches of many (batch, head) pairs with at most 128 queries (the first steps of a schedule at a large batch) run a
+kernel with one of each buffer where they have at most 64 keys or more than three pairs to a compute unit; one key more,
+or more queries, take the pipelined ones.  The arithmetic is the same, so every pair's output equals bit for bit what the same pair gives in a launch too
 small for that rule; two pairs are held against the oracle."""
 import math
 
@@ -13,13 +13,14 @@ from test_gpu_attention import _compare
 from var_q_amd import ops
 
 pytestmark = pytest.mark.gpu
-B, H = 19, 17   # 323 pairs: more than compute units, no multiple of 8
+H = 17
 
 
 @pytest.mark.parametrize('Lq,Lk', [(1, 1), (4, 5), (31, 32), (33, 33), (128, 63), (128, 64), (100, 65), (17, 129), (129, 64)])
+@pytest.mark.parametrize('B', [19])   # 323 pairs: more than compute units, no multiple of 8
 @pytest.mark.parametrize('bits,dtype', [(2, 'fp16'), (4, 'bf16'), (8, 'fp16'), (8, 'bf16')])
 @pytest.mark.parametrize('scales', ['g32', 'g64', 'channel'])
-def test_small_steps(dev, Lq, Lk, bits, dtype, scales):
+def test_small_steps(dev, Lq, Lk, bits, dtype, scales, B):
     D, scale = 64, 0.125
     dt = torch.float16 if dtype == 'fp16' else torch.bfloat16
     gen = torch.Generator(device=dev).manual_seed(Lq * 1000 + Lk)
@@ -55,3 +56,11 @@ def test_small_steps(dev, Lq, Lk, bits, dtype, scales):
             args[0] = args[0][:, :, live]
             ref = O.attention_ref(*args, scale, bias[live], dtype=dt)
             _compare(out[b, h][None, None][:, :, live], ref, O.attention_exact(args[0].float(), *args[1:], scale, bias[live]), 'one tile')
+
+
+@pytest.mark.parametrize('Lq,Lk', [(1, 65), (33, 127), (64, 128), (128, 191), (65, 257), (5, 700)])
+@pytest.mark.parametrize('bits,dtype', [(2, 'fp16'), (4, 'bf16'), (8, 'fp16')])
+@pytest.mark.parametrize('scales', ['g32', 'g64', 'channel'])
+def test_more_pairs_than_fit_at_once(dev, Lq, Lk, bits, dtype, scales):
+    """833 pairs: several tiles through the kernel with one of each buffer (2-bit codes in groups: through two)."""
+    test_small_steps(dev, Lq, Lk, bits, dtype, scales, 49)

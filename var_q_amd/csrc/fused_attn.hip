@@ -272,7 +272,8 @@ template <int G> __device__ __forceinline__ int k_octet(int ch, int h) {
 template <int D, int BITS, int GK, int GV, bool CHAN> struct AttnForms {
   static constexpr bool kHasExact = !CHAN && D / GK == 1 && D / GV == 1 && D == 128 && BITS != 8;
 };
-// ONE: no launch of the kernel has more than one tile of keys (Lk <= 64), so there is one of each buffer.
+// ONE: one of each buffer, so that more workgroups are resident; a tile is staged, widened and attended before the
+// next one is staged (see launch_d64 for when that is the better way).
 template <int D, int BITS, int GK, int GV, bool CHAN, bool EXACT = false, bool ONE = false> struct AttnLds {
   static_assert(!EXACT || AttnForms<D, BITS, GK, GV, CHAN>::kHasExact, "no exact-code form of this kernel");
   static constexpr bool kDeq = !EXACT;
@@ -439,7 +440,6 @@ __device__ __forceinline__ void attend_block(const AttnParams &p, int bh, int ou
     kv_end = lds_maxlim;
   }
   int n_tiles = (kv_end + BN - 1) / BN;
-  if constexpr (ONE) n_tiles = min(n_tiles, 1);
   // segment ends in LDS: indexing the kernel arguments with a run-time index would move
   // the whole argument block to scratch memory (literal indices only, for the same reason)
   __shared__ int lds_seg_end[kMaxSegments];
@@ -801,12 +801,14 @@ __device__ __forceinline__ void attend_block(const AttnParams &p, int bh, int ou
     }
   }
   load_q();
-  if (n_tiles > 0) { stage(0); widen_k(0); }
-  if (n_tiles > 1) { prefetch_k(1); prefetch(1); stage(1); }
-  __syncthreads();
-  if (n_tiles > 0) widen_v(0);
-  if (n_tiles > 2) prefetch(2);
-  __syncthreads();
+  if constexpr (!ONE) {
+    if (n_tiles > 0) { stage(0); widen_k(0); }
+    if (n_tiles > 1) { prefetch_k(1); prefetch(1); stage(1); }
+    __syncthreads();
+    if (n_tiles > 0) widen_v(0);
+    if (n_tiles > 2) prefetch(2);
+    __syncthreads();
+  }
 
   // ---- the three phases of one 32-key block, as lambdas over per-tile state --------
   // LDS operands are requested ahead of their use where the registers allow it (the
@@ -832,6 +834,7 @@ __device__ __forceinline__ void attend_block(const AttnParams &p, int bh, int ou
     wz = lds_wz + (tile % 3) * 8 * RSR;
     tile_rem = lds_flag[tile % 3] == tile + 1;   // tagged with the tile, so stale tags never match
     // slot (tile+2)%3 was last read during tile-1 (before the barrier): refill it
+    if constexpr (ONE) return;
     if (tile + 2 < n_tiles) stage(tile + 2);
     if (tile + 3 < n_tiles) prefetch(tile + 3);
   };
@@ -1081,8 +1084,7 @@ __device__ __forceinline__ void attend_block(const AttnParams &p, int bh, int ou
   // wavefronts still need.  A whole sequence of 680 tokens in ten steps, [8,680,16,64] fp16: a quarter of
   // the workgroups' key blocks; with the order of the query tiles (BlockOf) append and attention 47.5 -> 39.7 us.
   const int wave_tiles = wave_live ? min(n_tiles, (max(wave_end - tile_base, 0) + BN - 1) / BN) : 0;
-  int tile = 0;
-  for (; tile < wave_tiles; ++tile) {
+  auto attend = [&](int tile) {
     begin_tile(tile);
     const bool half_tile = wave_end - t0 <= 32;
 #pragma unroll
@@ -1096,8 +1098,25 @@ __device__ __forceinline__ void attend_block(const AttnParams &p, int bh, int ou
       }
       softmax(kb);
       pv_mfma(kb, HOIST);
-      if (kb == 0) widen_next(tile);
+      if (!ONE && kb == 0) widen_next(tile);
     }
+  };
+  int tile = 0;
+  if constexpr (ONE) {
+    // one of each buffer: a tile is staged, widened and attended in turn, with the next one's loads in flight
+    for (; tile < n_tiles; ++tile) {
+      if (tile) __syncthreads();   // (the tile before is attended)
+      stage(tile);
+      widen_k(tile);
+      if (tile + 1 < n_tiles) { prefetch_k(tile + 1); prefetch(tile + 1); }
+      __syncthreads();
+      widen_v(tile);
+      __syncthreads();
+      if (tile < wave_tiles) attend(tile);
+    }
+  }
+  for (; tile < wave_tiles; ++tile) {
+    attend(tile);
     __syncthreads();   // the one barrier per tile
   }
   // from there on (a wavefront without queries: from the start) the wavefront only helps with staging and
@@ -1375,11 +1394,16 @@ template <int BITS, int GK, int GV, bool CHAN, bool F16> void launch_d64(const A
   // of the tiles, which is what such a workgroup spends its time on (workgroups of two
   // wavefronts, also two to a compute unit by their LDS, took 20-35 % longer on 16-64 queries).
   // Such a workgroup is a chain of loads, barriers and short computations, so what counts is how many
-  // are resident: three to a compute unit, and with a single tile of keys and one of each buffer
-  // four or more.  [64,n,16,64] fp16, 8-bit codes with per-channel tables, us, two resident -> now: n=1 of 1 key
-  // 9.4 -> 7.2, 9 x 14 12.4 -> 8.8, 25 x 55 15.4 -> 11.4, 64 x 155 27.4 -> 26.3.
+  // are resident: three to a compute unit where tiles are pipelined through two of each buffer (2-bit
+  // codes in groups: four), four with one of each.  A single tile of keys has nothing to pipeline, and
+  // pairs that do not fit the device in one round of three are better off with four: two buffers -> one,
+  // us, [64,n,16,64] (1024 pairs), 8-bit codes with per-channel tables 36 queries x 91 keys 21.7 -> 14.6,
+  // 64 x 155 27.6 -> 19.1, 100 x 600 61.8 -> 47.0, 128 x 2500 206 -> 169; 4 bits in groups of 32 12.4 -> 11.9,
+  // 17.3 -> 15.7, 46.9 -> 43.9, 162 -> 152, 2 bits in groups 10.1 -> 10.6, 13.4 -> 14.2; with 768 pairs 8 bits in
+  // groups 8.2 -> 8.4, 10.8 -> 11.1, with 512 6.8 -> 7.1, 8.9 -> 9.3.
   if (p.Lq <= 128 && p.bh_total > device_cus()) {
-    if (p.Lk <= BN && p.nsplit == 1) launch_shape<64, BITS, GK, GV, CHAN, 4, 4, false, F16, true>(p, st);
+    const bool rounds = (int64_t)p.bh_total * p.nsplit > 3 * device_cus() && (CHAN || BITS != 2);
+    if (p.Lk <= BN || rounds) launch_shape<64, BITS, GK, GV, CHAN, 4, 4, false, F16, true>(p, st);
     else launch_shape<64, BITS, GK, GV, CHAN, 4, 3, false, F16>(p, st);
     return;
   }
