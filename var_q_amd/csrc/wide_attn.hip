@@ -34,26 +34,22 @@ struct ExpandParams {
   int places;                        // heads of the tile buffer per batch entry where head_map places them there (0: see the kernel)
 };
 
-template <int BITS> __device__ __forceinline__ void load_codes(const u32 *row, int oct, float (&f)[8]) {
-  if constexpr (BITS == 8) {
-    const uint2 w = *reinterpret_cast<const uint2 *>(row + 2 * oct);
+// the eight codes of octet `oct` of a packed row, as they lie, and as numbers
+template <int BITS> __device__ __forceinline__ uint2 load_codes(const u32 *row, int oct) {
+  if constexpr (BITS == 8) return *reinterpret_cast<const uint2 *>(row + 2 * oct);
+  else if constexpr (BITS == 4) return make_uint2(row[oct], 0u);
+  else return make_uint2(row[oct >> 1] >> ((oct & 1) * 16), 0u);
+}
+template <int BITS> __device__ __forceinline__ void code_values(uint2 w, float (&f)[8]) {
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      f[j] = (float)(int)__builtin_amdgcn_sbfe((int)w.x, 8 * j, 8);
-      f[4 + j] = (float)(int)__builtin_amdgcn_sbfe((int)w.y, 8 * j, 8);
-    }
-  } else if constexpr (BITS == 4) {
-    const int w = (int)row[oct];
-#pragma unroll
-    for (int j = 0; j < 8; ++j) f[j] = (float)(int)__builtin_amdgcn_sbfe(w, 4 * j, 4);
-  } else {
-    const int w = (int)(row[oct >> 1] >> ((oct & 1) * 16));
-#pragma unroll
-    for (int j = 0; j < 8; ++j) f[j] = (float)(int)__builtin_amdgcn_sbfe(w, 2 * j, 2);
-  }
+  for (int j = 0; j < 8; ++j)
+    f[j] = (float)(int)__builtin_amdgcn_sbfe((int)(BITS == 8 && j >= 4 ? w.y : w.x), BITS * (BITS == 8 ? j & 3 : j), BITS);
 }
 
-// One workgroup = one tile of one (batch, head).  HBM-bound by its writes.
+// One workgroup = one tile of one (batch, head).  HBM-bound by its writes: all codes and per-key parameters of the
+// tile are requested before the first is used, and the segment that a tile's keys belong to is looked up once (key by
+// key, and with each octet's loads behind a check of its key, [2,16,10521,128] took 51 us at 4 bits in groups and 76 at
+// 8 bits with 13 per-channel tables; now 43 and 49, 5.0 and 5.3 TB/s).
 template <int D, int BITS, bool CHAN, bool F16>
 __global__ __launch_bounds__(256) void expand_tiles_kernel(ExpandParams e) {
   constexpr int WPR = D * BITS / 32, NF = D / 16, OCT = D / 8;   // NF: fragments per 32 keys
@@ -68,27 +64,50 @@ __global__ __launch_bounds__(256) void expand_tiles_kernel(ExpandParams e) {
   // the order that it is packed)
   const int place = e.places ? b * e.places + p.head_map[hs] : bh;
   char *const out = e.tiles + ((int64_t)place * e.n_tiles + tile) * (2 * kHalfTile<D>);
+  constexpr int VI = BN / 2 * OCT / 256, KI = BN * OCT / 256;   // items of a thread: two keys' octets of V, one of K
+  const int key0 = tile * BN;
+  auto k_key = [&](int i) {
+    const int item = tid + i * 256, r = item & 15, frag = item >> 6;
+    return key0 + frag / NF * 32 + 8 * (r >> 2) + 4 * (frag & 1) + (r & 3);
+  };
+  auto k_oct = [&](int i) { const int item = tid + i * 256; return (item >> 6) % NF / 2 * 4 + ((item >> 4) & 3); };
+  auto v_key = [&](int i) { return key0 + (tid + i * 256) / OCT * 2; };
+  const int v_oct = tid % OCT;
+  // everything the tile needs is requested before the first use (rows past the end: the last row's)
+  uint2 kc[KI], vc[VI][2];
+  float ks[CHAN ? 1 : KI], kz[CHAN ? 1 : KI], vs[CHAN ? 1 : VI][2], vz[CHAN ? 1 : VI][2];
+  auto request = [&](const u32 *words, const float *scale, const float *zp, int g_shift, int key, int oct, uint2 &code, float &s, float &z) {
+    const int64_t row = kv_row0 + min(key, p.Lk - 1) * p.kv_ts;
+    code = load_codes<BITS>(words + row * WPR, oct);
+    if constexpr (!CHAN) {
+      const int64_t g = row * (D >> g_shift) + (oct * 8 >> g_shift);
+      s = scale[g];
+      z = zp ? zp[g] : 0.f;
+    }
+  };
+#pragma unroll
+  for (int i = 0; i < VI; ++i)
+#pragma unroll
+    for (int n = 0; n < 2; ++n) request(p.v_words, p.v_scale, p.v_zp, e.vg_shift, v_key(i) + n, v_oct, vc[i][n], vs[CHAN ? 0 : i][n], vz[CHAN ? 0 : i][n]);
+#pragma unroll
+  for (int i = 0; i < KI; ++i) request(p.k_words, p.k_scale, p.k_zp, e.kg_shift, k_key(i), k_oct(i), kc[i], ks[CHAN ? 0 : i], kz[CHAN ? 0 : i]);
+  // the segment of the tile's first key: of the ends that are not the last, how many are not behind it
+  int seg0 = 0;
+  bool one_seg = true;
   if constexpr (CHAN) {
     if (tid < kMaxSegments) seg_end[tid] = p.seg_end[tid];
     __syncthreads();
+    const int lane = tid & 63;
+    seg0 = __popcll(__ballot(lane + 1 < p.nseg && key0 >= seg_end[lane & (kMaxSegments - 1)]));
+    one_seg = seg0 + 1 >= p.nseg || key0 + BN <= seg_end[seg0];
   }
-  auto segment = [&](int key) {
-    int s = 0;
-    if constexpr (CHAN) while (s + 1 < p.nseg && key >= seg_end[s]) ++s;
-    return s;
-  };
-  // values of octet `oct` of one key
-  auto values = [&](const u32 *words, const float *scale, const float *zp, const float *cscale, const float *czp, int g_shift,
-                    int key, int oct, float (&f)[8]) {
-    if (key >= p.Lk) {
-#pragma unroll
-      for (int j = 0; j < 8; ++j) f[j] = 0.f;
-      return;
-    }
-    const int64_t row = kv_row0 + key * p.kv_ts;
-    load_codes<BITS>(words + row * WPR, oct, f);
+  const bool ragged = key0 + BN > p.Lk;
+  auto values = [&](uint2 code, float s1, float z1, const float *cscale, const float *czp, int key, int oct, float (&f)[8]) {
+    code_values<BITS>(code, f);
     if constexpr (CHAN) {
-      const int64_t t = ((int64_t)segment(key) * p.Hkv + hs) * D + oct * 8;
+      int seg = seg0;
+      if (!one_seg) while (seg + 1 < p.nseg && key >= seg_end[seg]) ++seg;
+      const int64_t t = ((int64_t)seg * p.Hkv + hs) * D + oct * 8;
       const float4 sa = *reinterpret_cast<const float4 *>(cscale + t), sb = *reinterpret_cast<const float4 *>(cscale + t + 4);
       const float s[8] = {sa.x, sa.y, sa.z, sa.w, sb.x, sb.y, sb.z, sb.w};
       if (czp) {
@@ -101,38 +120,37 @@ __global__ __launch_bounds__(256) void expand_tiles_kernel(ExpandParams e) {
         for (int j = 0; j < 8; ++j) f[j] = f[j] * s[j];
       }
     } else {
-      const int64_t g = row * (D >> g_shift) + (oct * 8 >> g_shift);
-      const float s = scale[g], z = zp ? zp[g] : 0.f;
 #pragma unroll
-      for (int j = 0; j < 8; ++j) f[j] = (f[j] - z) * s;
+      for (int j = 0; j < 8; ++j) f[j] = (f[j] - z1) * s1;
+    }
+    if (ragged && key >= p.Lk) {
+#pragma unroll
+      for (int j = 0; j < 8; ++j) f[j] = 0.f;
     }
   };
   // V: two adjacent keys x 8 channels -> the transposed tile in LDS
 #pragma unroll
-  for (int i = 0; i < BN / 2 * OCT / 256; ++i) {
-    const int item = tid + i * 256, oct = item % OCT, kp = item / OCT;
+  for (int i = 0; i < VI; ++i) {
     float f0[8], f1[8];
-    values(p.v_words, p.v_scale, p.v_zp, p.v_chan_scale, p.v_chan_zp, e.vg_shift, tile * BN + 2 * kp, oct, f0);
-    values(p.v_words, p.v_scale, p.v_zp, p.v_chan_scale, p.v_chan_zp, e.vg_shift, tile * BN + 2 * kp + 1, oct, f1);
+    const int c = CHAN ? 0 : i;
+    values(vc[i][0], vs[c][0], vz[c][0], p.v_chan_scale, p.v_chan_zp, v_key(i), v_oct, f0);
+    values(vc[i][1], vs[c][1], vz[c][1], p.v_chan_scale, p.v_chan_zp, v_key(i) + 1, v_oct, f1);
 #pragma unroll
-    for (int j = 0; j < 8; ++j) *reinterpret_cast<u32 *>(&vt[(oct * 8 + j) * VTS + 2 * kp]) = pack_io_rne<F16>(f0[j], f1[j]);
+    for (int j = 0; j < 8; ++j) *reinterpret_cast<u32 *>(&vt[(v_oct * 8 + j) * VTS + (tid + i * 256) / OCT * 2]) = pack_io_rne<F16>(f0[j], f1[j]);
   }
   // K: one octet of one key is one lane's 16 bytes
 #pragma unroll
-  for (int i = 0; i < BN * OCT / 256; ++i) {
-    const int item = tid + i * 256, r = item & 15, g = (item >> 4) & 3, frag = item >> 6;
-    const int t = frag & 1, ch = (frag % NF) >> 1, kb = frag / NF;
+  for (int i = 0; i < KI; ++i) {
     float f[8];
-    values(p.k_words, p.k_scale, p.k_zp, p.k_chan_scale, p.k_chan_zp, e.kg_shift, tile * BN + kb * 32 + 8 * (r >> 2) + 4 * t + (r & 3),
-           ch * 4 + g, f);
+    values(kc[i], ks[CHAN ? 0 : i], kz[CHAN ? 0 : i], p.k_chan_scale, p.k_chan_zp, k_key(i), k_oct(i), f);
     u32x4_t w;
 #pragma unroll
     for (int j = 0; j < 4; ++j) w[j] = pack_io_rne<F16>(f[2 * j], f[2 * j + 1]);
-    *reinterpret_cast<u32x4_t *>(out + item * 16) = w;
+    *reinterpret_cast<u32x4_t *>(out + (tid + i * 256) * 16) = w;
   }
   __syncthreads();
 #pragma unroll
-  for (int i = 0; i < BN * OCT / 256; ++i) {
+  for (int i = 0; i < KI; ++i) {
     const int item = tid + i * 256, r = item & 15, g = (item >> 4) & 3, frag = item >> 6;
     *reinterpret_cast<u32x4_t *>(out + kHalfTile<D> + item * 16) =
         *reinterpret_cast<const u32x4_t *>(&vt[((frag % NF) * 16 + r) * VTS + (frag / NF) * 32 + g * 8]);
