@@ -439,7 +439,7 @@ __device__ __forceinline__ void attend_block(const AttnParams &p, int bh, int ou
     __syncthreads();
     kv_end = lds_maxlim;
   }
-  int n_tiles = (kv_end + BN - 1) / BN;
+  int n_tiles = __builtin_amdgcn_readfirstlane((kv_end + BN - 1) / BN);   // (the limit comes from LDS: the compiler does not see that it is uniform)
   // segment ends in LDS: indexing the kernel arguments with a run-time index would move
   // the whole argument block to scratch memory (literal indices only, for the same reason)
   __shared__ int lds_seg_end[kMaxSegments];
@@ -1083,7 +1083,7 @@ __device__ __forceinline__ void attend_block(const AttnParams &p, int bh, int ou
   // would be exp2(-inf) = 0): the end of the cache and, under a key limit, whatever the workgroup's other
   // wavefronts still need.  A whole sequence of 680 tokens in ten steps, [8,680,16,64] fp16: a quarter of
   // the workgroups' key blocks; with the order of the query tiles (BlockOf) append and attention 47.5 -> 39.7 us.
-  const int wave_tiles = wave_live ? min(n_tiles, (max(wave_end - tile_base, 0) + BN - 1) / BN) : 0;
+  const int wave_tiles = __builtin_amdgcn_readfirstlane(wave_live ? min(n_tiles, (max(wave_end - tile_base, 0) + BN - 1) / BN) : 0);
   auto attend = [&](int tile) {
     begin_tile(tile);
     const bool half_tile = wave_end - t0 <= 32;
