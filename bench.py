@@ -849,7 +849,7 @@ def main():
         'pack_us_per_tensor_in_step': round(t_quant_step * 1e6, 2),
         'unpack_dequant_GBps': round(deq_bytes / t_deq / 1e9, 2), 'unpack_dequant_frac_hbm_peak': round(deq_bytes / t_deq / 1e9 / HBM_PEAK_GBPS, 4),
         'unpack_dequant_us_per_tensor': round(t_deq * 1e6, 2),
-        'roofline': {'kernel': 'fused_attn_kernel<128,4,128,128,token scales, reference rounding>', 'bound': 'mfma', 'achieved': round(attn_tflops, 2),
+        'roofline': {'kernel': 'expand_tiles_kernel<128,4,token scales> + wide_attn_kernel<128>, reference rounding', 'bound': 'mfma', 'achieved': round(attn_tflops, 2),
                      'peak': MFMA_BF16_PEAK_TFLOPS, 'unit': 'TFLOP/s', 'frac': round(attn_tflops / MFMA_BF16_PEAK_TFLOPS, 4),
                      'traffic': None if not traffic else traffic.get('fused_attn'),
                      'timing': 'HIP events around each of the timed steps\' launches'},
