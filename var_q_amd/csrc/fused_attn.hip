@@ -18,8 +18,9 @@
 //    tiles ahead, one workgroup barrier per tile).  K is widened once per workgroup,
 //    straight from the registers it was loaded into, to LDS rows that are MFMA A operands;
 //    V goes to LDS packed and is widened and transposed by 2 keys x 8 channels per thread
-//    (the PV contraction runs over keys).  Widened tiles are double-buffered, packed V and
-//    the per-key parameters triple-buffered.
+//    (the PV contraction runs over keys).  Widened tiles and packed V are double-buffered,
+//    the per-key parameters of the exact-code form triple-buffered; at head dim 64 there is also an
+//    instantiation with one of each buffer, for launches of many small workgroups (launch_d64).
 //  * Key rows are fed to the first MFMA in a permuted order chosen so that each
 //    lane's accumulator registers hold 8 consecutive keys per 16-key chunk,
 //    which makes the V^T operand a single 16-byte LDS read.
