@@ -1,0 +1,99 @@
+"""Per-token rules on packed caches: `cache()` leaves everything current that an attention reads, so a call
+launches the attention and nothing else -- from any stream that is ordered behind `cache()`, from several of
+them, and under graph capture."""
+import pytest
+import torch
+from torch.utils._python_dispatch import TorchDispatchMode
+
+from gpu_util import note
+from var_q_amd import VAR_Q
+from var_q_amd.quant import fused_attention
+
+pytestmark = pytest.mark.gpu
+RULES = [('G_TOKEN', True, None), ('G_TOKEN_HEAD', False, None), ('G_GROUP', False, 32), ('G_GROUP', True, 64)]
+
+
+class _Ops(TorchDispatchMode):
+    """The torch operators that run inside."""
+
+    def __enter__(self):
+        self.seen = []
+        return super().__enter__()
+
+    def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+        self.seen.append(str(func))
+        return func(*args, **(kwargs or {}))
+
+
+def _pair(dev, fmt, rule, steps=(1, 4, 30), B=2, H=3, c=64, seed=3):
+    method, symmetric, group = rule
+    gen = torch.Generator(device=dev).manual_seed(seed)
+    pair = [VAR_Q(4, fmt, method, symmetric=symmetric, group_size=group) for _ in range(2)]
+    shape = (lambda n: (B, H, n, c)) if fmt == 'BHLc' else (lambda n: (B, n, H, c))
+    for n in steps:
+        for z in pair:
+            z.quant(torch.randn(*shape(n), device=dev, generator=gen).half())
+            z.cache()
+    return pair, torch.randn(*shape(33), device=dev, generator=gen).half()
+
+
+def _expected(pair, q, fmt):
+    """softmax(q K^T / 8) V in fp64 over the dequantized caches, heads first."""
+    k, v, q = ((t if fmt == 'BHLc' else t.transpose(1, 2)).double().contiguous() for t in (pair[0].dequant_all(), pair[1].dequant_all(), q))
+    w = torch.softmax(torch.matmul(q, k.transpose(2, 3).contiguous()) * 0.125, -1)
+    o = torch.matmul(w, v)
+    return o if fmt == 'BHLc' else o.transpose(1, 2)
+
+
+def _close(out, want):
+    # fp16 rounding of K, V, weights and result (2^-11 each), sums of up to 35 weights that add up to 1
+    return float((out.double() - want).abs().max()) <= 1e-2 * max(1.0, float(want.abs().max()))
+
+
+@pytest.mark.parametrize('rule', RULES)
+@pytest.mark.parametrize('fmt', ['BHLc', 'BLHc'])
+def test_an_attention_copies_nothing(dev, fmt, rule):
+    note('token scales: operators of a call', fmt, rule)
+    pair, q = _pair(dev, fmt, rule)
+    with _Ops() as ops:
+        out = fused_attention(q, *pair, 0.125)
+    assert not [f for f in ops.seen if 'copy' in f or 'cat' in f or 'clone' in f], ops.seen
+    assert _close(out, _expected(pair, q, fmt))
+
+
+@pytest.mark.parametrize('rule', RULES)
+def test_two_streams_attend_one_cache(dev, rule):
+    note('token scales: two streams', rule)
+    pair, q = _pair(dev, 'BHLc', rule)
+    ready = torch.cuda.Event()
+    ready.record()
+    streams, outs = [torch.cuda.Stream(), torch.cuda.Stream()], []
+    for st in streams:
+        st.wait_event(ready)
+        with torch.cuda.stream(st):
+            outs.append(fused_attention(q, *pair, 0.125))
+    torch.cuda.synchronize()
+    want = _expected(pair, q, 'BHLc')
+    assert _close(outs[0], want) and torch.equal(outs[0], outs[1])
+
+
+@pytest.mark.parametrize('rule', RULES)
+def test_capture_behind_an_eager_cache(dev, rule):
+    note('token scales: capture', rule)
+    pair, q = _pair(dev, 'BHLc', rule)
+    out = torch.empty_like(q)
+    graph = torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    with torch.cuda.graph(graph):
+        fused_attention(q, *pair, 0.125, out=out)
+    eager = fused_attention(q, *pair, 0.125)           # before the first replay
+    torch.cuda.synchronize()
+    assert _close(eager, _expected(pair, q, 'BHLc'))
+    for _ in range(3):
+        out.fill_(7.0)
+        junk = [torch.full((n,), float('nan'), device=dev) for n in (8, 64, 512, 4096)]   # whatever was given back is taken again
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, eager)
+        del junk

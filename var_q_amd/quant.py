@@ -439,9 +439,11 @@ class VAR_Q:
         else:
             ng = self.scale.shape[3]
             shape = (B, H, n, ng) if bhl else (B, n, H, ng)
-            self._tok_scale.append_later(self.scale.expand(*shape))
+            # (copied here, on the stream of the step: a copy left for the attention would run on whatever stream
+            # attends first, or go into a graph that is being recorded, with nothing to order another reader behind it)
+            self._tok_scale.append(self.scale.expand(*shape))
             if self.zp is not None:
-                self._tok_zp.append_later(self.zp.expand(*shape))
+                self._tok_zp.append(self.zp.expand(*shape))
 
     # ---------------- dequantize ----------------
     def _dequant(self, q: torch.Tensor, scale: torch.Tensor, zp: Optional[torch.Tensor],
@@ -579,8 +581,6 @@ def fused_attention(q: torch.Tensor, k_quant: VAR_Q, v_quant: VAR_Q, softmax_sca
                                       v_quant._tab_zp, bits, Lk, softmax_scale, kv_limit=kv_limit, out=out,
                                       seg_ends=ends, layout=layout)
     if km in _TOKEN_METHODS and vm in _TOKEN_METHODS:
-        for qz in (k_quant, v_quant):
-            qz._tok_scale.view(), qz._tok_zp.view()      # (the steps appended since the last call)
         ks, kz, vs, vz = k_quant._tok_scale.buf, k_quant._tok_zp.buf, v_quant._tok_scale.buf, v_quant._tok_zp.buf
         if ks.shape[:3] != kbuf.shape[:3] or vs.shape[:3] != kbuf.shape[:3]:
             raise ValueError('fused_attention: scale buffers and code buffers differ in capacity')
