@@ -5,6 +5,7 @@ import pytest
 import torch
 from torch.utils._python_dispatch import TorchDispatchMode
 
+import varq_oracle as O
 from gpu_util import note
 from var_q_amd import VAR_Q
 from var_q_amd.quant import fused_attention
@@ -97,3 +98,36 @@ def test_capture_behind_an_eager_cache(dev, rule):
         torch.cuda.synchronize()
         assert torch.equal(out, eager)
         del junk
+
+
+@pytest.mark.parametrize('method,bits,c,steps,pack', [
+    ('G_SCALE_HEAD_DIM', 8, 64, 4, True), ('G_SCALE_HEAD_DIM', 8, 20, 4, True), ('G_SCALE_HEAD_DIM', 4, 64, 18, True),
+    ('G_SCALE', 8, 64, 3, True), ('G_TENSOR', 8, 64, 3, True), ('G_TOKEN', 4, 64, 3, True), ('G_TOKEN_HEAD', 2, 64, 18, True),
+    ('G_HEAD_DIM', 8, 64, 3, True), ('G_SCALE_HEAD_DIM', 8, 64, 3, False), ('G_TOKEN', 8, 64, 3, False)])
+@pytest.mark.parametrize('fmt', ['BHLc', 'BLHc'])
+def test_a_look_at_the_cached_scales_changes_nothing(dev, fmt, method, bits, c, steps, pack):
+    """Read while a graph is being recorded, then eagerly before any replay, then from the replays; and the
+    one-call step (`use_var_q`) leaves the same as `quant` and `cache`."""
+    note('cached scales', fmt, method, bits, c, steps, pack)
+    ref = O.OracleVARQ(bits, fmt, method, pack_to_int32=pack)
+    two, one = (VAR_Q(bits, fmt, method, pack_to_int32=pack) for _ in range(2))
+    gen = torch.Generator().manual_seed(c + steps)
+    for i in range(steps):
+        x = torch.randn(*((2, 3, i % 3 + 1, c) if fmt == 'BHLc' else (2, i % 3 + 1, 3, c)), generator=gen) * (i + 1)
+        want = ref.use_var_q(x)
+        two.quant(x.to(dev))
+        two.cache()
+        assert torch.equal(one.use_var_q(x.to(dev)).cpu(), want)
+    graph = torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    with torch.cuda.graph(graph):
+        recorded = two.cached_scale * 1.0
+    for z in (two, one):
+        assert torch.equal(z.cached_scale.cpu(), ref.cached_scale) and z.cached_zp is None
+    assert torch.equal(two.dequant_all().cpu(), want)
+    for _ in range(3):
+        torch.full((4096,), float('nan'), device=dev)
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(recorded.cpu(), ref.cached_scale)

@@ -54,19 +54,6 @@ class _Growable:
     def __init__(self, dim: int, min_capacity: int = 64):
         self.dim, self.buf, self.len = dim, None, 0
         self.min_capacity = min_capacity       # room of the first allocation (tokens)
-        self._pending = []
-
-    def append_later(self, t: torch.Tensor):
-        """Append when the buffer is next looked at.  The cached scales of the reference are
-        each step's scale expanded over the step's tokens (VAR_Q/quant.py:196-201): fp32 per
-        code, four times the bytes of the 8-bit codes themselves; a caller that attends the packed
-        cache through the tables never reads them."""
-        self._pending.append(t)
-
-    def _flush(self):
-        pending, self._pending = self._pending, []
-        for t in pending:
-            self.append(t() if callable(t) else t)     # (a callable builds the expanded view when asked)
 
     def append(self, t: torch.Tensor):
         n = t.size(self.dim)
@@ -100,11 +87,9 @@ class _Growable:
         return self.buf
 
     def replace(self, t: torch.Tensor):
-        self._pending = []
         self.buf, self.len = t, t.size(self.dim)
 
     def view(self) -> Optional[torch.Tensor]:
-        self._flush()
         return None if self.buf is None else self.buf.narrow(self.dim, 0, self.len)
 
 
@@ -191,7 +176,8 @@ class VAR_Q:
         # what the fused attention reads, kept up to date by cache(): the end of every cached
         # step with its (head, channel) tables for the methods whose scale is shared by the
         # tokens of a step, a full-size copy of the per-token scales (shaped like the code buffer,
-        # [.., capacity, .., groups]) for the others
+        # [.., capacity, .., groups]) for the others.  _c_scale and _c_zp hold the scales as the
+        # reference caches them only where those do not (see _shown)
         self._staged = None
         self._seg_ends: List[int] = []
         self._tab_scale: Optional[torch.Tensor] = None      # [MAX_TABLE_STEPS, H, c]
@@ -202,6 +188,7 @@ class VAR_Q:
         self._c_item = _Growable(self.dim_cat, room)
         self._c_scale = _Growable(self.dim_cat, room)
         self._c_zp = _Growable(self.dim_cat, room)
+        self._scale_shape: Tuple[int, ...] = ()             # of the cached steps' scales, one token each or per token
         # the dequantized cache as use_var_q hands it out, kept from step to step (see use_var_q)
         self._c_deq = _Growable(self.dim_cat, room)
 
@@ -220,11 +207,42 @@ class VAR_Q:
 
     @property
     def cached_scale(self) -> Optional[torch.Tensor]:
-        return self._c_scale.view()
+        return self._shown(self._c_scale, self._tok_scale, self._tab_scale)
 
     @property
     def cached_zp(self) -> Optional[torch.Tensor]:
-        return self._c_zp.view()
+        return None if self.symmetric else self._shown(self._c_zp, self._tok_zp, self._tab_zp)
+
+    def _shown(self, kept: _Growable, tok: _Growable, tab: Optional[torch.Tensor]) -> Optional[torch.Tensor]:
+        """The cached scales as the reference holds them: each step's scale expanded over the step's
+        tokens (VAR_Q/quant.py:196-201), for a shared scale fp32 per code, four times the bytes of
+        the 8-bit codes themselves.  A caller that goes through the tables never reads them, so they are made
+        from the tables when asked for, each time anew: a look changes nothing, whatever stream or graph
+        capture it happens in."""
+        n, d = self._c_item.len, self._c_item.dim
+        if kept.len == n:
+            return kept.view()
+        like = self._scale_shape
+        if self.quant_method in _TOKEN_METHODS:
+            t = tok.view()
+            for i in range(3):
+                if i != d:
+                    t = t.narrow(i, 0, like[i])
+            return t
+        h = 3 - d                                            # the dim of the heads
+        full = [1, tab.shape[1], tab.shape[2]]
+        full.insert(d, 1)
+        shape, parts, start = [-1] * 4, [], 0
+        for k, end in enumerate(self._seg_ends):
+            shape[d] = end - start
+            parts.append(tab[k].view(full).narrow(h, 0, like[h]).narrow(3, 0, like[3]).expand(shape))
+            start = end
+        return torch.cat(parts, d)
+
+    def _tables_hold(self, steps: int, c: int) -> bool:
+        """Whether the step tables stand in for the cached scales of so many steps."""
+        return self.pack_to_int32 and self.quant_method in _TABLE_METHODS and steps <= MAX_TABLE_STEPS \
+            and c % 8 == 0 and (c * self.quant_bits) % 32 == 0
 
     # ---------------- quantize ----------------
     def _quantize(self, x: torch.Tensor):
@@ -327,11 +345,10 @@ class VAR_Q:
         sshape = (1, H, 1, c) if d == 2 else (1, 1, H, c)
         self._window = (item.buf, d, start, n, srow, zrow, sshape)
         self._staged = None
+        if c % 8:
+            self._keep_scales(n, c)
+        self._scale_shape = sshape
         item.len = start + n
-        eshape = (-1, -1, n, -1) if d == 2 else (-1, n, -1, -1)
-        self._c_scale.append_later(lambda: srow.view(sshape).expand(*eshape))
-        if zrow is not None:
-            self._c_zp.append_later(lambda: zrow.view(sshape).expand(*eshape))
         ends = self._seg_ends
         ends.append(ends[-1] + n if ends else n)
 
@@ -383,8 +400,6 @@ class VAR_Q:
     def cache(self):
         m = self.quant_method
         q_cur = self.quantized_item
-        s_cur = self._expand_scale_like_L(q_cur, self.scale)
-        z_cur = None if self.zp is None else self._expand_scale_like_L(q_cur, self.zp)
         if m in ('G_SCALE_HEAD_DIM', 'G_SCALE', 'G_TOKEN', 'G_TOKEN_HEAD', 'G_TENSOR', 'G_GROUP', 'G_HEAD'):
             if self._c_item.dim != self.dim_cat:
                 # the layout was re-assigned: fine before the first step, an error once steps are
@@ -394,23 +409,36 @@ class VAR_Q:
                     raise ValueError('VAR_Q: qkv_format was changed to %s with %d tokens cached in the other layout'
                                      % (self.qkv_format, self._c_item.len))
                 self._reset_cache()
+            self._keep_scales(q_cur.size(self.dim_cat), self._pack_meta['orig_c'] if self.pack_to_int32 else q_cur.shape[3])
+            self._scale_shape = tuple(self.scale.shape)
             st, self._staged = self._staged, None
             if st is not None and st[0] is self._c_item.buf and st[1] == self._c_item.len and st[2] is q_cur:
                 self._c_item.len += q_cur.size(self.dim_cat)      # the codes are in place already
             else:
                 self._c_item.append(q_cur)
-            self._c_scale.append_later(s_cur)
-            if z_cur is not None:
-                self._c_zp.append_later(z_cur)
             self._note_step(q_cur, replace=False)
         elif m == 'G_HEAD_DIM':
             self._c_item.replace(q_cur)
-            self._c_scale.replace(s_cur)
-            if z_cur is not None:
-                self._c_zp.replace(z_cur)
+            self._c_scale.replace(self._expand_scale_like_L(q_cur, self.scale))
+            if self.zp is not None:
+                self._c_zp.replace(self._expand_scale_like_L(q_cur, self.zp))
             self._note_step(q_cur, replace=True)
         else:
             raise ValueError(f"[VAR-Q]: Invalid quantization method: {m}")
+
+    def _keep_scales(self, n: int, c: int):
+        """The scales of the current step, n tokens of c channels, behind those of the cached ones, where neither the step
+        tables nor the per-token scales hold them (called before the step is counted)."""
+        if self._tables_hold(len(self._seg_ends) + 1, c) or (self.pack_to_int32 and self.quant_method in _TOKEN_METHODS):
+            return
+        shape = [-1] * 4
+        shape[self.dim_cat] = n
+        for kept, earlier, t in ((self._c_scale, self.cached_scale, self.scale), (self._c_zp, self.cached_zp, self.zp)):
+            if t is None:
+                continue
+            if kept.len < self._c_item.len:                  # (the tables held them up to here)
+                kept.append(earlier)
+            kept.append(t.expand(shape))
 
     def _note_step(self, q_cur: torch.Tensor, replace: bool):
         """Book-keeping for `fused_attention` (packed codes only)."""
@@ -465,9 +493,9 @@ class VAR_Q:
         item, ends = self._c_item, self._seg_ends
         if item.len == 0:
             return self.dequant_current(out_dtype)
-        if self.pack_to_int32 and ends and len(ends) <= MAX_TABLE_STEPS and ends[-1] == item.len and item.dim == self.dim_cat:
+        if ends and ends[-1] == item.len and item.dim == self.dim_cat:
             c = self._pack_meta['orig_c']
-            if c % 8 == 0 and (c * self.quant_bits) % 32 == 0 and self._tab_scale.shape[2] == c:
+            if self._tables_hold(len(ends), c) and self._tab_scale.shape[2] == c:
                 # one scale table per step (the methods of _TABLE_METHODS): the expanded scales of
                 # cached_scale are neither made nor read
                 return _lib.host().dequant_steps(item.buf, ends, self._tab_scale, self._tab_zp, c, self.quant_bits,
