@@ -361,7 +361,11 @@ __device__ __forceinline__ void store_octet(const GenParams &p, int64_t row, int
   }
 }
 
-template <int DT, bool ASYM, bool KEEPC>
+// (Its own copy of the arithmetic of store_octet, and p.asym at run time: with a row's octet in every lane and one load in
+// flight the kernel is nearly as much bound by its instructions as by its bytes, and the shared form has more branches
+// per octet.  [32,30,680,64] affine 2 bits, four inputs in turn, three runs: 21.5-22.2 us through store_octet,
+// 21.1-21.4 like this; store_octet with these branches in it 22.3-23.8.)
+template <int DT, bool KEEPC>
 __global__ __launch_bounds__(256) void quant_tiled_kernel(GenParams p, Plan pl, const float *rinv, const u32 *plain) {
   constexpr int NV = KEEPC ? 8 : 1;
   if (take_second(p)) { rinv += p.ws1; plain += p.ws1; }
@@ -369,7 +373,7 @@ __global__ __launch_bounds__(256) void quant_tiled_kernel(GenParams p, Plan pl, 
   // 2-bit words are assembled from two adjacent column lanes: idle lanes must still reach the shuffle
   const bool live = l.live;
   const int64_t g = (int64_t)l.ko * pl.ko_gs + (int64_t)(live ? l.q : 0) * pl.q_gs + (KEEPC ? (live ? l.col : 0) * 8 : 0);
-  float s[NV], r[NV], z[NV] = {};
+  float s[NV], r[NV], z[NV];
   bool all_plain = true;
   if constexpr (KEEPC) {
     // the lane's eight groups are adjacent and start at a multiple of 8: 16-byte loads (the
@@ -380,17 +384,61 @@ __global__ __launch_bounds__(256) void quant_tiled_kernel(GenParams p, Plan pl, 
     };
     ld8(p.scale, s);
     ld8(rinv, r);
-    if constexpr (ASYM) ld8(p.zp, z);
+    if (p.asym) ld8(p.zp, z);
+    else {
+#pragma unroll
+      for (int j = 0; j < NV; ++j) z[j] = 0.f;
+    }
     const uint4 pa = reinterpret_cast<const uint4 *>(plain + g)[0], pb = reinterpret_cast<const uint4 *>(plain + g)[1];
     all_plain = (pa.x & pa.y & pa.z & pa.w & pb.x & pb.y & pb.z & pb.w) != 0u;
   } else {
     s[0] = p.scale[g];
     r[0] = rinv[g];
-    if (ASYM) z[0] = p.zp[g];
+    z[0] = p.asym ? p.zp[g] : 0.f;
     all_plain = plain[g] != 0u;
   }
+  const float qmin = (float)p.qmin, qmax = (float)p.qmax;
+  const u32 mask = (1u << p.bits) - 1u;
   if (!live) return;   // (only the 2-bit path shuffles, and there c8 is even: partners are live together)
-  for_rows<DT>(p, pl, l, [&](int64_t row, const float (&v)[8]) { store_octet<NV>(p, row, l.col, v, s, r, z, all_plain); });
+  for_rows<DT>(p, pl, l, [&](int64_t row, const float (&v)[8]) {
+    int q[8];
+    if (all_plain) {
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        const float sj = s[j % NV], rj = r[j % NV];
+        const float q0 = v[j] * rj;
+        const float t = __builtin_fmaf(__builtin_fmaf(-q0, sj, v[j]), rj, q0);
+        q[j] = (int)__builtin_amdgcn_fmed3f(rintf(t) + z[j % NV], qmin, qmax);
+      }
+    } else {
+#pragma unroll
+      for (int j = 0; j < 8; ++j) q[j] = (int)__builtin_amdgcn_fmed3f(rintf(v[j] / s[j % NV]) + z[j % NV], qmin, qmax);
+    }
+    const int64_t orow = out_row32(p, row);
+    const int64_t o = orow * p.c8 + l.col;
+    if (p.codes) {
+      u32 lo = (q[0] & 0xff) | ((q[1] & 0xff) << 8) | ((q[2] & 0xff) << 16) | ((u32)q[3] << 24);
+      u32 hi = (q[4] & 0xff) | ((q[5] & 0xff) << 8) | ((q[6] & 0xff) << 16) | ((u32)q[7] << 24);
+      *reinterpret_cast<uint2 *>(p.codes + o * 8) = make_uint2(lo, hi);
+    }
+    if (p.words) {
+      if (p.bits == 8) {
+        u32 lo = (q[0] & 0xff) | ((q[1] & 0xff) << 8) | ((q[2] & 0xff) << 16) | ((u32)q[3] << 24);
+        u32 hi = (q[4] & 0xff) | ((q[5] & 0xff) << 8) | ((q[6] & 0xff) << 16) | ((u32)q[7] << 24);
+        *reinterpret_cast<uint2 *>(p.words + orow * p.wpr + l.col * 2) = make_uint2(lo, hi);
+      } else {
+        u32 w = 0;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) w |= ((u32)q[j] & mask) << (j * p.bits);
+        if (p.bits == 4) {
+          p.words[orow * p.wpr + l.col] = (int32_t)w;
+        } else {  // 2 bits: 16 codes per word = two adjacent octets (c % 16 == 0 on this path)
+          u32 other = __shfl_xor(w, 1, 64);
+          if ((l.col & 1) == 0) p.words[orow * p.wpr + (l.col >> 1)] = (int32_t)(w | (other << 16));
+        }
+      }
+    }
+  });
 }
 
 // ---- one launch: a workgroup holds all rows of its groups -----------------------------------------
@@ -808,13 +856,8 @@ int run_tiled(GenParams &p, const Plan &pl, void *workspace, hipStream_t st) {
   // per thread measured alike, longer ones slower)
   const Plan &pb = pl;
   dim3 bgrid((unsigned)((int64_t)pb.nko * pb.tilesQ * pb.Z), nt);
-  if (p.asym) {
-    if (p.keepc) hipLaunchKernelGGL((quant_tiled_kernel<DT, true, true>), bgrid, dim3(256), 0, st, p, pb, rinv, plain);
-    else hipLaunchKernelGGL((quant_tiled_kernel<DT, true, false>), bgrid, dim3(256), 0, st, p, pb, rinv, plain);
-  } else {
-    if (p.keepc) hipLaunchKernelGGL((quant_tiled_kernel<DT, false, true>), bgrid, dim3(256), 0, st, p, pb, rinv, plain);
-    else hipLaunchKernelGGL((quant_tiled_kernel<DT, false, false>), bgrid, dim3(256), 0, st, p, pb, rinv, plain);
-  }
+  if (p.keepc) hipLaunchKernelGGL((quant_tiled_kernel<DT, true>), bgrid, dim3(256), 0, st, p, pb, rinv, plain);
+  else hipLaunchKernelGGL((quant_tiled_kernel<DT, false>), bgrid, dim3(256), 0, st, p, pb, rinv, plain);
   return 0;
 }
 
