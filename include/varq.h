@@ -222,7 +222,8 @@ int varq_dequant(const int32_t *words, const int8_t *codes_i8, const float *scal
  *   words        packed codes of a cache buffer of `capacity` tokens, of which host_seg_end[nseg-1] are read
  *   tokens_first 1: words [B, capacity, H, W], out [B, tokens, H, c]; 0: heads before tokens in both
  *   scale, zp    fp32 [nseg, H, c] (zp NULL = symmetric)
- * Requires c % 8 == 0, rows of whole words, nseg in 1..16.
+ * Requires c % 8 == 0, rows of whole words, nseg in 1..16, B (and with heads first H) at most 65535, fewer than
+ * 2^31 - 2048 octets of channels per batch entry (heads first: per (batch, head)).
  */
 int varq_dequant_steps(const int32_t *words, const float *scale, const float *zp, int nseg, const int32_t *host_seg_end,
                        int B, int H, int64_t capacity, int c, int bits, int tokens_first, void *out, int out_dtype, void *stream);
@@ -232,7 +233,8 @@ int varq_dequant_steps(const int32_t *words, const float *scale, const float *zp
  * cache, dequant_all), in one launch where the sizes allow: varq_quant_pack of x ([B, H, n, c], or
  * [B, n, H, c] with tokens_first) into tokens host_seg_end[nseg-2].. of `words` and row nseg-1 of the
  * tables, then varq_dequant_steps over all nseg steps.  The step's tokens are the last segment's.
- * Workspace: varq_quant_workspace_bytes of the step.  x, scale, zp, out: 16-byte aligned.
+ * Workspace: varq_quant_workspace_bytes of the step.  x, scale, zp, out: 16-byte aligned.  What
+ * varq_dequant_steps refuses is refused before anything is launched.
  */
 int varq_quant_step_dequant(const void *x, int x_dtype, int B, int H, int n, int c, int tokens_first, int bits, int asym, float eps,
                             int32_t *words, int64_t capacity, float *scale, float *zp, int nseg, const int32_t *host_seg_end,

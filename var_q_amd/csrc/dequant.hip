@@ -207,7 +207,7 @@ __global__ __launch_bounds__(256) void dequant_kernel(DeqParams p) {
 
 template <int ODT, int BITS>
 __global__ __launch_bounds__(256) void dequant_steps_kernel(StepParams p) {
-  dequant_steps_block<ODT, BITS, 256, 4>(p, blockIdx.y, blockIdx.x);
+  dequant_steps_block<ODT, BITS, 256, 4>(p, (int64_t)blockIdx.z * gridDim.y + blockIdx.y, blockIdx.x);
 }
 
 }  // namespace
@@ -223,12 +223,11 @@ extern "C" int varq_dequant_steps(const int32_t *words, const float *scale, cons
   const int64_t tokens = host_seg_end[nseg - 1];
   for (int s = 0, prev = 0; s < nseg; prev = host_seg_end[s++])
     VARQ_CHECK_ARG(host_seg_end[s] >= prev, "dequant_steps: segment ends must increase");
-  VARQ_CHECK_ARG(tokens <= capacity && set_steps(p, words, scale, zp, nseg, host_seg_end, H, capacity, c, bits, tokens_first, out),
+  VARQ_CHECK_ARG(tokens <= capacity && set_steps(p, words, scale, zp, nseg, host_seg_end, B, H, capacity, c, bits, tokens_first, out),
                  "dequant_steps: more tokens than the buffer or the grid holds");
   if (tokens <= 0) return VARQ_OK;
-  const int64_t pairs = tokens_first ? B : (int64_t)B * H;
-  VARQ_CHECK_ARG(pairs <= 65535, "dequant_steps: more than 65535 (batch, head) pairs");
-  dim3 grid((unsigned)((p.pair_octs + 1023) / 1024), (unsigned)pairs);
+  // (pair b * H + h is block (h, b): the grid's limit holds for each dim, as in varq_dequant)
+  dim3 grid((unsigned)((p.pair_octs + 1023) / 1024), (unsigned)(tokens_first ? 1 : H), (unsigned)B);
   hipStream_t st = (hipStream_t)stream;
 #define VARQ_STEPS(ODT_)                                                                                        \
   do {                                                                                                          \

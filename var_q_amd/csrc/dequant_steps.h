@@ -105,9 +105,10 @@ __device__ __forceinline__ void dequant_steps_block(const StepParams &p, int64_t
 }
 
 // The launch parameters for `nseg` steps that end at host_seg_end[..]; false where the octets of a pair exceed
-// 31 bits.  p.out_pair_octs is that of an output which holds these tokens and no others.
-inline bool set_steps(StepParams &p, const int32_t *words, const float *scale, const float *zp, int nseg, const int32_t *host_seg_end, int H,
+// 31 bits or a dim the grid's 65535.  p.out_pair_octs is that of an output which holds these tokens and no others.
+inline bool set_steps(StepParams &p, const int32_t *words, const float *scale, const float *zp, int nseg, const int32_t *host_seg_end, int B, int H,
                       int64_t capacity, int c, int bits, bool tokens_first, void *out) {
+  if (B > 65535 || (!tokens_first && H > 65535)) return false;
   const int64_t tokens = nseg ? host_seg_end[nseg - 1] : 0;
   p.words = reinterpret_cast<const u32 *>(words); p.scale = scale; p.zp = zp; p.out = out;
   p.H = H; p.c = c; p.nseg = nseg; p.row = (int64_t)H * c;

@@ -1052,8 +1052,11 @@ extern "C" int varq_quant_step_dequant(const void *x, int x_dtype, int B, int H,
   const int64_t shape[4] = {B, tokens_first ? n : H, tokens_first ? H : n, c}, map[3] = {n * per, (capacity - n) * per, start * per};
   StepOut o;
   const int64_t pairs = tokens_first ? B : (int64_t)B * H;
-  const bool fits = set_steps(o.earlier, words, scale, asym ? zp : nullptr, nseg - 1, host_seg_end, H, capacity, c, bits, tokens_first, out) &&
-                    pairs * start * o.earlier.octs <= (asym ? kStepMostAsym : kStepMostSym);
+  // (refused before the step is quantized)
+  VARQ_CHECK_ARG(set_steps(o.earlier, words, scale, asym ? zp : nullptr, nseg, host_seg_end, B, H, capacity, c, bits, tokens_first, out),
+                 "quant_step_dequant: more tokens or pairs than the grid holds");
+  set_steps(o.earlier, words, scale, asym ? zp : nullptr, nseg - 1, host_seg_end, B, H, capacity, c, bits, tokens_first, out);
+  const bool fits = pairs * start * o.earlier.octs <= (asym ? kStepMostAsym : kStepMostSym);
   o.earlier.out_pair_octs = tokens * o.earlier.octs;
   o.inner = map[0]; o.delta = (tokens - n) * per; o.off = map[2];
   o.odt = out_dtype; o.q_blocks = 0; o.pair_blocks = 0;

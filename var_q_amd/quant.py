@@ -245,6 +245,11 @@ class VAR_Q:
             and c % 8 == 0 and (c * self.quant_bits) % 32 == 0
 
     # ---------------- quantize ----------------
+    def _steps_fit(self, tokens: int, H: int, c: int) -> bool:
+        """Whether the launch that dequantizes through the step tables can count the octets of so many
+        tokens (it takes them as one run per batch entry, or per (batch, head); the general launch does not)."""
+        return tokens * (H if self.dim_cat == 1 else 1) * (c // 8) < (1 << 31) - 2048
+
     def _quantize(self, x: torch.Tensor):
         if not isinstance(x, torch.Tensor) or not x.is_cuda:
             raise VarqError('VAR_Q requires GPU tensors; there is no CPU path in this package')
@@ -495,7 +500,7 @@ class VAR_Q:
             return self.dequant_current(out_dtype)
         if ends and ends[-1] == item.len and item.dim == self.dim_cat:
             c = self._pack_meta['orig_c']
-            if self._tables_hold(len(ends), c) and self._tab_scale.shape[2] == c:
+            if self._tables_hold(len(ends), c) and self._tab_scale.shape[2] == c and self._steps_fit(item.len, self._tab_scale.shape[1], c):
                 # one scale table per step (the methods of _TABLE_METHODS): the expanded scales of
                 # cached_scale are neither made nor read
                 return _lib.host().dequant_steps(item.buf, ends, self._tab_scale, self._tab_zp, c, self.quant_bits,
@@ -519,7 +524,8 @@ class VAR_Q:
         172 MB per tensor at [2,16,10521,128].  `dequant_all()` itself always recomputes everything."""
         if not self.keep_dequantized:
             place = self._fast_place(item)
-            if place is not None and place[2] % 8 == 0 and (self._seg_ends[-1] if self._seg_ends else 0) == place[4] and item.data_ptr() % 16 == 0:
+            if place is not None and place[2] % 8 == 0 and (self._seg_ends[-1] if self._seg_ends else 0) == place[4] and item.data_ptr() % 16 == 0 \
+                    and self._steps_fit(place[4] + place[0], place[1], place[2]):
                 # the shipped rule: step and dequantized cache from one library call (and where the sizes allow, one launch)
                 out = _lib.host().quant_step_dequant(not self.symmetric, self.quant_bits, self.eps, self.dim_cat, item, self._c_item.buf,
                                                      self._tab_scale, self._tab_zp, self._seg_ends, ops._DT[out_dtype or torch.float32])
