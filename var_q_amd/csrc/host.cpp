@@ -38,6 +38,20 @@ void check(int rc, const char *what) {
   if (rc != VARQ_OK) raise(g_varq_error, "%s failed (status %d): %s", what, rc, varq_last_error());
 }
 
+// The interpreter's lock is given back while device memory is taken and launches are made: an allocation may wait
+// for the device and a launch for room in a full queue, and neither is a reason for the program's other threads to wait.
+// Once per call, around everything behind the reading of the arguments: inside, no Python object is touched and
+// nothing is raised that is not a C++ exception.
+struct NoGil {
+  PyThreadState *const state = PyEval_SaveThread();
+  ~NoGil() { PyEval_RestoreThread(state); }
+};
+template <class F> int status_unlocked(F &&f) {
+  const NoGil unlocked;
+  return f();
+}
+template <class F> void unlocked(const char *what, F &&f) { check(status_unlocked(f), what); }
+
 // ---- arguments ------------------------------------------------------------------------------
 const at::Tensor &gpu(PyObject *o, const char *name) {
   if (!THPVariable_Check(o)) raise(g_varq_error, "%s must be a GPU tensor (got %s); the VAR-Q HIP path has no CPU fallback", name, Py_TYPE(o)->tp_name);
@@ -104,21 +118,26 @@ void need_args(Py_ssize_t n, Py_ssize_t want, const char *name) {
 // ---- quantize + pack --------------------------------------------------------------------------
 // quant_rows(x, group, bits, asym, eps) -> (words, scale, zp | None)
 PyObject *quant_rows(PyObject *const *a) {
-  const at::Tensor x = gpu(a[0], "x").contiguous();
+  const at::Tensor &x0 = gpu(a[0], "x");
   const int64_t group = integer(a[1]), bits = integer(a[2]);
   const bool asym = truth(a[3]);
-  const int64_t c = x.dim() ? x.size(-1) : 0, rows = c ? x.numel() / c : 0;
-  ASSERT(x.dim() >= 1 && group != 0, "quant_pack_rows: a tensor of rows and a group size are needed");
-  c10::DimVector shape(x.sizes().begin(), x.sizes().end());
-  shape.back() = c * bits / 32;
-  const c10::DeviceGuard guard(x.device());
-  const at::Tensor words = empty(shape, at::kInt, x);
-  shape.back() = c / group;
-  const at::Tensor scale = empty(shape, at::kFloat, x);
-  at::Tensor zp;
-  if (asym) zp = empty(shape, at::kFloat, x);
-  check(varq_quant_pack_rows(x.data_ptr(), dtype_code(x), rows, (int)c, (int)group, (int)bits, asym, (float)real(a[4]), nullptr, nullptr,
-                             ptr<int32_t>(words), ptr<float>(scale), asym ? ptr<float>(zp) : nullptr, stream_of(x)), "varq_quant_pack_rows");
+  const float eps = (float)real(a[4]);
+  const int64_t c = x0.dim() ? x0.size(-1) : 0, rows = c ? x0.numel() / c : 0;
+  ASSERT(x0.dim() >= 1 && group != 0, "quant_pack_rows: a tensor of rows and a group size are needed");
+  const int dt = dtype_code(x0);
+  const c10::DeviceGuard guard(x0.device());
+  at::Tensor words, scale, zp;
+  unlocked("varq_quant_pack_rows", [&] {
+    const at::Tensor x = x0.contiguous();
+    c10::DimVector shape(x.sizes().begin(), x.sizes().end());
+    shape.back() = c * bits / 32;
+    words = empty(shape, at::kInt, x);
+    shape.back() = c / group;
+    scale = empty(shape, at::kFloat, x);
+    if (asym) zp = empty(shape, at::kFloat, x);
+    return varq_quant_pack_rows(x.data_ptr(), dt, rows, (int)c, (int)group, (int)bits, asym, eps, nullptr, nullptr, ptr<int32_t>(words),
+                                ptr<float>(scale), asym ? ptr<float>(zp) : nullptr, stream_of(x));
+  });
   return triple(words, scale, zp);
 }
 
@@ -138,22 +157,25 @@ struct Shared {   // shapes of a quantization with groups that span rows
 PyObject *quant_shared(PyObject *const *a) {
   const at::Tensor &x0 = gpu(a[0], "x");
   ASSERT(x0.dim() == 4, "expected a 4-D [B,L,H,c] / [B,H,L,c] tensor");
-  const at::Tensor x = x0.contiguous();
   const int mask = (int)integer(a[1]);
   const int64_t bits = integer(a[2]);
   const bool asym = truth(a[3]), pack = truth(a[5]);
+  const float eps = (float)real(a[4]);
   ASSERT(bits > 0 && bits <= 32, "bits must be in 2..8");
-  const Shared s(x, mask, bits, pack);
-  const c10::DeviceGuard guard(x.device());
-  const at::Tensor q = empty({s.sh[0], s.sh[1], s.sh[2], s.last}, pack ? at::kInt : at::kChar, x);
-  const at::Tensor scale = empty(at::IntArrayRef(s.sshape, 4), at::kFloat, x);
-  at::Tensor zp;
-  if (asym) zp = empty(at::IntArrayRef(s.sshape, 4), at::kFloat, x);
-  const size_t ws_bytes = std::max<size_t>(varq_quant_workspace_bytes(s.sh, mask), 8);
-  const at::Tensor ws = empty({(int64_t)ws_bytes}, at::kByte, x);
-  check(varq_quant_pack(x.data_ptr(), dtype_code(x), s.sh, mask, (int)bits, asym, (float)real(a[4]), pack ? ptr<int32_t>(q) : nullptr,
-                        pack ? nullptr : ptr<int8_t>(q), ptr<float>(scale), asym ? ptr<float>(zp) : nullptr, nullptr, ws.data_ptr(), ws_bytes,
-                        stream_of(x)), "varq_quant_pack");
+  const Shared s(x0, mask, bits, pack);
+  const int dt = dtype_code(x0);
+  const c10::DeviceGuard guard(x0.device());
+  at::Tensor q, scale, zp;
+  unlocked("varq_quant_pack", [&] {
+    const at::Tensor x = x0.contiguous();
+    q = empty({s.sh[0], s.sh[1], s.sh[2], s.last}, pack ? at::kInt : at::kChar, x);
+    scale = empty(at::IntArrayRef(s.sshape, 4), at::kFloat, x);
+    if (asym) zp = empty(at::IntArrayRef(s.sshape, 4), at::kFloat, x);
+    const size_t ws_bytes = std::max<size_t>(varq_quant_workspace_bytes(s.sh, mask), 8);
+    const at::Tensor ws = empty({(int64_t)ws_bytes}, at::kByte, x);
+    return varq_quant_pack(x.data_ptr(), dt, s.sh, mask, (int)bits, asym, eps, pack ? ptr<int32_t>(q) : nullptr, pack ? nullptr : ptr<int8_t>(q),
+                           ptr<float>(scale), asym ? ptr<float>(zp) : nullptr, nullptr, ws.data_ptr(), ws_bytes, stream_of(x));
+  });
   return triple(q, scale, zp);
 }
 
@@ -186,20 +208,22 @@ PyObject *quant_step(PyObject *const *a, Py_ssize_t n_args) {
   const int64_t per_tok = d == 1 ? sh[2] : 1, row = sh[d == 1 ? 2 : 1] * sh[3];
   const int64_t map[3] = {sh[d] * per_tok, (buf[0]->size(d) - sh[d]) * per_tok, start * per_tok};
   const c10::DeviceGuard guard(t.device());
-  const size_t one = std::max<size_t>(varq_quant_workspace_bytes(sh, mask), 8), ws_bytes = two ? 2 * one : one;
-  const at::Tensor ws = empty({(int64_t)ws_bytes}, at::kByte, t);
+  const int dt = dtype_code(t);
   const float eps = (float)real(a[3]);
   float *s[2], *z[2];
   for (int i = 0; i < (two ? 2 : 1); ++i) {
     s[i] = ptr<float>(tab[i]) + k * row;
     z[i] = asym ? ptr<float>(ztab[i]) + k * row : nullptr;
   }
-  if (two)
-    check(varq_quant_pack2(x[0]->data_ptr(), x[1]->data_ptr(), dtype_code(t), sh, mask, (int)bits, asym, eps, ptr<int32_t>(buf[0]), nullptr, s[0], z[0],
-                           ptr<int32_t>(buf[1]), nullptr, s[1], z[1], map, ws.data_ptr(), ws_bytes, stream_of(t)), "varq_quant_pack2");
-  else
-    check(varq_quant_pack(x[0]->data_ptr(), dtype_code(t), sh, mask, (int)bits, asym, eps, ptr<int32_t>(buf[0]), nullptr, s[0], z[0], map,
-                          ws.data_ptr(), ws_bytes, stream_of(t)), "varq_quant_pack");
+  unlocked(two ? "varq_quant_pack2" : "varq_quant_pack", [&] {
+    const size_t one = std::max<size_t>(varq_quant_workspace_bytes(sh, mask), 8), ws_bytes = two ? 2 * one : one;
+    const at::Tensor ws = empty({(int64_t)ws_bytes}, at::kByte, t);
+    if (two)
+      return varq_quant_pack2(x[0]->data_ptr(), x[1]->data_ptr(), dt, sh, mask, (int)bits, asym, eps, ptr<int32_t>(buf[0]), nullptr, s[0], z[0],
+                              ptr<int32_t>(buf[1]), nullptr, s[1], z[1], map, ws.data_ptr(), ws_bytes, stream_of(t));
+    return varq_quant_pack(x[0]->data_ptr(), dt, sh, mask, (int)bits, asym, eps, ptr<int32_t>(buf[0]), nullptr, s[0], z[0], map, ws.data_ptr(),
+                           ws_bytes, stream_of(t));
+  });
   Py_RETURN_NONE;
 }
 
@@ -221,36 +245,48 @@ PyObject *quant_step_dequant(PyObject *const *a) {
   ASSERT((k + 1) * H * c <= tab.numel() && tab.scalar_type() == at::kFloat && (!ztab || ztab->sizes() == tab.sizes()), "quant_step_dequant: tables");
   const int64_t sh[4] = {B, x.size(1), x.size(2), c};
   const c10::DeviceGuard guard(x.device());
-  const size_t ws_bytes = std::max<size_t>(varq_quant_workspace_bytes(sh, d == 1 ? 0b0011 : 0b0101), 8);
-  const at::Tensor ws = empty({(int64_t)ws_bytes}, at::kByte, x);
-  const at::Tensor out = d == 1 ? empty({B, start + n, H, c}, dtype_of((int)code), x) : empty({B, H, start + n, c}, dtype_of((int)code), x);
-  check(varq_quant_step_dequant(x.data_ptr(), dtype_code(x), (int)B, (int)H, (int)n, (int)c, d == 1, (int)bits, asym, (float)real(a[2]), ptr<int32_t>(buf), buf.size(d),
-                                ptr<float>(tab), asym ? ptr<float>(ztab) : nullptr, k + 1, ends, out.data_ptr(), (int)code, ws.data_ptr(), ws_bytes, stream_of(x)),
-        "varq_quant_step_dequant");
+  const int dt = dtype_code(x);
+  const float eps = (float)real(a[2]);
+  at::Tensor out;
+  unlocked("varq_quant_step_dequant", [&] {
+    const size_t ws_bytes = std::max<size_t>(varq_quant_workspace_bytes(sh, d == 1 ? 0b0011 : 0b0101), 8);
+    const at::Tensor ws = empty({(int64_t)ws_bytes}, at::kByte, x);
+    out = d == 1 ? empty({B, start + n, H, c}, dtype_of((int)code), x) : empty({B, H, start + n, c}, dtype_of((int)code), x);
+    return varq_quant_step_dequant(x.data_ptr(), dt, (int)B, (int)H, (int)n, (int)c, d == 1, (int)bits, asym, eps, ptr<int32_t>(buf), buf.size(d), ptr<float>(tab),
+                                   asym ? ptr<float>(ztab) : nullptr, k + 1, ends, out.data_ptr(), (int)code, ws.data_ptr(), ws_bytes, stream_of(x));
+  });
   return wrap(out);
 }
 
 // ---- pack / unpack of int8 codes ----------------------------------------------------------------
 // pack(codes, bits) -> words
 PyObject *pack(PyObject *const *a) {
-  const at::Tensor codes = gpu(a[0], "q_int8").contiguous();
-  const int64_t bits = integer(a[1]), c = codes.size(-1), vals = 32 / bits, rows = c ? codes.numel() / c : 0;
-  c10::DimVector shape(codes.sizes().begin(), codes.sizes().end());
+  const at::Tensor &codes0 = gpu(a[0], "q_int8");
+  const int64_t bits = integer(a[1]), c = codes0.size(-1), vals = 32 / bits, rows = c ? codes0.numel() / c : 0;
+  c10::DimVector shape(codes0.sizes().begin(), codes0.sizes().end());
   shape.back() = (c + vals - 1) / vals;
-  const c10::DeviceGuard guard(codes.device());
-  const at::Tensor words = empty(shape, at::kInt, codes);
-  check(varq_pack(ptr<int8_t>(codes), rows, (int)c, (int)bits, ptr<int32_t>(words), stream_of(codes)), "varq_pack");
+  const c10::DeviceGuard guard(codes0.device());
+  at::Tensor words;
+  unlocked("varq_pack", [&] {
+    const at::Tensor codes = codes0.contiguous();
+    words = empty(shape, at::kInt, codes);
+    return varq_pack(ptr<int8_t>(codes), rows, (int)c, (int)bits, ptr<int32_t>(words), stream_of(codes));
+  });
   return wrap(words);
 }
 // unpack(words, c, bits) -> codes
 PyObject *unpack(PyObject *const *a) {
-  const at::Tensor words = gpu(a[0], "packed").contiguous();
-  const int64_t c = integer(a[1]), bits = integer(a[2]), w = words.size(-1), rows = w ? words.numel() / w : 0;
-  c10::DimVector shape(words.sizes().begin(), words.sizes().end());
+  const at::Tensor &words0 = gpu(a[0], "packed");
+  const int64_t c = integer(a[1]), bits = integer(a[2]), w = words0.size(-1), rows = w ? words0.numel() / w : 0;
+  c10::DimVector shape(words0.sizes().begin(), words0.sizes().end());
   shape.back() = c;
-  const c10::DeviceGuard guard(words.device());
-  const at::Tensor codes = empty(shape, at::kChar, words);
-  check(varq_unpack(ptr<int32_t>(words), rows, (int)c, (int)bits, ptr<int8_t>(codes), stream_of(words)), "varq_unpack");
+  const c10::DeviceGuard guard(words0.device());
+  at::Tensor codes;
+  unlocked("varq_unpack", [&] {
+    const at::Tensor words = words0.contiguous();
+    codes = empty(shape, at::kChar, words);
+    return varq_unpack(ptr<int32_t>(words), rows, (int)c, (int)bits, ptr<int8_t>(codes), stream_of(words));
+  });
   return wrap(codes);
 }
 
@@ -278,34 +314,34 @@ PyObject *dequant(PyObject *const *a) {
   ASSERT(q.dim() == 4 && scale.dim() == 4, "dequant: 4-D codes and scale");
   const bool packed = q.scalar_type() == at::kInt;
   ASSERT(packed || q.scalar_type() == at::kChar, "dequant: int32 words or int8 codes");
-  const int64_t wq = q.size(3);
-  const bool dense = q.is_contiguous();
-  if (!dense && (q.stride(3) != 1 || !wq || q.stride(0) % wq || q.stride(1) % wq || q.stride(2) % wq)) q = q.contiguous();
-  if (zp.defined() && (zp.sizes() != scale.sizes() || zp.strides() != scale.strides())) {
-    zp = zp.expand_as(scale).contiguous();
-    scale = scale.contiguous();
-  }
-  const int64_t s3 = scale.size(3);
+  const int64_t wq = q.size(3), s3 = scale.size(3);
   ASSERT(s3 > 0 && c % s3 == 0, "scale last dim %lld does not divide c=%lld", (long long)s3, (long long)c);
   int64_t sh[4] = {q.size(0), q.size(1), q.size(2), c}, ss[4], map[8];
-  for (int d = 0; d < 4; ++d) {
+  for (int d = 0; d < 4; ++d)
     ASSERT(d == 3 || scale.size(d) == 1 || scale.size(d) == q.size(d), "scale dim %d = %lld vs %lld", d, (long long)scale.size(d), (long long)q.size(d));
-    ss[d] = scale.size(d) == 1 ? 0 : scale.stride(d);
-  }
   const c10::DeviceGuard guard(q.device());
-  const at::Tensor out = empty(at::IntArrayRef(sh, 4), dtype_of((int)code), q);
-  bool mapped = false;
-  if (q.is_contiguous()) {
-    // (leading dims that the scale does not depend on collapse: fuller blocks)
-    if (!ss[0] && !ss[1] && !ss[2]) { sh[2] = sh[0] * sh[1] * sh[2]; sh[0] = sh[1] = 1; }
-  } else {
-    const int64_t m[8] = {sh[0], sh[1], sh[2], q.stride(0) / wq, q.stride(1) / wq, q.stride(2) / wq, 0, -1};
-    std::copy(m, m + 8, map);
-    mapped = true;
-  }
-  rows_as_channels(packed, sh, ss, c / s3, bits, mapped ? map : nullptr);
-  check(varq_dequant(packed ? ptr<int32_t>(q) : nullptr, packed ? nullptr : ptr<int8_t>(q), ptr<float>(scale), zp.defined() ? ptr<float>(zp) : nullptr,
-                     sh, ss, (int)(c / s3), (int)bits, mapped ? map : nullptr, out.data_ptr(), (int)code, stream_of(q)), "varq_dequant");
+  at::Tensor out;
+  unlocked("varq_dequant", [&] {
+    if (!q.is_contiguous() && (q.stride(3) != 1 || !wq || q.stride(0) % wq || q.stride(1) % wq || q.stride(2) % wq)) q = q.contiguous();
+    if (zp.defined() && (zp.sizes() != scale.sizes() || zp.strides() != scale.strides())) {
+      zp = zp.expand_as(scale).contiguous();
+      scale = scale.contiguous();
+    }
+    for (int d = 0; d < 4; ++d) ss[d] = scale.size(d) == 1 ? 0 : scale.stride(d);
+    out = empty(at::IntArrayRef(sh, 4), dtype_of((int)code), q);
+    bool mapped = false;
+    if (q.is_contiguous()) {
+      // (leading dims that the scale does not depend on collapse: fuller blocks)
+      if (!ss[0] && !ss[1] && !ss[2]) { sh[2] = sh[0] * sh[1] * sh[2]; sh[0] = sh[1] = 1; }
+    } else {
+      const int64_t m[8] = {sh[0], sh[1], sh[2], q.stride(0) / wq, q.stride(1) / wq, q.stride(2) / wq, 0, -1};
+      std::copy(m, m + 8, map);
+      mapped = true;
+    }
+    rows_as_channels(packed, sh, ss, c / s3, bits, mapped ? map : nullptr);
+    return varq_dequant(packed ? ptr<int32_t>(q) : nullptr, packed ? nullptr : ptr<int8_t>(q), ptr<float>(scale), zp.defined() ? ptr<float>(zp) : nullptr,
+                        sh, ss, (int)(c / s3), (int)bits, mapped ? map : nullptr, out.data_ptr(), (int)code, stream_of(q));
+  });
   return wrap(out);
 }
 
@@ -322,9 +358,12 @@ PyObject *dequant_steps(PyObject *const *a) {
   const int64_t B = buf.size(0), H = buf.size(3 - d);
   ASSERT(tab.is_contiguous() && tab.scalar_type() == at::kFloat && tab.numel() >= nseg * H * c && (!ztab || ztab->sizes() == tab.sizes()), "dequant_steps: tables");
   const c10::DeviceGuard guard(buf.device());
-  const at::Tensor out = d == 1 ? empty({B, ends[nseg - 1], H, c}, dtype_of((int)code), buf) : empty({B, H, ends[nseg - 1], c}, dtype_of((int)code), buf);
-  check(varq_dequant_steps(ptr<int32_t>(buf), ptr<float>(tab), ptr<float>(ztab), nseg, ends, (int)B, (int)H, buf.size(d), (int)c, (int)bits, d == 1,
-                           out.data_ptr(), (int)code, stream_of(buf)), "varq_dequant_steps");
+  at::Tensor out;
+  unlocked("varq_dequant_steps", [&] {
+    out = d == 1 ? empty({B, ends[nseg - 1], H, c}, dtype_of((int)code), buf) : empty({B, H, ends[nseg - 1], c}, dtype_of((int)code), buf);
+    return varq_dequant_steps(ptr<int32_t>(buf), ptr<float>(tab), ptr<float>(ztab), nseg, ends, (int)B, (int)H, buf.size(d), (int)c, (int)bits, d == 1,
+                              out.data_ptr(), (int)code, stream_of(buf));
+  });
   return wrap(out);
 }
 
@@ -332,7 +371,11 @@ PyObject *dequant_steps(PyObject *const *a) {
 struct AttnShape {
   int64_t B, Hq, Lq, D, Hkv, Lstride;
   int layout;   // of the call, out included
+  int64_t out_size[4];
   at::Tensor out;
+  void new_out(const at::Tensor &q) {
+    if (!out.defined()) out = empty(at::IntArrayRef(out_size, 4), q.scalar_type(), q);
+  }
 };
 
 int layout_code(PyObject *o) {
@@ -342,7 +385,7 @@ int layout_code(PyObject *o) {
   return VARQ_LAYOUT_BLHC;
 }
 
-// the layout of the call and its result tensor
+// the layout of the call and its result tensor; s.out is not there yet (see new_out) unless the caller brought one
 void make_out(AttnShape &s, const at::Tensor &q, PyObject *out, int lay, int olay) {
   s.layout = lay;
   if (olay != lay) {
@@ -350,9 +393,8 @@ void make_out(AttnShape &s, const at::Tensor &q, PyObject *out, int lay, int ola
     s.layout = VARQ_LAYOUT_BHLC_OUT_BLHC;
   }
   const int64_t n[4] = {s.B, olay == VARQ_LAYOUT_BHLC ? s.Hq : s.Lq, olay == VARQ_LAYOUT_BHLC ? s.Lq : s.Hq, s.D};
-  if (out == Py_None) {
-    s.out = empty(at::IntArrayRef(n, 4), q.scalar_type(), q);
-  } else {
+  std::copy(n, n + 4, s.out_size);
+  if (out != Py_None) {
     s.out = gpu(out, "out");
     ASSERT(s.out.scalar_type() == q.scalar_type() && s.out.sizes() == at::IntArrayRef(n, 4) && s.out.is_contiguous(),
            "out must be contiguous, of the dtype of q and of the shape its layout implies");
@@ -396,7 +438,7 @@ PyObject *attn(PyObject *const *a) {
   const at::Tensor *kz = maybe(a[3], "k_zp"), *vz = maybe(a[6], "v_zp"), *limit = maybe(a[11], "kv_limit"), *map = maybe(a[12], "head_map");
   const int64_t k_bits = integer(a[7]), v_bits = integer(a[8]), Lk = integer(a[9]), splits = integer(a[14]);
   const c10::DeviceGuard guard(q.device());
-  const AttnShape s = attn_shape(q, kw, a[13], a[15], a[17]);
+  AttnShape s = attn_shape(q, kw, a[13], a[15], a[17]);
   ASSERT(vw.dim() == 4 && ks.dim() == 4 && vs.dim() == 4, "4-D cache tensors");
   for (int d = 0; d < 3; ++d)
     ASSERT(vw.size(d) == kw.size(d) && ks.size(d) == kw.size(d) && vs.size(d) == kw.size(d), "words and scales must agree in batch, heads and tokens");
@@ -408,13 +450,18 @@ PyObject *attn(PyObject *const *a) {
          "scales must be fp32 and words int32");
   ASSERT(0 <= Lk && Lk <= s.Lstride, "Lk=%lld outside the cache of %lld tokens", (long long)Lk, (long long)s.Lstride);
   check_limit_and_map(limit, map, s);
-  const size_t ws_bytes = workspace_bytes(s, Lk, 1, splits);
-  at::Tensor ws;
-  if (ws_bytes) ws = empty({(int64_t)ws_bytes}, at::kByte, q);
-  check(varq_fused_attn(q.data_ptr(), s.out.data_ptr(), ptr<int32_t>(kw), ptr<float>(ks), ptr<float>(kz), (int)k_bits, (int)(s.D / ks.size(3)),
-                        ptr<int32_t>(vw), ptr<float>(vs), ptr<float>(vz), (int)v_bits, (int)(s.D / vs.size(3)), (int)s.B, (int)s.Hq, (int)s.Hkv,
-                        ptr<int32_t>(map), (int)s.Lq, (int)Lk, (int)s.Lstride, (int)s.D, ptr<int32_t>(limit), (float)real(a[10]), s.layout, io_code(q),
-                        truth(a[16]), ws_bytes ? ws.data_ptr() : nullptr, ws_bytes, (int)splits, stream_of(q)), "varq_fused_attn");
+  const float softmax_scale = (float)real(a[10]);
+  const bool exact = truth(a[16]);
+  unlocked("varq_fused_attn", [&] {
+    s.new_out(q);
+    const size_t ws_bytes = workspace_bytes(s, Lk, 1, splits);
+    at::Tensor ws;
+    if (ws_bytes) ws = empty({(int64_t)ws_bytes}, at::kByte, q);
+    return varq_fused_attn(q.data_ptr(), s.out.data_ptr(), ptr<int32_t>(kw), ptr<float>(ks), ptr<float>(kz), (int)k_bits, (int)(s.D / ks.size(3)),
+                           ptr<int32_t>(vw), ptr<float>(vs), ptr<float>(vz), (int)v_bits, (int)(s.D / vs.size(3)), (int)s.B, (int)s.Hq, (int)s.Hkv,
+                           ptr<int32_t>(map), (int)s.Lq, (int)Lk, (int)s.Lstride, (int)s.D, ptr<int32_t>(limit), softmax_scale, s.layout, io_code(q),
+                           exact, ws_bytes ? ws.data_ptr() : nullptr, ws_bytes, (int)splits, stream_of(q));
+  });
   return wrap(s.out);
 }
 
@@ -425,7 +472,7 @@ PyObject *attn_channel(PyObject *const *a) {
   const at::Tensor *kz = maybe(a[3], "k_chan_zp"), *vz = maybe(a[6], "v_chan_zp"), *limit = maybe(a[10], "kv_limit"), *map = maybe(a[11], "head_map");
   const int64_t bits = integer(a[7]), Lk = integer(a[8]), splits = integer(a[14]);
   const c10::DeviceGuard guard(q.device());
-  const AttnShape s = attn_shape(q, kw, a[12], a[15], a[16]);
+  AttnShape s = attn_shape(q, kw, a[12], a[15], a[16]);
   ASSERT(vw.sizes() == kw.sizes() && kw.size(3) * 32 == s.D * bits, "K and V words must agree and match the head dim and the bit-width");
   int32_t ends[16];
   int nseg = 1;
@@ -449,52 +496,57 @@ PyObject *attn_channel(PyObject *const *a) {
   ASSERT(kw.scalar_type() == at::kInt && vw.scalar_type() == at::kInt, "words must be int32");
   ASSERT(0 <= Lk && Lk <= s.Lstride, "Lk=%lld outside the cache of %lld tokens", (long long)Lk, (long long)s.Lstride);
   check_limit_and_map(limit, map, s);
-  const size_t ws_bytes = workspace_bytes(s, Lk, nseg, splits);
-  at::Tensor ws;
-  if (ws_bytes) ws = empty({(int64_t)ws_bytes}, at::kByte, q);
-  check(varq_fused_attn_channel(q.data_ptr(), s.out.data_ptr(), ptr<int32_t>(kw), ptr<float>(ks), ptr<float>(kz), ptr<int32_t>(vw), ptr<float>(vs),
-                                ptr<float>(vz), nseg, seg ? ends : nullptr, (int)bits, (int)s.B, (int)s.Hq, (int)s.Hkv, ptr<int32_t>(map), (int)s.Lq,
-                                (int)Lk, (int)s.Lstride, (int)s.D, ptr<int32_t>(limit), (float)real(a[9]), s.layout, io_code(q),
-                                ws_bytes ? ws.data_ptr() : nullptr, ws_bytes, (int)splits, stream_of(q)), "varq_fused_attn_channel");
+  const float softmax_scale = (float)real(a[9]);
+  unlocked("varq_fused_attn_channel", [&] {
+    s.new_out(q);
+    const size_t ws_bytes = workspace_bytes(s, Lk, nseg, splits);
+    at::Tensor ws;
+    if (ws_bytes) ws = empty({(int64_t)ws_bytes}, at::kByte, q);
+    return varq_fused_attn_channel(q.data_ptr(), s.out.data_ptr(), ptr<int32_t>(kw), ptr<float>(ks), ptr<float>(kz), ptr<int32_t>(vw), ptr<float>(vs),
+                                   ptr<float>(vz), nseg, seg ? ends : nullptr, (int)bits, (int)s.B, (int)s.Hq, (int)s.Hkv, ptr<int32_t>(map), (int)s.Lq,
+                                   (int)Lk, (int)s.Lstride, (int)s.D, ptr<int32_t>(limit), softmax_scale, s.layout, io_code(q),
+                                   ws_bytes ? ws.data_ptr() : nullptr, ws_bytes, (int)splits, stream_of(q));
+  });
   return wrap(s.out);
 }
 
 // ---- packed cache -------------------------------------------------------------------------------
 // The cache hands its buffers over as one tuple of constants, built once:
 // (B, H, Lmax, D, group, asym, eps, ((bits, heads, k_words, k_scale, k_zp, v_words, v_scale, v_zp, slot, head_map), ...))
-struct Cache {
-  int64_t B, H, Lmax, D, group;
-  bool asym;
-  float eps;
-  PyObject *classes;
-  explicit Cache(PyObject *t) {
-    auto at_ = [&](int i) { return PyTuple_GET_ITEM(t, i); };
-    ASSERT(PyTuple_Check(t) && PyTuple_GET_SIZE(t) == 8, "cache tuple");
-    B = integer(at_(0)); H = integer(at_(1)); Lmax = integer(at_(2)); D = integer(at_(3)); group = integer(at_(4));
-    asym = truth(at_(5)); eps = (float)real(at_(6)); classes = at_(7);
-  }
-  Py_ssize_t size() const { return PyTuple_GET_SIZE(classes); }
-};
 struct CacheClass {
   int64_t bits, heads;
   at::Tensor k_words, k_scale, k_zp, v_words, v_scale, v_zp, slot, head_map;
-  explicit CacheClass(PyObject *t) {
+  void read(PyObject *t) {
     auto g = [&](int i) -> const at::Tensor & { return THPVariable_Unpack(PyTuple_GET_ITEM(t, i)); };
     bits = integer(PyTuple_GET_ITEM(t, 0)); heads = integer(PyTuple_GET_ITEM(t, 1));
     k_words = g(2); k_scale = g(3); k_zp = g(4); v_words = g(5); v_scale = g(6); v_zp = g(7); slot = g(8); head_map = g(9);
   }
 };
+struct Cache {
+  int64_t B, H, Lmax, D, group;
+  bool asym;
+  float eps;
+  int n;
+  CacheClass classes[3];
+  explicit Cache(PyObject *t) {
+    auto at_ = [&](int i) { return PyTuple_GET_ITEM(t, i); };
+    ASSERT(PyTuple_Check(t) && PyTuple_GET_SIZE(t) == 8, "cache tuple");
+    B = integer(at_(0)); H = integer(at_(1)); Lmax = integer(at_(2)); D = integer(at_(3)); group = integer(at_(4));
+    asym = truth(at_(5)); eps = (float)real(at_(6));
+    n = (int)PyTuple_GET_SIZE(at_(7));
+    ASSERT(n >= 1 && n <= 3, "a cache has 1..3 bit-width classes");
+    for (int i = 0; i < n; ++i) classes[i].read(PyTuple_GET_ITEM(at_(7), i));
+  }
+};
 
 // the classes of a cache as the C ABI takes them
 int class_table(const Cache &c, varq_kv_class (&t)[3]) {
-  const Py_ssize_t n = c.size();
-  ASSERT(n >= 1 && n <= 3, "a cache has 1..3 bit-width classes");
-  for (Py_ssize_t i = 0; i < n; ++i) {
-    const CacheClass k(PyTuple_GET_ITEM(c.classes, i));
+  for (int i = 0; i < c.n; ++i) {
+    const CacheClass &k = c.classes[i];
     t[i] = {(int)k.bits, (int)k.heads, ptr<int32_t>(k.head_map), ptr<int32_t>(k.slot), ptr<int32_t>(k.k_words), ptr<int32_t>(k.v_words),
             ptr<float>(k.k_scale), c.asym ? ptr<float>(k.k_zp) : nullptr, ptr<float>(k.v_scale), c.asym ? ptr<float>(k.v_zp) : nullptr};
   }
-  return (int)n;
+  return c.n;
 }
 
 // cache_attend(cache, len, q, softmax_scale, kv_limit, out, splits, out_layout) -> out: all classes of a mixed-width cache
@@ -513,12 +565,16 @@ PyObject *cache_attend(PyObject *const *a) {
   check_limit_and_map(limit, nullptr, s);
   varq_kv_class t[3];
   const int n = class_table(c, t);
-  const size_t ws_bytes = workspace_bytes(s, len, 1, splits);
-  at::Tensor ws;
-  if (ws_bytes) ws = empty({(int64_t)ws_bytes}, at::kByte, q);
-  check(varq_fused_attn_classes(q.data_ptr(), s.out.data_ptr(), t, n, (int)c.group, (int)c.B, (int)c.H, (int)s.Lq, (int)len, (int)c.Lmax, (int)c.D,
-                                ptr<int32_t>(limit), (float)real(a[3]), s.layout, io_code(q), ws_bytes ? ws.data_ptr() : nullptr, ws_bytes, (int)splits,
-                                stream_of(q)), "varq_fused_attn_classes");
+  const float softmax_scale = (float)real(a[3]);
+  unlocked("varq_fused_attn_classes", [&] {
+    s.new_out(q);
+    const size_t ws_bytes = workspace_bytes(s, len, 1, splits);
+    at::Tensor ws;
+    if (ws_bytes) ws = empty({(int64_t)ws_bytes}, at::kByte, q);
+    return varq_fused_attn_classes(q.data_ptr(), s.out.data_ptr(), t, n, (int)c.group, (int)c.B, (int)c.H, (int)s.Lq, (int)len, (int)c.Lmax, (int)c.D,
+                                   ptr<int32_t>(limit), softmax_scale, s.layout, io_code(q), ws_bytes ? ws.data_ptr() : nullptr, ws_bytes, (int)splits,
+                                   stream_of(q));
+  });
   return wrap(s.out);
 }
 
@@ -533,40 +589,48 @@ PyObject *cache_append(PyObject *const *a) {
   const int64_t n = k.size(3 - h);
   ASSERT(len + n <= c.Lmax, "cache overflow");
   gpu(a[2], "k"); gpu(a[3], "v");
-  k = k.contiguous(); v = v.contiguous();
   const c10::DeviceGuard guard(k.device());
-  void *const st = stream_of(k);
   const int kd = dtype_code(k), vd = dtype_code(v);
-  const int64_t rows = c.B * c.H * n;
-  if (c.size() > 1) {   // (one launch for all classes, where the sizes allow it)
-    varq_kv_class t[3];
-    const int nc = class_table(c, t);
-    auto classes = [&](const void *kp, const void *vp, int dt) {
-      return varq_quant_pack_classes(kp, vp, dt, lay, (int)c.B, (int)c.H, n, (int)c.D, (int)c.group, c.asym, c.eps, t, nc, c.Lmax, len, st);
-    };
-    int rc = kd == vd ? classes(k.data_ptr(), v.data_ptr(), kd) : classes(k.data_ptr(), nullptr, kd);
-    if (kd != vd && rc == VARQ_OK) rc = classes(nullptr, v.data_ptr(), vd);
-    if (rc == VARQ_OK) return PyLong_FromLongLong(n);
-    if (rc != VARQ_ERR_UNSUPPORTED) check(rc, "varq_quant_pack_classes");
-  }
-  for (Py_ssize_t i = 0; i < c.size(); ++i) {
-    const CacheClass cl(PyTuple_GET_ITEM(c.classes, i));
-    // input rows in memory order -> output row b*hc*Lmax + slot(h)*Lmax + len + l
-    const int64_t bs = cl.heads * c.Lmax;
-    const int64_t bhlc[8] = {c.B, c.H, n, bs, c.Lmax, 1, len, 1}, blhc[8] = {c.B, n, c.H, bs, 1, c.Lmax, len, 2};
-    const int64_t *map = lay == VARQ_LAYOUT_BHLC ? bhlc : blhc;
-    float *kz = c.asym ? ptr<float>(cl.k_zp) : nullptr, *vz = c.asym ? ptr<float>(cl.v_zp) : nullptr;
-    if (kd == vd && 2 * c.B <= 65535) {
-      check(varq_quant_pack_rows2(k.data_ptr(), v.data_ptr(), kd, rows, (int)c.D, (int)c.group, (int)cl.bits, c.asym, c.eps, map, ptr<int32_t>(cl.slot),
-                                  ptr<int32_t>(cl.k_words), ptr<float>(cl.k_scale), kz, ptr<int32_t>(cl.v_words), ptr<float>(cl.v_scale), vz, st),
-            "varq_quant_pack_rows2");
-    } else {   // K and V of different dtypes (Infinity: fp32 K after cos-norm, bf16 V)
-      check(varq_quant_pack_rows(k.data_ptr(), kd, rows, (int)c.D, (int)c.group, (int)cl.bits, c.asym, c.eps, map, ptr<int32_t>(cl.slot),
-                                 ptr<int32_t>(cl.k_words), ptr<float>(cl.k_scale), kz, st), "varq_quant_pack_rows");
-      check(varq_quant_pack_rows(v.data_ptr(), vd, rows, (int)c.D, (int)c.group, (int)cl.bits, c.asym, c.eps, map, ptr<int32_t>(cl.slot),
-                                 ptr<int32_t>(cl.v_words), ptr<float>(cl.v_scale), vz, st), "varq_quant_pack_rows");
+  const char *what = "varq_quant_pack_classes";
+  const int rc = status_unlocked([&] {
+    k = k.contiguous(); v = v.contiguous();
+    void *const st = stream_of(k);
+    const int64_t rows = c.B * c.H * n;
+    if (c.n > 1) {   // (one launch for all classes, where the sizes allow it)
+      varq_kv_class t[3];
+      const int nc = class_table(c, t);
+      auto classes = [&](const void *kp, const void *vp, int dt) {
+        return varq_quant_pack_classes(kp, vp, dt, lay, (int)c.B, (int)c.H, n, (int)c.D, (int)c.group, c.asym, c.eps, t, nc, c.Lmax, len, st);
+      };
+      int rc = kd == vd ? classes(k.data_ptr(), v.data_ptr(), kd) : classes(k.data_ptr(), nullptr, kd);
+      if (kd != vd && rc == VARQ_OK) rc = classes(nullptr, v.data_ptr(), vd);
+      if (rc != VARQ_ERR_UNSUPPORTED) return rc;
     }
-  }
+    for (int i = 0; i < c.n; ++i) {
+      const CacheClass &cl = c.classes[i];
+      // input rows in memory order -> output row b*hc*Lmax + slot(h)*Lmax + len + l
+      const int64_t bs = cl.heads * c.Lmax;
+      const int64_t bhlc[8] = {c.B, c.H, n, bs, c.Lmax, 1, len, 1}, blhc[8] = {c.B, n, c.H, bs, 1, c.Lmax, len, 2};
+      const int64_t *map = lay == VARQ_LAYOUT_BHLC ? bhlc : blhc;
+      float *kz = c.asym ? ptr<float>(cl.k_zp) : nullptr, *vz = c.asym ? ptr<float>(cl.v_zp) : nullptr;
+      int rc;
+      if (kd == vd && 2 * c.B <= 65535) {
+        what = "varq_quant_pack_rows2";
+        rc = varq_quant_pack_rows2(k.data_ptr(), v.data_ptr(), kd, rows, (int)c.D, (int)c.group, (int)cl.bits, c.asym, c.eps, map, ptr<int32_t>(cl.slot),
+                                   ptr<int32_t>(cl.k_words), ptr<float>(cl.k_scale), kz, ptr<int32_t>(cl.v_words), ptr<float>(cl.v_scale), vz, st);
+      } else {   // K and V of different dtypes (Infinity: fp32 K after cos-norm, bf16 V)
+        what = "varq_quant_pack_rows";
+        rc = varq_quant_pack_rows(k.data_ptr(), kd, rows, (int)c.D, (int)c.group, (int)cl.bits, c.asym, c.eps, map, ptr<int32_t>(cl.slot),
+                                  ptr<int32_t>(cl.k_words), ptr<float>(cl.k_scale), kz, st);
+        if (rc == VARQ_OK)
+          rc = varq_quant_pack_rows(v.data_ptr(), vd, rows, (int)c.D, (int)c.group, (int)cl.bits, c.asym, c.eps, map, ptr<int32_t>(cl.slot),
+                                    ptr<int32_t>(cl.v_words), ptr<float>(cl.v_scale), vz, st);
+      }
+      if (rc != VARQ_OK) return rc;
+    }
+    return (int)VARQ_OK;
+  });
+  check(rc, what);
   return PyLong_FromLongLong(n);
 }
 
@@ -574,7 +638,7 @@ PyObject *cache_append(PyObject *const *a) {
 PyObject *cache_prepare(PyObject *const *a) {
   const Cache c(a[0]);
   const int64_t len = integer(a[1]), start = integer(a[8]);
-  const at::Tensor qkv = gpu(a[2], "qkv").contiguous();
+  at::Tensor qkv = gpu(a[2], "qkv");
   ASSERT(qkv.dim() == 5 && qkv.size(2) == 3 && qkv.size(0) == c.B && qkv.size(3) == c.H && qkv.size(4) == c.D, "append_from_qkv: qkv [B,n,3,H,D] of the cache's sizes");
   const int64_t n = qkv.size(1);
   ASSERT(len + n <= c.Lmax, "cache overflow");
@@ -585,25 +649,34 @@ PyObject *cache_prepare(PyObject *const *a) {
   }
   if (mul) ASSERT(mul->scalar_type() == at::kFloat && mul->numel() == c.H && mul->is_contiguous(), "q_scale_mul must be contiguous fp32 [H]");
   const c10::DeviceGuard guard(qkv.device());
-  const at::Tensor q = empty({c.B, c.H, n, c.D}, at::kBFloat16, qkv);
-  if (c.size() > 1) {
-    varq_kv_class t[3];
-    const int nc = class_table(c, t);
-    const int rc = varq_qkv_prepare_classes(qkv.data_ptr(), dtype_code(qkv), (int)c.B, (int)n, (int)c.H, (int)c.D, ptr<float>(mul), truth(a[4]),
-                                            (float)real(a[5]), ptr<float>(cs), ptr<float>(sn), (int)start, q.data_ptr(), (int)c.group, c.asym,
-                                            c.eps, t, nc, c.Lmax, len, stream_of(qkv));
-    if (rc == VARQ_OK) return wrap(q);
-    if (rc != VARQ_ERR_UNSUPPORTED) check(rc, "varq_qkv_prepare_classes");
-  }
-  for (Py_ssize_t i = 0; i < c.size(); ++i) {
-    const CacheClass cl(PyTuple_GET_ITEM(c.classes, i));
-    const int64_t map[8] = {c.B, n, c.H, cl.heads * c.Lmax, 1, c.Lmax, len, 2};
-    check(varq_qkv_prepare_append(qkv.data_ptr(), dtype_code(qkv), (int)c.B, (int)n, (int)c.H, (int)c.D, ptr<float>(mul), truth(a[4]), (float)real(a[5]),
-                                  ptr<float>(cs), ptr<float>(sn), (int)start, q.data_ptr(), (int)c.group, (int)cl.bits, c.asym, c.eps, map,
-                                  ptr<int32_t>(cl.slot), ptr<int32_t>(cl.k_words), ptr<float>(cl.k_scale), c.asym ? ptr<float>(cl.k_zp) : nullptr,
-                                  ptr<int32_t>(cl.v_words), ptr<float>(cl.v_scale), c.asym ? ptr<float>(cl.v_zp) : nullptr, stream_of(qkv)),
-          "varq_qkv_prepare_append");
-  }
+  const int dt = dtype_code(qkv);
+  const bool l2norm = truth(a[4]);
+  const float norm_eps = (float)real(a[5]);
+  at::Tensor q;
+  const char *what = "varq_qkv_prepare_classes";
+  const int rc = status_unlocked([&] {
+    qkv = qkv.contiguous();
+    q = empty({c.B, c.H, n, c.D}, at::kBFloat16, qkv);
+    if (c.n > 1) {
+      varq_kv_class t[3];
+      const int nc = class_table(c, t);
+      const int rc = varq_qkv_prepare_classes(qkv.data_ptr(), dt, (int)c.B, (int)n, (int)c.H, (int)c.D, ptr<float>(mul), l2norm, norm_eps, ptr<float>(cs),
+                                              ptr<float>(sn), (int)start, q.data_ptr(), (int)c.group, c.asym, c.eps, t, nc, c.Lmax, len, stream_of(qkv));
+      if (rc != VARQ_ERR_UNSUPPORTED) return rc;
+    }
+    what = "varq_qkv_prepare_append";
+    for (int i = 0; i < c.n; ++i) {
+      const CacheClass &cl = c.classes[i];
+      const int64_t map[8] = {c.B, n, c.H, cl.heads * c.Lmax, 1, c.Lmax, len, 2};
+      const int rc = varq_qkv_prepare_append(qkv.data_ptr(), dt, (int)c.B, (int)n, (int)c.H, (int)c.D, ptr<float>(mul), l2norm, norm_eps, ptr<float>(cs),
+                                             ptr<float>(sn), (int)start, q.data_ptr(), (int)c.group, (int)cl.bits, c.asym, c.eps, map, ptr<int32_t>(cl.slot),
+                                             ptr<int32_t>(cl.k_words), ptr<float>(cl.k_scale), c.asym ? ptr<float>(cl.k_zp) : nullptr,
+                                             ptr<int32_t>(cl.v_words), ptr<float>(cl.v_scale), c.asym ? ptr<float>(cl.v_zp) : nullptr, stream_of(qkv));
+      if (rc != VARQ_OK) return rc;
+    }
+    return (int)VARQ_OK;
+  });
+  check(rc, what);
   return wrap(q);
 }
 
