@@ -511,31 +511,83 @@ PyObject *attn_channel(PyObject *const *a) {
 }
 
 // ---- packed cache -------------------------------------------------------------------------------
-// The cache hands its buffers over as one tuple of constants, built once:
-// (B, H, Lmax, D, group, asym, eps, ((bits, heads, k_words, k_scale, k_zp, v_words, v_scale, v_zp, slot, head_map), ...))
+// A PackedKVCache as its attributes say at the time of the call: a caller may have replaced buffers, or set others of them.
+// attribute `name` (an interned string) of o: out of the instance's own dictionary where it has one and the name is there, which
+// takes a third of the general way's time
+PyObject *attribute(PyObject *o, PyObject *name) {   // (a new reference)
+  PyObject **const d = _PyObject_GetDictPtr(o);
+  PyObject *v = d && *d ? PyDict_GetItemWithError(*d, name) : nullptr;
+  if (v) {
+    Py_INCREF(v);
+    return v;
+  }
+  if (PyErr_Occurred() || !(v = PyObject_GetAttr(o, name))) throw python_error();
+  return v;
+}
+struct Ref {   // owns the reference it is given
+  PyObject *const o;
+  explicit Ref(PyObject *owned) : o(owned) { if (!o) throw python_error(); }
+  Ref(const Ref &) = delete;
+  ~Ref() { Py_DECREF(o); }
+};
+#define NAME(id) ([]() { static PyObject *const name = PyUnicode_InternFromString(#id); return name; }())
+
 struct CacheClass {
   int64_t bits, heads;
   at::Tensor k_words, k_scale, k_zp, v_words, v_scale, v_zp, slot, head_map;
-  void read(PyObject *t) {
-    auto g = [&](int i) -> const at::Tensor & { return THPVariable_Unpack(PyTuple_GET_ITEM(t, i)); };
-    bits = integer(PyTuple_GET_ITEM(t, 0)); heads = integer(PyTuple_GET_ITEM(t, 1));
-    k_words = g(2); k_scale = g(3); k_zp = g(4); v_words = g(5); v_scale = g(6); v_zp = g(7); slot = g(8); head_map = g(9);
+
+  static at::Tensor dense(PyObject *of, PyObject *name, at::ScalarType dt) {
+    const Ref a(attribute(of, name));
+    const at::Tensor &t = gpu(a.o, PyUnicode_AsUTF8(name));
+    ASSERT(t.scalar_type() == dt && t.is_contiguous(), "cache buffer %U must be contiguous and of type %s", name, toString(dt));
+    return t;
+  }
+  void read(PyObject *o, int64_t H, bool asym) {
+    bits = integer(Ref(attribute(o, NAME(bits))).o);
+    const Py_ssize_t n = PyObject_Size(Ref(attribute(o, NAME(heads))).o);
+    if (n < 0) throw python_error();
+    heads = n;
+    k_words = dense(o, NAME(k_words), at::kInt); v_words = dense(o, NAME(v_words), at::kInt);
+    k_scale = dense(o, NAME(k_scale), at::kFloat); v_scale = dense(o, NAME(v_scale), at::kFloat);
+    if (asym) { k_zp = dense(o, NAME(k_zp), at::kFloat); v_zp = dense(o, NAME(v_zp), at::kFloat); }
+    slot = dense(o, NAME(slot), at::kInt); head_map = dense(o, NAME(head_map), at::kInt);
+    ASSERT(heads > 0 && slot.numel() == H && head_map.numel() == heads, "cache class of %lld bits: slot and head_map do not fit its heads", (long long)bits);
+  }
+  // the kernels trust the sizes: rows as long as the call implies, and the last one it reaches inside
+  void check(int64_t D, int64_t group, int64_t last) const {
+    const int64_t W = D * bits / 32, ng = D / group;
+    for (const auto &[w, sc, z] : {std::tuple(&k_words, &k_scale, &k_zp), std::tuple(&v_words, &v_scale, &v_zp)}) {
+      if (!w->dim() || !sc->dim() || w->size(-1) != W || sc->size(-1) != ng || (z->defined() && z->sizes() != sc->sizes()))
+        raise(g_varq_error, "cache class of %lld bits: rows of words, scales and zero-points must have %lld, %lld and %lld entries", (long long)bits, (long long)W, (long long)ng, (long long)ng);
+      if (last >= w->numel() / W || last >= sc->numel() / ng)
+        raise(g_varq_error, "cache class of %lld bits: the call reaches row %lld of buffers that hold %lld rows", (long long)bits, (long long)last,
+              (long long)std::min(w->numel() / W, sc->numel() / ng));
+    }
   }
 };
 struct Cache {
   int64_t B, H, Lmax, D, group;
   bool asym;
   float eps;
-  int n;
+  int n = 0;
   CacheClass classes[3];
-  explicit Cache(PyObject *t) {
-    auto at_ = [&](int i) { return PyTuple_GET_ITEM(t, i); };
-    ASSERT(PyTuple_Check(t) && PyTuple_GET_SIZE(t) == 8, "cache tuple");
-    B = integer(at_(0)); H = integer(at_(1)); Lmax = integer(at_(2)); D = integer(at_(3)); group = integer(at_(4));
-    asym = truth(at_(5)); eps = (float)real(at_(6));
-    n = (int)PyTuple_GET_SIZE(at_(7));
-    ASSERT(n >= 1 && n <= 3, "a cache has 1..3 bit-width classes");
-    for (int i = 0; i < n; ++i) classes[i].read(PyTuple_GET_ITEM(at_(7), i));
+  explicit Cache(PyObject *o) {
+    auto number = [&](PyObject *name) { return integer(Ref(attribute(o, name)).o); };
+    B = number(NAME(B)); H = number(NAME(H)); Lmax = number(NAME(Lmax)); D = number(NAME(D)); group = number(NAME(group));
+    asym = !truth(Ref(attribute(o, NAME(symmetric))).o);
+    eps = (float)real(Ref(attribute(o, NAME(eps))).o);
+    ASSERT(B > 0 && H > 0 && D >= 16 && group > 0 && D % group == 0, "cache sizes");
+    const Ref list(attribute(o, NAME(classes))), seq(PySequence_Fast(list.o, "classes must be a sequence"));
+    const Py_ssize_t count = PySequence_Fast_GET_SIZE(seq.o);
+    ASSERT(count >= 1 && count <= 3, "a cache has 1..3 bit-width classes");
+    for (; n < count; ++n) {
+      classes[n].read(PySequence_Fast_GET_ITEM(seq.o, n), H, asym);
+      ASSERT(classes[n].bits == 2 || classes[n].bits == 4 || classes[n].bits == 8, "a class has 2, 4 or 8 bits");
+    }
+  }
+  // every class holds tokens 0..len-1 (token j of a head lies Lmax rows from that of the next)
+  void check(int64_t len) const {
+    for (int i = 0; i < n; ++i) classes[i].check(D, group, (B * classes[i].heads - 1) * Lmax + len - 1);
   }
 };
 
@@ -558,6 +610,7 @@ PyObject *cache_attend(PyObject *const *a) {
   ASSERT((q.scalar_type() == at::kBFloat16 || q.scalar_type() == at::kHalf) && q.dim() == 4, "q must be bf16 or fp16");
   ASSERT(q.size(0) == c.B && q.size(1) == c.H && q.size(3) == c.D, "attend: q does not fit the cache");
   ASSERT(0 < len && len <= c.Lmax, "attend: the cache holds no such token");
+  c.check(len);
   const c10::DeviceGuard guard(q.device());
   AttnShape s;
   s.B = c.B; s.Hq = s.Hkv = c.H; s.Lq = q.size(2); s.D = c.D; s.Lstride = c.Lmax;
@@ -587,7 +640,8 @@ PyObject *cache_append(PyObject *const *a) {
   const int lay = layout_code(a[4]), h = lay == VARQ_LAYOUT_BHLC ? 1 : 2;
   ASSERT(k.dim() == 4 && k.size(0) == c.B && k.size(h) == c.H && k.size(3) == c.D && v.sizes() == k.sizes(), "append: the step does not fit the cache");
   const int64_t n = k.size(3 - h);
-  ASSERT(len + n <= c.Lmax, "cache overflow");
+  ASSERT(len >= 0 && len + n <= c.Lmax, "cache overflow");
+  c.check(len + n);
   gpu(a[2], "k"); gpu(a[3], "v");
   const c10::DeviceGuard guard(k.device());
   const int kd = dtype_code(k), vd = dtype_code(v);
@@ -641,7 +695,8 @@ PyObject *cache_prepare(PyObject *const *a) {
   at::Tensor qkv = gpu(a[2], "qkv");
   ASSERT(qkv.dim() == 5 && qkv.size(2) == 3 && qkv.size(0) == c.B && qkv.size(3) == c.H && qkv.size(4) == c.D, "append_from_qkv: qkv [B,n,3,H,D] of the cache's sizes");
   const int64_t n = qkv.size(1);
-  ASSERT(len + n <= c.Lmax, "cache overflow");
+  ASSERT(len >= 0 && len + n <= c.Lmax, "cache overflow");
+  c.check(len + n);
   const at::Tensor *mul = maybe(a[3], "q_scale_mul"), *cs = maybe(a[6], "rope cos"), *sn = maybe(a[7], "rope sin");
   if (cs || sn) {
     ASSERT(cs && sn && cs->dim() == 2 && cs->scalar_type() == at::kFloat && sn->scalar_type() == at::kFloat && cs->is_contiguous() && sn->is_contiguous(), "rope tables must be contiguous fp32");

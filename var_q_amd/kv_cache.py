@@ -50,10 +50,6 @@ class PackedKVCache:
         self.classes: List[_BitClass] = [
             _BitClass(b, [h for h in range(H) if per_head[h] == b], B, H, Lmax, D, group_size, device)
             for b in sorted(set(per_head))]
-        # what the native host layer reads, built once: sizes and the buffers of every class
-        self._native = (B, H, Lmax, D, group_size, not symmetric, eps,
-                        tuple((c.bits, len(c.heads), c.k_words, c.k_scale, c.k_zp, c.v_words, c.v_scale, c.v_zp, c.slot, c.head_map)
-                              for c in self.classes))
 
     def reset(self):
         self.len = 0
@@ -128,7 +124,7 @@ class PackedKVCache:
         """Quantize + pack one step into tokens len..len+n of the cache.  The step is
         [B,H,n,D] (layout 'BHLc') or [B,n,H,D] ('BLHc', the flash-attention layout of
         VAR/models/basic_var.py:127-131); either is read where it lies."""
-        self.len += _lib.host().cache_append(self._native, self.len, k, v, layout)
+        self.len += _lib.host().cache_append(self, self.len, k, v, layout)
 
     def append_from_qkv(self, qkv: torch.Tensor, q_scale_mul: Optional[torch.Tensor] = None, l2norm: bool = False,
                         norm_eps: float = 1e-12, rope=None, token_start: Optional[int] = None) -> torch.Tensor:
@@ -137,7 +133,7 @@ class PackedKVCache:
         as bf16 [B,H,n,D] (Infinity/infinity/models/basic.py:316-330 in one kernel).
         token_start (default: the cache length) selects the rotary table rows."""
         cos, sin = (None, None) if rope is None else rope
-        q = _lib.host().cache_prepare(self._native, self.len, qkv, q_scale_mul, l2norm, norm_eps, cos, sin,
+        q = _lib.host().cache_prepare(self, self.len, qkv, q_scale_mul, l2norm, norm_eps, cos, sin,
                                       self.len if token_start is None else token_start)
         self.len += q.shape[2]
         return q
@@ -157,7 +153,7 @@ class PackedKVCache:
                                     c.bits, c.bits, self.len, softmax_scale, kv_limit, None, out, self.splits, 'BHLc', exact_codes,
                                     out_layout)
         if self.concurrent_classes and not exact_codes:
-            return _lib.host().cache_attend(self._native, self.len, q, softmax_scale, kv_limit, out, self.splits, out_layout)
+            return _lib.host().cache_attend(self, self.len, q, softmax_scale, kv_limit, out, self.splits, out_layout)
         if out is None:
             B_, H_, Lq_, D_ = q.shape
             out = torch.empty((B_, Lq_, H_, D_) if out_layout == 'BLHc' else q.shape, dtype=q.dtype, device=q.device)
