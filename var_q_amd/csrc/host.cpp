@@ -259,10 +259,14 @@ PyObject *quant_step_dequant(PyObject *const *a) {
 }
 
 // ---- pack / unpack of int8 codes ----------------------------------------------------------------
+int64_t codes_per_word(int64_t bits) {
+  ASSERT(bits == 2 || bits == 4 || bits == 8, "bits must be 2, 4 or 8 (got %lld)", (long long)bits);
+  return 32 / bits;
+}
 // pack(codes, bits) -> words
 PyObject *pack(PyObject *const *a) {
   const at::Tensor &codes0 = gpu(a[0], "q_int8");
-  const int64_t bits = integer(a[1]), c = codes0.size(-1), vals = 32 / bits, rows = c ? codes0.numel() / c : 0;
+  const int64_t bits = integer(a[1]), c = codes0.size(-1), vals = codes_per_word(bits), rows = c ? codes0.numel() / c : 0;
   c10::DimVector shape(codes0.sizes().begin(), codes0.sizes().end());
   shape.back() = (c + vals - 1) / vals;
   const c10::DeviceGuard guard(codes0.device());
@@ -277,7 +281,8 @@ PyObject *pack(PyObject *const *a) {
 // unpack(words, c, bits) -> codes
 PyObject *unpack(PyObject *const *a) {
   const at::Tensor &words0 = gpu(a[0], "packed");
-  const int64_t c = integer(a[1]), bits = integer(a[2]), w = words0.size(-1), rows = w ? words0.numel() / w : 0;
+  const int64_t c = integer(a[1]), bits = integer(a[2]), w = words0.size(-1), rows = w ? words0.numel() / w : 0, vals = codes_per_word(bits);
+  ASSERT(rows == 0 || w == (c + vals - 1) / vals, "unpack: rows of %lld words do not hold %lld codes of %lld bits", (long long)w, (long long)c, (long long)bits);
   c10::DimVector shape(words0.sizes().begin(), words0.sizes().end());
   shape.back() = c;
   const c10::DeviceGuard guard(words0.device());
@@ -315,6 +320,8 @@ PyObject *dequant(PyObject *const *a) {
   const bool packed = q.scalar_type() == at::kInt;
   ASSERT(packed || q.scalar_type() == at::kChar, "dequant: int32 words or int8 codes");
   const int64_t wq = q.size(3), s3 = scale.size(3);
+  const int64_t vals = packed ? codes_per_word(bits) : 1;
+  ASSERT(!q.numel() || wq == (c + vals - 1) / vals, "dequant: rows of %lld entries do not hold %lld channels", (long long)wq, (long long)c);
   ASSERT(s3 > 0 && c % s3 == 0, "scale last dim %lld does not divide c=%lld", (long long)s3, (long long)c);
   int64_t sh[4] = {q.size(0), q.size(1), q.size(2), c}, ss[4], map[8];
   for (int d = 0; d < 4; ++d)
