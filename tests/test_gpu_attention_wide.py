@@ -12,6 +12,7 @@ import varq_oracle as O
 from gpu_util import note
 from test_gpu_attention import _compare
 from var_q_amd import ops
+from var_q_amd._lib import VarqError
 
 pytestmark = pytest.mark.gpu
 
@@ -88,6 +89,18 @@ def test_stepwise_tables_and_head_map(dev, D, bits, asym, dtype):
     back = torch.empty_like(perm)
     back[perm] = torch.arange(H)
     _check(run(), run(splits=1), q, deq[0][:, back.to(dev)], deq[1][:, back.to(dev)], 0.05, dt, what)
+
+
+@pytest.mark.parametrize('D,k_group,v_group', [(128, 16, 16), (128, 4, 4), (128, 64, 32), (128, 128, 64), (64, 8, 8), (64, 16, 32)])
+def test_groups_without_a_kernel_are_refused_at_every_size(dev, D, k_group, v_group):
+    """... also where the call is large enough for the path that could widen some of them."""
+    B, H, Lq, Lk = 2, 16, 1600, 2100
+    q = torch.zeros(B, H, Lq, D, dtype=torch.bfloat16, device=dev)
+    words, scale = torch.zeros(B, H, Lk, D // 8, dtype=torch.int32, device=dev), lambda g: torch.ones(B, H, Lk, D // g, device=dev)
+    for splits in (0, 1):
+        note('wide: groups', D, k_group, v_group, splits)
+        with pytest.raises(VarqError):
+            ops.fused_attn(q, words, scale(k_group), None, words, scale(v_group), None, 4, 4, Lk, 0.1, splits=splits)
 
 
 def test_logits_that_climb_move_the_reference(dev):

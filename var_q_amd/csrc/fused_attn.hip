@@ -1444,6 +1444,10 @@ int dispatch_groups(const AttnParams &p, int gk, int gv, hipStream_t st) {
 #undef VARQ_G
   return -1;
 }
+// the pairs above: what the other paths of the same call are held to as well
+bool groups_served(int D, int gk, int gv) {
+  return ((gk == gv && (gk == 128 || gk == 64 || gk == 32)) || (gk == 32 && gv == 64)) && gk <= D;
+}
 
 template <int D, int G, int NWV, int WPS, bool F16>
 void launch_classes_shape(const AttnParams &p, const ClassTable &t, hipStream_t st) {
@@ -2143,7 +2147,7 @@ extern "C" int varq_fused_attn(const void *q, void *out,
     VARQ_CHECK_LAUNCH("fused_attn");
     return VARQ_OK;
   }
-  if ((splits == 0 || splits == 1) && !p.exact_codes && wide_eligible(p.bh_total, Lq, Lk, D) &&
+  if ((splits == 0 || splits == 1) && !p.exact_codes && groups_served(D, k_group, v_group) && wide_eligible(p.bh_total, Lq, Lk, D) &&
       run_wide(p, D, splits, workspace, workspace_bytes, st, [&](char *ws) { launch_expand(p, D, k_bits, k_group, v_group, false, ws, st); })) {
     VARQ_CHECK_LAUNCH("fused_attn");
     return VARQ_OK;
