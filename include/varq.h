@@ -299,8 +299,10 @@ size_t varq_fused_attn_workspace_bytes(int B, int Hkv, int Lq, int Lk, int D, in
  * this many bytes and splits = 0 or 1, the attention entry points dequantize K and V once into matrix
  * operands kept there and stream those, instead of dequantizing every key tile again for each block of
  * queries.  Same operands, same result to rounding.  0: not worth it for this shape.  (A caller that
- * leaves the choice to the library passes a workspace of the larger of the two sizes.) */
+ * leaves the choice to the library passes a workspace of the larger of the two sizes.)
+ * ..._limits: the same for a call with kv_limit. */
 size_t varq_fused_attn_expand_bytes(int B, int Hkv, int Lq, int Lk, int D);
+size_t varq_fused_attn_expand_bytes_limits(int B, int Hkv, int Lq, int Lk, int D);
 /* Over how many workgroups varq_fused_attn shares the keys of a query block out when that is left
  * to it (splits = 0) and the workspace has room; 1 = not at all.  (A report for callers and
  * benchmarks; no counterpart in the reference.) */

@@ -83,6 +83,18 @@ template <bool F16> __device__ __forceinline__ floatx16_t mfma_32x32x16(u32x4_t 
 // holds key 16*(i/8) + 8*h + i%8.
 __device__ __forceinline__ int kperm(int r) { return (r & 0x13) | ((r & 4) << 1) | ((r & 8) >> 1); }
 
+// Workgroup `slot` of an XCD that has `groups` (batch, head) pairs of q_tiles query tiles, under a key limit that grows
+// with the query (the block-causal rule), which makes the query tiles of a pair differ in length: windows of `win` pairs
+// one after the other, in a window the last query tiles of all its pairs first, so that the short ones even out what is left.
+struct HeavyFirst {
+  int grp, qt;
+  __device__ __forceinline__ HeavyFirst(int slot, int q_tiles, int groups, int win) {
+    const int first = slot / (win * q_tiles) * win, n = min(win, groups - first);
+    const int r = slot - first * q_tiles;
+    qt = q_tiles - 1 - r / n;
+    grp = first + r % n;
+  }
+};
 
 // ---- the wide path (wide_attn.hip): K and V expanded once, then attended by many query blocks ----
 struct WidePlan {
@@ -90,7 +102,8 @@ struct WidePlan {
   size_t tile_bytes;    // the expanded tiles, at the start of the workspace
   size_t ws_bytes;      // ... and the partial results behind them
 };
-WidePlan plan_wide(int64_t bh, int Lq, int Lk, int D, int cus, bool share);   // share: whether blocks may be shared out
+// share: whether blocks may be shared out; limits: whether the queries have key limits
+WidePlan plan_wide(int64_t bh, int Lq, int Lk, int D, int cus, bool share, bool limits);
 // Expands the packed cache of p (per-key groups of k_group / v_group channels, or the per-channel
 // tables) into `tiles`, pair after pair; with `place`, the pairs of a bit-width class to the places of
 // their heads (p.head_map) among the p.Hq heads of the cache.

@@ -1184,13 +1184,10 @@ struct BlockOf {
     int grp = slot / p.q_tiles;
     qt = slot % p.q_tiles;
     if (p.kv_limit && p.q_tiles > 1) {
-      // Under a key limit that grows with the query (the block-causal rule) the query tiles of a pair differ in
-      // length: the pairs whose workgroups are resident together (64 on an XCD at two per compute unit) start
-      // their last query tiles first, and the short ones even out what is left.
-      const int win = max(64 / p.q_tiles, 1), first = slot / (win * p.q_tiles) * win, n = min(win, groups - first);
-      const int r = slot - first * p.q_tiles;
-      qt = p.q_tiles - 1 - r / n;
-      grp = first + r % n;
+      // (windows of the pairs whose workgroups are resident together, 64 on an XCD at two per compute unit)
+      const HeavyFirst k(slot, p.q_tiles, groups, max(64 / p.q_tiles, 1));
+      qt = k.qt;
+      grp = k.grp;
     }
     pair = p.kv_hs == 1 && p.kv_ts > 1 ? xcd * groups + grp : grp * 8 + xcd;
   }
@@ -2051,18 +2048,30 @@ template <int BITS> void launch_fewq(const AttnParams &p, hipStream_t st) {
 // kernel above / this): D=128 B=2 H=16 1024 x 2521 69 / 75, 1300 x 3000 109 / 104, 1600 x 4121 146 / 134,
 // 2304 x 6425 339 / 250; B=8 1024 x 2521 198 / 208, 1300 x 3000 325 / 311, 2304 x 6425 1116 / 953; B=1 H=8
 // 1600 x 4121 59 / 69; D=64 B=2 1600 x 4121 105 / 95, B=8 1300 x 3000 181 / 191, 2304 x 6425 609 / 578.
-bool wide_eligible(int64_t bh, int Lq, int Lk, int D) {
-  return Lq >= (D == 128 ? 1280 : 1536) && Lk >= 2048 && bh * ((Lq + 255) / 256) >= 160 && bh <= 65535;
+// Under key limits (measured with the block-causal rule over a whole sequence, pairs x tokens): D=128 all of 16 to 128
+// pairs x 2521 to 10521 are as fast or faster, 16 x 2521 99 / 98, 128 x 2521 353 / 346, 48 x 2952 243 / 192, 32 x 4121
+// 288 / 218, 32 x 10521 1303 / 1057.  D=64 gains where the longest query blocks are the whole of the time, up to about
+// a block and a quarter per compute unit, 16 x 2521 72 / 66, 24 x 3256 88 / 80, 16 x 4121 108 / 97, and in long sequences,
+// 32 x 6425 305 / 277, 128 x 6425 1112 / 1060; in between it goes either way, 32 x 3256 94 / 102, 128 x 4121 522 / 528,
+// 320 x 2952 665 / 715, 48 x 5417 321 / 330.
+bool wide_eligible(int64_t bh, int Lq, int Lk, int D, bool limits) {
+  const int64_t blocks = bh * ((Lq + 255) / 256);
+  if (limits && D == 64 && Lq < 6144 && blocks > device_cus() * 5 / 4) return false;
+  return Lq >= (D == 128 ? 1280 : 1536) && Lk >= 2048 && blocks >= 160 && bh <= 65535;
 }
 // The launches of the wide path, or false when the workspace does not hold what they need.
 template <class Expand>
 bool run_wide(const AttnParams &p, int D, int splits, void *workspace, size_t workspace_bytes, hipStream_t st, Expand &&expand) {
-  const WidePlan plan = plan_wide(p.bh_total, p.Lq, p.Lk, D, device_cus(), splits == 0);
+  const WidePlan plan = plan_wide(p.bh_total, p.Lq, p.Lk, D, device_cus(), splits == 0, p.kv_limit != nullptr);
   if (!workspace || ((uintptr_t)workspace & 15) || workspace_bytes < plan.ws_bytes) return false;
   char *const ws = reinterpret_cast<char *>(workspace);
   expand(ws);
   launch_wide(p, D, plan, ws, st);
   return true;
+}
+size_t expand_bytes(int B, int Hkv, int Lq, int Lk, int D, bool limits) {
+  if (B <= 0 || Hkv <= 0 || Lq <= 0 || Lk <= 0 || (D != 64 && D != 128) || !wide_eligible((int64_t)B * Hkv, Lq, Lk, D, limits)) return 0;
+  return plan_wide((int64_t)B * Hkv, Lq, Lk, D, device_cus(), true, limits).ws_bytes;
 }
 
 }  // namespace
@@ -2080,9 +2089,9 @@ extern "C" size_t varq_fused_attn_workspace_bytes(int B, int Hkv, int Lq, int Lk
 }
 
 extern "C" size_t varq_fused_attn_expand_bytes(int B, int Hkv, int Lq, int Lk, int D) {
-  if (B <= 0 || Hkv <= 0 || Lq <= 0 || Lk <= 0 || (D != 64 && D != 128) || !wide_eligible((int64_t)B * Hkv, Lq, Lk, D)) return 0;
-  return plan_wide((int64_t)B * Hkv, Lq, Lk, D, device_cus(), true).ws_bytes;
+  return expand_bytes(B, Hkv, Lq, Lk, D, false);
 }
+extern "C" size_t varq_fused_attn_expand_bytes_limits(int B, int Hkv, int Lq, int Lk, int D) { return expand_bytes(B, Hkv, Lq, Lk, D, true); }
 
 extern "C" int varq_fused_attn_key_shares(int B, int Hkv, int Lq, int Lk, int D, int k_group, int v_group) {
   if (B <= 0 || Hkv <= 0 || Lq <= 0 || Lk <= 0 || (D != 64 && D != 128)) return 0;
@@ -2147,7 +2156,7 @@ extern "C" int varq_fused_attn(const void *q, void *out,
     VARQ_CHECK_LAUNCH("fused_attn");
     return VARQ_OK;
   }
-  if ((splits == 0 || splits == 1) && !p.exact_codes && groups_served(D, k_group, v_group) && wide_eligible(p.bh_total, Lq, Lk, D) &&
+  if ((splits == 0 || splits == 1) && !p.exact_codes && groups_served(D, k_group, v_group) && wide_eligible(p.bh_total, Lq, Lk, D, kv_limit != nullptr) &&
       run_wide(p, D, splits, workspace, workspace_bytes, st, [&](char *ws) { launch_expand(p, D, k_bits, k_group, v_group, false, ws, st); })) {
     VARQ_CHECK_LAUNCH("fused_attn");
     return VARQ_OK;
@@ -2228,7 +2237,7 @@ extern "C" int varq_fused_attn_channel(const void *q, void *out,
   p.exact_codes = 0;
   if (int e = set_layout(p, layout, "fused_attn_channel")) return e;
   hipStream_t st = (hipStream_t)stream;
-  if ((splits == 0 || splits == 1) && wide_eligible(p.bh_total, Lq, Lk, D) &&
+  if ((splits == 0 || splits == 1) && wide_eligible(p.bh_total, Lq, Lk, D, kv_limit != nullptr) &&
       run_wide(p, D, splits, workspace, workspace_bytes, st, [&](char *ws) { launch_expand(p, D, bits, D, D, true, ws, st); })) {
     VARQ_CHECK_LAUNCH("fused_attn_channel");
     return VARQ_OK;
@@ -2298,7 +2307,7 @@ extern "C" int varq_fused_attn_classes(const void *q, void *out, const varq_kv_c
     set_few(p, workspace, workspace_bytes);
     hipLaunchKernelGGL(fused_attn_fewq_classes_kernel, few_grid(p), dim3(FQ_NW * 64), FewQLds::kBytes, st, p, t);
     if (p.nsplit > 1) launch_combine<FQ_D, false>(p, st);
-  } else if ((splits == 0 || splits == 1) && wide_eligible(p.bh_total, Lq, Lk, D) &&
+  } else if ((splits == 0 || splits == 1) && wide_eligible(p.bh_total, Lq, Lk, D, kv_limit != nullptr) &&
              run_wide(p, D, splits, workspace, workspace_bytes, st, [&](char *ws) {
                // (one expanding launch per class, into the places of its heads)
                for (int i = 0; i < 3; ++i) {

@@ -433,9 +433,10 @@ void check_limit_and_map(const at::Tensor *limit, const at::Tensor *map, const A
 int io_code(const at::Tensor &q) { return q.scalar_type() == at::kHalf ? VARQ_F16 : VARQ_BF16; }
 
 // device memory for a launch that shares keys out or expands them (0: neither)
-size_t workspace_bytes(const AttnShape &s, int64_t Lk, int nseg, int64_t splits) {
+size_t workspace_bytes(const AttnShape &s, int64_t Lk, int nseg, int64_t splits, bool limits) {
   const size_t shared = varq_fused_attn_workspace_bytes((int)s.B, (int)s.Hkv, (int)s.Lq, (int)Lk, (int)s.D, nseg, (int)splits);
-  return splits > 1 ? shared : std::max(shared, varq_fused_attn_expand_bytes((int)s.B, (int)s.Hkv, (int)s.Lq, (int)Lk, (int)s.D));
+  const auto expand = limits ? varq_fused_attn_expand_bytes_limits : varq_fused_attn_expand_bytes;
+  return splits > 1 ? shared : std::max(shared, expand((int)s.B, (int)s.Hkv, (int)s.Lq, (int)Lk, (int)s.D));
 }
 
 // attn(q, k_words, k_scale, k_zp, v_words, v_scale, v_zp, k_bits, v_bits, Lk, softmax_scale, kv_limit, head_map, out, splits,
@@ -461,7 +462,7 @@ PyObject *attn(PyObject *const *a) {
   const bool exact = truth(a[16]);
   unlocked("varq_fused_attn", [&] {
     s.new_out(q);
-    const size_t ws_bytes = workspace_bytes(s, Lk, 1, splits);
+    const size_t ws_bytes = workspace_bytes(s, Lk, 1, splits, limit != nullptr);
     at::Tensor ws;
     if (ws_bytes) ws = empty({(int64_t)ws_bytes}, at::kByte, q);
     return varq_fused_attn(q.data_ptr(), s.out.data_ptr(), ptr<int32_t>(kw), ptr<float>(ks), ptr<float>(kz), (int)k_bits, (int)(s.D / ks.size(3)),
@@ -506,7 +507,7 @@ PyObject *attn_channel(PyObject *const *a) {
   const float softmax_scale = (float)real(a[9]);
   unlocked("varq_fused_attn_channel", [&] {
     s.new_out(q);
-    const size_t ws_bytes = workspace_bytes(s, Lk, nseg, splits);
+    const size_t ws_bytes = workspace_bytes(s, Lk, nseg, splits, limit != nullptr);
     at::Tensor ws;
     if (ws_bytes) ws = empty({(int64_t)ws_bytes}, at::kByte, q);
     return varq_fused_attn_channel(q.data_ptr(), s.out.data_ptr(), ptr<int32_t>(kw), ptr<float>(ks), ptr<float>(kz), ptr<int32_t>(vw), ptr<float>(vs),
@@ -628,7 +629,7 @@ PyObject *cache_attend(PyObject *const *a) {
   const float softmax_scale = (float)real(a[3]);
   unlocked("varq_fused_attn_classes", [&] {
     s.new_out(q);
-    const size_t ws_bytes = workspace_bytes(s, len, 1, splits);
+    const size_t ws_bytes = workspace_bytes(s, len, 1, splits, limit != nullptr);
     at::Tensor ws;
     if (ws_bytes) ws = empty({(int64_t)ws_bytes}, at::kByte, q);
     return varq_fused_attn_classes(q.data_ptr(), s.out.data_ptr(), t, n, (int)c.group, (int)c.B, (int)c.H, (int)s.Lq, (int)len, (int)c.Lmax, (int)c.D,
