@@ -47,7 +47,7 @@ enum varq_layout { VARQ_LAYOUT_BHLC = 0, VARQ_LAYOUT_BLHC = 1,
 
 /*
  * What the matrix operands of the fused attention hold.
- * VARQ_ATTN_REFERENCE_ROUNDING (the default form): K and V are dequantized as tiles enter LDS,
+ * VARQ_ATTN_REFERENCE_ROUNDING (the default form): K and V are dequantized on their way into LDS,
  *   (code - zp) * scale in fp32, and rounded to the attention's 16-bit type -- the very operands
  *   the reference's attention backend sees after dequant_all() and the downcast of its call
  *   (VAR_Q/quant.py:216-224, VAR/models/basic_var.py:158, Infinity/infinity/models/basic.py:344).
@@ -247,7 +247,8 @@ int varq_quant_step_dequant(const void *x, int x_dtype, int B, int H, int n, int
  * Infinity/infinity/models/basic.py:339-351).
  *
  *   out[b,h,i,:] = softmax_j( softmax_scale * q[b,h,i,:] . K[b,h,j,:] + mask(i,j) ) V[b,h,j,:]
- *   K = (k_codes - k_zp) * k_scale,  V likewise, never materialized.
+ *   K = (k_codes - k_zp) * k_scale,  V likewise, never kept in fp32; in 16 bits only while
+ *       a call of many queries runs, in the workspace (varq_fused_attn_expand_bytes below).
  *
  *   q, out     [B, Hq, Lq, D] of io_dtype: VARQ_BF16 (the Infinity path, bf16 autocast:
  *              Infinity/tools/run_infinity.py:519) or VARQ_F16 (the VAR path, fp16 autocast:
@@ -299,7 +300,9 @@ size_t varq_fused_attn_workspace_bytes(int B, int Hkv, int Lq, int Lk, int D, in
  * this many bytes and splits = 0 or 1, the attention entry points dequantize K and V once into matrix
  * operands kept there and stream those, instead of dequantizing every key tile again for each block of
  * queries.  Same operands, same result to rounding.  0: not worth it for this shape.  (A caller that
- * leaves the choice to the library passes a workspace of the larger of the two sizes.)
+ * leaves the choice to the library passes a workspace of the larger of the two sizes; with less the call
+ * is served by the other kernels.)  At most 1 GiB for the operands, 512 bytes per key and (batch, head) at
+ * D=128, and up to 68 MB for partial results: a larger batch is served part after part.
  * ..._limits: the same for a call with kv_limit. */
 size_t varq_fused_attn_expand_bytes(int B, int Hkv, int Lq, int Lk, int D);
 size_t varq_fused_attn_expand_bytes_limits(int B, int Hkv, int Lq, int Lk, int D);
@@ -341,7 +344,7 @@ int varq_fused_attn_classes(const void *q, void *out, const varq_kv_class *host_
  *                        segment k_chan_zp may be NULL for an affine K as well: it shifts
  *                        every logit of a query by the same amount, which the softmax cancels
  *                        (K is then offset per channel before it is rounded to bf16)
- * K and V are dequantized with the tables of each key's segment as tiles enter LDS,
+ * K and V are dequantized with the tables of each key's segment on their way into LDS,
  * (code - zp) * scale in fp32 rounded to io_dtype (bf16 or fp16, as in varq_fused_attn): the
  * operands of the reference's attention after dequant_all (VAR_Q/quant.py:216-224) and the
  * downcast of its attention call.

@@ -2042,6 +2042,18 @@ template <int BITS> void launch_fewq(const AttnParams &p, hipStream_t st) {
 }
 
 // ---- many queries: K and V expanded once, then a plain flash attention (wide_attn.hip) ----------
+// The expanded K and V of a call take at most 1 GiB of the caller's memory at a time; a larger batch is expanded and attended
+// part after part.  2.1 GB at once gain nothing over two parts, smaller parts end up to 8 % later (256 MiB / 512 MiB /
+// 1 GiB / no bound, us, 4 bits): 384 pairs, 4096 x 10521, 7710 / 7710 / 7715 / 7760-8000; 1600 x 4121 1576 / 1508 / 1460 / 1460-1500; D=64,
+// 960 pairs, 1600 x 4121 2312 / 2243 / 2214 / 2220.
+constexpr int64_t kExpandBytes = 1ll << 30;
+// That many batch entries are a part (0: not even one fits, and the call takes the kernel above).
+int wide_batch(int B, int Hkv, int Lk, int D) {
+  const int64_t most = kExpandBytes / ((int64_t)Hkv * ((Lk + BN - 1) / BN) * (2 * BN * D * 2));
+  if (most >= B || most == 0) return most ? B : 0;
+  const int64_t parts = (B + most - 1) / most;
+  return (int)((B + parts - 1) / parts);
+}
 // Worth it from five (D = 128) or six blocks of 256 queries per (batch, head) on: expanding costs what
 // widening costs the kernel above in a block or two, and then its way through memory; and on a device
 // that is not nearly full the three launches cost more than they save.  Measured (us, 4-bit codes, the
@@ -2054,24 +2066,47 @@ template <int BITS> void launch_fewq(const AttnParams &p, hipStream_t st) {
 // a block and a quarter per compute unit, 16 x 2521 72 / 66, 24 x 3256 88 / 80, 16 x 4121 108 / 97, and in long sequences,
 // 32 x 6425 305 / 277, 128 x 6425 1112 / 1060; in between it goes either way, 32 x 3256 94 / 102, 128 x 4121 522 / 528,
 // 320 x 2952 665 / 715, 48 x 5417 321 / 330.
-bool wide_eligible(int64_t bh, int Lq, int Lk, int D, bool limits) {
-  const int64_t blocks = bh * ((Lq + 255) / 256);
+bool wide_eligible(int B, int Hkv, int Lq, int Lk, int D, bool limits) {
+  const int64_t bh = (int64_t)wide_batch(B, Hkv, Lk, D) * Hkv, blocks = bh * ((Lq + 255) / 256);
   if (limits && D == 64 && Lq < 6144 && blocks > device_cus() * 5 / 4) return false;
   return Lq >= (D == 128 ? 1280 : 1536) && Lk >= 2048 && blocks >= 160 && bh <= 65535;
 }
-// The launches of the wide path, or false when the workspace does not hold what they need.
+// The largest workspace of the parts that the call is done in.
+size_t wide_bytes(int B, int Hkv, int Lq, int Lk, int D, bool share, bool limits) {
+  const int n = wide_batch(B, Hkv, Lk, D), last = B - (B - 1) / n * n;
+  auto bytes = [&](int b) { return plan_wide((int64_t)b * Hkv, Lq, Lk, D, device_cus(), share, limits).ws_bytes; };
+  return std::max(bytes(n), bytes(last));
+}
+// The launches of the wide path, part after part, or false when the workspace does not hold what they need.
+// expand(p, first, ws): the tiles of the batch entries first.. of the call, p.B of them.
 template <class Expand>
 bool run_wide(const AttnParams &p, int D, int splits, void *workspace, size_t workspace_bytes, hipStream_t st, Expand &&expand) {
-  const WidePlan plan = plan_wide(p.bh_total, p.Lq, p.Lk, D, device_cus(), splits == 0, p.kv_limit != nullptr);
-  if (!workspace || ((uintptr_t)workspace & 15) || workspace_bytes < plan.ws_bytes) return false;
+  const bool share = splits == 0, limits = p.kv_limit != nullptr;
+  if (!workspace || ((uintptr_t)workspace & 15) || workspace_bytes < wide_bytes(p.B, p.Hkv, p.Lq, p.Lk, D, share, limits)) return false;
   char *const ws = reinterpret_cast<char *>(workspace);
-  expand(ws);
-  launch_wide(p, D, plan, ws, st);
+  const int n = wide_batch(p.B, p.Hkv, p.Lk, D);
+  for (int first = 0; first < p.B; first += n) {
+    AttnParams c = p;
+    c.B = std::min(n, p.B - first);
+    c.bh_total = c.B * p.Hkv;
+    c.q += first * p.q_bs * D;
+    c.out += first * p.o_bs * D;
+    expand(c, first, ws);
+    launch_wide(c, D, plan_wide(c.bh_total, p.Lq, p.Lk, D, device_cus(), share, limits), ws, st);
+  }
   return true;
 }
+// The packed K and V of batch entry `first` and on (rows of D channels of `bits` bits; per-key scales of `groups` per row).
+void skip_entries(AttnParams &p, int first, int D, int bits, int k_groups, int v_groups) {
+  const int64_t rows = first * p.kv_bs, words = rows * (D * bits / 32);
+  p.k_words += words; p.v_words += words;
+  if (p.k_scale) { p.k_scale += rows * k_groups; p.v_scale += rows * v_groups; }
+  if (p.k_zp) p.k_zp += rows * k_groups;
+  if (p.v_zp) p.v_zp += rows * v_groups;
+}
 size_t expand_bytes(int B, int Hkv, int Lq, int Lk, int D, bool limits) {
-  if (B <= 0 || Hkv <= 0 || Lq <= 0 || Lk <= 0 || (D != 64 && D != 128) || !wide_eligible((int64_t)B * Hkv, Lq, Lk, D, limits)) return 0;
-  return plan_wide((int64_t)B * Hkv, Lq, Lk, D, device_cus(), true, limits).ws_bytes;
+  if (B <= 0 || Hkv <= 0 || Lq <= 0 || Lk <= 0 || (D != 64 && D != 128) || !wide_eligible(B, Hkv, Lq, Lk, D, limits)) return 0;
+  return wide_bytes(B, Hkv, Lq, Lk, D, true, limits);
 }
 
 }  // namespace
@@ -2156,8 +2191,11 @@ extern "C" int varq_fused_attn(const void *q, void *out,
     VARQ_CHECK_LAUNCH("fused_attn");
     return VARQ_OK;
   }
-  if ((splits == 0 || splits == 1) && !p.exact_codes && groups_served(D, k_group, v_group) && wide_eligible(p.bh_total, Lq, Lk, D, kv_limit != nullptr) &&
-      run_wide(p, D, splits, workspace, workspace_bytes, st, [&](char *ws) { launch_expand(p, D, k_bits, k_group, v_group, false, ws, st); })) {
+  if ((splits == 0 || splits == 1) && !p.exact_codes && groups_served(D, k_group, v_group) && wide_eligible(B, p.Hkv, Lq, Lk, D, kv_limit != nullptr) &&
+      run_wide(p, D, splits, workspace, workspace_bytes, st, [&](AttnParams c, int first, char *ws) {
+        skip_entries(c, first, D, k_bits, D / k_group, D / v_group);
+        launch_expand(c, D, k_bits, k_group, v_group, false, ws, st);
+      })) {
     VARQ_CHECK_LAUNCH("fused_attn");
     return VARQ_OK;
   }
@@ -2237,8 +2275,11 @@ extern "C" int varq_fused_attn_channel(const void *q, void *out,
   p.exact_codes = 0;
   if (int e = set_layout(p, layout, "fused_attn_channel")) return e;
   hipStream_t st = (hipStream_t)stream;
-  if ((splits == 0 || splits == 1) && wide_eligible(p.bh_total, Lq, Lk, D, kv_limit != nullptr) &&
-      run_wide(p, D, splits, workspace, workspace_bytes, st, [&](char *ws) { launch_expand(p, D, bits, D, D, true, ws, st); })) {
+  if ((splits == 0 || splits == 1) && wide_eligible(B, p.Hkv, Lq, Lk, D, kv_limit != nullptr) &&
+      run_wide(p, D, splits, workspace, workspace_bytes, st, [&](AttnParams c, int first, char *ws) {
+        skip_entries(c, first, D, bits, 0, 0);
+        launch_expand(c, D, bits, D, D, true, ws, st);
+      })) {
     VARQ_CHECK_LAUNCH("fused_attn_channel");
     return VARQ_OK;
   }
@@ -2307,18 +2348,19 @@ extern "C" int varq_fused_attn_classes(const void *q, void *out, const varq_kv_c
     set_few(p, workspace, workspace_bytes);
     hipLaunchKernelGGL(fused_attn_fewq_classes_kernel, few_grid(p), dim3(FQ_NW * 64), FewQLds::kBytes, st, p, t);
     if (p.nsplit > 1) launch_combine<FQ_D, false>(p, st);
-  } else if ((splits == 0 || splits == 1) && wide_eligible(p.bh_total, Lq, Lk, D, kv_limit != nullptr) &&
-             run_wide(p, D, splits, workspace, workspace_bytes, st, [&](char *ws) {
+  } else if ((splits == 0 || splits == 1) && wide_eligible(B, p.Hkv, Lq, Lk, D, kv_limit != nullptr) &&
+             run_wide(p, D, splits, workspace, workspace_bytes, st, [&](const AttnParams &part, int first, char *ws) {
                // (one expanding launch per class, into the places of its heads)
                for (int i = 0; i < 3; ++i) {
                  if (!t.c[i].heads) continue;
-                 AttnParams c = p;
+                 AttnParams c = part;
                  c.k_words = t.c[i].k_words; c.v_words = t.c[i].v_words;
                  c.k_scale = t.c[i].k_scale; c.k_zp = t.c[i].k_zp; c.v_scale = t.c[i].v_scale; c.v_zp = t.c[i].v_zp;
                  c.head_map = t.c[i].head_map;
                  c.Hkv = t.c[i].heads;
-                 c.bh_total = B * c.Hkv;
+                 c.bh_total = c.B * c.Hkv;
                  c.kv_bs = (int64_t)c.Hkv * Lk_stride;
+                 skip_entries(c, first, D, 8 >> i, D / group, D / group);
                  launch_expand(c, D, 8 >> i, group, group, false, ws, st, true);
                }
              })) {

@@ -432,12 +432,22 @@ void check_limit_and_map(const at::Tensor *limit, const at::Tensor *map, const A
 }
 int io_code(const at::Tensor &q) { return q.scalar_type() == at::kHalf ? VARQ_F16 : VARQ_BF16; }
 
-// device memory for a launch that shares keys out or expands them (0: neither)
-size_t workspace_bytes(const AttnShape &s, int64_t Lk, int nseg, int64_t splits, bool limits) {
+// Device memory for a launch that shares keys out or expands them (undefined: neither).  Expanding takes more the longer the
+// cache is; where the device has no room for it the call does without.
+at::Tensor workspace(const AttnShape &s, const at::Tensor &q, int64_t Lk, int nseg, int64_t splits, bool limits, bool expands = true) {
   const size_t shared = varq_fused_attn_workspace_bytes((int)s.B, (int)s.Hkv, (int)s.Lq, (int)Lk, (int)s.D, nseg, (int)splits);
-  const auto expand = limits ? varq_fused_attn_expand_bytes_limits : varq_fused_attn_expand_bytes;
-  return splits > 1 ? shared : std::max(shared, expand((int)s.B, (int)s.Hkv, (int)s.Lq, (int)Lk, (int)s.D));
+  const auto bytes = limits ? varq_fused_attn_expand_bytes_limits : varq_fused_attn_expand_bytes;
+  const size_t expanded = expands && splits <= 1 ? bytes((int)s.B, (int)s.Hkv, (int)s.Lq, (int)Lk, (int)s.D) : 0;
+  if (expanded > shared) {
+    try {
+      return empty({(int64_t)expanded}, at::kByte, q);
+    } catch (const c10::OutOfMemoryError &) {
+    }
+  }
+  return shared ? empty({(int64_t)shared}, at::kByte, q) : at::Tensor();
 }
+void *bytes_of(const at::Tensor &ws) { return ws.defined() ? ws.data_ptr() : nullptr; }
+size_t size_of(const at::Tensor &ws) { return ws.defined() ? (size_t)ws.numel() : 0; }
 
 // attn(q, k_words, k_scale, k_zp, v_words, v_scale, v_zp, k_bits, v_bits, Lk, softmax_scale, kv_limit, head_map, out, splits,
 //      layout, exact_codes, out_layout) -> out
@@ -462,13 +472,11 @@ PyObject *attn(PyObject *const *a) {
   const bool exact = truth(a[16]);
   unlocked("varq_fused_attn", [&] {
     s.new_out(q);
-    const size_t ws_bytes = workspace_bytes(s, Lk, 1, splits, limit != nullptr);
-    at::Tensor ws;
-    if (ws_bytes) ws = empty({(int64_t)ws_bytes}, at::kByte, q);
+    const at::Tensor ws = workspace(s, q, Lk, 1, splits, limit != nullptr, !exact || io_code(q) == VARQ_F16);
     return varq_fused_attn(q.data_ptr(), s.out.data_ptr(), ptr<int32_t>(kw), ptr<float>(ks), ptr<float>(kz), (int)k_bits, (int)(s.D / ks.size(3)),
                            ptr<int32_t>(vw), ptr<float>(vs), ptr<float>(vz), (int)v_bits, (int)(s.D / vs.size(3)), (int)s.B, (int)s.Hq, (int)s.Hkv,
                            ptr<int32_t>(map), (int)s.Lq, (int)Lk, (int)s.Lstride, (int)s.D, ptr<int32_t>(limit), softmax_scale, s.layout, io_code(q),
-                           exact, ws_bytes ? ws.data_ptr() : nullptr, ws_bytes, (int)splits, stream_of(q));
+                           exact, bytes_of(ws), size_of(ws), (int)splits, stream_of(q));
   });
   return wrap(s.out);
 }
@@ -507,13 +515,11 @@ PyObject *attn_channel(PyObject *const *a) {
   const float softmax_scale = (float)real(a[9]);
   unlocked("varq_fused_attn_channel", [&] {
     s.new_out(q);
-    const size_t ws_bytes = workspace_bytes(s, Lk, nseg, splits, limit != nullptr);
-    at::Tensor ws;
-    if (ws_bytes) ws = empty({(int64_t)ws_bytes}, at::kByte, q);
+    const at::Tensor ws = workspace(s, q, Lk, nseg, splits, limit != nullptr);
     return varq_fused_attn_channel(q.data_ptr(), s.out.data_ptr(), ptr<int32_t>(kw), ptr<float>(ks), ptr<float>(kz), ptr<int32_t>(vw), ptr<float>(vs),
                                    ptr<float>(vz), nseg, seg ? ends : nullptr, (int)bits, (int)s.B, (int)s.Hq, (int)s.Hkv, ptr<int32_t>(map), (int)s.Lq,
                                    (int)Lk, (int)s.Lstride, (int)s.D, ptr<int32_t>(limit), softmax_scale, s.layout, io_code(q),
-                                   ws_bytes ? ws.data_ptr() : nullptr, ws_bytes, (int)splits, stream_of(q));
+                                   bytes_of(ws), size_of(ws), (int)splits, stream_of(q));
   });
   return wrap(s.out);
 }
@@ -629,11 +635,9 @@ PyObject *cache_attend(PyObject *const *a) {
   const float softmax_scale = (float)real(a[3]);
   unlocked("varq_fused_attn_classes", [&] {
     s.new_out(q);
-    const size_t ws_bytes = workspace_bytes(s, len, 1, splits, limit != nullptr);
-    at::Tensor ws;
-    if (ws_bytes) ws = empty({(int64_t)ws_bytes}, at::kByte, q);
+    const at::Tensor ws = workspace(s, q, len, 1, splits, limit != nullptr);
     return varq_fused_attn_classes(q.data_ptr(), s.out.data_ptr(), t, n, (int)c.group, (int)c.B, (int)c.H, (int)s.Lq, (int)len, (int)c.Lmax, (int)c.D,
-                                   ptr<int32_t>(limit), softmax_scale, s.layout, io_code(q), ws_bytes ? ws.data_ptr() : nullptr, ws_bytes, (int)splits,
+                                   ptr<int32_t>(limit), softmax_scale, s.layout, io_code(q), bytes_of(ws), size_of(ws), (int)splits,
                                    stream_of(q));
   });
   return wrap(s.out);

@@ -17,14 +17,15 @@ cached.  Three backends behind the same interface:
     modules do with flash-attn / xformers / their `slow_attn`;
   * `fused=True`: `PackedKVCache.append` + `PackedKVCache.attend`: the step is
     quantized in place into a pre-allocated packed cache and attention reads the
-    packed codes; no dequantized K/V exists.  Needs a row-local quantizer
+    packed codes; no dequantized K/V is kept (calls of many queries expand it to
+    16 bits while they run).  Needs a row-local quantizer
     (`quant_method='G_GROUP'`).  With `fused_producer=True` the normalisation,
     the per-head scale of q, the rotation and the quantization of k and v run as
     one kernel on the qkv projection output (`PackedKVCache.append_from_qkv`);
   * `fused='quantizer'`: the drop-in quantizers of any rule of the JSON files (the shipped
     G_SCALE_HEAD_DIM rule included) do `quant` + `cache` as in the first backend, and
     `var_q_amd.quant.fused_attention` attends over their packed caches, so the
-    dequantized full-length K/V of `dequant_all` is never built.  Either layout.
+    fp32 full-length K/V of `dequant_all` is never built.  Either layout.
 
 The transformer blocks around the attention (AdaLN, FFN, cross-attention) are
 outside this package.

@@ -566,9 +566,10 @@ MAX_TABLE_STEPS = 16
 def fused_attention(q: torch.Tensor, k_quant: VAR_Q, v_quant: VAR_Q, softmax_scale: float,
                     kv_limit: Optional[torch.Tensor] = None, out: Optional[torch.Tensor] = None) -> torch.Tensor:
     """softmax(scale * q K^T) V over the packed caches of two quantizers, without the
-    dequantized full-length K/V that `dequant_all` would produce (the reference computes
+    fp32 full-length K/V that `dequant_all` would produce (the reference computes
     exactly that and hands it to its attention backend: VAR_Q/quant.py:216-230,
-    Infinity/infinity/models/basic.py:339-351).
+    Infinity/infinity/models/basic.py:339-351).  Calls of many queries hold K and V in 16 bits
+    while they run, at most 1 GiB at a time.
 
     q [B,H,Lq,c] for quantizers in layout 'BHLc', [B,Lq,H,c] for 'BLHc' (the layout of the
     reference's flash-attention call and of VAR-VAR_Q-8.json).  The attention runs in q's dtype
