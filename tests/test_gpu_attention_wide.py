@@ -1,8 +1,8 @@
 """Attention of many queries over a packed cache that is expanded to matrix operands once
 (wide_attn.hip): the shapes below are above the line from which the library takes it, at the
 edges of its tiles (64 keys, 256 queries, 32 queries of a wavefront) and of its rounds over the
-compute units.  Every output is held against the kernel that widens per workgroup (`splits=1`), two (batch, head)
-pairs of each against the oracle."""
+compute units.  Every output is held against the kernel that widens per workgroup (`splits=2`: shares of the keys are its
+alone) and against this path without blocks shared out (`splits=1`), two (batch, head) pairs of each against the oracle."""
 import math
 
 import pytest
@@ -52,13 +52,14 @@ def test_token_scales(dev, D, bits, group, B, H, Lq, Lk, dtype):
     note(what)
     run = lambda **kw: ops.fused_attn(q, *kq, *vq, bits, bits, Lk, 1 / math.sqrt(D), **kw)
     out = run()
-    _check(out, run(splits=1), q, kd, vd, 1 / math.sqrt(D), dt, what)
+    _check(out, run(splits=2), q, kd, vd, 1 / math.sqrt(D), dt, what)
+    _check(run(splits=1), out, q, kd, vd, 1 / math.sqrt(D), dt, what)
     # the same with key limits (none, one, tile edges, all) and with the output tokens-first
     limit = torch.tensor([Lk, 0, 1, 64, 65, 33, Lk - 1, 2047], dtype=torch.int32, device=dev)[torch.arange(Lq, device=dev) // 50 % 8].contiguous()
     note(what, 'limits')
     out = run(kv_limit=limit, out_layout='BLHc').transpose(1, 2)
     assert bool((out[:, :, limit == 0] == 0).all())
-    _check(out, run(kv_limit=limit, splits=1), q, kd, vd, 1 / math.sqrt(D), dt, what + ' limits', limit)
+    _check(out, run(kv_limit=limit, splits=2), q, kd, vd, 1 / math.sqrt(D), dt, what + ' limits', limit)
     # tokens-first cache and queries: the same bits
     t = lambda z: z.transpose(1, 2).contiguous()
     note(what, 'tokens first')
@@ -88,7 +89,8 @@ def test_stepwise_tables_and_head_map(dev, D, bits, asym, dtype):
                                               head_map=perm.int().to(dev), **kw)
     back = torch.empty_like(perm)
     back[perm] = torch.arange(H)
-    _check(run(), run(splits=1), q, deq[0][:, back.to(dev)], deq[1][:, back.to(dev)], 0.05, dt, what)
+    _check(run(splits=1), run(splits=2), q, deq[0][:, back.to(dev)], deq[1][:, back.to(dev)], 0.05, dt, what)
+    _check(run(), run(splits=2), q, deq[0][:, back.to(dev)], deq[1][:, back.to(dev)], 0.05, dt, what)
 
 
 @pytest.mark.parametrize('D,k_group,v_group', [(128, 16, 16), (128, 4, 4), (128, 64, 32), (128, 128, 64), (64, 8, 8), (64, 16, 32)])
@@ -113,4 +115,4 @@ def test_logits_that_climb_move_the_reference(dev):
     kq, vq = (ops.quant_pack_rows(t.bfloat16(), 128, 8, True) for t in (k, v))
     note('wide climbing logits')
     run = lambda **kw: ops.fused_attn(q, *kq, *vq, 8, 8, Lk, 1.0, **kw)
-    _check(run(), run(splits=1), q, ops.dequant(*kq, D, 8), ops.dequant(*vq, D, 8), 1.0, torch.bfloat16, 'wide climbing logits')
+    _check(run(), run(splits=2), q, ops.dequant(*kq, D, 8), ops.dequant(*vq, D, 8), 1.0, torch.bfloat16, 'wide climbing logits')
