@@ -1244,7 +1244,8 @@ __global__ __launch_bounds__(NWV * 64, WPS) void fused_attn_classes_kernel(AttnP
 }
 
 // The shares' outputs weighted by their softmax mass l * 2^(m - M), M the largest reference among
-// the shares that saw a key.  A workgroup of 256 threads serves 2 query rows x (D/4) channel quads
+// the shares that saw a key.  (A share that saw none has the mass 0; one whose logits held a NaN has NaN for its mass, which
+// is not to be taken for 0, or the result would be finite where the unshared kernel's is NaN.)  A workgroup of 256 threads serves 2 query rows x (D/4) channel quads
 // x G groups of shares (G = 4 at D=128, 8 at D=64: the threads of a quad split the shares among
 // them): the weights of a row's shares are formed once, in LDS, and every thread then sums its
 // shares' quads with nothing between the loads but the weights.
@@ -1270,9 +1271,9 @@ __global__ __launch_bounds__(256) void combine_splits_kernel(AttnParams p) {
   if (tid < ROWS * kMaxS) {
     float m_max = -INFINITY;
     for (int t = 0; t < p.nsplit; ++t)
-      if (ml_lds[wr][t].y > 0.f) m_max = fmaxf(m_max, ml_lds[wr][t].x);
+      if (ml_lds[wr][t].y != 0.f) m_max = fmaxf(m_max, ml_lds[wr][t].x);
     const float2 ml = ml_lds[wr][wsh];
-    w_lds[wr][wsh] = ml.y > 0.f ? ml.y * __builtin_amdgcn_exp2f(ml.x - m_max) : 0.f;
+    w_lds[wr][wsh] = ml.y != 0.f ? ml.y * __builtin_amdgcn_exp2f(ml.x - m_max) : 0.f;
   }
   __syncthreads();
   const int r = tid / (QUADS * G), gq = tid % (QUADS * G), grp = gq / QUADS, c0 = (gq % QUADS) * 4;
@@ -1331,11 +1332,11 @@ __global__ __launch_bounds__(256) void combine_few_splits_kernel(AttnParams p) {
   float M = -INFINITY;
 #pragma unroll
   for (int s = 0; s < kMaxSplits_v; ++s)
-    if (ml[s].y > 0.f) M = fmaxf(M, ml[s].x);
+    if (ml[s].y != 0.f) M = fmaxf(M, ml[s].x);
   float acc[4] = {0.f, 0.f, 0.f, 0.f}, wsum = 0.f;
 #pragma unroll
   for (int s = 0; s < kMaxSplits_v; ++s)
-    if (s < p.nsplit && ml[s].y > 0.f) {
+    if (s < p.nsplit && ml[s].y != 0.f) {
       const float w = ml[s].y * __builtin_amdgcn_exp2f(ml[s].x - M);
       acc[0] = __builtin_fmaf(w, o[s].x, acc[0]); acc[1] = __builtin_fmaf(w, o[s].y, acc[1]);
       acc[2] = __builtin_fmaf(w, o[s].z, acc[2]); acc[3] = __builtin_fmaf(w, o[s].w, acc[3]);
@@ -1924,12 +1925,12 @@ __device__ __forceinline__ void attend_few(const AttnParams &p, int bh, int out_
 #pragma unroll
   for (int w = 0; w < FQ_NW; ++w) {
     const float2 ml = *reinterpret_cast<const float2 *>(lds_ml + (w * 32 + col) * 2);
-    if (ml.y > 0.f) { M = any_live ? fmaxf(M, ml.x) : ml.x; any_live = true; }
+    if (ml.y != 0.f) { M = any_live ? fmaxf(M, ml.x) : ml.x; any_live = true; }
   }
   auto weight_of = [&](int w, float &l_w) {
     const float2 ml = *reinterpret_cast<const float2 *>(lds_ml + (w * 32 + col) * 2);
     l_w = ml.y;
-    return ml.y > 0.f ? __builtin_amdgcn_exp2f(ml.x - M) : 0.f;
+    return ml.y != 0.f ? __builtin_amdgcn_exp2f(ml.x - M) : 0.f;
   };
   float l_sum = 0.f;   // (summed in the same order by every wavefront)
 #pragma unroll

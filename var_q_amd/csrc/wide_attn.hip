@@ -491,7 +491,7 @@ __global__ __launch_bounds__(512, 2) void wide_attn_kernel(WideParams e) {
 }
 
 // The query blocks that fell on several workgroups: the partial outputs weighted by their softmax
-// mass l * 2^(m - M).  A workgroup serves 1024 / D rows of one block, a thread four channels of a row.
+// mass l * 2^(m - M) (0: it saw no key; a NaN counts, and makes the result one).  A workgroup serves 1024 / D rows of one block, a thread four channels of a row.
 template <int D, bool F16>
 __global__ __launch_bounds__(256) void wide_combine_kernel(WideParams e, int n_wgs) {
   const AttnParams &p = e.a;
@@ -507,14 +507,14 @@ __global__ __launch_bounds__(256) void wide_combine_kernel(WideParams e, int n_w
   float M = -INFINITY;
   for (int w = w0; w <= w1; ++w) {
     const float2 ml = *reinterpret_cast<const float2 *>(e.ws_ml + slot_row(w) * 2);
-    if (ml.y > 0.f) M = fmaxf(M, ml.x);
+    if (ml.y != 0.f) M = fmaxf(M, ml.x);
   }
   float acc[4] = {0.f, 0.f, 0.f, 0.f}, sum = 0.f;
   for (int w = w0; w <= w1; ++w) {
     const int64_t r = slot_row(w);
     const float2 ml = *reinterpret_cast<const float2 *>(e.ws_ml + r * 2);
     const float4 o = *reinterpret_cast<const float4 *>(e.ws_o + r * D + c0);
-    if (ml.y > 0.f) {
+    if (ml.y != 0.f) {
       const float wt = ml.y * __builtin_amdgcn_exp2f(ml.x - M);
       acc[0] = __builtin_fmaf(wt, o.x, acc[0]); acc[1] = __builtin_fmaf(wt, o.y, acc[1]);
       acc[2] = __builtin_fmaf(wt, o.z, acc[2]); acc[3] = __builtin_fmaf(wt, o.w, acc[3]);
