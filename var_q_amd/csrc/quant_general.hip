@@ -763,8 +763,11 @@ bool make_one_plan(const int64_t *sh, int reduce_mask, int row_steps, int tensor
   if (c % 8 != 0 || c > 512 || rows <= 0 || rows >= (1ll << 31) - 512) return false;
   const Canonical k = canonical(sh, reduce_mask);
   const int64_t rr = k.nro * k.RI;
-  // above 16 MiB the three launches, with 2048 workgroups on either side of the fold, are the faster way
-  // through memory ([32,30,680,64], one scale per (token, head): 38 against 55 us)
+  // Up to 16 MiB (of both tensors) one launch was the faster way in everything measured; beyond, the three launches, with
+  // 2048 workgroups on either side of the fold, catch up sooner or later: three / one, us, one scale per (head, channel), K and V
+  // [2,16,n,128] 25 MiB 22.9 / 16.9, 36 25.6 / 21.7, 64 37.8 / 42.0, [64,n,16,64] 25 23.5 / 21.8, 30 26.2 / 25.0,
+  // [32,n,30,64] 40 29.7 / 24.3, 60 35.2 / 33.8, one tensor of it 20 20.5 / 23.0, 30 22.8 / 31.8; one scale per (token, head),
+  // [32,30,L,64] 20 16.8 / 12.6, 40 25.6 / 21.7, 80 43.8 / 48.7.
   if (rr > 8192 || rows * c * (row_steps == 8 ? 4 : 2) * tensors > (16ll << 20)) return false;
   const bool keepc = !(reduce_mask & 8);
   const int c8 = (int)(c / 8);
@@ -776,13 +779,16 @@ bool make_one_plan(const int64_t *sh, int reduce_mask, int row_steps, int tensor
   while ((1 << rr_shift) < rr) ++rr_shift;
   // column slices (channel dim kept): whole rows while that makes workgroups enough, 64 bytes of a row at least
   pl.c8s_shift = keepc && c8p_shift > 4 ? 4 : c8p_shift;
-  // Narrower slices mean more workgroups and smaller pieces of each row.  32 bytes where that leaves no more than
-  // half of the compute units without one; 16 (a word of 2-bit codes takes 32) where it does not and codes are all
-  // that is stored: K and V [64,n,16,64] fp16, 8 bits, 128 -> 256 workgroups, n = 64 24.9 -> 19.6 us, n = 16 9.9 ->
-  // 8.5; [4,400,24,128] one tensor, 192 -> 384 workgroups 13.5 -> 19.4.  The dequantized values of a step in 32-byte
-  // pieces from as many workgroups take a schedule of [8,n,30,64] from 208 to 227 us.
+  // Narrower slices mean more workgroups and smaller pieces of each row, down to 32 bytes where dequantized values are
+  // stored as well or a word of 2-bit codes takes two octets, to 16 otherwise.
+  // A workgroup of 1024 threads holds its rows in the registers of a whole compute unit, so slices are halved only
+  // while that leaves one for each of the 256, from 128 workgroups at most: K and V [64,n,16,64] fp16, 8 bits, 128 -> 256,
+  // n = 64 24.9 -> 19.6 us, n = 16 9.9 -> 8.5; one tensor [8,256,36,64] 144 -> 288 11.2 -> 18.1, [2,1024,18,128] the
+  // same 11.4 -> 18.0, [8,256,40,64] 160 -> 320 12.1 -> 18.6, [4,400,24,128] 192 -> 384 13.5 -> 19.4.
+  // Several workgroups of 256 threads are resident on one, and more of them are no loss: [8,64,36,64] 144 -> 288 6.8 ->
+  // 6.0, [8,64,48,64] 192 -> 384 6.8 -> 6.2; [2,400,18,128] 7.9 either way.  The dequantized values of a step in 32-byte pieces from
+  // twice as many workgroups take a schedule of [8,n,30,64] from 208 to 227 us.
   const int narrowest = bits == 2 || with_values ? 1 : 0;
-  const int enough = with_values ? 128 : 160;
   for (;; --pl.c8s_shift) {
     pl.slices = keepc ? (c8 + (1 << pl.c8s_shift) - 1) >> pl.c8s_shift : 1;
     // 256 threads where their rows suffice, 1024 otherwise; the row lanes of a q no more than its rows
@@ -798,6 +804,7 @@ bool make_one_plan(const int64_t *sh, int reduce_mask, int row_steps, int tensor
     pl.tilesQ = (int)((k.Q + (1 << pl.lq_shift) - 1) >> pl.lq_shift);
     pl.blocks = pl.nko * pl.tilesQ;
     const bool fits = pl.steps <= row_steps;
+    const int enough = with_values ? 128 : threads == 1024 ? 129 : 160;
     if (fits && ((int64_t)pl.blocks * pl.slices * tensors >= enough || !keepc || pl.c8s_shift <= narrowest)) return true;
     if (!keepc || pl.c8s_shift <= narrowest) return false;
   }
