@@ -546,36 +546,59 @@ struct Ref {   // owns the reference it is given
 };
 #define NAME(id) ([]() { static PyObject *const name = PyUnicode_InternFromString(#id); return name; }())
 
+// A tensor of a cache: held through its Python object, which is free under the interpreter's lock, as every place of use is
+// made and dropped.
+struct Held {
+  PyObject *o = nullptr;
+  const at::Tensor *t = nullptr;
+  Held() = default;
+  Held(const Held &) = delete;
+  ~Held() { Py_XDECREF(o); }
+  const at::Tensor *operator->() const { return t; }
+};
+template <typename T> T *ptr(const Held &h) { return h.t ? reinterpret_cast<T *>(h.t->data_ptr()) : nullptr; }
+
 struct CacheClass {
   int64_t bits, heads;
-  at::Tensor k_words, k_scale, k_zp, v_words, v_scale, v_zp, slot, head_map;
+  Held k_words, k_scale, k_zp, v_words, v_scale, v_zp, slot, head_map;
 
-  static at::Tensor dense(PyObject *of, PyObject *name, at::ScalarType dt) {
-    const Ref a(attribute(of, name));
-    const at::Tensor &t = gpu(a.o, PyUnicode_AsUTF8(name));
-    ASSERT(t.scalar_type() == dt && t.is_contiguous(), "cache buffer %U must be contiguous and of type %s", name, toString(dt));
-    return t;
+  // field i of a class, whose Python object is a list of its fields (another object: by name)
+  static PyObject *field(PyObject *of, int i, PyObject *name) {
+    if (!PyList_Check(of) || PyList_GET_SIZE(of) != 10) return attribute(of, name);
+    PyObject *const v = PyList_GET_ITEM(of, i);
+    Py_INCREF(v);
+    return v;
+  }
+  static void dense(Held &h, PyObject *of, int i, PyObject *name, at::ScalarType dt) {
+    h.o = field(of, i, name);
+    h.t = &gpu(h.o, "cache buffer");
+    ASSERT(h.t->scalar_type() == dt && h.t->is_contiguous(), "cache buffer %U must be contiguous and of type %s", name, toString(dt));
   }
   void read(PyObject *o, int64_t H, bool asym) {
-    bits = integer(Ref(attribute(o, NAME(bits))).o);
-    const Py_ssize_t n = PyObject_Size(Ref(attribute(o, NAME(heads))).o);
+    bits = integer(Ref(field(o, 0, NAME(bits))).o);
+    const Py_ssize_t n = PyObject_Size(Ref(field(o, 1, NAME(heads))).o);
     if (n < 0) throw python_error();
     heads = n;
-    k_words = dense(o, NAME(k_words), at::kInt); v_words = dense(o, NAME(v_words), at::kInt);
-    k_scale = dense(o, NAME(k_scale), at::kFloat); v_scale = dense(o, NAME(v_scale), at::kFloat);
-    if (asym) { k_zp = dense(o, NAME(k_zp), at::kFloat); v_zp = dense(o, NAME(v_zp), at::kFloat); }
-    slot = dense(o, NAME(slot), at::kInt); head_map = dense(o, NAME(head_map), at::kInt);
-    ASSERT(heads > 0 && slot.numel() == H && head_map.numel() == heads, "cache class of %lld bits: slot and head_map do not fit its heads", (long long)bits);
+    dense(k_words, o, 2, NAME(k_words), at::kInt);
+    dense(k_scale, o, 3, NAME(k_scale), at::kFloat);
+    if (asym) dense(k_zp, o, 4, NAME(k_zp), at::kFloat);
+    dense(v_words, o, 5, NAME(v_words), at::kInt);
+    dense(v_scale, o, 6, NAME(v_scale), at::kFloat);
+    if (asym) dense(v_zp, o, 7, NAME(v_zp), at::kFloat);
+    dense(slot, o, 8, NAME(slot), at::kInt);
+    dense(head_map, o, 9, NAME(head_map), at::kInt);
+    ASSERT(heads > 0 && slot->numel() == H && head_map->numel() == heads, "cache class of %lld bits: slot and head_map do not fit its heads", (long long)bits);
   }
   // the kernels trust the sizes: rows as long as the call implies, and the last one it reaches inside
   void check(int64_t D, int64_t group, int64_t last) const {
     const int64_t W = D * bits / 32, ng = D / group;
     for (const auto &[w, sc, z] : {std::tuple(&k_words, &k_scale, &k_zp), std::tuple(&v_words, &v_scale, &v_zp)}) {
-      if (!w->dim() || !sc->dim() || w->size(-1) != W || sc->size(-1) != ng || (z->defined() && z->sizes() != sc->sizes()))
+      const auto &ws = (*w)->sizes(), &ss = (*sc)->sizes();
+      if (ws.empty() || ss.empty() || ws.back() != W || ss.back() != ng || (z->t && (*z)->sizes() != ss))
         raise(g_varq_error, "cache class of %lld bits: rows of words, scales and zero-points must have %lld, %lld and %lld entries", (long long)bits, (long long)W, (long long)ng, (long long)ng);
-      if (last >= w->numel() / W || last >= sc->numel() / ng)
-        raise(g_varq_error, "cache class of %lld bits: the call reaches row %lld of buffers that hold %lld rows", (long long)bits, (long long)last,
-              (long long)std::min(w->numel() / W, sc->numel() / ng));
+      const int64_t rows = std::min((*w)->numel() / W, (*sc)->numel() / ng);
+      if (last >= rows)
+        raise(g_varq_error, "cache class of %lld bits: the call reaches row %lld of buffers that hold %lld rows", (long long)bits, (long long)last, (long long)rows);
     }
   }
 };

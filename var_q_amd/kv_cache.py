@@ -8,6 +8,7 @@ bit-widths; heads of equal width share one dense buffer ("class") and a table
 maps each head to (class, slot).  Layout BHLc: K/V steps are [B, H, n, D].
 """
 import json
+from operator import itemgetter
 from typing import Any, Dict, List, Optional, Sequence, Union
 
 import torch
@@ -15,18 +16,24 @@ import torch
 from . import _lib, ops
 
 
-class _BitClass:
+def _field(i: int) -> property:
+    return property(itemgetter(i), lambda self, value: self.__setitem__(i, value))
+
+
+class _BitClass(list):
+    """The heads of one bit-width and their buffers.  A list of its fields, which the native host layer reads at every call
+    in a third of the time that ten attributes by name take it."""
+    bits, heads, k_words, k_scale, k_zp, v_words, v_scale, v_zp, slot, head_map = (_field(i) for i in range(10))
+
     def __init__(self, bits, heads, B, H, Lmax, D, group, device):
-        self.bits, self.heads = bits, list(heads)
-        hc, w, ns = len(self.heads), D * bits // 32, D // group
+        heads = list(heads)
+        hc, w, ns = len(heads), D * bits // 32, D // group
         slot = torch.full((H,), -1, dtype=torch.int32)
-        slot[self.heads] = torch.arange(hc, dtype=torch.int32)
-        self.slot = slot.to(device)
-        self.head_map = torch.tensor(self.heads, dtype=torch.int32, device=device)
+        slot[heads] = torch.arange(hc, dtype=torch.int32)
         mk = lambda last, dt: torch.zeros((B, hc, Lmax, last), dtype=dt, device=device)
-        self.k_words, self.v_words = mk(w, torch.int32), mk(w, torch.int32)
-        self.k_scale, self.v_scale = mk(ns, torch.float32), mk(ns, torch.float32)
-        self.k_zp, self.v_zp = mk(ns, torch.float32), mk(ns, torch.float32)
+        words, scale = lambda: mk(w, torch.int32), lambda: mk(ns, torch.float32)
+        super().__init__((bits, heads, words(), scale(), scale(), words(), scale(), scale(),
+                          slot.to(device), torch.tensor(heads, dtype=torch.int32, device=device)))
 
 
 class PackedKVCache:
