@@ -409,15 +409,15 @@ void make_out(AttnShape &s, const at::Tensor &q, PyObject *out, int lay, int ola
 }
 
 // (the checks that both attention calls share; a: q, k_words, out, layout, out_layout)
-AttnShape attn_shape(const at::Tensor &q, const at::Tensor &kw, PyObject *out, PyObject *layout, PyObject *out_layout) {
+AttnShape attn_shape(const at::Tensor &q, const at::Tensor &kw, PyObject *out, int lay, int out_lay) {
   AttnShape s;
   ASSERT((q.scalar_type() == at::kBFloat16 || q.scalar_type() == at::kHalf) && q.dim() == 4, "q must be bf16 or fp16");
   ASSERT(kw.dim() == 4, "k_words must be 4-D");
-  const int lay = layout_code(layout), h = lay == VARQ_LAYOUT_BHLC ? 1 : 2, t = 3 - h;
+  const int h = lay == VARQ_LAYOUT_BHLC ? 1 : 2, t = 3 - h;
   s.B = q.size(0); s.Hq = q.size(h); s.Lq = q.size(t); s.D = q.size(3);
   s.Hkv = kw.size(h); s.Lstride = kw.size(t);
   ASSERT(kw.size(0) == s.B, "batch sizes of q and the cache differ");
-  make_out(s, q, out, lay, out_layout == Py_None ? lay : layout_code(out_layout));
+  make_out(s, q, out, lay, out_lay);
   return s;
 }
 const at::Tensor &dense(PyObject *o, const char *name) {
@@ -449,36 +449,48 @@ at::Tensor workspace(const AttnShape &s, const at::Tensor &q, int64_t Lk, int ns
 void *bytes_of(const at::Tensor &ws) { return ws.defined() ? ws.data_ptr() : nullptr; }
 size_t size_of(const at::Tensor &ws) { return ws.defined() ? (size_t)ws.numel() : 0; }
 
-// attn(q, k_words, k_scale, k_zp, v_words, v_scale, v_zp, k_bits, v_bits, Lk, softmax_scale, kv_limit, head_map, out, splits,
-//      layout, exact_codes, out_layout) -> out
-PyObject *attn(PyObject *const *a) {
-  const at::Tensor &q = dense(a[0], "q"), &kw = dense(a[1], "k_words"), &ks = dense(a[2], "k_scale"), &vw = dense(a[4], "v_words"), &vs = dense(a[5], "v_scale");
-  const at::Tensor *kz = maybe(a[3], "k_zp"), *vz = maybe(a[6], "v_zp"), *limit = maybe(a[11], "kv_limit"), *map = maybe(a[12], "head_map");
-  const int64_t k_bits = integer(a[7]), v_bits = integer(a[8]), Lk = integer(a[9]), splits = integer(a[14]);
+// Attention over the packed rows of one bit-width with scales per key.
+struct KeyScales {
+  const at::Tensor &kw, &ks, &vw, &vs;
+  const at::Tensor *kz, *vz;
+  int64_t k_bits, v_bits;
+};
+PyObject *attend_rows(const at::Tensor &q, const KeyScales &r, int64_t Lk, float softmax_scale, const at::Tensor *limit, const at::Tensor *map, PyObject *out,
+                      int64_t splits, int lay, int out_lay, bool exact) {
+  const at::Tensor &kw = r.kw, &ks = r.ks, &vw = r.vw, &vs = r.vs;
   const c10::DeviceGuard guard(q.device());
-  AttnShape s = attn_shape(q, kw, a[13], a[15], a[17]);
+  AttnShape s = attn_shape(q, kw, out, lay, out_lay);
   ASSERT(vw.dim() == 4 && ks.dim() == 4 && vs.dim() == 4, "4-D cache tensors");
   for (int d = 0; d < 3; ++d)
     ASSERT(vw.size(d) == kw.size(d) && ks.size(d) == kw.size(d) && vs.size(d) == kw.size(d), "words and scales must agree in batch, heads and tokens");
-  ASSERT(kw.size(3) * 32 == s.D * k_bits && vw.size(3) * 32 == s.D * v_bits, "words per row do not match the head dim and the bit-width");
+  ASSERT(kw.size(3) * 32 == s.D * r.k_bits && vw.size(3) * 32 == s.D * r.v_bits, "words per row do not match the head dim and the bit-width");
   ASSERT(ks.size(3) > 0 && vs.size(3) > 0, "empty scales");
-  for (const auto &[z, sc, n] : {std::tuple(kz, &ks, "k_zp"), std::tuple(vz, &vs, "v_zp")})
+  for (const auto &[z, sc, n] : {std::tuple(r.kz, &ks, "k_zp"), std::tuple(r.vz, &vs, "v_zp")})
     ASSERT(!z || (z->sizes() == sc->sizes() && z->scalar_type() == at::kFloat && z->is_contiguous()), "%s must look like its scale", n);
   ASSERT(ks.scalar_type() == at::kFloat && vs.scalar_type() == at::kFloat && kw.scalar_type() == at::kInt && vw.scalar_type() == at::kInt,
          "scales must be fp32 and words int32");
   ASSERT(0 <= Lk && Lk <= s.Lstride, "Lk=%lld outside the cache of %lld tokens", (long long)Lk, (long long)s.Lstride);
   check_limit_and_map(limit, map, s);
-  const float softmax_scale = (float)real(a[10]);
-  const bool exact = truth(a[16]);
   unlocked("varq_fused_attn", [&] {
     s.new_out(q);
     const at::Tensor ws = workspace(s, q, Lk, 1, splits, limit != nullptr, !exact || io_code(q) == VARQ_F16);
-    return varq_fused_attn(q.data_ptr(), s.out.data_ptr(), ptr<int32_t>(kw), ptr<float>(ks), ptr<float>(kz), (int)k_bits, (int)(s.D / ks.size(3)),
-                           ptr<int32_t>(vw), ptr<float>(vs), ptr<float>(vz), (int)v_bits, (int)(s.D / vs.size(3)), (int)s.B, (int)s.Hq, (int)s.Hkv,
+    return varq_fused_attn(q.data_ptr(), s.out.data_ptr(), ptr<int32_t>(kw), ptr<float>(ks), ptr<float>(r.kz), (int)r.k_bits, (int)(s.D / ks.size(3)),
+                           ptr<int32_t>(vw), ptr<float>(vs), ptr<float>(r.vz), (int)r.v_bits, (int)(s.D / vs.size(3)), (int)s.B, (int)s.Hq, (int)s.Hkv,
                            ptr<int32_t>(map), (int)s.Lq, (int)Lk, (int)s.Lstride, (int)s.D, ptr<int32_t>(limit), softmax_scale, s.layout, io_code(q),
                            exact, bytes_of(ws), size_of(ws), (int)splits, stream_of(q));
   });
   return wrap(s.out);
+}
+
+// attn(q, k_words, k_scale, k_zp, v_words, v_scale, v_zp, k_bits, v_bits, Lk, softmax_scale, kv_limit, head_map, out, splits,
+//      layout, exact_codes, out_layout) -> out
+PyObject *attn(PyObject *const *a) {
+  const at::Tensor &q = dense(a[0], "q");
+  const KeyScales r = {dense(a[1], "k_words"), dense(a[2], "k_scale"), dense(a[4], "v_words"), dense(a[5], "v_scale"), maybe(a[3], "k_zp"), maybe(a[6], "v_zp"),
+                       integer(a[7]), integer(a[8])};
+  const at::Tensor *limit = maybe(a[11], "kv_limit"), *map = maybe(a[12], "head_map");
+  const int lay = layout_code(a[15]);
+  return attend_rows(q, r, integer(a[9]), (float)real(a[10]), limit, map, a[13], integer(a[14]), lay, a[17] == Py_None ? lay : layout_code(a[17]), truth(a[16]));
 }
 
 // attn_channel(q, k_words, k_scale, k_zp, v_words, v_scale, v_zp, bits, Lk, softmax_scale, kv_limit, head_map, out, seg_ends, splits,
@@ -488,7 +500,8 @@ PyObject *attn_channel(PyObject *const *a) {
   const at::Tensor *kz = maybe(a[3], "k_chan_zp"), *vz = maybe(a[6], "v_chan_zp"), *limit = maybe(a[10], "kv_limit"), *map = maybe(a[11], "head_map");
   const int64_t bits = integer(a[7]), Lk = integer(a[8]), splits = integer(a[14]);
   const c10::DeviceGuard guard(q.device());
-  AttnShape s = attn_shape(q, kw, a[12], a[15], a[16]);
+  const int lay = layout_code(a[15]);
+  AttnShape s = attn_shape(q, kw, a[12], lay, a[16] == Py_None ? lay : layout_code(a[16]));
   ASSERT(vw.sizes() == kw.sizes() && kw.size(3) * 32 == s.D * bits, "K and V words must agree and match the head dim and the bit-width");
   int32_t ends[16];
   int nseg = 1;
@@ -638,12 +651,20 @@ int class_table(const Cache &c, varq_kv_class (&t)[3]) {
   return c.n;
 }
 
-// cache_attend(cache, len, q, softmax_scale, kv_limit, out, splits, out_layout) -> out: all classes of a mixed-width cache
+// cache_attend(cache, len, q, softmax_scale, kv_limit, out, splits, out_layout, exact_codes) -> out: all classes in one call
+// (exact codes: of a cache of one class only)
 PyObject *cache_attend(PyObject *const *a) {
   const Cache c(a[0]);
   const int64_t len = integer(a[1]), splits = integer(a[6]);
   const at::Tensor &q = dense(a[2], "q");
   const at::Tensor *limit = maybe(a[4], "kv_limit");
+  const bool exact = truth(a[8]);
+  if (c.n == 1) {
+    const CacheClass &k = c.classes[0];
+    const KeyScales r = {*k.k_words.t, *k.k_scale.t, *k.v_words.t, *k.v_scale.t, k.k_zp.t, k.v_zp.t, k.bits, k.bits};
+    return attend_rows(q, r, len, (float)real(a[3]), limit, nullptr, a[5], splits, VARQ_LAYOUT_BHLC, layout_code(a[7]), exact);
+  }
+  ASSERT(!exact, "exact codes: one class at a time");
   ASSERT((q.scalar_type() == at::kBFloat16 || q.scalar_type() == at::kHalf) && q.dim() == 4, "q must be bf16 or fp16");
   ASSERT(q.size(0) == c.B && q.size(1) == c.H && q.size(3) == c.D, "attend: q does not fit the cache");
   ASSERT(0 < len && len <= c.Lmax, "attend: the cache holds no such token");
@@ -792,7 +813,7 @@ PyObject *set_error(PyObject *, PyObject *e) {
 #define FIXED(name, n) {#name, (PyCFunction)(void (*)(void))fixed<name, n>, METH_FASTCALL, nullptr}
 PyMethodDef g_methods[] = {
     FIXED(quant_rows, 5), FIXED(quant_shared, 6), FIXED(pack, 2), FIXED(unpack, 3), FIXED(dequant, 6), FIXED(dequant_steps, 8), FIXED(quant_step_dequant, 10), FIXED(attn, 18), FIXED(attn_channel, 17),
-    FIXED(cache_attend, 8), FIXED(cache_append, 5), FIXED(cache_prepare, 9),
+    FIXED(cache_attend, 9), FIXED(cache_append, 5), FIXED(cache_prepare, 9),
     {"quant_step", (PyCFunction)(void (*)(void))varying<quant_step>, METH_FASTCALL, nullptr},
     {"set_error", set_error, METH_O, nullptr},
     {nullptr, nullptr, 0, nullptr}};

@@ -93,11 +93,13 @@ class PackedKVCache:
         """The cache buffers under the names the descriptor uses (no copies)."""
         out = {}
         for c in self.classes:
-            for kv in 'kv':
-                out[f'b{c.bits}.{kv}_words'] = getattr(c, f'{kv}_words')
-                out[f'b{c.bits}.{kv}_scale'] = getattr(c, f'{kv}_scale')
-                if not self.symmetric:
-                    out[f'b{c.bits}.{kv}_zp'] = getattr(c, f'{kv}_zp')
+            b = f'b{c.bits}.'
+            out[b + 'k_words'], out[b + 'k_scale'] = c.k_words, c.k_scale
+            if not self.symmetric:
+                out[b + 'k_zp'] = c.k_zp
+            out[b + 'v_words'], out[b + 'v_scale'] = c.v_words, c.v_scale
+            if not self.symmetric:
+                out[b + 'v_zp'] = c.v_zp
         return out
 
     def save(self, path: str):
@@ -154,13 +156,8 @@ class PackedKVCache:
         [B,Lq,C] for its output projection (no transposing copy)."""
         assert self.len > 0, 'attend on an empty cache: append keys and values first'
         assert out_layout in ('BHLc', 'BLHc')
-        if len(self.classes) == 1:
-            c, asym = self.classes[0], not self.symmetric
-            return _lib.host().attn(q, c.k_words, c.k_scale, c.k_zp if asym else None, c.v_words, c.v_scale, c.v_zp if asym else None,
-                                    c.bits, c.bits, self.len, softmax_scale, kv_limit, None, out, self.splits, 'BHLc', exact_codes,
-                                    out_layout)
-        if self.concurrent_classes and not exact_codes:
-            return _lib.host().cache_attend(self, self.len, q, softmax_scale, kv_limit, out, self.splits, out_layout)
+        if len(self.classes) == 1 or (self.concurrent_classes and not exact_codes):
+            return _lib.host().cache_attend(self, self.len, q, softmax_scale, kv_limit, out, self.splits, out_layout, exact_codes)
         if out is None:
             B_, H_, Lq_, D_ = q.shape
             out = torch.empty((B_, Lq_, H_, D_) if out_layout == 'BLHc' else q.shape, dtype=q.dtype, device=q.device)
