@@ -224,11 +224,7 @@ class VAR_Q:
             return kept.view()
         like = self._scale_shape
         if self.quant_method in _TOKEN_METHODS:
-            t = tok.view()
-            for i in range(3):
-                if i != d:
-                    t = t.narrow(i, 0, like[i])
-            return t
+            return tok.buf.as_strided(like[:d] + (n,) + like[d + 1:], tok.buf.stride())
         h = 3 - d                                            # the dim of the heads
         full = [1, tab.shape[1], tab.shape[2]]
         full.insert(d, 1)
