@@ -285,9 +285,9 @@ int varq_quant_step_dequant(const void *x, int x_dtype, int B, int H, int n, int
  *              up to 8 workgroups; their partial results (fp32) pass through the
  *              workspace and a second kernel combines them.  splits = 0: the library
  *              decides, and uses no more shares than the workspace holds (none
- *              without a workspace) -- with at most 64 queries over at least 1024 keys
- *              (D = 128, one scale group per key, bf16) it takes a kernel of its own for
- *              that regime, whose wavefronts all serve the same 32 queries on different
+ *              without a workspace) -- with at most 16 queries, and up to 128 where the cache is
+ *              long enough for them, it takes a kernel of its own (at most two scale groups per key;
+ *              the default operand form), whose wavefronts all serve the same queries on different
  *              keys, with up to 64 shares; 1: never; 2..8: exactly that many (an error if
  *              the workspace is too small).  varq_fused_attn_workspace_bytes gives the
  *              size for a shape (0 when the library would not share the keys out);

@@ -33,6 +33,7 @@ FLAGS = {
     'qkv_prepare.hip': ['-ffp-contract=off'],
     'fused_attn.hip': [],
     'wide_attn.hip': [],
+    'few_attn.hip': [],
 }
 
 

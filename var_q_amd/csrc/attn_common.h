@@ -44,11 +44,21 @@ struct AttnParams {
   int exact_codes;
   int f16;   // q, out and the MFMA operands are fp16 (host side only: it selects the instantiation)
   int fq_share_blocks;   // few-queries kernel: 32-key blocks per share of the keys
+  int few_waves;         // ... and wavefronts of a workgroup, 4 or 8 (host side only)
   // memory layout, in rows (a row = the D values of one token of one head):
   // q row = b*q_bs + h*q_hs + i*q_ts, out row likewise with o_*, key row = b*kv_bs + slot*kv_hs + j*kv_ts.
   // BHLc: (H*L, L, 1); BLHc (the layout of the flash-attention call): (L*H, 1, H).
   int64_t q_bs, q_hs, q_ts, o_bs, o_hs, o_ts, kv_bs, kv_hs, kv_ts;
 };
+
+// above 64 KiB of LDS the limit has to be raised, once per device the process launches on
+inline void allow_lds(const void *kernel, int bytes, bool (&configured)[64]) {
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) dev = -1;
+  if (dev >= 0 && configured[dev]) return;
+  (void)hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
+  if (dev >= 0) configured[dev] = true;
+}
 
 __device__ __forceinline__ u32 pack_bf16_rne(float lo, float hi) {
   typedef __bf16 bf2 __attribute__((ext_vector_type(2)));
@@ -95,6 +105,47 @@ struct HeavyFirst {
     grp = first + r % n;
   }
 };
+
+// A cache whose heads have several bit-widths, all classes in one launch: pair k of the launch belongs to the
+// class that its range falls in (8-bit codes first: the longest workgroups start first), and the workgroup
+// runs that class's code.  The registers and the LDS are those of the most demanding class, which is no
+// more than each class takes alone (see launch_shape); what is gained are the launches -- and that the
+// classes, which have a few heads each, fill the device together.  Three widths, one launch per class ->
+// one launch, us: [2,16,128] 100 queries x 600 keys 66 -> 18, [8,16,128] 256 x 500 78 -> 28, 576 x 1497 140 ->
+// 117, 1024 x 2521 230 -> 200 (the last two with a stream for each class).
+struct ClassParams {
+  const u32 *k_words, *v_words;
+  const float *k_scale, *k_zp, *v_scale, *v_zp;
+  const int32_t *head_map;
+  int heads, first;   // packed heads of the class; its first pair of the launch
+};
+struct ClassTable { ClassParams c[3]; };   // of 8, 4 and 2 bits; a width that the cache does not have has no heads
+__device__ __forceinline__ void enter_class(AttnParams &p, const ClassParams &c) {
+  p.k_words = c.k_words; p.v_words = c.v_words;
+  p.k_scale = c.k_scale; p.k_zp = c.k_zp; p.v_scale = c.v_scale; p.v_zp = c.v_zp;
+  p.head_map = c.head_map;
+  p.Hkv = c.heads;
+  p.kv_bs = (int64_t)c.heads * p.Lstride;
+}
+// F(bits, pair within the class, pair of the output) for the class of pair k
+template <class F> __device__ __forceinline__ void in_class(AttnParams &p, const ClassTable &t, int k, F &&f) {
+  const int H = p.Hq;
+  auto run = [&](auto bits, const ClassParams &c) __attribute__((always_inline)) {
+    enter_class(p, c);
+    const int bh = k - c.first;
+    f(bits, bh, bh / c.heads * H + c.head_map[bh % c.heads]);
+  };
+  if (k < t.c[1].first) run(std::integral_constant<int, 8>{}, t.c[0]);
+  else if (k < t.c[2].first) run(std::integral_constant<int, 4>{}, t.c[1]);
+  else run(std::integral_constant<int, 2>{}, t.c[2]);
+}
+
+// ---- few queries (few_attn.hip) ----
+constexpr int kFewBlock = 32;   // keys per block
+constexpr int kFewGroups = 2;   // scale groups of a row, at most
+// p.q_tiles: tiles of 32 queries (up to 16 queries are one of 16); p.nsplit, p.fq_share_blocks, p.ws_*: the shares of the keys
+void launch_few(const AttnParams &p, int D, int bits, int k_group, int v_group, hipStream_t st);
+void launch_few_classes(const AttnParams &p, int D, const ClassTable &t, int group, hipStream_t st);
 
 // ---- the wide path (wide_attn.hip): K and V expanded once, then attended by many query blocks ----
 struct WidePlan {

@@ -234,28 +234,6 @@ template <int BITS> __device__ __forceinline__ void k_values(const u32 *q4, int 
   }
 }
 
-// ---- dequantizing 4-bit codes through bytes (the kernel for few queries) ---------------------
-// That kernel is bound by its vector instructions, most of them widening: field -> float, minus
-// zero-point, times scale, round to bf16, 4.5 instructions per element.  For 4-bit codes there is a
-// shorter way to the same bits.  A staged word holds u = code + 8 per nibble; two masks put the
-// eight nibbles into the bytes of two dwords, one add per dword (no carries between bytes) makes
-// every byte t = u + A with A = 120 - zp, i.e. t - 128 = code - zp, v_cvt_f32_ubyte turns a byte
-// into a float in one instruction, and fma(t, s, -128 s) is RN((t - 128) s) = RN((code - zp) * scale),
-// the very product the reference rounds (VAR_Q/quant.py:123-124 with a zero-point): -128 s is exact
-// and an fma rounds once.  3 instructions per element.  It needs an integer zero-point with A in
-// [0, 240] (|zp| <= 120: every zero-point the quantizer derives from data that straddles or lies
-// near zero); a block with any other zero-point takes the general form, which computes the same
-// values.  (In the kernels for many queries, which are not bound by the count of their vector
-// instructions, the same change was measured: bit-identical results, no gain -- 752 against 745 us
-// on the configuration-4 shape, 74.7 against 71.4 us on configuration 2 -- so they keep one form.)
-__device__ __forceinline__ bool byte_bias4(float zp, u32 &a4) {
-  const float a = 120.f - zp;
-  const bool ok = a >= 0.f && a <= 240.f && a == __builtin_rintf(a);
-  a4 = ok ? (u32)(int)a * 0x01010101u : 0u;
-  return ok;
-}
-__device__ __forceinline__ float ubyte_f32(u32 x, int k) { return (float)((x >> (8 * k)) & 0xffu); }   // v_cvt_f32_ubyte<k>
-
 // octet (8-channel unit) of K that lane-half h contracts in 16-channel chunk ch;
 // chunks never straddle a scale group of `G` channels.
 template <int G> __device__ __forceinline__ int k_octet(int ch, int h) {
@@ -1200,40 +1178,6 @@ __global__ __launch_bounds__(NWV * 64, WPS) void fused_attn_kernel(AttnParams p)
   attend_block<D, BITS, GK, GV, CHAN, NWV, EXACT, F16, ONE>(p, k.pair, k.pair, k.qt, k.split);
 }
 
-// A cache whose heads have several bit-widths, all classes in one launch: pair k of the launch belongs to the
-// class that its range falls in (8-bit codes first: the longest workgroups start first), and the workgroup
-// runs that class's code.  The registers and the LDS are those of the most demanding class, which is no
-// more than each class takes alone (see launch_shape); what is gained are the launches -- and that the
-// classes, which have a few heads each, fill the device together.  Three widths, one launch per class ->
-// one launch, us: [2,16,128] 100 queries x 600 keys 66 -> 18, [8,16,128] 256 x 500 78 -> 28, 576 x 1497 140 ->
-// 117, 1024 x 2521 230 -> 200 (the last two with a stream for each class).
-struct ClassParams {
-  const u32 *k_words, *v_words;
-  const float *k_scale, *k_zp, *v_scale, *v_zp;
-  const int32_t *head_map;
-  int heads, first;   // packed heads of the class; its first pair of the launch
-};
-struct ClassTable { ClassParams c[3]; };   // of 8, 4 and 2 bits; a width that the cache does not have has no heads
-__device__ __forceinline__ void enter_class(AttnParams &p, const ClassParams &c) {
-  p.k_words = c.k_words; p.v_words = c.v_words;
-  p.k_scale = c.k_scale; p.k_zp = c.k_zp; p.v_scale = c.v_scale; p.v_zp = c.v_zp;
-  p.head_map = c.head_map;
-  p.Hkv = c.heads;
-  p.kv_bs = (int64_t)c.heads * p.Lstride;
-}
-// F(bits, pair within the class, pair of the output) for the class of pair k
-template <class F> __device__ __forceinline__ void in_class(AttnParams &p, const ClassTable &t, int k, F &&f) {
-  const int H = p.Hq;
-  auto run = [&](auto bits, const ClassParams &c) __attribute__((always_inline)) {
-    enter_class(p, c);
-    const int bh = k - c.first;
-    f(bits, bh, bh / c.heads * H + c.head_map[bh % c.heads]);
-  };
-  if (k < t.c[1].first) run(std::integral_constant<int, 8>{}, t.c[0]);
-  else if (k < t.c[2].first) run(std::integral_constant<int, 4>{}, t.c[1]);
-  else run(std::integral_constant<int, 2>{}, t.c[2]);
-}
-
 template <int D, int G, int NWV, int WPS, bool F16>
 __global__ __launch_bounds__(NWV * 64, WPS) void fused_attn_classes_kernel(AttnParams p, ClassTable t) {
   const BlockOf k(p);
@@ -1360,15 +1304,6 @@ template <int D, bool F16> void launch_combine(const AttnParams &p, hipStream_t 
 }
 
 int device_cus();
-
-// above 64 KiB of LDS the limit has to be raised, once per device the process launches on
-void allow_lds(const void *kernel, int bytes, bool (&configured)[64]) {
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) dev = -1;
-  if (dev >= 0 && configured[dev]) return;
-  (void)hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
-  if (dev >= 0) configured[dev] = true;
-}
 
 template <int D, int BITS, int GK, int GV, bool CHAN, int NWV, int WPS = 2, bool EXACT = false, bool F16 = false, bool ONE = false>
 void launch_shape(const AttnParams &p, hipStream_t st) {
@@ -1544,502 +1479,63 @@ int set_splits(AttnParams &p, int D, int tiles, int splits, void *workspace, siz
 }
 
 
-// ---- few queries over a long cache (the regime bound by the reads of the packed cache) -----------
-// With at most a few dozen queries per (batch, head) the arithmetic intensity of the attention,
-// 32 * Lq / (bits_K + bits_V) flop per packed byte, is below the machine balance: the kernel above,
-// built around 256 queries per workgroup, leaves seven of its eight wavefronts without queries and
-// spends a workgroup barrier per 64 keys on the remaining one.  This kernel turns the work round:
-// all wavefronts of a workgroup serve the SAME 32 queries and each takes its own 32-key blocks of
-// the workgroup's share of the keys, from global memory straight to registers, with nothing shared
-// between wavefronts inside the key loop and no workgroup barrier in it:
-//  * K: a lane loads half a key row (the half its MFMA A operands come from), dequantizes it in
-//    registers -- (code - zp) * scale in fp32, rounded to bf16, the operands the reference's
-//    attention sees -- and feeds S^T = K Q^T directly; the Q^T operands sit in LDS, written once;
-//  * V: a lane widens items of two adjacent keys x 8 channels into a wavefront-private V^T tile
-//    in LDS (the second contraction runs over keys), read back as MFMA A operands by the same
-//    wavefront -- LDS requests of one wavefront are served in order, so no barrier is needed;
-//  * online softmax per lane against a reference that moves only when a weight would pass 2^16;
-//  * a block runs S^T, then the V^T tile (under the S^T MFMAs), then the softmax, then O^T; the
-//    wavefront's next block is requested piece by piece as the current one frees its registers
-//    (K after S^T, V after the tile), each about a block's time ahead of its use.
-// The wavefronts' partial results are merged through LDS (each wavefront ends up with a quarter
-// of the channels), the workgroups' shares through the workspace and combine_splits_kernel, as
-// for the kernel above.
-// One scale group per key (group = D = 128), bf16, any layout, key limits, head maps.
-constexpr int FQ_NW = 4;             // wavefronts per workgroup
-constexpr int FQ_BK = 32;            // keys per block: one 32-row MFMA block
-constexpr int FQ_VTS = FQ_BK + 8;    // V^T row stride (bf16): 16-byte rows, bank spread
-constexpr int FQ_D = 128;
-constexpr int kFewQueries = 64;      // launches with at most this many queries per (batch, head) ...
-constexpr int kFewQMinKeys = 1024;   // ... over at least this many keys take this kernel
+// ---- few queries (few_attn.hip) -----------------------------------------------------------------
+// Launches of at most kFewQueries queries per (batch, head), in tiles of 32 that each dequantize the cache for themselves,
+// against 256 a workgroup and staged tiles of 64 keys in the kernel above.  Measured, us, the kernel above / that one, 4-bit
+// codes, one group, pairs of (batch, head) x queries x keys: up to 16 queries it is faster everywhere, D=64 32 x 16 x 32 4.2 / 3.8, 128 x 16 x 4096 44.7 /
+// 18.9, 240 x 16 x 1024 22 / 9.5, D=128 32 x 8 x 21 5.3 / 4.5, 240 x 16 x 1024 27.7 / 18.0.  More queries have two columns of 16 to prepare first: from the
+// second tile of keys on, D=64 32 x 24 x 64 4.4 / 5.0, x 128 5.6 / 4.9; D=128 5.7 / 6.6, 7.6 / 6.6.  Several tiles of queries that do not fit the device
+// at once pay with longer caches only, D=64 240 x 64 (480 tiles) x 128 6.7 / 7.3, x 256 9.4 / 9.1, x 1024 23.6 / 17.9, 480 x 64 (960) x 256 12.5 / 13.6, x 512
+// 19.8 / 18.6; three and four tiles not beyond the device, 240 x 100 x 1024 23.7 / 28.8, and not where the widening dominates, 128 x
+// 100 x 1024 21.2 / 18.0, x 2048 29.7 / 29.2, x 4096 48.4 / 52.0.
+constexpr int kFewQueries = 128;
 constexpr int kMaxKeyShares = kMaxKeyShares_v;
-struct FewQLds {
-  static constexpr int kVt = 0;                                        // [FQ_NW][D][FQ_VTS] bf16
-  // the merge slots -- for every wavefront, a quarter of each other wavefront's accumulators --
-  // start at the V^T tiles and need a little more
-  static constexpr int kSlotBytes = FQ_NW * (FQ_NW - 1) * 16 * 64 * 4;
-  static constexpr int kMl = kVt + (FQ_NW * FQ_D * FQ_VTS * 2 > kSlotBytes ? FQ_NW * FQ_D * FQ_VTS * 2 : kSlotBytes);   // [FQ_NW][32][2] fp32 (merge)
-  static constexpr int kBytes = kMl + FQ_NW * 32 * 2 * 4;
-};
-
-template <int BITS>
-__device__ __forceinline__ void attend_few(const AttnParams &p, int bh, int out_pair, int qt, int split) {
-  constexpr int D = FQ_D, WPR = D * BITS / 32, NCH = D / 16, NDB = D / 32;
-  constexpr int HW = WPR / 2;                 // packed words of half a key row
-  constexpr int KP = HW / 4;                  // 16-byte pieces of it
-  constexpr int OPQ = 16 / BITS;              // octets per piece
-  constexpr int UPR = BITS == 2 ? 8 : 16;     // V units per key row: a word, or the two words of an octet of bytes
-  constexpr int WPU = BITS == 8 ? 2 : 1;      // words per unit
-  constexpr int OPU = BITS == 2 ? 2 : 1;      // octets per unit
-  constexpr int IPL = 16 * UPR / 64;          // V items (two keys x one unit) per lane and block
-  static_assert(NDB == FQ_NW, "the merge gives every wavefront one 32-channel block of the output");
-  extern __shared__ __attribute__((aligned(16))) unsigned char lds_raw[];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int col = lane & 31, half = lane >> 5;
-  uint16_t *const vt = reinterpret_cast<uint16_t *>(lds_raw + FewQLds::kVt) + wave * D * FQ_VTS;
-  float *const lds_ml = reinterpret_cast<float *>(lds_raw + FewQLds::kMl);
-
-  const int b = bh / p.Hkv, hs = bh % p.Hkv;
-  const int hq = p.head_map ? p.head_map[hs] : hs;
-
-  const int qrow = qt * 32 + col;
-  const bool q_live = qrow < p.Lq;
-  int limit = p.kv_limit ? min(p.kv_limit[min(qrow, p.Lq - 1)], p.Lk) : p.Lk;
-  if (limit < 0) limit = 0;
-  // every wavefront holds the same queries: the largest and smallest limit need no exchange between them
-  int kv_end = q_live ? limit : 0, minlim = q_live ? limit : p.Lk;
-  if (p.kv_limit) {
-    for (int off = 1; off < 64; off <<= 1) {
-      kv_end = max(kv_end, __shfl_xor(kv_end, off, 64));
-      minlim = min(minlim, __shfl_xor(minlim, off, 64));
-    }
-  } else {
-    kv_end = p.Lk; minlim = p.Lk;   // (some query of the tile is live)
-  }
-  // the share's blocks: a fixed number per share (set by the host from Lk), cut at the tile's last key
-  const int nb = (kv_end + FQ_BK - 1) / FQ_BK;
-  const int b_begin = split * p.fq_share_blocks, b_end = min(b_begin + p.fq_share_blocks, nb);
-  // Block j of the share goes to wavefront (j + rot) % 4: the wavefront that gets the odd block
-  // more differs between the workgroups that are likely to sit on one compute unit.  (A function
-  // of the (batch, head) pair, the query tile and the share only, not of where the workgroup
-  // sits in the grid: the two cache layouts add up in the same order.)
-  const int slot_s = ((p.q_tiles == 2 ? ((bh >> 3) << 1) | qt : (bh >> 3))) * p.nsplit + split;
-  const int rot = (slot_s + (slot_s >> 5)) & 3;
-  const int blk0 = b_begin + ((wave - rot) & 3);
-
-  u32 kmask = KCodec<BITS>::kMask;
-  asm volatile("" : "+v"(kmask));
-
-  // Packed words and parameters of a block as loaded.  The registers are refilled with the
-  // wavefront's next block as soon as the current one has used them: K after S^T, V after the
-  // V^T tile is written.  The requests are issued without conditions around them (past the end
-  // they re-read the last key row; a missing zero-point array reads the scales instead): with a
-  // branch around a load the compiler no longer knows how many loads are in flight and waits for
-  // all of them where it needs the oldest.
-  // Addresses: the (batch, head) bases are uniform; a lane keeps 32-bit byte offsets of its rows
-  // from them, advanced by four blocks per request and clamped at the last key of the wavefront's
-  // own last block (the host checks that they fit) -- an add and a min per stream instead of the
-  // products of key and strides; the one request past the wavefront's blocks re-reads that row
-  // instead of fetching a block of another wavefront's.
-  const int64_t kv_row0 = b * p.kv_bs + hs * p.kv_hs;
-  const char *const kw_base = reinterpret_cast<const char *>(p.k_words + kv_row0 * WPR);
-  const char *const vw_base = reinterpret_cast<const char *>(p.v_words + kv_row0 * WPR);
-  const char *const ks_base = reinterpret_cast<const char *>(p.k_scale + kv_row0);
-  const char *const kz_base = reinterpret_cast<const char *>((p.k_zp ? p.k_zp : p.k_scale) + kv_row0);
-  const char *const vs_base = reinterpret_cast<const char *>(p.v_scale + kv_row0);
-  const char *const vz_base = reinterpret_cast<const char *>((p.v_zp ? p.v_zp : p.v_scale) + kv_row0);
-  const bool has_kzp = p.k_zp != nullptr, has_vzp = p.v_zp != nullptr;
-  const u32 row_b = (u32)p.kv_ts * (WPR * 4), par_b = (u32)p.kv_ts * 4;   // bytes from one key to the next
-  static_assert(FQ_NW == 4, "a wavefront's blocks are four apart");
-  const int last_blk = blk0 + ((max(b_end - 1 - blk0, 0) >> 2) << 2);   // (this wavefront's last block, if it has any)
-  const u32 last_key = (u32)min(last_blk * FQ_BK + FQ_BK - 1, p.Lk - 1);
-  const u32 par_last = last_key * par_b;
-  const u32 k_lane = half * (HW * 4), v_lane = (lane >> 4) * (WPU * 4);     // this lane's place inside a row
-  const u32 k_row_last = last_key * row_b + k_lane, v_row_last = last_key * row_b + v_lane;
-  const u32 row_step = FQ_NW * FQ_BK * row_b, par_step = FQ_NW * FQ_BK * par_b;
-  // MFMA row `col` carries key kperm(col) of the block; V: item = lane + 64 i covers keys 2 kp, 2 kp + 1
-  // (kp = lane & 15: the lanes of a tile row write 16 adjacent banks) and unit (lane >> 4) + 4 i
-  u32 ok_row = (u32)(blk0 * FQ_BK + kperm(col)) * row_b + k_lane, ok_par = (u32)(blk0 * FQ_BK + kperm(col)) * par_b;
-  u32 ov_row = (u32)(blk0 * FQ_BK + 2 * (lane & 15)) * row_b + v_lane, ov_par = (u32)(blk0 * FQ_BK + 2 * (lane & 15)) * par_b;
-  u32x4_t kraw[KP];
-  u32 vraw[IPL][2][WPU];
-  float ksc, kzp, vsc[2], vzp[2];   // (V: of this lane's two keys)
-  auto umin = [](u32 x, u32 y) { return x < y ? x : y; };
-  auto request_k = [&]() {   // the wavefront's next block
-    const u32 orow = umin(ok_row, k_row_last), opar = umin(ok_par, par_last);
-    ok_row += row_step; ok_par += par_step;
-#pragma unroll
-    for (int i = 0; i < KP; ++i) kraw[i] = *reinterpret_cast<const u32x4_t *>(kw_base + orow + 16 * i);
-    ksc = *reinterpret_cast<const float *>(ks_base + opar);
-    kzp = *reinterpret_cast<const float *>(kz_base + opar);
-  };
-  auto request_v = [&]() {
-    const u32 orow[2] = {umin(ov_row, v_row_last), umin(ov_row + row_b, v_row_last)};
-    const u32 opar[2] = {umin(ov_par, par_last), umin(ov_par + par_b, par_last)};
-    ov_row += row_step; ov_par += par_step;
-#pragma unroll
-    for (int r = 0; r < 2; ++r) {   // (the parameters first: the block's V work starts with them)
-      vsc[r] = *reinterpret_cast<const float *>(vs_base + opar[r]);
-      vzp[r] = *reinterpret_cast<const float *>(vz_base + opar[r]);
-    }
-#pragma unroll
-    for (int i = 0; i < IPL; ++i)
-#pragma unroll
-      for (int r = 0; r < 2; ++r) {
-        const char *src = vw_base + orow[r] + i * (4 * WPU * 4);
-        if constexpr (WPU == 2) { const uint2 t = *reinterpret_cast<const uint2 *>(src); vraw[i][r][0] = t.x; vraw[i][r][1] = t.y; }
-        else vraw[i][r][0] = *reinterpret_cast<const u32 *>(src);
-      }
-  };
-  // ---- this lane's query: the eight Q^T operands (channels in the slot order of the K codec)
-  // stay in registers for the whole key loop; the loads go out ahead of the first block's ----
-  u32x4_t qop[NCH];
-  {
-    const __bf16 *qp = p.q + (b * p.q_bs + hq * p.q_hs + min(qrow, p.Lq - 1) * p.q_ts) * D + half * 64;
-#pragma unroll
-    for (int ch = 0; ch < NCH; ++ch) qop[ch] = *reinterpret_cast<const u32x4_t *>(qp + ch * 8);
-  }
-  // (the loads keep this order -- queries, K, V: the compiler's count of loads in flight on the
-  // way into the key loop becomes what it waits for inside it)
-  __builtin_amdgcn_sched_barrier(0);
-  request_k();
-  __builtin_amdgcn_sched_barrier(0);
-  request_v();
-  __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-  for (int ch = 0; ch < NCH; ++ch) {
-    const u32x4_t raw = qop[ch];
-#pragma unroll
-    for (int j2 = 0; j2 < 4; ++j2) {
-      const int d0 = KCodec<BITS>::slot_d(2 * j2), d1 = KCodec<BITS>::slot_d(2 * j2 + 1);
-      const u32 lo = (raw[d0 >> 1] >> (16 * (d0 & 1))) & 0xffffu, hi = (raw[d1 >> 1] >> (16 * (d1 & 1))) << 16;
-      qop[ch][j2] = lo | hi;
-    }
-  }
-
-  floatx16_t oacc[NDB];
-#pragma unroll
-  for (int d = 0; d < NDB; ++d)
-#pragma unroll
-    for (int j = 0; j < 16; ++j) oacc[d][j] = 0.f;
-  float m_ref = 0.f, l_part = 0.f;
-  bool first = true;
-
-  // One block of 32 keys.  BYTES: 4-bit codes through bytes (see byte_bias4), with the bias ka4
-  // of this lane's K row; V goes through bytes too if its zero-points fit.
-  auto block = [&](const int blk, auto bytes_tag, const u32 ka4) {
-    constexpr bool BYTES = decltype(bytes_tag)::value;
-    const int t0 = blk * FQ_BK;
-    // (code - zp) * scale = (raw - (zp + kOff) / kMul) * (kMul * scale) for the code image `raw`
-    const float kz = has_kzp ? kzp : 0.f;
-    const float zk = (kz + KCodec<BITS>::kOff) * (1.f / KCodec<BITS>::kMul), sk = ksc * KCodec<BITS>::kMul;
-    const float ks_plain = ksc, kc = -128.f * ksc;
-
-    // ---- S^T = K Q^T, K dequantized in registers ----
-    floatx16_t sacc;
-#pragma unroll
-    for (int j = 0; j < 16; ++j) sacc[j] = 0.f;
-#pragma unroll
-    for (int ch = 0; ch < NCH; ++ch) {
-      const int pc = ch / OPQ, j = ch % OPQ;
-      u32 q4[4];
-#pragma unroll
-      for (int w = 0; w < 4; ++w) q4[w] = kraw[pc][w] ^ KCodec<BITS>::kStageXor;
-      u32x4_t a;
-      if constexpr (BYTES) {
-        const u32 e = (q4[j] & 0x0f0f0f0fu) + ka4, o = ((q4[j] >> 4) & 0x0f0f0f0fu) + ka4;
-        // operand slots (2m, 2m+1) hold channels (m, m+4): bytes 0 and 2 of e are channels 0 and 4, ...
-        a[0] = pack_bf16_rne(__builtin_fmaf(ubyte_f32(e, 0), ks_plain, kc), __builtin_fmaf(ubyte_f32(e, 2), ks_plain, kc));
-        a[1] = pack_bf16_rne(__builtin_fmaf(ubyte_f32(o, 0), ks_plain, kc), __builtin_fmaf(ubyte_f32(o, 2), ks_plain, kc));
-        a[2] = pack_bf16_rne(__builtin_fmaf(ubyte_f32(e, 1), ks_plain, kc), __builtin_fmaf(ubyte_f32(e, 3), ks_plain, kc));
-        a[3] = pack_bf16_rne(__builtin_fmaf(ubyte_f32(o, 1), ks_plain, kc), __builtin_fmaf(ubyte_f32(o, 3), ks_plain, kc));
-      } else {
-        float f[8];
-        k_values<BITS>(q4, j, kmask, f);
-#pragma unroll
-        for (int m = 0; m < 4; ++m) a[m] = pack_bf16_rne((f[2 * m] - zk) * sk, (f[2 * m + 1] - zk) * sk);
-      }
-      sacc = mfma_32x32x16<false>(a, qop[ch], sacc);
-    }
-    request_k();
-
-    // ---- V of the block -> V^T tile of this wavefront (bf16 values) ----
-    // (z2, s2: byte biases and plain scales of the lane's two keys, or the general form's parameters)
-    bool vbytes = false;
-    float2 z2, s2;
-    {
-      u32 va0 = 0, va1 = 0;
-      const float vz0 = has_vzp ? vzp[0] : 0.f, vz1 = has_vzp ? vzp[1] : 0.f;
-      if constexpr (BYTES) {
-        const bool ok0 = byte_bias4(vz0, va0), ok1 = byte_bias4(vz1, va1);
-        vbytes = !__any(!(ok0 && ok1));
-      }
-      z2.x = vbytes ? u2f(va0) : (vz0 + VCodec<BITS>::kOff) * (1.f / VCodec<BITS>::kMul);
-      z2.y = vbytes ? u2f(va1) : (vz1 + VCodec<BITS>::kOff) * (1.f / VCodec<BITS>::kMul);
-      s2.x = vbytes ? vsc[0] : vsc[0] * VCodec<BITS>::kMul;
-      s2.y = vbytes ? vsc[1] : vsc[1] * VCodec<BITS>::kMul;
-    }
-#pragma unroll
-    for (int i = 0; i < IPL; ++i) {
-      const int item = lane + 64 * i, kp = item & 15, u = item >> 4;   // (key pair fastest: the lanes of a row write 16 adjacent banks)
-      u32 r0[WPU], r1[WPU];
-#pragma unroll
-      for (int w = 0; w < WPU; ++w) { r0[w] = vraw[i][0][w] ^ VCodec<BITS>::kStageXor; r1[w] = vraw[i][1][w] ^ VCodec<BITS>::kStageXor; }
-      if (BYTES && vbytes) {
-        // (z2 holds the two keys' byte biases, s2 their plain scales)
-        const u32 e0 = (r0[0] & 0x0f0f0f0fu) + f2u(z2.x), o0 = ((r0[0] >> 4) & 0x0f0f0f0fu) + f2u(z2.x);
-        const u32 e1 = (r1[0] & 0x0f0f0f0fu) + f2u(z2.y), o1 = ((r1[0] >> 4) & 0x0f0f0f0fu) + f2u(z2.y);
-        const float c0 = -128.f * s2.x, c1 = -128.f * s2.y;
-#pragma unroll
-        for (int j2 = 0; j2 < 4; ++j2) {
-          *reinterpret_cast<u32 *>(&vt[(u * 8 + 2 * j2) * FQ_VTS + kp * 2]) =
-              pack_bf16_rne(__builtin_fmaf(ubyte_f32(e0, j2), s2.x, c0), __builtin_fmaf(ubyte_f32(e1, j2), s2.y, c1));
-          *reinterpret_cast<u32 *>(&vt[(u * 8 + 2 * j2 + 1) * FQ_VTS + kp * 2]) =
-              pack_bf16_rne(__builtin_fmaf(ubyte_f32(o0, j2), s2.x, c0), __builtin_fmaf(ubyte_f32(o1, j2), s2.y, c1));
-        }
-      } else {
-#pragma unroll
-        for (int o = 0; o < OPU; ++o) {
-          float f0[8], f1[8];
-          v_pair_values<BITS>(r0, r1, o, kmask, f0, f1);
-          const int oct = u * OPU + o;
-#pragma unroll
-          for (int j = 0; j < 8; ++j)
-            *reinterpret_cast<u32 *>(&vt[(oct * 8 + j) * FQ_VTS + kp * 2]) = pack_bf16_rne((f0[j] - z2.x) * s2.x, (f1[j] - z2.y) * s2.y);
-        }
-      }
-    }
-    request_v();
-
-    // ---- softmax of the block: register i <-> key t0 + 16*(i/8) + 8*half + i%8 ----
-    // The logits are taken against the reference as it stands (log2 domain) and the reference
-    // moves only when a weight would exceed 2^16, which the block's sum of weights shows -- the
-    // denominator needs that sum anyway, and the common block then has no search for the row
-    // maximum and no rescaling of the 64 output accumulators.
-    float z[16];
-#pragma unroll
-    for (int i = 0; i < 16; ++i) z[i] = __builtin_fmaf(p.scale_log2e, sacc[i], -m_ref);
-    if (t0 + FQ_BK > minlim) {
-#pragma unroll
-      for (int i = 0; i < 16; ++i)
-        if (t0 + 16 * (i >> 3) + 8 * half + (i & 7) >= limit) z[i] = -INFINITY;
-    }
-    // Moves the reference to the row's current maximum: up only once something has been
-    // accumulated; the first block takes its maximum as it is (the accumulators are zero).
-    auto move_reference = [&]() {
-      float zmax = z[0];
-#pragma unroll
-      for (int i = 1; i < 16; ++i) zmax = fmaxf(zmax, z[i]);
-      {
-        const auto sw = __builtin_amdgcn_permlane32_swap(f2u(zmax), f2u(zmax), false, false);
-        zmax = fmaxf(u2f(sw[0]), u2f(sw[1]));
-      }
-      const float delta = first ? ((zmax == -INFINITY) ? 0.f : zmax) : fmaxf(zmax, 0.f);
-      const float alpha = first ? 1.f : __builtin_amdgcn_exp2f(-delta);
-      m_ref += delta;
-#pragma unroll
-      for (int i = 0; i < 16; ++i) z[i] -= delta;
-#pragma unroll
-      for (int d = 0; d < NDB; ++d)
-#pragma unroll
-        for (int j = 0; j < 16; ++j) oacc[d][j] *= alpha;
-      l_part *= alpha;
-    };
-    u32 pop[2][4];
-    float bsum = 0.f;
-    auto weights = [&]() {
-      bsum = 0.f;
-#pragma unroll
-      for (int i2 = 0; i2 < 8; ++i2) {
-        const int i = 2 * i2;
-        const u32 w = pack_bf16_rne(__builtin_amdgcn_exp2f(z[i]), __builtin_amdgcn_exp2f(z[i + 1]));
-        pop[i >> 3][(i & 7) >> 1] = w;
-        typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
-        bsum = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2_t, w), __builtin_bit_cast(bf16x2_t, 0x3f803f80u), bsum, false);
-      }
-    };
-    if (first) move_reference();
-    weights();
-    if (!first && __any(!(bsum <= 65536.f))) {
-      move_reference();
-      weights();
-    }
-    l_part += bsum;
-    first = false;
-
-    // ---- O^T += V^T P^T ----
-#pragma unroll
-    for (int c = 0; c < 2; ++c) {
-      const u32x4_t bv = {pop[c][0], pop[c][1], pop[c][2], pop[c][3]};
-#pragma unroll
-      for (int d = 0; d < NDB; ++d) {
-        const u32x4_t av = *reinterpret_cast<const u32x4_t *>(&vt[(d * 32 + col) * FQ_VTS + c * 16 + half * 8]);
-        oacc[d] = mfma_32x32x16<false>(av, bv, oacc[d]);
-      }
-    }
-  };
-
-  // 4-bit codes go through bytes until a K zero-point of a block does not fit; from there on (and
-  // for the other widths) the general form.  Two loops one after the other rather than two arms
-  // inside one: arms that both update the output accumulators make the compiler copy them at
-  // the join, twice per block.
-  int blk = blk0;
-  if constexpr (BITS == 4) {
-    for (; blk < b_end; blk += FQ_NW) {
-      u32 ka4 = 0;
-      if (__any(!byte_bias4(has_kzp ? kzp : 0.f, ka4))) break;
-      // Two workgroups share a compute unit and the SIMD's arbiter prefers the older wavefront:
-      // left alone, the older workgroup finishes about a quarter earlier and the younger one
-      // then runs its rest at one wavefront per SIMD.  Priority by the quarter of its own
-      // blocks a wavefront is in lets the one that is behind catch up.
-      {
-        const int q4 = (blk - blk0) * 4 / max(b_end - blk0, 1);
-        if (q4 == 0) __builtin_amdgcn_s_setprio(3);
-        else if (q4 == 1) __builtin_amdgcn_s_setprio(2);
-        else if (q4 == 2) __builtin_amdgcn_s_setprio(1);
-        else __builtin_amdgcn_s_setprio(0);
-      }
-      block(blk, std::true_type{}, ka4);
-    }
-  }
-  for (; blk < b_end; blk += FQ_NW) block(blk, std::false_type{}, 0u);
-
-  // ---- merge the wavefronts' partial results: wavefront t ends up with channels 32t .. 32t+31 ----
-  // Every wavefront hands the other three their quarters of its accumulators through LDS (one
-  // barrier on each side), forms the four weights from everyone's (m, l) and sums its quarter.
-  const float l_own = l_part + __shfl_xor(l_part, 32, 64);
-  float *const slots = reinterpret_cast<float *>(lds_raw + FewQLds::kVt);   // [target][source - target - 1 mod 4][16 registers][64 lanes]
-  __syncthreads();   // every wavefront is done with its V^T tile
-#pragma unroll
-  for (int t = 0; t < FQ_NW; ++t) {
-    if (t == wave) continue;
-    float *dst = slots + ((t * 3 + ((wave - t - 1) & 3)) * 16) * 64 + lane;
-#pragma unroll
-    for (int j = 0; j < 16; ++j) dst[j * 64] = oacc[t][j];
-  }
-  if (half == 0) *reinterpret_cast<float2 *>(lds_ml + (wave * 32 + col) * 2) = make_float2(m_ref, l_own);
-  __syncthreads();
-  // (the partial results are addressed through LDS, not through register arrays with a run-time index)
-  float M = 0.f;
-  bool any_live = false;
-#pragma unroll
-  for (int w = 0; w < FQ_NW; ++w) {
-    const float2 ml = *reinterpret_cast<const float2 *>(lds_ml + (w * 32 + col) * 2);
-    if (ml.y != 0.f) { M = any_live ? fmaxf(M, ml.x) : ml.x; any_live = true; }
-  }
-  auto weight_of = [&](int w, float &l_w) {
-    const float2 ml = *reinterpret_cast<const float2 *>(lds_ml + (w * 32 + col) * 2);
-    l_w = ml.y;
-    return ml.y != 0.f ? __builtin_amdgcn_exp2f(ml.x - M) : 0.f;
-  };
-  float l_sum = 0.f;   // (summed in the same order by every wavefront)
-#pragma unroll
-  for (int w = 0; w < FQ_NW; ++w) {
-    float l_w;
-    const float wt = weight_of(w, l_w);
-    l_sum = __builtin_fmaf(l_w, wt, l_sum);
-  }
-  float mine[16];
-  {
-    float l_w;
-    const float w_own = weight_of(wave, l_w);
-#pragma unroll
-    for (int t = 0; t < FQ_NW; ++t)
-      if (t == wave) {   // (a wavefront-uniform choice among the four accumulator blocks)
-#pragma unroll
-        for (int j = 0; j < 16; ++j) mine[j] = oacc[t][j] * w_own;
-      }
-  }
-#pragma unroll
-  for (int s = 0; s < FQ_NW - 1; ++s) {
-    float l_w;
-    const float ws = weight_of((wave + 1 + s) & 3, l_w);
-    const float *src = slots + ((wave * 3 + s) * 16) * 64 + lane;
-#pragma unroll
-    for (int j = 0; j < 16; ++j) mine[j] = __builtin_fmaf(src[j * 64], ws, mine[j]);
-  }
-  if (!q_live) return;
-  const float inv = l_sum > 0.f ? 1.0f / l_sum : 0.f;
-  // registers 4*g4 .. 4*g4+3 are rows 32*wave + 8*g4 + 4*half + 0..3 of O^T
-  if (p.nsplit > 1) {
-    const int64_t prow = ((int64_t)split * p.bh_total + out_pair) * p.Lq + qrow;
-    float *wptr = p.ws_o + prow * D + wave * 32 + 4 * half;
-    if (wave == 0 && half == 0) *reinterpret_cast<float2 *>(p.ws_ml + prow * 2) = make_float2(M, l_sum);
-#pragma unroll
-    for (int g4 = 0; g4 < 4; ++g4)
-      *reinterpret_cast<float4 *>(wptr + 8 * g4) = make_float4(mine[4 * g4] * inv, mine[4 * g4 + 1] * inv, mine[4 * g4 + 2] * inv, mine[4 * g4 + 3] * inv);
-  } else {
-    __bf16 *optr = p.out + (b * p.o_bs + hq * p.o_hs + qrow * p.o_ts) * D + wave * 32 + 4 * half;
-#pragma unroll
-    for (int g4 = 0; g4 < 4; ++g4)
-      *reinterpret_cast<uint2 *>(optr + 8 * g4) =
-          make_uint2(pack_bf16_rne(mine[4 * g4] * inv, mine[4 * g4 + 1] * inv), pack_bf16_rne(mine[4 * g4 + 2] * inv, mine[4 * g4 + 3] * inv));
-  }
-}
-
-// Workgroup -> (pair, query tile, share) without a division: the grid is (8, shares, groups of eight
-// (batch, head) x query tiles); x runs fastest in the dispatch order, so the workgroups of one (batch,
-// head) sit on one XCD (one L2), as in the kernel above.
-struct FewBlockOf {
-  int pair, qt, split;
-  __device__ __forceinline__ explicit FewBlockOf(const AttnParams &p) {
-    static_assert(kFewQueries <= 64, "at most two query tiles");
-    const int xcd = blockIdx.x, slot = blockIdx.z;
-    split = blockIdx.y;
-    qt = p.q_tiles == 2 ? (slot & 1) : 0;
-    const int grp = p.q_tiles == 2 ? (slot >> 1) : slot;
-    pair = p.kv_hs == 1 && p.kv_ts > 1 ? xcd * ((p.bh_total + 7) >> 3) + grp : grp * 8 + xcd;   // (as in BlockOf)
-  }
-};
-template <int BITS>
-__global__ __launch_bounds__(FQ_NW * 64, 2) void fused_attn_fewq_kernel(AttnParams p) {
-  const FewBlockOf k(p);
-  if (k.pair >= p.bh_total) return;
-  attend_few<BITS>(p, k.pair, k.pair, k.qt, k.split);
-}
-__global__ __launch_bounds__(FQ_NW * 64, 2) void fused_attn_fewq_classes_kernel(AttnParams p, ClassTable t) {
-  const FewBlockOf k(p);
-  if (k.pair >= p.bh_total) return;
-  in_class(p, t, k.pair, [&](auto bits, int bh, int out_pair) __attribute__((always_inline)) {
-    attend_few<decltype(bits)::value>(p, bh, out_pair, k.qt, k.split);
-  });
-}
-
-// Whether a launch takes the few-queries kernel, and over how many workgroups the keys of a
-// (batch, head, 32 queries) are shared out then: enough for the two resident workgroups per
-// compute unit (the kernel holds ~200 registers), at least eight blocks per workgroup.
 bool fewq_eligible(int B, int Hkv, int Lq, int Lk, int D, int k_group, int v_group) {
   // (the kernel keeps 32-bit byte offsets inside one (batch, head): rows of up to D bytes, up to
   // Hkv rows from one key to the next, a few blocks of overshoot before the clamp)
-  return D == FQ_D && k_group == D && v_group == D && Lq > 0 && Lq <= kFewQueries && Lk >= kFewQMinKeys &&
-         ((int64_t)Lk + 8 * FQ_BK) * Hkv * D < (1ll << 32) &&
-         ((int64_t)B * Hkv + 7) / 8 * ((Lq + 31) / 32) <= 65535;   // (the grid's z extent)
+  const int64_t q_tiles = (Lq + 31) / 32, tiles = (int64_t)B * Hkv * q_tiles;
+  if (!((D == 64 || D == 128) && D % k_group == 0 && D % v_group == 0 && D / k_group <= kFewGroups && D / v_group <= kFewGroups && Lq > 0 &&
+        Lq <= kFewQueries && ((int64_t)Lk + 32 * kFewBlock) * Hkv * D < (1ll << 32) && ((int64_t)B * Hkv + 7) / 8 * q_tiles <= 65535))   // (the grid's z extent)
+    return false;
+  if (Lq <= 16) return true;
+  const int cus = device_cus();
+  if (q_tiles > 2 && (tiles > 2 * cus || Lk > 2048)) return false;
+  return Lk > (q_tiles == 1 || tiles <= cus ? 64 : tiles <= 2 * cus ? 255 : 511);
 }
-int fewq_shares(int bh_total, int Lq, int Lk) {
-  const int64_t tiles = (int64_t)((bh_total + 7) / 8 * 8) * ((Lq + 31) / 32);
-  int64_t s = (2 * (int64_t)device_cus() + tiles - 1) / tiles;
-  const int64_t nb = (Lk + FQ_BK - 1) / FQ_BK;
-  if (s > nb / 8) s = nb / 8;
-  if (s > kMaxKeyShares) s = kMaxKeyShares;
+// Over how many workgroups the keys of a tile of queries are shared out: as many as are resident together (more would
+// be a second round: 56 pairs x 2 queries x 41576 keys, ten shares each 108 us, nine 92), at least eight blocks each, and not
+// at all for a cache so short that the second launch costs more.
+int fewq_shares(int bh_total, int Lq, int Lk, int D, int k_group, int v_group) {
+  const int64_t tiles = (int64_t)((bh_total + 7) / 8 * 8) * ((Lq + 31) / 32), nb = (Lk + kFewBlock - 1) / kFewBlock;
+  if (nb < 24) return 1;
+  const int64_t resident = D == 128 && k_group == D && v_group == D ? 2 * (int64_t)device_cus() : (int64_t)device_cus();
+  const int64_t s = std::min(std::min(resident / tiles, nb / 8), (int64_t)kMaxKeyShares);
   return s < 1 ? 1 : (int)s;
 }
 
 // The split fields of a launch of the few-queries kernel: no more shares than the workspace holds.
-void set_few(AttnParams &p, void *workspace, size_t workspace_bytes) {
+void set_few(AttnParams &p, int D, int k_group, int v_group, void *workspace, size_t workspace_bytes) {
   const int64_t rows = (int64_t)p.bh_total * p.Lq;
-  int n = fewq_shares(p.bh_total, p.Lq, p.Lk);
-  while (n > 1 && (!workspace || ((uintptr_t)workspace & 15) || workspace_bytes < split_workspace_bytes(n, rows, FQ_D))) --n;
+  int n = fewq_shares(p.bh_total, p.Lq, p.Lk, D, k_group, v_group);
+  while (n > 1 && (!workspace || ((uintptr_t)workspace & 15) || workspace_bytes < split_workspace_bytes(n, rows, D))) --n;
   p.q_tiles = (p.Lq + 31) / 32;
   p.nsplit = n;
-  p.fq_share_blocks = ((p.Lk + FQ_BK - 1) / FQ_BK + n - 1) / n;
+  p.fq_share_blocks = ((p.Lk + kFewBlock - 1) / kFewBlock + n - 1) / n;
+  // Eight wavefronts instead of four halve the chain of blocks of a share; where several workgroups run on a compute unit they
+  // only cost registers (two columns of queries: one workgroup instead of three).  Below 1024 keys the number of
+  // pairs does not matter, so that a pair's result does not depend on how many others the launch has.
+  const int nb = (p.Lk + kFewBlock - 1) / kFewBlock;
+  const bool alone = nb < 32 ? p.Lq <= 16 : (int64_t)p.bh_total * p.q_tiles * n <= device_cus();
+  p.few_waves = p.fq_share_blocks > 8 && alone ? 8 : 4;
   p.ws_o = n > 1 ? reinterpret_cast<float *>(workspace) : nullptr;
-  p.ws_ml = n > 1 ? p.ws_o + (size_t)n * (size_t)rows * (size_t)FQ_D : nullptr;
+  p.ws_ml = n > 1 ? p.ws_o + (size_t)n * (size_t)rows * (size_t)D : nullptr;
 }
-
-dim3 few_grid(const AttnParams &p) { return dim3(8, (unsigned)p.nsplit, (unsigned)((p.bh_total + 7) / 8 * p.q_tiles)); }
-template <int BITS> void launch_fewq(const AttnParams &p, hipStream_t st) {
-  hipLaunchKernelGGL((fused_attn_fewq_kernel<BITS>), few_grid(p), dim3(FQ_NW * 64), FewQLds::kBytes, st, p);
-  if (p.nsplit > 1) launch_combine<FQ_D, false>(p, st);
+// ... the second launch of one with shares
+void combine_few(const AttnParams &p, int D, hipStream_t st) {
+  if (p.nsplit <= 1) return;
+  if (D == 128) launch_combine<128, false>(p, st);
+  else if (p.f16) launch_combine<64, true>(p, st);
+  else launch_combine<64, false>(p, st);
 }
 
 // ---- many queries: K and V expanded once, then a plain flash attention (wide_attn.hip) ----------
@@ -2120,7 +1616,7 @@ extern "C" size_t varq_fused_attn_workspace_bytes(int B, int Hkv, int Lq, int Lk
   int n = splits ? splits : choose_splits((int64_t)B * Hkv * ((Lq + BM - 1) / BM), tiles, rows, D);
   // (the group sizes are not known here: room for the few-queries kernel's shares whenever the
   // other sizes would admit it)
-  if (splits == 0 && fewq_eligible(B, Hkv, Lq, Lk, D, D, D)) n = max(n, fewq_shares(B * Hkv, Lq, Lk));
+  if (splits == 0 && fewq_eligible(B, Hkv, Lq, Lk, D, D, D)) n = max(n, fewq_shares(B * Hkv, Lq, Lk, D, D, D));
   return split_workspace_bytes(n, rows, D);
 }
 
@@ -2131,7 +1627,7 @@ extern "C" size_t varq_fused_attn_expand_bytes_limits(int B, int Hkv, int Lq, in
 
 extern "C" int varq_fused_attn_key_shares(int B, int Hkv, int Lq, int Lk, int D, int k_group, int v_group) {
   if (B <= 0 || Hkv <= 0 || Lq <= 0 || Lk <= 0 || (D != 64 && D != 128)) return 0;
-  if (fewq_eligible(B, Hkv, Lq, Lk, D, k_group, v_group)) return fewq_shares(B * Hkv, Lq, Lk);
+  if (fewq_eligible(B, Hkv, Lq, Lk, D, k_group, v_group)) return fewq_shares(B * Hkv, Lq, Lk, D, k_group, v_group);
   return choose_splits((int64_t)B * Hkv * ((Lq + BM - 1) / BM), (Lk + BN - 1) / BN, (int64_t)B * Hkv * Lq, D);
 }
 
@@ -2183,12 +1679,12 @@ extern "C" int varq_fused_attn(const void *q, void *out,
   p.exact_codes = operand_form == VARQ_ATTN_EXACT_CODES && !p.f16;
   if (int e = set_layout(p, layout, "fused_attn")) return e;
   hipStream_t st = (hipStream_t)stream;
-  // few queries over a long cache, left to the library: the kernel whose wavefronts share the keys
-  if (splits == 0 && !p.f16 && !p.exact_codes && fewq_eligible(B, Hkv, Lq, Lk, D, k_group, v_group)) {
-    set_few(p, workspace, workspace_bytes);
-    if (k_bits == 4) launch_fewq<4>(p, st);
-    else if (k_bits == 8) launch_fewq<8>(p, st);
-    else launch_fewq<2>(p, st);
+  // few queries, left to the library: the kernel whose wavefronts share the keys (it has no exact form)
+  const bool exact_form = p.exact_codes && D == 128 && k_group == D && v_group == D && k_bits != 8;
+  if (splits == 0 && !exact_form && groups_served(D, k_group, v_group) && fewq_eligible(B, Hkv, Lq, Lk, D, k_group, v_group)) {
+    set_few(p, D, k_group, v_group, workspace, workspace_bytes);
+    launch_few(p, D, k_bits, k_group, v_group, st);
+    combine_few(p, D, st);
     VARQ_CHECK_LAUNCH("fused_attn");
     return VARQ_OK;
   }
@@ -2345,10 +1841,10 @@ extern "C" int varq_fused_attn_classes(const void *q, void *out, const varq_kv_c
   p.f16 = io_dtype == VARQ_F16;
   if (int e = set_layout(p, layout, "fused_attn_classes")) return e;
   hipStream_t st = (hipStream_t)stream;
-  if (splits == 0 && !p.f16 && fewq_eligible(B, H, Lq, Lk, D, group, group)) {
-    set_few(p, workspace, workspace_bytes);
-    hipLaunchKernelGGL(fused_attn_fewq_classes_kernel, few_grid(p), dim3(FQ_NW * 64), FewQLds::kBytes, st, p, t);
-    if (p.nsplit > 1) launch_combine<FQ_D, false>(p, st);
+  if (splits == 0 && fewq_eligible(B, H, Lq, Lk, D, group, group)) {
+    set_few(p, D, group, group, workspace, workspace_bytes);
+    launch_few_classes(p, D, t, group, st);
+    combine_few(p, D, st);
   } else if ((splits == 0 || splits == 1) && wide_eligible(B, p.Hkv, Lq, Lk, D, kv_limit != nullptr) &&
              run_wide(p, D, splits, workspace, workspace_bytes, st, [&](const AttnParams &part, int first, char *ws) {
                // (one expanding launch per class, into the places of its heads)
