@@ -45,6 +45,22 @@ __device__ __forceinline__ float dec_ord(u32 e) {
   return u2f((e & 0x80000000u) ? (e & 0x7fffffffu) : ~e);
 }
 
+// n / d for n < 2^31 by a product: with s = ceil(log2 d) - 1 and mul = floor(2^(32 + s) / d) + 1 the product is too large by
+// n e / (2^(32 + s) d) for some e <= d <= 2^(s + 1), less than 1 / d.  (d = 1: mul = 0 and `all` takes n itself.)  A division of the
+// compiler's is some twenty instructions, and the kernels below have two for every octet.
+struct FastDiv {
+  u32 mul, all;
+  int shift;
+  static FastDiv by(int64_t d) {   // (anything from 2^31 on divides to 0)
+    if (d <= 1) return {0u, 0xffffffffu, 0};
+    if (d >= (1ll << 31)) return {0u, 0u, 0};
+    int s = 0;
+    while ((2ll << s) < d) ++s;
+    return {(u32)((1ull << (32 + s)) / (unsigned long long)d + 1), 0u, s};
+  }
+  __device__ __forceinline__ u32 operator()(u32 n) const { return (__umulhi(n, mul) + (n & all)) >> shift; }
+};
+
 struct GenParams {
   const void *x;
   u32 *ws_max;   // [n_groups] encoded max (or max-abs)
@@ -67,6 +83,7 @@ struct GenParams {
   // [B,H,cap,..] is (n, cap - n, len), a step [B,n,H,c] into [B,cap,H,..] is (n*H, (cap - n)*H, len*H).
   int out_mapped;
   int64_t out_inner, out_delta, out_off;
+  FastDiv by_inner;
   // a second tensor of the same shape in the same launches (blockIdx.y == 1): its input,
   // its outputs and the distance (in 4-byte words) to its part of the workspace
   const void *x1;
@@ -88,7 +105,7 @@ __device__ __forceinline__ int64_t out_row(const GenParams &p, int64_t row) {
 }
 // (rows of the tiled kernels fit 31 bits)
 __device__ __forceinline__ int64_t out_row32(const GenParams &p, int64_t row) {
-  return p.out_mapped ? row + (int64_t)((u32)row / (u32)p.out_inner) * p.out_delta + p.out_off : row;
+  return p.out_mapped ? row + (int64_t)p.by_inner((u32)row) * p.out_delta + p.out_off : row;
 }
 
 __global__ void init_ws_kernel(u32 *ws_max, u32 *ws_min, int64_t n) {
@@ -155,33 +172,27 @@ __device__ __forceinline__ Lane decode(const Plan &pl) {
 // this lane's octet.
 template <int DT, typename F>
 __device__ __forceinline__ void for_rows(const GenParams &p, const Plan &pl, const Lane &l, F body) {
-  const int s0 = l.z * pl.steps_per_chunk, s1 = min(s0 + pl.steps_per_chunk, pl.steps);
-  const int64_t base = (int64_t)l.ko * pl.ko_rs + l.q;
-  const int64_t col8 = l.col * 8;
+  // (scalars: the rows of a step differ between the lanes by what lane_row holds)
+  const int s0 = __builtin_amdgcn_readfirstlane(l.z * pl.steps_per_chunk), s1 = min(s0 + pl.steps_per_chunk, pl.steps);
+  const int64_t lane_row = (int64_t)l.ko * pl.ko_rs + l.q + (pl.fold_ro ? l.f * pl.ro_rs : l.f);
+  const char *const lane_x = reinterpret_cast<const char *>(p.x) + (lane_row * p.c + l.col * 8) * In8<DT>::kBytes;
+  const int64_t row_bytes = (int64_t)p.c * In8<DT>::kBytes;
+  auto take = [&](int64_t step_row) __attribute__((always_inline)) {
+    float v[8];
+    In8<DT>::load(lane_x + step_row * row_bytes, 0, v);
+    body((u32)lane_row + (u32)step_row, v);
+  };
   // (one load in flight per lane: issuing two steps' loads before either is used, or the next
   // row's load ahead of the current row's arithmetic, was measured 5-15 % slower on both phases)
   if (pl.fold_ro) {
     // d2 kept: a step is `sub` consecutive reduced positions
-    for (int s = s0; s < s1; ++s) {
-      const int ro = s * pl.sub + l.f;
-      if (ro < pl.nro) {
-        const int64_t r = base + (int64_t)ro * pl.ro_rs;
-        float v[8];
-        In8<DT>::load(p.x, r * p.c + col8, v);
-        body(r, v);
-      }
-    }
+    for (int s = s0; s < s1; ++s)
+      if (s * pl.sub + l.f < pl.nro) take((int64_t)s * pl.sub * pl.ro_rs);
   } else {
     // d2 reduced: a step is `sub` (= R) consecutive rows of one ro
     int ro = s0 / pl.T, t = s0 - ro * pl.T;
     for (int s = s0; s < s1; ++s) {
-      const int ri = t * pl.sub + l.f;
-      if (ri < pl.RI) {
-        const int64_t r = base + (int64_t)ro * pl.ro_rs + ri;
-        float v[8];
-        In8<DT>::load(p.x, r * p.c + col8, v);
-        body(r, v);
-      }
+      if (t * pl.sub + l.f < pl.RI) take((int64_t)ro * pl.ro_rs + t * pl.sub);
       if (++t == pl.T) { t = 0; ++ro; }
     }
   }
@@ -198,7 +209,7 @@ __global__ __launch_bounds__(256) void minmax_tiled_kernel(GenParams p, Plan pl,
 #pragma unroll
   for (int j = 0; j < NV; ++j) { mx[j] = ASYM ? -INFINITY : 0.f; mn[j] = INFINITY; }
   if (l.live) {
-    for_rows<DT>(p, pl, l, [&](int64_t, const float (&v)[8]) {
+    for_rows<DT>(p, pl, l, [&](u32, const float (&v)[8]) {
       if (KEEPC) {
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
@@ -303,10 +314,11 @@ __global__ __launch_bounds__(256) void finalize_tiled_kernel(GenParams p, int Z,
   if (zl != 0 || g >= p.n_groups) return;
   mx = lds_mx[threadIdx.x];
   mn = lds_mn[threadIdx.x];
-  float s;
+  float s, z = 0.f;
   if (ASYM) {
     s = fmaxf((mx - mn) / (float)((1 << p.bits) - 1), p.eps);
-    p.zp[g] = (float)p.qmin - rintf(mn / s);
+    z = (float)p.qmin - rintf(mn / s);
+    p.zp[g] = z;
   } else {
     s = fmaxf(mx / (float)p.qmax, p.eps);
   }
@@ -314,32 +326,21 @@ __global__ __launch_bounds__(256) void finalize_tiled_kernel(GenParams p, int Z,
   rinv[g] = 1.0f / s;
   // x/s == RN(q0 + (x - q0*s)*r) with q0 = RN(x*r), r = RN(1/s), for every finite x unless the
   // significand of s is all ones or the residual can underflow
-  plain[g] = (s > 0x1p-96f && s < 0x1p96f && (f2u(s) & 0x7fffffu) != 0x7fffffu) ? 1u : 0u;
+  // (nor may the zero-point be too large for the rounding trick of FastOctet)
+  plain[g] = (s > 0x1p-96f && s < 0x1p96f && (f2u(s) & 0x7fffffu) != 0x7fffffu && fabsf(z) <= 0x1p21f) ? 1u : 0u;
 }
 
-// Quantizes and stores one octet (column `col`) of row `row`: s, r, z the scale, RN(1 / scale) and the
-// zero-point of the octet's groups (one per channel or one), plain whether all scales allow the exact
-// quotient shortcut.
+// Quantizes and stores one octet (column `col`) of row `row`: s, z the scale and the zero-point of the octet's groups (one per channel or one).
 // also(codes): what else the caller wants from them.
 struct Nothing { __device__ __forceinline__ void operator()(const int (&)[8]) const {} };
 template <int NV, class F = Nothing>
-__device__ __forceinline__ void store_octet(const GenParams &p, int64_t row, int col, const float (&v)[8], const float (&s)[NV], const float (&r)[NV],
-                                            const float (&z)[NV], bool plain, F &&also = F()) {
+__device__ __forceinline__ void store_octet(const GenParams &p, int64_t row, int col, const float (&v)[8], const float (&s)[NV],
+                                            const float (&z)[NV], F &&also = F()) {
   const float qmin = (float)p.qmin, qmax = (float)p.qmax;
   const u32 mask = (1u << p.bits) - 1u;
   int q[8];
-  if (plain) {
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      const float sj = s[j % NV], rj = r[j % NV];
-      const float q0 = v[j] * rj;
-      const float t = __builtin_fmaf(__builtin_fmaf(-q0, sj, v[j]), rj, q0);
-      q[j] = (int)__builtin_amdgcn_fmed3f(rintf(t) + z[j % NV], qmin, qmax);
-    }
-  } else {
-#pragma unroll
-    for (int j = 0; j < 8; ++j) q[j] = (int)__builtin_amdgcn_fmed3f(rintf(v[j] / s[j % NV]) + z[j % NV], qmin, qmax);
-  }
+  for (int j = 0; j < 8; ++j) q[j] = (int)__builtin_amdgcn_fmed3f(rintf(v[j] / s[j % NV]) + z[j % NV], qmin, qmax);
   also(q);
   const int64_t orow = out_row32(p, row);
   if (p.codes || p.bits == 8) {
@@ -361,20 +362,72 @@ __device__ __forceinline__ void store_octet(const GenParams &p, int64_t row, int
   }
 }
 
-// (Its own copy of the arithmetic of store_octet, and p.asym at run time: with a row's octet in every lane and one load in
-// flight the kernel is nearly as much bound by its instructions as by its bytes, and the shared form has more branches
-// per octet.  [32,30,680,64] affine 2 bits, four inputs in turn, three runs: 21.5-22.2 us through store_octet,
-// 21.1-21.4 like this; store_octet with these branches in it 22.3-23.8.)
-template <int DT, bool KEEPC>
+// The groups of one octet (one per channel or one) where all scales allow the exact quotient shortcut and the zero-points are
+// below 2^21: clamp(rint(t) + z, qmin, qmax) = rint(clamp(t, qmin - z, qmax - z)) + z, adding 1.5 * 2^23 rounds to nearest-even and leaves
+// the integer in the low bits, four of them are a dword of bytes, and the zero-points are added to its bytes at once.  About eight
+// instructions per element with the conversion; store_octet takes twelve, and the quantizing kernels are bound by their number as
+// much as by the bytes.
+template <int NV, bool ASYM> struct FastOctet {
+  float s[NV], r[NV], lo[NV], span, hi;
+  u32 zw[ASYM ? 2 : 1];   // zero-points, one byte per channel
+  __device__ __forceinline__ FastOctet(const GenParams &p, const float (&s_)[NV], const float (&r_)[NV], const float (&z)[NV]) {
+    span = (float)(p.qmax - p.qmin); hi = (float)p.qmax;
+#pragma unroll
+    for (int j = 0; j < NV; ++j) { s[j] = s_[j]; r[j] = r_[j]; lo[j] = ASYM ? (float)p.qmin - z[j] : (float)p.qmin; }
+    if constexpr (ASYM) {
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        zw[h] = 0;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) zw[h] |= ((u32)(int)z[(4 * h + j) % NV] & 0xffu) << (8 * j);
+      }
+    }
+  }
+  // number(j): the code of v[j] less its zero-point, in the low bits of a float of 1.5 * 2^23
+  __device__ __forceinline__ float number(float x, int j) const {
+    const int n = j % NV;
+    const float q0 = x * r[n];
+    const float t = __builtin_fmaf(__builtin_fmaf(-q0, s[n], x), r[n], q0);
+    return __builtin_amdgcn_fmed3f(t, lo[n], ASYM ? lo[n] + span : hi) + 12582912.f;
+  }
+  __device__ __forceinline__ u32 bytes(const float (&u)[8], int h) const {
+    const u32 a = __builtin_amdgcn_perm(f2u(u[4 * h + 1]), f2u(u[4 * h]), 0x0c0c0400u), b = __builtin_amdgcn_perm(f2u(u[4 * h + 3]), f2u(u[4 * h + 2]), 0x0c0c0400u);
+    const u32 w = __builtin_amdgcn_perm(b, a, 0x05040100u);
+    if constexpr (ASYM) return ((w & 0x7f7f7f7fu) + (zw[h] & 0x7f7f7f7fu)) ^ ((w ^ zw[h]) & 0x80808080u);
+    else return w;
+  }
+  // Quantizes and stores an octet; also(u): what else the caller wants from its numbers.
+  template <class F> __device__ __forceinline__ void store(const GenParams &p, int64_t orow, int col, const float (&v)[8], F &&also) const {
+    float u[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) u[j] = number(v[j], j);
+    also(u);
+    const u32 lo8 = bytes(u, 0), hi8 = bytes(u, 1);
+    if (p.codes) *reinterpret_cast<uint2 *>(p.codes + (orow * p.c8 + col) * 8) = make_uint2(lo8, hi8);
+    if (!p.words) return;
+    if (p.bits == 8) {
+      *reinterpret_cast<uint2 *>(p.words + orow * p.wpr + col * 2) = make_uint2(lo8, hi8);
+    } else if (p.bits == 4) {
+      const u32 a = lo8 & 0x0f0f0f0fu, b = hi8 & 0x0f0f0f0fu;
+      p.words[orow * p.wpr + col] = (int32_t)__builtin_amdgcn_perm(b | b >> 4, a | a >> 4, 0x06040200u);
+    } else {  // 2 bits: 16 codes per word = two adjacent octets (c % 16 == 0 on this path), the partner lane's in the upper half
+      auto four = [](u32 w) { w &= 0x03030303u; w |= w >> 6; return (w & 0xfu) | (w >> 12 & 0xf0u); };
+      const u32 w = four(lo8) | four(hi8) << 8;
+      const u32 other = (u32)__builtin_amdgcn_update_dpp(0, (int)w, 0xB1, 0xf, 0xf, false);
+      if ((col & 1) == 0) p.words[orow * p.wpr + (col >> 1)] = (int32_t)(w | (other << 16));
+    }
+  }
+};
+
+template <int DT, bool ASYM, bool KEEPC>
 __global__ __launch_bounds__(256) void quant_tiled_kernel(GenParams p, Plan pl, const float *rinv, const u32 *plain) {
   constexpr int NV = KEEPC ? 8 : 1;
   if (take_second(p)) { rinv += p.ws1; plain += p.ws1; }
   const Lane l = decode(pl);
-  // 2-bit words are assembled from two adjacent column lanes: idle lanes must still reach the shuffle
-  const bool live = l.live;
-  const int64_t g = (int64_t)l.ko * pl.ko_gs + (int64_t)(live ? l.q : 0) * pl.q_gs + (KEEPC ? (live ? l.col : 0) * 8 : 0);
-  float s[NV], r[NV], z[NV];
-  bool all_plain = true;
+  if (!l.live) return;   // (only the 2-bit path exchanges between lanes, and there c8 is even: partners are live together)
+  const int64_t g = (int64_t)l.ko * pl.ko_gs + (int64_t)l.q * pl.q_gs + (KEEPC ? l.col * 8 : 0);
+  float s[NV], r[NV], z[NV] = {};
+  bool fast = true;
   if constexpr (KEEPC) {
     // the lane's eight groups are adjacent and start at a multiple of 8: 16-byte loads (the
     // workspace and the outputs are 16-byte aligned; checked on the host)
@@ -384,61 +437,21 @@ __global__ __launch_bounds__(256) void quant_tiled_kernel(GenParams p, Plan pl, 
     };
     ld8(p.scale, s);
     ld8(rinv, r);
-    if (p.asym) ld8(p.zp, z);
-    else {
-#pragma unroll
-      for (int j = 0; j < NV; ++j) z[j] = 0.f;
-    }
+    if (ASYM) ld8(p.zp, z);
     const uint4 pa = reinterpret_cast<const uint4 *>(plain + g)[0], pb = reinterpret_cast<const uint4 *>(plain + g)[1];
-    all_plain = (pa.x & pa.y & pa.z & pa.w & pb.x & pb.y & pb.z & pb.w) != 0u;
+    fast = (pa.x & pa.y & pa.z & pa.w & pb.x & pb.y & pb.z & pb.w) != 0u;
   } else {
     s[0] = p.scale[g];
     r[0] = rinv[g];
-    z[0] = p.asym ? p.zp[g] : 0.f;
-    all_plain = plain[g] != 0u;
+    if (ASYM) z[0] = p.zp[g];
+    fast = plain[g] != 0u;
   }
-  const float qmin = (float)p.qmin, qmax = (float)p.qmax;
-  const u32 mask = (1u << p.bits) - 1u;
-  if (!live) return;   // (only the 2-bit path shuffles, and there c8 is even: partners are live together)
-  for_rows<DT>(p, pl, l, [&](int64_t row, const float (&v)[8]) {
-    int q[8];
-    if (all_plain) {
-#pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        const float sj = s[j % NV], rj = r[j % NV];
-        const float q0 = v[j] * rj;
-        const float t = __builtin_fmaf(__builtin_fmaf(-q0, sj, v[j]), rj, q0);
-        q[j] = (int)__builtin_amdgcn_fmed3f(rintf(t) + z[j % NV], qmin, qmax);
-      }
-    } else {
-#pragma unroll
-      for (int j = 0; j < 8; ++j) q[j] = (int)__builtin_amdgcn_fmed3f(rintf(v[j] / s[j % NV]) + z[j % NV], qmin, qmax);
-    }
-    const int64_t orow = out_row32(p, row);
-    const int64_t o = orow * p.c8 + l.col;
-    if (p.codes) {
-      u32 lo = (q[0] & 0xff) | ((q[1] & 0xff) << 8) | ((q[2] & 0xff) << 16) | ((u32)q[3] << 24);
-      u32 hi = (q[4] & 0xff) | ((q[5] & 0xff) << 8) | ((q[6] & 0xff) << 16) | ((u32)q[7] << 24);
-      *reinterpret_cast<uint2 *>(p.codes + o * 8) = make_uint2(lo, hi);
-    }
-    if (p.words) {
-      if (p.bits == 8) {
-        u32 lo = (q[0] & 0xff) | ((q[1] & 0xff) << 8) | ((q[2] & 0xff) << 16) | ((u32)q[3] << 24);
-        u32 hi = (q[4] & 0xff) | ((q[5] & 0xff) << 8) | ((q[6] & 0xff) << 16) | ((u32)q[7] << 24);
-        *reinterpret_cast<uint2 *>(p.words + orow * p.wpr + l.col * 2) = make_uint2(lo, hi);
-      } else {
-        u32 w = 0;
-#pragma unroll
-        for (int j = 0; j < 8; ++j) w |= ((u32)q[j] & mask) << (j * p.bits);
-        if (p.bits == 4) {
-          p.words[orow * p.wpr + l.col] = (int32_t)w;
-        } else {  // 2 bits: 16 codes per word = two adjacent octets (c % 16 == 0 on this path)
-          u32 other = __shfl_xor(w, 1, 64);
-          if ((l.col & 1) == 0) p.words[orow * p.wpr + (l.col >> 1)] = (int32_t)(w | (other << 16));
-        }
-      }
-    }
-  });
+  if (!__any(!fast)) {
+    const FastOctet<NV, ASYM> o(p, s, r, z);
+    for_rows<DT>(p, pl, l, [&](u32 row, const float (&v)[8]) { o.store(p, out_row32(p, row), l.col, v, [](const float (&)[8]) {}); });
+  } else {
+    for_rows<DT>(p, pl, l, [&](u32 row, const float (&v)[8]) { store_octet<NV>(p, row, l.col, v, s, z); });
+  }
 }
 
 // ---- one launch: a workgroup holds all rows of its groups -----------------------------------------
@@ -449,19 +462,24 @@ __global__ __launch_bounds__(256) void quant_tiled_kernel(GenParams p, Plan pl, 
 // three launches -> one: n = 1 12.7 -> 4.4 us / 9.9 -> 4.7, n = 16 11.8 -> 8.6 / 9.9 -> 4.6, n = 64 22.7 ->
 // 14.7, n = 400 14.3 -> 9.9, n = 1024 22.6 -> 16.5.
 // A workgroup owns, for one ko, 2^lq_shift kept inner indices x c8s column lanes; thread
-// ((lq * sub + f) * c8s + col) takes the reduced rows f, f + sub, ... of its q.  With the channel dim kept
+// ((lq * sub + f) * c8s + col) takes the reduced rows f, f + sub, ... of its q.  A row is straight-line code, once per held row and pass: what it
+// costs are its instructions, issued and fetched.  With two divisions of 64-bit rows, the conversion to integers and
+// the division's own path in every row, 45 KB for 16 rows, and that kernel for four rows as well, the launches of fp16 [64,n,16,64]
+// took 13.1 us (n = 9), 15.3 (25), 13.1 (36) and 20.6 (64); now 6.8, 10.2, 11.8 and 18.6; with the dequantized cache, [8,n,30,64] to
+// fp32, 11.4 -> 7.8 (n = 25), 12.4 -> 10.3 (64), 21.5 -> 19.3 (256).  With the channel dim kept
 // the columns are cut into slices of c8s octets, one workgroup each, until there are workgroups enough: the
 // steps of one batch have few groups, and narrow slices (64, 32, then 16 bytes of a row, whose cache lines
 // the slices of one XCD share) still read faster than few workgroups do.
 struct OnePlan {
   int64_t ko_rs, ro_rs, ko_gs, q_gs;
   int nko, Q, RR, RI;           // kept outer, kept inner; reduced rows, of which RI are contiguous
+  FastDiv by_RI;
   int c8s_shift, sub_shift, lq_shift;
   int slices, tilesQ, steps;
   int blocks;                   // nko * tilesQ
 };
 
-// also(row, col, codes, scales, zero-points): what else is made of an octet once it is quantized
+// also(row, col, codes less their zero-points, scales): what else is made of an octet once it is quantized
 template <int DT, bool ASYM, bool KEEPC, int NT, int NI, class F>
 __device__ __forceinline__ void quant_one_block(const GenParams &p, const OnePlan &pl, F &&also) {
   constexpr int NV = KEEPC ? 8 : 1, MAXG = 2048;
@@ -477,15 +495,20 @@ __device__ __forceinline__ void quant_one_block(const GenParams &p, const OnePla
   const int lcol = tid & (c8s - 1), col = slice * c8s + lcol, f = (tid >> pl.c8s_shift) & (sub - 1), lq = tid >> (pl.c8s_shift + pl.sub_shift);
   const int q = (tq << pl.lq_shift) + lq;
   const bool live = col < p.c8 && q < pl.Q && lq < (1 << pl.lq_shift);
-  const int64_t row0 = (int64_t)ko * pl.ko_rs + (live ? q : 0);
-  auto row_of = [&](int j) { return pl.RI == 1 ? row0 + j * pl.ro_rs : row0 + (j / pl.RI) * pl.ro_rs + j % pl.RI; };
+  // (the tensor is at most 16 MiB, so rows and byte offsets fit 32 bits)
+  const u32 row0 = (u32)ko * (u32)pl.ko_rs + (live ? q : 0);
+  auto row_of = [&](int j) {
+    const u32 o = pl.by_RI((u32)j);
+    return row0 + o * (u32)pl.ro_rs + ((u32)j - o * (u32)pl.RI);
+  };
+  auto octet_at = [&](u32 row) { return reinterpret_cast<const Raw8<DT> *>(reinterpret_cast<const char *>(p.x) + (row * (u32)p.c + col * 8) * (u32)In8<DT>::kBytes); };
 
   Raw8<DT> raw[NI];
 #pragma unroll
   for (int s = 0; s < NI; ++s) {
     const int j = (s << pl.sub_shift) + f;
     if (s < pl.steps && live && j < pl.RR)
-      raw[s] = *reinterpret_cast<const Raw8<DT> *>(reinterpret_cast<const char *>(p.x) + (row_of(j) * p.c + col * 8) * In8<DT>::kBytes);
+      raw[s] = *octet_at(row_of(j));
   }
   float mx[NV], mn[NV];
 #pragma unroll
@@ -542,7 +565,7 @@ __device__ __forceinline__ void quant_one_block(const GenParams &p, const OnePla
     }
     par_s[t] = s;
     // (the exact-quotient shortcut, see finalize_tiled_kernel; 0: this group takes the division)
-    par_r[t] = (s > 0x1p-96f && s < 0x1p96f && (f2u(s) & 0x7fffffu) != 0x7fffffu) ? 1.0f / s : 0.f;
+    par_r[t] = (s > 0x1p-96f && s < 0x1p96f && (f2u(s) & 0x7fffffu) != 0x7fffffu && fabsf(zp) <= 0x1p21f) ? 1.0f / s : 0.f;
     if (mine) {
       const int64_t g = (int64_t)ko * pl.ko_gs + (int64_t)tqi * pl.q_gs + (KEEPC ? slice * c8s * 8 + g8 : 0);
       p.scale[g] = s;
@@ -561,20 +584,41 @@ __device__ __forceinline__ void quant_one_block(const GenParams &p, const OnePla
     if (ASYM) z[j] = par_z[t0 + j];
     plain = plain && r[j] != 0.f;
   }
+  if (__any(!plain)) {   // (rare, and once in the code: the rows are read again)
+    for (int j = f; j < pl.RR; j += sub) {
+      const u32 row = row_of(j);
+      float v[8];
+      octet_at(row)->widen(v);
+      store_octet<NV>(p, row, col, v, s, z, [&](const int (&codes)[8]) {
+        float x[8];
+#pragma unroll
+        for (int k = 0; k < 8; ++k) x[k] = ASYM ? (float)codes[k] - z[k % NV] : (float)codes[k];
+        also(row, col, x, s);
+      });
+    }
+    return;
+  }
+  const FastOctet<NV, ASYM> o(p, s, r, z);
 #pragma unroll
   for (int i = 0; i < NI; ++i) {
     const int j = (i << pl.sub_shift) + f;
     if (i >= pl.steps || j >= pl.RR) continue;
     float v[8];
     raw[i].widen(v);
-    const int64_t row = row_of(j);
-    store_octet<NV>(p, row, col, v, s, r, z, plain, [&](const int (&codes)[8]) { also(row, col, codes, s, z); });
+    const u32 row = row_of(j);
+    o.store(p, out_row32(p, row), col, v, [&](const float (&u)[8]) {
+      float x[8];
+#pragma unroll
+      for (int k = 0; k < 8; ++k) x[k] = u[k] - 12582912.f;
+      also(row, col, x, s);
+    });
+    __builtin_amdgcn_sched_barrier(0);   // (rows started ahead of their turn cost registers that the held ones need)
   }
 }
 template <int DT, bool ASYM, bool KEEPC, int NT, int NI>
 __global__ __launch_bounds__(NT) void quant_one_kernel(GenParams p, OnePlan pl) {
   take_second(p);
-  quant_one_block<DT, ASYM, KEEPC, NT, NI>(p, pl, [](int64_t, int, const auto &, const auto &, const auto &) {});
+  quant_one_block<DT, ASYM, KEEPC, NT, NI>(p, pl, [](u32, int, const auto &, const auto &) {});
 }
 
 // A step of a quantizer with a scale per (head, channel), and the whole cache dequantized behind it, in one launch:
@@ -585,31 +629,25 @@ __global__ __launch_bounds__(NT) void quant_one_kernel(GenParams p, OnePlan pl) 
 struct StepOut {
   StepParams earlier;             // the tokens before this step (none: nseg = 0)
   int64_t inner, delta, off;      // input row r is output row r + r / inner * delta + off
+  FastDiv by_inner;
   int odt, q_blocks, pair_blocks; // workgroups that quantize; workgroups of a pair of `earlier`
 };
-template <int DT, bool ASYM, int NT, int NI>
+template <int DT, bool ASYM, int ODT, int NT, int NI>
 __global__ __launch_bounds__(NT) void quant_one_step_kernel(GenParams p, OnePlan pl, StepOut o) {
-  auto typed = [&](auto &&f) __attribute__((always_inline)) {
-    if (o.odt == VARQ_F32) f(std::integral_constant<int, VARQ_F32>{});
-    else if (o.odt == VARQ_BF16) f(std::integral_constant<int, VARQ_BF16>{});
-    else f(std::integral_constant<int, VARQ_F16>{});
-  };
   if ((int)blockIdx.x >= o.q_blocks) {
+    constexpr int U = kStepOctets / NT;
     const int b = blockIdx.x - o.q_blocks, pair = b / o.pair_blocks, block = b - pair * o.pair_blocks;
-    typed([&](auto t) __attribute__((always_inline)) {
-      constexpr int ODT = decltype(t)::value, U = kStepOctets / NT;
-      if (p.bits == 8) dequant_steps_block<ODT, 8, NT, U>(o.earlier, pair, block);
-      else if (p.bits == 4) dequant_steps_block<ODT, 4, NT, U>(o.earlier, pair, block);
-      else dequant_steps_block<ODT, 2, NT, U>(o.earlier, pair, block);
-    });
+    if (p.bits == 8) dequant_steps_block<ODT, 8, NT, U>(o.earlier, pair, block);
+    else if (p.bits == 4) dequant_steps_block<ODT, 4, NT, U>(o.earlier, pair, block);
+    else dequant_steps_block<ODT, 2, NT, U>(o.earlier, pair, block);
     return;
   }
-  quant_one_block<DT, ASYM, true, NT, NI>(p, pl, [&](int64_t row, int col, const auto &q, const auto &s, const auto &z) __attribute__((always_inline)) {
+  quant_one_block<DT, ASYM, true, NT, NI>(p, pl, [&](u32 row, int col, const auto &x, const auto &s) __attribute__((always_inline)) {
     float f[8];
 #pragma unroll
-    for (int j = 0; j < 8; ++j) f[j] = ASYM ? ((float)q[j] - z[j]) * s[j] : (float)q[j] * s[j];
-    const int64_t orow = row + (int64_t)((u32)row / (u32)o.inner) * o.delta + o.off;
-    typed([&](auto t) __attribute__((always_inline)) { store8<decltype(t)::value>(o.earlier.out, orow * p.c + col * 8, f, 8); });
+    for (int j = 0; j < 8; ++j) f[j] = x[j] * s[j];
+    const int64_t orow = row + (int64_t)o.by_inner(row) * o.delta + o.off;
+    store8<ODT>(o.earlier.out, orow * p.c + col * 8, f, 8);
   });
 }
 
@@ -774,7 +812,7 @@ bool make_one_plan(const int64_t *sh, int reduce_mask, int row_steps, int tensor
   int c8p_shift = 0;
   while ((1 << c8p_shift) < c8) ++c8p_shift;
   pl.ko_rs = k.ko_rs; pl.ro_rs = k.ro_rs; pl.ko_gs = k.ko_gs; pl.q_gs = k.q_gs;
-  pl.nko = (int)k.nko; pl.Q = (int)k.Q; pl.RR = (int)rr; pl.RI = (int)k.RI;
+  pl.nko = (int)k.nko; pl.Q = (int)k.Q; pl.RR = (int)rr; pl.RI = (int)k.RI; pl.by_RI = FastDiv::by(k.RI);
   int rr_shift = 0;
   while ((1 << rr_shift) < rr) ++rr_shift;
   // column slices (channel dim kept): whole rows while that makes workgroups enough, 64 bytes of a row at least
@@ -814,20 +852,33 @@ template <int DT, bool ASYM, bool KEEPC>
 void launch_one(const GenParams &p, const OnePlan &pl, int threads, hipStream_t st) {
   constexpr int NI = DT == VARQ_F32 ? 8 : 16;
   dim3 grid((unsigned)((pl.blocks + 7) / 8 * 8 * pl.slices), p.x1 ? 2u : 1u);
-  if (threads == 1024) hipLaunchKernelGGL((quant_one_kernel<DT, ASYM, KEEPC, 1024, NI>), grid, dim3(1024), 0, st, p, pl);
+  // (256 threads have at most four steps, see make_one_plan; a kernel for more has their code and registers)
+  if (threads == 1024 && pl.steps > 4) hipLaunchKernelGGL((quant_one_kernel<DT, ASYM, KEEPC, 1024, NI>), grid, dim3(1024), 0, st, p, pl);
+  else if (threads == 1024) hipLaunchKernelGGL((quant_one_kernel<DT, ASYM, KEEPC, 1024, 4>), grid, dim3(1024), 0, st, p, pl);
   else if (pl.steps <= 2) hipLaunchKernelGGL((quant_one_kernel<DT, ASYM, KEEPC, 256, 2>), grid, dim3(256), 0, st, p, pl);
-  else hipLaunchKernelGGL((quant_one_kernel<DT, ASYM, KEEPC, 256, NI>), grid, dim3(256), 0, st, p, pl);
+  else hipLaunchKernelGGL((quant_one_kernel<DT, ASYM, KEEPC, 256, 4>), grid, dim3(256), 0, st, p, pl);
 }
 template <int DT> void run_one(const GenParams &p, const OnePlan &pl, int threads, hipStream_t st) {
   if (p.asym) { if (p.keepc) launch_one<DT, true, true>(p, pl, threads, st); else launch_one<DT, true, false>(p, pl, threads, st); }
   else { if (p.keepc) launch_one<DT, false, true>(p, pl, threads, st); else launch_one<DT, false, false>(p, pl, threads, st); }
 }
 
-template <int DT, bool ASYM> void launch_one_step(const GenParams &p, const OnePlan &pl, int threads, const StepOut &o, unsigned blocks, hipStream_t st) {
+template <int DT, bool ASYM, int ODT> void launch_one_step(const GenParams &p, const OnePlan &pl, int threads, const StepOut &o, unsigned blocks, hipStream_t st) {
   constexpr int NI = DT == VARQ_F32 ? 8 : 16;
-  if (threads == 1024) hipLaunchKernelGGL((quant_one_step_kernel<DT, ASYM, 1024, NI>), dim3(blocks), dim3(1024), 0, st, p, pl, o);
-  else if (pl.steps <= 2) hipLaunchKernelGGL((quant_one_step_kernel<DT, ASYM, 256, 2>), dim3(blocks), dim3(256), 0, st, p, pl, o);
-  else hipLaunchKernelGGL((quant_one_step_kernel<DT, ASYM, 256, NI>), dim3(blocks), dim3(256), 0, st, p, pl, o);
+  if (threads == 1024 && pl.steps > 4) hipLaunchKernelGGL((quant_one_step_kernel<DT, ASYM, ODT, 1024, NI>), dim3(blocks), dim3(1024), 0, st, p, pl, o);
+  else if (threads == 1024) hipLaunchKernelGGL((quant_one_step_kernel<DT, ASYM, ODT, 1024, 4>), dim3(blocks), dim3(1024), 0, st, p, pl, o);
+  else if (pl.steps <= 2) hipLaunchKernelGGL((quant_one_step_kernel<DT, ASYM, ODT, 256, 2>), dim3(blocks), dim3(256), 0, st, p, pl, o);
+  else hipLaunchKernelGGL((quant_one_step_kernel<DT, ASYM, ODT, 256, 4>), dim3(blocks), dim3(256), 0, st, p, pl, o);
+}
+template <int DT> void run_one_step(const GenParams &p, const OnePlan &pl, int threads, const StepOut &o, unsigned blocks, hipStream_t st) {
+  auto typed = [&](auto odt) {
+    constexpr int ODT = decltype(odt)::value;
+    if (p.asym) launch_one_step<DT, true, ODT>(p, pl, threads, o, blocks, st);
+    else launch_one_step<DT, false, ODT>(p, pl, threads, o, blocks, st);
+  };
+  if (o.odt == VARQ_F32) typed(std::integral_constant<int, VARQ_F32>{});
+  else if (o.odt == VARQ_BF16) typed(std::integral_constant<int, VARQ_BF16>{});
+  else typed(std::integral_constant<int, VARQ_F16>{});
 }
 
 size_t plan_workspace_bytes(const Plan &pl, int64_t n_groups) {
@@ -863,8 +914,13 @@ int run_tiled(GenParams &p, const Plan &pl, void *workspace, hipStream_t st) {
   // per thread measured alike, longer ones slower)
   const Plan &pb = pl;
   dim3 bgrid((unsigned)((int64_t)pb.nko * pb.tilesQ * pb.Z), nt);
-  if (p.keepc) hipLaunchKernelGGL((quant_tiled_kernel<DT, true>), bgrid, dim3(256), 0, st, p, pb, rinv, plain);
-  else hipLaunchKernelGGL((quant_tiled_kernel<DT, false>), bgrid, dim3(256), 0, st, p, pb, rinv, plain);
+  if (p.asym) {
+    if (p.keepc) hipLaunchKernelGGL((quant_tiled_kernel<DT, true, true>), bgrid, dim3(256), 0, st, p, pb, rinv, plain);
+    else hipLaunchKernelGGL((quant_tiled_kernel<DT, true, false>), bgrid, dim3(256), 0, st, p, pb, rinv, plain);
+  } else {
+    if (p.keepc) hipLaunchKernelGGL((quant_tiled_kernel<DT, false, true>), bgrid, dim3(256), 0, st, p, pb, rinv, plain);
+    else hipLaunchKernelGGL((quant_tiled_kernel<DT, false, false>), bgrid, dim3(256), 0, st, p, pb, rinv, plain);
+  }
   return 0;
 }
 
@@ -962,6 +1018,7 @@ int quant_pack_impl(const void *x, const void *x1, int x_dtype, const int64_t *h
                    (long long)host_out_map[0], (long long)host_out_map[1], (long long)host_out_map[2], (long long)rows);
     p.out_mapped = 1; p.out_inner = host_out_map[0]; p.out_delta = host_out_map[1]; p.out_off = host_out_map[2];
   }
+  p.by_inner = FastDiv::by(p.out_inner);
   p.n0 = s[0]; p.n1 = s[1]; p.n2 = s[2];
   p.c = (int)s[3];
   p.keepc = !(reduce_mask & 8);
@@ -991,9 +1048,9 @@ int quant_pack_impl(const void *x, const void *x1, int x_dtype, const int64_t *h
       const int64_t blocks = step->q_blocks + step_pairs * step->pair_blocks;
       if (blocks < (1ll << 31)) {
         const unsigned n = (unsigned)blocks;
-        if (x_dtype == VARQ_F32) { if (asym) launch_one_step<VARQ_F32, true>(p, one, threads, *step, n, st); else launch_one_step<VARQ_F32, false>(p, one, threads, *step, n, st); }
-        else if (x_dtype == VARQ_BF16) { if (asym) launch_one_step<VARQ_BF16, true>(p, one, threads, *step, n, st); else launch_one_step<VARQ_BF16, false>(p, one, threads, *step, n, st); }
-        else { if (asym) launch_one_step<VARQ_F16, true>(p, one, threads, *step, n, st); else launch_one_step<VARQ_F16, false>(p, one, threads, *step, n, st); }
+        if (x_dtype == VARQ_F32) run_one_step<VARQ_F32>(p, one, threads, *step, n, st);
+        else if (x_dtype == VARQ_BF16) run_one_step<VARQ_BF16>(p, one, threads, *step, n, st);
+        else run_one_step<VARQ_F16>(p, one, threads, *step, n, st);
         VARQ_CHECK_LAUNCH("quant_step_dequant");
         step->q_blocks = -1;   // done
         return VARQ_OK;
@@ -1065,7 +1122,7 @@ extern "C" int varq_quant_step_dequant(const void *x, int x_dtype, int B, int H,
   set_steps(o.earlier, words, scale, asym ? zp : nullptr, nseg - 1, host_seg_end, B, H, capacity, c, bits, tokens_first, out);
   const bool fits = pairs * start * o.earlier.octs <= (asym ? kStepMostAsym : kStepMostSym);
   o.earlier.out_pair_octs = tokens * o.earlier.octs;
-  o.inner = map[0]; o.delta = (tokens - n) * per; o.off = map[2];
+  o.inner = map[0]; o.by_inner = FastDiv::by(map[0]); o.delta = (tokens - n) * per; o.off = map[2];
   o.odt = out_dtype; o.q_blocks = 0; o.pair_blocks = 0;
   float *const s = scale + (nseg - 1) * row, *const z = asym ? zp + (nseg - 1) * row : nullptr;
   if (const int e = quant_pack_impl(x, nullptr, x_dtype, shape, tokens_first ? 0b0011 : 0b0101, bits, asym, eps, words, nullptr, s, z, nullptr, nullptr,
