@@ -167,6 +167,18 @@ int varq_quant_pack2(const void *x0, const void *x1, int x_dtype, const int64_t 
                      const int64_t *host_out_map, void *workspace, size_t workspace_bytes, void *stream);
 
 /*
+ * varq_quant_pack / varq_quant_pack2 (x1 != NULL) of groups that take in whole rows (reduce bit 3 set), with the scale of a group
+ * written to every place that reads it -- the tokens, heads and batch entries that it serves -- instead of once: what a
+ * cache of scales per token, or of one table per step, holds after the reference's expand and concatenation (VAR_Q/quant.py:196-201).
+ * host_scale_map {gi, go, ge, off, r_in, r_out, s_out}: the scale (and zero-point) of group g, numbered as varq_quant_pack
+ * writes them, goes to elements (g / gi) go + (g % gi) ge + off + i + o s_out for i < r_in, o < r_out.  One launch, no workspace;
+ * VARQ_ERR_UNSUPPORTED, and nothing done, for tensors that varq_quant_pack quantizes in several.
+ */
+int varq_quant_pack_spread(const void *x0, const void *x1, int x_dtype, const int64_t *host_shape4, int reduce_mask, int bits, int asym,
+                           float eps, int32_t *words0, float *scale0, float *zp0, int32_t *words1, float *scale1, float *zp1,
+                           const int64_t *host_out_map, const int64_t *host_scale_map, void *stream);
+
+/*
  * varq_quant_pack for callers that cannot allocate device memory (code under HIP graph
  * capture, tight serving loops, harnesses that forbid hipMalloc).  It has no counterpart
  * in the reference.  Same arguments and results as varq_quant_pack, without a workspace:

@@ -9,6 +9,8 @@
 // VarqError for tensors off the GPU and for statuses of the library.
 #include <Python.h>
 
+#include <optional>
+
 #include <ATen/core/Tensor.h>
 #include <ATen/ops/empty.h>
 #include <c10/core/DeviceGuard.h>
@@ -179,6 +181,16 @@ PyObject *quant_shared(PyObject *const *a) {
   return triple(q, scale, zp);
 }
 
+// x and, in the same launches, x1 (or null), which is like it
+int pack_rows(const at::Tensor &x, const void *x1, int dt, const int64_t *sh, int mask, int bits, bool asym, float eps, int32_t *w0, int32_t *w1,
+              float *const *s, float *const *z, const int64_t *map) {
+  const size_t one = std::max<size_t>(varq_quant_workspace_bytes(sh, mask), 8), ws_bytes = x1 ? 2 * one : one;
+  const at::Tensor ws = empty({(int64_t)ws_bytes}, at::kByte, x);
+  if (x1)
+    return varq_quant_pack2(x.data_ptr(), x1, dt, sh, mask, bits, asym, eps, w0, nullptr, s[0], z[0], w1, nullptr, s[1], z[1], map, ws.data_ptr(), ws_bytes, stream_of(x));
+  return varq_quant_pack(x.data_ptr(), dt, sh, mask, bits, asym, eps, w0, nullptr, s[0], z[0], map, ws.data_ptr(), ws_bytes, stream_of(x));
+}
+
 // One step of a quantizer with a scale per (head, channel): codes into tokens start.. of the cache
 // buffer, scale and zero-point into row k of the step tables.
 // quant_step(mask, bits, asym, eps, token_dim, start, k, x, buf, tab, ztab | None [, x1, buf1, tab1, ztab1])
@@ -210,52 +222,15 @@ PyObject *quant_step(PyObject *const *a, Py_ssize_t n_args) {
   const c10::DeviceGuard guard(t.device());
   const int dt = dtype_code(t);
   const float eps = (float)real(a[3]);
-  float *s[2], *z[2];
+  float *s[2] = {}, *z[2] = {};
   for (int i = 0; i < (two ? 2 : 1); ++i) {
     s[i] = ptr<float>(tab[i]) + k * row;
     z[i] = asym ? ptr<float>(ztab[i]) + k * row : nullptr;
   }
-  unlocked(two ? "varq_quant_pack2" : "varq_quant_pack", [&] {
-    const size_t one = std::max<size_t>(varq_quant_workspace_bytes(sh, mask), 8), ws_bytes = two ? 2 * one : one;
-    const at::Tensor ws = empty({(int64_t)ws_bytes}, at::kByte, t);
-    if (two)
-      return varq_quant_pack2(x[0]->data_ptr(), x[1]->data_ptr(), dt, sh, mask, (int)bits, asym, eps, ptr<int32_t>(buf[0]), nullptr, s[0], z[0],
-                              ptr<int32_t>(buf[1]), nullptr, s[1], z[1], map, ws.data_ptr(), ws_bytes, stream_of(t));
-    return varq_quant_pack(x[0]->data_ptr(), dt, sh, mask, (int)bits, asym, eps, ptr<int32_t>(buf[0]), nullptr, s[0], z[0], map, ws.data_ptr(),
-                           ws_bytes, stream_of(t));
+  unlocked("varq_quant_pack", [&] {
+    return pack_rows(t, two ? x[1]->data_ptr() : nullptr, dt, sh, mask, (int)bits, asym, eps, ptr<int32_t>(buf[0]), two ? ptr<int32_t>(buf[1]) : nullptr, s, z, map);
   });
   Py_RETURN_NONE;
-}
-
-// quant_step_dequant(asym, bits, eps, token_dim, x, buf, tab, ztab | None, earlier seg_ends, out dtype code)
-// -> the dequantized cache; the step goes behind the earlier ones, its scales into the next row of the tables.
-PyObject *quant_step_dequant(PyObject *const *a) {
-  const bool asym = truth(a[0]);
-  const int64_t bits = integer(a[1]), d = integer(a[3]), code = integer(a[9]);
-  const at::Tensor &x = gpu(a[4], "x"), &buf = gpu(a[5], "buffer"), &tab = gpu(a[6], "scale table");
-  const at::Tensor *ztab = maybe(a[7], "zero-point table");
-  ASSERT(PyList_Check(a[8]) && PyList_GET_SIZE(a[8]) < 16 && (d == 1 || d == 2), "quant_step_dequant: 1..16 steps");
-  const int k = (int)PyList_GET_SIZE(a[8]);
-  int32_t ends[16];
-  for (int i = 0; i < k; ++i) ends[i] = (int32_t)integer(PyList_GET_ITEM(a[8], i));
-  ASSERT(x.dim() == 4 && x.is_contiguous() && buf.dim() == 4 && buf.is_contiguous() && buf.scalar_type() == at::kInt && tab.is_contiguous(), "quant_step_dequant: operands");
-  const int64_t B = x.size(0), H = x.size(3 - d), n = x.size(d), c = x.size(3), start = k ? ends[k - 1] : 0;
-  ends[k] = (int32_t)(start + n);
-  ASSERT((!asym || ztab) && buf.size(3) * 32 == c * bits && start + n <= buf.size(d) && buf.size(0) == B && buf.size(3 - d) == H, "quant_step_dequant: buffers");
-  ASSERT((k + 1) * H * c <= tab.numel() && tab.scalar_type() == at::kFloat && (!ztab || ztab->sizes() == tab.sizes()), "quant_step_dequant: tables");
-  const int64_t sh[4] = {B, x.size(1), x.size(2), c};
-  const c10::DeviceGuard guard(x.device());
-  const int dt = dtype_code(x);
-  const float eps = (float)real(a[2]);
-  at::Tensor out;
-  unlocked("varq_quant_step_dequant", [&] {
-    const size_t ws_bytes = std::max<size_t>(varq_quant_workspace_bytes(sh, d == 1 ? 0b0011 : 0b0101), 8);
-    const at::Tensor ws = empty({(int64_t)ws_bytes}, at::kByte, x);
-    out = d == 1 ? empty({B, start + n, H, c}, dtype_of((int)code), x) : empty({B, H, start + n, c}, dtype_of((int)code), x);
-    return varq_quant_step_dequant(x.data_ptr(), dt, (int)B, (int)H, (int)n, (int)c, d == 1, (int)bits, asym, eps, ptr<int32_t>(buf), buf.size(d), ptr<float>(tab),
-                                   asym ? ptr<float>(ztab) : nullptr, k + 1, ends, out.data_ptr(), (int)code, ws.data_ptr(), ws_bytes, stream_of(x));
-  });
-  return wrap(out);
 }
 
 // ---- pack / unpack of int8 codes ----------------------------------------------------------------
@@ -791,6 +766,233 @@ PyObject *cache_prepare(PyObject *const *a) {
   return wrap(q);
 }
 
+// ---- drop-in quantizers -------------------------------------------------------------------------
+// A step of VAR_Q (quant.py) and the attention over two of them, with their state read from and left in the Python objects'
+// attributes: what quant() followed by cache() leaves.  Anything out of the ordinary -- other rules, no room yet, a tensor of
+// another kind -- is refused with nothing done, and the Python methods take the call.
+enum class Rule { kHeadDim, kScale, kHead, kToken, kTokenHead, kOtherTable, kOtherToken, kNone };
+Rule rule_of(PyObject *m) {
+  const std::pair<PyObject *, Rule> rules[] = {{NAME(G_SCALE_HEAD_DIM), Rule::kHeadDim}, {NAME(G_SCALE), Rule::kScale}, {NAME(G_HEAD), Rule::kHead},
+                                               {NAME(G_TOKEN), Rule::kToken}, {NAME(G_TOKEN_HEAD), Rule::kTokenHead}, {NAME(G_HEAD_DIM), Rule::kOtherTable},
+                                               {NAME(G_TENSOR), Rule::kOtherTable}, {NAME(G_GROUP), Rule::kOtherToken}};
+  for (const auto &[name, rule] : rules)
+    if (m == name) return rule;
+  for (const auto &[name, rule] : rules)
+    if (PyUnicode_Check(m) && PyUnicode_Compare(m, name) == 0) return rule;
+  return Rule::kNone;
+}
+bool per_token(Rule r) { return r == Rule::kToken || r == Rule::kTokenHead || r == Rule::kOtherToken; }
+void set_attribute(PyObject *o, PyObject *name, PyObject *v) {   // (takes the reference)
+  const Ref value(v);
+  if (PyObject_SetAttr(o, name, v)) throw python_error();
+}
+int64_t number_of(PyObject *o, PyObject *name) { return integer(Ref(attribute(o, name)).o); }
+
+// a dense GPU tensor of that type in attribute `name`, or an empty place
+bool tensor_of(Held &h, PyObject *o, PyObject *name, at::ScalarType dt) {
+  PyObject *const v = attribute(o, name);
+  if (THPVariable_Check(v)) {
+    const at::Tensor &t = THPVariable_Unpack(v);
+    if (t.is_cuda() && t.scalar_type() == dt && t.is_contiguous()) {
+      h.o = v;
+      h.t = &t;
+      return true;
+    }
+  }
+  Py_DECREF(v);
+  return false;
+}
+
+struct Quantizer {
+  PyObject *const o;
+  Rule rule;
+  int64_t bits, d, k = 0, len, c;      // token dim, cached steps, cached tokens, channels
+  bool asym, packed;
+  Held buf, scale, zp;                 // codes; the step tables or the scales per token
+  Ref item, ends;
+  Held tok, tokz;                      // (the growable buffers of the scales per token, as objects)
+  bool ready = false;                  // everything above is there, and of the kinds that the kernels read
+
+  explicit Quantizer(PyObject *obj)
+      : o(obj), rule(rule_of(Ref(attribute(obj, NAME(quant_method))).o)), bits(number_of(obj, NAME(quant_bits))), d(number_of(obj, NAME(dim_cat))),
+        asym(!truth(Ref(attribute(obj, NAME(symmetric))).o)), packed(truth(Ref(attribute(obj, NAME(pack_to_int32))).o)),
+        item(attribute(obj, NAME(_c_item))), ends(attribute(obj, NAME(_seg_ends))) {
+    if (rule == Rule::kNone || !packed || (bits != 2 && bits != 4 && bits != 8) || (d != 1 && d != 2) || !PyList_Check(ends.o)) return;
+    len = number_of(item.o, NAME(len));
+    if (number_of(item.o, NAME(dim)) != d || !tensor_of(buf, item.o, NAME(buf), at::kInt) || buf->dim() != 4) return;
+    const Ref meta(attribute(o, NAME(_pack_meta)));
+    if (!PyDict_Check(meta.o)) return;
+    PyObject *const oc = PyDict_GetItem(meta.o, NAME(orig_c)), *const ob = PyDict_GetItem(meta.o, NAME(bits));
+    if (!oc || !ob || integer(ob) != bits) return;
+    c = integer(oc);
+    if (buf->size(3) * 32 != c * bits) return;
+    k = PyList_GET_SIZE(ends.o);
+    if (per_token(rule)) {
+      tok.o = attribute(o, NAME(_tok_scale));
+      tokz.o = attribute(o, NAME(_tok_zp));
+      if (number_of(tok.o, NAME(dim)) != d || number_of(tok.o, NAME(len)) != len || !tensor_of(scale, tok.o, NAME(buf), at::kFloat) || scale->dim() != 4) return;
+      if (asym ? number_of(tokz.o, NAME(len)) != len || !tensor_of(zp, tokz.o, NAME(buf), at::kFloat) || zp->sizes() != scale->sizes()
+               : Ref(attribute(tokz.o, NAME(buf))).o != Py_None)
+        return;
+      if (scale->size(0) != buf->size(0) || scale->size(1) != buf->size(1) || scale->size(2) != buf->size(2)) return;
+    } else {
+      if (!tensor_of(scale, o, NAME(_tab_scale), at::kFloat) || scale->dim() != 3 || scale->size(1) != buf->size(3 - d) || scale->size(2) != c) return;
+      if (asym ? !tensor_of(zp, o, NAME(_tab_zp), at::kFloat) || zp->sizes() != scale->sizes() : Ref(attribute(o, NAME(_tab_zp))).o != Py_None) return;
+    }
+    ready = len >= 0 && len <= buf->size(d);
+  }
+  int64_t heads() const { return buf->size(3 - d); }
+  int64_t last_end() const { return k ? integer(PyList_GET_ITEM(ends.o, k - 1)) : 0; }
+
+  // whether a step can go behind the cached ones as it is
+  bool takes(PyObject *x) const {
+    if (!ready || rule == Rule::kOtherTable || rule == Rule::kOtherToken || !THPVariable_Check(x)) return false;
+    const at::Tensor &t = THPVariable_Unpack(x);
+    if (!t.is_cuda() || t.device() != buf->device() || t.dim() != 4 || !t.is_contiguous() || t.numel() == 0 || c % 8 != 0) return false;
+    if (t.scalar_type() != at::kFloat && t.scalar_type() != at::kBFloat16 && t.scalar_type() != at::kHalf) return false;
+    if (t.size(0) != buf->size(0) || t.size(3 - d) != heads() || t.size(3) != c || len + t.size(d) > buf->size(d)) return false;
+    return per_token(rule) ? scale->size(3) == 1 : k < 16 && k < scale->size(0);
+  }
+  int mask() const {   // the dims that the rule reduces (VAR_Q/quant.py:78-95)
+    switch (rule) {
+      case Rule::kHeadDim: return d == 1 ? 0b0011 : 0b0101;
+      case Rule::kScale: return 0b1111;
+      case Rule::kHead: return d == 1 ? 0b1011 : 0b1101;
+      case Rule::kToken: return d == 1 ? 0b1101 : 0b1011;
+      default: return 0b1001;
+    }
+  }
+  // Where the scales of a step of n tokens go (see varq_quant_pack_spread): into the step's row of the tables, or to its tokens
+  // of the scales per token, [B, H, cap, 1] or [B, cap, H, 1], of every batch entry (and head).
+  void spread(int64_t n, int64_t (&m)[7]) const {
+    const int64_t B = buf->size(0), H = heads(), cap = buf->size(d);
+    auto set = [&](int64_t gi, int64_t go, int64_t ge, int64_t off, int64_t r_in, int64_t r_out, int64_t s_out) {
+      const int64_t v[7] = {gi, go, ge, off, r_in, r_out, s_out};
+      std::copy(v, v + 7, m);
+    };
+    if (rule == Rule::kScale) set(1, 0, 0, k * H * c, H * c, 1, 0);
+    else if (rule == Rule::kHead) set(1, c, 0, k * H * c, c, 1, 0);
+    else if (rule == Rule::kTokenHead) {
+      if (d == 2) set(n, cap, 1, len, 1, B, H * cap);
+      else set(1, 1, 0, len * H, 1, B, cap * H);
+    } else if (d == 2) set(1, 1, 0, len, 1, B * H, cap);
+    else set(1, H, 0, len * H, H, B, cap * H);
+  }
+  // the state that quant() followed by cache() leaves, the kernels having written codes and scales in place
+  void commit(int64_t n) const {
+    const int64_t H = heads(), s1 = d == 1 ? n : H, s2 = d == 1 ? H : n;
+    const bool tokens = per_token(rule);
+    const int64_t shape[4] = {1, rule == Rule::kTokenHead || (tokens && d == 1) || (!tokens && d == 2 && rule != Rule::kScale) ? s1 : 1,
+                              rule == Rule::kTokenHead || (tokens && d == 2) || (!tokens && d == 1 && rule != Rule::kScale) ? s2 : 1,
+                              rule == Rule::kHeadDim ? c : 1};
+    const Ref sshape(Py_BuildValue("(LLLL)", (long long)shape[0], (long long)shape[1], (long long)shape[2], (long long)shape[3]));
+    set_attribute(o, NAME(_window), Py_BuildValue("(OLLLOOLO)", buf.o, (long long)d, (long long)len, (long long)n, scale.o, asym ? zp.o : Py_None,
+                                                  (long long)(tokens ? -1 : k), sshape.o));
+    Py_INCREF(Py_None);
+    set_attribute(o, NAME(_staged), Py_None);
+    Py_INCREF(sshape.o);
+    set_attribute(o, NAME(_scale_shape), sshape.o);
+    set_attribute(item.o, NAME(len), PyLong_FromLongLong(len + n));
+    if (tokens) {
+      set_attribute(tok.o, NAME(len), PyLong_FromLongLong(len + n));
+      if (asym) set_attribute(tokz.o, NAME(len), PyLong_FromLongLong(len + n));
+    } else {
+      const Ref end(PyLong_FromLongLong(last_end() + n));
+      if (PyList_Append(ends.o, end.o)) throw python_error();
+    }
+  }
+};
+
+// quantizer_step(k_quant, k, v_quant | None, v | None) -> whether the step was taken: quant and cache, K and V of a step in the same launches.
+// One call with the scales written where the cache keeps them took a step of the rules with scales per token from 72 us of host work
+// (two quantizers: reductions, expand, copies into the growing buffers) to that of the shipped rule.
+PyObject *quantizer_step(PyObject *const *a) {
+  const bool two = a[2] != Py_None;
+  const Quantizer kq(a[0]);
+  if (!kq.takes(a[1])) Py_RETURN_FALSE;
+  std::optional<Quantizer> vq;
+  const at::Tensor &k = THPVariable_Unpack(a[1]);
+  const double eps = real(Ref(attribute(a[0], NAME(eps))).o);
+  if (two) {
+    vq.emplace(a[2]);
+    if (a[0] == a[2] || !vq->takes(a[3])) Py_RETURN_FALSE;
+    const at::Tensor &v = THPVariable_Unpack(a[3]);
+    // (one window of two buffers, one row of two tables)
+    if (kq.rule != vq->rule || kq.bits != vq->bits || kq.asym != vq->asym || kq.d != vq->d || kq.len != vq->len || kq.k != vq->k || v.sizes() != k.sizes() ||
+        v.scalar_type() != k.scalar_type() || v.device() != k.device() || kq.buf->sizes() != vq->buf->sizes() || eps != real(Ref(attribute(a[2], NAME(eps))).o))
+      Py_RETURN_FALSE;
+  }
+  const int64_t sh[4] = {k.size(0), k.size(1), k.size(2), k.size(3)}, d = kq.d, n = sh[d], per_tok = d == 1 ? sh[2] : 1, row = kq.k * kq.heads() * kq.c;
+  const int64_t map[3] = {n * per_tok, (kq.buf->size(d) - n) * per_tok, kq.len * per_tok};
+  const c10::DeviceGuard guard(k.device());
+  const int dt = dtype_code(k), mask = kq.mask(), bits = (int)kq.bits;
+  const bool asym = kq.asym, rows = kq.rule == Rule::kHeadDim;
+  auto at_row = [&](const Held &h) { return h.t ? ptr<float>(h) + (rows ? row : 0) : nullptr; };
+  const void *const x1 = two ? THPVariable_Unpack(a[3]).data_ptr() : nullptr;
+  int32_t *const w0 = ptr<int32_t>(kq.buf), *const w1 = two ? ptr<int32_t>(vq->buf) : nullptr;
+  float *const s[2] = {at_row(kq.scale), two ? at_row(vq->scale) : nullptr}, *const z[2] = {at_row(kq.zp), two ? at_row(vq->zp) : nullptr};
+  int64_t spread[7];
+  if (!rows) kq.spread(n, spread);
+  const int rc = status_unlocked([&] {
+    if (rows) return pack_rows(k, x1, dt, sh, mask, bits, asym, (float)eps, w0, w1, s, z, map);
+    return varq_quant_pack_spread(k.data_ptr(), x1, dt, sh, mask, bits, asym, (float)eps, w0, s[0], z[0], w1, s[1], z[1], map, spread, stream_of(k));
+  });
+  if (!rows && rc == VARQ_ERR_UNSUPPORTED) Py_RETURN_FALSE;
+  check(rc, "varq_quant_pack");
+  kq.commit(n);
+  if (two) vq->commit(n);
+  Py_RETURN_TRUE;
+}
+
+// quantizer_use(quantizer, x, out dtype code) -> the dequantized cache with the step behind the earlier ones (the shipped rule), or None
+PyObject *quantizer_use(PyObject *const *a) {
+  const Quantizer z(a[0]);
+  if (z.rule != Rule::kHeadDim || !z.takes(a[1]) || z.last_end() != z.len) Py_RETURN_NONE;
+  const at::Tensor &x = THPVariable_Unpack(a[1]);
+  const int64_t d = z.d, n = x.size(d), B = x.size(0), H = z.heads(), c = z.c, code = integer(a[2]);
+  if ((uintptr_t)x.data_ptr() & 15 || (z.len + n) * (d == 1 ? H : 1) * (c / 8) >= (1ll << 31) - 2048) Py_RETURN_NONE;
+  int32_t ends[16];
+  for (int i = 0; i < z.k; ++i) ends[i] = (int32_t)integer(PyList_GET_ITEM(z.ends.o, i));
+  ends[z.k] = (int32_t)(z.len + n);
+  const int64_t sh[4] = {B, x.size(1), x.size(2), c};
+  const float eps = (float)real(Ref(attribute(a[0], NAME(eps))).o);
+  const c10::DeviceGuard guard(x.device());
+  const int dt = dtype_code(x);
+  at::Tensor out;
+  unlocked("varq_quant_step_dequant", [&] {
+    const size_t ws_bytes = std::max<size_t>(varq_quant_workspace_bytes(sh, z.mask()), 8);
+    const at::Tensor ws = empty({(int64_t)ws_bytes}, at::kByte, x);
+    out = d == 1 ? empty({B, z.len + n, H, c}, dtype_of((int)code), x) : empty({B, H, z.len + n, c}, dtype_of((int)code), x);
+    return varq_quant_step_dequant(x.data_ptr(), dt, (int)B, (int)H, (int)n, (int)c, d == 1, (int)z.bits, z.asym, eps, ptr<int32_t>(z.buf), z.buf->size(d),
+                                   ptr<float>(z.scale), ptr<float>(z.zp), (int)z.k + 1, ends, out.data_ptr(), (int)code, ws.data_ptr(), ws_bytes, stream_of(x));
+  });
+  z.commit(n);
+  return wrap(out);
+}
+
+// quantizer_attend(q, k_quant, v_quant, softmax_scale, kv_limit, out) -> out, or None where fused_attention has to look closer
+PyObject *quantizer_attend(PyObject *const *a) {
+  const Quantizer k(a[1]), v(a[2]);
+  if (!k.ready || !v.ready || k.len == 0 || k.d != v.d || k.bits != v.bits || k.len != v.len || k.c != v.c || (k.c != 64 && k.c != 128) || per_token(k.rule) != per_token(v.rule) ||
+      k.buf->sizes() != v.buf->sizes() || !THPVariable_Check(a[0]))
+    Py_RETURN_NONE;
+  const at::Tensor &q = THPVariable_Unpack(a[0]);
+  if (!q.is_cuda() || q.dim() != 4 || !q.is_contiguous() || !((q.scalar_type() == at::kHalf && k.c == 64) || q.scalar_type() == at::kBFloat16) ||
+      q.size(0) != k.buf->size(0) || q.size(3 - k.d) != k.heads() || q.size(3) != k.c)
+    Py_RETURN_NONE;
+  const Ref bits(PyLong_FromLongLong(k.bits)), len(PyLong_FromLongLong(k.len)), zero(PyLong_FromLong(0));
+  PyObject *const kz = k.asym ? k.zp.o : Py_None, *const vz = v.asym ? v.zp.o : Py_None, *const layout = k.d == 1 ? NAME(BLHc) : NAME(BHLc);
+  if (per_token(k.rule)) {
+    PyObject *const args[18] = {a[0], k.buf.o, k.scale.o, kz, v.buf.o, v.scale.o, vz, bits.o, bits.o, len.o, a[3], a[4], Py_None, a[5], zero.o, layout, Py_False, Py_None};
+    return attn(args);
+  }
+  const int same = PyObject_RichCompareBool(k.ends.o, v.ends.o, Py_EQ);
+  if (same < 0) throw python_error();
+  if (!same || k.k == 0 || k.k > 16 || k.last_end() != k.len) Py_RETURN_NONE;
+  PyObject *const args[17] = {a[0], k.buf.o, k.scale.o, kz, v.buf.o, v.scale.o, vz, bits.o, len.o, a[3], a[4], Py_None, a[5], k.ends.o, zero.o, layout, Py_None};
+  return attn_channel(args);
+}
+
 // ---- module -------------------------------------------------------------------------------------
 template <PyObject *(*F)(PyObject *const *), int N> PyObject *fixed(PyObject *, PyObject *const *a, Py_ssize_t n) {
   HANDLE_TH_ERRORS
@@ -812,9 +1014,10 @@ PyObject *set_error(PyObject *, PyObject *e) {
 
 #define FIXED(name, n) {#name, (PyCFunction)(void (*)(void))fixed<name, n>, METH_FASTCALL, nullptr}
 PyMethodDef g_methods[] = {
-    FIXED(quant_rows, 5), FIXED(quant_shared, 6), FIXED(pack, 2), FIXED(unpack, 3), FIXED(dequant, 6), FIXED(dequant_steps, 8), FIXED(quant_step_dequant, 10), FIXED(attn, 18), FIXED(attn_channel, 17),
+    FIXED(quant_rows, 5), FIXED(quant_shared, 6), FIXED(pack, 2), FIXED(unpack, 3), FIXED(dequant, 6), FIXED(dequant_steps, 8), FIXED(attn, 18), FIXED(attn_channel, 17),
     FIXED(cache_attend, 9), FIXED(cache_append, 5), FIXED(cache_prepare, 9),
     {"quant_step", (PyCFunction)(void (*)(void))varying<quant_step>, METH_FASTCALL, nullptr},
+    FIXED(quantizer_step, 4), FIXED(quantizer_use, 3), FIXED(quantizer_attend, 6),
     {"set_error", set_error, METH_O, nullptr},
     {nullptr, nullptr, 0, nullptr}};
 PyModuleDef g_module = {PyModuleDef_HEAD_INIT, "_host", nullptr, -1, g_methods, nullptr, nullptr, nullptr, nullptr};

@@ -11,6 +11,7 @@
 // in which partial results meet.  Channel counts that are not a multiple of 8 and
 // rows wider than 512 channels take scalar kernels with ordered-integer atomics.
 #include "dequant_steps.h"
+#include <algorithm>
 #include <mutex>
 #include <type_traits>
 
@@ -61,6 +62,15 @@ struct FastDiv {
   __device__ __forceinline__ u32 operator()(u32 n) const { return (__umulhi(n, mul) + (n & all)) >> shift; }
 };
 
+// Where the scale of group g goes when it is written once per token that it serves (and the zero-point like it): elements
+// (g / gi) go + (g % gi) ge + off + i + o * s_out, i < r_in, o < r_out.
+struct Spread {
+  int on;
+  FastDiv by_gi, by_in;
+  u32 gi, r_in, reps;        // reps = r_in * r_out
+  int64_t go, ge, off, s_out;
+};
+
 struct GenParams {
   const void *x;
   u32 *ws_max;   // [n_groups] encoded max (or max-abs)
@@ -84,6 +94,7 @@ struct GenParams {
   int out_mapped;
   int64_t out_inner, out_delta, out_off;
   FastDiv by_inner;
+  Spread spread;
   // a second tensor of the same shape in the same launches (blockIdx.y == 1): its input,
   // its outputs and the distance (in 4-byte words) to its part of the workspace
   const void *x1;
@@ -566,13 +577,27 @@ __device__ __forceinline__ void quant_one_block(const GenParams &p, const OnePla
     par_s[t] = s;
     // (the exact-quotient shortcut, see finalize_tiled_kernel; 0: this group takes the division)
     par_r[t] = (s > 0x1p-96f && s < 0x1p96f && (f2u(s) & 0x7fffffu) != 0x7fffffu && fabsf(zp) <= 0x1p21f) ? 1.0f / s : 0.f;
-    if (mine) {
+    if (mine && (KEEPC || !p.spread.on)) {
       const int64_t g = (int64_t)ko * pl.ko_gs + (int64_t)tqi * pl.q_gs + (KEEPC ? slice * c8s * 8 + g8 : 0);
       p.scale[g] = s;
       if (ASYM) p.zp[g] = zp;
     }
   }
   __syncthreads();
+  if constexpr (!KEEPC) {
+    if (p.spread.on) {
+      // all threads, the groups of the workgroup fastest (n_par, one per q, is a power of two)
+      for (u32 i = tid; i < (u32)n_par * p.spread.reps; i += NT) {
+        const int t = i & (n_par - 1), tqi = (tq << pl.lq_shift) + t;
+        const u32 rep = i >> pl.lq_shift, o = p.spread.by_in(rep);
+        if (tqi >= pl.Q) continue;
+        const u32 g = (u32)(ko * pl.ko_gs + tqi * pl.q_gs), a = p.spread.by_gi(g);
+        const int64_t at = a * p.spread.go + (int64_t)(g - a * p.spread.gi) * p.spread.ge + p.spread.off + (rep - o * p.spread.r_in) + o * p.spread.s_out;
+        p.scale[at] = par_s[t];
+        if (ASYM) p.zp[at] = par_z[t];
+      }
+    }
+  }
   if (!live) return;   // (2-bit words take two adjacent columns, which are live together: c is a multiple of 16 there)
   const int t0 = lq * gcols + lcol * (KEEPC ? 8 : 0);
   float s[NV], r[NV], z[NV] = {};
@@ -974,7 +999,7 @@ int quant_pack_impl(const void *x, const void *x1, int x_dtype, const int64_t *h
                     int asym, float eps, int32_t *words, int8_t *codes, float *scale, float *zp,
                     int32_t *words1, int8_t *codes1, float *scale1, float *zp1,
                     const int64_t *host_out_map, void *workspace, size_t workspace_bytes, void *stream,
-                    StepOut *step = nullptr, int64_t step_pairs = 0) {
+                    StepOut *step = nullptr, int64_t step_pairs = 0, const int64_t *host_scale_map = nullptr) {
   VARQ_CHECK_ARG(host_shape4, "quant_pack: null shape");
   const int64_t *s = host_shape4;
   VARQ_CHECK_ARG(s[0] >= 0 && s[1] >= 0 && s[2] >= 0 && s[3] > 0 && s[3] <= (1 << 20), "quant_pack: bad shape");
@@ -986,7 +1011,7 @@ int quant_pack_impl(const void *x, const void *x1, int x_dtype, const int64_t *h
   if (rows == 0) return VARQ_OK;
   VARQ_CHECK_ARG(words || codes, "quant_pack: no output requested");
   VARQ_CHECK_ARG(scale && (!asym || zp), "quant_pack: scale/zp output missing");
-  VARQ_CHECK_ARG(x && workspace, "quant_pack: null pointer");
+  VARQ_CHECK_ARG(x && (workspace || host_scale_map), "quant_pack: null pointer");
   if (x1) {
     VARQ_CHECK_ARG((!words == !words1) && (!codes == !codes1) && scale1 && (!asym || zp1),
                    "quant_pack: the second tensor needs the same kinds of output as the first");
@@ -996,7 +1021,7 @@ int quant_pack_impl(const void *x, const void *x1, int x_dtype, const int64_t *h
   // the tiled kernels pack whole words per octet: c*bits must fill words (always true for 4 and 8 bits)
   const bool tiled = make_plan(s, reduce_mask, ng, pl) && (!words || (s[3] * bits) % 32 == 0);
   const size_t need = tiled ? plan_workspace_bytes(pl, ng) * (x1 ? 2 : 1) : (size_t)ng * 2 * sizeof(u32);
-  if (workspace_bytes < need)
+  if (workspace_bytes < need && !host_scale_map)
     return varq_set_error(VARQ_ERR_WORKSPACE, "quant_pack: workspace %zu < %zu bytes", workspace_bytes, need);
   VARQ_CHECK_ARG(rows * s[3] < (1ll << 40), "quant_pack: tensor too large");
   // only the tiled kernels that keep the channel dim move scales, zero-points and partials in
@@ -1019,6 +1044,14 @@ int quant_pack_impl(const void *x, const void *x1, int x_dtype, const int64_t *h
     p.out_mapped = 1; p.out_inner = host_out_map[0]; p.out_delta = host_out_map[1]; p.out_off = host_out_map[2];
   }
   p.by_inner = FastDiv::by(p.out_inner);
+  p.spread.on = 0;
+  if (const int64_t *m = host_scale_map) {
+    VARQ_CHECK_ARG(m[0] > 0 && m[4] > 0 && m[5] > 0 && (reduce_mask & 8), "quant_pack: scales of whole rows can be spread, over at least one place each");
+    // (places counted in 32 bits, times the 512 groups that a workgroup has at most)
+    if (m[4] > (1 << 22) || m[4] * m[5] > (1 << 22))
+      return varq_set_error(VARQ_ERR_UNSUPPORTED, "quant_pack: scales are spread over at most 4 million places each");
+    p.spread = {1, FastDiv::by(m[0]), FastDiv::by(m[4]), (u32)std::min(m[0], (int64_t)0x7fffffff), (u32)m[4], (u32)(m[4] * m[5]), m[1], m[2], m[3], m[6]};
+  }
   p.n0 = s[0]; p.n1 = s[1]; p.n2 = s[2];
   p.c = (int)s[3];
   p.keepc = !(reduce_mask & 8);
@@ -1060,6 +1093,8 @@ int quant_pack_impl(const void *x, const void *x1, int x_dtype, const int64_t *h
     if (x_dtype == VARQ_F32) run_one<VARQ_F32>(p, one, threads, st);
     else if (x_dtype == VARQ_BF16) run_one<VARQ_BF16>(p, one, threads, st);
     else run_one<VARQ_F16>(p, one, threads, st);
+  } else if (host_scale_map) {
+    return varq_set_error(VARQ_ERR_UNSUPPORTED, "quant_pack: spread scales come with groups that one launch quantizes");
   } else if (tiled) {
     if (x1) { p.x1 = x1; p.scale1 = scale1; p.zp1 = zp1; p.words1 = words1; p.codes1 = codes1; }
     if (x_dtype == VARQ_F32) run_tiled<VARQ_F32>(p, pl, workspace, st);
@@ -1096,6 +1131,14 @@ extern "C" int varq_quant_pack2(const void *x0, const void *x1, int x_dtype, con
   VARQ_CHECK_ARG(x1, "quant_pack2: null second tensor");
   return quant_pack_impl(x0, x1, x_dtype, host_shape4, reduce_mask, bits, asym, eps, words0, codes0, scale0, zp0,
                          words1, codes1, scale1, zp1, host_out_map, workspace, workspace_bytes, stream);
+}
+
+extern "C" int varq_quant_pack_spread(const void *x0, const void *x1, int x_dtype, const int64_t *host_shape4, int reduce_mask, int bits, int asym,
+                                      float eps, int32_t *words0, float *scale0, float *zp0, int32_t *words1, float *scale1, float *zp1,
+                                      const int64_t *host_out_map, const int64_t *host_scale_map, void *stream) {
+  VARQ_CHECK_ARG(host_scale_map, "quant_pack_spread: null scale map");
+  return quant_pack_impl(x0, x1, x_dtype, host_shape4, reduce_mask, bits, asym, eps, words0, nullptr, scale0, zp0, words1, nullptr, scale1, zp1,
+                         host_out_map, nullptr, 0, stream, nullptr, 0, host_scale_map);
 }
 
 // Quantizes a step into its tokens of the cache buffer and dequantizes the whole cache: in one launch where the step

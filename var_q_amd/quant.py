@@ -143,8 +143,13 @@ class VAR_Q:
         w = self._window
         if w is not None:
             self._window = None
-            buf, dim, start, n, srow, zrow, sshape = w
-            self._current = [buf.narrow(dim, start, n), srow.view(sshape), None if zrow is None else zrow.view(sshape)]
+            buf, dim, start, n, scales, zps, k, shape = w
+            self._current = [buf.narrow(dim, start, n)]
+            for t in (scales, zps):
+                if t is not None:            # the step's row of the tables, or its tokens of the scales per token
+                    t = t.narrow(dim, start, n) if k < 0 else t[k].unsqueeze(0).unsqueeze(dim)
+                    t = t[tuple(slice(m) for m in shape)]
+                self._current.append(t)
         return self._current
 
     @property
@@ -309,85 +314,50 @@ class VAR_Q:
             self._pack_meta = meta
         self._window, self._current = None, [q, s, z]
 
-    def _fast_place(self, x: torch.Tensor):
-        """Where the one-call step (see `_step_fast`) puts a step of the shipped rule: (tokens, heads,
-        channels, table row, first token), room in the cache buffer and the tables made; nothing
-        launched, no step added.  None when the quantizer or the item is of another kind."""
+    def _make_room(self, x: torch.Tensor) -> bool:
+        """Room for a step of the shipped rule in the cache buffer and the step tables, as quant() and cache() make it;
+        nothing launched, no step added.  False when the quantizer or the item is of another kind."""
         bits = self.quant_bits
         if self.quant_method != 'G_SCALE_HEAD_DIM' or not self.pack_to_int32 or bits not in (2, 4, 8):
-            return None
+            return False
         if not isinstance(x, torch.Tensor) or x.dim() != 4 or not x.is_cuda or not x.is_contiguous() or x.dtype not in ops._DT:
-            return None
-        item, d, k = self._c_item, self.dim_cat, len(self._seg_ends)
+            return False
+        item, d = self._c_item, self.dim_cat
         s0, s1, s2, c = x.shape
         vals = 32 // bits
-        if item.dim != d or k >= MAX_TABLE_STEPS or c % vals or s0 * s1 * s2 == 0:
-            return None                       # (quant() says why an empty step is refused)
-        n, H = (s1, s2) if d == 1 else (s2, s1)
+        if item.dim != d or len(self._seg_ends) >= MAX_TABLE_STEPS or c % vals or c % 8 or s0 * s1 * s2 == 0:
+            return False                      # (quant() says why an empty step is refused)
         meta = self._pack_meta
         if meta is None:
             self._pack_meta = {'orig_c': c, 'vals_per_word': vals, 'pad_len': 0, 'bits': bits}
         elif meta['orig_c'] != c or meta['bits'] != bits:
-            return None                       # (quant() raises the reference's assertion for this)
-        buf, start = item.buf, item.len
-        if buf is None or start + n > buf.shape[d] or buf.shape[0] != s0 or buf.shape[3 - d] != H:
-            if item.reserve([s0, s1, s2, c // vals], torch.int32, x.device) is None:
-                return None
-        if self._tab_scale is None or self._tab_scale.shape[1] != H or self._tab_scale.shape[2] != c:
-            self._table_rows(H, c, x.device)
-        return n, H, c, k, start
-
-    def _fast_commit(self, place):
-        """The state that quant() followed by cache() leaves, the kernels having written the codes
-        and the table row in place."""
-        n, H, c, k, start = place
-        item, d = self._c_item, self.dim_cat
-        srow, zrow = self._tab_scale[k], None if self.symmetric else self._tab_zp[k]
-        sshape = (1, H, 1, c) if d == 2 else (1, 1, H, c)
-        self._window = (item.buf, d, start, n, srow, zrow, sshape)
-        self._staged = None
-        if c % 8:
-            self._keep_scales(n, c)
-        self._scale_shape = sshape
-        item.len = start + n
-        ends = self._seg_ends
-        ends.append(ends[-1] + n if ends else n)
+            return False                      # (quant() raises the reference's assertion for this)
+        if item.reserve([s0, s1, s2, c // vals], torch.int32, x.device) is None:
+            return False
+        self._table_rows(x.shape[3 - d], c, x.device)
+        return True
 
     def _step_fast(self, x: torch.Tensor) -> bool:
-        """quant(x) followed by cache() for the shipped rule (G_SCALE_HEAD_DIM, packed codes)
-        with the host work of a generation step cut to one library call: same kernels, same
-        state afterwards.  False (nothing done) when the quantizer or the item is of another
-        kind; the caller then takes the two general calls."""
-        place = self._fast_place(x)
-        if place is None:
-            return False
-        d = self.dim_cat
-        _lib.host().quant_step(0b0011 if d == 1 else 0b0101, self.quant_bits, not self.symmetric, self.eps, d, place[4], place[3],
-                               x, self._c_item.buf, self._tab_scale, self._tab_zp)
-        self._fast_commit(place)
-        return True
+        """quant(x) followed by cache() with the host work of a generation step cut to one native call: same kernels, same
+        state afterwards.  It takes the rules whose codes and scales the kernels can write where the cache keeps them (one
+        scale per (head, channel), per head, per step, per token or per (token, head); packed codes), once there is room:
+        the general methods make it, with the first step and where the buffers have to grow.  False (nothing done) for
+        everything else; the caller then takes the two general calls."""
+        return self._takes_native() and (_lib.host().quantizer_step(self, x, None, None)
+                                         or self._make_room(x) and _lib.host().quantizer_step(self, x, None, None))
+
+    def _takes_native(self) -> bool:
+        # (a subclass may have its own quant() or cache(), which the rules other than the shipped one go through)
+        return self.quant_method == 'G_SCALE_HEAD_DIM' or type(self) is VAR_Q
 
     @staticmethod
     def _step_fast_pair(kq: 'VAR_Q', vq: 'VAR_Q', k: torch.Tensor, v: torch.Tensor) -> bool:
         """`_step_fast` for K and V of a step in the same launches, when the two quantizers are
         configured alike and their caches stand at the same place."""
-        if not (isinstance(k, torch.Tensor) and isinstance(v, torch.Tensor)):
+        if not (kq._takes_native() and vq._takes_native()):
             return False
-        if kq is vq or kq.quant_bits != vq.quant_bits or kq.symmetric != vq.symmetric or kq.eps != vq.eps \
-                or kq._qkv_format != vq._qkv_format or k.shape != v.shape or k.dtype != v.dtype or k.device != v.device:
-            return False
-        pk = kq._fast_place(k)
-        if pk is None:
-            return False
-        pv = vq._fast_place(v)
-        d = kq.dim_cat
-        if pv is None or pk[3:] != pv[3:] or kq._c_item.buf.shape[d] != vq._c_item.buf.shape[d]:   # (same window of the two cache buffers)
-            return False
-        _lib.host().quant_step(0b0011 if d == 1 else 0b0101, kq.quant_bits, not kq.symmetric, kq.eps, d, pk[4], pk[3],
-                               k, kq._c_item.buf, kq._tab_scale, kq._tab_zp, v, vq._c_item.buf, vq._tab_scale, vq._tab_zp)
-        kq._fast_commit(pk)
-        vq._fast_commit(pv)
-        return True
+        step = _lib.host().quantizer_step
+        return step(kq, k, vq, v) or kq is not vq and kq._make_room(k) and vq._make_room(v) and step(kq, k, vq, v)
 
     # ---------------- cache ----------------
     def _expand_scale_like_L(self, q: torch.Tensor, scale: torch.Tensor) -> torch.Tensor:
@@ -519,14 +489,13 @@ class VAR_Q:
         two to four times an unquantized bf16 cache, resident until the quantizer is deleted --
         172 MB per tensor at [2,16,10521,128].  `dequant_all()` itself always recomputes everything."""
         if not self.keep_dequantized:
-            place = self._fast_place(item)
-            if place is not None and place[2] % 8 == 0 and (self._seg_ends[-1] if self._seg_ends else 0) == place[4] and item.data_ptr() % 16 == 0 \
-                    and self._steps_fit(place[4] + place[0], place[1], place[2]):
-                # the shipped rule: step and dequantized cache from one library call (and where the sizes allow, one launch)
-                out = _lib.host().quant_step_dequant(not self.symmetric, self.quant_bits, self.eps, self.dim_cat, item, self._c_item.buf,
-                                                     self._tab_scale, self._tab_zp, self._seg_ends, ops._DT[out_dtype or torch.float32])
-                self._fast_commit(place)
-                return out
+            # the shipped rule: step and dequantized cache from one library call (and where the sizes allow, one launch)
+            use, code = _lib.host().quantizer_use, ops._DT[out_dtype or torch.float32]
+            res = use(self, item, code)
+            if res is None and self.quant_method == 'G_SCALE_HEAD_DIM' and self._make_room(item):
+                res = use(self, item, code)
+            if res is not None:
+                return res
         if not self._step_fast(item):
             self.quant(item)
             self.cache()
@@ -580,6 +549,9 @@ def fused_attention(q: torch.Tensor, k_quant: VAR_Q, v_quant: VAR_Q, softmax_sca
     kernels read is kept current by `cache()`, so a call launches the attention and nothing
     else.  kv_limit: int32 [Lq], query i sees keys j < kv_limit[i].  Returns a tensor of the
     attention's dtype in the shape of q."""
+    res = _lib.host().quantizer_attend(q, k_quant, v_quant, softmax_scale, kv_limit, out)
+    if res is not None:
+        return res
     layout = k_quant._qkv_format
     if v_quant._qkv_format != layout:
         raise ValueError(f'fused_attention: K is cached in layout {layout}, V in {v_quant.qkv_format}')
@@ -625,8 +597,8 @@ def fused_step(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, k_quant: VAR_Q
     """One generation step on the packed caches: quantize and cache the step's K and V with
     their quantizers (`quant` + `cache`, VAR_Q/quant.py:232-235 without the dequantization),
     then `fused_attention` of q over everything cached.  For the shipped rule K and V are
-    quantized by one library call (three launches for both); any other rule goes through the
-    general methods."""
+    quantized by one library call, and likewise for the other rules whose scales the kernels can
+    write where the cache keeps them (see `_step_fast`)."""
     if isinstance(k, torch.Tensor) and isinstance(v, torch.Tensor):
         k, v = k.contiguous(), v.contiguous()      # (views of a qkv projection; the quantizers need dense rows)
     if not VAR_Q._step_fast_pair(k_quant, v_quant, k, v):
