@@ -30,6 +30,13 @@ def _limits(order, Lq, Lk, dev):
     (128, 2, 128, 13, 16, 1290, 2050, 'falling', 'bf16'),   # 26 pairs of a class: two windows, of 21 and 5
     (64, 4, 32, 1, 23, 1550, 2111, 'rising', 'fp16'),
     (64, 4, 64, 1, 13, 6150, 2048, 'rising', 'bf16'),
+    # few pairs: blocks of 128 queries, the last one full, of one query or of 33 and more; one tile of keys, and two with one key in the second
+    (128, 4, 128, 1, 11, 193, 64, 'rising', 'bf16'),
+    (128, 2, 64, 2, 5, 256, 65, 'falling', 'bf16'),
+    (128, 8, 128, 2, 16, 1441, 1441, 'rising', 'bf16'),
+    (64, 4, 32, 1, 16, 680, 680, 'rising', 'fp16'),
+    (64, 8, 64, 1, 13, 225, 193, 'falling', 'bf16'),
+    (64, 2, 64, 3, 10, 257, 129, 'rising', 'fp16'),
 ])
 def test_blocks_that_end_at_different_keys(dev, D, bits, group, B, H, Lq, Lk, order, dtype, layout):
     dt = torch.float16 if dtype == 'fp16' else torch.bfloat16

@@ -149,17 +149,20 @@ void launch_few_classes(const AttnParams &p, int D, const ClassTable &t, int gro
 
 // ---- the wide path (wide_attn.hip): K and V expanded once, then attended by many query blocks ----
 struct WidePlan {
+  int waves;            // wavefronts of a workgroup: 8 (blocks of 256 queries) or 4 (128)
   int n_wgs, rounds;    // workgroups of the attention kernel; blocks that each of them takes whole
   size_t tile_bytes;    // the expanded tiles, at the start of the workspace
   size_t ws_bytes;      // ... and the partial results behind them
 };
+// Whether a launch takes workgroups of four wavefronts.
+bool wide_four(int64_t bh, int Lq, int Lk, int D, int cus, bool limits);
 // share: whether blocks may be shared out; limits: whether the queries have key limits
 WidePlan plan_wide(int64_t bh, int Lq, int Lk, int D, int cus, bool share, bool limits);
 // Expands the packed cache of p (per-key groups of k_group / v_group channels, or the per-channel
 // tables) into `tiles`, pair after pair; with `place`, the pairs of a bit-width class to the places of
 // their heads (p.head_map) among the p.Hq heads of the cache.
 void launch_expand(const AttnParams &p, int D, int bits, int k_group, int v_group, bool chan, char *tiles, hipStream_t st, bool place = false);
-// Attends the expanded tiles at the start of `ws`; p.q_tiles counts blocks of 256 queries.
+// Attends the expanded tiles at the start of `ws`.
 void launch_wide(const AttnParams &p, int D, const WidePlan &plan, char *ws, hipStream_t st);
 
 }  // namespace varq_attn

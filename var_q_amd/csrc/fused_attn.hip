@@ -1562,9 +1562,10 @@ int wide_batch(int B, int Hkv, int Lk, int D) {
 // 288 / 218, 32 x 10521 1303 / 1057.  D=64 gains where the longest query blocks are the whole of the time, up to about
 // a block and a quarter per compute unit, 16 x 2521 72 / 66, 24 x 3256 88 / 80, 16 x 4121 108 / 97, and in long sequences,
 // 32 x 6425 305 / 277, 128 x 6425 1112 / 1060; in between it goes either way, 32 x 3256 94 / 102, 128 x 4121 522 / 528,
-// 320 x 2952 665 / 715, 48 x 5417 321 / 330.
+// 320 x 2952 665 / 715, 48 x 5417 321 / 330.  (Few pairs: wide_four.)
 bool wide_eligible(int B, int Hkv, int Lq, int Lk, int D, bool limits) {
   const int64_t bh = (int64_t)wide_batch(B, Hkv, Lk, D) * Hkv, blocks = bh * ((Lq + 255) / 256);
+  if (bh > 0 && wide_four(bh, Lq, Lk, D, device_cus(), limits)) return true;
   if (limits && D == 64 && Lq < 6144 && blocks > device_cus() * 5 / 4) return false;
   return Lq >= (D == 128 ? 1280 : 1536) && Lk >= 2048 && blocks >= 160 && bh <= 65535;
 }

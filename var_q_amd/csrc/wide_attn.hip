@@ -168,7 +168,23 @@ template <bool F16> __device__ __forceinline__ floatx4_t mfma_16x16x32(u32x4_t a
   }
 }
 
-// Work comes in blocks of 256 queries of one (batch, head), block bh * q_tiles + qt, and is dealt out to
+// A wavefront copies N KiB from global memory (`src`: the lane's 16 bytes of the first) to LDS, from address `dst` on,
+// past the registers.  The compiler does not count these loads: wait_copies<N> waits until at most the N KiB last asked
+// for are under way.
+template <int N> __device__ __forceinline__ void to_lds(const char *src, u32 dst) {
+  static_assert(N == 1 || N == 2 || N == 4, "N");
+  dst = __builtin_amdgcn_readfirstlane(dst);
+  if constexpr (N == 1)
+    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(src), "s"(dst) : "memory");
+  else if constexpr (N == 2)
+    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off\n\tglobal_load_lds_dwordx4 %0, off offset:1024" ::"v"(src), "s"(dst) : "memory");
+  else
+    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off\n\tglobal_load_lds_dwordx4 %0, off offset:1024\n\t"
+                 "global_load_lds_dwordx4 %0, off offset:2048\n\tglobal_load_lds_dwordx4 %0, off offset:3072" ::"v"(src), "s"(dst) : "memory");
+}
+template <int N> __device__ __forceinline__ void wait_copies() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory"); }
+
+// Work comes in blocks of 256 queries (128: see wide_four) of one (batch, head), block bh * q_tiles + qt, and is dealt out to
 // n workgroups in rounds: in each of the first `rounds` rounds workgroup w takes block round * n + w
 // whole; the blocks left over are shared out by the key tile, workgroup w taking units [T w / n, T (w + 1) / n)
 // of their T = blocks * tiles units, and a block that falls on several workgroups is put together
@@ -197,12 +213,18 @@ struct SharedUnits {
 // 2147 / 2123 / 2202; D=64, 32 of 4121 172 / 171 / 145, 128 of 5021 725 / 721 / 669.
 constexpr int kLimitWindow = 128;
 
-// One workgroup = 8 wavefronts = 256 queries of one (batch, head) at a time; a wavefront owns 32 queries
-// (two columns of 16) and walks blocks of 32 keys, transposed: S^T = K Q^T, O^T = V^T P^T.
-template <int D, bool F16>
-__global__ __launch_bounds__(512, 2) void wide_attn_kernel(WideParams e) {
-  constexpr int NT = 512, NF = D / 16, HT = kHalfTile<D>, PIECES = HT / (NT * 16);
-  extern __shared__ __attribute__((aligned(16))) char lds[];   // K slots [3][HT], V slots [3][HT]
+// One workgroup = NW wavefronts = 32 NW queries of one (batch, head) at a time (8; 4: see wide_four); a wavefront owns
+// 32 queries (two columns of 16) and walks blocks of 32 keys, transposed: S^T = K Q^T, O^T = V^T P^T.
+// The tiles go to LDS past the registers: with loads and LDS stores of the wavefront's own, a block of 128 queries took 12 % longer
+// (1024 x 2521, 32 pairs, D=128: 66 -> 57 us; 680 x 680, 128 pairs, D=64: 44 -> 32), and
+// blocks of 256, where two wavefronts of a SIMD cover for one another, 2-3 % (4096 x 10521, 32 pairs, with its quantizer
+// and the expansion 623 -> 607; 13 scales of 128 pairs 4600 -> 4497).  Also measured and the same: operands requested eight fragments
+// ahead, scheduling fences after every fragment, 32x32x16 instructions (2-6 % slower).
+template <int D, bool F16, int NW>
+__global__ __launch_bounds__(NW * 64, NW / 4) void wide_attn_kernel(WideParams e) {
+  constexpr int NT = NW * 64, NF = D / 16, HT = kHalfTile<D>, PIECES = HT / (NT * 16);
+  constexpr int BQ = NW * 32;   // queries of a block
+  extern __shared__ __attribute__((aligned(16))) char lds[];   // K slots [4][HT], V slots [4][HT]
   __shared__ int lds_maxlim;
   const AttnParams &p = e.a;
   const int all_tiles = e.all_tiles, n_wgs = gridDim.x;
@@ -214,7 +236,6 @@ __global__ __launch_bounds__(512, 2) void wide_attn_kernel(WideParams e) {
   const int r16 = lane & 15, quarter = lane >> 4;
   const float scale = p.scale_log2e;
   const char *const frag0 = lds + lane * 16;
-  const u32 my16 = tid * 16;
 
   for (int round = 0; round < e.rounds || unit < unit_end; ++round) {
   int qblock = round * n_wgs + w, tbase = 0, tlast = all_tiles;
@@ -236,7 +257,7 @@ __global__ __launch_bounds__(512, 2) void wide_attn_kernel(WideParams e) {
   }
   const int b = bh / p.Hkv, hs = bh - b * p.Hkv;
   const int hq = p.head_map ? p.head_map[hs] : hs;
-  const int qrow0 = qt * 256 + wave * 32;
+  const int qrow0 = qt * BQ + wave * 32;
   const bool wave_live = qrow0 < p.Lq;   // wave-uniform
   int limit[2], qrow_c[2];
   int maxlim = 0, minlim = p.Lk;
@@ -261,53 +282,43 @@ __global__ __launch_bounds__(512, 2) void wide_attn_kernel(WideParams e) {
   const int n_full = __builtin_amdgcn_readfirstlane(min(max(minlim / BN - tbase, 0), n_tiles));
 
   const char *const src = e.tiles + ((int64_t)bh * all_tiles + tbase) * (2 * HT);
-  u32x4_t kreg[PIECES], vreg[PIECES];
-  auto load_k = [&](int t) __attribute__((always_inline)) {   // (past the end: the last tile again, never used)
-    const char *s = src + (int64_t)min(t, n_tiles - 1) * (2 * HT);
-#pragma unroll
-    for (int i = 0; i < PIECES; ++i) kreg[i] = *reinterpret_cast<const u32x4_t *>(s + i * (NT * 16) + my16);
+  // Tile t of K and of V sits in slot t % 4.  The copies to LDS go past the registers, each wavefront its own stretch of a
+  // tile; their addresses are a scalar and what the lane adds to it.
+  const int my_part = __builtin_amdgcn_readfirstlane(wave * (PIECES * 1024));
+  const u32 my_lds = (u32)(uintptr_t)(__attribute__((address_space(3))) char *)lds + my_part;
+  const char *const my_src = src + my_part + lane * 16;
+  auto copy_k = [&](int t) __attribute__((always_inline)) {   // (past the end: the last tile again, never used)
+    to_lds<PIECES>(my_src + (int64_t)min(t, n_tiles - 1) * (2 * HT), (t & 3) * HT + my_lds);
   };
-  auto load_v = [&](int t) __attribute__((always_inline)) {
-    const char *s = src + (int64_t)min(t, n_tiles - 1) * (2 * HT) + HT;
-#pragma unroll
-    for (int i = 0; i < PIECES; ++i) vreg[i] = *reinterpret_cast<const u32x4_t *>(s + i * (NT * 16) + my16);
-  };
-  auto put_k = [&](int sl) __attribute__((always_inline)) {
-#pragma unroll
-    for (int i = 0; i < PIECES; ++i) *reinterpret_cast<u32x4_t *>(lds + sl * HT + i * (NT * 16) + my16) = kreg[i];
-  };
-  auto put_v = [&](int sl) __attribute__((always_inline)) {
-#pragma unroll
-    for (int i = 0; i < PIECES; ++i) *reinterpret_cast<u32x4_t *>(lds + (3 + sl) * HT + i * (NT * 16) + my16) = vreg[i];
+  auto copy_v = [&](int t) __attribute__((always_inline)) {
+    to_lds<PIECES>(my_src + (int64_t)min(t, n_tiles - 1) * (2 * HT) + HT, (4 + (t & 3)) * HT + my_lds);
   };
 
-  // ---- prologue: K of tiles 0 and 1 and V of tile 0 in LDS, K of tile 2 and V of tile 1 in registers;
+  // ---- prologue: K of tiles 0 and 1 and V of tile 0 in LDS, K of tile 2 and V of tile 1 on their way;
   //      the V slot of "tile -1" holds zeros ----
   u32x4_t qb[2][NF / 2];
   if (n_tiles > 0) {
-    load_k(0); load_v(0);
+    copy_k(0); copy_v(0); copy_k(1);
 #pragma unroll
     for (int n = 0; n < 2; ++n) {
       const __bf16 *qptr = p.q + (b * p.q_bs + hq * p.q_hs + qrow_c[n] * p.q_ts) * D + quarter * 8;
 #pragma unroll
       for (int ch = 0; ch < NF / 2; ++ch) qb[n][ch] = *reinterpret_cast<const u32x4_t *>(qptr + ch * 32);
     }
-    put_k(0); put_v(0);
-    load_k(1);
 #pragma unroll
-    for (int i = 0; i < PIECES; ++i) *reinterpret_cast<u32x4_t *>(lds + 5 * HT + i * (NT * 16) + my16) = u32x4_t{0, 0, 0, 0};
-    put_k(1);
-    load_k(2); load_v(1);
+    for (int i = 0; i < PIECES; ++i) *reinterpret_cast<u32x4_t *>(lds + 7 * HT + i * (NT * 16) + tid * 16) = u32x4_t{0, 0, 0, 0};
+    __builtin_amdgcn_s_waitcnt(0x0f70);   // vmcnt(0)
+    copy_k(2); copy_v(1);
   }
   __syncthreads();
 
   if (!wave_live) {
-    for (int t = 0, s0 = 0, s1 = 1, s2 = 2; t < n_tiles; ++t) {
-      put_k(s2); put_v(s1);
-      load_k(t + 3); load_v(t + 2);
+    for (int t = 0; t < n_tiles; ++t) {
+      copy_k(t + 3); copy_v(t + 2);
+      wait_copies<2 * PIECES>();
       __syncthreads();
-      const int x = s0; s0 = s1; s1 = s2; s2 = x;
     }
+    wait_copies<0>();
     continue;
   }
 
@@ -425,7 +436,6 @@ __global__ __launch_bounds__(512, 2) void wide_attn_kernel(WideParams e) {
     l_part[1] += blk[1];
   };
 
-  int s0 = 0, s1 = 1, s2 = 2;   // slots of tiles t, t+1, t+2 (= t-1)
   if (n_tiles > 0) {
 #pragma unroll
     for (int t = 0; t < 2; ++t) sacc[0][t][0] = sacc[0][t][1] = floatx4_t{0.f, 0.f, 0.f, 0.f};
@@ -439,25 +449,24 @@ __global__ __launch_bounds__(512, 2) void wide_attn_kernel(WideParams e) {
       m_ref[n] = zmax == -INFINITY ? 0.f : zmax;
     }
 #pragma unroll
-    for (int i = 0; i < 4; ++i) { kf[i] = frag(frag0 + NF * 1024, i); vf[i] = frag(frag0 + 5 * HT + NF * 1024, i); }
+    for (int i = 0; i < 4; ++i) { kf[i] = frag(frag0 + NF * 1024, i); vf[i] = frag(frag0 + 7 * HT + NF * 1024, i); }
   }
   auto tile_step = [&](int t, auto mask_tag) __attribute__((always_inline)) {
-    put_k(s2); put_v(s1);
-    load_k(t + 3); load_v(t + 2);
+    copy_k(t + 3); copy_v(t + 2);
     const int key0 = (tbase + t) * BN;
-    const char *const ka = frag0 + s0 * HT + NF * 1024, *const va = frag0 + (3 + s2) * HT + NF * 1024;
-    const char *const kb = frag0 + s1 * HT, *const vb = frag0 + (3 + s0) * HT;
+    const char *const ka = frag0 + (t & 3) * HT + NF * 1024, *const va = frag0 + (4 + ((t + 3) & 3)) * HT + NF * 1024;
+    const char *const kb = frag0 + ((t + 1) & 3) * HT, *const vb = frag0 + (4 + (t & 3)) * HT;
     step(ka, va, kb, vb, sacc[0], sacc[1], pop[1], pop[0], key0, mask_tag);
     step(kb, vb, kb + NF * 1024, vb + NF * 1024, sacc[1], sacc[0], pop[0], pop[1], key0 + 32, mask_tag);
+    wait_copies<2 * PIECES>();   // (what the tile before asked for: the next tile reads it)
     __syncthreads();
-    const int x = s0; s0 = s1; s1 = s2; s2 = x;
   };
   int t = 0;
   for (; t < n_full; ++t) tile_step(t, std::false_type{});
   for (; t < n_tiles; ++t) tile_step(t, std::true_type{});
   if (n_tiles > 0) {
-    // (the slots have been rotated: the last tile's is s2)
-    const char *vp = frag0 + (3 + s2) * HT + NF * 1024;
+    wait_copies<0>();   // (none may be under way when the next block fills the slots, or when the workgroup ends)
+    const char *vp = frag0 + (4 + ((n_tiles - 1) & 3)) * HT + NF * 1024;
 #pragma unroll
     for (int i = 0; i < NF; ++i)
 #pragma unroll
@@ -473,7 +482,7 @@ __global__ __launch_bounds__(512, 2) void wide_attn_kernel(WideParams e) {
     if (qrow >= p.Lq) continue;
     // register i of tile d is channel 16*d + 4*quarter + i
     if (partial) {
-      const int64_t prow = (int64_t)(2 * w + (round == e.rounds ? 0 : 1)) * 256 + wave * 32 + n * 16 + r16;
+      const int64_t prow = (int64_t)(2 * w + (round == e.rounds ? 0 : 1)) * BQ + wave * 32 + n * 16 + r16;
       if (quarter == 0) *reinterpret_cast<float2 *>(e.ws_ml + prow * 2) = make_float2(m_ref[n], l_sum);
       float *wptr = e.ws_o + prow * D + 4 * quarter;
 #pragma unroll
@@ -540,29 +549,44 @@ template <int D, int BITS> void expand_bits(const ExpandParams &e, bool chan, di
   else hipLaunchKernelGGL((expand_tiles_kernel<D, BITS, false, false>), grid, dim3(256), 0, st, e);
 }
 
-template <int D, bool F16> void launch_wide_shape(const WideParams &e, int n_wgs, hipStream_t st) {
-  constexpr int lds_bytes = 6 * kHalfTile<D>;
-  // above 64 KiB the limit has to be raised, once per device the process launches on
+template <int D, bool F16, int NW> void launch_wide_shape(const WideParams &e, int n_wgs, hipStream_t st) {
+  constexpr int lds_bytes = 8 * kHalfTile<D>;
   static bool configured[64] = {false};
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) dev = -1;
-  if (dev < 0 || !configured[dev]) {
-    (void)hipFuncSetAttribute(reinterpret_cast<const void *>(&wide_attn_kernel<D, F16>), hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes);
-    if (dev >= 0) configured[dev] = true;
+  allow_lds(reinterpret_cast<const void *>(&wide_attn_kernel<D, F16, NW>), lds_bytes, configured);
+  hipLaunchKernelGGL((wide_attn_kernel<D, F16, NW>), dim3((unsigned)n_wgs), dim3(NW * 64), lds_bytes, st, e);
+}
+template <int D, bool F16> void launch_wide_waves(const WideParams &e, const WidePlan &plan, hipStream_t st) {
+  if (plan.waves == 4) {
+    launch_wide_shape<D, F16, 4>(e, plan.n_wgs, st);
+    return;
   }
-  hipLaunchKernelGGL((wide_attn_kernel<D, F16>), dim3((unsigned)n_wgs), dim3(512), lds_bytes, st, e);
-  const int64_t left = (int64_t)e.a.bh_total * e.a.q_tiles - (int64_t)e.rounds * n_wgs;   // (none under key limits)
+  launch_wide_shape<D, F16, 8>(e, plan.n_wgs, st);
+  const int64_t left = (int64_t)e.a.bh_total * e.a.q_tiles - (int64_t)e.rounds * plan.n_wgs;   // (none under key limits)
   if (left > 0)
-    hipLaunchKernelGGL((wide_combine_kernel<D, F16>), dim3(256 / (1024 / D), (unsigned)left), dim3(256), 0, st, e, n_wgs);
+    hipLaunchKernelGGL((wide_combine_kernel<D, F16>), dim3(256 / (1024 / D), (unsigned)left), dim3(256), 0, st, e, plan.n_wgs);
 }
 
 }  // namespace
 
 namespace varq_attn {
 
+// A sequence attended as a whole under key limits ends when its last query blocks do, which see every key: with few pairs
+// most of the device waits for them, and blocks of 128 queries are done sooner (a tile takes four wavefronts 1.25 us where it takes eight 1.8)
+// and are twice as many to fill it with.  Block-causal rule, 4-bit codes, us, the kernel that widens per workgroup / blocks of
+// 256 / of 128: D=64, 16 pairs of 680 tokens 24.7 / 24.2 / 19.4, of 2440 66.9 / 58.1 / 47.1, of 5064 140 / 113 / 104; 32 pairs of 255
+// 14.4 / 16.9 / 14.0, of 680 25.0 / 26.2 / 21.7, of 1656 49.6 / 47.7 / 40.5, of 2440 71.1 / 65.1 / 63.8, of 3464 102 / 102 / 101; D=128, 16 of 680 31.2 / 34.6 / 26.3,
+// of 2440 93.6 / 84.5 / 65.3, of 5064 181 / 154 / 165; 32 of 680 33.1 / 38.1 / 29.9, of 1656 68.8 / 68.5 / 64.9, of 2440 97 / 89 / 105.  With 64 pairs the
+// device is full: 680 tokens 25.4 / 29.7 / 27.2 and 34.5 / 44.1 / 44.8.  Without limits, and with fewer than ten pairs, the shares
+// of the keys do better (8 pairs, widening / 128: D=64 1656 tokens 30.1 / 31.5, 2440 39.9 / 43.2; 10 pairs of 2440 48.8 / 45.8,
+// of 5064 112 / 99; D=128 50 / 44 at 1656, 161 / 165 at 5064), and 155 tokens are too few (11.3 / 12.8).
+bool wide_four(int64_t bh, int Lq, int Lk, int D, int cus, bool limits) {
+  return limits && Lk <= Lq && Lq > 192 && bh * 26 >= cus && bh * 8 <= cus && bh * ((Lq + 127) / 128) * 4 <= (D == 128 ? 7 : 10) * (int64_t)cus;
+}
 WidePlan plan_wide(int64_t bh, int Lq, int Lk, int D, int cus, bool share, bool limits) {
   WidePlan w;
-  const int64_t blocks = bh * ((Lq + 255) / 256), tiles = (Lk + BN - 1) / BN;
+  w.waves = wide_four(bh, Lq, Lk, D, cus, limits) ? 4 : 8;
+  const int block = 32 * w.waves;
+  const int64_t blocks = bh * ((Lq + block - 1) / block), tiles = (Lk + BN - 1) / BN;
   w.tile_bytes = (size_t)bh * (size_t)tiles * (size_t)(2 * BN * D * 2);
   w.n_wgs = (int)blocks;
   w.rounds = 1;
@@ -572,7 +596,7 @@ WidePlan plan_wide(int64_t bh, int Lq, int Lk, int D, int cus, bool share, bool 
     // HeavyFirst (an XCD takes every eighth pair; the grid is padded to whole eighths).  Dealt out beforehand in equal
     // numbers of blocks, or of all tiles, the longest workgroup has as much to do as without limits: 32 pairs of 10521
     // tokens, D=128, block-causal, 1386 us against 1057 like this (1598 without limits).
-    w.n_wgs = (int)((bh + 7) / 8 * 8 * ((Lq + 255) / 256));
+    w.n_wgs = (int)((bh + 7) / 8 * 8 * ((Lq + block - 1) / block));
     return w;
   }
   // One workgroup runs on a compute unit.  Whole blocks take ceil(blocks / cus) rounds; sharing the
@@ -622,9 +646,10 @@ void launch_wide(const AttnParams &p, int D, const WidePlan &plan, char *ws, hip
   e.rounds = plan.rounds;
   e.ws_o = reinterpret_cast<float *>(ws + plan.tile_bytes);
   e.ws_ml = e.ws_o + (size_t)(2 * plan.n_wgs) * 256 * (size_t)D;
-  if (D == 128) launch_wide_shape<128, false>(e, plan.n_wgs, st);
-  else if (p.f16) launch_wide_shape<64, true>(e, plan.n_wgs, st);
-  else launch_wide_shape<64, false>(e, plan.n_wgs, st);
+  e.a.q_tiles = (p.Lq + 32 * plan.waves - 1) / (32 * plan.waves);
+  if (D == 128) launch_wide_waves<128, false>(e, plan, st);
+  else if (p.f16) launch_wide_waves<64, true>(e, plan, st);
+  else launch_wide_waves<64, false>(e, plan, st);
 }
 
 }  // namespace varq_attn
