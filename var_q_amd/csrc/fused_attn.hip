@@ -760,15 +760,32 @@ __device__ __forceinline__ void attend_block(const AttnParams &p, int bh, int ou
 #pragma unroll
   for (int ch = 0; ch < NCH; ++ch) qb[ch] = *reinterpret_cast<const u32x4_t *>(qptr + k_octet<GK>(ch, half) * 8);
   if constexpr (CHAN) {
-    // the head's tables, as the widening steps use them (see lds_tab above)
-    for (int i = tid; i < p.nseg * TR * D; i += NT) {
-      const int seg = i / (TR * D), which = (i / D) % TR, d = i % D;
-      const bool is_k = which < 2, is_zp = which & 1;
-      const float *src = which == 0 ? p.k_chan_scale : which == 1 ? p.k_chan_zp : which == 2 ? p.v_chan_scale : p.v_chan_zp;
-      const int c = is_k ? (d & ~7) + KCodec<BITS>::slot_d(d & 7) : d;   // K rows: the operand's slot order inside an octet
-      const float x = src ? src[((int64_t)seg * p.Hkv + hs) * D + c] : 0.f;
-      const float mul = is_k ? KCodec<BITS>::kMul : VCodec<BITS>::kMul, off = is_k ? KCodec<BITS>::kOff : VCodec<BITS>::kOff;
-      lds_tab[i] = is_zp ? (x + off) * (1.f / mul) : x * mul;
+    // The head's tables, as the widening steps use them (see lds_tab above): a thread takes one value of every segment (or
+    // every second).  kTabLoads of them are under way before the first is used: one after the other, each a trip to memory,
+    // they were what a launch began with, 1.6 us (five segments) to 4.1 us (eight, four wavefronts) of the 10 to 20 that
+    // the smaller steps of a schedule take.
+    constexpr int kTabLoads = 8, SEGS = NT / (TR * D);
+    static_assert(NT % (TR * D) == 0 && D % 64 == 0, "which of the tables a thread loads is the same for a wavefront and every segment");
+    const int which = __builtin_amdgcn_readfirstlane(tid / D) % TR, seg0 = __builtin_amdgcn_readfirstlane(tid / (TR * D)), d = tid % D;
+    const bool is_k = which < 2, is_zp = which & 1;
+    // (as a global pointer: behind the choice the compiler no longer knows it for one, and flat loads wait for LDS too)
+    const auto src = (const __attribute__((address_space(1))) float *)(uintptr_t)(which == 0 ? p.k_chan_scale : which == 1 ? p.k_chan_zp : which == 2 ? p.v_chan_scale : p.v_chan_zp);
+    const int c = is_k ? (d & ~7) + KCodec<BITS>::slot_d(d & 7) : d;   // K rows: the operand's slot order inside an octet
+    const float mul = is_k ? KCodec<BITS>::kMul : VCodec<BITS>::kMul, off = is_k ? KCodec<BITS>::kOff : VCodec<BITS>::kOff;
+#pragma unroll
+    for (int round = 0; round < kMaxSegments / (kTabLoads * SEGS); ++round) {
+      const int first = seg0 + round * (kTabLoads * SEGS);
+      if (first >= p.nseg) break;
+      float x[kTabLoads] = {};
+      if (src) {
+#pragma unroll
+        for (int u = 0; u < kTabLoads; ++u) x[u] = src[((int64_t)min(first + u * SEGS, p.nseg - 1) * p.Hkv + hs) * D + c];
+      }
+#pragma unroll
+      for (int u = 0; u < kTabLoads; ++u) {
+        const int seg = first + u * SEGS;
+        if (seg < p.nseg) lds_tab[seg * (TR * D) + which * D + d] = is_zp ? (x[u] + off) * (1.f / mul) : x[u] * mul;
+      }
     }
   }
   __syncthreads();
