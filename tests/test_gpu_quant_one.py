@@ -70,3 +70,29 @@ def test_narrow_slices(dev, shape, dims, dtype):
         for x, (_, words, tab, _) in zip(xs, pair):
             q, s, _ = O.quant_reduce(x, dims, bits, False)
             assert torch.equal(words.cpu(), O.pack_last_dim(q, bits)[0]) and torch.equal(tab[2].cpu(), s.reshape(H, c))
+
+
+@pytest.mark.parametrize('shape,dims,dtype', [
+    ((8, 30, 1024, 64), (0, 2), torch.bfloat16),      # two tensors: 60 MiB, all 16 register steps
+    ((8, 400, 16, 128), (0, 1), torch.float16),       # two tensors: 25 MiB, one: 16-byte pieces
+    ((3, 24, 701, 128), (0, 2), torch.bfloat16),
+    ((5, 20, 333, 72), (0, 2), torch.float32),        # nine octets of sixteen lanes
+    ((24, 6, 171, 64), (0, 2), torch.float16),        # few heads: one tensor is left to the three launches
+    ((32, 30, 201, 64), (0, 3), torch.bfloat16),      # groups of whole rows: 24 MiB of one tensor, 47 of two
+])
+def test_sizes_where_one_launch_takes_over(dev, shape, dims, dtype):
+    """The same groups with the batch behind itself until they are too long for one launch, or the tensor too large: max and min,
+    scales, zero-points and codes are those of the three launches bit for bit, whichever way the call itself goes."""
+    gen = torch.Generator(device=dev).manual_seed(shape[2])
+    xs = [(torch.randn(*shape, generator=gen, device=dev) * 2).to(dtype) for _ in range(2)]
+    xs[0][..., 3] *= 15
+    xs[1][:, :, 0] = 0
+    rows = xs[0].numel() // shape[3] // (1 if 3 in dims else shape[1] if dims == (0, 2) else shape[2])
+    times = 8192 // rows + 1 if 3 not in dims else (128 << 20) // (xs[0].numel() * xs[0].element_size()) + 1
+    for bits, asym in ((8, False), (4, True), (2, False)):
+        note('quant one, sizes', shape, dims, dtype, bits, asym)
+        pair = ops.quant_pack_pair(*xs, dims, bits, asym)
+        for x, two in zip(xs, pair):
+            q, s, z = ops.quant_pack(x.repeat(times, 1, 1, 1), dims, bits, asym=asym)
+            for got in (two, ops.quant_pack(x, dims, bits, asym=asym)):
+                assert torch.equal(got[0], q[:shape[0]]) and torch.equal(got[1], s) and (not asym or torch.equal(got[2], z))

@@ -506,7 +506,7 @@ __device__ __forceinline__ void quant_one_block(const GenParams &p, const OnePla
   const int lcol = tid & (c8s - 1), col = slice * c8s + lcol, f = (tid >> pl.c8s_shift) & (sub - 1), lq = tid >> (pl.c8s_shift + pl.sub_shift);
   const int q = (tq << pl.lq_shift) + lq;
   const bool live = col < p.c8 && q < pl.Q && lq < (1 << pl.lq_shift);
-  // (the tensor is at most 16 MiB, so rows and byte offsets fit 32 bits)
+  // (the tensors are at most 128 MiB, so rows and byte offsets fit 32 bits)
   const u32 row0 = (u32)ko * (u32)pl.ko_rs + (live ? q : 0);
   auto row_of = [&](int j) {
     const u32 o = pl.by_RI((u32)j);
@@ -820,18 +820,39 @@ bool make_plan(const int64_t *sh, int reduce_mask, int64_t n_groups, Plan &pl) {
   return true;
 }
 
+// Whether the one-launch kernel takes less time than the three launches, with their 2048 workgroups on either side of the fold.
+// Those take 12.4 us and 0.44 per MiB (of padded rows), for two tensors 16.2 and 0.41.  A workgroup of 1024 threads of the one-launch
+// kernel, which has a compute unit to itself, takes 4.5 us and 0.22 per KiB in pieces of 16 bytes, 0.175 while there are no more than 128 of them, 0.135
+// in pieces of 32 (0.17 where the rows lie multiples of 1 KiB apart), 0.10 in longer ones.  Three / one, us, 8 bits, a scale per (head, channel), two tensors:
+// [2,16,n,128] 16 MiB 23.3 / 12.5, 25 25.0 / 18.9, 36 29.5 / 24.5, 64 44.2 / 39.4; [32,n,30,64] 23 24.7 / 18.6, 40 32.2 / 27.2, 60 42.1 / 38.2;
+// [8,n,16,128] 36 30.2 / 28.4, 64 44.1 / 51.0; [64,n,16,64] 16 23.8 / 18.3, 25 25.4 / 27.8, 64 43.3 / 63.9; [4,8,n,128] 16 24.5 / 17.7, 25 25.7 / 27.0;
+// [64,n,8,64] 12.5 21.3 / 24.2; one tensor: [64,n,16,64] 8 17.0 / 15.9, 12.5 18.0 / 24.2; [32,n,30,64] 11.7 16.9 / 15.1, 20 20.6 / 23.9; [16,n,12,64]
+// 6 14.9 / 15.6, 9.4 15.7 / 23.9; [64,n,8,64] 6.2 15.8 / 22.9, 16 19.6 / 51.6; [2,16,n,128] 12.5 17.6 / 14.7, 18 19.3 / 20.6; fp32 [2,16,1600,128] 50 31.2 / 22.2.
+// (The line was 16 MiB in all.)  Groups of whole rows, one scale per (token, head), [32,30,L,64]: 20 MiB 18.6 / 15.6, 40 30.2 / 27.0, 80 48.0 / 50.1; with
+// zero-points two tensors of 40 29.0 / 35.4.  With the step dequantized in the same launch the other way has one
+// more, whose work the one launch does beside: three and that / one, per tensor to fp32, [64,100,16,64] 40 / 74, [32,169,16,64] 41 / 64, [32,256,16,64]
+// 51 / 71, [32,12,256,64] 46 / 62, [64,100,8,64] 26 / 30, [32,169,30,64] 58 / 48, [16,256,8,128] 43 / 38, [32,100,16,64] 25 / 19.
+bool one_launch_pays(const OnePlan &pl, int c8, int c8p, int threads, bool keepc, double mib, int elem, int tensors, bool asym, bool with_values) {
+  if (!keepc) return mib <= (asym ? 16 : 48);
+  if (threads == 256) return mib <= 16;
+  const int64_t wgs = (int64_t)pl.blocks * pl.slices * tensors;
+  const int piece = (8 * elem) << pl.c8s_shift;
+  const bool apart = pl.RI == 1 && pl.ro_rs * c8 * 8 * elem % 1024 == 0;
+  const double per_kib = piece <= 16 ? (wgs <= 128 ? 0.175 : 0.22) : piece == 32 ? (apart ? 0.17 : 0.135) : 0.10;
+  const double one = 4.5 + per_kib * (asym ? 1.1 : 1.0) * mib * 1024.0 / (double)wgs * (double)((wgs + 255) / 256);
+  const double three = (tensors == 2 ? 16.2 + 0.41 * mib * c8p / c8 : 12.4 + 0.44 * mib * c8p / c8) + (asym ? 3.0 : 0.0) + (with_values ? 10.5 : 0.0);
+  return one < three;
+}
+
 // The one-launch plan, or false when a group has too many rows for a workgroup's registers.
-bool make_one_plan(const int64_t *sh, int reduce_mask, int row_steps, int tensors, int bits, bool with_values, OnePlan &pl, int &threads) {
+bool make_one_plan(const int64_t *sh, int reduce_mask, int elem, int tensors, int bits, bool asym, bool with_values, OnePlan &pl, int &threads) {
   const int64_t c = sh[3], rows = sh[0] * sh[1] * sh[2];
+  const int row_steps = elem == 4 ? 8 : 16;
   if (c % 8 != 0 || c > 512 || rows <= 0 || rows >= (1ll << 31) - 512) return false;
   const Canonical k = canonical(sh, reduce_mask);
   const int64_t rr = k.nro * k.RI;
-  // Up to 16 MiB (of both tensors) one launch was the faster way in everything measured; beyond, the three launches, with
-  // 2048 workgroups on either side of the fold, catch up sooner or later: three / one, us, one scale per (head, channel), K and V
-  // [2,16,n,128] 25 MiB 22.9 / 16.9, 36 25.6 / 21.7, 64 37.8 / 42.0, [64,n,16,64] 25 23.5 / 21.8, 30 26.2 / 25.0,
-  // [32,n,30,64] 40 29.7 / 24.3, 60 35.2 / 33.8, one tensor of it 20 20.5 / 23.0, 30 22.8 / 31.8; one scale per (token, head),
-  // [32,30,L,64] 20 16.8 / 12.6, 40 25.6 / 21.7, 80 43.8 / 48.7.
-  if (rr > 8192 || rows * c * (row_steps == 8 ? 4 : 2) * tensors > (16ll << 20)) return false;
+  const double mib = (double)(rows * c * elem * tensors) / (1 << 20);
+  if (rr > 8192 || mib > 128) return false;   // (rows and byte offsets of the kernel are of 32 bits)
   const bool keepc = !(reduce_mask & 8);
   const int c8 = (int)(c / 8);
   int c8p_shift = 0;
@@ -868,7 +889,7 @@ bool make_one_plan(const int64_t *sh, int reduce_mask, int row_steps, int tensor
     pl.blocks = pl.nko * pl.tilesQ;
     const bool fits = pl.steps <= row_steps;
     const int enough = with_values ? 128 : threads == 1024 ? 129 : 160;
-    if (fits && ((int64_t)pl.blocks * pl.slices * tensors >= enough || !keepc || pl.c8s_shift <= narrowest)) return true;
+    if (fits && ((int64_t)pl.blocks * pl.slices * tensors >= enough || !keepc || pl.c8s_shift <= narrowest)) return one_launch_pays(pl, c8, 1 << c8p_shift, threads, keepc, mib, elem, tensors, asym, with_values);
     if (!keepc || pl.c8s_shift <= narrowest) return false;
   }
 }
@@ -1074,7 +1095,7 @@ int quant_pack_impl(const void *x, const void *x1, int x_dtype, const int64_t *h
   hipStream_t st = (hipStream_t)stream;
   OnePlan one;
   int threads;
-  if (tiled && make_one_plan(s, reduce_mask, x_dtype == VARQ_F32 ? 8 : 16, x1 ? 2 : 1, words ? bits : 8, step != nullptr, one, threads)) {
+  if (tiled && make_one_plan(s, reduce_mask, x_dtype == VARQ_F32 ? 4 : 2, x1 ? 2 : 1, words ? bits : 8, asym != 0, step != nullptr, one, threads)) {
     if (step) {
       step->q_blocks = (one.blocks + 7) / 8 * 8 * one.slices;
       step->pair_blocks = (int)((step->earlier.pair_octs + kStepOctets - 1) / kStepOctets);
