@@ -1459,16 +1459,17 @@ size_t split_workspace_bytes(int splits, int64_t rows, int D) {
 // a grid that already fills the device in whole rounds does not.
 int choose_splits(int64_t wgs, int tiles, int64_t rows, int D) {
   const double cus = device_cus();
-  const double tile_us = D == 128 ? 2.3 : 1.4, fixed_us = 9.0;
+  // (D=64, no sharing / what the former 9 us and 4 TB/s chose / now: 32 pairs, 256 x 521 18.8 / 18.8 / 15.6; 128 pairs, 256 x 1500 44.8 / 44.8 / 36.0)
+  const double tile_us = D == 128 ? 2.3 : 1.4, fixed_us = D == 128 ? 9.0 : 6.0, bytes_us = D == 128 ? 4.0e6 : 5.0e6, gain = D == 128 ? 0.9 : 0.92;
   double base = 0.0, best = 0.0;
   int best_s = 1;
   for (int s = 1; s <= kMaxSplits; ++s) {
     if (s > 1 && tiles / s < 2) break;
     const double rounds = (double)((wgs * s + (int64_t)cus - 1) / (int64_t)cus);
     double t = rounds * ((double)((tiles + s - 1) / s) * tile_us + fixed_us);
-    if (s > 1) t += 4.0 + 2.0 * (double)split_workspace_bytes(s, rows, D) / 4.0e6;   // 4 TB/s, in us
+    if (s > 1) t += 4.0 + 2.0 * (double)split_workspace_bytes(s, rows, D) / bytes_us;   // written and read
     if (s == 1) base = best = t;
-    else if (t < 0.9 * base && t < best) { best = t; best_s = s; }   // sharing must gain a tenth
+    else if (t < gain * base && t < best) { best = t; best_s = s; }   // sharing must gain a tenth or so
   }
   return best_s;
 }
