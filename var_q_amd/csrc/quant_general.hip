@@ -344,15 +344,7 @@ __global__ __launch_bounds__(256) void finalize_tiled_kernel(GenParams p, int Z,
 // Quantizes and stores one octet (column `col`) of row `row`: s, z the scale and the zero-point of the octet's groups (one per channel or one).
 // also(codes): what else the caller wants from them.
 struct Nothing { __device__ __forceinline__ void operator()(const int (&)[8]) const {} };
-template <int NV, class F = Nothing>
-__device__ __forceinline__ void store_octet(const GenParams &p, int64_t row, int col, const float (&v)[8], const float (&s)[NV],
-                                            const float (&z)[NV], F &&also = F()) {
-  const float qmin = (float)p.qmin, qmax = (float)p.qmax;
-  const u32 mask = (1u << p.bits) - 1u;
-  int q[8];
-#pragma unroll
-  for (int j = 0; j < 8; ++j) q[j] = (int)__builtin_amdgcn_fmed3f(rintf(v[j] / s[j % NV]) + z[j % NV], qmin, qmax);
-  also(q);
+__device__ __forceinline__ void store_codes(const GenParams &p, int64_t row, int col, const int (&q)[8], u32 mask) {
   const int64_t orow = out_row32(p, row);
   if (p.codes || p.bits == 8) {
     const u32 lo = (q[0] & 0xff) | ((q[1] & 0xff) << 8) | ((q[2] & 0xff) << 16) | ((u32)q[3] << 24);
@@ -371,6 +363,17 @@ __device__ __forceinline__ void store_octet(const GenParams &p, int64_t row, int
       if ((col & 1) == 0) p.words[orow * p.wpr + (col >> 1)] = (int32_t)(w | (other << 16));
     }
   }
+}
+template <int NV, class F = Nothing>
+__device__ __forceinline__ void store_octet(const GenParams &p, int64_t row, int col, const float (&v)[8], const float (&s)[NV],
+                                            const float (&z)[NV], F &&also = F()) {
+  const float qmin = (float)p.qmin, qmax = (float)p.qmax;
+  const u32 mask = (1u << p.bits) - 1u;
+  int q[8];
+#pragma unroll
+  for (int j = 0; j < 8; ++j) q[j] = (int)__builtin_amdgcn_fmed3f(rintf(v[j] / s[j % NV]) + z[j % NV], qmin, qmax);
+  also(q);
+  store_codes(p, row, col, q, mask);
 }
 
 // The groups of one octet (one per channel or one) where all scales allow the exact quotient shortcut and the zero-points are
@@ -457,12 +460,27 @@ __global__ __launch_bounds__(256) void quant_tiled_kernel(GenParams p, Plan pl, 
     if (ASYM) z[0] = p.zp[g];
     fast = plain[g] != 0u;
   }
-  if (!__any(!fast)) {
-    const FastOctet<NV, ASYM> o(p, s, r, z);
-    for_rows<DT>(p, pl, l, [&](u32 row, const float (&v)[8]) { o.store(p, out_row32(p, row), l.col, v, [](const float (&)[8]) {}); });
-  } else {
-    for_rows<DT>(p, pl, l, [&](u32 row, const float (&v)[8]) { store_octet<NV>(p, row, l.col, v, s, z); });
-  }
+  // (The longer arithmetic of the two: with FastOctet's, the chunks run ahead of what the Infinity Cache serves.  us for the three launches, this /
+  // that: a scale per (head, channel) of [32,30,680,64] 8 bits 51.0 / 53.0, fp32 78.4 / 79.8, 4 bits affine 49.0 / 51.1, of [2,16,10521,128] 52.5 / 54.5,
+  // [64,256,16,64] 26.5 / 27.1; one scale 50.8 / 52.0; but one per (token, head) 48.8 / 47.8.)
+  const float qmin = (float)p.qmin, qmax = (float)p.qmax;
+  const u32 mask = (1u << p.bits) - 1u;
+  for_rows<DT>(p, pl, l, [&](u32 row, const float (&v)[8]) {
+    int q[8];
+    if (fast) {
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        const float sj = s[j % NV], rj = r[j % NV];
+        const float q0 = v[j] * rj;
+        const float t = __builtin_fmaf(__builtin_fmaf(-q0, sj, v[j]), rj, q0);
+        q[j] = (int)__builtin_amdgcn_fmed3f(rintf(t) + z[j % NV], qmin, qmax);
+      }
+    } else {
+#pragma unroll
+      for (int j = 0; j < 8; ++j) q[j] = (int)__builtin_amdgcn_fmed3f(rintf(v[j] / s[j % NV]) + z[j % NV], qmin, qmax);
+    }
+    store_codes(p, row, l.col, q, mask);
+  });
 }
 
 // ---- one launch: a workgroup holds all rows of its groups -----------------------------------------
@@ -960,12 +978,11 @@ int run_tiled(GenParams &p, const Plan &pl, void *workspace, hipStream_t st) {
   // per thread measured alike, longer ones slower)
   const Plan &pb = pl;
   dim3 bgrid((unsigned)((int64_t)pb.nko * pb.tilesQ * pb.Z), nt);
-  // Five workgroups on a compute unit instead of eight (by LDS that they do not use) where a large tensor has long groups: the chunks that
-  // are read at once are fewer, and the second read comes faster out of the Infinity Cache.  Eight / five, us for the three
-  // launches, 8 bits, a scale per (head, channel): [32,30,680,64] bf16 53.0 / 50.6, [2,16,10521,128] 54.7 / 52.1, [64,30,680,128] 215 /
-  // 201, one scale for [32,30,680,64] fp32 75.7 / 72.4; but [2,16,2304,128] 19.3 / 20.2, two tensors [64,256,16,64] 42.6 / 44.9, a scale per (token,
-  // head) of [32,30,680,64] 47.9 / 48.6.
-  const bool large = !p.x1 && p.rows * p.c * In8<DT>::kBytes >= (60ll << 20) && pl.Z >= 16;
+  // Five workgroups on a compute unit instead of eight (by LDS that they do not use) where the Infinity Cache does not hold a tensor
+  // with long groups: fewer chunks are read at once, and more of the second read comes out of it.  Eight / five, us for the three launches:
+  // [64,30,680,128] bf16, a scale per (head, channel) 219 / 202, 4 bits affine 207 / 188, one scale for [32,30,680,64] fp32 75.6 / 72.8; at half the size it
+  // turns round, [32,30,680,64] bf16 with its dequantization behind it 60.6 / 63.6.
+  const bool large = !p.x1 && p.rows * p.c * In8<DT>::kBytes >= (128ll << 20) && pl.Z >= 16;
   const unsigned lds = large ? 32000 : 0;
   if (p.asym) {
     if (p.keepc) hipLaunchKernelGGL((quant_tiled_kernel<DT, true, true>), bgrid, dim3(256), lds, st, p, pb, rinv, plain);
