@@ -308,7 +308,8 @@ int varq_quant_step_dequant(const void *x, int x_dtype, int B, int H, int n, int
  * dividing D.
  */
 size_t varq_fused_attn_workspace_bytes(int B, int Hkv, int Lq, int Lk, int D, int nseg, int splits);
-/* Many queries over a long cache (five or more blocks of 256 per (batch, head)): given a workspace of
+/* Many queries over a long cache (five or more blocks of 256 per (batch, head); with key limits also a whole
+ * sequence of few (batch, head) pairs): given a workspace of
  * this many bytes and splits = 0 or 1, the attention entry points dequantize K and V once into matrix
  * operands kept there and stream those, instead of dequantizing every key tile again for each block of
  * queries.  Same operands, same result to rounding.  0: not worth it for this shape.  (A caller that

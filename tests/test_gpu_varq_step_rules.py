@@ -29,6 +29,7 @@ def _same(a, b):
     (2, 7, 128, 8, False, torch.float32, (5, 300, 1)),
     (2, 2, 24, 8, True, torch.bfloat16, (1, 17, 3)),                   # (no attention over 24 channels)
     (4, 16, 128, 4, True, torch.bfloat16, (3, 2, 2100, 1)),            # a step that takes several launches between two that take one
+    (16, 16, 64, 8, True, torch.float16, (3, 600, 1)),                 # 37 MiB of K and V in one launch under the rules of whole rows
 ])
 def test_same_state_as_the_general_calls(dev, method, layout, B, H, c, bits, symmetric, dtype, steps):
     g = torch.Generator().manual_seed(B * 1000 + H * 10 + bits)
