@@ -159,9 +159,10 @@ bool wide_four(int64_t bh, int Lq, int Lk, int D, int cus, bool limits);
 // share: whether blocks may be shared out; limits: whether the queries have key limits
 WidePlan plan_wide(int64_t bh, int Lq, int Lk, int D, int cus, bool share, bool limits);
 // Expands the packed cache of p (per-key groups of k_group / v_group channels, or the per-channel
-// tables) into `tiles`, pair after pair; with `place`, the pairs of a bit-width class to the places of
-// their heads (p.head_map) among the p.Hq heads of the cache.
-void launch_expand(const AttnParams &p, int D, int bits, int k_group, int v_group, bool chan, char *tiles, hipStream_t st, bool place = false);
+// tables) into `tiles`, pair after pair.
+void launch_expand(const AttnParams &p, int D, int bits, int k_group, int v_group, bool chan, char *tiles, hipStream_t st);
+// ... and a cache whose heads have several bit-widths, every class to the places of its heads among the p.Hq heads of the cache.
+void launch_expand_classes(const AttnParams &p, int D, const ClassTable &t, int group, char *tiles, hipStream_t st);
 // Attends the expanded tiles at the start of `ws`.
 void launch_wide(const AttnParams &p, int D, const WidePlan &plan, char *ws, hipStream_t st);
 

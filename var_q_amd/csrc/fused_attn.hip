@@ -1866,19 +1866,20 @@ extern "C" int varq_fused_attn_classes(const void *q, void *out, const varq_kv_c
     combine_few(p, D, st);
   } else if ((splits == 0 || splits == 1) && wide_eligible(B, p.Hkv, Lq, Lk, D, kv_limit != nullptr) &&
              run_wide(p, D, splits, workspace, workspace_bytes, st, [&](const AttnParams &part, int first, char *ws) {
-               // (one expanding launch per class, into the places of its heads)
+               ClassTable of = t;   // the part's batch entries of every class
+               int pairs = 0;
                for (int i = 0; i < 3; ++i) {
-                 if (!t.c[i].heads) continue;
-                 AttnParams c = part;
-                 c.k_words = t.c[i].k_words; c.v_words = t.c[i].v_words;
-                 c.k_scale = t.c[i].k_scale; c.k_zp = t.c[i].k_zp; c.v_scale = t.c[i].v_scale; c.v_zp = t.c[i].v_zp;
-                 c.head_map = t.c[i].head_map;
-                 c.Hkv = t.c[i].heads;
-                 c.bh_total = c.B * c.Hkv;
-                 c.kv_bs = (int64_t)c.Hkv * Lk_stride;
-                 skip_entries(c, first, D, 8 >> i, D / group, D / group);
-                 launch_expand(c, D, 8 >> i, group, group, false, ws, st, true);
+                 ClassParams &d = of.c[i];
+                 d.first = pairs;
+                 if (!d.heads) continue;
+                 const int64_t rows = (int64_t)first * d.heads * Lk_stride, words = rows * (D * (8 >> i) / 32), groups = rows * (D / group);
+                 d.k_words += words; d.v_words += words;
+                 d.k_scale += groups; d.v_scale += groups;
+                 if (d.k_zp) d.k_zp += groups;
+                 if (d.v_zp) d.v_zp += groups;
+                 pairs += part.B * d.heads;
                }
+               launch_expand_classes(part, D, of, group, ws, st);
              })) {
   } else {
     if (int e = set_splits(p, D, (Lk + BN - 1) / BN, splits, workspace, workspace_bytes, "fused_attn_classes")) return e;

@@ -31,7 +31,6 @@ struct ExpandParams {
   AttnParams a;
   char *tiles;
   int n_tiles, kg_shift, vg_shift;   // log2 of the channels per scale group
-  int places;                        // heads of the tile buffer per batch entry where head_map places them there (0: see the kernel)
 };
 
 // the eight codes of octet `oct` of a packed row, as they lie, and as numbers
@@ -50,19 +49,15 @@ template <int BITS> __device__ __forceinline__ void code_values(uint2 w, float (
 // tile are requested before the first is used, and the segment that a tile's keys belong to is looked up once (key by
 // key, and with each octet's loads behind a check of its key, [2,16,10521,128] took 51 us at 4 bits in groups and 76 at
 // 8 bits with 13 per-channel tables; now 43 and 49, 5.0 and 5.3 TB/s).
+constexpr int kTransposed = BN + 8;   // keys of a row of the transposed tile
+// (vt: [D][kTransposed], seg_end: [kMaxSegments] in LDS; place: the pair of the tile buffer)
 template <int D, int BITS, bool CHAN, bool F16>
-__global__ __launch_bounds__(256) void expand_tiles_kernel(ExpandParams e) {
+__device__ __forceinline__ void expand_tile(const ExpandParams &e, const AttnParams &p, int tile, int bh, int place, uint16_t *vt, int *seg_end) {
   constexpr int WPR = D * BITS / 32, NF = D / 16, OCT = D / 8;   // NF: fragments per 32 keys
-  constexpr int VTS = BN + 8;
-  __shared__ uint16_t vt[D * VTS];
-  __shared__ int seg_end[kMaxSegments];
-  const AttnParams &p = e.a;
-  const int tile = blockIdx.x, bh = blockIdx.y, tid = threadIdx.x;
+  constexpr int VTS = kTransposed;
+  const int tid = threadIdx.x;
   const int b = bh / p.Hkv, hs = bh - b * p.Hkv;
   const int64_t kv_row0 = b * p.kv_bs + hs * p.kv_hs;
-  // (the place of the head that a packed head of a mixed-width cache serves; the others attend what they hold in
-  // the order that it is packed)
-  const int place = e.places ? b * e.places + p.head_map[hs] : bh;
   char *const out = e.tiles + ((int64_t)place * e.n_tiles + tile) * (2 * kHalfTile<D>);
   constexpr int VI = BN / 2 * OCT / 256, KI = BN * OCT / 256;   // items of a thread: two keys' octets of V, one of K
   const int key0 = tile * BN;
@@ -155,6 +150,23 @@ __global__ __launch_bounds__(256) void expand_tiles_kernel(ExpandParams e) {
     *reinterpret_cast<u32x4_t *>(out + kHalfTile<D> + item * 16) =
         *reinterpret_cast<const u32x4_t *>(&vt[((frag % NF) * 16 + r) * VTS + (frag / NF) * 32 + g * 8]);
   }
+}
+
+template <int D, int BITS, bool CHAN, bool F16>
+__global__ __launch_bounds__(256) void expand_tiles_kernel(ExpandParams e) {
+  __shared__ uint16_t vt[D * kTransposed];
+  __shared__ int seg_end[kMaxSegments];
+  expand_tile<D, BITS, CHAN, F16>(e, e.a, blockIdx.x, blockIdx.y, blockIdx.y, vt, seg_end);
+}
+// All bit-widths of a cache in one launch, each head's tiles to its place among the heads: [8,16,n,128] with 8, 3 and 5 heads
+// of 8, 4 and 2 bits, us, a launch per width -> one: n = 4121 88 -> 77, 6425 123 -> 111, 10521 192 -> 179 (5.3 TB/s).
+template <int D, bool F16>
+__global__ __launch_bounds__(256) void expand_classes_kernel(ExpandParams e, ClassTable t) {
+  __shared__ uint16_t vt[D * kTransposed];
+  AttnParams p = e.a;
+  in_class(p, t, blockIdx.y, [&](auto bits, int bh, int place) __attribute__((always_inline)) {
+    expand_tile<D, decltype(bits)::value, false, F16>(e, p, blockIdx.x, bh, place, vt, nullptr);
+  });
 }
 
 typedef __attribute__((__vector_size__(4 * sizeof(float)))) float floatx4_t;
@@ -618,9 +630,8 @@ WidePlan plan_wide(int64_t bh, int Lq, int Lk, int D, int cus, bool share, bool 
   return w;
 }
 
-void launch_expand(const AttnParams &p, int D, int bits, int k_group, int v_group, bool chan, char *tiles, hipStream_t st, bool place) {
+void launch_expand(const AttnParams &p, int D, int bits, int k_group, int v_group, bool chan, char *tiles, hipStream_t st) {
   ExpandParams e;
-  e.places = place ? p.Hq : 0;
   e.a = p;
   e.tiles = tiles;
   e.n_tiles = (p.Lk + BN - 1) / BN;
@@ -636,6 +647,18 @@ void launch_expand(const AttnParams &p, int D, int bits, int k_group, int v_grou
   if (D == 128) VARQ_EXPAND(128);
   else VARQ_EXPAND(64);
 #undef VARQ_EXPAND
+}
+
+void launch_expand_classes(const AttnParams &p, int D, const ClassTable &t, int group, char *tiles, hipStream_t st) {
+  ExpandParams e;
+  e.a = p;
+  e.tiles = tiles;
+  e.n_tiles = (p.Lk + BN - 1) / BN;
+  e.kg_shift = e.vg_shift = varq_log2_exact(group);
+  dim3 grid((unsigned)e.n_tiles, (unsigned)p.bh_total);
+  if (D == 128) hipLaunchKernelGGL((expand_classes_kernel<128, false>), grid, dim3(256), 0, st, e, t);
+  else if (p.f16) hipLaunchKernelGGL((expand_classes_kernel<64, true>), grid, dim3(256), 0, st, e, t);
+  else hipLaunchKernelGGL((expand_classes_kernel<64, false>), grid, dim3(256), 0, st, e, t);
 }
 
 void launch_wide(const AttnParams &p, int D, const WidePlan &plan, char *ws, hipStream_t st) {
