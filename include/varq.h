@@ -177,6 +177,15 @@ int varq_quant_pack2(const void *x0, const void *x1, int x_dtype, const int64_t 
 int varq_quant_pack_spread(const void *x0, const void *x1, int x_dtype, const int64_t *host_shape4, int reduce_mask, int bits, int asym,
                            float eps, int32_t *words0, float *scale0, float *zp0, int32_t *words1, float *scale1, float *zp1,
                            const int64_t *host_out_map, const int64_t *host_scale_map, void *stream);
+/*
+ * varq_quant_pack_spread, with the scale (and zero-point) of every group also written once, to element g of once_scale0 and once_zp0
+ * (once_scale1 and once_zp1 of x1), fp32 [n_groups] as varq_quant_pack writes them: the parameters of the step by
+ * themselves (VAR_Q/quant.py:112-116), which a caller may change without changing the cache.  All NULL: varq_quant_pack_spread.
+ */
+int varq_quant_pack_spread_once(const void *x0, const void *x1, int x_dtype, const int64_t *host_shape4, int reduce_mask, int bits, int asym,
+                                float eps, int32_t *words0, float *scale0, float *zp0, int32_t *words1, float *scale1, float *zp1,
+                                float *once_scale0, float *once_zp0, float *once_scale1, float *once_zp1,
+                                const int64_t *host_out_map, const int64_t *host_scale_map, void *stream);
 
 /*
  * varq_quant_pack for callers that cannot allocate device memory (code under HIP graph

@@ -9,6 +9,7 @@
 // VarqError for tensors off the GPU and for statuses of the library.
 #include <Python.h>
 
+#include <array>
 #include <optional>
 
 #include <ATen/core/Tensor.h>
@@ -878,16 +879,21 @@ struct Quantizer {
     } else if (d == 2) set(1, 1, 0, len, 1, B * H, cap);
     else set(1, H, 0, len * H, H, B, cap * H);
   }
-  // the state that quant() followed by cache() leaves, the kernels having written codes and scales in place
-  void commit(int64_t n) const {
+  // the shape of the scale of a step of n tokens
+  std::array<int64_t, 4> scale_shape(int64_t n) const {
     const int64_t H = heads(), s1 = d == 1 ? n : H, s2 = d == 1 ? H : n;
     const bool tokens = per_token(rule);
-    const int64_t shape[4] = {1, rule == Rule::kTokenHead || (tokens && d == 1) || (!tokens && d == 2 && rule != Rule::kScale) ? s1 : 1,
-                              rule == Rule::kTokenHead || (tokens && d == 2) || (!tokens && d == 1 && rule != Rule::kScale) ? s2 : 1,
-                              rule == Rule::kHeadDim ? c : 1};
+    return {1, rule == Rule::kTokenHead || (tokens && d == 1) || (!tokens && d == 2 && rule != Rule::kScale) ? s1 : 1,
+            rule == Rule::kTokenHead || (tokens && d == 2) || (!tokens && d == 1 && rule != Rule::kScale) ? s2 : 1, rule == Rule::kHeadDim ? c : 1};
+  }
+  // the state that quant() followed by cache() leaves, the kernels having written codes and scales in place; once: the step's
+  // scale and zero-point by themselves (undefined: its row of the step tables is they)
+  void commit(int64_t n, const at::Tensor *once = nullptr) const {
+    const bool tokens = per_token(rule);
+    const auto shape = scale_shape(n);
     const Ref sshape(Py_BuildValue("(LLLL)", (long long)shape[0], (long long)shape[1], (long long)shape[2], (long long)shape[3]));
-    set_attribute(o, NAME(_window), Py_BuildValue("(OLLLOOLO)", buf.o, (long long)d, (long long)len, (long long)n, scale.o, asym ? zp.o : Py_None,
-                                                  (long long)(tokens ? -1 : k), sshape.o));
+    const Ref s(once ? wrap(once[0]) : Py_NewRef(scale.o)), z(!asym ? Py_NewRef(Py_None) : once ? wrap(once[1]) : Py_NewRef(zp.o));
+    set_attribute(o, NAME(_window), Py_BuildValue("(OLLLOOLO)", buf.o, (long long)d, (long long)len, (long long)n, s.o, z.o, (long long)(once ? -1 : k), sshape.o));
     Py_INCREF(Py_None);
     set_attribute(o, NAME(_staged), Py_None);
     Py_INCREF(sshape.o);
@@ -933,14 +939,20 @@ PyObject *quantizer_step(PyObject *const *a) {
   float *const s[2] = {at_row(kq.scale), two ? at_row(vq->scale) : nullptr}, *const z[2] = {at_row(kq.zp), two ? at_row(vq->zp) : nullptr};
   int64_t spread[7];
   if (!rows) kq.spread(n, spread);
+  at::Tensor once[2][2];   // [K, V][scale, zero-point] of the step by themselves: scale and zp are a caller's to change, the cache's copies are not
   const int rc = status_unlocked([&] {
     if (rows) return pack_rows(k, x1, dt, sh, mask, bits, asym, (float)eps, w0, w1, s, z, map);
-    return varq_quant_pack_spread(k.data_ptr(), x1, dt, sh, mask, bits, asym, (float)eps, w0, s[0], z[0], w1, s[1], z[1], map, spread, stream_of(k));
+    const auto shape = kq.scale_shape(n);
+    for (int i = 0; i < (two ? 2 : 1); ++i)
+      for (int j = 0; j < (asym ? 2 : 1); ++j) once[i][j] = empty(shape, at::kFloat, k);
+    auto at_once = [&](int i, int j) { return once[i][j].defined() ? ptr<float>(once[i][j]) : nullptr; };
+    return varq_quant_pack_spread_once(k.data_ptr(), x1, dt, sh, mask, bits, asym, (float)eps, w0, s[0], z[0], w1, s[1], z[1], at_once(0, 0), at_once(0, 1),
+                                       at_once(1, 0), at_once(1, 1), map, spread, stream_of(k));
   });
   if (!rows && rc == VARQ_ERR_UNSUPPORTED) Py_RETURN_FALSE;
   check(rc, "varq_quant_pack");
-  kq.commit(n);
-  if (two) vq->commit(n);
+  kq.commit(n, rows ? nullptr : once[0]);
+  if (two) vq->commit(n, rows ? nullptr : once[1]);
   Py_RETURN_TRUE;
 }
 

@@ -69,6 +69,7 @@ struct Spread {
   FastDiv by_gi, by_in;
   u32 gi, r_in, reps;        // reps = r_in * r_out
   int64_t go, ge, off, s_out;
+  float *scale, *zp, *scale1, *zp1;   // where they go once each as well, in the order of the groups (or null)
 };
 
 struct GenParams {
@@ -78,13 +79,12 @@ struct GenParams {
   float *scale, *zp;
   int32_t *words;
   int8_t *codes;
-  int64_t n0, n1, n2;      // leading dims
+  int64_t n1, n2;          // the last two leading dims
   int64_t gs0, gs1, gs2;   // group-id stride of each leading dim (0 = reduced)
   int64_t rows;            // n0*n1*n2
   int64_t n_groups;
-  int c, c8, c8p, c8p_shift; // channels, octets per row, lanes per row (pow2)
+  int c, c8;               // channels, octets per row
   int keepc;               // last dim kept (one group per channel) or reduced
-  int rows_per_block;
   int bits, qmin, qmax, wpr; // wpr = words per row
   int asym;
   float eps;
@@ -108,6 +108,7 @@ struct GenParams {
 __device__ __forceinline__ bool take_second(GenParams &p) {
   if (blockIdx.y == 0) return false;
   p.x = p.x1; p.scale = p.scale1; p.zp = p.zp1; p.words = p.words1; p.codes = p.codes1;
+  p.spread.scale = p.spread.scale1; p.spread.zp = p.spread.zp1;
   return true;
 }
 
@@ -595,10 +596,11 @@ __device__ __forceinline__ void quant_one_block(const GenParams &p, const OnePla
     par_s[t] = s;
     // (the exact-quotient shortcut, see finalize_tiled_kernel; 0: this group takes the division)
     par_r[t] = (s > 0x1p-96f && s < 0x1p96f && (f2u(s) & 0x7fffffu) != 0x7fffffu && fabsf(zp) <= 0x1p21f) ? 1.0f / s : 0.f;
-    if (mine && (KEEPC || !p.spread.on)) {
+    float *const once = KEEPC || !p.spread.on ? p.scale : p.spread.scale;
+    if (mine && once) {
       const int64_t g = (int64_t)ko * pl.ko_gs + (int64_t)tqi * pl.q_gs + (KEEPC ? slice * c8s * 8 + g8 : 0);
-      p.scale[g] = s;
-      if (ASYM) p.zp[g] = zp;
+      once[g] = s;
+      if (ASYM) (KEEPC || !p.spread.on ? p.zp : p.spread.zp)[g] = zp;
     }
   }
   __syncthreads();
@@ -1044,7 +1046,7 @@ int quant_pack_impl(const void *x, const void *x1, int x_dtype, const int64_t *h
                     int asym, float eps, int32_t *words, int8_t *codes, float *scale, float *zp,
                     int32_t *words1, int8_t *codes1, float *scale1, float *zp1,
                     const int64_t *host_out_map, void *workspace, size_t workspace_bytes, void *stream,
-                    StepOut *step = nullptr, int64_t step_pairs = 0, const int64_t *host_scale_map = nullptr) {
+                    StepOut *step = nullptr, int64_t step_pairs = 0, const int64_t *host_scale_map = nullptr, float *const *once = nullptr) {
   VARQ_CHECK_ARG(host_shape4, "quant_pack: null shape");
   const int64_t *s = host_shape4;
   VARQ_CHECK_ARG(s[0] >= 0 && s[1] >= 0 && s[2] >= 0 && s[3] > 0 && s[3] <= (1 << 20), "quant_pack: bad shape");
@@ -1095,9 +1097,11 @@ int quant_pack_impl(const void *x, const void *x1, int x_dtype, const int64_t *h
     // (places counted in 32 bits, times the 512 groups that a workgroup has at most)
     if (m[4] > (1 << 22) || m[4] * m[5] > (1 << 22))
       return varq_set_error(VARQ_ERR_UNSUPPORTED, "quant_pack: scales are spread over at most 4 million places each");
-    p.spread = {1, FastDiv::by(m[0]), FastDiv::by(m[4]), (u32)std::min(m[0], (int64_t)0x7fffffff), (u32)m[4], (u32)(m[4] * m[5]), m[1], m[2], m[3], m[6]};
+    VARQ_CHECK_ARG(!once || !once[0] || ((!asym || once[1]) && (!x1 || (once[2] && (!asym || once[3])))), "quant_pack: scales once per group come with zero-points, and for both tensors");
+    p.spread = {1, FastDiv::by(m[0]), FastDiv::by(m[4]), (u32)std::min(m[0], (int64_t)0x7fffffff), (u32)m[4], (u32)(m[4] * m[5]), m[1], m[2], m[3], m[6],
+                once ? once[0] : nullptr, once ? once[1] : nullptr, once ? once[2] : nullptr, once ? once[3] : nullptr};
   }
-  p.n0 = s[0]; p.n1 = s[1]; p.n2 = s[2];
+  p.n1 = s[1]; p.n2 = s[2];
   p.c = (int)s[3];
   p.keepc = !(reduce_mask & 8);
   // group-id strides of the kept leading dims, row-major over the kept dims
@@ -1108,10 +1112,6 @@ int quant_pack_impl(const void *x, const void *x1, int x_dtype, const int64_t *h
   p.rows = rows;
   p.n_groups = ng;
   p.c8 = (p.c + 7) / 8;
-  int c8p = 1, sh = 0;
-  while (c8p < p.c8) { c8p <<= 1; ++sh; }
-  p.c8p = c8p; p.c8p_shift = sh;
-  p.rows_per_block = 0;
   p.bits = bits; p.qmin = -(1 << (bits - 1)); p.qmax = (1 << (bits - 1)) - 1;
   p.wpr = words ? (p.c + 32 / bits - 1) / (32 / bits) : 0;
   p.asym = asym ? 1 : 0;
@@ -1178,12 +1178,21 @@ extern "C" int varq_quant_pack2(const void *x0, const void *x1, int x_dtype, con
                          words1, codes1, scale1, zp1, host_out_map, workspace, workspace_bytes, stream);
 }
 
+extern "C" int varq_quant_pack_spread_once(const void *x0, const void *x1, int x_dtype, const int64_t *host_shape4, int reduce_mask, int bits, int asym,
+                                           float eps, int32_t *words0, float *scale0, float *zp0, int32_t *words1, float *scale1, float *zp1,
+                                           float *once_scale0, float *once_zp0, float *once_scale1, float *once_zp1,
+                                           const int64_t *host_out_map, const int64_t *host_scale_map, void *stream) {
+  VARQ_CHECK_ARG(host_scale_map, "quant_pack_spread: null scale map");
+  float *const once[4] = {once_scale0, once_zp0, once_scale1, once_zp1};
+  return quant_pack_impl(x0, x1, x_dtype, host_shape4, reduce_mask, bits, asym, eps, words0, nullptr, scale0, zp0, words1, nullptr, scale1, zp1,
+                         host_out_map, nullptr, 0, stream, nullptr, 0, host_scale_map, once);
+}
+
 extern "C" int varq_quant_pack_spread(const void *x0, const void *x1, int x_dtype, const int64_t *host_shape4, int reduce_mask, int bits, int asym,
                                       float eps, int32_t *words0, float *scale0, float *zp0, int32_t *words1, float *scale1, float *zp1,
                                       const int64_t *host_out_map, const int64_t *host_scale_map, void *stream) {
-  VARQ_CHECK_ARG(host_scale_map, "quant_pack_spread: null scale map");
-  return quant_pack_impl(x0, x1, x_dtype, host_shape4, reduce_mask, bits, asym, eps, words0, nullptr, scale0, zp0, words1, nullptr, scale1, zp1,
-                         host_out_map, nullptr, 0, stream, nullptr, 0, host_scale_map);
+  return varq_quant_pack_spread_once(x0, x1, x_dtype, host_shape4, reduce_mask, bits, asym, eps, words0, scale0, zp0, words1, scale1, zp1,
+                                     nullptr, nullptr, nullptr, nullptr, host_out_map, host_scale_map, stream);
 }
 
 // Quantizes a step into its tokens of the cache buffer and dequantizes the whole cache: in one launch where the step

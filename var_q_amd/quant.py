@@ -143,13 +143,10 @@ class VAR_Q:
         w = self._window
         if w is not None:
             self._window = None
-            buf, dim, start, n, scales, zps, k, shape = w
-            self._current = [buf.narrow(dim, start, n)]
-            for t in (scales, zps):
-                if t is not None:            # the step's row of the tables, or its tokens of the scales per token
-                    t = t.narrow(dim, start, n) if k < 0 else t[k].unsqueeze(0).unsqueeze(dim)
-                    t = t[tuple(slice(m) for m in shape)]
-                self._current.append(t)
+            buf, dim, start, n, scale, zp, k, shape = w
+            if k >= 0:                       # the step's row of the tables (the shipped rule); else the tensors themselves
+                scale, zp = scale[k].view(shape), None if zp is None else zp[k].view(shape)
+            self._current = [buf.narrow(dim, start, n), scale, zp]
         return self._current
 
     @property
