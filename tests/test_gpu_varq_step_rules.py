@@ -53,3 +53,31 @@ def test_same_state_as_the_general_calls(dev, method, layout, B, H, c, bits, sym
             for name in ('quantized_item', 'scale', 'zp', 'cached_item', 'cached_scale', 'cached_zp'):
                 _same(getattr(a, name), getattr(b, name))
             assert a._seg_ends == b._seg_ends and a._scale_shape == b._scale_shape and a._pack_meta == b._pack_meta
+
+
+@pytest.mark.parametrize('layout', ['BLHc', 'BHLc'])
+@pytest.mark.parametrize('symmetric', [True, False])
+@pytest.mark.parametrize('c', [4, 12, 20, 100])
+def test_channels_that_are_no_whole_octets(dev, layout, symmetric, c):
+    """The shipped rule at 8 bits takes whole words of channels in one call: alone, both tensors of a step, and with the cache
+    dequantized; the state is that of quant() and cache(), past the steps that the tables hold too."""
+    g = torch.Generator().manual_seed(c)
+    make = lambda: VAR_Q(8, layout, symmetric=symmetric)
+    alone, pair, used, general = make(), [make(), make()], make(), [make(), make()]
+    for i in range(18):
+        n = (3, 1, 70)[i % 3]
+        shape = (2, n, 3, c) if layout == 'BLHc' else (2, 3, n, c)
+        k, v = [torch.randn(*shape, generator=g).to(dev) for _ in range(2)]
+        note('step of', c, 'channels', layout, symmetric, i)
+        took = [alone._step_fast(k), VAR_Q._step_fast_pair(*pair, k, v)]
+        assert took == [i < 16] * 2
+        for z, x in zip([alone, *pair][0 if i >= 16 else 3:] + general, (k, k, v, k, v)[0 if i >= 16 else 3:]):
+            z.quant(x)
+            z.cache()
+        _same(used.use_var_q(k), general[0].dequant_all())
+        for a, b in ((alone, general[0]), (pair[0], general[0]), (pair[1], general[1]), (used, general[0])):
+            for name in ('quantized_item', 'scale', 'zp', 'cached_item', 'cached_scale', 'cached_zp'):
+                _same(getattr(a, name), getattr(b, name))
+            _same(a.dequant_current(), b.dequant_current())
+            _same(a.dequant_all(), b.dequant_all())
+            assert a._seg_ends == b._seg_ends and a._scale_shape == b._scale_shape and a._pack_meta == b._pack_meta

@@ -849,7 +849,7 @@ struct Quantizer {
   bool takes(PyObject *x) const {
     if (!ready || rule == Rule::kOtherTable || rule == Rule::kOtherToken || !THPVariable_Check(x)) return false;
     const at::Tensor &t = THPVariable_Unpack(x);
-    if (!t.is_cuda() || t.device() != buf->device() || t.dim() != 4 || !t.is_contiguous() || t.numel() == 0 || c % 8 != 0) return false;
+    if (!t.is_cuda() || t.device() != buf->device() || t.dim() != 4 || !t.is_contiguous() || t.numel() == 0 || (c % 8 != 0 && rule != Rule::kHeadDim)) return false;
     if (t.scalar_type() != at::kFloat && t.scalar_type() != at::kBFloat16 && t.scalar_type() != at::kHalf) return false;
     if (t.size(0) != buf->size(0) || t.size(3 - d) != heads() || t.size(3) != c || len + t.size(d) > buf->size(d)) return false;
     return per_token(rule) ? scale->size(3) == 1 : k < 16 && k < scale->size(0);
@@ -896,6 +896,10 @@ struct Quantizer {
     set_attribute(o, NAME(_window), Py_BuildValue("(OLLLOOLO)", buf.o, (long long)d, (long long)len, (long long)n, s.o, z.o, (long long)(once ? -1 : k), sshape.o));
     Py_INCREF(Py_None);
     set_attribute(o, NAME(_staged), Py_None);
+    if (c % 8) {   // (rows that are no whole octets are not dequantized through the tables: see _keep_scales)
+      const Ref tokens_n(PyLong_FromLongLong(n)), channels(PyLong_FromLongLong(c));
+      Ref(PyObject_CallMethodObjArgs(o, NAME(_keep_scales), tokens_n.o, channels.o, nullptr));
+    }
     Py_INCREF(sshape.o);
     set_attribute(o, NAME(_scale_shape), sshape.o);
     set_attribute(item.o, NAME(len), PyLong_FromLongLong(len + n));
@@ -959,7 +963,7 @@ PyObject *quantizer_step(PyObject *const *a) {
 // quantizer_use(quantizer, x, out dtype code) -> the dequantized cache with the step behind the earlier ones (the shipped rule), or None
 PyObject *quantizer_use(PyObject *const *a) {
   const Quantizer z(a[0]);
-  if (z.rule != Rule::kHeadDim || !z.takes(a[1]) || z.last_end() != z.len) Py_RETURN_NONE;
+  if (z.rule != Rule::kHeadDim || !z.takes(a[1]) || z.c % 8 != 0 || z.last_end() != z.len) Py_RETURN_NONE;
   const at::Tensor &x = THPVariable_Unpack(a[1]);
   const int64_t d = z.d, n = x.size(d), B = x.size(0), H = z.heads(), c = z.c, code = integer(a[2]);
   if ((uintptr_t)x.data_ptr() & 15 || (z.len + n) * (d == 1 ? H : 1) * (c / 8) >= (1ll << 31) - 2048) Py_RETURN_NONE;

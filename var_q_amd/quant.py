@@ -322,7 +322,7 @@ class VAR_Q:
         item, d = self._c_item, self.dim_cat
         s0, s1, s2, c = x.shape
         vals = 32 // bits
-        if item.dim != d or len(self._seg_ends) >= MAX_TABLE_STEPS or c % vals or c % 8 or s0 * s1 * s2 == 0:
+        if item.dim != d or len(self._seg_ends) >= MAX_TABLE_STEPS or c % vals or s0 * s1 * s2 == 0:
             return False                      # (quant() says why an empty step is refused)
         meta = self._pack_meta
         if meta is None:
