@@ -183,17 +183,22 @@ template <bool F16> __device__ __forceinline__ floatx4_t mfma_16x16x32(u32x4_t a
 // A wavefront copies N KiB from global memory (`src`: the lane's 16 bytes of the first) to LDS, from address `dst` on,
 // past the registers.  The compiler does not count these loads: wait_copies<N> waits until at most the N KiB last asked
 // for are under way.
+// (m0 is written here and named for it: the compiler sets it for instructions of its own and may take a value to be still there.  It
+// warns of every reserved register that is named.)
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"
 template <int N> __device__ __forceinline__ void to_lds(const char *src, u32 dst) {
   static_assert(N == 1 || N == 2 || N == 4, "N");
   dst = __builtin_amdgcn_readfirstlane(dst);
   if constexpr (N == 1)
-    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(src), "s"(dst) : "memory");
+    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(src), "s"(dst) : "m0", "memory");
   else if constexpr (N == 2)
-    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off\n\tglobal_load_lds_dwordx4 %0, off offset:1024" ::"v"(src), "s"(dst) : "memory");
+    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off\n\tglobal_load_lds_dwordx4 %0, off offset:1024" ::"v"(src), "s"(dst) : "m0", "memory");
   else
     asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off\n\tglobal_load_lds_dwordx4 %0, off offset:1024\n\t"
-                 "global_load_lds_dwordx4 %0, off offset:2048\n\tglobal_load_lds_dwordx4 %0, off offset:3072" ::"v"(src), "s"(dst) : "memory");
+                 "global_load_lds_dwordx4 %0, off offset:2048\n\tglobal_load_lds_dwordx4 %0, off offset:3072" ::"v"(src), "s"(dst) : "m0", "memory");
 }
+#pragma clang diagnostic pop
 template <int N> __device__ __forceinline__ void wait_copies() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory"); }
 
 // Work comes in blocks of 256 queries (128: see wide_four) of one (batch, head), block bh * q_tiles + qt, and is dealt out to
