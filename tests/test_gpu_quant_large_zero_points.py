@@ -40,3 +40,18 @@ def test_step_and_cache(dev, bits):
         steps.cache()
         assert torch.equal(one.use_var_q(x), steps.dequant_all(torch.float32)) and torch.equal(one.cached_item, steps.cached_item)
         assert torch.equal(one.cached_zp, steps.cached_zp) and float(one.cached_zp.abs().max()) > 2 ** 21
+
+
+@pytest.mark.parametrize('bits', [2, 4, 8])
+@pytest.mark.parametrize('shape', [(2, 4, 70, 64), (300, 4, 33, 64)])      # one launch; three
+def test_quotients_up_to_the_largest_float(dev, shape, bits):
+    """Constant groups, whose scale is eps: values over eps up to where a product with the reciprocal may pass the largest float and the
+    quotient does not."""
+    eps, largest = 1e-12, torch.finfo(torch.float32).max
+    x = torch.tensor([1e13, -2.0 ** 79, 2.0 ** 81, -largest * eps * 0.99999]).view(1, 4, 1, 1).expand(shape).contiguous()
+    q, s, z = O.quant_reduce(x, (0, 2), bits, True, eps)
+    assert bool(torch.isfinite(z).all()) and float(z.abs().max()) > 2.0 ** 127
+    note('quotients up to the largest float', shape, bits)
+    words, gs, gz = ops.quant_pack(x.to(dev), (0, 2), bits, asym=True, eps=eps)
+    assert torch.equal(gs.cpu().reshape(s.shape), s) and torch.equal(gz.cpu().reshape(z.shape), z)
+    assert torch.equal(words.cpu(), O.pack_last_dim(q, bits)[0])

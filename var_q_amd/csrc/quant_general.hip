@@ -336,12 +336,22 @@ __global__ __launch_bounds__(256) void finalize_tiled_kernel(GenParams p, int Z,
   }
   p.scale[g] = s;
   rinv[g] = 1.0f / s;
-  // x/s == RN(q0 + (x - q0*s)*r) with q0 = RN(x*r), r = RN(1/s), for every finite x unless the
-  // significand of s is all ones or the residual can underflow
-  // (nor may the zero-point be too large for the rounding trick of FastOctet)
-  plain[g] = (s > 0x1p-96f && s < 0x1p96f && (f2u(s) & 0x7fffffu) != 0x7fffffu && fabsf(z) <= 0x1p21f) ? 1u : 0u;
+  // whether exact_quotient holds (about x/s = -zp: the values of a group may lie far from 0 in a narrow range)
+  plain[g] = (s > 0x1p-96f && s < 0x1p96f && (f2u(s) & 0x7fffffu) != 0x7fffffu && fabsf(z) <= 0x1p120f) ? 1u : 0u;
 }
 
+// x/s == RN(q0 + (x - q0*s)*r) with q0 = RN(x*r), r = RN(1/s), for every finite x unless the significand of s is all ones, the
+// residual can underflow or the quotient comes near the largest float
+__device__ __forceinline__ float exact_quotient(float x, float s, float r) {
+  const float q0 = x * r;
+  return __builtin_fmaf(__builtin_fmaf(-q0, s, x), r, q0);
+}
+// The codes of an octet by division
+template <int NV>
+__device__ __forceinline__ void divided(const float (&v)[8], const float (&s)[NV], const float (&z)[NV], float qmin, float qmax, int (&q)[8]) {
+#pragma unroll
+  for (int j = 0; j < 8; ++j) q[j] = (int)__builtin_amdgcn_fmed3f(rintf(v[j] / s[j % NV]) + z[j % NV], qmin, qmax);
+}
 // Quantizes and stores one octet (column `col`) of row `row`: s, z the scale and the zero-point of the octet's groups (one per channel or one).
 // also(codes): what else the caller wants from them.
 struct Nothing { __device__ __forceinline__ void operator()(const int (&)[8]) const {} };
@@ -368,16 +378,13 @@ __device__ __forceinline__ void store_codes(const GenParams &p, int64_t row, int
 template <int NV, class F = Nothing>
 __device__ __forceinline__ void store_octet(const GenParams &p, int64_t row, int col, const float (&v)[8], const float (&s)[NV],
                                             const float (&z)[NV], F &&also = F()) {
-  const float qmin = (float)p.qmin, qmax = (float)p.qmax;
-  const u32 mask = (1u << p.bits) - 1u;
   int q[8];
-#pragma unroll
-  for (int j = 0; j < 8; ++j) q[j] = (int)__builtin_amdgcn_fmed3f(rintf(v[j] / s[j % NV]) + z[j % NV], qmin, qmax);
+  divided<NV>(v, s, z, (float)p.qmin, (float)p.qmax, q);
   also(q);
-  store_codes(p, row, col, q, mask);
+  store_codes(p, row, col, q, (1u << p.bits) - 1u);
 }
 
-// The groups of one octet (one per channel or one) where all scales allow the exact quotient shortcut and the zero-points are
+// The groups of one octet (one per channel or one) where all scales allow exact_quotient and the zero-points are
 // below 2^21: clamp(rint(t) + z, qmin, qmax) = rint(clamp(t, qmin - z, qmax - z)) + z, adding 1.5 * 2^23 rounds to nearest-even and leaves
 // the integer in the low bits, four of them are a dword of bytes, and the zero-points are added to its bytes at once.  About eight
 // instructions per element with the conversion; store_octet takes twelve, and the quantizing kernels are bound by their number as
@@ -401,9 +408,7 @@ template <int NV, bool ASYM> struct FastOctet {
   // number(j): the code of v[j] less its zero-point, in the low bits of a float of 1.5 * 2^23
   __device__ __forceinline__ float number(float x, int j) const {
     const int n = j % NV;
-    const float q0 = x * r[n];
-    const float t = __builtin_fmaf(__builtin_fmaf(-q0, s[n], x), r[n], q0);
-    return __builtin_amdgcn_fmed3f(t, lo[n], ASYM ? lo[n] + span : hi) + 12582912.f;
+    return __builtin_amdgcn_fmed3f(exact_quotient(x, s[n], r[n]), lo[n], ASYM ? lo[n] + span : hi) + 12582912.f;
   }
   __device__ __forceinline__ u32 bytes(const float (&u)[8], int h) const {
     const u32 a = __builtin_amdgcn_perm(f2u(u[4 * h + 1]), f2u(u[4 * h]), 0x0c0c0400u), b = __builtin_amdgcn_perm(f2u(u[4 * h + 3]), f2u(u[4 * h + 2]), 0x0c0c0400u);
@@ -470,15 +475,9 @@ __global__ __launch_bounds__(256) void quant_tiled_kernel(GenParams p, Plan pl, 
     int q[8];
     if (fast) {
 #pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        const float sj = s[j % NV], rj = r[j % NV];
-        const float q0 = v[j] * rj;
-        const float t = __builtin_fmaf(__builtin_fmaf(-q0, sj, v[j]), rj, q0);
-        q[j] = (int)__builtin_amdgcn_fmed3f(rintf(t) + z[j % NV], qmin, qmax);
-      }
+      for (int j = 0; j < 8; ++j) q[j] = (int)__builtin_amdgcn_fmed3f(rintf(exact_quotient(v[j], s[j % NV], r[j % NV])) + z[j % NV], qmin, qmax);
     } else {
-#pragma unroll
-      for (int j = 0; j < 8; ++j) q[j] = (int)__builtin_amdgcn_fmed3f(rintf(v[j] / s[j % NV]) + z[j % NV], qmin, qmax);
+      divided<NV>(v, s, z, qmin, qmax, q);
     }
     store_codes(p, row, l.col, q, mask);
   });
@@ -594,7 +593,7 @@ __device__ __forceinline__ void quant_one_block(const GenParams &p, const OnePla
       s = fmaxf(m / (float)p.qmax, p.eps);
     }
     par_s[t] = s;
-    // (the exact-quotient shortcut, see finalize_tiled_kernel; 0: this group takes the division)
+    // (exact_quotient, where FastOctet's rounding holds the zero-point; 0: this group takes the division)
     par_r[t] = (s > 0x1p-96f && s < 0x1p96f && (f2u(s) & 0x7fffffu) != 0x7fffffu && fabsf(zp) <= 0x1p21f) ? 1.0f / s : 0.f;
     float *const once = KEEPC || !p.spread.on ? p.scale : p.spread.scale;
     if (mine && once) {
