@@ -7,7 +7,7 @@ import torch
 
 import varq_oracle as O
 from gpu_util import note
-from var_q_amd import _lib, ops
+from var_q_amd import VAR_Q, ops
 
 pytestmark = pytest.mark.gpu
 
@@ -59,17 +59,15 @@ def test_narrow_slices(dev, shape, dims, dtype):
     test_one_launch_edges(dev, shape, dims, dtype)
     g = torch.Generator().manual_seed(1)
     xs = [torch.randn(*shape, generator=g).to(dtype) for _ in range(2)]
-    tok = 1 if dims == (0, 1) else 2
-    H, c = shape[3 - tok], shape[3]
     for bits in (8, 4, 2):
-        if c * bits % 32:
+        if shape[3] * bits % 32:
             continue
-        pair = [[x.to(dev), torch.zeros(*shape[:3], c * bits // 32, dtype=torch.int32, device=dev), torch.zeros(16, H, c, device=dev), None] for x in xs]
+        pair = [VAR_Q(bits, 'BLHc' if dims == (0, 1) else 'BHLc') for _ in xs]
         note('quant one, two tensors', shape, dims, dtype, bits)
-        _lib.host().quant_step(0b0011 if tok == 1 else 0b0101, bits, False, 1e-12, tok, 0, 2, *pair[0], *pair[1])
-        for x, (_, words, tab, _) in zip(xs, pair):
+        assert VAR_Q._step_fast_pair(*pair, *[x.to(dev) for x in xs])
+        for x, z in zip(xs, pair):
             q, s, _ = O.quant_reduce(x, dims, bits, False)
-            assert torch.equal(words.cpu(), O.pack_last_dim(q, bits)[0]) and torch.equal(tab[2].cpu(), s.reshape(H, c))
+            assert torch.equal(z.cached_item.cpu(), O.pack_last_dim(q, bits)[0]) and torch.equal(z.scale.cpu(), s)
 
 
 @pytest.mark.parametrize('shape,dims,dtype', [

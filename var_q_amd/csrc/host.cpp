@@ -192,48 +192,6 @@ int pack_rows(const at::Tensor &x, const void *x1, int dt, const int64_t *sh, in
   return varq_quant_pack(x.data_ptr(), dt, sh, mask, bits, asym, eps, w0, nullptr, s[0], z[0], map, ws.data_ptr(), ws_bytes, stream_of(x));
 }
 
-// One step of a quantizer with a scale per (head, channel): codes into tokens start.. of the cache
-// buffer, scale and zero-point into row k of the step tables.
-// quant_step(mask, bits, asym, eps, token_dim, start, k, x, buf, tab, ztab | None [, x1, buf1, tab1, ztab1])
-// -> None; the second tensor (K and V of a step) goes through the same launches.
-PyObject *quant_step(PyObject *const *a, Py_ssize_t n_args) {
-  if (n_args != 11 && n_args != 15) need_args(n_args, 11, "quant_step");
-  const bool two = n_args == 15;
-  const int mask = (int)integer(a[0]);
-  const int64_t bits = integer(a[1]), d = integer(a[4]), start = integer(a[5]), k = integer(a[6]);
-  const bool asym = truth(a[2]);
-  const at::Tensor *x[2], *buf[2], *tab[2], *ztab[2];
-  for (int i = 0; i < (two ? 2 : 1); ++i) {
-    x[i] = &gpu(a[7 + 4 * i], "x");
-    buf[i] = &gpu(a[8 + 4 * i], "buffer");
-    tab[i] = &gpu(a[9 + 4 * i], "scale table");
-    ztab[i] = maybe(a[10 + 4 * i], "zero-point table");
-    const at::Tensor &t = *x[i], &b = *buf[i];
-    ASSERT(t.dim() == 4 && t.is_contiguous() && b.dim() == 4 && b.is_contiguous() && b.scalar_type() == at::kInt && tab[i]->is_contiguous() &&
-               t.sizes() == x[0]->sizes() && t.scalar_type() == x[0]->scalar_type() && b.sizes() == buf[0]->sizes(), "quant_step: operands");
-    ASSERT((!asym || ztab[i]) && b.size(3) * 32 == t.size(3) * bits && start >= 0 && start + t.size(d) <= b.size(d) &&
-               b.size(0) == t.size(0) && b.size(3 - d) == t.size(3 - d), "quant_step: buffers");
-    const int64_t row = t.size(d == 1 ? 2 : 1) * t.size(3);
-    ASSERT(k >= 0 && (k + 1) * row <= tab[i]->numel() && tab[i]->scalar_type() == at::kFloat, "quant_step: tables");
-  }
-  const at::Tensor &t = *x[0];
-  const int64_t sh[4] = {t.size(0), t.size(1), t.size(2), t.size(3)};
-  const int64_t per_tok = d == 1 ? sh[2] : 1, row = sh[d == 1 ? 2 : 1] * sh[3];
-  const int64_t map[3] = {sh[d] * per_tok, (buf[0]->size(d) - sh[d]) * per_tok, start * per_tok};
-  const c10::DeviceGuard guard(t.device());
-  const int dt = dtype_code(t);
-  const float eps = (float)real(a[3]);
-  float *s[2] = {}, *z[2] = {};
-  for (int i = 0; i < (two ? 2 : 1); ++i) {
-    s[i] = ptr<float>(tab[i]) + k * row;
-    z[i] = asym ? ptr<float>(ztab[i]) + k * row : nullptr;
-  }
-  unlocked("varq_quant_pack", [&] {
-    return pack_rows(t, two ? x[1]->data_ptr() : nullptr, dt, sh, mask, (int)bits, asym, eps, ptr<int32_t>(buf[0]), two ? ptr<int32_t>(buf[1]) : nullptr, s, z, map);
-  });
-  Py_RETURN_NONE;
-}
-
 // ---- pack / unpack of int8 codes ----------------------------------------------------------------
 int64_t codes_per_word(int64_t bits) {
   ASSERT(bits == 2 || bits == 4 || bits == 8, "bits must be 2, 4 or 8 (got %lld)", (long long)bits);
@@ -1016,11 +974,6 @@ template <PyObject *(*F)(PyObject *const *), int N> PyObject *fixed(PyObject *, 
   return F(a);
   END_HANDLE_TH_ERRORS
 }
-template <PyObject *(*F)(PyObject *const *, Py_ssize_t)> PyObject *varying(PyObject *, PyObject *const *a, Py_ssize_t n) {
-  HANDLE_TH_ERRORS
-  return F(a, n);
-  END_HANDLE_TH_ERRORS
-}
 PyObject *set_error(PyObject *, PyObject *e) {
   Py_INCREF(e);
   Py_XDECREF(g_varq_error);
@@ -1032,7 +985,6 @@ PyObject *set_error(PyObject *, PyObject *e) {
 PyMethodDef g_methods[] = {
     FIXED(quant_rows, 5), FIXED(quant_shared, 6), FIXED(pack, 2), FIXED(unpack, 3), FIXED(dequant, 6), FIXED(dequant_steps, 8), FIXED(attn, 18), FIXED(attn_channel, 17),
     FIXED(cache_attend, 9), FIXED(cache_append, 5), FIXED(cache_prepare, 9),
-    {"quant_step", (PyCFunction)(void (*)(void))varying<quant_step>, METH_FASTCALL, nullptr},
     FIXED(quantizer_step, 4), FIXED(quantizer_use, 3), FIXED(quantizer_attend, 6),
     {"set_error", set_error, METH_O, nullptr},
     {nullptr, nullptr, 0, nullptr}};

@@ -356,7 +356,6 @@ __device__ __forceinline__ void divided(const float (&v)[8], const float (&s)[NV
 }
 // Quantizes and stores one octet (column `col`) of row `row`: s, z the scale and the zero-point of the octet's groups (one per channel or one).
 // also(codes): what else the caller wants from them.
-struct Nothing { __device__ __forceinline__ void operator()(const int (&)[8]) const {} };
 __device__ __forceinline__ void store_codes(const GenParams &p, int64_t row, int col, const int (&q)[8], u32 mask) {
   const int64_t orow = out_row32(p, row);
   if (p.codes || p.bits == 8) {
@@ -377,9 +376,9 @@ __device__ __forceinline__ void store_codes(const GenParams &p, int64_t row, int
     }
   }
 }
-template <int NV, class F = Nothing>
+template <int NV, class F>
 __device__ __forceinline__ void store_octet(const GenParams &p, int64_t row, int col, const float (&v)[8], const float (&s)[NV],
-                                            const float (&z)[NV], F &&also = F()) {
+                                            const float (&z)[NV], F &&also) {
   int q[8];
   divided<NV>(v, s, z, (float)p.qmin, (float)p.qmax, q);
   also(q);
