@@ -1320,8 +1320,6 @@ template <int D, bool F16> void launch_combine(const AttnParams &p, hipStream_t 
     hipLaunchKernelGGL((combine_splits_kernel<D, F16>), dim3((unsigned)((rows + 1) / 2)), dim3(256), 0, st, p);
 }
 
-int device_cus();
-
 template <int D, int BITS, int GK, int GV, bool CHAN, int NWV, int WPS = 2, bool EXACT = false, bool F16 = false, bool ONE = false>
 void launch_shape(const AttnParams &p, hipStream_t st) {
   // (the per-channel tables take LDS by the number of segments of the launch)
@@ -1436,18 +1434,6 @@ int set_layout(AttnParams &p, int layout, const char *who) {
 
 // ---- sharing the keys of a query block out over several workgroups ---------------------
 constexpr int kMaxSplits = kMaxSplits_v;
-
-int device_cus() {
-  static int cus[64] = {0};
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
-  if (!cus[dev]) {
-    int n = 0;
-    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) n = 256;
-    cus[dev] = n;
-  }
-  return cus[dev];
-}
 
 size_t split_workspace_bytes(int splits, int64_t rows, int D) {
   return splits > 1 ? (size_t)splits * (size_t)rows * (size_t)(D + 2) * sizeof(float) : 0;

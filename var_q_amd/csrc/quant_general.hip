@@ -855,11 +855,11 @@ bool make_plan(const int64_t *sh, int reduce_mask, int64_t n_groups, Plan &pl) {
 bool one_launch_pays(const OnePlan &pl, int c8, int c8p, int threads, bool keepc, double mib, int elem, int tensors, bool asym, bool with_values) {
   if (!keepc) return mib <= (asym ? 16 : 48);
   if (threads == 256) return mib <= 16;
-  const int64_t wgs = (int64_t)pl.blocks * pl.slices * tensors;
+  const int64_t wgs = (int64_t)pl.blocks * pl.slices * tensors, cus = device_cus();
   const int piece = (8 * elem) << pl.c8s_shift;
   const bool apart = pl.RI == 1 && pl.ro_rs * c8 * 8 * elem % 1024 == 0;
   const double per_kib = piece <= 16 ? (wgs <= 128 ? 0.175 : 0.22) : piece == 32 ? (apart ? 0.17 : 0.135) : 0.10;
-  const double one = 4.5 + per_kib * (asym ? 1.1 : 1.0) * mib * 1024.0 / (double)wgs * (double)((wgs + 255) / 256);
+  const double one = 4.5 + per_kib * (asym ? 1.1 : 1.0) * mib * 1024.0 / (double)wgs * (double)((wgs + cus - 1) / cus);
   const double three = (tensors == 2 ? 16.2 + 0.41 * mib * c8p / c8 : 12.4 + 0.44 * mib * c8p / c8) + (asym ? 3.0 : 0.0) + (with_values ? 10.5 : 0.0);
   return one < three;
 }

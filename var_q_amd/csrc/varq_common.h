@@ -11,6 +11,7 @@
 
 // ---- host-side error plumbing -------------------------------------------
 int varq_set_error(int code, const char *fmt, ...);
+int device_cus();   // compute units of the current device
 
 #define VARQ_CHECK_ARG(cond, ...)                                   \
   do {                                                              \
