@@ -980,11 +980,14 @@ int run_tiled(GenParams &p, const Plan &pl, void *workspace, hipStream_t st) {
   // per thread measured alike, longer ones slower)
   const Plan &pb = pl;
   dim3 bgrid((unsigned)((int64_t)pb.nko * pb.tilesQ * pb.Z), nt);
-  // Five workgroups on a compute unit instead of eight (by LDS that they do not use) where the Infinity Cache does not hold a tensor
-  // with long groups: fewer chunks are read at once, and more of the second read comes out of it.  Eight / five, us for the three launches:
-  // [64,30,680,128] bf16, a scale per (head, channel) 219 / 202, 4 bits affine 207 / 188, one scale for [32,30,680,64] fp32 75.6 / 72.8; at half the size it
-  // turns round, [32,30,680,64] bf16 with its dequantization behind it 60.6 / 63.6.
-  const bool large = !p.x1 && p.rows * p.c * In8<DT>::kBytes >= (128ll << 20) && pl.Z >= 16;
+  // Five workgroups on a compute unit instead of eight (by LDS that they do not use) for large tensors of 32 bits with long
+  // groups: fewer chunks are read at once, and more of the second read comes out of the Infinity Cache.  Eight / five, us for the three
+  // launches on tensors in turn, a scale per (head, channel), 8 bits, then 4 bits affine: [B,30,680,64] fp32, 80 MiB 43.1 / 43.7, 43.6 / 44.3; 120 62.0 / 61.5,
+  // 59.0 / 59.1; 194 94.6 / 91.9, 87.8 / 86.7; 264 139 / 133, 130 / 122; 319 170 / 164, 160 / 150; 398 209 / 208, 195 / 193; 702 364 / 358, 328 / 315; [B,30,680,128]
+  // the same, one scale for all of it 319 MiB 168 / 162, 156 / 147; the same tensor again and again, its dequantization behind it, 1-3 % at all of them.  Tensors of
+  // 16 bits, whose launch has more instructions per byte, lose by it up to 256 MiB and go either way beyond: bf16 120 MiB 70.7 / 73.3, 65.9 / 70.1; 159
+  // 91.0 / 93.3, 82.0 / 89.7; 192 109 / 114, 98 / 101; 264 174 / 164, 164 / 154 (D=128 154 / 154, 139 / 145); 401 233 / 238, 222 / 225; 513 339 / 318, 320 / 297 (292 / 294, 274 / 277).
+  const bool large = DT == VARQ_F32 && !p.x1 && p.rows * p.c * In8<DT>::kBytes >= (128ll << 20) && pl.Z >= 16;
   const unsigned lds = large ? 32000 : 0;
   if (p.asym) {
     if (p.keepc) hipLaunchKernelGGL((quant_tiled_kernel<DT, true, true>), bgrid, dim3(256), lds, st, p, pb, rinv, plain);
