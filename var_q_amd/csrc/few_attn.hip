@@ -14,7 +14,9 @@
 //    eight keys of every one of its channels: matrix instruction m takes channel m of every lane.  Row r of its
 //    result is channel (D / 16) r + m, and the order is undone at the end, when the wavefronts' results are put together.
 // K and V enter the products as (code - zp) * scale in fp32 rounded to the attention's 16-bit type, the operands that
-// the other kernels have.  Online softmax per lane against a reference that moves only when a weight would pass 2^16
+// the other kernels have -- but for V of a group whose zero-point is no whole number or beyond +-896: there (code - near) * scale is rounded,
+// near the whole number within +-896 next to the zero-point, and (near - zp) * scale, the same for all channels of the group, is summed with the weights in
+// fp32 and added to the result (another operand, nearer to the unrounded value).  Online softmax per lane against a reference that moves only when a weight would pass 2^16
 // (2^15 in fp16).
 // The wavefronts' partial results meet in LDS, the workgroups' shares of the keys in the workspace (combine_splits_kernel).
 //

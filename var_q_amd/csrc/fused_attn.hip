@@ -1526,8 +1526,9 @@ void set_few(AttnParams &p, int D, int k_group, int v_group, void *workspace, si
   p.nsplit = n;
   p.fq_share_blocks = ((p.Lk + kFewBlock - 1) / kFewBlock + n - 1) / n;
   // Eight wavefronts instead of four halve the chain of blocks of a share; where several workgroups run on a compute unit they
-  // only cost registers (two columns of queries: one workgroup instead of three).  Below 1024 keys the number of
-  // pairs does not matter, so that a pair's result does not depend on how many others the launch has.
+  // only cost registers (two columns of queries: one workgroup instead of three).  Below 1024 keys this does not go by the
+  // number of pairs.  A pair's result is then the same whatever others the launch has, bit for bit, up to 736 keys and 16 queries: from 24 blocks
+  // on fewq_shares goes by it, and beyond 16 queries fewq_eligible.
   const int nb = (p.Lk + kFewBlock - 1) / kFewBlock;
   const bool alone = nb < 32 ? p.Lq <= 16 : (int64_t)p.bh_total * p.q_tiles * n <= device_cus();
   p.few_waves = p.fq_share_blocks > 8 && alone ? 8 : 4;

@@ -848,8 +848,10 @@ bool make_plan(const int64_t *sh, int reduce_mask, int64_t n_groups, Plan &pl) {
 // [8,n,16,128] 36 30.2 / 28.4, 64 44.1 / 51.0; [64,n,16,64] 16 23.8 / 18.3, 25 25.4 / 27.8, 64 43.3 / 63.9; [4,8,n,128] 16 24.5 / 17.7, 25 25.7 / 27.0;
 // [64,n,8,64] 12.5 21.3 / 24.2; one tensor: [64,n,16,64] 8 17.0 / 15.9, 12.5 18.0 / 24.2; [32,n,30,64] 11.7 16.9 / 15.1, 20 20.6 / 23.9; [16,n,12,64]
 // 6 14.9 / 15.6, 9.4 15.7 / 23.9; [64,n,8,64] 6.2 15.8 / 22.9, 16 19.6 / 51.6; [2,16,n,128] 12.5 17.6 / 14.7, 18 19.3 / 20.6; fp32 [2,16,1600,128] 50 31.2 / 22.2.
-// (The line was 16 MiB in all.)  Groups of whole rows, one scale per (token, head), [32,30,L,64]: 20 MiB 18.6 / 15.6, 40 30.2 / 27.0, 80 48.0 / 50.1; with
-// zero-points two tensors of 40 29.0 / 35.4.  With the step dequantized in the same launch the other way has one
+// (The line was 16 MiB in all.)  Groups of whole rows keep to the sizes at which the one launch is never behind: up to 48 MiB symmetric, [32,30,L,64] bf16, one
+// scale per (token, head), 24 MiB 22.8 / 18.1, 32 24.0 / 23.9, 48 36.1 / 32.0, 64 37.8 / 42.3, two tensors 48 33.6 / 32.1, 64 38.1 / 44.6; affine up to 16, 8 MiB
+// 13.8 / 8.6, 16 17.0 / 17.2, 24 22.3 / 23.4, 48 33.9 / 42.8.  Other forms would gain beyond these lines: [64,16,L,64] fp16 64 MiB 37.7 / 31.1, affine 24
+// 22.5 / 17.8, 64 36.8 / 40.5; [8,16,L,128] fp32 96 MiB 45.5 / 32.4, affine 43.3 / 40.7; one scale per token, [32,30,L,64] bf16 96 62.0 / 51.6, affine 48 34.2 / 28.7.  With the step dequantized in the same launch the other way has one
 // more, whose work the one launch does beside: three and that / one, per tensor to fp32, [64,100,16,64] 40 / 74, [32,169,16,64] 41 / 64, [32,256,16,64]
 // 51 / 71, [32,12,256,64] 46 / 62, [64,100,8,64] 26 / 30, [32,169,30,64] 58 / 48, [16,256,8,128] 43 / 38, [32,100,16,64] 25 / 19.
 bool one_launch_pays(const OnePlan &pl, int c8, int c8p, int threads, bool keepc, double mib, int elem, int tensors, bool asym, bool with_values) {
