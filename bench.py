@@ -510,7 +510,8 @@ def hbm_regime_rates(torch, dev, kv_sets):
     over the whole packed cache of configuration 4 (INT4 group 128, B=2, H=16, 10 521 keys),
     Lq = 16 and 64, where the arithmetic intensity (4 * Lq flop per packed byte) is below or near
     the machine balance.  The four packed caches of the timed steps are cycled (4 x 48.5 MB of
-    codes, scales and zero-points), so the reads come from HBM.  Reports the time, the packed-KV
+    codes, scales and zero-points, which the 256 MiB Infinity Cache can hold; the longer and the INT8
+    caches, 776 and 366 MB, come from HBM).  Reports the time, the packed-KV
     GB/s and its fraction of the 8 TB/s peak, and how the keys were shared out."""
     from var_q_amd import _lib, ops
     lib = _lib.load()

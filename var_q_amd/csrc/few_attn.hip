@@ -20,11 +20,12 @@
 // (2^15 in fp16).
 // The wavefronts' partial results meet in LDS, the workgroups' shares of the keys in the workspace (combine_splits_kernel).
 //
-// What bounds it: 4-bit codes at D = 128 are 23 vector instructions per eight elements, 460 per block and wavefront with the
-// softmax and the addresses, most of them of the classes that issue once in four cycles; [7,8,41576,128], 2 queries: 73 us without the
+// What bounds it: 4-bit codes at D = 128 are 23 vector instructions per eight elements, 446 per block and wavefront with the
+// softmax and the addresses (and 520 per wavefront around the loop), most of them of the classes that issue once in four cycles: the vector ALU is busy for 0.64 of
+// the launch over [2,16,10521,128], 0.76 over four times as many keys; [7,8,41576,128], 2 queries: 73 us without the
 // loads of the loop, 68 us without the dequantization, 91 us whole (335 MB, 3.7 TB/s; INT8 121 us, 5.2 TB/s).  The kernel that this one replaced (32
 // queries to a wavefront, V transposed through LDS, one scale group at D = 128 only) took 140 and 167 us.  [2,16,10521,128], 16 queries, with the
-// launch that combines the shares: 28.4 -> 22.7 us; D = 64, [15,30,5049,64] 2-bit in groups of 32, 28 queries, on the kernel for many queries: 123 -> 62.
+// launch that combines the shares: 25.4 -> 20.6 us over one cache again and again, out of the Infinity Cache, 26.2 -> 21.9 over 24 in turn, out of HBM; D = 64, [15,30,5049,64] 2-bit in groups of 32, 28 queries, on the kernel for many queries: 123 -> 62.
 #include <type_traits>
 
 #include "attn_common.h"
