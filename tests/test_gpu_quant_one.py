@@ -75,6 +75,7 @@ def test_narrow_slices(dev, shape, dims, dtype):
     ((8, 400, 16, 128), (0, 1), torch.float16),       # two tensors: 25 MiB, one: 16-byte pieces
     ((3, 24, 701, 128), (0, 2), torch.bfloat16),
     ((5, 20, 333, 72), (0, 2), torch.float32),        # nine octets of sixteen lanes
+    ((6, 30, 1024, 128), (0, 2), torch.float32),      # 90 MiB, behind itself 180: fewer workgroups per compute unit in the second pass
     ((24, 6, 171, 64), (0, 2), torch.float16),        # few heads: one tensor is left to the three launches
     ((32, 30, 201, 64), (0, 3), torch.bfloat16),      # groups of whole rows: 24 MiB of one tensor, 47 of two
 ])
