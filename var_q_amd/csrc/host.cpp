@@ -844,14 +844,30 @@ struct Quantizer {
     return {1, rule == Rule::kTokenHead || (tokens && d == 1) || (!tokens && d == 2 && rule != Rule::kScale) ? s1 : 1,
             rule == Rule::kTokenHead || (tokens && d == 2) || (!tokens && d == 1 && rule != Rule::kScale) ? s2 : 1, rule == Rule::kHeadDim ? c : 1};
   }
-  // the state that quant() followed by cache() leaves, the kernels having written codes and scales in place; once: the step's
-  // scale and zero-point by themselves (undefined: its row of the step tables is they)
-  void commit(int64_t n, const at::Tensor *once = nullptr) const {
+  // Where the scale (and `half` behind it the zero-point) of a step of n tokens goes by itself, which is a caller's to change where the
+  // cache's copies are not: its stretch of a buffer with one for every token, or step, that the cache has room for (see VAR_Q._own_room).
+  // (A tensor for each took 0.9 us of the host apiece, of a step of 20.)
+  struct Own {
+    Held buf;
+    int64_t at, half;
+    float *data() const { return ptr<float>(buf) + at; }
+  };
+  bool own_place(Own &w, int64_t n) const {
+    const bool tokens = per_token(rule);
+    const int64_t per = rule == Rule::kTokenHead || rule == Rule::kHead ? heads() : 1, slots = tokens ? buf->size(d) : 16;
+    if (!tensor_of(w.buf, o, NAME(_own_scales), at::kFloat) || w.buf->device() != buf->device() || w.buf->numel() < slots * per * (asym ? 2 : 1)) return false;
+    w.at = (tokens ? len : k) * per;
+    w.half = w.buf->numel() / 2;
+    return true;
+  }
+  // the state that quant() followed by cache() leaves, the kernels having written codes and scales in place; own: where the step's
+  // scale and zero-point are by themselves (null: its row of the step tables is they)
+  void commit(int64_t n, const Own *own = nullptr) const {
     const bool tokens = per_token(rule);
     const auto shape = scale_shape(n);
     const Ref sshape(Py_BuildValue("(LLLL)", (long long)shape[0], (long long)shape[1], (long long)shape[2], (long long)shape[3]));
-    const Ref s(once ? wrap(once[0]) : Py_NewRef(scale.o)), z(!asym ? Py_NewRef(Py_None) : once ? wrap(once[1]) : Py_NewRef(zp.o));
-    set_attribute(o, NAME(_window), Py_BuildValue("(OLLLOOLO)", buf.o, (long long)d, (long long)len, (long long)n, s.o, z.o, (long long)(once ? -1 : k), sshape.o));
+    set_attribute(o, NAME(_window), Py_BuildValue("(OLLLOOLO)", buf.o, (long long)d, (long long)len, (long long)n, own ? own->buf.o : scale.o,
+                                                  !asym ? Py_None : own ? own->buf.o : zp.o, (long long)(own ? -1 - own->at : k), sshape.o));
     Py_INCREF(Py_None);
     set_attribute(o, NAME(_staged), Py_None);
     if (c % 8) {   // (rows that are no whole octets are not dequantized through the tables: see _keep_scales)
@@ -901,20 +917,18 @@ PyObject *quantizer_step(PyObject *const *a) {
   float *const s[2] = {at_row(kq.scale), two ? at_row(vq->scale) : nullptr}, *const z[2] = {at_row(kq.zp), two ? at_row(vq->zp) : nullptr};
   int64_t spread[7];
   if (!rows) kq.spread(n, spread);
-  at::Tensor once[2][2];   // [K, V][scale, zero-point] of the step by themselves: scale and zp are a caller's to change, the cache's copies are not
+  Quantizer::Own own[2];
+  if (!rows && (!kq.own_place(own[0], n) || (two && !vq->own_place(own[1], n)))) Py_RETURN_FALSE;
   const int rc = status_unlocked([&] {
     if (rows) return pack_rows(k, x1, dt, sh, mask, bits, asym, (float)eps, w0, w1, s, z, map);
-    const auto shape = kq.scale_shape(n);
-    for (int i = 0; i < (two ? 2 : 1); ++i)
-      for (int j = 0; j < (asym ? 2 : 1); ++j) once[i][j] = empty(shape, at::kFloat, k);
-    auto at_once = [&](int i, int j) { return once[i][j].defined() ? ptr<float>(once[i][j]) : nullptr; };
-    return varq_quant_pack_spread_once(k.data_ptr(), x1, dt, sh, mask, bits, asym, (float)eps, w0, s[0], z[0], w1, s[1], z[1], at_once(0, 0), at_once(0, 1),
-                                       at_once(1, 0), at_once(1, 1), map, spread, stream_of(k));
+    float *const s0 = own[0].data(), *const s1 = two ? own[1].data() : nullptr;
+    return varq_quant_pack_spread_once(k.data_ptr(), x1, dt, sh, mask, bits, asym, (float)eps, w0, s[0], z[0], w1, s[1], z[1], s0, asym ? s0 + own[0].half : nullptr, s1,
+                                       asym && two ? s1 + own[1].half : nullptr, map, spread, stream_of(k));
   });
   if (!rows && rc == VARQ_ERR_UNSUPPORTED) Py_RETURN_FALSE;
   check(rc, "varq_quant_pack");
-  kq.commit(n, rows ? nullptr : once[0]);
-  if (two) vq->commit(n, rows ? nullptr : once[1]);
+  kq.commit(n, rows ? nullptr : &own[0]);
+  if (two) vq->commit(n, rows ? nullptr : &own[1]);
   Py_RETURN_TRUE;
 }
 

@@ -29,6 +29,7 @@ affine quantizer (attributes `zp`, `cached_zp`); quant_method 'G_GROUP' with
 without dequantizing them.
 GPU tensors only.
 """
+import math
 from typing import Dict, List, Optional, Tuple
 
 import torch
@@ -144,8 +145,11 @@ class VAR_Q:
         if w is not None:
             self._window = None
             buf, dim, start, n, scale, zp, k, shape = w
-            if k >= 0:                       # the step's row of the tables (the shipped rule); else the tensors themselves
+            if k >= 0:                       # the step's row of the tables (the shipped rule)
                 scale, zp = scale[k].view(shape), None if zp is None else zp[k].view(shape)
+            else:                            # ... or its stretch of the steps' own scales, zero-points from the middle on
+                at, count, half = -1 - k, math.prod(shape), scale.numel() // 2
+                scale, zp = scale.narrow(0, at, count).view(shape), None if zp is None else zp.narrow(0, half + at, count).view(shape)
             self._current = [buf.narrow(dim, start, n), scale, zp]
         return self._current
 
@@ -181,6 +185,7 @@ class VAR_Q:
         # [.., capacity, .., groups]) for the others.  _c_scale and _c_zp hold the scales as the
         # reference caches them only where those do not (see _shown)
         self._staged = None
+        self._own_scales: Optional[torch.Tensor] = None     # `scale` and `zp` of the native steps, stretch after stretch
         self._seg_ends: List[int] = []
         self._tab_scale: Optional[torch.Tensor] = None      # [MAX_TABLE_STEPS, H, c]
         self._tab_zp: Optional[torch.Tensor] = None
@@ -440,6 +445,21 @@ class VAR_Q:
             self._tok_scale.append(self.scale.expand(*shape))
             if self.zp is not None:
                 self._tok_zp.append(self.zp.expand(*shape))
+        self._own_room(H)
+
+    def _own_room(self, H: int):
+        """Room for `scale` and `zp` of the steps that the native call takes, by themselves: a stretch for every token, or step,
+        that the cache has room for, used by one step only."""
+        m, tokens = self.quant_method, self.quant_method in _TOKEN_METHODS
+        if m not in ('G_TOKEN', 'G_TOKEN_HEAD', 'G_SCALE', 'G_HEAD'):
+            return
+        n = (H if m in ('G_TOKEN_HEAD', 'G_HEAD') else 1) * (self._c_item.buf.size(self.dim_cat) if tokens else MAX_TABLE_STEPS)
+        n *= 1 if self.symmetric else 2
+        old = self._own_scales
+        if old is None or old.numel() < n or old.device != self._c_item.buf.device:
+            if old is not None:
+                old.record_stream(torch.cuda.current_stream(old.device))    # (written by steps of this stream, if not made on it)
+            self._own_scales = torch.empty(n, dtype=torch.float32, device=self._c_item.buf.device)
 
     # ---------------- dequantize ----------------
     def _dequant(self, q: torch.Tensor, scale: torch.Tensor, zp: Optional[torch.Tensor],
