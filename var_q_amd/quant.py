@@ -49,6 +49,13 @@ def _dim_map(qkv_format: str) -> Dict[str, Tuple[int, ...]]:
             'G_TOKEN_HEAD': (0, 3), 'G_SCALE': (0, 1, 2, 3), 'G_HEAD': (0, 2, 3), 'G_GROUP': (3,)}
 
 
+def _let_go(t: Optional[torch.Tensor]):
+    """For a buffer that is about to be replaced: its memory is used again only when what the current stream
+    has still to do with it is done (it may have been made on another stream)."""
+    if t is not None and t.is_cuda:
+        t.record_stream(torch.cuda.current_stream(t.device))
+
+
 class _Growable:
     """Buffer that grows along one dim; `view()` is the valid prefix."""
 
@@ -65,6 +72,7 @@ class _Growable:
             new = torch.empty(shape, dtype=t.dtype, device=t.device)
             if self.buf is not None and self.len:
                 new.narrow(self.dim, 0, self.len).copy_(self.buf.narrow(self.dim, 0, self.len))
+            _let_go(self.buf)
             self.buf = new
         self.buf.narrow(self.dim, self.len, n).copy_(t)
         self.len += n
@@ -84,10 +92,12 @@ class _Growable:
             new = torch.empty(shape, dtype=dtype, device=device)
             if self.buf is not None and self.len:
                 new.narrow(self.dim, 0, self.len).copy_(self.buf.narrow(self.dim, 0, self.len))
+            _let_go(self.buf)
             self.buf = new
         return self.buf
 
     def replace(self, t: torch.Tensor):
+        _let_go(self.buf)
         self.buf, self.len = t, t.size(self.dim)
 
     def view(self) -> Optional[torch.Tensor]:
@@ -457,8 +467,7 @@ class VAR_Q:
         n *= 1 if self.symmetric else 2
         old = self._own_scales
         if old is None or old.numel() < n or old.device != self._c_item.buf.device:
-            if old is not None:
-                old.record_stream(torch.cuda.current_stream(old.device))    # (written by steps of this stream, if not made on it)
+            _let_go(old)
             self._own_scales = torch.empty(n, dtype=torch.float32, device=self._c_item.buf.device)
 
     # ---------------- dequantize ----------------
