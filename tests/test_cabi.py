@@ -128,3 +128,16 @@ def test_missing_library_fails_loudly(monkeypatch, tmp_path):
     monkeypatch.setattr(_lib, 'LIB_PATH', str(tmp_path / 'nope.so'))
     with pytest.raises(_lib.VarqError, match='no fallback'):
         _lib.load()
+
+
+def test_scales_once_per_group_come_whole():
+    """varq_quant_pack_spread_once: with zero-points where there are some, and for both tensors."""
+    lib, i64, fake = _lib.load(), _lib.i64arr, ctypes.c_void_p(0x1000)
+    shape, spread = i64([2, 4, 3, 64]), i64([1, 1, 0, 0, 1, 1, 0])
+    def call(x1, asym, once, scale_map=spread):
+        w1 = fake if x1 else None
+        return lib.varq_quant_pack_spread_once(fake, fake if x1 else None, 0, shape, 0b1111, 8, asym, 1e-12, fake, fake, fake if asym else None, w1, w1,
+                                               w1 if asym else None, *once, None, scale_map, None)
+    for x1, asym, once in ((0, 1, (fake, None, None, None)), (1, 0, (fake, None, None, None)), (1, 1, (fake, fake, fake, None))):
+        assert call(x1, asym, once) == -1 and b'once per group' in lib.varq_last_error()
+    assert call(0, 0, (fake, None, None, None), None) == -1 and b'scale map' in lib.varq_last_error()
