@@ -213,6 +213,8 @@ class VAR_Q:
         """Size the cache buffers for n_tokens at their first allocation (an extension: the
         reference grows its cache by torch.cat, VAR_Q/quant.py:200-201; here the buffers double
         when they run out, and a caller that knows the schedule's length avoids those copies).
+        Needed where steps behind cached ones are recorded into a graph: a buffer that grows meanwhile is
+        copied, at every replay, out of memory that is given back when the recording ends.
         Takes effect for buffers not allocated yet."""
         self._reserved_tokens = int(n_tokens)
         for g in (self._tok_scale, self._tok_zp, self._c_item, self._c_scale, self._c_zp, self._c_deq):
