@@ -88,6 +88,31 @@ template <bool F16> __device__ __forceinline__ floatx16_t mfma_32x32x16(u32x4_t 
     return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, a), __builtin_bit_cast(bf16x8_t, b), c, 0, 0, 0);
   }
 }
+// The smallest or largest of the values of a wavefront's first ROWS rows of 16 lanes (the other rows hold copies), the same for all lanes.
+template <bool IS_MAX, int ROWS> __device__ __forceinline__ int wave_fold(int v) {
+  auto op = [](int a, int b) { return IS_MAX ? max(a, b) : min(a, b); };
+  v = op(v, __builtin_amdgcn_update_dpp(v, v, 0xb1, 0xf, 0xf, false));    // quad_perm:[1,0,3,2]
+  v = op(v, __builtin_amdgcn_update_dpp(v, v, 0x4e, 0xf, 0xf, false));    // quad_perm:[2,3,0,1]
+  v = op(v, __builtin_amdgcn_update_dpp(v, v, 0x141, 0xf, 0xf, false));   // row_half_mirror
+  v = op(v, __builtin_amdgcn_update_dpp(v, v, 0x140, 0xf, 0xf, false));   // row_mirror
+  int r = __builtin_amdgcn_readlane(v, 0);
+#pragma unroll
+  for (int i = 1; i < ROWS; ++i) r = op(r, __builtin_amdgcn_readlane(v, 16 * i));
+  return r;
+}
+// The largest key limit of the N queries from row `first` on.  Every wavefront looks at all of them: as an atomic maximum in LDS, which takes the
+// lanes one at a time, and two barriers, this was 7 000 to 10 000 of the 58 000 cycles of a workgroup that attends 680 keys (a whole
+// sequence of 680 tokens under the block-causal rule, [8,680,16,64]: append and attention 40.3 -> 37.1 us).
+template <int N> __device__ __forceinline__ int block_limit(const int32_t *kv_limit, int first, int Lq, int Lk) {
+  static_assert(N % 64 == 0, "whole wavefronts");
+  int m = 0;
+#pragma unroll
+  for (int i = 0; i < N / 64; ++i) {
+    const int row = first + i * 64 + (int)(threadIdx.x & 63), limit = kv_limit[min(row, Lq - 1)];   // (past the end: the last row's again)
+    m = max(m, min(limit, Lk));
+  }
+  return wave_fold<true, 4>(m);
+}
 // MFMA row r (0..31) of the S^T block carries key kperm(r) of the 32-key block
 // (bits 2 and 3 of r swapped), so accumulator register i of a lane in half h
 // holds key 16*(i/8) + 8*h + i%8.

@@ -112,14 +112,10 @@ __device__ __forceinline__ void attend_few(const AttnParams &p, int k_shift, int
     limit[n] = p.kv_limit ? max(min(p.kv_limit[min(qrow[n], p.Lq - 1)], p.Lk), 0) : p.Lk;
     if (qrow[n] < p.Lq) { kv_end = max(kv_end, limit[n]); minlim = min(minlim, limit[n]); }
   }
-  // (every wavefront holds the same queries: the largest and the smallest limit need no exchange between them)
+  // (every wavefront holds the same queries, and every quarter of it: the largest and the smallest limit need no exchange between them)
   if (p.kv_limit) {
-    for (int off = 1; off < 16; off <<= 1) {
-      kv_end = max(kv_end, __shfl_xor(kv_end, off, 64));
-      minlim = min(minlim, __shfl_xor(minlim, off, 64));
-    }
-    kv_end = __builtin_amdgcn_readfirstlane(kv_end);
-    minlim = __builtin_amdgcn_readfirstlane(minlim);
+    kv_end = wave_fold<true, 1>(kv_end);
+    minlim = wave_fold<false, 1>(minlim);
   } else {
     kv_end = p.Lk; minlim = p.Lk;
   }

@@ -409,16 +409,8 @@ __device__ __forceinline__ void attend_block(const AttnParams &p, int bh, int ou
     }
   };
   // ---- tile range: every lane of the workgroup runs the same number of tiles ----
-  __shared__ int lds_maxlim;
-  int kv_end = p.Lk;   // without per-query limits every query sees all keys
-  if (p.kv_limit) {
-    if (tid == 0) lds_maxlim = 0;
-    __syncthreads();
-    atomicMax(&lds_maxlim, q_live ? limit : 0);
-    __syncthreads();
-    kv_end = lds_maxlim;
-  }
-  int n_tiles = __builtin_amdgcn_readfirstlane((kv_end + BN - 1) / BN);   // (the limit comes from LDS: the compiler does not see that it is uniform)
+  const int kv_end = p.kv_limit ? block_limit<BM>(p.kv_limit, qt * BM, p.Lq, p.Lk) : p.Lk;   // without limits every query sees all keys
+  int n_tiles = (kv_end + BN - 1) / BN;
   // segment ends in LDS: indexing the kernel arguments with a run-time index would move
   // the whole argument block to scratch memory (literal indices only, for the same reason)
   __shared__ int lds_seg_end[kMaxSegments];
@@ -447,14 +439,9 @@ __device__ __forceinline__ void attend_block(const AttnParams &p, int bh, int ou
   int wseg = 0, wseg_end = p.Lk;
   // the keys that every query of this wavefront sees, and those that some query sees
   int wave_minlim = p.Lk, wave_end = kv_end;
-  if (p.kv_limit) {
-    wave_minlim = q_live ? limit : p.Lk;
-    wave_end = q_live ? limit : 0;
-    for (int off = 1; off < 64; off <<= 1) {
-      wave_minlim = min(wave_minlim, __shfl_xor(wave_minlim, off, 64));
-      wave_end = max(wave_end, __shfl_xor(wave_end, off, 64));
-    }
-    wave_end = __builtin_amdgcn_readfirstlane(wave_end);
+  if (p.kv_limit) {   // (the two halves of the wavefront hold the same queries)
+    wave_minlim = wave_fold<false, 2>(q_live ? limit : p.Lk);
+    wave_end = wave_fold<true, 2>(q_live ? limit : 0);
   }
 
   floatx16_t oacc[NDB];

@@ -242,7 +242,6 @@ __global__ __launch_bounds__(NW * 64, NW / 4) void wide_attn_kernel(WideParams e
   constexpr int NT = NW * 64, NF = D / 16, HT = kHalfTile<D>, PIECES = HT / (NT * 16);
   constexpr int BQ = NW * 32;   // queries of a block
   extern __shared__ __attribute__((aligned(16))) char lds[];   // K slots [4][HT], V slots [4][HT]
-  __shared__ int lds_maxlim;
   const AttnParams &p = e.a;
   const int all_tiles = e.all_tiles, n_wgs = gridDim.x;
   const int w = (blockIdx.x & 7) * (n_wgs >> 3) + min(blockIdx.x & 7, n_wgs & 7) + (blockIdx.x >> 3);
@@ -277,26 +276,18 @@ __global__ __launch_bounds__(NW * 64, NW / 4) void wide_attn_kernel(WideParams e
   const int qrow0 = qt * BQ + wave * 32;
   const bool wave_live = qrow0 < p.Lq;   // wave-uniform
   int limit[2], qrow_c[2];
-  int maxlim = 0, minlim = p.Lk;
+  int minlim = p.Lk;
 #pragma unroll
   for (int n = 0; n < 2; ++n) {
     const int row = qrow0 + n * 16 + r16;
     qrow_c[n] = min(row, p.Lq - 1);
     limit[n] = p.kv_limit ? max(min(p.kv_limit[qrow_c[n]], p.Lk), 0) : p.Lk;
-    if (row < p.Lq) { maxlim = max(maxlim, limit[n]); minlim = min(minlim, limit[n]); }
+    if (row < p.Lq) minlim = min(minlim, limit[n]);
   }
-  int kv_end = p.Lk;
-  if (p.kv_limit) {
-    if (tid == 0) lds_maxlim = 0;
-    __syncthreads();
-    atomicMax(&lds_maxlim, maxlim);
-    __syncthreads();
-    kv_end = lds_maxlim;
-  }
+  const int kv_end = p.kv_limit ? block_limit<BQ>(p.kv_limit, qt * BQ, p.Lq, p.Lk) : p.Lk;
   const int n_tiles = __builtin_amdgcn_readfirstlane(max(min((kv_end + BN - 1) / BN, tlast) - tbase, 0));
-  for (int off = 1; off < 64; off <<= 1) minlim = min(minlim, __shfl_xor(minlim, off, 64));
   // tiles that no query of the wavefront has to mask
-  const int n_full = __builtin_amdgcn_readfirstlane(min(max(minlim / BN - tbase, 0), n_tiles));
+  const int n_full = __builtin_amdgcn_readfirstlane(min(max(wave_fold<false, 1>(minlim) / BN - tbase, 0), n_tiles));
 
   const char *const src = e.tiles + ((int64_t)bh * all_tiles + tbase) * (2 * HT);
   // Tile t of K and of V sits in slot t % 4.  The copies to LDS go past the registers, each wavefront its own stretch of a
