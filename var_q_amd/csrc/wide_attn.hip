@@ -356,16 +356,6 @@ __global__ __launch_bounds__(NW * 64, NW / 4) void wide_attn_kernel(WideParams e
     zmax = fmaxf(zmax, __shfl_xor(zmax, 16, 64));
     return fmaxf(zmax, __shfl_xor(zmax, 32, 64));
   };
-  // the sum grows by a pair of weights as rounded for the matrix product
-  auto add_pair = [&](u32 w, float blk) __attribute__((always_inline)) {
-    if constexpr (F16) {
-      typedef _Float16 f16x2_t __attribute__((ext_vector_type(2)));
-      return __builtin_amdgcn_fdot2(__builtin_bit_cast(f16x2_t, w), __builtin_bit_cast(f16x2_t, 0x3c003c00u), blk, false);
-    } else {
-      typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
-      return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2_t, w), __builtin_bit_cast(bf16x2_t, 0x3f803f80u), blk, false);
-    }
-  };
 
   // operands of the next matrix instructions, requested ahead: K and V fragments i sit in slot i % 4
   u32x4_t kf[4], vf[4];
@@ -377,7 +367,7 @@ __global__ __launch_bounds__(NW * 64, NW / 4) void wide_attn_kernel(WideParams e
   auto step = [&](const char *kp, const char *vp, const char *kn, const char *vn, const floatx4_t (&s_in)[2][2], floatx4_t (&s_out)[2][2],
                   const u32x4_t (&p_in)[2], u32x4_t (&p_out)[2], int key0, auto mask_tag) __attribute__((always_inline)) {
     constexpr int HALVES = 16 / (2 * NF);   // exponentials per fragment
-    float blk[2] = {0.f, 0.f}, z[16], e[16];   // element h: query column h / 8, key h % 8
+    float blk[2], z[16], e[16];   // element h: query column h / 8, key h % 8
     auto form = [&](int j) __attribute__((always_inline)) {   // the logits of pair j
       z[2 * j] = logit(s_in, j >> 2, (2 * j) & 7, key0, mask_tag);
       z[2 * j + 1] = logit(s_in, j >> 2, (2 * j + 1) & 7, key0, mask_tag);
@@ -385,7 +375,7 @@ __global__ __launch_bounds__(NW * 64, NW / 4) void wide_attn_kernel(WideParams e
     auto pack = [&](int j) __attribute__((always_inline)) {   // the weights of pair j are rounded, kept and summed
       const u32 w = pack_io_rne<F16>(e[2 * j], e[2 * j + 1]);
       p_out[j >> 2][j & 3] = w;
-      blk[j >> 2] = add_pair(w, blk[j >> 2]);
+      if (j % 4 == 3) blk[j >> 2] = sum_weights<F16>(p_out[j >> 2]);
     };
     form(0);
     floatx4_t acc[2][2];
@@ -430,7 +420,6 @@ __global__ __launch_bounds__(NW * 64, NW / 4) void wide_attn_kernel(WideParams e
 #pragma unroll
         for (int d = 0; d < NF; ++d) oacc[d][n] *= alpha;
         l_part[n] *= alpha;
-        blk[n] = 0.f;
       }
 #pragma unroll
       for (int j = 0; j < 8; ++j) {
