@@ -15,7 +15,6 @@ constexpr int BN = 64;   // keys per tile
 constexpr int kMaxSegments = 16;
 constexpr int kMaxSplits_v = 8;        // shares of a query block's keys in the general kernel
 constexpr int kMaxKeyShares_v = 64;    // ... and in the kernel for few queries
-constexpr int kChanTableRows = 4;   // LDS rows per segment of the per-channel tables
 
 struct AttnParams {
   const __bf16 *q;
@@ -42,6 +41,7 @@ struct AttnParams {
   float *ws_o, *ws_ml;
   // the caller asked for exact codes in the MFMA operands where such a kernel exists (host side only)
   int exact_codes;
+  int k_shift, v_shift;   // log2 of the channels per scale group (fused_attn.hip)
   int f16;   // q, out and the MFMA operands are fp16 (host side only: it selects the instantiation)
   int fq_share_blocks;   // few-queries kernel: 32-key blocks per share of the keys
   int few_waves;         // ... and wavefronts of a workgroup, 4 or 8 (host side only)

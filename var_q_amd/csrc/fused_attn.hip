@@ -14,16 +14,12 @@
 //    S^T = K Q^T and O^T = V^T P^T, so that a lane owns one query column: row
 //    max/sum are per-lane (one cross-half exchange per tile) and the S^T
 //    accumulator registers are directly the B operand of the second MFMA.
-//  * Packed K and V tiles go HBM -> registers -> LDS (16-byte loads, issued one to three
-//    tiles ahead, one workgroup barrier per tile).  K is widened once per workgroup,
-//    straight from the registers it was loaded into, to LDS rows that are MFMA A operands;
-//    V goes to LDS packed and is widened and transposed by 2 keys x 8 channels per thread
-//    (the PV contraction runs over keys).  Widened tiles and packed V are double-buffered,
-//    the per-key parameters of the exact-code form triple-buffered; at head dim 64 there is also an
-//    instantiation with one of each buffer, for launches of many small workgroups (launch_d64).
+//  * Packed K and V go HBM -> registers, requested a tile ahead, are widened once per workgroup and put into LDS as rows of
+//    16-bit values, which are the MFMA A operands of the first product; those of the second, which runs over keys, are read
+//    from the rows of V with the transposing LDS read.  The tiles are double-buffered, with one workgroup barrier per tile; at head
+//    dim 64 there is also an instantiation with one buffer, for launches of many small workgroups (launch_d64).
 //  * Key rows are fed to the first MFMA in a permuted order chosen so that each
-//    lane's accumulator registers hold 8 consecutive keys per 16-key chunk,
-//    which makes the V^T operand a single 16-byte LDS read.
+//    lane's accumulator registers hold 8 consecutive keys per 16-key chunk, which is the order of the V^T operand.
 //  * Online softmax in the log2 domain against a reference that is only moved when a logit
 //    gets 16 octaves above the maximum it was set from, and that is found out from the weights
 //    (their sum, or the exponent bits of the packed bf16 pairs), not by a search for the row
@@ -32,8 +28,8 @@
 //  * Two forms of the operands:
 //    - dequantized (the default of every kernel): (code - zp) * scale in fp32, rounded to the
 //      attention's 16-bit type (bf16, or fp16 for the VAR path) when a tile is widened -- the
-//      operands the reference's attention sees -- and a plain flash attention behind it;
-//    - exact codes (opt-in; one group per key of 4- or 2-bit codes at head dim 128, bf16): the MFMA operands
+//      operands the reference's attention sees -- and a plain flash attention behind it (attend_tiles);
+//    - exact codes (opt-in, attend_codes; one group per key of 4- or 2-bit codes at head dim 128, bf16): the MFMA operands
 //      are exact small numbers derived from the codes, never scaled or rounded.  A code lands in
 //      the top mantissa bits of a bf16 1.x (raw = (code + kOff) / kMul), which costs one shift and
 //      one and-or per two elements.  Scales are applied in fp32, zero-points ride on extra MFMA
@@ -64,10 +60,6 @@ constexpr int BM = NW * 32;    // queries per workgroup (32 per wavefront)
 // head) pairs with at most 128 queries each -- the first steps of a scale schedule at a large
 // batch -- see launch().)
 constexpr float kHeadroom = 15.f;   // exact-code kernels: octaves between a fresh softmax reference and the row maximum
-
-__device__ __forceinline__ u32 pack_bf16_hi(float lo, float hi) {  // exact for values with <= 8 significant bits
-  return __builtin_amdgcn_perm(f2u(hi), f2u(lo), 0x07060302u);   // {hi[31:16], lo[31:16]} in one v_perm_b32
-}
 
 // ---- V side code widening ----------------------------------------------------
 // The V^T operand of the second MFMA holds, like the K operand of the first, an
@@ -110,42 +102,6 @@ template <> struct VCodec<2> {
     o[7] = ((x >> 9) & M) | B;
   }
 };
-template <> struct VCodec<8> {
-  static constexpr float kMul = 1.f, kOff = 0.f, kZmax = 256.f;
-  static constexpr u32 kStageXor = 0u;
-  __device__ static __forceinline__ void pairs(const u32 *row0, const u32 *row1, int oct, u32, u32 (&o)[8]) {
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      const int w0 = (int)row0[2 * oct + h], w1 = (int)row1[2 * oct + h];
-#pragma unroll
-      for (int j = 0; j < 4; ++j)
-        o[4 * h + j] = pack_bf16_hi((float)(int)__builtin_amdgcn_sbfe(w0, 8 * j, 8),
-                                    (float)(int)__builtin_amdgcn_sbfe(w1, 8 * j, 8));
-    }
-  }
-};
-// The kernels that dequantize want the images as fp32 numbers: f0[j], f1[j] = raw of channel j of
-// the octet in the two rows.  Bytes are converted once; the narrower fields come out of `pairs`.
-template <int BITS>
-__device__ __forceinline__ void v_pair_values(const u32 *row0, const u32 *row1, int oct, u32 M, float (&f0)[8], float (&f1)[8]) {
-  if constexpr (BITS == 8) {
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      const int w0 = (int)row0[2 * oct + h], w1 = (int)row1[2 * oct + h];
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        f0[4 * h + j] = (float)(int)__builtin_amdgcn_sbfe(w0, 8 * j, 8);
-        f1[4 * h + j] = (float)(int)__builtin_amdgcn_sbfe(w1, 8 * j, 8);
-      }
-    }
-  } else {
-    u32 pr[8];
-    VCodec<BITS>::pairs(row0, row1, oct, M, pr);
-#pragma unroll
-    for (int j = 0; j < 8; ++j) { f0[j] = __builtin_bit_cast(float, pr[j] << 16); f1[j] = __builtin_bit_cast(float, pr[j] & 0xffff0000u); }
-  }
-}
-
 // x = h0 + h1 + h2 exactly, each piece a bf16 (returned as its 16 bits): three
 // 8-bit slices of the 24-bit significand
 __device__ __forceinline__ void split3_bf16(float x, u32 &h0, u32 &h1, u32 &h2) {
@@ -199,158 +155,82 @@ template <> struct KCodec<2> {
   }
 };
 
-template <> struct KCodec<8> {
-  // bytes are widened through fp32 (exact), raw = code.
-  static constexpr float kMul = 1.f, kOff = 0.f;
-  __device__ static __forceinline__ int slot_d(int j) { return j; }
-  static constexpr u32 kStageXor = 0u, kMask = 0u;
-  __device__ static __forceinline__ void expand(const u32 *lds_row, int oct, u32, u32 (&o)[4]) {
-    const u32 w0 = lds_row[2 * oct], w1 = lds_row[2 * oct + 1];
-    float f[8];
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      f[j] = (float)(int)__builtin_amdgcn_sbfe((int)w0, 8 * j, 8);
-      f[4 + j] = (float)(int)__builtin_amdgcn_sbfe((int)w1, 8 * j, 8);
-    }
-#pragma unroll
-    for (int j = 0; j < 4; ++j) o[j] = pack_bf16_hi(f[2 * j], f[2 * j + 1]);
-  }
-};
+// octet (8-channel unit) of K that lane-half h contracts in 16-channel chunk ch
+__device__ __forceinline__ int k_octet(int ch, int h) { return h * 8 + ch; }
 
-// The kernels that dequantize want the images as fp32 numbers, in the operand's slot order.
-template <int BITS> __device__ __forceinline__ void k_values(const u32 *q4, int oct, u32 M, float (&f)[8]) {
-  if constexpr (BITS == 8) {
-    const u32 w0 = q4[2 * oct], w1 = q4[2 * oct + 1];
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      f[j] = (float)(int)__builtin_amdgcn_sbfe((int)w0, 8 * j, 8);
-      f[4 + j] = (float)(int)__builtin_amdgcn_sbfe((int)w1, 8 * j, 8);
-    }
-  } else {
-    u32 a[4];
-    KCodec<BITS>::expand(q4, oct, M, a);
-#pragma unroll
-    for (int m = 0; m < 4; ++m) { f[2 * m] = __builtin_bit_cast(float, a[m] << 16); f[2 * m + 1] = __builtin_bit_cast(float, a[m] & 0xffff0000u); }
-  }
-}
-
-// octet (8-channel unit) of K that lane-half h contracts in 16-channel chunk ch;
-// chunks never straddle a scale group of `G` channels.
-template <int G> __device__ __forceinline__ int k_octet(int ch, int h) {
-  constexpr int CPS = G / 16;  // chunks per group
-  const int seg = ch / CPS, cl = ch % CPS;
-  return seg * (G / 8) + h * CPS + cl;
-}
-
-// LDS layout of the attention kernel (bytes), shared by kernel and launcher.
-// kDeq: the kernel dequantizes when a tile is widened (see the kernel) and has no rank-1 operands.
-// That is the form of every kernel unless the caller asks for exact codes (EXACT), which exist
-// where they were measured to be the faster form: one group per key of 4- or 2-bit codes at
-// D=128.  (Per-channel tables, more than one K or V group per key, every kernel at D=64 and the
-// 8-bit kernels at D=128 are faster dequantizing, and have no exact-code instantiation.)
-template <int D, int BITS, int GK, int GV, bool CHAN> struct AttnForms {
-  static constexpr bool kHasExact = !CHAN && D / GK == 1 && D / GV == 1 && D == 128 && BITS != 8;
-};
-// ONE: one of each buffer, so that more workgroups are resident; a tile is staged, widened and attended before the
-// next one is staged (see launch_d64 for when that is the better way).
-template <int D, int BITS, int GK, int GV, bool CHAN, bool EXACT = false, bool ONE = false> struct AttnLds {
-  static_assert(!EXACT || AttnForms<D, BITS, GK, GV, CHAN>::kHasExact, "no exact-code form of this kernel");
-  static constexpr bool kDeq = !EXACT;
-  static constexpr int WPR = D * BITS / 32;
+// LDS layout of the kernel with exact codes (bytes), shared by kernel and launcher.
+template <int BITS> struct ExactLds {
+  static constexpr int D = 128, WPR = D * BITS / 32;
   static constexpr int RSV = WPR + 1;       // packed V row stride (words): odd, bank spread
-  static constexpr bool kFoldSv = !kDeq && (D / GV == 1);   // one V group: its scale rides inside the logits
-  static constexpr int kParFloats = CHAN ? 0 : ((kDeq ? 0 : D / GK) + (kFoldSv ? 1 : 2) * (D / GV)) * 64;
-  // Widened tiles and what only the widening reads (packed V and, where the kernel dequantizes, the per-key
-  // parameters) have two buffers, what the exact-code form reads while it attends three.
-  static constexpr int kBufs = ONE ? 1 : 2, kParBufs = kDeq ? kBufs : 3;
+  static constexpr int kParFloats = 2 * 64;
+  // Widened tiles and packed V have two buffers, what the kernel reads while it attends three.
   static constexpr int RSR = 64 + 8;        // stride (bf16) of the rows feeding the extra PV MFMA
   static constexpr int KXS = D + 8;         // stride (bf16) of a widened K row: 16-byte rows, bank spread
   static constexpr int kKx = 0;             // widened K
-  static constexpr int kVp = kKx + kBufs * 64 * KXS * 2;
-  static constexpr int kVt = (kVp + kBufs * 64 * RSV * 4 + 15) / 16 * 16;
-  static constexpr int kKz = kVt + kBufs * D * (64 + 8) * 2;          // rank-1 operands of S^T, 2 x 16 bytes per key and group
-  static constexpr int kWz = kKz + (kDeq ? 0 : 3 * (D / GK) * 64 * 32);   // 8 rows per slot for the extra PV MFMA
-  static constexpr int kPar = kWz + (kDeq ? 0 : 3 * 8 * RSR * 2);
-  static constexpr int kFlag = kPar + kParBufs * kParFloats * 4;
+  static constexpr int kVp = kKx + 2 * 64 * KXS * 2;
+  static constexpr int kVt = (kVp + 2 * 64 * RSV * 4 + 15) / 16 * 16;
+  static constexpr int kKz = kVt + 2 * D * (64 + 8) * 2;   // rank-1 operands of S^T, 2 x 16 bytes per key
+  static constexpr int kWz = kKz + 3 * 64 * 32;            // 8 rows per slot for the extra PV MFMA
+  static constexpr int kPar = kWz + 3 * 8 * RSR * 2;
+  static constexpr int kFlag = kPar + 3 * kParFloats * 4;
   static constexpr int kBytes = kFlag + 16;
 };
 
-// CHAN: scales and zero-points per (head, channel) instead of per (key, channel group), in up
-// to 16 tables that change along the keys (a cache quantized step by step has one per step).
-// Such a kernel dequantizes when a tile is widened, like the kernels for several groups per key
-// (DEQ below): K[l,d] = (code[l,d] - zk_s[d]) * sk_s[d] with s the segment of key l, rounded to
-// bf16 -- what the reference's attention sees -- and likewise V.  The tables of the head sit in
-// LDS; a tile inside one segment reads that segment's rows, a tile that straddles segments
-// looks the segment up per key.  Everything behind the widening is a plain bf16 flash attention
-// that knows nothing of tables or segments.
-// WPS: wavefronts per SIMD the register allocation aims at (2, or 4: two 8-wavefront workgroups
-// per compute unit at 128 registers, which the D=64 kernels that dequantize afford)
-// F16: q, out and the MFMA operands are fp16 instead of bf16 (dequantized K and V are rounded to
-// fp16, as the reference's fp16 attention call sees them: VAR/models/basic_var.py:157-158 under the
-// fp16 autocast of scripts/inference_multi_VAR.py:123); dequantizing kernels only.
+// A lane's column of O^T (16 registers of every block of 32 channels) to its place: the output, or with the keys shared out the normalized fp32
+// output and (reference, denominator) of this share, for the combining kernel.
+template <int D, bool F16, class Value>
+__device__ __forceinline__ void store_block(const AttnParams &p, int b, int hq, int qrow, bool q_live, int half, int split, int out_pair, float m_ref, float l_sum,
+                                            const floatx16_t (&oacc)[D / 32], Value &&value) {
+  const float inv = l_sum > 0.f ? 1.0f / l_sum : 0.f;
+  if (!q_live) return;
+  __bf16 *optr = p.out + (b * p.o_bs + hq * p.o_hs + qrow * p.o_ts) * D;
+  const bool shared_out = p.nsplit > 1;
+  const int64_t prow = ((int64_t)split * p.bh_total + out_pair) * p.Lq + qrow;
+  float *wptr = p.ws_o + prow * D;
+  if (shared_out && half == 0) *reinterpret_cast<float2 *>(p.ws_ml + prow * 2) = make_float2(m_ref, l_sum);
+#pragma unroll
+  for (int d = 0; d < D / 32; ++d) {
+#pragma unroll
+    for (int g4 = 0; g4 < 4; ++g4) {
+      // registers 4*g4 .. 4*g4+3 are rows d*32 + 8*g4 + 4*half + 0..3 of O^T
+      const float o0 = value(oacc[d][4 * g4 + 0]) * inv, o1 = value(oacc[d][4 * g4 + 1]) * inv;
+      const float o2 = value(oacc[d][4 * g4 + 2]) * inv, o3 = value(oacc[d][4 * g4 + 3]) * inv;
+      if (shared_out) *reinterpret_cast<float4 *>(wptr + d * 32 + 8 * g4 + 4 * half) = make_float4(o0, o1, o2, o3);
+      else *reinterpret_cast<uint2 *>(optr + d * 32 + 8 * g4 + 4 * half) = make_uint2(pack_io_rne<F16>(o0, o1), pack_io_rne<F16>(o2, o3));
+    }
+  }
+}
+
+// The opt-in kernel with exact codes: one group per key of 4- or 2-bit codes at D=128.
 // One workgroup's work: query tile qt of packed pair bh (= batch * p.Hkv + packed head), share `split` of its
 // keys; partial results go to the rows of pair `out_pair`.
-template <int D, int BITS, int GK, int GV, bool CHAN, int NWV, bool EXACT, bool F16, bool ONE = false>
-__device__ __forceinline__ void attend_block(const AttnParams &p, int bh, int out_pair, int qt, int split) {
-  static_assert(!(F16 && EXACT), "the exact-code form builds bf16 images of the codes");
-  static_assert(!CHAN || (GK == D && GV == D), "per-channel tables go with the single-group kernels");
-  constexpr int NW = NWV, NT = NWV * 64, BM = NWV * 32;   // (shadow the defaults of the file)
-  constexpr int NSK = D / GK, NSV = D / GV;
-  // DEQ: the kernel dequantizes when a tile is widened -- (code - zp) * scale in fp32, rounded to
-  // bf16, the very values the reference's attention sees after its dequantize and downcast
-  // (VAR_Q/quant.py:216-224, VAR/models/basic_var.py:158) -- and then runs like a plain bf16 flash
-  // attention: one accumulator, one set of weights, whatever the group count, no rank-1 MFMA and
-  // no extra O^T block (the softmax denominator is summed on the vector ALU).  With several K or
-  // V groups per key, exact codes in the MFMAs would need one logit accumulator and one rank-1
-  // MFMA per K group and one set of weights and one extra MFMA per V group (19 -> 28 MFMAs per
-  // key block at four groups, and registers that do not exist); where there is one group, which
-  // form is faster was measured (see AttnForms).
-  constexpr bool DEQ = AttnLds<D, BITS, GK, GV, CHAN, EXACT>::kDeq;
-  constexpr int NSKA = DEQ ? 1 : NSK, NSVA = DEQ ? 1 : NSV;   // accumulators / weight sets
-  // (Exact codes are instantiated for one group per key only, so NSKA = NSVA = 1 in every kernel that
-  // exists; the exact-code form is nevertheless written for any group count -- its loops over
-  // groups are single passes today -- because AttnForms::kHasExact is a measured choice that may move.)
-  static_assert(DEQ || (NSK == 1 && NSV == 1), "exact codes with several groups per key: AttnForms sends those to the dequantizing form");
-  static_assert(NW >= NSK && NW >= NSV && NW >= 2, "one wavefront per K group and per V group stages the parameters");
-  constexpr int WPR = D * BITS / 32;        // packed words per key row
+template <int BITS>
+__device__ __forceinline__ void attend_codes(const AttnParams &p, int bh, int out_pair, int qt, int split) {
+  using L = ExactLds<BITS>;
+  constexpr int D = L::D, NT = NW * 64, WPR = L::WPR;
   constexpr int NCH = D / 16;               // contraction chunks of QK^T
   constexpr int NDB = D / 32;               // 32-row blocks of O^T
   constexpr int VTS = BN + 8;               // V^T row stride (bf16 elements)
-  using L = AttnLds<D, BITS, GK, GV, CHAN, EXACT, ONE>;
-  constexpr int NB = L::kBufs, NPB = L::kParBufs;
 
   // Pipelined LDS buffers (one workgroup barrier per tile):
   //   packed V, the widened K and the widened V^T of tile t live in slot t % 2 (packed V is
-  //   read one iteration before its tile is attended, so tile t+2 may take its slot then), like
-  //   the per-key parameters where only the widening reads them; in the exact-code form those
-  //   live in slot t % 3.
+  //   read one iteration before its tile is attended, so tile t+2 may take its slot then), the
+  //   per-key parameters in slot t % 3.
   // While tile t is being attended, K and V of tile t+1 are widened (K straight
   // from the registers it was loaded into one iteration earlier, once per
   // workgroup, so the eight wavefronts share the work) and packed V of tile t+2 is
   // written from its registers.
   extern __shared__ __attribute__((aligned(16))) unsigned char lds_raw[];
-  uint16_t *const lds_kx = reinterpret_cast<uint16_t *>(lds_raw + L::kKx);  // [NB][BN][KXS] widened K codes (MFMA A operands)
-  u32 *const lds_vp = reinterpret_cast<u32 *>(lds_raw + L::kVp);          // [NB][BN][RSV]
-  uint16_t *const lds_vt = reinterpret_cast<uint16_t *>(lds_raw + L::kVt);  // [NB][D][VTS]  raw V codes, transposed
-  u32x4_t *const lds_kz = reinterpret_cast<u32x4_t *>(lds_raw + L::kKz);  // [3][NSK][BN][2] rank-1 A operands (per lane half)
-  // [3][8][RSR] bf16 rows of the extra PV MFMA: row s < NSV = vzp_c + kOff of group s,
-  // rows 4..6 = the three bf16 pieces of 1/vs of group 0, row 7 = zeros
+  uint16_t *const lds_kx = reinterpret_cast<uint16_t *>(lds_raw + L::kKx);  // [2][BN][KXS] widened K codes (MFMA A operands)
+  u32 *const lds_vp = reinterpret_cast<u32 *>(lds_raw + L::kVp);          // [2][BN][RSV]
+  uint16_t *const lds_vt = reinterpret_cast<uint16_t *>(lds_raw + L::kVt);  // [2][D][VTS]  raw V codes, transposed
+  u32x4_t *const lds_kz = reinterpret_cast<u32x4_t *>(lds_raw + L::kKz);  // [3][BN][2] rank-1 A operands (per lane half)
+  // [3][8][RSR] bf16 rows of the extra PV MFMA: row 0 = vzp_c + kOff,
+  // rows 4..6 = the three bf16 pieces of 1/vs, row 7 = zeros
   uint16_t *const lds_wz = reinterpret_cast<uint16_t *>(lds_raw + L::kWz);
-  float *const lds_par = reinterpret_cast<float *>(lds_raw + L::kPar);    // [NPB][L::kParFloats]
+  float *const lds_par = reinterpret_cast<float *>(lds_raw + L::kPar);    // [3][kParFloats]: ck [BN], vr [BN]
   int *const lds_flag = reinterpret_cast<int *>(lds_raw + L::kFlag);      // [3] tile+1 if that tile has a zero-point remainder
-  // CHAN: the tables of this head for every segment, [nseg][4][D] fp32, filled once in the
-  // prologue, as the widening steps use them: row 0 = kMul * sk and row 1 = (zk + kOff) / kMul in
-  // the slot order of the K operand octets, row 2 = kMul * sv and row 3 = (zv + kOff) / kMul by
-  // channel ((code - z) * s = (raw - z') * s' for the code image raw = (code + kOff) / kMul, both
-  // rescalings exact)
-  float *const lds_tab = reinterpret_cast<float *>(lds_raw + (L::kBytes + 15) / 16 * 16);
-  constexpr int TR = kChanTableRows;
-  constexpr int KXS = L::KXS, RSV = L::RSV;
-  // parameter block of one tile: ck [NSK][BN]; vr [NSV][BN]; sv [NSV][BN] unless folded
-  constexpr bool FOLD_SV = L::kFoldSv;
-  constexpr int RSR = L::RSR;
-  constexpr int P_CK = 0, P_VR = (DEQ ? 0 : NSK) * BN, P_SV = P_VR + NSV * BN;
-  constexpr int P_VZ = P_VR;   // DEQ: per (V group, key) the zero-point image; P_SV holds the scale image
+  constexpr int KXS = L::KXS, RSV = L::RSV, RSR = L::RSR, P_VR = BN;
 
   const int b = bh / p.Hkv, hs = bh % p.Hkv;
   const int hq = p.head_map ? p.head_map[hs] : hs;
@@ -369,21 +249,19 @@ __device__ __forceinline__ void attend_block(const AttnParams &p, int bh, int ou
 
   // Q^T operands, gathered in the slot order of the K codec
   u32x4_t qb[NCH];
-  u32x4_t bq[NSK];
+  u32x4_t bq;
   // The K zero-point term -(kzp+kOff)/kMul * sum(q) is a rank-1 update of S^T and
-  // rides on one more MFMA per key block and group.  Both factors are split into
+  // rides on one more MFMA per key block.  Both factors are split into
   // three bf16 pieces (a0+a1+a2, b0+b1+b2, exact) and the 9 products are laid on
   // the 16 contraction slots: slots 0..7 (lower lane half) carry
   // A = a0 a0 a0 a1 a1 a1 a2 a2 against B = b0 b1 b2 b0 b1 b2 b0 b1 (a2*b2, 2^-32 of
-  // the term, is dropped).  With a single V group, slots 0..2 of the upper half add
+  // the term, is dropped).  Slots 0..2 of the upper half add
   // log2(vs)/ck (three pieces against 1.0), which makes exp2(logit) come out as
   // p * vs without a multiplication; the other upper slots are zero.
   // (the raw values were requested into qb earlier -- the prologue does, to overlap the trip
   // with its other loads)
   auto load_q = [&]() {
-    float qsum[NSK];
-#pragma unroll
-    for (int s = 0; s < NSK; ++s) qsum[s] = 0.f;
+    float qsum = 0.f;
 #pragma unroll
     for (int ch = 0; ch < NCH; ++ch) {
       // the octet's eight channels, loaded in one 16-byte piece, into the codec's slot order
@@ -394,23 +272,514 @@ __device__ __forceinline__ void attend_block(const AttnParams &p, int bh, int ou
         const int d0 = KCodec<BITS>::slot_d(2 * j2), d1 = KCodec<BITS>::slot_d(2 * j2 + 1);   // channels within the octet
         const u32 lo = (raw[d0 >> 1] >> (16 * (d0 & 1))) << 16, hi = (raw[d1 >> 1] >> (16 * (d1 & 1))) << 16;
         qb[ch][j2] = (lo >> 16) | hi;
-        qsum[ch / (GK / 16)] += u2f(lo) + u2f(hi);
+        qsum += u2f(lo) + u2f(hi);
       }
     }
-#pragma unroll
-    for (int s = 0; s < NSK; ++s) qsum[s] += __shfl_xor(qsum[s], 32, 64);
-#pragma unroll
-    for (int s = 0; s < (DEQ ? 0 : NSK); ++s) {
-      u32 b0, b1, b2;
-      split3_bf16(qsum[s], b0, b1, b2);
-      if (half == 0) bq[s] = u32x4_t{b0 | (b1 << 16), b2 | (b0 << 16), b1 | (b2 << 16), b0 | (b1 << 16)};
-      else if (FOLD_SV && s == 0) bq[s] = u32x4_t{0x3f803f80u, 0x00003f80u, 0u, 0u};
-      else bq[s] = u32x4_t{0u, 0u, 0u, 0u};
-    }
+    qsum += __shfl_xor(qsum, 32, 64);
+    u32 b0, b1, b2;
+    split3_bf16(qsum, b0, b1, b2);
+    if (half == 0) bq = u32x4_t{b0 | (b1 << 16), b2 | (b0 << 16), b1 | (b2 << 16), b0 | (b1 << 16)};
+    else bq = u32x4_t{0x3f803f80u, 0x00003f80u, 0u, 0u};
   };
   // ---- tile range: every lane of the workgroup runs the same number of tiles ----
   const int kv_end = p.kv_limit ? block_limit<BM>(p.kv_limit, qt * BM, p.Lq, p.Lk) : p.Lk;   // without limits every query sees all keys
-  int n_tiles = (kv_end + BN - 1) / BN;
+  int n_tiles = (kv_end + BN - 1) / BN, tbase = 0;   // tbase: this workgroup's first tile in the block's tile sequence
+  if (p.nsplit > 1) {
+    // this workgroup's share of the tiles: [t_begin, t_end) of the block's tile sequence
+    const int t_begin = n_tiles * split / p.nsplit, t_end = n_tiles * (split + 1) / p.nsplit;
+    tbase = t_begin;
+    n_tiles = t_end - t_begin;
+  }
+  const int tile_base = tbase * BN;   // first key of this workgroup's tiles
+  // The K prefetch and the V prefetch each walk the tiles in order.
+  int pk_tile = 0, pv_tile = 0;
+  // the keys that every query of this wavefront sees, and those that some query sees
+  int wave_minlim = p.Lk, wave_end = kv_end;
+  if (p.kv_limit) {   // (the two halves of the wavefront hold the same queries)
+    wave_minlim = wave_fold<false, 2>(q_live ? limit : p.Lk);
+    wave_end = wave_fold<true, 2>(q_live ? limit : 0);
+  }
+
+  floatx16_t oacc[NDB];
+#pragma unroll
+  for (int i = 0; i < NDB; ++i)
+#pragma unroll
+    for (int j = 0; j < 16; ++j) oacc[i][j] = 0.f;
+  // extra O^T block: row 0: sum_l p'[l] * (vzp_c + kOff); rows 4..6: pieces of the
+  // softmax denominator sum_l p'[l] / vs, i.e. the sum of the weights as rounded for the MFMA
+  floatx16_t racc;
+#pragma unroll
+  for (int j = 0; j < 16; ++j) racc[j] = 0.f;
+  float m_ref = 0.f;                 // softmax reference (log2 domain)
+  float r_run = 0.f;                 // sum_l p' * vzp_r, only fed on tiles with a remainder
+
+  const int64_t kv_row0 = b * p.kv_bs + hs * p.kv_hs;
+  const int64_t kv_ts = p.kv_ts;
+  const u32 *kw = p.k_words + kv_row0 * WPR;
+  const u32 *vw = p.v_words + kv_row0 * WPR;
+
+  constexpr int QUADS = BN * WPR / 4;                 // 16-byte pieces per packed tile
+  constexpr int LPT = (QUADS + NT - 1) / NT;          // pieces per thread
+  u32x4_t kreg[LPT], vreg[LPT];
+  float ksc = 0.f, kzp = 0.f, vsc = 0.f, vzp = 0.f, ksc0 = 0.f;
+
+  auto prefetch_k = [&]() {   // the next tile of the K stream
+    const int t0 = tile_base + pk_tile * BN;
+    ++pk_tile;
+#pragma unroll
+    for (int i = 0; i < LPT; ++i) {
+      const int piece = tid + i * NT;
+      if (LPT * NT == QUADS || piece < QUADS) {
+        const int key = min(t0 + piece / (WPR / 4), p.Lk - 1);
+        kreg[i] = *reinterpret_cast<const u32x4_t *>(kw + key * kv_ts * WPR + (piece % (WPR / 4)) * 4);
+      }
+    }
+  };
+  auto prefetch = [&]() {   // the next tile of the V stream
+    const int t0 = tile_base + pv_tile * BN;
+    ++pv_tile;
+#pragma unroll
+    for (int i = 0; i < LPT; ++i) {
+      const int piece = tid + i * NT;
+      if (LPT * NT == QUADS || piece < QUADS) {
+        const int key = min(t0 + piece / (WPR / 4), p.Lk - 1);
+        vreg[i] = *reinterpret_cast<const u32x4_t *>(vw + key * kv_ts * WPR + (piece % (WPR / 4)) * 4);
+      }
+    }
+    // scales: thread t handles key t % 64; wavefront 0 takes K's and the last one V's, which puts the K and the V arithmetic on
+    // different wavefronts
+    const int key = min(t0 + (tid & 63), p.Lk - 1), seg = tid >> 6, vseg = NW - 1 - seg;
+    if (seg < 1) {
+      const int64_t g = kv_row0 + key * kv_ts;
+      ksc = p.k_scale[g];
+      kzp = p.k_zp ? p.k_zp[g] : 0.f;
+    }
+    if (vseg < 1) {
+      const int64_t g = kv_row0 + key * kv_ts;
+      vsc = p.v_scale[g];
+      vzp = p.v_zp ? p.v_zp[g] : 0.f;
+      ksc0 = p.k_scale[g];
+    }
+  };
+
+  // registers -> LDS slot of `tile` (packed words as they are, parameters precombined)
+  auto stage = [&](int tile) {
+    const int sl = tile % 3;
+    u32 *vp = lds_vp + tile % 2 * BN * RSV;
+#pragma unroll
+    for (int i = 0; i < LPT; ++i) {
+      const int piece = tid + i * NT;
+      if (LPT * NT == QUADS || piece < QUADS) {
+        const int key = piece / (WPR / 4), w4 = (piece % (WPR / 4)) * 4;
+        constexpr u32 VX = VCodec<BITS>::kStageXor;
+        // V rows use an odd stride (bank spread for the column reads of the widening step)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) vp[key * RSV + w4 + j] = vreg[i][j] ^ VX;
+      }
+    }
+    float *par = lds_par + sl * L::kParFloats;
+    const int key = tid & 63, seg = tid >> 6, vseg = NW - 1 - seg;
+    // |ck| is kept away from zero so that log2(vs)/ck stays finite for a constant group
+    auto ck_of = [&](float ks) {
+      const float c = ks * p.scale_log2e * KCodec<BITS>::kMul;
+      return __builtin_fabsf(c) < 1e-30f ? 1e-30f : c;
+    };
+    if (seg < 1) {
+      par[key] = ck_of(ksc);
+      u32 a0, a1, a2;
+      split3_bf16(-(kzp + KCodec<BITS>::kOff) * (1.f / KCodec<BITS>::kMul), a0, a1, a2);
+      lds_kz[(sl * BN + key) * 2] = u32x4_t{a0 | (a0 << 16), a0 | (a1 << 16), a1 | (a1 << 16), a2 | (a2 << 16)};
+    }
+    if (vseg < 1) {
+      u32 l0, l1, l2;
+      split3_bf16(__builtin_amdgcn_logf(vsc) * __builtin_amdgcn_rcpf(ck_of(ksc0)), l0, l1, l2);
+      lds_kz[(sl * BN + key) * 2 + 1] = u32x4_t{l0 | (l1 << 16), l2, 0u, 0u};
+      // integer part of the zero-point within +-kZmax rides on the MFMA, the rest (none
+      // for zero-points produced by the quantizer of ordinary data) on the fp32 remainder
+      const float zc = __builtin_amdgcn_fmed3f(__builtin_rintf(vzp), -VCodec<BITS>::kZmax, VCodec<BITS>::kZmax);
+      const float zr = vzp - zc;
+      par[P_VR + key] = zr;
+      uint16_t *rows = lds_wz + sl * 8 * RSR;
+      rows[key] = (uint16_t)(f2u(zc + VCodec<BITS>::kOff) >> 16);
+      u32 i0, i1, i2;
+      split3_bf16(__builtin_amdgcn_rcpf(vsc), i0, i1, i2);
+      rows[4 * RSR + key] = (uint16_t)i0;
+      rows[5 * RSR + key] = (uint16_t)i1;
+      rows[6 * RSR + key] = (uint16_t)i2;
+      if (!(zr == 0.f)) lds_flag[sl] = tile + 1;   // benign race: every writer stores the same tag
+    }
+  };
+
+  u32 kmask = KCodec<BITS>::kMask;
+  asm volatile("" : "+v"(kmask));   // keep the mask in a vector register (see KCodec::expand)
+
+  // row of the extra PV block this lane feeds (as element offset)
+  const int rowsel = (col == 0 ? 0 : (col >= 4 && col < 7) ? col : 7) * RSR;
+
+  // packed V of `tile` -> V^T bf16: a work item is 2 adjacent keys x 8 channels (one
+  // packed word of each key), written as 8 dwords of the transposed tile
+  auto widen_v = [&](int tile) {
+    const u32 *vp = lds_vp + (tile % 2) * BN * RSV;
+    uint16_t *vt = lds_vt + (tile % 2) * D * VTS;
+    static_assert((BN / 2) * (D / 8) == NT, "an item for every thread");
+    const int kp2 = tid & (BN / 2 - 1), oct = tid / (BN / 2);
+    const u32 *row = &vp[kp2 * 2 * RSV];
+    u32 pr[8];
+    VCodec<BITS>::pairs(row, row + RSV, oct, kmask, pr);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) *reinterpret_cast<u32 *>(&vt[(oct * 8 + j) * VTS + kp2 * 2]) = pr[j];
+  };
+
+  // packed K of `tile` (in kreg) -> widened bf16 rows: each piece holds OPQ octets
+  // of one key, every octet becomes one 16-byte MFMA A operand
+  auto widen_k = [&](int tile) {
+    uint16_t *kx = lds_kx + (tile % 2) * BN * KXS;
+    constexpr int OPQ = 16 / BITS;       // octets per piece
+#pragma unroll
+    for (int i = 0; i < LPT; ++i) {
+      const int piece = tid + i * NT;
+      if (LPT * NT == QUADS || piece < QUADS) {
+        const int key = piece / (WPR / 4), oct0 = (piece % (WPR / 4)) * OPQ;
+        constexpr u32 KX = KCodec<BITS>::kStageXor;
+        u32 q4[4];
+#pragma unroll
+        for (int w = 0; w < 4; ++w) q4[w] = kreg[i][w] ^ KX;
+#pragma unroll
+        for (int j = 0; j < OPQ; ++j) {
+          u32 a[4];
+          KCodec<BITS>::expand(q4, j, kmask, a);
+          *reinterpret_cast<u32x4_t *>(&kx[key * KXS + (oct0 + j) * 8]) = u32x4_t{a[0], a[1], a[2], a[3]};
+        }
+      }
+    }
+  };
+
+  // ---- prologue: V tiles 0 and 1 staged, K and V of tile 0 widened, K of tile 1 and V
+  //      of tile 2 in registers ------------------------------------------------------------
+  if (tid < 3) lds_flag[tid] = 0;
+  for (int i = tid; i < 3 * RSR; i += NT) lds_wz[((i / RSR) * 8 + 7) * RSR + i % RSR] = 0;   // the all-zero row of each slot
+  if (n_tiles > 0) { prefetch_k(); prefetch(); }
+  // the query values, behind the first tile's requests
+#pragma unroll
+  for (int ch = 0; ch < NCH; ++ch) qb[ch] = *reinterpret_cast<const u32x4_t *>(qptr + k_octet(ch, half) * 8);
+  __syncthreads();
+  load_q();
+  if (n_tiles > 0) { stage(0); widen_k(0); }
+  if (n_tiles > 1) { prefetch_k(); prefetch(); stage(1); }
+  __syncthreads();
+  if (n_tiles > 0) widen_v(0);
+  if (n_tiles > 2) prefetch();
+  __syncthreads();
+
+  // ---- the three phases of one 32-key block, as lambdas over per-tile state --------
+  // LDS operands are requested ahead of their use where the registers allow it (the
+  // scheduling fences keep the requests where they are written).
+  int t0 = 0;
+  const uint16_t *kx = nullptr, *vt = nullptr, *wz = nullptr;
+  const float *par = nullptr;
+  const u32x4_t *kz = nullptr;
+  bool tile_rem = false, first = true;
+  // register i of this lane <-> key kb*32 + 16*(i/8) + 8*half + i%8 of the tile
+  floatx16_t sacc;
+  u32 pop[2][4];          // P'^T operands: p * vs as bf16, [16-key chunk][dword]
+  float ckv[16];
+  u32x4_t vta[NDB], wza;
+
+  auto begin_tile = [&](int tile) {
+    t0 = tile_base + tile * BN;
+    kx = lds_kx + (tile % 2) * BN * KXS;
+    par = lds_par + (tile % 3) * L::kParFloats;
+    vt = lds_vt + (tile % 2) * D * VTS;
+    kz = lds_kz + (tile % 3) * BN * 2;
+    wz = lds_wz + (tile % 3) * 8 * RSR;
+    tile_rem = lds_flag[tile % 3] == tile + 1;   // tagged with the tile, so stale tags never match
+    // slot (tile+2)%3 was last read during tile-1 (before the barrier): refill it
+    if (tile + 2 < n_tiles) stage(tile + 2);
+    if (tile + 3 < n_tiles) prefetch();
+  };
+  // with the PV MFMAs of a block in flight: widen the next tile's K and V into the other slots
+  auto widen_next = [&](int tile) {
+    if (tile + 1 < n_tiles) {
+      widen_v(tile + 1);
+      widen_k(tile + 1);
+      if (tile + 2 < n_tiles) prefetch_k();
+    }
+  };
+  auto load_scales = [&](int kb) {
+#pragma unroll
+    for (int i4 = 0; i4 < 4; ++i4) {
+      const int key = kb * 32 + 16 * (i4 >> 1) + 8 * half + 4 * (i4 & 1);
+      const float4 t = *reinterpret_cast<const float4 *>(&par[key]);
+      ckv[4 * i4] = t.x; ckv[4 * i4 + 1] = t.y; ckv[4 * i4 + 2] = t.z; ckv[4 * i4 + 3] = t.w;
+    }
+  };
+  auto load_v_operands = [&](int kb, int c) {
+#pragma unroll
+    for (int d = 0; d < NDB; ++d)
+      vta[d] = *reinterpret_cast<const u32x4_t *>(&vt[(d * 32 + col) * VTS + (kb * 2 + c) * 16 + half * 8]);
+    wza = *reinterpret_cast<const u32x4_t *>(&wz[rowsel + (kb * 2 + c) * 16 + half * 8]);
+  };
+
+  // (raised priority around the matrix instructions: see attend_tiles)
+  constexpr bool MFMA_PRIO = BITS == 4;
+  // S^T = K Q^T for one 32-key block; the A operands are the widened K rows in LDS
+  auto qk = [&](int kb) {
+    if constexpr (MFMA_PRIO) __builtin_amdgcn_s_setprio(1);
+    const int krow_i = kb * 32 + kperm(col);
+    floatx16_t zero;
+#pragma unroll
+    for (int j = 0; j < 16; ++j) zero[j] = 0.f;
+    // starts the accumulator with the zero-point term (see bq above)
+    sacc = mfma_32x32x16<false>(kz[krow_i * 2 + half], bq, zero);
+    const uint16_t *krow = &kx[krow_i * KXS];
+#pragma unroll
+    for (int ch = 0; ch < NCH; ++ch) sacc = mfma_32x32x16<false>(*reinterpret_cast<const u32x4_t *>(&krow[k_octet(ch, half) * 8]), qb[ch], sacc);
+    if constexpr (MFMA_PRIO) __builtin_amdgcn_s_setprio(0);
+  };
+
+  // logits -> P'^T operands of one block: online softmax against a lazily moved reference
+  auto softmax = [&](int kb) {
+    float z[16];
+#pragma unroll
+    for (int i = 0; i < 16; ++i) z[i] = __builtin_fmaf(ckv[i], sacc[i], -m_ref);
+    // mask: block-causal key limit and the ragged last tile
+    if (t0 + BN > wave_minlim) {
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        const int key = t0 + kb * 32 + 16 * (i >> 3) + 8 * half + (i & 7);
+        if (key >= limit) z[i] = -INFINITY;
+      }
+    }
+    // Moves the softmax reference kHeadroom octaves above the row's current maximum: up only (never down) once
+    // something has been accumulated; the very first block takes its maximum as it is, negative
+    // or not (the accumulators are still zero, so alpha = 1 is exact).
+    auto move_reference = [&]() {
+      float zmax = z[0];
+#pragma unroll
+      for (int i = 1; i < 16; ++i) zmax = fmaxf(zmax, z[i]);
+      // the other lane half of the same query, without a trip through LDS
+      const auto sw = __builtin_amdgcn_permlane32_swap(f2u(zmax), f2u(zmax), false, false);
+      zmax = fmaxf(u2f(sw[0]), u2f(sw[1]));
+      const float delta = first ? ((zmax == -INFINITY) ? 0.f : zmax + kHeadroom) : fmaxf(zmax + kHeadroom, 0.f);
+      const float alpha = first ? 1.f : __builtin_amdgcn_exp2f(-delta);
+      m_ref += delta;
+#pragma unroll
+      for (int i = 0; i < 16; ++i) z[i] -= delta;
+#pragma unroll
+      for (int d = 0; d < NDB; ++d)
+#pragma unroll
+        for (int j = 0; j < 16; ++j) oacc[d][j] *= alpha;
+#pragma unroll
+      for (int j = 0; j < 16; ++j) racc[j] *= alpha;
+      r_run *= alpha;
+    };
+    // exp2 of the logits, rounded to bf16 pairs for the MFMA
+    auto weights = [&]() {
+      float pv[16];
+#pragma unroll
+      for (int i = 0; i < 16; ++i) pv[i] = __builtin_amdgcn_exp2f(z[i]);
+#pragma unroll
+      for (int i = 0; i < 16; i += 2) pop[i >> 3][(i & 7) >> 1] = pack_bf16_rne(pv[i], pv[i + 1]);
+    };
+    // The denominator is summed by the MFMA, so there is no sum to look at (as in attend_tiles); the packed
+    // weights themselves are: all are >= 0, so bit 14 of a bf16 (the top exponent bit) says
+    // "this weight is 2 or more" (infinities included), and an OR over the block's eight words
+    // finds one.  The reference is put kHeadroom octaves above the maximum when it moves, so
+    // weights start at 2^-kHeadroom or below -- bf16 and the fp32 sums keep their relative
+    // precision there -- and it moves again only for a logit 1 + kHeadroom octaves above that
+    // maximum.
+    if (first) move_reference();
+    weights();
+    if (!first) {
+      u32 any_w = 0;
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) any_w |= pop[h][j];
+      if (__any((any_w & 0x40004000u) != 0)) {
+        move_reference();
+        weights();
+      }
+    }
+    first = false;
+    if (tile_rem) {
+      // the remainder term must see the same bf16-rounded weights as the MFMA
+#pragma unroll
+      for (int i = 0; i < 16; i += 2) {
+        const int key = kb * 32 + 16 * (i >> 3) + 8 * half + (i & 7);
+        const u32 pk = pop[i >> 3][(i & 7) >> 1];
+        r_run = __builtin_fmaf(u2f(pk << 16), par[P_VR + key], r_run);
+        r_run = __builtin_fmaf(u2f(pk & 0xffff0000u), par[P_VR + key + 1], r_run);
+      }
+    }
+  };
+
+  // O^T += V^T P'^T for the 32 keys of one block; one more MFMA per chunk
+  // feeds the extra block: its row 0 collects the zero-point sum and rows
+  // 4..6 the softmax denominator
+  auto pv_mfma = [&](int kb) {
+    if constexpr (MFMA_PRIO) __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {
+      u32x4_t av[NDB];
+#pragma unroll
+      for (int d = 0; d < NDB; ++d) av[d] = vta[d];
+      const u32x4_t aw = wza;
+      if (c == 0) {
+        load_v_operands(kb, 1);   // in flight under this chunk's MFMAs
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      const u32x4_t bv = {pop[c][0], pop[c][1], pop[c][2], pop[c][3]};
+#pragma unroll
+      for (int d = 0; d < NDB; ++d) oacc[d] = mfma_32x32x16<false>(av[d], bv, oacc[d]);
+      racc = mfma_32x32x16<false>(aw, bv, racc);
+    }
+    if constexpr (MFMA_PRIO) __builtin_amdgcn_s_setprio(0);
+  };
+
+  // (the key blocks behind the last key that a query of this wavefront sees: see attend_tiles)
+  const int wave_tiles = __builtin_amdgcn_readfirstlane(wave_live ? min(n_tiles, (max(wave_end - tile_base, 0) + BN - 1) / BN) : 0);
+  auto attend = [&](int tile) {
+    begin_tile(tile);
+    const bool half_tile = wave_end - t0 <= 32;
+#pragma unroll
+    for (int kb = 0; kb < 2; ++kb) {
+      if (kb == 1 && half_tile) continue;
+      load_scales(kb);
+      qk(kb);
+      load_v_operands(kb, 0);   // used after the softmax arithmetic
+      __builtin_amdgcn_sched_barrier(0);
+      softmax(kb);
+      pv_mfma(kb);
+      if (kb == 0) widen_next(tile);
+    }
+  };
+  int tile = 0;
+  for (; tile < wave_tiles; ++tile) {
+    attend(tile);
+    __syncthreads();   // the one barrier per tile
+  }
+  // from there on (a wavefront without queries: from the start) the wavefront only helps with staging and
+  // widening, at the same barrier count as the others
+  for (; tile < n_tiles; ++tile) {
+    if (tile + 2 < n_tiles) stage(tile + 2);
+    if (tile + 3 < n_tiles) prefetch();
+    widen_next(tile);
+    __syncthreads();
+  }
+  if (!wave_live) return;
+
+  // ---- epilogue -------------------------------------------------------------------
+  r_run += __shfl_xor(r_run, 32, 64);
+  // rows 4..6 of racc are registers 0..2 of the upper lane half, row 0 register 0 of the lower
+  const float l_sum = __shfl(racc[0] + racc[1] + racc[2], col + 32, 64);
+  const float r = __shfl(racc[0], col, 64) + r_run;
+  constexpr float VM = VCodec<BITS>::kMul;
+  store_block<D, false>(p, b, hq, qrow, q_live, half, split, out_pair, m_ref, l_sum, oacc, [&](float o) { return VM * o - r; });
+}
+
+// ---- the kernel that dequantizes ----------------------------------------------------------------
+// K and V of a tile are widened alike, straight from the registers they were loaded into: a thread takes an eighth of a key's
+// channels, of K and of V, dequantizes them -- (code - zp) * scale in fp32, rounded to the attention's 16-bit type, the very
+// operands that the reference's attention sees after its dequantize and downcast (VAR_Q/quant.py:216-224,
+// VAR/models/basic_var.py:158) -- and puts them into LDS as a row of that key.  The rows of K are operands of S^T = K Q^T as they lie; the
+// operands of O^T = V^T P^T, 8 keys of one channel, come out of the rows of V through the transposing LDS read (ds_read_b64_tr_b16).
+// Before, V went to LDS packed and its parameters with it, was read back, and was written transposed two keys at a time; a table without
+// zero-points cost as much as one with.  Attention calls, before -> now, us: [64,256,16,64] over 680 keys, 8 bits, ten tables 95 -> 81, its
+// ten scales with the quantizers 401 -> 372..392 (boxes differ); 128 pairs x 680 tokens block-causal, 4 bits in groups of 32 34 -> 31.
+// What bounds it: at D=64 and four wavefronts per SIMD the vector ALU (some 200 instructions per wavefront and tile beside 24
+// matrix instructions); with one workgroup per compute unit the chain through a tile, 1.6 us at D=64 and 2.1 to 2.5 at D=128.
+//
+// A thread's codes as numbers, divided by kUnit: a power of two, which the scale and the zero-point take up exactly.
+template <int BITS> struct Widen {
+  static constexpr float kUnit = BITS == 8 ? 1.f : BITS == 4 ? 16.f : 4.f;
+  // octet `o` of the piece that begins at w; the low four bits of a word as a signed number, a sixteenth of it, are one instruction
+  __device__ static __forceinline__ void octet(const u32 *w, int o, float (&f)[8]) {
+    if constexpr (BITS == 8) {
+#pragma unroll
+      for (int j = 0; j < 8; ++j) f[j] = (float)(int)__builtin_amdgcn_sbfe((int)w[2 * o + (j >> 2)], 8 * (j & 3), 8);
+    } else if constexpr (BITS == 4) {
+      const u32 low = w[o], high = low >> 4;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) f[j] = __builtin_amdgcn_cvt_off_f32_i4((int)__builtin_amdgcn_ubfe(j & 1 ? high : low, 8 * (j >> 1), 8));
+    } else {
+      const u32 h = w[o >> 1] >> (16 * (o & 1)), odd = h & 0xccccu, even = (h << 2) & 0xccccu;   // fields in the upper halves of nibbles
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        const u32 x = j & 1 ? odd : even;
+        f[j] = __builtin_amdgcn_cvt_off_f32_i4((int)__builtin_amdgcn_ubfe(j & 2 ? x >> 4 : x, 8 * (j >> 2), 8));
+      }
+    }
+  }
+};
+// Rows of K and V in LDS (stride in elements).  K: 16 lanes read 16 bytes of 16 rows each, 4 banks apart.  V: 32 lanes read 64 bytes of four
+// rows each, 16 banks apart (4 banks apart, as K's, they got in one another's way).
+template <int D> constexpr int kKRow = D + 8;
+template <int D> constexpr int kVRow = D + (D == 128 ? 32 : 8);
+template <int D> constexpr int kKBuf = BN * kKRow<D>;   // a tile (elements)
+template <int D> constexpr int kVBuf = BN * kVRow<D>;
+// LDS of the kernel (bytes).  ONE: one buffer instead of two, so that more workgroups are resident; a tile is widened and
+// attended before the next one is widened (see launch_d64 for when that is the better way).
+template <int D, bool ONE> struct TileLds {
+  static constexpr int kBufs = ONE ? 1 : 2;
+  static constexpr int kTables = kBufs * (kKBuf<D> + kVBuf<D>) * 2;   // behind K's and V's buffers: the per-channel tables of the launch
+};
+
+// CHAN: scales and zero-points per (head, channel) instead of per (key, channel group), in up to 16 tables that change along the
+// keys (a cache quantized step by step has one per step): K[l,d] = (code[l,d] - zk_s[d]) * sk_s[d] with s the segment of key l, and
+// likewise V.  The tables of the head sit in LDS; a tile inside one segment reads that segment's rows, a tile that
+// straddles segments looks the segment up per key.
+// F16: q, out and the MFMA operands are fp16 instead of bf16 (dequantized K and V are rounded to fp16, as the reference's fp16
+// attention call sees them: VAR/models/basic_var.py:157-158 under the fp16 autocast of scripts/inference_multi_VAR.py:123).
+// One workgroup's work: query tile qt of packed pair bh (= batch * p.Hkv + packed head), share `split` of its
+// keys; partial results go to the rows of pair `out_pair`.
+template <int D, int BITS, bool CHAN, int NWV, bool F16, bool ONE = false>
+__device__ __forceinline__ void attend_tiles(const AttnParams &p, int bh, int out_pair, int qt, int split) {
+  constexpr int NT = NWV * 64, BM = NWV * 32;
+  constexpr int WPR = D * BITS / 32;        // packed words per key row
+  constexpr int NCH = D / 16;               // contraction chunks of QK^T
+  constexpr int NDB = D / 32;               // 32-row blocks of O^T
+  constexpr int CH = D / 8, OCT = CH / 8;   // channels and octets of a thread's piece of a row
+  constexpr int PB = CH * BITS / 8, PW = PB < 4 ? 1 : PB / 4;   // bytes and words of it
+  constexpr int IT = BN * 8 / NT;           // pieces of a tile per thread
+  using L = TileLds<D, ONE>;
+  constexpr int KS = kKRow<D>, VS = kVRow<D>;
+  constexpr float kUnit = Widen<BITS>::kUnit;
+  extern __shared__ __attribute__((aligned(16))) unsigned char lds_raw[];
+  uint16_t *const lds_k = reinterpret_cast<uint16_t *>(lds_raw);   // [kBufs][BN][KS]
+  uint16_t *const lds_v = lds_k + L::kBufs * kKBuf<D>;             // [kBufs][BN][VS]
+  float *const lds_tab = reinterpret_cast<float *>(lds_raw + L::kTables);   // [nseg][2 or 4][D]: scales of K and V times kUnit, zero-points over kUnit
+  const bool has_zp = p.k_chan_zp || p.v_chan_zp;
+  const int tab_rows = has_zp ? 4 : 2;
+
+  const int b = bh / p.Hkv, hs = bh % p.Hkv;
+  const int hq = p.head_map ? p.head_map[hs] : hs;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int col = lane & 31, half = lane >> 5;
+
+  // ---- this lane's query ----------------------------------------------------
+  const int qrow = qt * BM + wave * 32 + col;
+  const bool q_live = qrow < p.Lq;
+  const bool wave_live = qt * BM + wave * 32 < p.Lq;   // wave-uniform
+  const int qrow_c = q_live ? qrow : p.Lq - 1;
+  const __bf16 *const qptr = p.q + (b * p.q_bs + hq * p.q_hs + qrow_c * p.q_ts) * D + half * 8;
+  const int limit = p.kv_limit ? max(min(p.kv_limit[qrow_c], p.Lk), 0) : p.Lk;
+
+  // ---- tile range: every lane of the workgroup runs the same number of tiles ----
+  const int kv_end = p.kv_limit ? block_limit<BM>(p.kv_limit, qt * BM, p.Lq, p.Lk) : p.Lk;   // without limits every query sees all keys
+  int n_tiles = (kv_end + BN - 1) / BN, tbase = 0;   // tbase: this workgroup's first tile in the block's tile sequence
+  if (p.nsplit > 1) {
+    const int t_begin = n_tiles * split / p.nsplit, t_end = n_tiles * (split + 1) / p.nsplit;
+    tbase = t_begin;
+    n_tiles = t_end - t_begin;
+  }
+  const int tile_base = tbase * BN;   // first key of this workgroup's tiles
+  // the keys that every query of this wavefront sees, and those that some query sees
+  int wave_minlim = p.Lk, wave_end = kv_end;
+  if (p.kv_limit) {   // (the two halves of the wavefront hold the same queries)
+    wave_minlim = wave_fold<false, 2>(q_live ? limit : p.Lk);
+    wave_end = wave_fold<true, 2>(q_live ? limit : 0);
+  }
   // segment ends in LDS: indexing the kernel arguments with a run-time index would move
   // the whole argument block to scratch memory (literal indices only, for the same reason)
   __shared__ int lds_seg_end[kMaxSegments];
@@ -424,490 +793,214 @@ __device__ __forceinline__ void attend_block(const AttnParams &p, int bh, int ou
     }
     // (read behind the prologue's first barrier)
   }
-  int tbase = 0;   // index of this workgroup's first tile in the block's tile sequence
-  if (p.nsplit > 1) {
-    // this workgroup's share of the tiles: [t_begin, t_end) of the block's tile sequence
-    const int t_begin = n_tiles * split / p.nsplit, t_end = n_tiles * (split + 1) / p.nsplit;
-    tbase = t_begin;
-    n_tiles = t_end - t_begin;
-  }
-  const int tile_base = tbase * BN;   // first key of this workgroup's tiles
-  // The K prefetch, the V prefetch and the widening each walk the tiles in order.
-  int pk_tile = 0, pv_tile = 0;
-  // CHAN: segment of the first key of the next tile to be widened, and where that segment ends
-  // (wave-uniform; the tiles are widened in order, K and V of a tile one after the other)
-  int wseg = 0, wseg_end = p.Lk;
-  // the keys that every query of this wavefront sees, and those that some query sees
-  int wave_minlim = p.Lk, wave_end = kv_end;
-  if (p.kv_limit) {   // (the two halves of the wavefront hold the same queries)
-    wave_minlim = wave_fold<false, 2>(q_live ? limit : p.Lk);
-    wave_end = wave_fold<true, 2>(q_live ? limit : 0);
-  }
 
-  floatx16_t oacc[NDB];
-#pragma unroll
-  for (int i = 0; i < NDB; ++i)
-#pragma unroll
-    for (int j = 0; j < 16; ++j) oacc[i][j] = 0.f;
-  // extra O^T block: row s < NSV: sum_l p'_s * (vzp_c + kOff); rows 4..6: pieces of the
-  // softmax denominator sum_l p'_0 / vs_0, i.e. the sum of the weights as rounded for the MFMA
-  floatx16_t racc;
-#pragma unroll
-  for (int j = 0; j < 16; ++j) racc[j] = 0.f;
-  // DEQ: no extra block; the softmax denominator is summed on the vector ALU from the weights as
-  // rounded for the MFMA (this lane's keys; the two lane halves are added in the epilogue)
-  float l_part = 0.f;
-  float m_ref = 0.f;                 // softmax reference (log2 domain)
-  float r_run[NSVA];                 // sum_l p' * vzp_r, only fed on tiles with a remainder
-#pragma unroll
-  for (int s = 0; s < NSVA; ++s) r_run[s] = 0.f;
-
+  // ---- loads: piece i of the thread is eighth `part` of key tid / 8 + i * NT / 8 of the tile ----
+  const int part = tid & 7, key_l = tid >> 3;
   const int64_t kv_row0 = b * p.kv_bs + hs * p.kv_hs;
-  const int64_t kv_ts = p.kv_ts;
-  const u32 *kw = p.k_words + kv_row0 * WPR;
-  const u32 *vw = p.v_words + kv_row0 * WPR;
-
-  constexpr int QUADS = BN * WPR / 4;                 // 16-byte pieces per packed tile
-  constexpr int LPT = (QUADS + NT - 1) / NT;          // pieces per thread
-  // The K tile is loaded in pieces of KPW words, small enough that every thread of the workgroup
-  // has one where the tile allows it (the thread that loads a piece widens it, so this spreads
-  // the widening evenly: 2-bit codes at D=64 would otherwise occupy a single wavefront).
-  // (the V tile is widened in (BN/2)*(D/8) items by the upper wavefronts; where those are fewer than
-  // the threads, the K pieces go to the threads that are left)
-  constexpr int K_THREADS = ((BN / 2) * (D / 8) < NT) ? NT - (BN / 2) * (D / 8) : NT;
-  // (measured: 5-9 % faster for 2-bit codes and at D=64; 4-bit codes at D=128 are 5 % slower in
-  // 8-byte pieces -- twice the per-piece parameter loads -- and keep 16-byte ones)
-  constexpr int KPW = (DEQ && (D == 64 || BITS == 2) && BN * WPR / K_THREADS < 4) ? (BN * WPR / K_THREADS < 2 ? 1 : 2) : 4;
-  constexpr int KPIECES = BN * WPR / KPW, KPPR = WPR / KPW;   // pieces per tile, per key row
-  constexpr int KLPT = (KPIECES + NT - 1) / NT;
-  u32x4_t kreg[KLPT], vreg[LPT];   // (a K piece uses the first KPW words of its register)
-  float ksc = 0.f, kzp = 0.f, vsc = 0.f, vzp = 0.f, ksc0 = 0.f;
-  // DEQ: scale and zero-point of the K groups that the thread's 16-byte pieces hold (a piece is
-  // 128 / BITS channels of one key: one group, or two for 2-bit codes in groups of 32)
-  constexpr int CPP = KPW * 32 / BITS;                  // channels per piece
-  constexpr int GPP = (DEQ && CPP > GK) ? CPP / GK : 1; // groups per piece
-  constexpr bool KGP = DEQ && !CHAN;                    // K group parameters travel with the pieces
-  float kgs[KGP ? KLPT * GPP : 1], kgz[KGP ? KLPT * GPP : 1];
-
-  auto prefetch_k = [&](int) {   // the next tile of the K stream
-    const int t0 = tile_base + pk_tile * BN;
-    ++pk_tile;
+  const int k_groups = CHAN ? 0 : D >> p.k_shift, v_groups = CHAN ? 0 : D >> p.v_shift;
+  const int64_t word_row = p.kv_ts * (WPR * 4), ks_row = p.kv_ts * (4 * k_groups), vs_row = p.kv_ts * (4 * v_groups);   // bytes from key to key
+  const char *const kw = reinterpret_cast<const char *>(p.k_words) + kv_row0 * (WPR * 4), *const vw = reinterpret_cast<const char *>(p.v_words) + kv_row0 * (WPR * 4);
+  const char *const ksc = reinterpret_cast<const char *>(p.k_scale) + kv_row0 * (4 * k_groups), *const kzp = reinterpret_cast<const char *>(p.k_zp) + kv_row0 * (4 * k_groups);
+  const char *const vsc = reinterpret_cast<const char *>(p.v_scale) + kv_row0 * (4 * v_groups), *const vzp = reinterpret_cast<const char *>(p.v_zp) + kv_row0 * (4 * v_groups);
+  const int k_g4 = CHAN ? 0 : (part * CH >> p.k_shift) * 4, v_g4 = CHAN ? 0 : (part * CH >> p.v_shift) * 4;
+  struct Piece { u32 k[PW], v[PW]; float ks, kz, vs, vz; } next[IT];
+  auto load_piece = [](const char *src, u32 (&dst)[PW]) __attribute__((always_inline)) {
+    if constexpr (PB == 16) {
+      const u32x4_t t = *reinterpret_cast<const u32x4_t *>(src);
 #pragma unroll
-    for (int i = 0; i < KLPT; ++i) {
-      const int piece = tid + i * NT;
-      if (KLPT * NT == KPIECES || piece < KPIECES) {
-        const int key = min(t0 + piece / KPPR, p.Lk - 1);
-        const u32 *src = kw + key * kv_ts * WPR + (piece % KPPR) * KPW;
-        if constexpr (KPW == 4) kreg[i] = *reinterpret_cast<const u32x4_t *>(src);
-        else if constexpr (KPW == 2) { const uint2 t = *reinterpret_cast<const uint2 *>(src); kreg[i][0] = t.x; kreg[i][1] = t.y; }
-        else kreg[i][0] = src[0];
-        if constexpr (KGP) {
-          const int g0 = (piece % KPPR) * CPP / GK;   // first group of the piece
-#pragma unroll
-          for (int j = 0; j < GPP; ++j) {
-            const int64_t g = (kv_row0 + key * kv_ts) * NSK + g0 + j;
-            kgs[i * GPP + j] = p.k_scale[g];
-            kgz[i * GPP + j] = p.k_zp ? p.k_zp[g] : 0.f;
-          }
-        }
-      }
+      for (int i = 0; i < 4; ++i) dst[i] = t[i];
+    } else if constexpr (PB == 8) {
+      const uint2 t = *reinterpret_cast<const uint2 *>(src);
+      dst[0] = t.x; dst[1] = t.y;
+    } else if constexpr (PB == 4) {
+      dst[0] = *reinterpret_cast<const u32 *>(src);
+    } else {
+      dst[0] = *reinterpret_cast<const uint16_t *>(src);
     }
   };
-  auto prefetch = [&](int) {   // the next tile of the V stream
-    const int t0 = tile_base + pv_tile * BN;
-    ++pv_tile;
+  auto request = [&](int tile) {
+    const int64_t t0 = tile_base + tile * BN;
+    const int last = p.Lk - 1 - (int)t0;   // (rows past the end: the last row's)
 #pragma unroll
-    for (int i = 0; i < LPT; ++i) {
-      const int piece = tid + i * NT;
-      if (LPT * NT == QUADS || piece < QUADS) {
-        const int key = min(t0 + piece / (WPR / 4), p.Lk - 1);
-        vreg[i] = *reinterpret_cast<const u32x4_t *>(vw + key * kv_ts * WPR + (piece % (WPR / 4)) * 4);
-      }
-    }
-    // scales: thread t handles key t % 64; wavefront w takes K group w and V group
-    // 3 - w, which puts the K and the V arithmetic of the single-group case on
-    // different wavefronts
-    if constexpr (!CHAN) {   // (per-channel tables: no per-key parameters)
-      const int key = min(t0 + (tid & 63), p.Lk - 1), seg = tid >> 6, vseg = NW - 1 - seg;
-      if (!DEQ && seg < NSK) {
-        const int64_t g = (kv_row0 + key * kv_ts) * NSK + seg;
-        ksc = p.k_scale[g];
-        kzp = p.k_zp ? p.k_zp[g] : 0.f;
-      }
-      if (vseg < NSV) {
-        const int64_t g = (kv_row0 + key * kv_ts) * NSV + vseg;
-        vsc = p.v_scale[g];
-        vzp = p.v_zp ? p.v_zp[g] : 0.f;
-        if (FOLD_SV) ksc0 = p.k_scale[(kv_row0 + key * kv_ts) * NSK];
+    for (int i = 0; i < IT; ++i) {
+      const int key = min(key_l + i * (NT / 8), last);
+      const int64_t w_at = key * word_row + part * PB;
+      load_piece(kw + t0 * word_row + w_at, next[i].k);
+      load_piece(vw + t0 * word_row + w_at, next[i].v);
+      if constexpr (!CHAN) {
+        const int64_t ks_at = key * ks_row + k_g4, vs_at = key * vs_row + v_g4;
+        next[i].ks = *reinterpret_cast<const float *>(ksc + t0 * ks_row + ks_at);
+        next[i].kz = p.k_zp ? *reinterpret_cast<const float *>(kzp + t0 * ks_row + ks_at) : 0.f;
+        next[i].vs = *reinterpret_cast<const float *>(vsc + t0 * vs_row + vs_at);
+        next[i].vz = p.v_zp ? *reinterpret_cast<const float *>(vzp + t0 * vs_row + vs_at) : 0.f;
       }
     }
   };
 
-  // registers -> LDS slot of `tile` (packed words as they are, parameters precombined)
-  auto stage = [&](int tile) {
-    const int sl = tile % 3;
-    u32 *vp = lds_vp + tile % NB * BN * RSV;
-#pragma unroll
-    for (int i = 0; i < LPT; ++i) {
-      const int piece = tid + i * NT;
-      if (LPT * NT == QUADS || piece < QUADS) {
-        const int key = piece / (WPR / 4), w4 = (piece % (WPR / 4)) * 4;
-        constexpr u32 VX = VCodec<BITS>::kStageXor;
-        // V rows use an odd stride (bank spread for the column reads of the widening step)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) vp[key * RSV + w4 + j] = vreg[i][j] ^ VX;
-      }
-    }
-    float *par = lds_par + tile % NPB * L::kParFloats;
-    const int key = tid & 63, seg = tid >> 6, vseg = NW - 1 - seg;
-    // |ck| is kept away from zero so that log2(vs)/ck stays finite for a constant group
-    auto ck_of = [&](float ks) {
-      const float c = ks * p.scale_log2e * KCodec<BITS>::kMul;
-      return __builtin_fabsf(c) < 1e-30f ? 1e-30f : c;
-    };
-    if (!DEQ && seg < NSK) {
-      par[P_CK + seg * BN + key] = ck_of(ksc);
-      u32 a0, a1, a2;
-      split3_bf16(-(kzp + KCodec<BITS>::kOff) * (1.f / KCodec<BITS>::kMul), a0, a1, a2);
-      u32x4_t *dst = &lds_kz[((sl * NSK + seg) * BN + key) * 2];
-      dst[0] = u32x4_t{a0 | (a0 << 16), a0 | (a1 << 16), a1 | (a1 << 16), a2 | (a2 << 16)};
-      if (!(FOLD_SV && seg == 0)) dst[1] = u32x4_t{0u, 0u, 0u, 0u};
-    }
-    if (CHAN) {
-      // (the tables are in LDS already)
-    } else if (DEQ) {
-      // (code - zp) * vs = (raw - (zp + kOff) / kMul) * (kMul * vs) for the code image `raw` the
-      // widening step produces; both factors are exact rescalings by powers of two
-      if (vseg < NSV) {
-        par[P_VZ + vseg * BN + key] = (vzp + VCodec<BITS>::kOff) * (1.f / VCodec<BITS>::kMul);
-        par[P_SV + vseg * BN + key] = vsc * VCodec<BITS>::kMul;
-      }
-    } else if (vseg < NSV) {
-      const int seg = vseg;
-      if (FOLD_SV) {
-        u32 l0, l1, l2;
-        split3_bf16(__builtin_amdgcn_logf(vsc) * __builtin_amdgcn_rcpf(ck_of(ksc0)), l0, l1, l2);
-        lds_kz[(sl * NSK * BN + key) * 2 + 1] = u32x4_t{l0 | (l1 << 16), l2, 0u, 0u};
-      }
-      // integer part of the zero-point within +-kZmax rides on the MFMA, the rest (none
-      // for zero-points produced by the quantizer of ordinary data) on the fp32 remainder
-      const float zc = __builtin_amdgcn_fmed3f(__builtin_rintf(vzp), -VCodec<BITS>::kZmax, VCodec<BITS>::kZmax);
-      const float zr = vzp - zc;
-      if (!FOLD_SV) par[P_SV + seg * BN + key] = vsc;
-      par[P_VR + seg * BN + key] = zr;
-      uint16_t *rows = lds_wz + sl * 8 * RSR;
-      rows[seg * RSR + key] = (uint16_t)(f2u(zc + VCodec<BITS>::kOff) >> 16);
-      if (seg == 0) {
-        u32 i0, i1, i2;
-        split3_bf16(__builtin_amdgcn_rcpf(vsc), i0, i1, i2);
-        rows[4 * RSR + key] = (uint16_t)i0;
-        rows[5 * RSR + key] = (uint16_t)i1;
-        rows[6 * RSR + key] = (uint16_t)i2;
-      }
-      if (!(zr == 0.f)) lds_flag[sl] = tile + 1;   // benign race: every writer stores the same tag
-    }
-  };
-
-  u32 kmask = KCodec<BITS>::kMask;
-  asm volatile("" : "+v"(kmask));   // keep the mask in a vector register (see KCodec::expand)
-
-  // row of the extra PV block this lane feeds in the MFMA of V group s (as element offset)
-  int rowsel[NSVA];
-#pragma unroll
-  for (int s = 0; s < NSVA; ++s) rowsel[s] = ((col == s) ? s : (s == 0 && col >= 4 && col < 7) ? col : 7) * RSR;
-
-  // CHAN: the widening of `tile` begins: (wseg, wseg_end) follow the tile's first key
-  auto widen_cursor = [&](int tile) {
+  // CHAN: segment of the first key of the next tile to be widened, and where that segment ends
+  // (wave-uniform; the tiles are widened in order)
+  int wseg = 0, wseg_end = p.Lk;
+  // the requested tile -> rows of K and V
+  auto widen = [&](int tile) {
+    uint16_t *const kx = lds_k + tile % L::kBufs * kKBuf<D>, *const vx = lds_v + tile % L::kBufs * kVBuf<D>;
+    bool one_seg = true;
     if constexpr (CHAN) {
       const int t0w = tile_base + tile * BN;
       while (wseg + 1 < p.nseg && t0w >= wseg_end) {
         ++wseg;
         wseg_end = __builtin_amdgcn_readfirstlane(lds_seg_end[wseg]);
       }
+      one_seg = wseg + 1 >= p.nseg || t0w + BN <= wseg_end;
     }
-  };
-  // CHAN: segment of a key of the tile being widened, searched upwards from the tile's first
-  auto key_segment = [&](int key) {
-    int sg = wseg;
-    while (sg + 1 < p.nseg && key >= lds_seg_end[sg]) ++sg;
-    return sg;
-  };
-  // CHAN: all keys of the tile being widened belong to segment wseg (wave-uniform)
-  auto tile_in_one_segment = [&](int tile) { return wseg + 1 >= p.nseg || tile_base + tile * BN + BN <= wseg_end; };
-
-  // packed V of `tile` -> V^T bf16: a work item is 2 adjacent keys x 8 channels (one
-  // packed word of each key), written as 8 dwords of the transposed tile
-  auto widen_v = [&](int tile) {
-    const u32 *vp = lds_vp + (tile % NB) * BN * RSV;
-    uint16_t *vt = lds_vt + (tile % NB) * D * VTS;
-    widen_cursor(tile);
-    const bool one_seg = !CHAN || tile_in_one_segment(tile);
-    // (where the tile has fewer items than the workgroup has threads, the upper wavefronts take
-    // them: the K pieces are widened by the lower ones)
-    constexpr int V_ITEMS = (BN / 2) * (D / 8);
-    constexpr int V_ROT = V_ITEMS < NT ? NT - V_ITEMS : 0;
-    for (int item = tid - V_ROT; item < V_ITEMS; item += NT) {
-      if (V_ROT && item < 0) continue;
-      const int kp2 = item & (BN / 2 - 1), oct = item / (BN / 2);
-      const u32 *row = &vp[kp2 * 2 * RSV];
-      u32 pr[8];
-      float f0[8], f1[8];
-      if constexpr (DEQ) v_pair_values<BITS>(row, row + RSV, oct, kmask, f0, f1);
-      else VCodec<BITS>::pairs(row, row + RSV, oct, kmask, pr);
-      if constexpr (CHAN) {
-        // code images -> values, (raw - z') * s' per channel in fp32, rounded to bf16
-        int sg0 = wseg, sg1 = wseg;
-        if (!one_seg) {
-          const int k0 = min(tile_base + tile * BN + 2 * kp2, p.Lk - 1);
-          sg0 = key_segment(k0);
-          sg1 = key_segment(min(k0 + 1, p.Lk - 1));
-        }
-        const float *t0s = lds_tab + (sg0 * TR + 2) * D + oct * 8;
-        const float4 sa = *reinterpret_cast<const float4 *>(t0s), sb = *reinterpret_cast<const float4 *>(t0s + 4);
-        const float4 za = *reinterpret_cast<const float4 *>(t0s + D), zb = *reinterpret_cast<const float4 *>(t0s + D + 4);
-        const float s0[8] = {sa.x, sa.y, sa.z, sa.w, sb.x, sb.y, sb.z, sb.w}, z0[8] = {za.x, za.y, za.z, za.w, zb.x, zb.y, zb.z, zb.w};
-        if (one_seg || sg1 == sg0) {
+    auto put = [&](auto zp_tag) __attribute__((always_inline)) {
+      constexpr bool ZP = decltype(zp_tag)::value;
 #pragma unroll
-          for (int j = 0; j < 8; ++j) pr[j] = pack_io_rne<F16>((f0[j] - z0[j]) * s0[j], (f1[j] - z0[j]) * s0[j]);
-        } else {
-          const float *t1s = lds_tab + (sg1 * TR + 2) * D + oct * 8;
-#pragma unroll
-          for (int j = 0; j < 8; ++j) pr[j] = pack_io_rne<F16>((f0[j] - z0[j]) * s0[j], (f1[j] - t1s[D + j]) * t1s[j]);
-        }
-      } else if constexpr (DEQ) {
-        // code images -> values of the two keys, (raw - z') * s' in fp32, rounded to bf16
-        const float *pt = lds_par + (tile % NPB) * L::kParFloats + (oct * 8 / GV) * BN + kp2 * 2;
-        const float2 z2 = *reinterpret_cast<const float2 *>(pt + P_VZ), s2 = *reinterpret_cast<const float2 *>(pt + P_SV);
-#pragma unroll
-        for (int j = 0; j < 8; ++j) pr[j] = pack_io_rne<F16>((f0[j] - z2.x) * s2.x, (f1[j] - z2.y) * s2.y);
-      }
-#pragma unroll
-      for (int j = 0; j < 8; ++j) *reinterpret_cast<u32 *>(&vt[(oct * 8 + j) * VTS + kp2 * 2]) = pr[j];
-    }
-  };
-
-  // packed K of `tile` (in kreg) -> widened bf16 rows: each piece holds OPQ octets
-  // of one key, every octet becomes one 16-byte MFMA A operand
-  auto widen_k = [&](int tile) {
-    uint16_t *kx = lds_kx + (tile % NB) * BN * KXS;
-    constexpr int OPQ = KPW * 4 / BITS;       // octets per piece
-    widen_cursor(tile);
-    const bool one_seg = !CHAN || tile_in_one_segment(tile);
-#pragma unroll
-    for (int i = 0; i < KLPT; ++i) {
-      const int piece = tid + i * NT;
-      if (KLPT * NT == KPIECES || piece < KPIECES) {
-        const int key = piece / KPPR, oct0 = (piece % KPPR) * OPQ;
-        constexpr u32 KX = KCodec<BITS>::kStageXor;
-        u32 q4[4];
-#pragma unroll
-        for (int w = 0; w < 4; ++w) q4[w] = w < KPW ? kreg[i][w] ^ KX : 0u;
-        int sg = wseg;
+      for (int i = 0; i < IT; ++i) {
+        const int key = key_l + i * (NT / 8);
+        const float *tab = lds_tab;
         if constexpr (CHAN) {
-          if (!one_seg) sg = key_segment(min(tile_base + tile * BN + key, p.Lk - 1));
-        }
-#pragma unroll
-        for (int j = 0; j < OPQ; ++j) {
-          u32 a[4];
-          float f[8];
-          if constexpr (DEQ) k_values<BITS>(q4, j, kmask, f);
-          else KCodec<BITS>::expand(q4, j, kmask, a);
-          if constexpr (CHAN) {
-            // code images -> values: (raw - z') * s' per channel (rows 0 and 1 of the segment's
-            // tables, in the operand's slot order), the reference's (code - zp) * scale, rounded to bf16
-            const float *tk = lds_tab + sg * TR * D + (oct0 + j) * 8;
-            const float4 sa = *reinterpret_cast<const float4 *>(tk), sb = *reinterpret_cast<const float4 *>(tk + 4);
-            const float4 za = *reinterpret_cast<const float4 *>(tk + D), zb = *reinterpret_cast<const float4 *>(tk + D + 4);
-            const float sc[8] = {sa.x, sa.y, sa.z, sa.w, sb.x, sb.y, sb.z, sb.w}, zc[8] = {za.x, za.y, za.z, za.w, zb.x, zb.y, zb.z, zb.w};
-#pragma unroll
-            for (int m = 0; m < 4; ++m)
-              a[m] = pack_io_rne<F16>((f[2 * m] - zc[2 * m]) * sc[2 * m], (f[2 * m + 1] - zc[2 * m + 1]) * sc[2 * m + 1]);
-          } else if constexpr (DEQ) {
-            // code images -> values: (raw - (zp + kOff) / kMul) * (kMul * ks), the reference's
-            // (code - zp) * scale with both factors rescaled exactly, rounded to bf16
-            const int gl = (j * 8) / GK < GPP ? (j * 8) / GK : GPP - 1;   // group of octet j inside the piece
-            const float zk = (kgz[i * GPP + gl] + KCodec<BITS>::kOff) * (1.f / KCodec<BITS>::kMul);
-            const float sk = kgs[i * GPP + gl] * KCodec<BITS>::kMul;
-#pragma unroll
-            for (int m = 0; m < 4; ++m) a[m] = pack_io_rne<F16>((f[2 * m] - zk) * sk, (f[2 * m + 1] - zk) * sk);
+          int sg = wseg;
+          if (!one_seg) {
+            const int k = min(tile_base + tile * BN + key, p.Lk - 1);
+            while (sg + 1 < p.nseg && k >= lds_seg_end[sg]) ++sg;
           }
-          *reinterpret_cast<u32x4_t *>(&kx[key * KXS + (oct0 + j) * 8]) = u32x4_t{a[0], a[1], a[2], a[3]};
+          tab += sg * (tab_rows * D) + part * CH;
         }
+        auto rows = [&](const u32 (&w)[PW], float s, float z, int row, uint16_t *dst) __attribute__((always_inline)) {
+          const float s1 = s * kUnit, z1 = z * (1.f / kUnit);
+#pragma unroll
+          for (int o = 0; o < OCT; ++o) {
+            float f[8];
+            Widen<BITS>::octet(w, o, f);
+            u32x4_t r;
+            if constexpr (CHAN) {
+              const float4 sa = *reinterpret_cast<const float4 *>(tab + row * D + o * 8), sb = *reinterpret_cast<const float4 *>(tab + row * D + o * 8 + 4);
+              const float sc[8] = {sa.x, sa.y, sa.z, sa.w, sb.x, sb.y, sb.z, sb.w};
+              if constexpr (ZP) {
+                const float4 za = *reinterpret_cast<const float4 *>(tab + (row + 2) * D + o * 8), zb = *reinterpret_cast<const float4 *>(tab + (row + 2) * D + o * 8 + 4);
+                const float zc[8] = {za.x, za.y, za.z, za.w, zb.x, zb.y, zb.z, zb.w};
+#pragma unroll
+                for (int j = 0; j < 8; ++j) f[j] -= zc[j];
+              }
+#pragma unroll
+              for (int j = 0; j < 4; ++j) r[j] = pack_io_rne<F16>(f[2 * j] * sc[2 * j], f[2 * j + 1] * sc[2 * j + 1]);
+            } else {
+#pragma unroll
+              for (int j = 0; j < 4; ++j) r[j] = pack_io_rne<F16>((f[2 * j] - z1) * s1, (f[2 * j + 1] - z1) * s1);
+            }
+            *reinterpret_cast<u32x4_t *>(dst + o * 8) = r;
+          }
+        };
+        rows(next[i].k, next[i].ks, next[i].kz, 0, kx + key * KS + part * CH);
+        rows(next[i].v, next[i].vs, next[i].vz, 1, vx + key * VS + part * CH);
       }
+    };
+    if constexpr (CHAN) {
+      if (has_zp) put(std::true_type{});
+      else put(std::false_type{});
+    } else {
+      put(std::true_type{});
     }
   };
 
-  // ---- prologue: V tiles 0 and 1 staged, K and V of tile 0 widened, K of tile 1 and V
-  //      of tile 2 in registers ------------------------------------------------------------
-  if (tid < 3) lds_flag[tid] = 0;
-  for (int i = tid; i < (DEQ ? 0 : 3 * RSR); i += NT) lds_wz[((i / RSR) * 8 + 7) * RSR + i % RSR] = 0;   // the all-zero row of each slot
-  if (n_tiles > 0) { prefetch_k(0); prefetch(0); }
-  // the query values, behind the first tile's requests and ahead of the table loads: one
-  // round trip for all three
+  // ---- prologue: tile 0 widened, tile 1 requested ----
+  if (n_tiles > 0) request(0);
+  // the query values, behind the first tile's requests and ahead of the table loads: one round trip for all three
+  u32x4_t qb[NCH];
 #pragma unroll
-  for (int ch = 0; ch < NCH; ++ch) qb[ch] = *reinterpret_cast<const u32x4_t *>(qptr + k_octet<GK>(ch, half) * 8);
+  for (int ch = 0; ch < NCH; ++ch) qb[ch] = *reinterpret_cast<const u32x4_t *>(qptr + ch * 16);
   if constexpr (CHAN) {
-    // The head's tables, as the widening steps use them (see lds_tab above): a thread takes one value of every segment (or
-    // every second).  kTabLoads of them are under way before the first is used: one after the other, each a trip to memory,
-    // they were what a launch began with, 1.6 us (five segments) to 4.1 us (eight, four wavefronts) of the 10 to 20 that
-    // the smaller steps of a schedule take.
-    constexpr int kTabLoads = 8, SEGS = NT / (TR * D);
-    static_assert(NT % (TR * D) == 0 && D % 64 == 0, "which of the tables a thread loads is the same for a wavefront and every segment");
-    const int which = __builtin_amdgcn_readfirstlane(tid / D) % TR, seg0 = __builtin_amdgcn_readfirstlane(tid / (TR * D)), d = tid % D;
-    const bool is_k = which < 2, is_zp = which & 1;
-    // (as a global pointer: behind the choice the compiler no longer knows it for one, and flat loads wait for LDS too)
-    const auto src = (const __attribute__((address_space(1))) float *)(uintptr_t)(which == 0 ? p.k_chan_scale : which == 1 ? p.k_chan_zp : which == 2 ? p.v_chan_scale : p.v_chan_zp);
-    const int c = is_k ? (d & ~7) + KCodec<BITS>::slot_d(d & 7) : d;   // K rows: the operand's slot order inside an octet
-    const float mul = is_k ? KCodec<BITS>::kMul : VCodec<BITS>::kMul, off = is_k ? KCodec<BITS>::kOff : VCodec<BITS>::kOff;
-#pragma unroll
-    for (int round = 0; round < kMaxSegments / (kTabLoads * SEGS); ++round) {
-      const int first = seg0 + round * (kTabLoads * SEGS);
-      if (first >= p.nseg) break;
+    // The head's tables (see lds_tab): row by row, NT / D of them at a time.  kTabLoads rows are
+    // under way before the first is used: one after the other, each a trip to memory, they were what a launch began with, 1.6 us (five
+    // segments) to 4.1 us (eight, four wavefronts) of the 10 to 20 that the smaller steps of a schedule take.
+    constexpr int kTabLoads = 8, G = NT / D;
+    static_assert(NT % D == 0 && D % 64 == 0, "the row that a thread loads is the same for a wavefront");
+    const int row0 = __builtin_amdgcn_readfirstlane(tid / D), d = tid % D, rows = p.nseg * tab_rows;
+    for (int first = row0; first < rows; first += kTabLoads * G) {
       float x[kTabLoads] = {};
-      if (src) {
 #pragma unroll
-        for (int u = 0; u < kTabLoads; ++u) x[u] = src[((int64_t)min(first + u * SEGS, p.nseg - 1) * p.Hkv + hs) * D + c];
+      for (int u = 0; u < kTabLoads; ++u) {
+        const int r = min(first + u * G, rows - 1), which = r & (tab_rows - 1), seg = r >> (has_zp ? 2 : 1);
+        const float *const of_k = which & 2 ? p.k_chan_zp : p.k_chan_scale, *const of_v = which & 2 ? p.v_chan_zp : p.v_chan_scale;
+        // (as a global pointer: behind the choice the compiler no longer knows it for one, and flat loads wait for LDS too)
+        const auto src = (const __attribute__((address_space(1))) float *)(uintptr_t)(which & 1 ? of_v : of_k);
+        if (src) x[u] = src[((int64_t)seg * p.Hkv + hs) * D + d];
       }
 #pragma unroll
       for (int u = 0; u < kTabLoads; ++u) {
-        const int seg = first + u * SEGS;
-        if (seg < p.nseg) lds_tab[seg * (TR * D) + which * D + d] = is_zp ? (x[u] + off) * (1.f / mul) : x[u] * mul;
+        const int r = first + u * G;
+        if (r < rows) lds_tab[r * D + d] = r & 2 & tab_rows >> 1 ? x[u] * (1.f / kUnit) : x[u] * kUnit;
       }
     }
+    __syncthreads();
+    if (p.nseg > 1) wseg_end = __builtin_amdgcn_readfirstlane(lds_seg_end[0]);   // (a share of the keys may begin mid-cache: widen goes on to its segment)
   }
-  __syncthreads();
-  if constexpr (CHAN) {
-    if (p.nseg > 1) {
-      // the segment of this workgroup's first key (a share of the keys may begin mid-cache)
-      wseg_end = __builtin_amdgcn_readfirstlane(lds_seg_end[0]);
-      widen_cursor(0);
-    }
-  }
-  load_q();
   if constexpr (!ONE) {
-    if (n_tiles > 0) { stage(0); widen_k(0); }
-    if (n_tiles > 1) { prefetch_k(1); prefetch(1); stage(1); }
-    __syncthreads();
-    if (n_tiles > 0) widen_v(0);
-    if (n_tiles > 2) prefetch(2);
+    if (n_tiles > 0) widen(0);
+    if (n_tiles > 1) request(1);
     __syncthreads();
   }
 
-  // ---- the three phases of one 32-key block, as lambdas over per-tile state --------
-  // LDS operands are requested ahead of their use where the registers allow it (the
-  // scheduling fences keep the requests where they are written).
-  constexpr bool HOIST = (NSKA == 1 && NSVA == 1);
-  int t0 = 0;
-  const uint16_t *kx = nullptr, *vt = nullptr, *wz = nullptr;
-  const float *par = nullptr;
-  const u32x4_t *kz = nullptr;
-  bool tile_rem = false, first = true;
-  // register i of this lane <-> key kb*32 + 16*(i/8) + 8*half + i%8 of the tile
-  floatx16_t sacc[2][NSKA];
-  u32 pop[2][NSVA][2][4];          // P'^T operands: p * vs as bf16, [block][V group][16-key chunk][dword]
-  float ckv[2][NSKA][16], svv[2][NSVA][16];
-  u32x4_t vta[NDB], wza[NSVA];
+  // (the queries are there: otherwise the compiler has the key loop wait for them, and with them for the tile that is on its way)
+#pragma unroll
+  for (int ch = 0; ch < NCH; ++ch) asm volatile("" : "+v"(qb[ch]));
 
-  auto begin_tile = [&](int tile) {
-    t0 = tile_base + tile * BN;
-    kx = lds_kx + (tile % NB) * BN * KXS;
-    par = lds_par + (tile % NPB) * L::kParFloats;
-    vt = lds_vt + (tile % NB) * D * VTS;
-    kz = lds_kz + (tile % 3) * NSK * BN * 2;
-    wz = lds_wz + (tile % 3) * 8 * RSR;
-    tile_rem = lds_flag[tile % 3] == tile + 1;   // tagged with the tile, so stale tags never match
-    // slot (tile+2)%3 was last read during tile-1 (before the barrier): refill it
-    if constexpr (ONE) return;
-    if (tile + 2 < n_tiles) stage(tile + 2);
-    if (tile + 3 < n_tiles) prefetch(tile + 3);
-  };
-  // with the PV MFMAs of a block in flight: widen the next tile's K and V into the other slots
-  auto widen_next = [&](int tile) {
-    if (tile + 1 < n_tiles) {
-      widen_v(tile + 1);
-      widen_k(tile + 1);
-      if (tile + 2 < n_tiles) prefetch_k(tile + 2);
-    }
-  };
-  auto load_scales = [&](int kb) {
+  floatx16_t oacc[NDB];
 #pragma unroll
-    for (int s = 0; s < ((HOIST && !DEQ) ? NSK : 0); ++s)
+  for (int i = 0; i < NDB; ++i)
 #pragma unroll
-      for (int i4 = 0; i4 < 4; ++i4) {
-        const int key = kb * 32 + 16 * (i4 >> 1) + 8 * half + 4 * (i4 & 1);
-        const float4 t = *reinterpret_cast<const float4 *>(&par[P_CK + s * BN + key]);
-        ckv[kb][s][4 * i4] = t.x; ckv[kb][s][4 * i4 + 1] = t.y; ckv[kb][s][4 * i4 + 2] = t.z; ckv[kb][s][4 * i4 + 3] = t.w;
-      }
-#pragma unroll
-    for (int s = 0; s < ((HOIST && !FOLD_SV && !DEQ) ? NSV : 0); ++s)
-#pragma unroll
-      for (int i4 = 0; i4 < 4; ++i4) {
-        const int key = kb * 32 + 16 * (i4 >> 1) + 8 * half + 4 * (i4 & 1);
-        const float4 t = *reinterpret_cast<const float4 *>(&par[P_SV + s * BN + key]);
-        svv[kb][s][4 * i4] = t.x; svv[kb][s][4 * i4 + 1] = t.y; svv[kb][s][4 * i4 + 2] = t.z; svv[kb][s][4 * i4 + 3] = t.w;
-      }
-  };
-  auto load_v_operands = [&](int kb, int c) {
-#pragma unroll
-    for (int d = 0; d < NDB; ++d)
-      vta[d] = *reinterpret_cast<const u32x4_t *>(&vt[(d * 32 + col) * VTS + (kb * 2 + c) * 16 + half * 8]);
-#pragma unroll
-    for (int s = 0; s < (DEQ ? 0 : NSV); ++s)
-      wza[s] = *reinterpret_cast<const u32x4_t *>(&wz[rowsel[s] + (kb * 2 + c) * 16 + half * 8]);
-  };
+    for (int j = 0; j < 16; ++j) oacc[i][j] = 0.f;
+  float l_part = 0.f;   // the softmax denominator, from the weights as rounded for the MFMA (this lane's keys; the lane halves are added in the epilogue)
+  float m_ref = 0.f;    // softmax reference (log2 domain)
+  bool first = true;
 
   // A wavefront raises its priority while it issues the MFMAs of a phase.  Measured per kernel
   // (same run, bit-identical results): at D=128 that is worth 5 % for 4-bit codes (0.725 against
   // 0.762 ms at the configuration-4 shape) and costs 1-3.5 % for 2-bit and 8-bit codes, whose
   // widening has more to do beside the MFMAs; at D=64 it makes no difference.
   constexpr bool MFMA_PRIO = !(D == 128 && BITS != 4);
-  // S^T = K Q^T for one 32-key block; the A operands are the widened K rows in LDS
+  // LDS operands are requested ahead of their use where the registers allow it (the
+  // scheduling fences keep the requests where they are written).
+  floatx16_t sacc;
+  u32 pop[2][4];       // P^T operands, [16-key chunk][dword]
+  u32x4_t vta[NDB];
+  int t0 = 0;
+  const uint16_t *kx = nullptr, *vx = nullptr;
+  // V^T operand of block kb, chunk c, rows d: the lane's 8 keys of channel d * 32 + col, four of them by each read (16 lanes read 4 keys x 16
+  // channels, 8 bytes each, and are handed a channel's four keys)
+  const uint16_t *const v_lane = lds_v + (half * 8 + (lane & 15) / 4) * VS + (lane & 16) + (lane & 3) * 4;
+  typedef short s16x4_t __attribute__((ext_vector_type(4)));
+  typedef __attribute__((address_space(3))) s16x4_t *lds_s16x4;
+  auto load_v_operands = [&](int kb, int c) {
+#pragma unroll
+    for (int d = 0; d < NDB; ++d) {
+      const uint16_t *at = vx + (kb * 32 + c * 16) * VS + d * 32;
+      const uint2 lo = __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4)(at)));
+      const uint2 hi = __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4)(at + 4 * VS)));
+      vta[d] = u32x4_t{lo.x, lo.y, hi.x, hi.y};
+    }
+  };
   auto qk = [&](int kb) {
     if constexpr (MFMA_PRIO) __builtin_amdgcn_s_setprio(1);
-    const int krow_i = kb * 32 + kperm(col);
 #pragma unroll
-    for (int s = 0; s < NSKA; ++s) {
-      floatx16_t zero;
+    for (int j = 0; j < 16; ++j) sacc[j] = 0.f;
+    const uint16_t *const krow = kx + (kb * 32 + kperm(col)) * KS + half * 8;
 #pragma unroll
-      for (int j = 0; j < 16; ++j) zero[j] = 0.f;
-      if constexpr (DEQ) {
-        sacc[kb][s] = zero;   // (dequantized operands: no zero-point term)
-      } else {
-        // starts the accumulator with the zero-point term (see bq above)
-        sacc[kb][s] = mfma_32x32x16<F16>(kz[(s * BN + krow_i) * 2 + half], bq[s], zero);
-      }
-    }
-    const uint16_t *krow = &kx[krow_i * KXS];
-#pragma unroll
-    for (int ch = 0; ch < NCH; ++ch) {
-      const u32x4_t av = *reinterpret_cast<const u32x4_t *>(&krow[k_octet<GK>(ch, half) * 8]);
-      constexpr int kAcc = DEQ ? 0 : 1;
-      sacc[kb][kAcc * (ch / (GK / 16))] = mfma_32x32x16<F16>(av, qb[ch], sacc[kb][kAcc * (ch / (GK / 16))]);
-    }
+    for (int ch = 0; ch < NCH; ++ch) sacc = mfma_32x32x16<F16>(*reinterpret_cast<const u32x4_t *>(krow + ch * 16), qb[ch], sacc);
     if constexpr (MFMA_PRIO) __builtin_amdgcn_s_setprio(0);
   };
 
-  // logits -> P'^T operands of one block: online softmax against a lazily moved reference
+  // logits -> P^T operands of one block: online softmax against a lazily moved reference
   auto softmax = [&](int kb) {
     float z[16];
 #pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      float v = -m_ref;
-#pragma unroll
-      for (int s = 0; s < NSKA; ++s) {
-        const int key = kb * 32 + 16 * (i >> 3) + 8 * half + (i & 7);
-        v = __builtin_fmaf(DEQ ? p.scale_log2e : HOIST ? ckv[kb][s][i] : par[P_CK + s * BN + key],
-                           sacc[kb][s][i], v);
-      }
-      z[i] = v;
-    }
-    // mask: block-causal key limit and the ragged last tile
-    const int lim_t = limit;
+    for (int i = 0; i < 16; ++i) z[i] = __builtin_fmaf(p.scale_log2e, sacc[i], -m_ref);
+    // mask: block-causal key limit and the ragged last tile (register i of this lane <-> key kb*32 + 16*(i/8) + 8*half + i%8 of the tile)
     if (t0 + BN > wave_minlim) {
 #pragma unroll
       for (int i = 0; i < 16; ++i) {
         const int key = t0 + kb * 32 + 16 * (i >> 3) + 8 * half + (i & 7);
-        if (key >= lim_t) z[i] = -INFINITY;
+        if (key >= limit) z[i] = -INFINITY;
       }
     }
     // Moves the softmax reference to the row's current maximum: up only (never down) once
@@ -917,29 +1010,23 @@ __device__ __forceinline__ void attend_block(const AttnParams &p, int bh, int ou
       float zmax = z[0];
 #pragma unroll
       for (int i = 1; i < 16; ++i) zmax = fmaxf(zmax, z[i]);
-      {
-        // the other lane half of the same query, without a trip through LDS
-        const auto sw = __builtin_amdgcn_permlane32_swap(f2u(zmax), f2u(zmax), false, false);
-        zmax = fmaxf(u2f(sw[0]), u2f(sw[1]));
-      }
-      // exact codes: the reference goes kHeadroom octaves above the maximum (see below)
-      constexpr float up = DEQ ? 0.f : kHeadroom;
-      const float delta = first ? ((zmax == -INFINITY) ? 0.f : zmax + up) : fmaxf(zmax + up, 0.f);
-      const float alpha = first ? 1.f : __builtin_amdgcn_exp2f(-delta);
+      // the other lane half of the same query, without a trip through LDS
+      const auto sw = __builtin_amdgcn_permlane32_swap(f2u(zmax), f2u(zmax), false, false);
+      zmax = fmaxf(u2f(sw[0]), u2f(sw[1]));
+      const float delta = first ? (zmax == -INFINITY ? 0.f : zmax) : fmaxf(zmax, 0.f);
       m_ref += delta;
 #pragma unroll
       for (int i = 0; i < 16; ++i) z[i] -= delta;
+      if (!first) {
+        const float alpha = __builtin_amdgcn_exp2f(-delta);
 #pragma unroll
-      for (int d = 0; d < NDB; ++d)
+        for (int d = 0; d < NDB; ++d)
 #pragma unroll
-        for (int j = 0; j < 16; ++j) oacc[d][j] *= alpha;
-#pragma unroll
-      for (int j = 0; j < (DEQ ? 0 : 16); ++j) racc[j] *= alpha;
-      if constexpr (DEQ) l_part *= alpha;
-#pragma unroll
-      for (int s = 0; s < NSVA; ++s) r_run[s] *= alpha;
+          for (int j = 0; j < 16; ++j) oacc[d][j] *= alpha;
+        l_part *= alpha;
+      }
     };
-    // exp2 of the logits, rounded to bf16 pairs for the MFMA; DEQ: also their sum (this lane's keys)
+    // exp2 of the logits, rounded to pairs of the attention's type for the MFMA, and their sum (this lane's keys)
     float blk = 0.f;
     auto weights = [&]() {
       float pv[16];
@@ -947,117 +1034,50 @@ __device__ __forceinline__ void attend_block(const AttnParams &p, int bh, int ou
       for (int i = 0; i < 16; ++i) pv[i] = __builtin_amdgcn_exp2f(z[i]);
       blk = 0.f;
 #pragma unroll
-      for (int s = 0; s < NSVA; ++s)
+      for (int i = 0; i < 16; i += 2) {
+        const u32 w = pack_io_rne<F16>(pv[i], pv[i + 1]);
+        pop[i >> 3][(i & 7) >> 1] = w;
+      }
+      float part[4];   // (four of its weights each, and no sum waits for another)
 #pragma unroll
-        for (int i2 = 0; i2 < 8; ++i2) {
-          const int i = 2 * i2;
-          const int key = kb * 32 + 16 * (i >> 3) + 8 * half + (i & 7);
-          if constexpr (FOLD_SV || DEQ) pop[kb][s][i >> 3][(i & 7) >> 1] = pack_io_rne<F16>(pv[i], pv[i + 1]);
-          else if constexpr (HOIST)
-            pop[kb][s][i >> 3][(i & 7) >> 1] = pack_bf16_rne(pv[i] * svv[kb][s][i], pv[i + 1] * svv[kb][s][i + 1]);
-          else
-            pop[kb][s][i >> 3][(i & 7) >> 1] =
-                pack_bf16_rne(pv[i] * par[P_SV + s * BN + key], pv[i + 1] * par[P_SV + s * BN + key + 1]);
-          if constexpr (DEQ) {   // += the two rounded weights (one v_dot2 against a pair of ones)
-            if constexpr (F16) {
-              typedef _Float16 f16x2_t __attribute__((ext_vector_type(2)));
-              blk = __builtin_amdgcn_fdot2(__builtin_bit_cast(f16x2_t, pop[kb][s][i >> 3][(i & 7) >> 1]),
-                                           __builtin_bit_cast(f16x2_t, 0x3c003c00u), blk, false);
-            } else {
-              typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
-              blk = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2_t, pop[kb][s][i >> 3][(i & 7) >> 1]),
-                                                    __builtin_bit_cast(bf16x2_t, 0x3f803f80u), blk, false);
-            }
-          }
-        }
+      for (int c = 0; c < 2; ++c)
+#pragma unroll
+        for (int i = 0; i < 2; ++i) part[2 * c + i] = add4<F16>(f32x4_t{0.f, 0.f, 0.f, 0.f}, make_uint2(pop[c][2 * i], pop[c][2 * i + 1]))[0];
+      blk = (part[0] + part[1]) + (part[2] + part[3]);
     };
-    if constexpr (DEQ) {
-      // The reference has to move when a logit exceeds it by 2^16.  Rather than look for the
-      // row maximum in every block (eleven instructions of sixty), the weights are computed
-      // against the reference as it stands and their sum is looked at, which the denominator
-      // needs anyway: a weight above 2^16 (or an overflow to infinity) shows in it, and the block
-      // is then redone with the reference moved.  (A sum above 2^16 without such a weight moves
-      // the reference too, which is harmless.)
-      if (first) move_reference();
+    // The reference has to move when a logit exceeds it by 2^16.  Rather than look for the
+    // row maximum in every block (eleven instructions of sixty), the weights are computed
+    // against the reference as it stands and their sum is looked at, which the denominator
+    // needs anyway: a weight above 2^16 (or an overflow to infinity) shows in it, and the block
+    // is then redone with the reference moved.  (A sum above 2^16 without such a weight moves
+    // the reference too, which is harmless.)
+    // (fp16 weights end at 65504: there the reference moves at a block sum of 2^15, which keeps
+    // every weight of an accepted block finite; an overflowed one makes the sum infinite)
+    constexpr float kMoveAt = F16 ? 32768.f : 65536.f;
+    if (first) move_reference();
+    weights();
+    if (!first && __any(!(blk <= kMoveAt))) {
+      move_reference();
       weights();
-      // (fp16 weights end at 65504: there the reference moves at a block sum of 2^15, which keeps
-      // every weight of an accepted block finite; an overflowed one makes the sum infinite)
-      constexpr float kMoveAt = F16 ? 32768.f : 65536.f;
-      if (!first && __any(!(blk <= kMoveAt))) {
-        move_reference();
-        weights();
-      }
-      l_part += blk;
-      first = false;
-    } else {
-      // Here the denominator is summed by the MFMA, so there is no sum to look at; the packed
-      // weights themselves are: all are >= 0, so bit 14 of a bf16 (the top exponent bit) says
-      // "this weight is 2 or more" (infinities included), and an OR over the block's eight words
-      // finds one.  The reference is put kHeadroom octaves above the maximum when it moves, so
-      // weights start at 2^-kHeadroom or below -- bf16 and the fp32 sums keep their relative
-      // precision there -- and it moves again only for a logit 1 + kHeadroom octaves above that
-      // maximum.
-      if (first) move_reference();
-      weights();
-      if (!first) {
-        u32 any_w = 0;
-#pragma unroll
-        for (int s = 0; s < NSVA; ++s)
-#pragma unroll
-          for (int h = 0; h < 2; ++h)
-#pragma unroll
-            for (int j = 0; j < 4; ++j) any_w |= pop[kb][s][h][j];
-        if (__any((any_w & 0x40004000u) != 0)) {
-          move_reference();
-          weights();
-        }
-      }
-      first = false;
     }
-    if (!DEQ && tile_rem) {
-      // the remainder term must see the same bf16-rounded weights as the MFMA
-#pragma unroll
-      for (int s = 0; s < NSVA; ++s)
-#pragma unroll
-        for (int i2 = 0; i2 < 8; ++i2) {
-          const int i = 2 * i2;
-          const int key = kb * 32 + 16 * (i >> 3) + 8 * half + (i & 7);
-          const u32 pk = pop[kb][s][i >> 3][(i & 7) >> 1];
-          r_run[s] = __builtin_fmaf(u2f(pk << 16), par[P_VR + s * BN + key], r_run[s]);
-          r_run[s] = __builtin_fmaf(u2f(pk & 0xffff0000u), par[P_VR + s * BN + key + 1], r_run[s]);
-        }
-    }
+    l_part += blk;
+    first = false;
   };
 
-  // O^T += V^T P'^T for the 32 keys of one block; one more MFMA per chunk and V group
-  // feeds the extra block: its row s collects the zero-point sum of group s and rows
-  // 4..6 (group 0 only) the softmax denominator
-  auto pv_mfma = [&](int kb, bool preloaded) {
+  // O^T += V^T P^T for the 32 keys of one block
+  auto pv_mfma = [&](int kb) {
     if constexpr (MFMA_PRIO) __builtin_amdgcn_s_setprio(1);
 #pragma unroll
     for (int c = 0; c < 2; ++c) {
-      u32x4_t av[NDB], aw[NSVA];
-      if (!(preloaded && c == 0) && !(HOIST && c == 1)) load_v_operands(kb, c);
+      u32x4_t av[NDB];
 #pragma unroll
       for (int d = 0; d < NDB; ++d) av[d] = vta[d];
-#pragma unroll
-      for (int s = 0; s < (DEQ ? 0 : NSVA); ++s) aw[s] = wza[s];
-      if (HOIST && c == 0) {
+      if (c == 0) {
         load_v_operands(kb, 1);   // in flight under this chunk's MFMAs
         __builtin_amdgcn_sched_barrier(0);
       }
 #pragma unroll
-      for (int d = 0; d < NDB; ++d) {
-        constexpr int DBS = GV / 32;  // 32-row blocks per V scale group
-        const int s = DEQ ? 0 : d / DBS;
-        u32x4_t bv = {pop[kb][s][c][0], pop[kb][s][c][1], pop[kb][s][c][2], pop[kb][s][c][3]};
-        oacc[d] = mfma_32x32x16<F16>(av[d], bv, oacc[d]);
-      }
-#pragma unroll
-      for (int s = 0; s < (DEQ ? 0 : NSVA); ++s) {
-        u32x4_t bv = {pop[kb][s][c][0], pop[kb][s][c][1], pop[kb][s][c][2], pop[kb][s][c][3]};
-        racc = mfma_32x32x16<F16>(aw[s], bv, racc);
-      }
+      for (int d = 0; d < NDB; ++d) oacc[d] = mfma_32x32x16<F16>(av[d], u32x4_t{pop[c][0], pop[c][1], pop[c][2], pop[c][3]}, oacc[d]);
     }
     if constexpr (MFMA_PRIO) __builtin_amdgcn_s_setprio(0);
   };
@@ -1067,88 +1087,55 @@ __device__ __forceinline__ void attend_block(const AttnParams &p, int bh, int ou
   // wavefronts still need.  A whole sequence of 680 tokens in ten steps, [8,680,16,64] fp16: a quarter of
   // the workgroups' key blocks; with the order of the query tiles (BlockOf) append and attention 47.5 -> 39.7 us.
   const int wave_tiles = __builtin_amdgcn_readfirstlane(wave_live ? min(n_tiles, (max(wave_end - tile_base, 0) + BN - 1) / BN) : 0);
+  // with the MFMAs of a block in flight: the next tile is widened into the other buffers
+  auto widen_next = [&](int tile) {
+    if (tile + 1 >= n_tiles) return;
+    widen(tile + 1);
+    if (tile + 2 < n_tiles) request(tile + 2);
+  };
   auto attend = [&](int tile) {
-    begin_tile(tile);
+    t0 = tile_base + tile * BN;
+    kx = lds_k + tile % L::kBufs * kKBuf<D>;
+    vx = v_lane + tile % L::kBufs * kVBuf<D>;
     const bool half_tile = wave_end - t0 <= 32;
 #pragma unroll
     for (int kb = 0; kb < 2; ++kb) {
       if (kb == 1 && half_tile) continue;
-      load_scales(kb);
       qk(kb);
-      if constexpr (HOIST) {
-        load_v_operands(kb, 0);   // used after the softmax arithmetic
-        __builtin_amdgcn_sched_barrier(0);
-      }
+      load_v_operands(kb, 0);   // used after the softmax arithmetic
+      __builtin_amdgcn_sched_barrier(0);
       softmax(kb);
-      pv_mfma(kb, HOIST);
+      pv_mfma(kb);
       if (!ONE && kb == 0) widen_next(tile);
     }
   };
   int tile = 0;
   if constexpr (ONE) {
-    // one of each buffer: a tile is staged, widened and attended in turn, with the next one's loads in flight
+    // one of each buffer: a tile is widened and attended in turn, with the next one's loads in flight
     for (; tile < n_tiles; ++tile) {
       if (tile) __syncthreads();   // (the tile before is attended)
-      stage(tile);
-      widen_k(tile);
-      if (tile + 1 < n_tiles) { prefetch_k(tile + 1); prefetch(tile + 1); }
-      __syncthreads();
-      widen_v(tile);
+      widen(tile);
+      if (tile + 1 < n_tiles) request(tile + 1);
       __syncthreads();
       if (tile < wave_tiles) attend(tile);
     }
-  }
-  for (; tile < wave_tiles; ++tile) {
-    attend(tile);
-    __syncthreads();   // the one barrier per tile
-  }
-  // from there on (a wavefront without queries: from the start) the wavefront only helps with staging and
-  // widening, at the same barrier count as the others
-  for (; tile < n_tiles; ++tile) {
-    if (tile + 2 < n_tiles) stage(tile + 2);
-    if (tile + 3 < n_tiles) prefetch(tile + 3);
-    widen_next(tile);
-    __syncthreads();
+  } else {
+    for (; tile < wave_tiles; ++tile) {
+      attend(tile);
+      __syncthreads();   // the one barrier per tile
+    }
+    // from there on (a wavefront without queries: from the start) the wavefront only helps with the
+    // widening, at the same barrier count as the others
+    for (; tile < n_tiles; ++tile) {
+      widen_next(tile);
+      __syncthreads();
+    }
   }
   if (!wave_live) return;
 
   // ---- epilogue -------------------------------------------------------------------
-#pragma unroll
-  for (int s = 0; s < NSVA; ++s) r_run[s] += __shfl_xor(r_run[s], 32, 64);
-  // rows 4..6 of racc are registers 0..2 of the upper lane half, rows 0..3 registers 0..3 of the lower
-  // (DEQ: the denominator is row 0, the sum of the weights against the row of ones)
-  const float l_sum = DEQ ? l_part + __shfl_xor(l_part, 32, 64) : __shfl(racc[0] + racc[1] + racc[2], col + 32, 64);
-  const float inv = l_sum > 0.f ? 1.0f / l_sum : 0.f;
-  float rq[NSVA];
-#pragma unroll
-  for (int s = 0; s < NSVA; ++s) rq[s] = DEQ ? 0.f : __shfl(racc[s], col, 64) + r_run[s];
-  if (q_live) {
-    __bf16 *optr = p.out + (b * p.o_bs + hq * p.o_hs + qrow * p.o_ts) * D;
-    // with the keys shared out: the normalized fp32 output and (reference, denominator) of
-    // this share, for the combining kernel
-    const bool shared_out = p.nsplit > 1;
-    const int64_t prow = ((int64_t)split * p.bh_total + out_pair) * p.Lq + qrow;
-    float *wptr = p.ws_o + prow * D;
-    if (shared_out && half == 0) *reinterpret_cast<float2 *>(p.ws_ml + prow * 2) = make_float2(m_ref, l_sum);
-#pragma unroll
-    for (int d = 0; d < NDB; ++d) {
-      constexpr int DBS = GV / 32;
-      const float r = rq[DEQ ? 0 : d / DBS];
-      constexpr float VM = DEQ ? 1.f : VCodec<BITS>::kMul;   // (DEQ: the accumulators hold values already)
-#pragma unroll
-      for (int g4 = 0; g4 < 4; ++g4) {
-        // registers 4*g4 .. 4*g4+3 are rows d*32 + 8*g4 + 4*half + 0..3 of O^T
-        float o0 = (VM * oacc[d][4 * g4 + 0] - r) * inv, o1 = (VM * oacc[d][4 * g4 + 1] - r) * inv;
-        float o2 = (VM * oacc[d][4 * g4 + 2] - r) * inv, o3 = (VM * oacc[d][4 * g4 + 3] - r) * inv;
-        if (shared_out) {
-          *reinterpret_cast<float4 *>(wptr + d * 32 + 8 * g4 + 4 * half) = make_float4(o0, o1, o2, o3);
-        } else {
-          uint2 v = make_uint2(pack_io_rne<F16>(o0, o1), pack_io_rne<F16>(o2, o3));
-          *reinterpret_cast<uint2 *>(optr + d * 32 + 8 * g4 + 4 * half) = v;
-        }
-      }
-    }
-  }
+  const float l_sum = l_part + __shfl_xor(l_part, 32, 64);
+  store_block<D, F16>(p, b, hq, qrow, q_live, half, split, out_pair, m_ref, l_sum, oacc, [](float o) { return o; });
 }
 
 // Workgroup -> (pair, query tile, share of the keys).  XCD-aware: consecutive workgroup ids go to different
@@ -1175,20 +1162,30 @@ struct BlockOf {
   }
 };
 
-template <int D, int BITS, int GK, int GV, bool CHAN, int NWV = 8, int WPS = 2, bool EXACT = false, bool F16 = false, bool ONE = false>
+// WPS: wavefronts per SIMD the register allocation aims at (2, or 4: two 8-wavefront workgroups
+// per compute unit at 128 registers, which the D=64 kernels afford)
+template <int D, int BITS, bool CHAN, int NWV, int WPS, bool F16, bool ONE>
 __global__ __launch_bounds__(NWV * 64, WPS) void fused_attn_kernel(AttnParams p) {
   const BlockOf k(p);
   if (k.pair >= p.bh_total) return;
-  attend_block<D, BITS, GK, GV, CHAN, NWV, EXACT, F16, ONE>(p, k.pair, k.pair, k.qt, k.split);
+  attend_tiles<D, BITS, CHAN, NWV, F16, ONE>(p, k.pair, k.pair, k.qt, k.split);
 }
 
-template <int D, int G, int NWV, int WPS, bool F16>
+template <int D, int NWV, int WPS, bool F16>
 __global__ __launch_bounds__(NWV * 64, WPS) void fused_attn_classes_kernel(AttnParams p, ClassTable t) {
   const BlockOf k(p);
   if (k.pair >= p.bh_total) return;
   in_class(p, t, k.pair, [&](auto bits, int bh, int out_pair) __attribute__((always_inline)) {
-    attend_block<D, decltype(bits)::value, G, G, false, NWV, false, F16>(p, bh, out_pair, k.qt, k.split);
+    attend_tiles<D, decltype(bits)::value, false, NWV, F16>(p, bh, out_pair, k.qt, k.split);
   });
+}
+
+// ... and with exact codes
+template <int BITS>
+__global__ __launch_bounds__(NW * 64, 2) void exact_attn_kernel(AttnParams p) {
+  const BlockOf k(p);
+  if (k.pair >= p.bh_total) return;
+  attend_codes<BITS>(p, k.pair, k.pair, k.qt, k.split);
 }
 
 // The shares' outputs weighted by their softmax mass l * 2^(m - M), M the largest reference among
@@ -1307,23 +1304,28 @@ template <int D, bool F16> void launch_combine(const AttnParams &p, hipStream_t 
     hipLaunchKernelGGL((combine_splits_kernel<D, F16>), dim3((unsigned)((rows + 1) / 2)), dim3(256), 0, st, p);
 }
 
-template <int D, int BITS, int GK, int GV, bool CHAN, int NWV, int WPS = 2, bool EXACT = false, bool F16 = false, bool ONE = false>
+dim3 tiles_grid(const AttnParams &p) { return dim3((unsigned)((p.bh_total + 7) / 8 * 8 * p.q_tiles * p.nsplit)); }
+template <int D, int BITS, bool CHAN, int NWV, int WPS = 2, bool F16 = false, bool ONE = false>
 void launch_shape(const AttnParams &p, hipStream_t st) {
-  // (the per-channel tables take LDS by the number of segments of the launch)
-  constexpr int lds_base = (AttnLds<D, BITS, GK, GV, CHAN, EXACT, ONE>::kBytes + 15) / 16 * 16, lds_seg = CHAN ? kChanTableRows * D * 4 : 0;
-  constexpr int lds_max = lds_base + kMaxSegments * lds_seg;
+  // (the per-channel tables take LDS by the number of segments of the launch, and half of it without zero-points)
+  constexpr int lds_base = TileLds<D, ONE>::kTables, lds_max = lds_base + (CHAN ? kMaxSegments * 4 * D * 4 : 0);
   static_assert(lds_max <= 160 * 1024, "LDS budget");
-  const int lds_bytes = lds_base + p.nseg * lds_seg;
+  const int lds_bytes = lds_base + (CHAN ? p.nseg * (p.k_chan_zp || p.v_chan_zp ? 4 : 2) * D * 4 : 0);
   static bool configured[64] = {false};
-  allow_lds(reinterpret_cast<const void *>(&fused_attn_kernel<D, BITS, GK, GV, CHAN, NWV, WPS, EXACT, F16, ONE>), lds_max, configured);
-  const int bh_pad = (p.bh_total + 7) / 8 * 8;
-  dim3 grid((unsigned)(bh_pad * p.q_tiles * p.nsplit));
-  hipLaunchKernelGGL((fused_attn_kernel<D, BITS, GK, GV, CHAN, NWV, WPS, EXACT, F16, ONE>), grid, dim3(NWV * 64), lds_bytes, st, p);
+  allow_lds(reinterpret_cast<const void *>(&fused_attn_kernel<D, BITS, CHAN, NWV, WPS, F16, ONE>), lds_max, configured);
+  hipLaunchKernelGGL((fused_attn_kernel<D, BITS, CHAN, NWV, WPS, F16, ONE>), tiles_grid(p), dim3(NWV * 64), lds_bytes, st, p);
   if (p.nsplit > 1) launch_combine<D, F16>(p, st);
+}
+template <int BITS> void launch_exact(const AttnParams &p, hipStream_t st) {
+  constexpr int lds_bytes = ExactLds<BITS>::kBytes;
+  static bool configured[64] = {false};
+  allow_lds(reinterpret_cast<const void *>(&exact_attn_kernel<BITS>), lds_bytes, configured);
+  hipLaunchKernelGGL((exact_attn_kernel<BITS>), tiles_grid(p), dim3(NW * 64), lds_bytes, st, p);
+  if (p.nsplit > 1) launch_combine<128, false>(p, st);
 }
 
 // The workgroups at D=64, F16 or not.
-template <int BITS, int GK, int GV, bool CHAN, bool F16> void launch_d64(const AttnParams &p, hipStream_t st) {
+template <int BITS, bool CHAN, bool F16> void launch_d64(const AttnParams &p, hipStream_t st) {
   // More (batch, head) pairs than compute units, at most four wavefronts of queries each:
   // workgroups of four wavefronts (same arithmetic, same results).  Also for one or two
   // wavefronts of queries: the wavefronts without queries share the staging and the widening
@@ -1339,68 +1341,58 @@ template <int BITS, int GK, int GV, bool CHAN, bool F16> void launch_d64(const A
   // groups 8.2 -> 8.4, 10.8 -> 11.1, with 512 6.8 -> 7.1, 8.9 -> 9.3.
   if (p.Lq <= 128 && p.bh_total > device_cus()) {
     const bool rounds = (int64_t)p.bh_total * p.nsplit > 3 * device_cus() && (CHAN || BITS != 2);
-    if (p.Lk <= BN || rounds) launch_shape<64, BITS, GK, GV, CHAN, 4, 4, false, F16, true>(p, st);
-    else launch_shape<64, BITS, GK, GV, CHAN, 4, 3, false, F16>(p, st);
+    if (p.Lk <= BN || rounds) launch_shape<64, BITS, CHAN, 4, 4, F16, true>(p, st);
+    else launch_shape<64, BITS, CHAN, 4, 3, F16>(p, st);
     return;
   }
   // The kernels at D=64 fit 128 registers at the price of 24-48 bytes of spills,
   // and two resident workgroups per compute unit hide each other's prologue and barriers
   // (8-15 % faster than one workgroup at 140 registers).
-  launch_shape<64, BITS, GK, GV, CHAN, 8, 4, false, F16>(p, st);
+  launch_shape<64, BITS, CHAN, 8, 4, F16>(p, st);
 }
 
-template <int D, int BITS, int GK, int GV, bool CHAN = false>
-void launch(const AttnParams &p, hipStream_t st) {
+template <int D, int BITS, bool CHAN> void launch(const AttnParams &p, hipStream_t st) {
   if constexpr (D == 64) {
     // fp16 operands (the VAR path; every VAR model has head dim 64) or bf16 ones
-    if (p.f16) launch_d64<BITS, GK, GV, CHAN, true>(p, st);
-    else launch_d64<BITS, GK, GV, CHAN, false>(p, st);
+    if (p.f16) launch_d64<BITS, CHAN, true>(p, st);
+    else launch_d64<BITS, CHAN, false>(p, st);
   } else {
-    if constexpr (AttnForms<D, BITS, GK, GV, CHAN>::kHasExact) {
-      if (p.exact_codes) {
-        launch_shape<D, BITS, GK, GV, CHAN, 8, 2, true>(p, st);
-        return;
-      }
-    }
-    launch_shape<D, BITS, GK, GV, CHAN, 8>(p, st);
+    launch_shape<D, BITS, CHAN, 8>(p, st);
+  }
+}
+template <bool CHAN> void launch_any(const AttnParams &p, int D, int bits, hipStream_t st) {
+  if (D == 128) {
+    if (bits == 4) launch<128, 4, CHAN>(p, st);
+    else if (bits == 8) launch<128, 8, CHAN>(p, st);
+    else launch<128, 2, CHAN>(p, st);
+  } else {
+    if (bits == 4) launch<64, 4, CHAN>(p, st);
+    else if (bits == 8) launch<64, 8, CHAN>(p, st);
+    else launch<64, 2, CHAN>(p, st);
   }
 }
 
-template <int D, int BITS>
-int dispatch_groups(const AttnParams &p, int gk, int gv, hipStream_t st) {
-#define VARQ_G(GK_, GV_)                                   \
-  if (gk == GK_ && gv == GV_) {                            \
-    if constexpr (GK_ <= D && GV_ <= D) {                  \
-      launch<D, BITS, GK_, GV_>(p, st);                    \
-      return 0;                                            \
-    }                                                      \
-  }
-  VARQ_G(128, 128) VARQ_G(64, 64) VARQ_G(32, 32) VARQ_G(32, 64)
-#undef VARQ_G
-  return -1;
-}
-// the pairs above: what the other paths of the same call are held to as well
+// the scale groups that are served
 bool groups_served(int D, int gk, int gv) {
   return ((gk == gv && (gk == 128 || gk == 64 || gk == 32)) || (gk == 32 && gv == 64)) && gk <= D;
 }
 
-template <int D, int G, int NWV, int WPS, bool F16>
+template <int D, int NWV, int WPS, bool F16>
 void launch_classes_shape(const AttnParams &p, const ClassTable &t, hipStream_t st) {
-  constexpr int lds = std::max({AttnLds<D, 8, G, G, false>::kBytes, AttnLds<D, 4, G, G, false>::kBytes, AttnLds<D, 2, G, G, false>::kBytes});
+  constexpr int lds = TileLds<D, false>::kTables;
   static bool configured[64] = {false};
-  allow_lds(reinterpret_cast<const void *>(&fused_attn_classes_kernel<D, G, NWV, WPS, F16>), lds, configured);
-  dim3 grid((unsigned)((p.bh_total + 7) / 8 * 8 * p.q_tiles * p.nsplit));
-  hipLaunchKernelGGL((fused_attn_classes_kernel<D, G, NWV, WPS, F16>), grid, dim3(NWV * 64), lds, st, p, t);
+  allow_lds(reinterpret_cast<const void *>(&fused_attn_classes_kernel<D, NWV, WPS, F16>), lds, configured);
+  hipLaunchKernelGGL((fused_attn_classes_kernel<D, NWV, WPS, F16>), tiles_grid(p), dim3(NWV * 64), lds, st, p, t);
   if (p.nsplit > 1) launch_combine<D, F16>(p, st);
 }
 // (the workgroup sizes by the rules of launch())
-template <int D, int G> void launch_classes(const AttnParams &p, const ClassTable &t, hipStream_t st) {
+template <int D> void launch_classes(const AttnParams &p, const ClassTable &t, hipStream_t st) {
   if constexpr (D == 64) {
     const bool four = p.Lq <= 128 && p.bh_total > device_cus();
-    if (p.f16) { if (four) launch_classes_shape<D, G, 4, 3, true>(p, t, st); else launch_classes_shape<D, G, 8, 4, true>(p, t, st); }
-    else { if (four) launch_classes_shape<D, G, 4, 3, false>(p, t, st); else launch_classes_shape<D, G, 8, 4, false>(p, t, st); }
+    if (p.f16) { if (four) launch_classes_shape<D, 4, 3, true>(p, t, st); else launch_classes_shape<D, 8, 4, true>(p, t, st); }
+    else { if (four) launch_classes_shape<D, 4, 3, false>(p, t, st); else launch_classes_shape<D, 8, 4, false>(p, t, st); }
   } else {
-    launch_classes_shape<D, G, 8, 2, false>(p, t, st);
+    launch_classes_shape<D, 8, 2, false>(p, t, st);
   }
 }
 
@@ -1690,19 +1682,17 @@ extern "C" int varq_fused_attn(const void *q, void *out,
     return VARQ_OK;
   }
   if (int e = set_splits(p, D, (Lk + BN - 1) / BN, splits, workspace, workspace_bytes, "fused_attn")) return e;
-  int rc = -1;
-  if (D == 128) {
-    if (k_bits == 4) rc = dispatch_groups<128, 4>(p, k_group, v_group, st);
-    else if (k_bits == 8) rc = dispatch_groups<128, 8>(p, k_group, v_group, st);
-    else rc = dispatch_groups<128, 2>(p, k_group, v_group, st);
-  } else {
-    if (k_bits == 4) rc = dispatch_groups<64, 4>(p, k_group, v_group, st);
-    else if (k_bits == 8) rc = dispatch_groups<64, 8>(p, k_group, v_group, st);
-    else rc = dispatch_groups<64, 2>(p, k_group, v_group, st);
-  }
-  if (rc)
+  if (!groups_served(D, k_group, v_group))
     return varq_set_error(VARQ_ERR_UNSUPPORTED, "fused_attn: no kernel for D=%d bits=%d k_group=%d v_group=%d", D, k_bits,
                           k_group, v_group);
+  p.k_shift = varq_log2_exact(k_group);
+  p.v_shift = varq_log2_exact(v_group);
+  if (exact_form) {
+    if (k_bits == 4) launch_exact<4>(p, st);
+    else launch_exact<2>(p, st);
+  } else {
+    launch_any<false>(p, D, k_bits, st);
+  }
   VARQ_CHECK_LAUNCH("fused_attn");
   return VARQ_OK;
 }
@@ -1775,15 +1765,7 @@ extern "C" int varq_fused_attn_channel(const void *q, void *out,
   }
   if (int e = set_splits(p, D, (Lk + BN - 1) / BN, splits, workspace, workspace_bytes, "fused_attn_channel"))
     return e;
-  if (D == 128) {
-    if (bits == 4) launch<128, 4, 128, 128, true>(p, st);
-    else if (bits == 8) launch<128, 8, 128, 128, true>(p, st);
-    else launch<128, 2, 128, 128, true>(p, st);
-  } else {
-    if (bits == 4) launch<64, 4, 64, 64, true>(p, st);
-    else if (bits == 8) launch<64, 8, 64, 64, true>(p, st);
-    else launch<64, 2, 64, 64, true>(p, st);
-  }
+  launch_any<true>(p, D, bits, st);
   VARQ_CHECK_LAUNCH("fused_attn_channel");
   return VARQ_OK;
 }
@@ -1857,14 +1839,9 @@ extern "C" int varq_fused_attn_classes(const void *q, void *out, const varq_kv_c
              })) {
   } else {
     if (int e = set_splits(p, D, (Lk + BN - 1) / BN, splits, workspace, workspace_bytes, "fused_attn_classes")) return e;
-    if (D == 128) {
-      if (group == 128) launch_classes<128, 128>(p, t, st);
-      else if (group == 64) launch_classes<128, 64>(p, t, st);
-      else launch_classes<128, 32>(p, t, st);
-    } else {
-      if (group == 64) launch_classes<64, 64>(p, t, st);
-      else launch_classes<64, 32>(p, t, st);
-    }
+    p.k_shift = p.v_shift = varq_log2_exact(group);
+    if (D == 128) launch_classes<128>(p, t, st);
+    else launch_classes<64>(p, t, st);
   }
   VARQ_CHECK_LAUNCH("fused_attn_classes");
   return VARQ_OK;
