@@ -1197,43 +1197,41 @@ __global__ __launch_bounds__(NW * 64, 2) void exact_attn_kernel(AttnParams p) {
 template <int D, bool F16>
 __global__ __launch_bounds__(256) void combine_splits_kernel(AttnParams p) {
   constexpr int QUADS = D / 4, ROWS = 2, G = 256 / (ROWS * QUADS);
-  constexpr int kMaxS = 64;
+  constexpr int kMaxS = 64, kEarly = 4;
   static_assert(G >= 1 && kMaxS >= kMaxKeyShares_v && kMaxS >= kMaxSplits_v, "share counts");
   __shared__ float w_lds[ROWS][kMaxS];
   const int64_t rows = (int64_t)p.bh_total * p.Lq;
   const int tid = threadIdx.x;
   const int64_t row0 = (int64_t)blockIdx.x * ROWS;
-  // weights of the rows' shares
-  __shared__ float2 ml_lds[ROWS][kMaxS];
-  static_assert(ROWS * kMaxS <= 256, "one (row, share) per thread");
-  const int wr = tid / kMaxS, wsh = tid % kMaxS;
+  const int r = tid / (QUADS * G), gq = tid % (QUADS * G), grp = gq / QUADS, c0 = (gq % QUADS) * 4;
+  const int64_t row = row0 + r, row_c = row < rows ? row : rows - 1;
+  // The thread's first shares are requested along with the statistics, and a row's weights are formed by the wavefront whose lanes are its
+  // shares: one trip to memory instead of two, and no loop over the shares (16 shares of 512 rows, D=128, with the launch before it: 20.4 -> 19.4 us).
+  const float *const o_row = p.ws_o + row_c * D + c0;
+  float4 o[kEarly];
+#pragma unroll
+  for (int u = 0; u < kEarly; ++u) o[u] = *reinterpret_cast<const float4 *>(o_row + (int64_t)min(grp + u * G, p.nsplit - 1) * rows * D);
+  static_assert(kMaxS == 64 && ROWS * kMaxS <= 256, "one wavefront per row, one lane per share");
   if (tid < ROWS * kMaxS) {
+    const int wr = tid / kMaxS, wsh = tid % kMaxS;
     float2 ml = make_float2(0.f, 0.f);   // (denominator 0: an empty share)
     if (wsh < p.nsplit && row0 + wr < rows) ml = *reinterpret_cast<const float2 *>(p.ws_ml + ((int64_t)wsh * rows + row0 + wr) * 2);
-    ml_lds[wr][wsh] = ml;
-  }
-  __syncthreads();
-  if (tid < ROWS * kMaxS) {
-    float m_max = -INFINITY;
-    for (int t = 0; t < p.nsplit; ++t)
-      if (ml_lds[wr][t].y != 0.f) m_max = fmaxf(m_max, ml_lds[wr][t].x);
-    const float2 ml = ml_lds[wr][wsh];
+    const float m_max = group_allreduce<64, true>(ml.y != 0.f ? ml.x : -INFINITY);
     w_lds[wr][wsh] = ml.y != 0.f ? ml.y * __builtin_amdgcn_exp2f(ml.x - m_max) : 0.f;
   }
   __syncthreads();
-  const int r = tid / (QUADS * G), gq = tid % (QUADS * G), grp = gq / QUADS, c0 = (gq % QUADS) * 4;
-  const int64_t row = row0 + r;
   float acc[4] = {0.f, 0.f, 0.f, 0.f}, wsum = 0.f;
-  if (row < rows) {
+  auto add = [&](int share, float4 x) {
+    const float w = w_lds[r][share];
+    acc[0] = __builtin_fmaf(w, x.x, acc[0]); acc[1] = __builtin_fmaf(w, x.y, acc[1]);
+    acc[2] = __builtin_fmaf(w, x.z, acc[2]); acc[3] = __builtin_fmaf(w, x.w, acc[3]);
+    wsum += w;
+  };
+#pragma unroll
+  for (int u = 0; u < kEarly; ++u)
+    if (grp + u * G < p.nsplit) add(grp + u * G, o[u]);
 #pragma unroll 4
-    for (int s_ = grp; s_ < p.nsplit; s_ += G) {
-      const float w = w_lds[r][s_];
-      const float4 o = *reinterpret_cast<const float4 *>(p.ws_o + ((int64_t)s_ * rows + row) * D + c0);
-      acc[0] = __builtin_fmaf(w, o.x, acc[0]); acc[1] = __builtin_fmaf(w, o.y, acc[1]);
-      acc[2] = __builtin_fmaf(w, o.z, acc[2]); acc[3] = __builtin_fmaf(w, o.w, acc[3]);
-      wsum += w;
-    }
-  }
+  for (int s_ = grp + kEarly * G; s_ < p.nsplit; s_ += G) add(s_, *reinterpret_cast<const float4 *>(o_row + (int64_t)s_ * rows * D));
   if constexpr (G > 1) {
     // the groups of a row's shares meet through LDS (group 0 collects)
     __shared__ float part[256][5];
