@@ -131,8 +131,8 @@ int varq_quant_pack_classes(const void *k, const void *v, int x_dtype, int layou
 /*
  * General quantizer for the six grouping methods of VAR_Q/quant.py:75-95 and
  * any other reduce set: a group is every element sharing the indices of the
- * dims NOT in reduce_mask (bit d set = dim d reduced).  Two phases: group
- * min/max into `workspace`, then scale/zp and codes (VAR_Q/quant.py:112-121).
+ * dims NOT in reduce_mask (bit d set = dim d reduced): group min/max, through
+ * `workspace` where workgroups exchange it, then scale/zp and codes (VAR_Q/quant.py:112-121).
  *   x       [shape[0..3]] contiguous
  *   scale   [n_groups] fp32 in the order of the kept dims; zp likewise or NULL
  *   words   packed output [rows, ceil(c/(32/bits))] or NULL
@@ -158,13 +158,21 @@ int varq_quant_pack(const void *x, int x_dtype, const int64_t *host_shape4, int 
 /*
  * The same for two tensors of one shape and dtype with separate outputs and a shared output
  * map -- K and V of a step, which the reference quantizes one after the other
- * (Infinity/infinity/models/basic.py:329-330) -- in the same three launches.  The workspace
+ * (Infinity/infinity/models/basic.py:329-330) -- in the same launches.  The workspace
  * holds 2 * varq_quant_workspace_bytes(...) bytes.  Results are those of two varq_quant_pack calls.
  */
 int varq_quant_pack2(const void *x0, const void *x1, int x_dtype, const int64_t *host_shape4, int reduce_mask,
                      int bits, int asym, float eps, int32_t *words0, int8_t *codes0, float *scale0, float *zp0,
                      int32_t *words1, int8_t *codes1, float *scale1, float *zp1,
                      const int64_t *host_out_map, void *workspace, size_t workspace_bytes, void *stream);
+
+/*
+ * varq_quant_pack with the time given that a workgroup waits for the others with which it shares its groups, in ticks of 10 ns, before
+ * it reads all of their rows by itself (0: without waiting).  Results do not depend on it.
+ */
+int varq_quant_pack_wait(const void *x, int x_dtype, const int64_t *host_shape4, int reduce_mask, int bits, int asym, float eps, int32_t *words,
+                         int8_t *codes, float *scale, float *zp, const int64_t *host_out_map, uint32_t wait_ticks, void *workspace,
+                         size_t workspace_bytes, void *stream);
 
 /*
  * varq_quant_pack / varq_quant_pack2 (x1 != NULL) of groups that take in whole rows (reduce bit 3 set), with the scale of a group

@@ -1,0 +1,74 @@
+"""Workgroups that share their groups (`quant_shared_kernel`): rows that do not fill the last workgroup or step, more rows than the
+registers hold, octets that are no power of two, kept inner indices that do not fill the last tile, groups of whole rows; with the
+others' extremes waited for and, without waiting, with all rows read by whoever comes first.  Bit-exact against the CPU oracle."""
+import pytest
+import torch
+
+import varq_oracle as O
+from gpu_util import note
+from var_q_amd import _lib, ops
+
+pytestmark = pytest.mark.gpu
+
+
+def _without_waiting(x, dims, bits, asym, pack):
+    mask = sum(1 << d for d in dims)
+    lib, sh = _lib.load(), _lib.i64arr(list(x.shape))
+    groups = [1 if d in dims else n for d, n in enumerate(x.shape)]
+    s = torch.empty(groups, device=x.device)
+    z = torch.empty(groups, device=x.device) if asym else None
+    q = torch.empty(*x.shape[:3], x.shape[3] * bits // 32 if pack else x.shape[3], dtype=torch.int32 if pack else torch.int8, device=x.device)
+    size = lib.varq_quant_workspace_bytes(sh, mask)
+    ws = torch.full(((size + 3) // 4,), -1, dtype=torch.int32, device=x.device)   # (any contents)
+    dt = {torch.float32: 0, torch.bfloat16: 1, torch.float16: 2}[x.dtype]
+    _lib.check(lib.varq_quant_pack_wait(x.data_ptr(), dt, sh, mask, bits, int(asym), 1e-12, q.data_ptr() if pack else None,
+                                        None if pack else q.data_ptr(), s.data_ptr(), z.data_ptr() if asym else None, None, 0, ws.data_ptr(), size,
+                                        torch.cuda.current_stream().cuda_stream), 'varq_quant_pack_wait')
+    return q, s, z
+
+
+@pytest.mark.parametrize('shape,dims,dtype', [
+    ((2, 4, 16500, 64), (0, 2), torch.bfloat16),      # 1024 workgroups of five steps
+    ((64, 513, 3, 64), (0, 1), torch.float16),        # two kept indices to a block, the last block half full
+    ((3, 11003, 5, 72), (0, 1), torch.float32),       # nine octets of sixteen lanes
+    ((1, 2, 70001, 96), (0, 2), torch.bfloat16),      # 18 steps: two beyond the held ones
+    ((2, 2, 35001, 128), (0, 2), torch.float32),      # 18 steps of which 8 are held
+    ((1, 4, 8300, 256), (0, 2), torch.float16),       # as many groups as a workgroup takes
+    ((2, 30, 7000, 64), (0, 2, 3), torch.bfloat16),   # groups of whole rows
+    ((32, 30, 421, 64), (0, 1, 3), torch.bfloat16),
+])
+def test_shared_groups(dev, shape, dims, dtype):
+    g = torch.Generator().manual_seed(sum(shape))
+    x = (torch.randn(*shape, generator=g) * 2).to(dtype)
+    x[..., 3] *= 15
+    x[0, 0, 0] = 0
+    x[-1, -1, -1] = 40                                # the extreme of its groups, in the last rows of the last workgroup
+    for bits, asym, pack in ((8, False, True), (2 if shape[3] % 16 == 0 else 4, True, True), (5, False, False)):
+        note('quant shared', shape, dims, dtype, bits, asym, pack)
+        q, s, z = O.quant_reduce(x, dims, bits, asym)
+        if pack:
+            q = O.pack_last_dim(q, bits)[0]
+        for got in (ops.quant_pack(x.to(dev), dims, bits, asym=asym, pack=pack), _without_waiting(x.to(dev), dims, bits, asym, pack)):
+            torch.cuda.synchronize()
+            assert torch.equal(got[1].cpu(), s)
+            assert not asym or torch.equal(got[2].cpu(), z)
+            assert torch.equal(got[0].cpu(), q)
+
+
+def test_shared_groups_in_a_graph(dev):
+    """The words that the workgroups exchange are cleared by every replay; K and V of a step in one launch."""
+    shape, dims = (64, 129, 16, 64), (0, 1)
+    xs = [torch.randn(*shape, device=dev).half() for _ in range(2)]
+    ops.quant_pack_pair(*xs, dims, 8, asym=True)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        got = ops.quant_pack_pair(*xs, dims, 8, asym=True)
+    for factor in (4.0, 0.25, 0.5, 2.0):              # (groups that shrink: extremes left by the last replay would show)
+        for x in xs:
+            x.mul_(factor)
+        note('quant shared, replay', factor)
+        graph.replay()
+        torch.cuda.synchronize()
+        for (q, s, z), x in zip(got, xs):
+            rq, rs, rz = O.quant_reduce(x.cpu(), dims, 8, True)
+            assert torch.equal(s.cpu(), rs) and torch.equal(z.cpu(), rz) and torch.equal(q.cpu(), O.pack_last_dim(rq, 8)[0])

@@ -2,7 +2,7 @@
 library is missing or a call fails, an exception is raised."""
 import ctypes
 import os
-from ctypes import POINTER, c_char_p, c_float, c_int, c_int32, c_int64, c_size_t, c_void_p
+from ctypes import POINTER, c_char_p, c_float, c_int, c_int32, c_int64, c_size_t, c_uint32, c_void_p
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(HERE, 'libvarq_hip.so')
@@ -22,6 +22,8 @@ SYMBOLS = {
     'varq_quant_workspace_bytes': (c_size_t, [POINTER(c_int64), c_int]),
     'varq_quant_pack': (c_int, [c_void_p, c_int, POINTER(c_int64), c_int, c_int, c_int, c_float,
                                 c_void_p, c_void_p, c_void_p, c_void_p, POINTER(c_int64), c_void_p, c_size_t, c_void_p]),
+    'varq_quant_pack_wait': (c_int, [c_void_p, c_int, POINTER(c_int64), c_int, c_int, c_int, c_float, c_void_p, c_void_p, c_void_p, c_void_p,
+                                     POINTER(c_int64), c_uint32, c_void_p, c_size_t, c_void_p]),
     'varq_quant_pack2': (c_int, [c_void_p, c_void_p, c_int, POINTER(c_int64), c_int, c_int, c_int, c_float,
                                  c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p,
                                  POINTER(c_int64), c_void_p, c_size_t, c_void_p]),

@@ -1,6 +1,7 @@
 // General two-phase quantizer: groups that span rows (the six grouping methods
 // of VAR_Q/quant.py:75-95, which all reduce over the batch dim, plus any other
-// reduce set).  A single HBM read cannot serve such groups, so:
+// reduce set).  Where workgroups can hold the rows in registers, one launch reads the input once (quant_one_kernel,
+// quant_shared_kernel); otherwise:
 //   phase A  group min/max (or max-abs): one partial per (chunk, group) in the
 //            workspace, no atomics (tiled path below)
 //   finalize fold the partials -> scale / zero-point      (VAR_Q/quant.py:112-116)
@@ -666,6 +667,215 @@ __global__ __launch_bounds__(NT) void quant_one_kernel(GenParams p, OnePlan pl) 
   quant_one_block<DT, ASYM, KEEPC, NT, NI>(p, pl, [](u32, int, const auto &, const auto &) {});
 }
 
+// ---- one pass by workgroups that share their groups ----------------------------------------------
+// Where the rows of a group are too many for a workgroup: `n` workgroups of 256 threads take a block's rows, full rows of 256 bytes
+// together with their neighbours', hold 16 octets (fp32: 8) per thread, exchange the extremes and quantize what they hold.  All of them
+// are on the chip at once, four to a compute unit, and rows beyond the held ones are read again, the last ones first.  Bound by memory: the input
+// is read once where the three launches read it twice, and where one launch holds a group in one workgroup, pieces of 16 bytes of
+// a row cost it a request to the L2 each.  What the exchange costs, with the launch that clears its words, is about 9 us.  Three launches or one -> this,
+// us, 8 bits, a scale per (head, channel): fp16 [64,n,16,64], two tensors, n = 100 23.8 -> 18.1, 169 31.0 -> 24.0, 256 40.9 -> 32.7; bf16
+// [2,16,4096,128], two, 36.3 -> 32.1; affine, 2 bits, [B,30,680,64] B = 8 21.6 -> 16.8, 32 45.3 -> 38.5; fp32 B = 16 42.3 -> 29.2, 80 207 -> 168;
+// bf16 [600,30,680,64] 940 -> 859; one scale per head, [32,30,680,64] 4 bits 44.7 -> 34.9, one per token 45.7 -> 34.7.
+// The workgroups that share the groups of a block (see quant_shared_kernel): `n` of them, what they exchange and how long one
+// waits for the others, in ticks of 10 ns.
+struct Shards {
+  int n;
+  u32 *mx, *mn, *arrived;       // per group, `stride` words apart; per block, `spacing` words apart: how many have arrived, and half of that on, whether all
+  int stride, spacing;
+  u32 ticks;
+};
+constexpr int kSharedGroups = 1024;   // groups of a workgroup, and values of its fold
+__global__ __launch_bounds__(256) void clear_shards_kernel(GenParams p, Shards sh, int64_t n_groups, int blocks) {
+  if (take_second(p)) { sh.mx += p.ws1; sh.mn += p.ws1; sh.arrived += p.ws1; }
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (i < n_groups) { sh.mx[i * sh.stride] = 0u; sh.mn[i * sh.stride] = 0xffffffffu; }
+  if (i < blocks) { sh.arrived[sh.spacing * i] = 0u; sh.arrived[sh.spacing * i + sh.spacing / 2] = 0u; }
+}
+template <int DT, bool ASYM, bool KEEPC>
+__global__ __launch_bounds__(256, 4) void quant_shared_kernel(GenParams p, OnePlan pl, Shards sh) {
+  constexpr int NV = KEEPC ? 8 : 1, NI = DT == VARQ_F32 ? 8 : 16, kAhead = NI / 4;   // octets held; requested at once beyond them
+  __shared__ float lds_mx[kSharedGroups];
+  __shared__ float lds_mn[ASYM ? kSharedGroups : 1];
+  __shared__ float par_s[kSharedGroups], par_r[kSharedGroups];
+  __shared__ float par_z[ASYM ? kSharedGroups : 1];
+  __shared__ u32 all_here;
+  if (take_second(p)) { sh.mx += p.ws1; sh.mn += p.ws1; sh.arrived += p.ws1; }
+  const int blk = blockIdx.x / sh.n, shard = blockIdx.x - blk * sh.n, tq = blk % pl.tilesQ, ko = blk / pl.tilesQ;
+  const int tid = threadIdx.x, c8s = 1 << pl.c8s_shift, sub = 1 << pl.sub_shift;
+  const int col = tid & (c8s - 1), f = (tid >> pl.c8s_shift) & (sub - 1), lq = tid >> (pl.c8s_shift + pl.sub_shift);
+  const int f0 = shard * (pl.steps << pl.sub_shift) + f, q = (tq << pl.lq_shift) + lq;   // f0: the thread's first row
+  const bool live = col < p.c8 && q < pl.Q;
+  // (rows fit 31 bits and the bytes of a tensor 32)
+  const u32 row0 = (u32)ko * (u32)pl.ko_rs + (live ? q : 0);
+  auto row_at = [&](int step) { return (step << pl.sub_shift) + f0; };
+  auto has = [&](int step) { return step < pl.steps && row_at(step) < pl.RR; };
+  auto row_of = [&](int j) {
+    const u32 o = pl.by_RI((u32)j);
+    return row0 + o * (u32)pl.ro_rs + ((u32)j - o * (u32)pl.RI);
+  };
+  auto octet_at = [&](u32 row) { return reinterpret_cast<const Raw8<DT> *>(reinterpret_cast<const char *>(p.x) + (row * (u32)p.c + col * 8) * (u32)In8<DT>::kBytes); };
+
+  Raw8<DT> raw[NI];
+#pragma unroll
+  for (int s = 0; s < NI; ++s)
+    if (live && has(s)) raw[s] = *octet_at(row_of(row_at(s)));
+  float mx[NV], mn[NV];
+#pragma unroll
+  for (int j = 0; j < NV; ++j) { mx[j] = ASYM ? -INFINITY : 0.f; mn[j] = INFINITY; }
+  auto extend = [&](const Raw8<DT> &octet) __attribute__((always_inline)) {
+    float v[8];
+    octet.widen(v);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      if (ASYM) { mx[j % NV] = fmaxf(mx[j % NV], v[j]); mn[j % NV] = fminf(mn[j % NV], v[j]); }
+      else mx[j % NV] = fmaxf(mx[j % NV], fabsf(v[j]));
+    }
+  };
+#pragma unroll
+  for (int s = 0; s < NI; ++s)
+    if (live && has(s)) extend(raw[s]);
+  if (live) {
+    for (int i = NI; i < pl.steps; i += kAhead) {
+      Raw8<DT> more[kAhead];
+#pragma unroll
+      for (int u = 0; u < kAhead; ++u) if (has(i + u)) more[u] = *octet_at(row_of(row_at(i + u)));
+#pragma unroll
+      for (int u = 0; u < kAhead; ++u) if (has(i + u)) extend(more[u]);
+    }
+  }
+  // fold over f (and, with the channel dim reduced, over the columns), inside the wavefront first, as in quant_one_block
+  const int q_lanes = sub << pl.c8s_shift, gcols = KEEPC ? c8s * 8 : 1;
+  const int parts = q_lanes > 64 ? q_lanes >> 6 : 1, lane_in_part = q_lanes > 64 ? tid & 63 : tid & (q_lanes - 1);
+  const int part = q_lanes > 64 ? tid >> 6 : tid / q_lanes;
+  auto fold = [&]() __attribute__((always_inline)) {
+    for (int off = KEEPC ? c8s : 1; off < 64 && off < q_lanes; off <<= 1) {
+#pragma unroll
+      for (int j = 0; j < NV; ++j) {
+        mx[j] = fmaxf(mx[j], __shfl_xor(mx[j], off, 64));
+        if (ASYM) mn[j] = fminf(mn[j], __shfl_xor(mn[j], off, 64));
+      }
+    }
+    if (lane_in_part < (KEEPC ? c8s : 1)) {
+#pragma unroll
+      for (int j = 0; j < NV; ++j) {
+        lds_mx[part * gcols + col * NV + j] = mx[j];
+        if (ASYM) lds_mn[part * gcols + col * NV + j] = mn[j];
+      }
+    }
+    __syncthreads();
+  };
+  fold();
+  // body(t, whether there is such a group, its number, its extremes in this workgroup), a thread per group
+  const int n_par = gcols << pl.lq_shift;
+  auto per_group = [&](auto &&body) __attribute__((always_inline)) {
+    for (int t = tid; t < n_par; t += 256) {
+      const int tl = t / gcols, g8 = t - tl * gcols, tqi = (tq << pl.lq_shift) + tl;
+      float m = ASYM ? -INFINITY : 0.f, n = INFINITY;
+      for (int w = 0; w < parts; ++w) {
+        m = fmaxf(m, lds_mx[(tl * parts + w) * gcols + g8]);
+        if (ASYM) n = fminf(n, lds_mn[(tl * parts + w) * gcols + g8]);
+      }
+      body(t, tqi < pl.Q && (!KEEPC || g8 < p.c), (int64_t)ko * pl.ko_gs + (int64_t)tqi * pl.q_gs + (KEEPC ? g8 : 0), m, n);
+    }
+  };
+  // The extremes of all workgroups of the block meet in memory.  Nothing but these words goes from one workgroup to another, and every
+  // access to them is an atomic of the device's scope, which all XCDs perform at one place: an extreme whose old value has come back is
+  // there, the count goes up after that, and who has seen the count reads behind it.  (A release and an acquire instead write back and drop
+  // whole L2s, once per workgroup: [64,256,16,64] fp16, two tensors, 33 -> 76 us.)  The last to arrive sets a word of its own,
+  // half a `spacing` from the count, which the others look at: with all of them polling the counts, side by side, 56 us.
+  per_group([&](int, bool mine, int64_t g, float m, float n) __attribute__((always_inline)) {
+    if (!mine) return;
+    const u32 a = __hip_atomic_fetch_max(sh.mx + g * sh.stride, ASYM ? enc_ord(m) : f2u(m), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    u32 b = 0;
+    if (ASYM) b = __hip_atomic_fetch_min(sh.mn + g * sh.stride, enc_ord(n), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    asm volatile("" :: "v"(a), "v"(b) : "memory");   // (the old values have come back)
+  });
+  __syncthreads();
+  if (tid == 0) {
+    u32 *const arrived = sh.arrived + sh.spacing * blk, *const all = arrived + sh.spacing / 2;
+    u32 here = __hip_atomic_fetch_add(arrived, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1;
+    if (here == (u32)sh.n) __hip_atomic_store(all, here, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const long long t0 = wall_clock64();
+    while (here < (u32)sh.n && wall_clock64() - t0 < sh.ticks) {
+      __builtin_amdgcn_s_sleep(8);
+      here = __hip_atomic_load(all, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    all_here = here;
+  }
+  __syncthreads();
+  const bool met = all_here >= (u32)sh.n;
+  // The others may be waiting for a place on the chip, for as long as other launches please: after `ticks` all rows of the groups are read
+  // here, and no workgroup depends on another one's progress.
+  if (!met) {
+    if (live)
+      for (int j = f; j < pl.RR; j += sub) extend(*octet_at(row_of(j)));
+    fold();
+  }
+  per_group([&](int t, bool mine, int64_t g, float m, float n) __attribute__((always_inline)) {
+    if (met && mine) {
+      const u32 a = __hip_atomic_load(sh.mx + g * sh.stride, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      m = ASYM ? dec_ord(a) : u2f(a);
+      if (ASYM) n = dec_ord(__hip_atomic_load(sh.mn + g * sh.stride, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+    }
+    float s, zp = 0.f;
+    if (ASYM) {
+      s = fmaxf((m - n) / (float)((1 << p.bits) - 1), p.eps);
+      zp = (float)p.qmin - rintf(n / s);
+      par_z[t] = zp;
+    } else {
+      s = fmaxf(m / (float)p.qmax, p.eps);
+    }
+    par_s[t] = s;
+    // (as in quant_one_block)
+    par_r[t] = (s > 0x1p-96f && s < 0x1p96f && (f2u(s) & 0x7fffffu) != 0x7fffffu && fabsf(zp) <= 0x1p21f) ? 1.0f / s : 0.f;
+    if (mine && shard == 0) {
+      p.scale[g] = s;
+      if (ASYM) p.zp[g] = zp;
+    }
+  });
+  __syncthreads();
+  if (!live) return;   // (2-bit words take two adjacent columns, which are live together: c is a multiple of 16 there)
+  const int t0 = lq * gcols + col * (KEEPC ? 8 : 0);
+  float s[NV], r[NV], z[NV] = {};
+  bool plain = true;
+#pragma unroll
+  for (int j = 0; j < NV; ++j) {
+    s[j] = par_s[t0 + j];
+    r[j] = par_r[t0 + j];
+    if (ASYM) z[j] = par_z[t0 + j];
+    plain = plain && r[j] != 0.f;
+  }
+  if (__any(!plain)) {   // (rare, and once in the code: the rows are read again)
+    for (int i = 0; has(i); ++i) {
+      const u32 row = row_of(row_at(i));
+      float v[8];
+      octet_at(row)->widen(v);
+      store_octet<NV>(p, row, col, v, s, z, [](const int (&)[8]) {});
+    }
+    return;
+  }
+  const FastOctet<NV, ASYM> o(p, s, r, z);
+  auto finish = [&](int step, const Raw8<DT> &octet) __attribute__((always_inline)) {
+    float v[8];
+    octet.widen(v);
+    o.store(p, out_row32(p, row_of(row_at(step))), col, v, [](const float (&)[8]) {});
+  };
+#pragma unroll
+  for (int i = 0; i < NI; ++i) {
+    if (!has(i)) continue;
+    finish(i, raw[i]);
+    __builtin_amdgcn_sched_barrier(0);   // (rows started ahead of their turn cost registers that the held ones need)
+  }
+  // (those read last are the likeliest to be in a cache still)
+  for (int i = NI + (pl.steps - 1 - NI) / kAhead * kAhead; i >= NI; i -= kAhead) {
+    Raw8<DT> more[kAhead];
+#pragma unroll
+    for (int u = 0; u < kAhead; ++u) if (has(i + u)) more[u] = *octet_at(row_of(row_at(i + u)));
+#pragma unroll
+    for (int u = 0; u < kAhead; ++u) if (has(i + u)) finish(i + u, more[u]);
+  }
+}
+
 // A step of a quantizer with a scale per (head, channel), and the whole cache dequantized behind it, in one launch:
 // the first workgroups quantize the step and write its dequantized values from the codes in their registers, the
 // others dequantize the earlier tokens.  The values are those of the two launches.  Bound by launches and by
@@ -840,8 +1050,11 @@ bool make_plan(const int64_t *sh, int reduce_mask, int64_t n_groups, Plan &pl) {
   return true;
 }
 
-// Whether the one-launch kernel takes less time than the three launches, with their 2048 workgroups on either side of the fold.
-// Those take 12.4 us and 0.44 per MiB (of padded rows), for two tensors 16.2 and 0.41.  A workgroup of 1024 threads of the one-launch
+// Whether the one-launch kernel takes less time than the other way: workgroups that share their groups where `shared`, or the three launches, with their
+// 2048 workgroups on either side of the fold.  Workgroups that share take 11 us and 0.37 per MiB (0.25 in fp32) as launches from the host, two less in a graph, where one launch is
+// a tenth below what is said here: that / one, in a graph, us, [2,16,n,128] 8 bits, two tensors, 16 MiB 14.1 / 10.7, 25 17.7 / 15.2, 36 21.0 / 21.2, 64 31.9 / 36.3; [64,n,16,64] 9 12.6 / 10.7, 16
+// 14.9 / 15.4; one tensor 4.5 10.9 / 9.0, 8 12.3 / 12.6; [B,30,680,64] fp32 20 13.0 / 11.9, 30 15.0 / 16.2, 40 17.8 / 21.7, affine 20 14.3 / 12.6, 40 18.8 / 20.2.
+// The three take 12.4 us and 0.44 per MiB (of padded rows), for two tensors 16.2 and 0.41.  A workgroup of 1024 threads of the one-launch
 // kernel, which has a compute unit to itself, takes 4.5 us and 0.22 per KiB in pieces of 16 bytes, 0.175 while there are no more than 128 of them, 0.135
 // in pieces of 32 (0.17 where the rows lie multiples of 1 KiB apart), 0.10 in longer ones.  Three / one, us, 8 bits, a scale per (head, channel), two tensors:
 // [2,16,n,128] 16 MiB 23.3 / 12.5, 25 25.0 / 18.9, 36 29.5 / 24.5, 64 44.2 / 39.4; [32,n,30,64] 23 24.7 / 18.6, 40 32.2 / 27.2, 60 42.1 / 38.2;
@@ -854,7 +1067,7 @@ bool make_plan(const int64_t *sh, int reduce_mask, int64_t n_groups, Plan &pl) {
 // 22.5 / 17.8, 64 36.8 / 40.5; [8,16,L,128] fp32 96 MiB 45.5 / 32.4, affine 43.3 / 40.7; one scale per token, [32,30,L,64] bf16 96 62.0 / 51.6, affine 48 34.2 / 28.7.  With the step dequantized in the same launch the other way has one
 // more, whose work the one launch does beside: three and that / one, per tensor to fp32, [64,100,16,64] 40 / 74, [32,169,16,64] 41 / 64, [32,256,16,64]
 // 51 / 71, [32,12,256,64] 46 / 62, [64,100,8,64] 26 / 30, [32,169,30,64] 58 / 48, [16,256,8,128] 43 / 38, [32,100,16,64] 25 / 19.
-bool one_launch_pays(const OnePlan &pl, int c8, int c8p, int threads, bool keepc, double mib, int elem, int tensors, bool asym, bool with_values) {
+bool one_launch_pays(const OnePlan &pl, int c8, int c8p, int threads, bool keepc, double mib, int elem, int tensors, bool asym, bool with_values, bool shared) {
   if (!keepc) return mib <= (asym ? 16 : 48);
   if (threads == 256) return mib <= 16;
   const int64_t wgs = (int64_t)pl.blocks * pl.slices * tensors, cus = device_cus();
@@ -862,12 +1075,14 @@ bool one_launch_pays(const OnePlan &pl, int c8, int c8p, int threads, bool keepc
   const bool apart = pl.RI == 1 && pl.ro_rs * c8 * 8 * elem % 1024 == 0;
   const double per_kib = piece <= 16 ? (wgs <= 128 ? 0.175 : 0.22) : piece == 32 ? (apart ? 0.17 : 0.135) : 0.10;
   const double one = 4.5 + per_kib * (asym ? 1.1 : 1.0) * mib * 1024.0 / (double)wgs * (double)((wgs + cus - 1) / cus);
-  const double three = (tensors == 2 ? 16.2 + 0.41 * mib * c8p / c8 : 12.4 + 0.44 * mib * c8p / c8) + (asym ? 3.0 : 0.0) + (with_values ? 10.5 : 0.0);
+  const double pad = (double)c8p / c8;
+  if (shared) return 0.9 * one < 11.0 + (elem == 4 ? 0.25 : 0.37) * mib * pad + (asym ? 1.0 : 0.0) + (with_values ? 10.5 : 0.0);
+  const double three = (tensors == 2 ? 16.2 + 0.41 * mib * pad : 12.4 + 0.44 * mib * pad) + (asym ? 3.0 : 0.0) + (with_values ? 10.5 : 0.0);
   return one < three;
 }
 
 // The one-launch plan, or false when a group has too many rows for a workgroup's registers.
-bool make_one_plan(const int64_t *sh, int reduce_mask, int elem, int tensors, int bits, bool asym, bool with_values, OnePlan &pl, int &threads) {
+bool make_one_plan(const int64_t *sh, int reduce_mask, int elem, int tensors, int bits, bool asym, bool with_values, bool shared, OnePlan &pl, int &threads) {
   const int64_t c = sh[3], rows = sh[0] * sh[1] * sh[2];
   const int row_steps = elem == 4 ? 8 : 16;
   if (c % 8 != 0 || c > 512 || rows <= 0 || rows >= (1ll << 31) - 512) return false;
@@ -911,9 +1126,57 @@ bool make_one_plan(const int64_t *sh, int reduce_mask, int elem, int tensors, in
     pl.blocks = pl.nko * pl.tilesQ;
     const bool fits = pl.steps <= row_steps;
     const int enough = with_values ? 128 : threads == 1024 ? 129 : 160;
-    if (fits && ((int64_t)pl.blocks * pl.slices * tensors >= enough || !keepc || pl.c8s_shift <= narrowest)) return one_launch_pays(pl, c8, 1 << c8p_shift, threads, keepc, mib, elem, tensors, asym, with_values);
+    if (fits && ((int64_t)pl.blocks * pl.slices * tensors >= enough || !keepc || pl.c8s_shift <= narrowest)) return one_launch_pays(pl, c8, 1 << c8p_shift, threads, keepc, mib, elem, tensors, asym, with_values, shared);
     if (!keepc || pl.c8s_shift <= narrowest) return false;
   }
+}
+
+// The plan of workgroups that share their groups, in `words` of workspace per tensor, or false where it does not pay whatever one launch
+// takes.  Tokens first, tensors of 16 bits lose beyond 192 MiB, where the second read comes from memory and 256 bytes of a row in eight
+// sets of workgroups are the worse way through it: [64,n,16,64] fp16 125 MiB 71.8 -> 63.5 us, 187 105 -> 99, 250 135 -> 144, 500 266 -> 301; fp32
+// 250 119 -> 107, 375 195 -> 174.  Groups of whole rows gain from 48 MiB: 8 bits affine, a scale per head of [B,30,680,64] bf16, 20 MiB
+// 18.1 -> 21.9, 30 22.6 -> 19.4, 40 27.4 -> 31.3, 50 33.1 -> 27.6, 80 48.9 -> 38.0, per token 50 34.2 -> 25.7.
+bool make_shared_plan(const int64_t *sh, int reduce_mask, int64_t n_groups, int elem, int tensors, size_t words, OnePlan &pl, Shards &s) {
+  const int64_t c = sh[3], rows = sh[0] * sh[1] * sh[2];
+  if (c % 8 != 0 || c > 512 || rows <= 0 || rows >= (1ll << 31) - 512) return false;
+  const Canonical k = canonical(sh, reduce_mask);
+  const int64_t rr = k.nro * k.RI;
+  const int64_t bytes = rows * c * elem * tensors;
+  const bool keepc = !(reduce_mask & 8);
+  if (rows * c * elem > (1ll << 31)) return false;   // (rows and byte offsets of the kernel are of 32 bits)
+  if (!keepc && bytes < (48ll << 20)) return false;
+  if (k.RI == 1 && elem == 2 && bytes > (192ll << 20)) return false;
+  const int c8 = (int)(c / 8);
+  int c8p_shift = 0;
+  while ((1 << c8p_shift) < c8) ++c8p_shift;
+  pl.ko_rs = k.ko_rs; pl.ro_rs = k.ro_rs; pl.ko_gs = k.ko_gs; pl.q_gs = k.q_gs;
+  pl.nko = (int)k.nko; pl.Q = (int)k.Q; pl.RR = (int)rr; pl.RI = (int)k.RI; pl.by_RI = FastDiv::by(k.RI);
+  pl.c8s_shift = c8p_shift; pl.slices = 1;
+  // pieces of 256 bytes
+  pl.lq_shift = 0;
+  while (k.RI == 1 && (2 << pl.lq_shift) <= k.Q && ((8 * elem) << (c8p_shift + pl.lq_shift)) < 256) ++pl.lq_shift;
+  if (8 - c8p_shift - pl.lq_shift < 0) return false;
+  pl.sub_shift = 8 - c8p_shift - pl.lq_shift;
+  pl.tilesQ = (int)((k.Q + (1 << pl.lq_shift) - 1) >> pl.lq_shift);
+  if (k.nko * pl.tilesQ > 512) return false;
+  pl.blocks = pl.nko * pl.tilesQ;
+  // as many workgroups as the chip holds at once, of at least four steps (groups of whole rows: eight), and no more than meet quickly; of
+  // less than two per compute unit the three launches read faster
+  const int64_t least = (keepc ? 4ll : 8ll) << pl.sub_shift;
+  int64_t n = std::min<int64_t>({(int64_t)device_cus() * 4 / ((int64_t)pl.blocks * tensors), (rr + least - 1) / least, 256});
+  if (n < 2 || n * pl.blocks * tensors < 2 * device_cus()) return false;
+  pl.steps = (int)((rr + (n << pl.sub_shift) - 1) / (n << pl.sub_shift));
+  n = (rr + ((int64_t)pl.steps << pl.sub_shift) - 1) / ((int64_t)pl.steps << pl.sub_shift);
+  const int n_par = (keepc ? 8 << c8p_shift : 1) << pl.lq_shift, fold_vals = n_par * std::max(1, (1 << (pl.sub_shift + c8p_shift)) / 64);
+  if (n < 2 || std::max(n_par, fold_vals) > kSharedGroups) return false;
+  // (lines of their own for the extremes of each group of whole rows and for the words of a block, where there is room: atomics on
+  // one line wait for one another)
+  s.n = (int)n;
+  s.stride = !keepc && 64 * (size_t)(n_groups + pl.blocks) <= words ? 32 : 1;
+  const size_t left = words - std::min(words, 2 * s.stride * (size_t)n_groups);
+  for (s.spacing = 64; s.spacing >= 8 && (size_t)s.spacing * pl.blocks > left;) s.spacing /= 2;
+  s.ticks = (u32)(10000 + (bytes >> 20) * 100);   // 0.1 ms, and 1 us for each MiB, several times what it takes
+  return s.spacing >= 8;
 }
 
 template <int DT, bool ASYM, bool KEEPC>
@@ -947,6 +1210,18 @@ template <int DT> void run_one_step(const GenParams &p, const OnePlan &pl, int t
   if (o.odt == VARQ_F32) typed(std::integral_constant<int, VARQ_F32>{});
   else if (o.odt == VARQ_BF16) typed(std::integral_constant<int, VARQ_BF16>{});
   else typed(std::integral_constant<int, VARQ_F16>{});
+}
+
+template <int DT, bool ASYM, bool KEEPC>
+void launch_shared(const GenParams &p, const OnePlan &pl, const Shards &sh, hipStream_t st) {
+  const unsigned nt = p.x1 ? 2u : 1u;
+  const int64_t n = std::max(p.n_groups, (int64_t)pl.blocks);
+  hipLaunchKernelGGL(clear_shards_kernel, dim3((unsigned)((n + 255) / 256), nt), dim3(256), 0, st, p, sh, p.n_groups, pl.blocks);
+  hipLaunchKernelGGL((quant_shared_kernel<DT, ASYM, KEEPC>), dim3((unsigned)(pl.blocks * sh.n), nt), dim3(256), 0, st, p, pl, sh);
+}
+template <int DT> void run_shared(const GenParams &p, const OnePlan &pl, const Shards &sh, hipStream_t st) {
+  if (p.asym) { if (p.keepc) launch_shared<DT, true, true>(p, pl, sh, st); else launch_shared<DT, true, false>(p, pl, sh, st); }
+  else { if (p.keepc) launch_shared<DT, false, true>(p, pl, sh, st); else launch_shared<DT, false, false>(p, pl, sh, st); }
 }
 
 size_t plan_workspace_bytes(const Plan &pl, int64_t n_groups) {
@@ -1051,7 +1326,7 @@ int quant_pack_impl(const void *x, const void *x1, int x_dtype, const int64_t *h
                     int asym, float eps, int32_t *words, int8_t *codes, float *scale, float *zp,
                     int32_t *words1, int8_t *codes1, float *scale1, float *zp1,
                     const int64_t *host_out_map, void *workspace, size_t workspace_bytes, void *stream,
-                    StepOut *step = nullptr, int64_t step_pairs = 0, const int64_t *host_scale_map = nullptr, float *const *once = nullptr) {
+                    StepOut *step = nullptr, int64_t step_pairs = 0, const int64_t *host_scale_map = nullptr, float *const *once = nullptr, const u32 *host_wait_ticks = nullptr) {
   VARQ_CHECK_ARG(host_shape4, "quant_pack: null shape");
   const int64_t *s = host_shape4;
   VARQ_CHECK_ARG(s[0] >= 0 && s[1] >= 0 && s[2] >= 0 && s[3] > 0 && s[3] <= (1 << 20), "quant_pack: bad shape");
@@ -1123,7 +1398,12 @@ int quant_pack_impl(const void *x, const void *x1, int x_dtype, const int64_t *h
   hipStream_t st = (hipStream_t)stream;
   OnePlan one;
   int threads;
-  if (tiled && make_one_plan(s, reduce_mask, x_dtype == VARQ_F32 ? 4 : 2, x1 ? 2 : 1, words ? bits : 8, asym != 0, step != nullptr, one, threads)) {
+  const int elem = x_dtype == VARQ_F32 ? 4 : 2, tensors = x1 ? 2 : 1;
+  const size_t words_each = tiled ? plan_workspace_bytes(pl, ng) / sizeof(u32) : 0;
+  OnePlan by_many;
+  Shards sh = {};
+  const bool shared = tiled && !host_scale_map && make_shared_plan(s, reduce_mask, ng, elem, tensors, words_each, by_many, sh);
+  if (tiled && make_one_plan(s, reduce_mask, elem, tensors, words ? bits : 8, asym != 0, step != nullptr, shared, one, threads)) {
     if (step) {
       step->q_blocks = (one.blocks + 7) / 8 * 8 * one.slices;
       step->pair_blocks = (int)((step->earlier.pair_octs + kStepOctets - 1) / kStepOctets);
@@ -1142,6 +1422,14 @@ int quant_pack_impl(const void *x, const void *x1, int x_dtype, const int64_t *h
     if (x_dtype == VARQ_F32) run_one<VARQ_F32>(p, one, threads, st);
     else if (x_dtype == VARQ_BF16) run_one<VARQ_BF16>(p, one, threads, st);
     else run_one<VARQ_F16>(p, one, threads, st);
+  } else if (shared) {
+    if (x1) { p.x1 = x1; p.scale1 = scale1; p.zp1 = zp1; p.words1 = words1; p.codes1 = codes1; }
+    p.ws1 = (int64_t)words_each;
+    sh.mx = p.ws; sh.mn = p.ws + ng * sh.stride; sh.arrived = p.ws + 2 * ng * sh.stride;
+    if (host_wait_ticks) sh.ticks = *host_wait_ticks;
+    if (x_dtype == VARQ_F32) run_shared<VARQ_F32>(p, by_many, sh, st);
+    else if (x_dtype == VARQ_BF16) run_shared<VARQ_BF16>(p, by_many, sh, st);
+    else run_shared<VARQ_F16>(p, by_many, sh, st);
   } else if (host_scale_map) {
     return varq_set_error(VARQ_ERR_UNSUPPORTED, "quant_pack: spread scales come with groups that one launch quantizes");
   } else if (tiled) {
@@ -1180,6 +1468,13 @@ extern "C" int varq_quant_pack2(const void *x0, const void *x1, int x_dtype, con
   VARQ_CHECK_ARG(x1, "quant_pack2: null second tensor");
   return quant_pack_impl(x0, x1, x_dtype, host_shape4, reduce_mask, bits, asym, eps, words0, codes0, scale0, zp0,
                          words1, codes1, scale1, zp1, host_out_map, workspace, workspace_bytes, stream);
+}
+
+extern "C" int varq_quant_pack_wait(const void *x, int x_dtype, const int64_t *host_shape4, int reduce_mask, int bits, int asym, float eps, int32_t *words,
+                                    int8_t *codes, float *scale, float *zp, const int64_t *host_out_map, uint32_t wait_ticks, void *workspace,
+                                    size_t workspace_bytes, void *stream) {
+  return quant_pack_impl(x, nullptr, x_dtype, host_shape4, reduce_mask, bits, asym, eps, words, codes, scale, zp, nullptr, nullptr, nullptr, nullptr,
+                         host_out_map, workspace, workspace_bytes, stream, nullptr, 0, nullptr, nullptr, &wait_ticks);
 }
 
 extern "C" int varq_quant_pack_spread_once(const void *x0, const void *x1, int x_dtype, const int64_t *host_shape4, int reduce_mask, int bits, int asym,
