@@ -1,11 +1,14 @@
 """Workgroups that share their groups (`quant_shared_kernel`): rows that do not fill the last workgroup or step, more rows than the
 registers hold, octets that are no power of two, kept inner indices that do not fill the last tile, groups of whole rows; with the
 others' extremes waited for and, without waiting, with all rows read by whoever comes first.  Bit-exact against the CPU oracle."""
+import math
+
 import pytest
 import torch
 
 import varq_oracle as O
 from gpu_util import note
+from test_gpu_nonfinite import WHAT, _bits, _spoil
 from var_q_amd import _lib, ops
 
 pytestmark = pytest.mark.gpu
@@ -72,3 +75,24 @@ def test_shared_groups_in_a_graph(dev):
         for (q, s, z), x in zip(got, xs):
             rq, rs, rz = O.quant_reduce(x.cpu(), dims, 8, True)
             assert torch.equal(s.cpu(), rs) and torch.equal(z.cpu(), rz) and torch.equal(q.cpu(), O.pack_last_dim(rq, 8)[0])
+
+
+@pytest.mark.parametrize('what', WHAT)
+@pytest.mark.parametrize('shape,dims,dtype', [
+    ((2, 4, 300, 64), (0, 2), torch.bfloat16),
+    ((4, 70, 8, 64), (0, 1), torch.float16),
+    ((2, 4, 300, 64), (0, 2), torch.float32),
+    ((2, 5, 33, 32), (0, 3), torch.bfloat16),
+])
+def test_infinities_and_nan(dev, shape, dims, dtype, what):
+    """The batch behind itself leaves every group what it is and takes workgroups that share it; alone it takes one launch."""
+    x = _spoil(torch.randn(*shape, generator=torch.Generator().manual_seed(7)).to(dtype).to(dev), 1 if dims == (0, 1) else 2, what)
+    rows = math.prod(shape[d] for d in dims if d != 3)
+    times = max(24000 // rows + 1, (48 << 20) // (x.numel() * x.element_size()) + 1 if 3 in dims else 0)
+    for bits, asym in ((8, False), (8, True), (4, True), (2, True)):
+        note('quant shared, non-finite', shape, dims, dtype, what, bits, asym)
+        q1, s1, z1 = ops.quant_pack(x, dims, bits, asym=asym)
+        many = x.repeat(times, 1, 1, 1)
+        for q, s, z in (ops.quant_pack(many, dims, bits, asym=asym), _without_waiting(many, dims, bits, asym, True)):
+            assert torch.equal(_bits(s1), _bits(s)) and (not asym or torch.equal(_bits(z1), _bits(z)))
+            assert torch.equal(q.view(times, *q1.shape), q1.expand(times, *q1.shape))
