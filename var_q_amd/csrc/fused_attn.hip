@@ -1188,6 +1188,14 @@ __global__ __launch_bounds__(NW * 64, 2) void exact_attn_kernel(AttnParams p) {
   attend_codes<BITS>(p, k.pair, k.pair, k.qt, k.split);
 }
 
+// Where four channels of a packed row go.  (Rows fit 32 bits: so many, times the shares of a partial result, are more than any memory.  Divided in
+// 64 bits they were half of the combining kernels' instructions.)
+template <int D> __device__ __forceinline__ __bf16 *out_of_row(const AttnParams &p, u32 row, int c0) {
+  const u32 bh = row / (u32)p.Lq, qrow = row - bh * (u32)p.Lq, b = bh / (u32)p.Hkv, hs = bh - b * (u32)p.Hkv;
+  const int hq = p.head_map ? p.head_map[hs] : (int)hs;
+  return p.out + ((int64_t)b * p.o_bs + hq * p.o_hs + (int64_t)qrow * p.o_ts) * D + c0;
+}
+
 // The shares' outputs weighted by their softmax mass l * 2^(m - M), M the largest reference among
 // the shares that saw a key.  (A share that saw none has the mass 0; one whose logits held a NaN has NaN for its mass, which
 // is not to be taken for 0, or the result would be finite where the unshared kernel's is NaN.)  A workgroup of 256 threads serves 2 query rows x (D/4) channel quads
@@ -1246,58 +1254,64 @@ __global__ __launch_bounds__(256) void combine_splits_kernel(AttnParams p) {
   }
   if (row >= rows) return;
   const float inv = wsum > 0.f ? 1.0f / wsum : 0.f;
-  const int bh = (int)(row / p.Lq), qrow = (int)(row % p.Lq);
-  const int b = bh / p.Hkv, hs = bh % p.Hkv;
-  const int hq = p.head_map ? p.head_map[hs] : hs;
-  __bf16 *optr = p.out + (b * p.o_bs + hq * p.o_hs + qrow * p.o_ts) * D + c0;
-  *reinterpret_cast<uint2 *>(optr) = make_uint2(pack_io_rne<F16>(acc[0] * inv, acc[1] * inv), pack_io_rne<F16>(acc[2] * inv, acc[3] * inv));
+  *reinterpret_cast<uint2 *>(out_of_row<D>(p, (u32)row, c0)) = make_uint2(pack_io_rne<F16>(acc[0] * inv, acc[1] * inv), pack_io_rne<F16>(acc[2] * inv, acc[3] * inv));
 }
 
 // The same for a handful of shares and many rows: a thread sums four channels of one row over all
 // shares, nothing passes through LDS.  (With the kernel above, two rows and three barriers to a
 // workgroup, two shares of 32 768 rows took 18.9 us for the 50 MB they are.)
-template <int D, bool F16>
+// NS: the shares, or the most of them; U: rows of a thread (two shares, D=128, 1024 queries of 32 pairs, the call with its producer and
+// attention: one row 77.5 us, two 76.7, four 77.7; 77.9 with rows divided in 64 bits).
+template <int D, bool F16, int NS, int U>
 __global__ __launch_bounds__(256) void combine_few_splits_kernel(AttnParams p) {
   const int64_t rows = (int64_t)p.bh_total * p.Lq;
-  const int64_t row = (int64_t)blockIdx.x * (1024 / D) + threadIdx.x / (D / 4);
-  const int c0 = threadIdx.x % (D / 4) * 4;
-  if (row >= rows) return;
-  float2 ml[kMaxSplits_v];
-  float4 o[kMaxSplits_v];
+  const int64_t row0 = (int64_t)blockIdx.x * (U * 1024 / D) + threadIdx.x / (D / 4);
+  const int c0 = threadIdx.x % (D / 4) * 4, n = NS == 2 ? 2 : p.nsplit;
+  float2 ml[U][NS];
+  float4 o[U][NS];
 #pragma unroll
-  for (int s = 0; s < kMaxSplits_v; ++s) {
-    ml[s] = make_float2(0.f, 0.f);
-    if (s < p.nsplit) {
-      ml[s] = *reinterpret_cast<const float2 *>(p.ws_ml + ((int64_t)s * rows + row) * 2);
-      o[s] = *reinterpret_cast<const float4 *>(p.ws_o + ((int64_t)s * rows + row) * D + c0);
+  for (int u = 0; u < U; ++u) {
+    const int64_t row = row0 + u * (1024 / D);
+#pragma unroll
+    for (int s = 0; s < NS; ++s) {
+      ml[u][s] = make_float2(0.f, 0.f);
+      if (s < n && row < rows) {
+        ml[u][s] = *reinterpret_cast<const float2 *>(p.ws_ml + ((int64_t)s * rows + row) * 2);
+        o[u][s] = *reinterpret_cast<const float4 *>(p.ws_o + ((int64_t)s * rows + row) * D + c0);
+      }
     }
   }
-  float M = -INFINITY;
 #pragma unroll
-  for (int s = 0; s < kMaxSplits_v; ++s)
-    if (ml[s].y != 0.f) M = fmaxf(M, ml[s].x);
-  float acc[4] = {0.f, 0.f, 0.f, 0.f}, wsum = 0.f;
+  for (int u = 0; u < U; ++u) {
+    const int64_t row = row0 + u * (1024 / D);
+    if (row >= rows) return;
+    float M = -INFINITY;
 #pragma unroll
-  for (int s = 0; s < kMaxSplits_v; ++s)
-    if (s < p.nsplit && ml[s].y != 0.f) {
-      const float w = ml[s].y * __builtin_amdgcn_exp2f(ml[s].x - M);
-      acc[0] = __builtin_fmaf(w, o[s].x, acc[0]); acc[1] = __builtin_fmaf(w, o[s].y, acc[1]);
-      acc[2] = __builtin_fmaf(w, o[s].z, acc[2]); acc[3] = __builtin_fmaf(w, o[s].w, acc[3]);
-      wsum += w;
-    }
-  const float inv = wsum > 0.f ? 1.0f / wsum : 0.f;
-  const int bh = (int)(row / p.Lq), qrow = (int)(row - (int64_t)bh * p.Lq);
-  const int b = bh / p.Hkv, hs = bh - b * p.Hkv;
-  const int hq = p.head_map ? p.head_map[hs] : hs;
-  *reinterpret_cast<uint2 *>(p.out + (b * p.o_bs + hq * p.o_hs + qrow * p.o_ts) * D + c0) =
-      make_uint2(pack_io_rne<F16>(acc[0] * inv, acc[1] * inv), pack_io_rne<F16>(acc[2] * inv, acc[3] * inv));
+    for (int s = 0; s < NS; ++s)
+      if (ml[u][s].y != 0.f) M = fmaxf(M, ml[u][s].x);
+    float acc[4] = {0.f, 0.f, 0.f, 0.f}, wsum = 0.f;
+#pragma unroll
+    for (int s = 0; s < NS; ++s)
+      if (s < n && ml[u][s].y != 0.f) {
+        const float w = ml[u][s].y * __builtin_amdgcn_exp2f(ml[u][s].x - M);
+        acc[0] = __builtin_fmaf(w, o[u][s].x, acc[0]); acc[1] = __builtin_fmaf(w, o[u][s].y, acc[1]);
+        acc[2] = __builtin_fmaf(w, o[u][s].z, acc[2]); acc[3] = __builtin_fmaf(w, o[u][s].w, acc[3]);
+        wsum += w;
+      }
+    const float inv = wsum > 0.f ? 1.0f / wsum : 0.f;
+    *reinterpret_cast<uint2 *>(out_of_row<D>(p, (u32)row, c0)) =
+        make_uint2(pack_io_rne<F16>(acc[0] * inv, acc[1] * inv), pack_io_rne<F16>(acc[2] * inv, acc[3] * inv));
+  }
 }
 
 template <int D, bool F16> void launch_combine(const AttnParams &p, hipStream_t st) {
   const int64_t rows = (int64_t)p.bh_total * p.Lq;
   // (few rows: the threads of a row sharing its shares out are what fills the device)
-  if (p.nsplit <= kMaxSplits_v && rows >= 4096)
-    hipLaunchKernelGGL((combine_few_splits_kernel<D, F16>), dim3((unsigned)((rows + 1024 / D - 1) / (1024 / D))), dim3(256), 0, st, p);
+  constexpr int R = 1024 / D;
+  if (p.nsplit == 2 && rows >= 4096)
+    hipLaunchKernelGGL((combine_few_splits_kernel<D, F16, 2, 2>), dim3((unsigned)((rows + 2 * R - 1) / (2 * R))), dim3(256), 0, st, p);
+  else if (p.nsplit <= kMaxSplits_v && rows >= 4096)
+    hipLaunchKernelGGL((combine_few_splits_kernel<D, F16, kMaxSplits_v, 1>), dim3((unsigned)((rows + R - 1) / R)), dim3(256), 0, st, p);
   else
     hipLaunchKernelGGL((combine_splits_kernel<D, F16>), dim3((unsigned)((rows + 1) / 2)), dim3(256), 0, st, p);
 }
