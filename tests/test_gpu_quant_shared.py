@@ -32,10 +32,10 @@ def _without_waiting(x, dims, bits, asym, pack):
 
 @pytest.mark.parametrize('shape,dims,dtype', [
     ((2, 4, 16500, 64), (0, 2), torch.bfloat16),      # 1024 workgroups of five steps
-    ((64, 513, 3, 64), (0, 1), torch.float16),        # two kept indices to a block, the last block half full
+    ((64, 513, 7, 64), (0, 1), torch.float16),        # two kept indices to a block, the last block half full
     ((3, 11003, 5, 72), (0, 1), torch.float32),       # nine octets of sixteen lanes
-    ((1, 2, 70001, 96), (0, 2), torch.bfloat16),      # 18 steps: two beyond the held ones
-    ((2, 2, 35001, 128), (0, 2), torch.float32),      # 18 steps of which 8 are held
+    ((1, 4, 70001, 96), (0, 2), torch.bfloat16),      # 18 steps: two beyond the held ones
+    ((2, 3, 35001, 128), (0, 2), torch.float32),      # 18 steps of which 8 are held
     ((1, 4, 8300, 256), (0, 2), torch.float16),       # as many groups as a workgroup takes
     ((2, 30, 7000, 64), (0, 2, 3), torch.bfloat16),   # groups of whole rows
     ((32, 30, 421, 64), (0, 1, 3), torch.bfloat16),
@@ -88,7 +88,7 @@ def test_infinities_and_nan(dev, shape, dims, dtype, what):
     """The batch behind itself leaves every group what it is and takes workgroups that share it; alone it takes one launch."""
     x = _spoil(torch.randn(*shape, generator=torch.Generator().manual_seed(7)).to(dtype).to(dev), 1 if dims == (0, 1) else 2, what)
     rows = math.prod(shape[d] for d in dims if d != 3)
-    times = max(24000 // rows + 1, (48 << 20) // (x.numel() * x.element_size()) + 1 if 3 in dims else 0)
+    times = max(26000 // rows + 1, (48 << 20) // (x.numel() * x.element_size()) + 1 if 3 in dims else 0)
     for bits, asym in ((8, False), (8, True), (4, True), (2, True)):
         note('quant shared, non-finite', shape, dims, dtype, what, bits, asym)
         q1, s1, z1 = ops.quant_pack(x, dims, bits, asym=asym)

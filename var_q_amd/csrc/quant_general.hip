@@ -1161,10 +1161,11 @@ bool make_shared_plan(const int64_t *sh, int reduce_mask, int64_t n_groups, int 
   if (k.nko * pl.tilesQ > 512) return false;
   pl.blocks = pl.nko * pl.tilesQ;
   // as many workgroups as the chip holds at once, of at least four steps (groups of whole rows: eight), and no more than meet quickly; of
-  // less than two per compute unit the three launches read faster
+  // fewer than three per compute unit, or than nearly four where lanes idle, the three launches read faster (two heads: fp32 [1,2,381944,72], one scale per
+  // head, 103 -> 128 us, fp16 [2,2,381944,72] 139 -> 261; three: fp16 [2,3,23148,72] 22.3 -> 23.6, but fp32 [5,3,28645,128] 104 -> 87)
   const int64_t least = (keepc ? 4ll : 8ll) << pl.sub_shift;
   int64_t n = std::min<int64_t>({(int64_t)device_cus() * 4 / ((int64_t)pl.blocks * tensors), (rr + least - 1) / least, 256});
-  if (n < 2 || n * pl.blocks * tensors < 2 * device_cus()) return false;
+  if (n < 2 || n * pl.blocks * tensors * 4 < (int64_t)device_cus() * (c8 == 1 << c8p_shift ? 12 : 15)) return false;
   pl.steps = (int)((rr + (n << pl.sub_shift) - 1) / (n << pl.sub_shift));
   n = (rr + ((int64_t)pl.steps << pl.sub_shift) - 1) / ((int64_t)pl.steps << pl.sub_shift);
   const int n_par = (keepc ? 8 << c8p_shift : 1) << pl.lq_shift, fold_vals = n_par * std::max(1, (1 << (pl.sub_shift + c8p_shift)) / 64);
