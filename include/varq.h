@@ -168,7 +168,7 @@ int varq_quant_pack2(const void *x0, const void *x1, int x_dtype, const int64_t 
 
 /*
  * varq_quant_pack with the time given that a workgroup waits for the others with which it shares its groups, in ticks of 10 ns, before
- * it reads all of their rows by itself (0: without waiting).  Results do not depend on it.
+ * it helps to read their rows (0: without waiting).  Results do not depend on it.
  */
 int varq_quant_pack_wait(const void *x, int x_dtype, const int64_t *host_shape4, int reduce_mask, int bits, int asym, float eps, int32_t *words,
                          int8_t *codes, float *scale, float *zp, const int64_t *host_out_map, uint32_t wait_ticks, void *workspace,

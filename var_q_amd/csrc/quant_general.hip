@@ -680,16 +680,18 @@ __global__ __launch_bounds__(NT) void quant_one_kernel(GenParams p, OnePlan pl) 
 // waits for the others, in ticks of 10 ns.
 struct Shards {
   int n;
-  u32 *mx, *mn, *arrived;       // per group, `stride` words apart; per block, `spacing` words apart: how many have arrived, and half of that on, whether all
+  u32 *mx, *mn;                 // per group, `stride` words apart
+  u32 *words;                   // per block, `spacing` words apart, four of them a quarter of that from one another: see quant_shared_kernel
   int stride, spacing;
   u32 ticks;
 };
 constexpr int kSharedGroups = 1024;   // groups of a workgroup, and values of its fold
 __global__ __launch_bounds__(256) void clear_shards_kernel(GenParams p, Shards sh, int64_t n_groups, int blocks) {
-  if (take_second(p)) { sh.mx += p.ws1; sh.mn += p.ws1; sh.arrived += p.ws1; }
+  if (take_second(p)) { sh.mx += p.ws1; sh.mn += p.ws1; sh.words += p.ws1; }
   const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
   if (i < n_groups) { sh.mx[i * sh.stride] = 0u; sh.mn[i * sh.stride] = 0xffffffffu; }
-  if (i < blocks) { sh.arrived[sh.spacing * i] = 0u; sh.arrived[sh.spacing * i + sh.spacing / 2] = 0u; }
+  if (i < blocks)
+    for (int w = 0; w < 4; ++w) sh.words[sh.spacing * i + sh.spacing / 4 * w] = 0u;
 }
 template <int DT, bool ASYM, bool KEEPC>
 __global__ __launch_bounds__(256, 4) void quant_shared_kernel(GenParams p, OnePlan pl, Shards sh) {
@@ -698,8 +700,8 @@ __global__ __launch_bounds__(256, 4) void quant_shared_kernel(GenParams p, OnePl
   __shared__ float lds_mn[ASYM ? kSharedGroups : 1];
   __shared__ float par_s[kSharedGroups], par_r[kSharedGroups];
   __shared__ float par_z[ASYM ? kSharedGroups : 1];
-  __shared__ u32 all_here;
-  if (take_second(p)) { sh.mx += p.ws1; sh.mn += p.ws1; sh.arrived += p.ws1; }
+  __shared__ u32 lds_next;
+  if (take_second(p)) { sh.mx += p.ws1; sh.mn += p.ws1; sh.words += p.ws1; }
   const int blk = blockIdx.x / sh.n, shard = blockIdx.x - blk * sh.n, tq = blk % pl.tilesQ, ko = blk / pl.tilesQ;
   const int tid = threadIdx.x, c8s = 1 << pl.c8s_shift, sub = 1 << pl.sub_shift;
   const int col = tid & (c8s - 1), f = (tid >> pl.c8s_shift) & (sub - 1), lq = tid >> (pl.c8s_shift + pl.sub_shift);
@@ -764,7 +766,6 @@ __global__ __launch_bounds__(256, 4) void quant_shared_kernel(GenParams p, OnePl
     }
     __syncthreads();
   };
-  fold();
   // body(t, whether there is such a group, its number, its extremes in this workgroup), a thread per group
   const int n_par = gcols << pl.lq_shift;
   auto per_group = [&](auto &&body) __attribute__((always_inline)) {
@@ -783,36 +784,64 @@ __global__ __launch_bounds__(256, 4) void quant_shared_kernel(GenParams p, OnePl
   // there, the count goes up after that, and who has seen the count reads behind it.  (A release and an acquire instead write back and drop
   // whole L2s, once per workgroup: [64,256,16,64] fp16, two tensors, 33 -> 76 us.)  The last to arrive sets a word of its own,
   // half a `spacing` from the count, which the others look at: with all of them polling the counts, side by side, 56 us.
-  per_group([&](int, bool mine, int64_t g, float m, float n) __attribute__((always_inline)) {
-    if (!mine) return;
-    const u32 a = __hip_atomic_fetch_max(sh.mx + g * sh.stride, ASYM ? enc_ord(m) : f2u(m), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    u32 b = 0;
-    if (ASYM) b = __hip_atomic_fetch_min(sh.mn + g * sh.stride, enc_ord(n), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    asm volatile("" :: "v"(a), "v"(b) : "memory");   // (the old values have come back)
-  });
-  __syncthreads();
-  if (tid == 0) {
-    u32 *const arrived = sh.arrived + sh.spacing * blk, *const all = arrived + sh.spacing / 2;
-    u32 here = __hip_atomic_fetch_add(arrived, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1;
-    if (here == (u32)sh.n) __hip_atomic_store(all, here, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    const long long t0 = wall_clock64();
-    while (here < (u32)sh.n && wall_clock64() - t0 < sh.ticks) {
-      __builtin_amdgcn_s_sleep(8);
-      here = __hip_atomic_load(all, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
-    all_here = here;
-  }
-  __syncthreads();
-  const bool met = all_here >= (u32)sh.n;
-  // The others may be waiting for a place on the chip, for as long as other launches please: after `ticks` all rows of the groups are read
-  // here, and no workgroup depends on another one's progress.
-  if (!met) {
-    if (live)
-      for (int j = f; j < pl.RR; j += sub) extend(*octet_at(row_of(j)));
+  //
+  // The others may be waiting for a place on the chip, for as long as other launches please.  After `ticks` those that are here read the parts of the block's
+  // rows over again, each part once, by whoever asks for it next (an extreme may be raised twice): the extremes are complete when all have arrived or all parts are
+  // read, whichever is first.  And so that no workgroup depends on another one's progress, whoever finds no part left and has waited `ticks` for
+  // those who read the last ones reads all rows by itself.  (With all rows read by everyone who had waited, us, beside 1000 workgroups of
+  // another stream that keep their places for 2.2 ms, then / now / three launches: fp32 [2,3,35001,128] 2791 / 1310 / 1257, [60,3,35001,64] 2350 to 34000 /
+  // 2378 / 2154, bf16 [300,30,680,64] affine 4467 / 2168 / 1932; on a device of their own after 3 us of patience, [2,3,35001,128] 1577 / 67,
+  // [32,30,680,64] affine 291 / 62, a scale per head 267 / 55; waiting 55, 54, 50.)
+  u32 *const arrived = sh.words + sh.spacing * blk, *const asked = arrived + sh.spacing / 4, *const all = arrived + sh.spacing / 2, *const read = all + sh.spacing / 4;
+  constexpr u32 kOwn = ~0u, kEvery = ~0u - 1, kMet = ~0u - 2;   // what a round has read: the own part, all rows, or the part of that number; kMet: nothing is left to read
+  const u32 n_shards = (u32)sh.n;
+  for (u32 what = kOwn;;) {
     fold();
+    per_group([&](int, bool mine, int64_t g, float m, float n) __attribute__((always_inline)) {
+      if (!mine) return;
+      const u32 a = __hip_atomic_fetch_max(sh.mx + g * sh.stride, ASYM ? enc_ord(m) : f2u(m), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      u32 b = 0;
+      if (ASYM) b = __hip_atomic_fetch_min(sh.mn + g * sh.stride, enc_ord(n), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      asm volatile("" :: "v"(a), "v"(b) : "memory");   // (the old values have come back)
+    });
+    __syncthreads();
+    if (tid == 0) {
+      auto wait = [&](u32 here) {
+        const long long t0 = wall_clock64();
+        while (here < n_shards && wall_clock64() - t0 < sh.ticks) {
+          __builtin_amdgcn_s_sleep(8);
+          here = __hip_atomic_load(all, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+        return here;
+      };
+      u32 here = n_shards;
+      if (what != kEvery) here = __hip_atomic_fetch_add(what == kOwn ? arrived : read, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1;
+      if (here == n_shards) __hip_atomic_store(all, here, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      else if (what == kOwn) here = wait(here);
+      else here = __hip_atomic_load(all, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      u32 next = kMet;
+      if (here < n_shards) {
+        next = __hip_atomic_fetch_add(asked, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (next >= n_shards) next = wait(0u) < n_shards ? kEvery : kMet;
+      }
+      lds_next = next;
+    }
+    __syncthreads();
+    what = lds_next;
+    if (what == kMet) break;
+    if (live) {
+      const int first = what == kEvery ? f : (int)what * (pl.steps << pl.sub_shift) + f, last = what == kEvery ? pl.RR : min(pl.RR, (int)(what + 1) * (pl.steps << pl.sub_shift));
+      for (int j = first; j < last; j += kAhead << pl.sub_shift) {
+        Raw8<DT> more[kAhead];
+#pragma unroll
+        for (int u = 0; u < kAhead; ++u) if (j + (u << pl.sub_shift) < last) more[u] = *octet_at(row_of(j + (u << pl.sub_shift)));
+#pragma unroll
+        for (int u = 0; u < kAhead; ++u) if (j + (u << pl.sub_shift) < last) extend(more[u]);
+      }
+    }
   }
   per_group([&](int t, bool mine, int64_t g, float m, float n) __attribute__((always_inline)) {
-    if (met && mine) {
+    if (mine) {
       const u32 a = __hip_atomic_load(sh.mx + g * sh.stride, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       m = ASYM ? dec_ord(a) : u2f(a);
       if (ASYM) n = dec_ord(__hip_atomic_load(sh.mn + g * sh.stride, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
@@ -1426,7 +1455,7 @@ int quant_pack_impl(const void *x, const void *x1, int x_dtype, const int64_t *h
   } else if (shared) {
     if (x1) { p.x1 = x1; p.scale1 = scale1; p.zp1 = zp1; p.words1 = words1; p.codes1 = codes1; }
     p.ws1 = (int64_t)words_each;
-    sh.mx = p.ws; sh.mn = p.ws + ng * sh.stride; sh.arrived = p.ws + 2 * ng * sh.stride;
+    sh.mx = p.ws; sh.mn = p.ws + ng * sh.stride; sh.words = p.ws + 2 * ng * sh.stride;
     if (host_wait_ticks) sh.ticks = *host_wait_ticks;
     if (x_dtype == VARQ_F32) run_shared<VARQ_F32>(p, by_many, sh, st);
     else if (x_dtype == VARQ_BF16) run_shared<VARQ_BF16>(p, by_many, sh, st);
