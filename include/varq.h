@@ -167,14 +167,6 @@ int varq_quant_pack2(const void *x0, const void *x1, int x_dtype, const int64_t 
                      const int64_t *host_out_map, void *workspace, size_t workspace_bytes, void *stream);
 
 /*
- * varq_quant_pack with the time given that a workgroup waits for the others with which it shares its groups, in ticks of 10 ns, before
- * it helps to read their rows (0: without waiting).  Results do not depend on it.
- */
-int varq_quant_pack_wait(const void *x, int x_dtype, const int64_t *host_shape4, int reduce_mask, int bits, int asym, float eps, int32_t *words,
-                         int8_t *codes, float *scale, float *zp, const int64_t *host_out_map, uint32_t wait_ticks, void *workspace,
-                         size_t workspace_bytes, void *stream);
-
-/*
  * varq_quant_pack / varq_quant_pack2 (x1 != NULL) of groups that take in whole rows (reduce bit 3 set), with the scale of a group
  * written to every place that reads it -- the tokens, heads and batch entries that it serves -- instead of once: what a
  * cache of scales per token, or of one table per step, holds after the reference's expand and concatenation (VAR_Q/quant.py:196-201).

@@ -1,0 +1,31 @@
+/*
+ * varq_testing.h -- entry points of libvarq_hip.so that its tests need to reach and to recognise paths of varq_quant_pack.  They are not part
+ * of the interface and may change with any build; the conventions are those of varq.h.
+ */
+#ifndef VARQ_TESTING_H
+#define VARQ_TESTING_H
+
+#include "varq.h"
+
+#ifdef __cplusplus
+extern "C" {
+#endif
+
+/*
+ * varq_quant_pack with the time given that a workgroup waits for the others with which it shares its groups, in ticks of 10 ns, before
+ * it helps to read their rows (0: without waiting).  Results do not depend on it.
+ */
+int varq_quant_pack_wait(const void *x, int x_dtype, const int64_t *host_shape4, int reduce_mask, int bits, int asym, float eps, int32_t *words,
+                         int8_t *codes, float *scale, float *zp, const int64_t *host_out_map, uint32_t wait_ticks, void *workspace,
+                         size_t workspace_bytes, void *stream);
+
+/*
+ * How varq_quant_pack (tensors = 1) or varq_quant_pack2 (2) go about a valid call on the current device: n > 1: that many workgroups share each
+ * block of groups; 1: one workgroup takes each by itself; 0: neither, the input is read twice.  word_bits: bits of the packed codes, 8 for int8 codes.
+ */
+int varq_quant_pack_shards(const int64_t *host_shape4, int reduce_mask, int x_dtype, int tensors, int word_bits, int asym);
+
+#ifdef __cplusplus
+}
+#endif
+#endif /* VARQ_TESTING_H */

@@ -1,6 +1,6 @@
 """Workgroups that share their groups (`quant_shared_kernel`): rows that do not fill the last workgroup or step, more rows than the
 registers hold, octets that are no power of two, kept inner indices that do not fill the last tile, groups of whole rows; with the
-others' extremes waited for and, without waiting, with all rows read by whoever comes first.  Bit-exact against the CPU oracle."""
+others' extremes waited for and, without waiting, with their rows read by whoever comes first.  Bit-exact against the CPU oracle."""
 import math
 
 import pytest
@@ -14,6 +14,14 @@ from var_q_amd import _lib, ops
 pytestmark = pytest.mark.gpu
 
 
+DTYPE = {torch.float32: 0, torch.bfloat16: 1, torch.float16: 2}
+
+
+def _shards(x, dims, word_bits, asym, tensors=1):
+    """Workgroups that share each group; 1: one workgroup by itself, 0: the input is read twice."""
+    return _lib.load().varq_quant_pack_shards(_lib.i64arr(list(x.shape)), sum(1 << d for d in dims), DTYPE[x.dtype], tensors, word_bits, int(asym))
+
+
 def _without_waiting(x, dims, bits, asym, pack, ticks=0):
     mask = sum(1 << d for d in dims)
     lib, sh = _lib.load(), _lib.i64arr(list(x.shape))
@@ -23,15 +31,14 @@ def _without_waiting(x, dims, bits, asym, pack, ticks=0):
     q = torch.empty(*x.shape[:3], x.shape[3] * bits // 32 if pack else x.shape[3], dtype=torch.int32 if pack else torch.int8, device=x.device)
     size = lib.varq_quant_workspace_bytes(sh, mask)
     ws = torch.full(((size + 3) // 4,), -1, dtype=torch.int32, device=x.device)   # (any contents)
-    dt = {torch.float32: 0, torch.bfloat16: 1, torch.float16: 2}[x.dtype]
-    _lib.check(lib.varq_quant_pack_wait(x.data_ptr(), dt, sh, mask, bits, int(asym), 1e-12, q.data_ptr() if pack else None,
+    _lib.check(lib.varq_quant_pack_wait(x.data_ptr(), DTYPE[x.dtype], sh, mask, bits, int(asym), 1e-12, q.data_ptr() if pack else None,
                                         None if pack else q.data_ptr(), s.data_ptr(), z.data_ptr() if asym else None, None, ticks, ws.data_ptr(), size,
                                         torch.cuda.current_stream().cuda_stream), 'varq_quant_pack_wait')
     return q, s, z
 
 
 @pytest.mark.parametrize('shape,dims,dtype', [
-    ((2, 4, 16500, 64), (0, 2), torch.bfloat16),      # 1024 workgroups of five steps
+    ((2, 4, 16500, 64), (0, 2), torch.bfloat16),      # 828 workgroups of five steps
     ((64, 513, 7, 64), (0, 1), torch.float16),        # two kept indices to a block, the last block half full
     ((3, 11003, 5, 72), (0, 1), torch.float32),       # nine octets of sixteen lanes
     ((1, 4, 70001, 96), (0, 2), torch.bfloat16),      # 18 steps: two beyond the held ones
@@ -48,6 +55,7 @@ def test_shared_groups(dev, shape, dims, dtype):
     x[-1, -1, -1] = 40                                # the extreme of its groups, in the last rows of the last workgroup
     for bits, asym, pack in ((8, False, True), (2 if shape[3] % 16 == 0 else 4, True, True), (5, False, False)):
         note('quant shared', shape, dims, dtype, bits, asym, pack)
+        assert _shards(x, dims, bits if pack else 8, asym) > 1
         q, s, z = O.quant_reduce(x, dims, bits, asym)
         if pack:
             q = O.pack_last_dim(q, bits)[0]
@@ -62,6 +70,7 @@ def test_shared_groups_in_a_graph(dev):
     """The words that the workgroups exchange are cleared by every replay; K and V of a step in one launch."""
     shape, dims = (64, 129, 16, 64), (0, 1)
     xs = [torch.randn(*shape, device=dev).half() for _ in range(2)]
+    assert _shards(xs[0], dims, 8, True, tensors=2) > 1
     ops.quant_pack_pair(*xs, dims, 8, asym=True)
     graph = torch.cuda.CUDAGraph()
     with torch.cuda.graph(graph):
@@ -82,17 +91,18 @@ def test_shared_groups_in_a_graph(dev):
     ((2, 4, 300, 64), (0, 2), torch.bfloat16),
     ((4, 70, 8, 64), (0, 1), torch.float16),
     ((2, 4, 300, 64), (0, 2), torch.float32),
-    ((2, 5, 33, 32), (0, 3), torch.bfloat16),
+    ((2, 5, 33, 32), (0, 3), torch.bfloat16),       # groups of whole rows, whose extremes are folded over the columns too
+    ((2, 30, 35, 64), (0, 2, 3), torch.float32),
 ])
 def test_infinities_and_nan(dev, shape, dims, dtype, what):
     """The batch behind itself leaves every group what it is and takes workgroups that share it; alone it takes one launch."""
     x = _spoil(torch.randn(*shape, generator=torch.Generator().manual_seed(7)).to(dtype).to(dev), 1 if dims == (0, 1) else 2, what)
-    rows = math.prod(shape[d] for d in dims if d != 3)
-    times = max(26000 // rows + 1, (48 << 20) // (x.numel() * x.element_size()) + 1 if 3 in dims else 0)
+    times = (48 << 20) // (x.numel() * x.element_size()) + 1 if 3 in dims else 26000 // math.prod(shape[d] for d in dims) + 1
     for bits, asym in ((8, False), (8, True), (4, True), (2, True)):
         note('quant shared, non-finite', shape, dims, dtype, what, bits, asym)
         q1, s1, z1 = ops.quant_pack(x, dims, bits, asym=asym)
         many = x.repeat(times, 1, 1, 1)
+        assert _shards(x, dims, bits, asym) == 1 and _shards(many, dims, bits, asym) > 1
         for q, s, z in (ops.quant_pack(many, dims, bits, asym=asym), _without_waiting(many, dims, bits, asym, True)):
             assert torch.equal(_bits(s1), _bits(s)) and (not asym or torch.equal(_bits(z1), _bits(z)))
             assert torch.equal(q.view(times, *q1.shape), q1.expand(times, *q1.shape))
@@ -120,6 +130,7 @@ def test_giving_up_on_the_others_reads_the_rows_once_more(dev, shape, dims, dtyp
         return sorted(times)[7], got
 
     note('quant shared, giving up', shape, dims)
+    assert _shards(x, dims, 8, asym) > 1
     (patient, a), (hasty, b) = median_us(1000000), median_us(300)
     assert all(torch.equal(i, j) for i, j in zip(a, b) if i is not None)
     assert hasty < 3 * patient, (patient, hasty)

@@ -22,8 +22,6 @@ SYMBOLS = {
     'varq_quant_workspace_bytes': (c_size_t, [POINTER(c_int64), c_int]),
     'varq_quant_pack': (c_int, [c_void_p, c_int, POINTER(c_int64), c_int, c_int, c_int, c_float,
                                 c_void_p, c_void_p, c_void_p, c_void_p, POINTER(c_int64), c_void_p, c_size_t, c_void_p]),
-    'varq_quant_pack_wait': (c_int, [c_void_p, c_int, POINTER(c_int64), c_int, c_int, c_int, c_float, c_void_p, c_void_p, c_void_p, c_void_p,
-                                     POINTER(c_int64), c_uint32, c_void_p, c_size_t, c_void_p]),
     'varq_quant_pack2': (c_int, [c_void_p, c_void_p, c_int, POINTER(c_int64), c_int, c_int, c_int, c_float,
                                  c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p,
                                  POINTER(c_int64), c_void_p, c_size_t, c_void_p]),
@@ -79,6 +77,13 @@ SYMBOLS = {
                                          c_void_p, c_int, c_int64, c_int64, c_void_p]),
 }
 
+# include/varq_testing.h
+TESTING = {
+    'varq_quant_pack_wait': (c_int, [c_void_p, c_int, POINTER(c_int64), c_int, c_int, c_int, c_float, c_void_p, c_void_p, c_void_p, c_void_p,
+                                     POINTER(c_int64), c_uint32, c_void_p, c_size_t, c_void_p]),
+    'varq_quant_pack_shards': (c_int, [POINTER(c_int64), c_int, c_int, c_int, c_int, c_int]),
+}
+
 _lib = None
 _host = None
 
@@ -97,7 +102,7 @@ def load():
             f'{LIB_PATH} is missing: build it with `python -m var_q_amd.build` '
             '(hipcc, gfx950).  There is no fallback path.')
     lib = ctypes.CDLL(LIB_PATH)
-    for name, (res, args) in SYMBOLS.items():
+    for name, (res, args) in {**SYMBOLS, **TESTING}.items():
         fn = getattr(lib, name)  # AttributeError if the symbol is not exported
         fn.restype = res
         fn.argtypes = args

@@ -12,6 +12,7 @@
 // in which partial results meet.  Channel counts that are not a multiple of 8 and
 // rows wider than 512 channels take scalar kernels with ordered-integer atomics.
 #include "dequant_steps.h"
+#include "../../include/varq_testing.h"
 #include <algorithm>
 #include <mutex>
 #include <type_traits>
@@ -1350,6 +1351,15 @@ extern "C" size_t varq_quant_workspace_bytes(const int64_t *host_shape4, int red
 }
 
 namespace {
+// the launches that a tensor (or two of one shape) takes
+enum class Way { kOne, kShared, kThree, kAnyShape };
+Way choose_way(const int64_t *sh, int reduce_mask, int64_t n_groups, int elem, int tensors, int word_bits, bool asym, bool with_values, bool may_share, size_t words_each,
+               OnePlan &one, int &threads, OnePlan &by_many, Shards &shards) {
+  const bool shared = may_share && make_shared_plan(sh, reduce_mask, n_groups, elem, tensors, words_each, by_many, shards);
+  if (make_one_plan(sh, reduce_mask, elem, tensors, word_bits, asym, with_values, shared, one, threads)) return Way::kOne;
+  return shared ? Way::kShared : Way::kThree;
+}
+
 // x1 != NULL: a second tensor of the same shape with its own outputs, in the same launches
 // where the tiled kernels apply, one after the other through the same workspace otherwise
 int quant_pack_impl(const void *x, const void *x1, int x_dtype, const int64_t *host_shape4, int reduce_mask, int bits,
@@ -1428,12 +1438,13 @@ int quant_pack_impl(const void *x, const void *x1, int x_dtype, const int64_t *h
   hipStream_t st = (hipStream_t)stream;
   OnePlan one;
   int threads;
-  const int elem = x_dtype == VARQ_F32 ? 4 : 2, tensors = x1 ? 2 : 1;
   const size_t words_each = tiled ? plan_workspace_bytes(pl, ng) / sizeof(u32) : 0;
   OnePlan by_many;
   Shards sh = {};
-  const bool shared = tiled && !host_scale_map && make_shared_plan(s, reduce_mask, ng, elem, tensors, words_each, by_many, sh);
-  if (tiled && make_one_plan(s, reduce_mask, elem, tensors, words ? bits : 8, asym != 0, step != nullptr, shared, one, threads)) {
+  const Way way = tiled ? choose_way(s, reduce_mask, ng, x_dtype == VARQ_F32 ? 4 : 2, x1 ? 2 : 1, words ? bits : 8, asym != 0, step != nullptr, !host_scale_map,
+                                     words_each, one, threads, by_many, sh)
+                        : Way::kAnyShape;
+  if (way == Way::kOne) {
     if (step) {
       step->q_blocks = (one.blocks + 7) / 8 * 8 * one.slices;
       step->pair_blocks = (int)((step->earlier.pair_octs + kStepOctets - 1) / kStepOctets);
@@ -1452,7 +1463,7 @@ int quant_pack_impl(const void *x, const void *x1, int x_dtype, const int64_t *h
     if (x_dtype == VARQ_F32) run_one<VARQ_F32>(p, one, threads, st);
     else if (x_dtype == VARQ_BF16) run_one<VARQ_BF16>(p, one, threads, st);
     else run_one<VARQ_F16>(p, one, threads, st);
-  } else if (shared) {
+  } else if (way == Way::kShared) {
     if (x1) { p.x1 = x1; p.scale1 = scale1; p.zp1 = zp1; p.words1 = words1; p.codes1 = codes1; }
     p.ws1 = (int64_t)words_each;
     sh.mx = p.ws; sh.mn = p.ws + ng * sh.stride; sh.words = p.ws + 2 * ng * sh.stride;
@@ -1462,7 +1473,7 @@ int quant_pack_impl(const void *x, const void *x1, int x_dtype, const int64_t *h
     else run_shared<VARQ_F16>(p, by_many, sh, st);
   } else if (host_scale_map) {
     return varq_set_error(VARQ_ERR_UNSUPPORTED, "quant_pack: spread scales come with groups that one launch quantizes");
-  } else if (tiled) {
+  } else if (way == Way::kThree) {
     if (x1) { p.x1 = x1; p.scale1 = scale1; p.zp1 = zp1; p.words1 = words1; p.codes1 = codes1; }
     if (x_dtype == VARQ_F32) run_tiled<VARQ_F32>(p, pl, workspace, st);
     else if (x_dtype == VARQ_BF16) run_tiled<VARQ_BF16>(p, pl, workspace, st);
@@ -1505,6 +1516,18 @@ extern "C" int varq_quant_pack_wait(const void *x, int x_dtype, const int64_t *h
                                     size_t workspace_bytes, void *stream) {
   return quant_pack_impl(x, nullptr, x_dtype, host_shape4, reduce_mask, bits, asym, eps, words, codes, scale, zp, nullptr, nullptr, nullptr, nullptr,
                          host_out_map, workspace, workspace_bytes, stream, nullptr, 0, nullptr, nullptr, &wait_ticks);
+}
+
+extern "C" int varq_quant_pack_shards(const int64_t *host_shape4, int reduce_mask, int x_dtype, int tensors, int word_bits, int asym) {
+  const int64_t ng = count_groups(host_shape4, reduce_mask);
+  Plan pl;
+  if (!make_plan(host_shape4, reduce_mask, ng, pl) || (host_shape4[3] * word_bits) % 32 != 0) return 0;
+  OnePlan one, by_many;
+  Shards sh = {};
+  int threads;
+  const Way way = choose_way(host_shape4, reduce_mask, ng, x_dtype == VARQ_F32 ? 4 : 2, tensors, word_bits, asym != 0, false, true, plan_workspace_bytes(pl, ng) / sizeof(u32),
+                             one, threads, by_many, sh);
+  return way == Way::kShared ? sh.n : way == Way::kOne ? 1 : 0;
 }
 
 extern "C" int varq_quant_pack_spread_once(const void *x0, const void *x1, int x_dtype, const int64_t *host_shape4, int reduce_mask, int bits, int asym,
