@@ -16,15 +16,14 @@ from var_q_amd import ops
 pytestmark = pytest.mark.gpu
 
 SIZES = [(1, 1), (33, 63), (130, 64), (257, 65), (31, 128), (200, 129), (129, 321)]
+GROUPS = [(64, 32, 64, 'fp16'), (64, 64, 64, 'bf16'), (128, 32, 64, 'bf16'), (128, 128, 128, 'bf16')]
+# (300 pairs: workgroups of four wavefronts, at head dim 64 and up to 128 queries; 130 are on the other side of that line)
+CASES = [(*g, B, H, *size) for size in SIZES for B, H in ((1, 3), (75, 4)) for g in GROUPS if B == 1 or (g[0] == 64 and size[0] <= 130)]
 
 
-@pytest.mark.parametrize('Lq,Lk', SIZES)
-@pytest.mark.parametrize('B,H', [(1, 3), (75, 4)])      # 300 pairs: workgroups of four wavefronts, at head dim 64
-@pytest.mark.parametrize('D,gk,gv,dtype', [(64, 32, 64, 'fp16'), (64, 64, 64, 'bf16'), (128, 32, 64, 'bf16'), (128, 128, 128, 'bf16')])
+@pytest.mark.parametrize('D,gk,gv,dtype,B,H,Lq,Lk', CASES)
 @pytest.mark.parametrize('bits', [2, 4, 8])
 def test_groups(dev, bits, D, gk, gv, dtype, B, H, Lq, Lk):
-    if B > 1 and (D == 128 or Lq > 130):
-        pytest.skip('the same workgroups as with few pairs')
     seed = bits + D + gk + Lq * 7 + Lk
     gen = torch.Generator().manual_seed(seed)
     dt, scale = torch.float16 if dtype == 'fp16' else torch.bfloat16, 1 / math.sqrt(D)
