@@ -134,3 +134,31 @@ def test_giving_up_on_the_others_reads_the_rows_once_more(dev, shape, dims, dtyp
     (patient, a), (hasty, b) = median_us(1000000), median_us(300)
     assert all(torch.equal(i, j) for i, j in zip(a, b) if i is not None)
     assert hasty < 3 * patient, (patient, hasty)
+
+
+def _us(f, times=15):
+    got = []
+    for _ in range(times):
+        start, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        start.record()
+        for _ in range(10):
+            f()
+        end.record()
+        torch.cuda.synchronize()
+        got.append(start.elapsed_time(end) * 100)
+    return sorted(got)[times // 2]
+
+
+def test_extremes_of_whole_rows_lie_apart_where_the_workspace_is_small(dev):
+    """30 groups whose three launches have 60 chunks leave no room for a line for each extreme; 30 others of as many bytes do.  (Side by side in
+    memory the exchange took 1.8 times as long.)"""
+    dims = (0, 2, 3)
+    x, y = (torch.randn(*shape, device=dev) for shape in ((60, 30, 66, 128), (80, 30, 50, 128)))
+    assert _shards(x, dims, 4, True) > 1 and _shards(y, dims, 4, True) > 1
+    note('quant shared, room for half a line')
+    one, other = _us(lambda: ops.quant_pack(x, dims, 4, asym=True)), _us(lambda: ops.quant_pack(y, dims, 4, asym=True))
+    assert one < 1.35 * other, (one, other)
+    for t in (x, y):
+        s, z = O.quant_reduce(t.cpu(), dims, 4, True)[1:]
+        got = ops.quant_pack(t, dims, 4, asym=True)
+        assert torch.equal(got[1].cpu(), s) and torch.equal(got[2].cpu(), z)

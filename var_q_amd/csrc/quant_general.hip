@@ -1200,10 +1200,11 @@ bool make_shared_plan(const int64_t *sh, int reduce_mask, int64_t n_groups, int 
   n = (rr + ((int64_t)pl.steps << pl.sub_shift) - 1) / ((int64_t)pl.steps << pl.sub_shift);
   const int n_par = (keepc ? 8 << c8p_shift : 1) << pl.lq_shift, fold_vals = n_par * std::max(1, (1 << (pl.sub_shift + c8p_shift)) / 64);
   if (n < 2 || std::max(n_par, fold_vals) > kSharedGroups) return false;
-  // (lines of their own for the extremes of each group of whole rows and for the words of a block, where there is room: atomics on
-  // one line wait for one another)
+  // (lines of their own for the extremes of each group of whole rows and for the words of a block, and as far apart as there is room
+  // otherwise: atomics on one line wait for one another.  One scale per head of 30 heads, 60 or 61 chunks of the three launches and thus room for
+  // half a line: fp32 [60,30,66,128] affine 36.4 -> 19.7 us (side by side / 16 words apart; three launches 28.1), [3,30,3843,40] 33.7 -> 21.0 (26.4))
   s.n = (int)n;
-  s.stride = !keepc && 64 * (size_t)(n_groups + pl.blocks) <= words ? 32 : 1;
+  for (s.stride = keepc ? 1 : 32; s.stride > 1 && 2 * (size_t)s.stride * (size_t)n_groups + 64 * (size_t)pl.blocks > words;) s.stride /= 2;
   const size_t left = words - std::min(words, 2 * s.stride * (size_t)n_groups);
   for (s.spacing = 64; s.spacing >= 8 && (size_t)s.spacing * pl.blocks > left;) s.spacing /= 2;
   s.ticks = (u32)(10000 + (bytes >> 20) * 100);   // 0.1 ms, and 1 us for each MiB, several times what it takes
