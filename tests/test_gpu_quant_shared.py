@@ -18,8 +18,12 @@ DTYPE = {torch.float32: 0, torch.bfloat16: 1, torch.float16: 2}
 
 
 def _shards(x, dims, word_bits, asym, tensors=1):
+    return _shards_of(x.shape, x.dtype, dims, word_bits, asym, tensors)
+
+
+def _shards_of(shape, dtype, dims, word_bits, asym, tensors=1):
     """Workgroups that share each group; 1: one workgroup by itself, 0: the input is read twice."""
-    return _lib.load().varq_quant_pack_shards(_lib.i64arr(list(x.shape)), sum(1 << d for d in dims), DTYPE[x.dtype], tensors, word_bits, int(asym))
+    return _lib.load().varq_quant_pack_shards(_lib.i64arr(list(shape)), sum(1 << d for d in dims), DTYPE[dtype], tensors, word_bits, int(asym))
 
 
 def _without_waiting(x, dims, bits, asym, pack, ticks=0):
@@ -162,3 +166,24 @@ def test_extremes_of_whole_rows_lie_apart_where_the_workspace_is_small(dev):
         s, z = O.quant_reduce(t.cpu(), dims, 4, True)[1:]
         got = ops.quant_pack(t, dims, 4, asym=True)
         assert torch.equal(got[1].cpu(), s) and torch.equal(got[2].cpu(), z)
+
+
+@pytest.mark.parametrize('shape,dims,dtype,tensors,shared', [
+    # heads first, 16 bits, beyond 192 MiB: where the three launches are one round of workgroups, and where they are a little more
+    ((39, 8, 6115, 64), (0, 2), torch.float16, 1, False),
+    ((526, 16, 64, 128), (0, 2), torch.float16, 2, False),
+    ((635, 16, 508, 40), (0, 2, 3), torch.bfloat16, 1, False),
+    ((4, 24, 17568, 72), (0, 2), torch.bfloat16, 1, False),      # (of lanes that idle a smaller tensor)
+    ((2, 30, 40914, 72), (0, 2), torch.bfloat16, 1, False),      # (of nearly half of them: always)
+    ((402, 24, 517, 64), (0, 2), torch.bfloat16, 1, True),
+    ((39, 8, 5000, 64), (0, 2), torch.float16, 1, True),
+    ((36, 6, 5196, 64), (0, 2), torch.float32, 1, True),
+    # few workgroups, 16 bits: up to 24 steps of a workgroup, 16 of them held
+    ((4, 3, 12000, 64), (0, 2), torch.float16, 1, True),
+    ((284, 3, 680, 128), (0, 2), torch.float16, 1, False),
+    ((2, 3, 125467, 128), (0, 2, 3), torch.bfloat16, 1, False),
+    ((1, 3, 91810, 128), (0, 2), torch.float32, 1, True),
+])
+def test_where_the_launches_that_read_twice_are_faster(dev, shape, dims, dtype, tensors, shared):
+    """Sizes on either side of the lines, with both ways timed on a device of their own (the figures are at make_shared_plan)."""
+    assert (_shards_of(shape, dtype, dims, 4, True, tensors) > 1) == shared

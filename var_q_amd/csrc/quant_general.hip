@@ -1162,11 +1162,16 @@ bool make_one_plan(const int64_t *sh, int reduce_mask, int elem, int tensors, in
 }
 
 // The plan of workgroups that share their groups, in `words` of workspace per tensor, or false where it does not pay whatever one launch
-// takes.  Tokens first, tensors of 16 bits lose beyond 192 MiB, where the second read comes from memory and 256 bytes of a row in eight
-// sets of workgroups are the worse way through it: [64,n,16,64] fp16 125 MiB 71.8 -> 63.5 us, 187 105 -> 99, 250 135 -> 144, 500 266 -> 301; fp32
-// 250 119 -> 107, 375 195 -> 174.  Groups of whole rows gain from 48 MiB: 8 bits affine, a scale per head of [B,30,680,64] bf16, 20 MiB
+// takes; three_wgs: the workgroups of either of the large ones among the three launches.  Tokens first, tensors of 16 bits lose beyond 192 MiB, where the second
+// read comes from memory and 256 bytes of a row in eight sets of workgroups are the worse way through it: [64,n,16,64] fp16 125 MiB 71.8 -> 63.5 us, 187
+// 105 -> 99, 250 135 -> 144, 500 266 -> 301; fp32 250 119 -> 107, 375 195 -> 174.  Heads first they lose from there on (lanes that idle counted in) where the three
+// launches come out as one round of eight workgroups per compute unit, three -> this: [2199,8,256,72] 618 MiB 357 -> 486, [4,24,17568,72] 232 125 -> 148, [8,16,14491,64] 226
+// 109 -> 116, [39,8,6115,64] 233 affine 115 -> 126, a scale per head of [635,16,508,40] 394 240 -> 296; with 2050 to 2070 workgroups, where a few are a second round,
+// the three take longer: [402,24,517,64] 609 397 -> 322, [162,30,169,128] 201 110 -> 90, unless nearly half of the lanes idle, [339,20,680,72] 633
+// 483 -> 518, [2,30,40914,72] 337 230 -> 274 (against [3184,12,169,40] 493 370 -> 355).  Of 394 forms of 16 bits from 11 to 880 MiB 51 were slower by more than 2.5 % than the three
+// without this line and that of `few`, six with them, the worst of which are tokens first in idle lanes ([2223,36,30,40] 104 -> 134).  Groups of whole rows gain from 48 MiB: 8 bits affine, a scale per head of [B,30,680,64] bf16, 20 MiB
 // 18.1 -> 21.9, 30 22.6 -> 19.4, 40 27.4 -> 31.3, 50 33.1 -> 27.6, 80 48.9 -> 38.0, per token 50 34.2 -> 25.7.
-bool make_shared_plan(const int64_t *sh, int reduce_mask, int64_t n_groups, int elem, int tensors, size_t words, OnePlan &pl, Shards &s) {
+bool make_shared_plan(const int64_t *sh, int reduce_mask, int64_t n_groups, int elem, int tensors, size_t words, int64_t three_wgs, OnePlan &pl, Shards &s) {
   const int64_t c = sh[3], rows = sh[0] * sh[1] * sh[2];
   if (c % 8 != 0 || c > 512 || rows <= 0 || rows >= (1ll << 31) - 512) return false;
   const Canonical k = canonical(sh, reduce_mask);
@@ -1179,6 +1184,8 @@ bool make_shared_plan(const int64_t *sh, int reduce_mask, int64_t n_groups, int 
   const int c8 = (int)(c / 8);
   int c8p_shift = 0;
   while ((1 << c8p_shift) < c8) ++c8p_shift;
+  const bool half_idle = 7 * c8 <= 4 << c8p_shift;
+  if (k.RI > 1 && elem == 2 && (half_idle || three_wgs <= 8 * (int64_t)device_cus()) && (bytes / c8 << c8p_shift) > (192ll << 20)) return false;
   pl.ko_rs = k.ko_rs; pl.ro_rs = k.ro_rs; pl.ko_gs = k.ko_gs; pl.q_gs = k.q_gs;
   pl.nko = (int)k.nko; pl.Q = (int)k.Q; pl.RR = (int)rr; pl.RI = (int)k.RI; pl.by_RI = FastDiv::by(k.RI);
   pl.c8s_shift = c8p_shift; pl.slices = 1;
@@ -1192,12 +1199,16 @@ bool make_shared_plan(const int64_t *sh, int reduce_mask, int64_t n_groups, int 
   pl.blocks = pl.nko * pl.tilesQ;
   // as many workgroups as the chip holds at once, of at least four steps (groups of whole rows: eight), and no more than meet quickly; of
   // fewer than three per compute unit, or than nearly four where lanes idle, the three launches read faster (two heads: fp32 [1,2,381944,72], one scale per
-  // head, 103 -> 128 us, fp16 [2,2,381944,72] 139 -> 261; three: fp16 [2,3,23148,72] 22.3 -> 23.6, but fp32 [5,3,28645,128] 104 -> 87)
+  // head, 103 -> 128 us, fp16 [2,2,381944,72] 139 -> 261; three: fp16 [2,3,23148,72] 22.3 -> 23.6, but fp32 [5,3,28645,128] 104 -> 87), in 16 bits also of fewer than
+  // three and a half where more rows are read again than half of those that the registers hold (three heads, 768 workgroups: 16 steps 31.8 -> 30.9, 18 31.5 -> 30.4,
+  // 25 38.5 -> 40.1, 48 62.5 -> 65.1, 89 109 -> 139, 283 417 -> 537)
   const int64_t least = (keepc ? 4ll : 8ll) << pl.sub_shift;
   int64_t n = std::min<int64_t>({(int64_t)device_cus() * 4 / ((int64_t)pl.blocks * tensors), (rr + least - 1) / least, 256});
   if (n < 2 || n * pl.blocks * tensors * 4 < (int64_t)device_cus() * (c8 == 1 << c8p_shift ? 12 : 15)) return false;
   pl.steps = (int)((rr + (n << pl.sub_shift) - 1) / (n << pl.sub_shift));
   n = (rr + ((int64_t)pl.steps << pl.sub_shift) - 1) / ((int64_t)pl.steps << pl.sub_shift);
+  const bool few = n * pl.blocks * tensors * 2 < (int64_t)device_cus() * 7;
+  if (elem == 2 && few && pl.steps > 24) return false;
   const int n_par = (keepc ? 8 << c8p_shift : 1) << pl.lq_shift, fold_vals = n_par * std::max(1, (1 << (pl.sub_shift + c8p_shift)) / 64);
   if (n < 2 || std::max(n_par, fold_vals) > kSharedGroups) return false;
   // (lines of their own for the extremes of each group of whole rows and for the words of a block, and as far apart as there is room
@@ -1256,6 +1267,8 @@ template <int DT> void run_shared(const GenParams &p, const OnePlan &pl, const S
   else { if (p.keepc) launch_shared<DT, false, true>(p, pl, sh, st); else launch_shared<DT, false, false>(p, pl, sh, st); }
 }
 
+// workgroups of the min/max launch, and of the one that quantizes
+int64_t large_wgs(const Plan &pl) { return (int64_t)pl.nko * pl.tilesQ * pl.Z; }
 size_t plan_workspace_bytes(const Plan &pl, int64_t n_groups) {
   return (size_t)n_groups * (2 + 2 * (size_t)pl.Z) * sizeof(float);
 }
@@ -1269,7 +1282,7 @@ int run_tiled(GenParams &p, const Plan &pl, void *workspace, hipStream_t st) {
   float *part_min = part_max + (int64_t)pl.Z * ng;
   const unsigned nt = p.x1 ? 2u : 1u;   // tensors per launch (grid.y)
   p.ws1 = (int64_t)(plan_workspace_bytes(pl, ng) / sizeof(float));
-  dim3 grid((unsigned)((int64_t)pl.nko * pl.tilesQ * pl.Z), nt);
+  dim3 grid((unsigned)large_wgs(pl), nt);
   if (p.asym) {
     if (p.keepc) hipLaunchKernelGGL((minmax_tiled_kernel<DT, true, true>), grid, dim3(256), 0, st, p, pl, part_max, part_min);
     else hipLaunchKernelGGL((minmax_tiled_kernel<DT, true, false>), grid, dim3(256), 0, st, p, pl, part_max, part_min);
@@ -1355,8 +1368,8 @@ namespace {
 // the launches that a tensor (or two of one shape) takes
 enum class Way { kOne, kShared, kThree, kAnyShape };
 Way choose_way(const int64_t *sh, int reduce_mask, int64_t n_groups, int elem, int tensors, int word_bits, bool asym, bool with_values, bool may_share, size_t words_each,
-               OnePlan &one, int &threads, OnePlan &by_many, Shards &shards) {
-  const bool shared = may_share && make_shared_plan(sh, reduce_mask, n_groups, elem, tensors, words_each, by_many, shards);
+               int64_t three_wgs, OnePlan &one, int &threads, OnePlan &by_many, Shards &shards) {
+  const bool shared = may_share && make_shared_plan(sh, reduce_mask, n_groups, elem, tensors, words_each, three_wgs, by_many, shards);
   if (make_one_plan(sh, reduce_mask, elem, tensors, word_bits, asym, with_values, shared, one, threads)) return Way::kOne;
   return shared ? Way::kShared : Way::kThree;
 }
@@ -1443,7 +1456,7 @@ int quant_pack_impl(const void *x, const void *x1, int x_dtype, const int64_t *h
   OnePlan by_many;
   Shards sh = {};
   const Way way = tiled ? choose_way(s, reduce_mask, ng, x_dtype == VARQ_F32 ? 4 : 2, x1 ? 2 : 1, words ? bits : 8, asym != 0, step != nullptr, !host_scale_map,
-                                     words_each, one, threads, by_many, sh)
+                                     words_each, large_wgs(pl), one, threads, by_many, sh)
                         : Way::kAnyShape;
   if (way == Way::kOne) {
     if (step) {
@@ -1527,7 +1540,7 @@ extern "C" int varq_quant_pack_shards(const int64_t *host_shape4, int reduce_mas
   Shards sh = {};
   int threads;
   const Way way = choose_way(host_shape4, reduce_mask, ng, x_dtype == VARQ_F32 ? 4 : 2, tensors, word_bits, asym != 0, false, true, plan_workspace_bytes(pl, ng) / sizeof(u32),
-                             one, threads, by_many, sh);
+                             large_wgs(pl), one, threads, by_many, sh);
   return way == Way::kShared ? sh.n : way == Way::kOne ? 1 : 0;
 }
 
