@@ -187,3 +187,18 @@ def test_extremes_of_whole_rows_lie_apart_where_the_workspace_is_small(dev):
 def test_where_the_launches_that_read_twice_are_faster(dev, shape, dims, dtype, tensors, shared):
     """Sizes on either side of the lines, with both ways timed on a device of their own (the figures are at make_shared_plan)."""
     assert (_shards_of(shape, dtype, dims, 4, True, tensors) > 1) == shared
+
+
+@pytest.mark.parametrize('shape,dims,dtype,tensors,asym,one', [
+    ((32, 30, 55, 96), (0, 2), torch.float32, 2, True, True),
+    ((8, 476, 30, 96), (0, 1), torch.float32, 1, False, True),
+    ((4, 24, 987, 128), (0, 2), torch.float32, 1, False, True),
+    ((8, 16, 498, 72), (0, 2), torch.float32, 1, False, True),
+    ((16, 16, 494, 72), (0, 2), torch.float32, 1, True, False),
+    ((2, 30, 1060, 96), (0, 2), torch.float32, 2, True, False),    # two rounds of workgroups
+    ((1, 24, 4270, 128), (0, 2), torch.float16, 1, True, False),
+    ((1, 30, 5888, 96), (0, 2), torch.float32, 1, False, False),   # pieces of 32 bytes
+])
+def test_where_one_workgroup_per_group_is_faster(dev, shape, dims, dtype, tensors, asym, one):
+    """Sizes on either side of the line, with both ways timed (the figures are at one_launch_pays)."""
+    assert (_shards_of(shape, dtype, dims, 4, asym, tensors) == 1) == one

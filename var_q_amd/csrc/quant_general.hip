@@ -1106,6 +1106,13 @@ bool one_launch_pays(const OnePlan &pl, int c8, int c8p, int threads, bool keepc
   const double per_kib = piece <= 16 ? (wgs <= 128 ? 0.175 : 0.22) : piece == 32 ? (apart ? 0.17 : 0.135) : 0.10;
   const double one = 4.5 + per_kib * (asym ? 1.1 : 1.0) * mib * 1024.0 / (double)wgs * (double)((wgs + cus - 1) / cus);
   const double pad = (double)c8p / c8;
+  // (32 bits, one round, long pieces, or heads first where lanes of the other way idle and a thread has few rows: the estimates of both ways are too
+  // far off, and the one launch stays where it was before workgroups could share. One / shared: [32,30,55,96] two tensors affine 14.9 / 18.3,
+  // [16,112,24,96] tokens first, two 12.8 / 15.2, [8,476,30,96] 15.9 / 17.9, [3,24,973,128] 12.7 / 14.2, [2,16,1779,128] two affine 19.1 / 21.1,
+  // [4,24,987,128] 16.9 / 17.9, but [1,2611,12,128] two affine 15.1 / 14.7, [4,838,20,128] affine 17.4 / 15.2; short pieces, [8,16,498,72] 9.5 /
+  // 12.5, [1,16,4718,72] 10.1 / 13.3, [2,6,3020,72] two 12.5 / 13.7, [8,30,708,40] affine 14.4 / 15.7, of eight rows [16,16,494,72] affine 23.2 /
+  // 18.9)
+  if (shared && elem == 4 && wgs <= cus && (piece >= 64 || (pl.RI > 1 && pad >= 1.6 && pl.steps <= 6))) shared = false;
   if (shared) return 0.9 * one < 11.0 + (elem == 4 ? 0.25 : 0.37) * mib * pad + (asym ? 1.0 : 0.0) + (with_values ? 10.5 : 0.0);
   const double three = (tensors == 2 ? 16.2 + 0.41 * mib * pad : 12.4 + 0.44 * mib * pad) + (asym ? 3.0 : 0.0) + (with_values ? 10.5 : 0.0);
   return one < three;
