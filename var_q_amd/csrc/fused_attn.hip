@@ -713,7 +713,7 @@ template <int BITS> struct Widen {
   }
 };
 // Rows of K and V in LDS (stride in elements).  K: 16 lanes read 16 bytes of 16 rows each, 4 banks apart.  V: 32 lanes read 64 bytes of four
-// rows each, 16 banks apart (4 banks apart, as K's, they got in one another's way).
+// rows each, at D=128 16 banks apart (4 banks apart, as K's, they got in one another's way); at D=64 they are 4 apart too, where 16 measured the same.
 template <int D> constexpr int kKRow = D + 8;
 template <int D> constexpr int kVRow = D + (D == 128 ? 32 : 8);
 template <int D> constexpr int kKBuf = BN * kKRow<D>;   // a tile (elements)
@@ -1340,26 +1340,26 @@ template <int BITS> void launch_exact(const AttnParams &p, hipStream_t st) {
 template <int BITS, bool CHAN, bool F16> void launch_d64(const AttnParams &p, hipStream_t st) {
   // More (batch, head) pairs than compute units, at most four wavefronts of queries each:
   // workgroups of four wavefronts (same arithmetic, same results).  Also for one or two
-  // wavefronts of queries: the wavefronts without queries share the staging and the widening
-  // of the tiles, which is what such a workgroup spends its time on (workgroups of two
-  // wavefronts, also two to a compute unit by their LDS, took 20-35 % longer on 16-64 queries).
-  // Such a workgroup is a chain of loads, barriers and short computations, so what counts is how many
-  // are resident: three to a compute unit where tiles are pipelined through two of each buffer (2-bit
-  // codes in groups: four), four with one of each.  A single tile of keys has nothing to pipeline, and
-  // pairs that do not fit the device in one round of three are better off with four: two buffers -> one,
-  // us, [64,n,16,64] (1024 pairs), 8-bit codes with per-channel tables 36 queries x 91 keys 21.7 -> 14.6,
-  // 64 x 155 27.6 -> 19.1, 100 x 600 61.8 -> 47.0, 128 x 2500 206 -> 169; 4 bits in groups of 32 12.4 -> 11.9,
-  // 17.3 -> 15.7, 46.9 -> 43.9, 162 -> 152, 2 bits in groups 10.1 -> 10.6, 13.4 -> 14.2; with 768 pairs 8 bits in
-  // groups 8.2 -> 8.4, 10.8 -> 11.1, with 512 6.8 -> 7.1, 8.9 -> 9.3.
+  // wavefronts of queries: the wavefronts without queries share the widening
+  // of the tiles, which is what such a workgroup spends its time on.
+  // Such a workgroup is a chain of loads, barriers and short computations, so what counts is how many are resident.  Two of each
+  // buffer are 36 864 bytes: four workgroups to a compute unit, three with the tables of eight steps or more (four with zero-points) behind
+  // them and, by its registers (132), with 8-bit codes in groups.  One of each: four always, though for 8-bit codes in groups at the price of
+  // 24 bytes of spills.  From more pairs on than one round of three, one buffer gains where two would leave three workgroups, and elsewhere
+  // they come out the same; 2-bit codes in groups lose a little and keep two.  Two buffers / one, us, fp16 [64,n,16,64] (1024 pairs), 36 queries x
+  // 91 keys, 64 x 155, 100 x 600, 128 x 1250: 8 bits with ten tables 14.7 / 11.1, 19.6 / 14.8, 43.8 / 38.1, 81.3 / 71.1, with five
+  // 10.5 / 10.3, 13.4 / 13.7, 37.2 / 36.9, 70.8 / 70.8, in groups of 32 10.6 / 10.4, 16.4 / 15.5, 43.5 / 42.5, 85.2 / 81.2; 4 bits in groups 9.6 /
+  // 9.6, 13.8 / 13.5, 39.9 / 40.2, 78.8 / 79.1; 2 bits in groups 10.0 / 10.0, 13.9 / 13.8, 41.3 / 42.1, 79.8 / 80.4; 768 pairs, 8 bits with ten tables
+  // 9.6 / 9.8, 11.9 / 12.5, 31.4 / 31.3, 56.9 / 56.8, in groups 8.2 / 9.0, 11.1 / 12.3, 32.5 / 33.4, 63.4 / 64.7.  A single tile of keys has nothing to pipeline, and one
+  // buffer is the same with tables (64 queries x 64 keys, three tables, 512 pairs 6.5 / 6.6, 1920 16.3 / 16.1); in groups it is behind,
+  // 4 bits 5.6 / 5.8, 13.6 / 13.8, 8 bits 5.6 / 6.5, 15.6 / 16.4.
   if (p.Lq <= 128 && p.bh_total > device_cus()) {
     const bool rounds = (int64_t)p.bh_total * p.nsplit > 3 * device_cus() && (CHAN || BITS != 2);
     if (p.Lk <= BN || rounds) launch_shape<64, BITS, CHAN, 4, 4, F16, true>(p, st);
     else launch_shape<64, BITS, CHAN, 4, 3, F16>(p, st);
     return;
   }
-  // The kernels at D=64 fit 128 registers at the price of 24-48 bytes of spills,
-  // and two resident workgroups per compute unit hide each other's prologue and barriers
-  // (8-15 % faster than one workgroup at 140 registers).
+  // (114 to 122 registers, no spills: two resident workgroups per compute unit hide each other's prologue and barriers)
   launch_shape<64, BITS, CHAN, 8, 4, F16>(p, st);
 }
 
@@ -1436,7 +1436,10 @@ size_t split_workspace_bytes(int splits, int64_t rows, int D) {
 // a grid that already fills the device in whole rounds does not.
 int choose_splits(int64_t wgs, int tiles, int64_t rows, int D) {
   const double cus = device_cus();
-  // (D=64, no sharing / what the former 9 us and 4 TB/s chose / now: 32 pairs, 256 x 521 18.8 / 18.8 / 15.6; 128 pairs, 256 x 1500 44.8 / 44.8 / 36.0)
+  // (No sharing / what this chooses / the best of one to eight, us, 4 bits: D=64, 32 pairs, 256 x 521 17.3 / 14.8 / 14.8, 256 x 1500 38.2 / 19.9 / 18.5, 128 pairs, 256 x 1500
+  // 39.0 / 31.6 / 31.5, 1024 x 2521 110 / 111 / 110, 240 pairs, 256 x 1500 41.1 / 41.2 / 41.1; D=128, 16 pairs, 576 x 1497 56.1 / 32.2 / 32.1, 32 pairs, 256 x 521 25.5 / 22.8 / 21.5, 1024 x 2521
+  // 89.8 / 62.7 / 62.7, 128 pairs, 256 x 2521 90.4 / 62.5 / 62.4, 240 pairs 94.7 / 94.8 / 94.7; 8 bits with tables likewise.  Of 140 forms eight are 6 to 10 % behind the best, for instance few queries x many keys on a
+  // nearly full device, D=64, 128 pairs, 200 x 4096 97.4 / 59.2 / 54.2, 240 pairs 98.8 / 99.1 / 90.5, and D=128, 64 pairs, 512 x 1024 41.8 / 41.8 / 38.5.)
   const double tile_us = D == 128 ? 2.3 : 1.4, fixed_us = D == 128 ? 9.0 : 6.0, bytes_us = D == 128 ? 4.0e6 : 5.0e6, gain = D == 128 ? 0.9 : 0.92;
   double base = 0.0, best = 0.0;
   int best_s = 1;
@@ -1477,12 +1480,13 @@ int set_splits(AttnParams &p, int D, int tiles, int splits, void *workspace, siz
 // ---- few queries (few_attn.hip) -----------------------------------------------------------------
 // Launches of at most kFewQueries queries per (batch, head), in tiles of 32 that each dequantize the cache for themselves,
 // against 256 a workgroup and staged tiles of 64 keys in the kernel above.  Measured, us, the kernel above / that one, 4-bit
-// codes, one group, pairs of (batch, head) x queries x keys: up to 16 queries it is faster everywhere, D=64 32 x 16 x 32 4.2 / 3.8, 128 x 16 x 4096 44.7 /
-// 18.9, 240 x 16 x 1024 22 / 9.5, D=128 32 x 8 x 21 5.3 / 4.5, 240 x 16 x 1024 27.7 / 18.0.  More queries have two columns of 16 to prepare first: from the
-// second tile of keys on, D=64 32 x 24 x 64 4.4 / 5.0, x 128 5.6 / 4.9; D=128 5.7 / 6.6, 7.6 / 6.6.  Several tiles of queries that do not fit the device
-// at once pay with longer caches only, D=64 240 x 64 (480 tiles) x 128 6.7 / 7.3, x 256 9.4 / 9.1, x 1024 23.6 / 17.9, 480 x 64 (960) x 256 12.5 / 13.6, x 512
-// 19.8 / 18.6; three and four tiles not beyond the device, 240 x 100 x 1024 23.7 / 28.8, and not where the widening dominates, 128 x
-// 100 x 1024 21.2 / 18.0, x 2048 29.7 / 29.2, x 4096 48.4 / 52.0.
+// codes, one group, pairs of (batch, head) x queries x keys: up to 16 queries it is faster everywhere, D=64 32 x 16 x 32 3.9 / 3.8, 128 x 16 x 4096 40.4 /
+// 18.1, 240 x 16 x 1024 19.7 / 8.6, D=128 32 x 8 x 21 4.7 / 4.6, 240 x 16 x 1024 28.1 / 17.5.  More queries have two columns of 16 to prepare first: from the
+// second tile of keys on, D=64 32 x 24 x 64 4.1 / 5.0, x 128 5.1 / 5.0, x 256 7.1 / 5.9; D=128 5.2 / 6.6, 6.7 / 6.7.  Several tiles of queries that do not fit the device
+// at once pay with longer caches only, D=64 240 x 64 (480 tiles) x 128 5.7 / 6.7, x 256 7.7 / 8.1, x 400 10.6 / 10.6, x 1024 20.3 / 17.4, 480 x 64 (960) x 256 10.6 / 12.7, x 512
+// 17.7 / 18.4, x 768 25.0 / 24.2; three and four tiles not beyond the device, 240 x 100 x 1024 21.4 / 29.0, and not where the widening dominates, 128 x
+// 100 x 1024 18.5 / 17.2, x 2048 27.1 / 29.5, x 4096 43.1 / 53.4.  (The kernel above got faster since these lines were drawn: where they cross at 256, 512 and
+// 2048 keys it is up to a tenth ahead by now, at D=128, 128 x 100 x 2048, 37.5 / 44.1; 8-bit codes the same.)
 constexpr int kFewQueries = 128;
 constexpr int kMaxKeyShares = kMaxKeyShares_v;
 bool fewq_eligible(int B, int Hkv, int Lq, int Lk, int D, int k_group, int v_group) {
@@ -1549,16 +1553,17 @@ int wide_batch(int B, int Hkv, int Lk, int D) {
 }
 // Worth it from five (D = 128) or six blocks of 256 queries per (batch, head) on: expanding costs what
 // widening costs the kernel above in a block or two, and then its way through memory; and on a device
-// that is not nearly full the three launches cost more than they save.  Measured (us, 4-bit codes, the
-// kernel above / this): D=128 B=2 H=16 1024 x 2521 69 / 75, 1300 x 3000 109 / 104, 1600 x 4121 146 / 134,
-// 2304 x 6425 339 / 250; B=8 1024 x 2521 198 / 208, 1300 x 3000 325 / 311, 2304 x 6425 1116 / 953; B=1 H=8
-// 1600 x 4121 59 / 69; D=64 B=2 1600 x 4121 105 / 95, B=8 1300 x 3000 181 / 191, 2304 x 6425 609 / 578.
+// that is not nearly full the three launches cost more than they save.  Measured (us, 4-bit codes in groups, 8-bit ones with five tables,
+// the kernel above / this): D=128 B=2 H=16 1024 x 2521 69.8 / 71.3, 63.3 / 71.8, 1300 x 3000 107 / 95, 104 / 95, 1600 x 4121 145 / 123, 138 / 125,
+// 2304 x 6425 331 / 232, 329 / 243; B=8 1024 x 2521 191 / 194, 191 / 204, 1300 x 3000 318 / 285, 308 / 300, 2304 x 6425 1085 / 884, 1081 / 914; B=1 H=8
+// 1600 x 4121 55 / 60, 54 / 63; D=64 B=2 1600 x 4121 98 / 90, 95 / 86, B=8 1300 x 3000 182 / 178, 177 / 180, 1600 x 4121 317 / 285, 304 / 294, 2304 x 6425 626 / 553,
+// 607 / 567, but B=30 1600 x 4121 1030 / 1047, 995 / 1062.
 // Under key limits (measured with the block-causal rule over a whole sequence, pairs x tokens): D=128 all of 16 to 128
-// pairs x 2521 to 10521 are as fast or faster, 16 x 2521 99 / 98, 128 x 2521 353 / 346, 48 x 2952 243 / 192, 32 x 4121
-// 288 / 218, 32 x 10521 1303 / 1057.  D=64 gains where the longest query blocks are the whole of the time, up to about
-// a block and a quarter per compute unit, 16 x 2521 72 / 66, 24 x 3256 88 / 80, 16 x 4121 108 / 97, and in long sequences,
-// 32 x 6425 305 / 277, 128 x 6425 1112 / 1060; in between it goes either way, 32 x 3256 94 / 102, 128 x 4121 522 / 528,
-// 320 x 2952 665 / 715, 48 x 5417 321 / 330.  (Few pairs: wide_four.)
+// pairs x 2521 to 10521 are faster, 16 x 2521 91 / 86, 128 x 2521 339 / 322, 48 x 2952 228 / 183, 32 x 4121
+// 284 / 197, 32 x 10521 1325 / 1038.  D=64 gains where the longest query blocks are the whole of the time, up to about
+// a block and a quarter per compute unit, 16 x 2521 62.6 / 56.8, 24 x 3256 84.5 / 76.8 (though 16 x 4121 85.6 / 88.2), and in long sequences,
+// 32 x 6425 322 / 272, 128 x 6425 1142 / 1050; in between it goes either way, 32 x 3256 89.5 / 100, 128 x 4121 513 / 489,
+// 320 x 2952 645 / 683, 48 x 5417 328 / 319.  (Few pairs: wide_four.)
 bool wide_eligible(int B, int Hkv, int Lq, int Lk, int D, bool limits) {
   const int64_t bh = (int64_t)wide_batch(B, Hkv, Lk, D) * Hkv, blocks = bh * ((Lq + 255) / 256);
   if (bh > 0 && wide_four(bh, Lq, Lk, D, device_cus(), limits)) return true;

@@ -586,28 +586,29 @@ namespace varq_attn {
 // A sequence attended as a whole under key limits ends when its last query blocks do, which see every key: with few pairs
 // most of the device waits for them, and blocks of 128 queries are done sooner (a tile takes four wavefronts 1.25 us where it takes eight 1.8)
 // and are twice as many to fill it with.  Block-causal rule, 4-bit codes, us, the kernel that widens per workgroup / blocks of
-// 256 / of 128: D=64, 16 pairs of 680 tokens 24.7 / 24.2 / 19.4, of 2440 66.9 / 58.1 / 47.1, of 5064 140 / 113 / 104; 32 pairs of 255
-// 14.4 / 16.9 / 14.0, of 680 25.0 / 26.2 / 21.7, of 1656 49.6 / 47.7 / 40.5, of 2440 71.1 / 65.1 / 63.8, of 3464 102 / 102 / 101; D=128, 16 of 680 31.2 / 34.6 / 26.3,
-// of 2440 93.6 / 84.5 / 65.3, of 5064 181 / 154 / 165; 32 of 680 33.1 / 38.1 / 29.9, of 1656 68.8 / 68.5 / 64.9, of 2440 97 / 89 / 105.  With 64 pairs the
-// device is full: 680 tokens 25.4 / 29.7 / 27.2 and 34.5 / 44.1 / 44.8.  With fewer than ten pairs the shares of the keys do
-// better (8 pairs, widening / 128: D=64 1656 tokens 30.1 / 31.5, 2440 39.9 / 43.2; 10 pairs of 2440 48.8 / 45.8,
-// of 5064 112 / 99; D=128 50 / 44 at 1656, 161 / 165 at 5064), and 155 tokens are too few (11.3 / 12.8).
+// 256 / of 128: D=64, 16 pairs of 680 tokens 19.3 / 21.8 / 16.7, of 2440 61.1 / 56.0 / 42.1, of 5064 130 / 114 / 116; 32 pairs of 255
+// 10.9 / 14.8 / 11.5, of 680 21.9 / 23.5 / 18.7, of 1656 43.4 / 45.2 / 35.6, of 2440 63.7 / 61.8 / 63.6, of 3464 130 / 139 / 116; D=128, 16 of 680 29.4 / 31.6 / 24.2,
+// of 2440 89.2 / 83.5 / 64.6, of 5064 176 / 156 / 184; 32 of 680 32.2 / 35.6 / 28.7, of 1656 63.6 / 65.0 / 59.7, of 2440 91 / 86 / 99.  With 64 pairs the
+// device is full: 680 tokens 22.3 / 26.9 / 23.1 and 33.3 / 41.4 / 41.4.  With fewer than ten pairs the shares of the keys do
+// better (8 pairs, widening / 128: D=64 1656 tokens 26.0 / 27.7, 2440 35.5 / 37.8; 10 pairs of 2440 43.8 / 39.0,
+// of 5064 127 / 106; D=128 44.5 / 40.9 at 1656, 178 / 185 at 5064), and 155 tokens are too few (11.3 / 15.0).
 // Without limits, where the shares of the keys fill the device, a block of 128 gains at most a tenth, and only where it takes exactly the
-// device and the keys are few.  All launches, 4-bit codes, us, widening per workgroup with its shares / blocks of 256 / of 128:
+// device and the keys are few.  All launches, 4-bit codes, us, widening per workgroup with its shares / blocks of 256 / of 128 (the last
+// measured earlier and on another card than the others, by up to a tenth slower):
 //   D=128, queries x keys   16 pairs          32 pairs          64 pairs           128 pairs
-//    256 x  521         20.2 / 28.6 / 21.6   21.9 / 31.2 / 25.0   26.1 / 38.9 / 32.2   27.0 / 44.5 / 38.6
-//    256 x 2521         28.5 / 41.4 / 61.9   34.1 / 47.3 / 64.6   43.1 / 61.2 / 67.0   65.2 / 102 / 87.1
-//    512 x  521         23.9 / 28.3 / 21.9   26.6 / 31.8 / 25.1   27.7 / 40.4 / 34.2   31.2 / 47.2 / 49.1
-//    512 x 1024         28.3 / 38.2 / 29.5   33.0 / 47.2 / 37.8   42.1 / 56.1 / 46.0   46.4 / 59.8 / 67.9
-//    512 x 2521         36.1 / 44.1 / 62.0   44.4 / 52.6 / 64.9   65.1 / 77.9 / 70.1   98.6 / 118 / 135
-//   1024 x 1024         34.0 / 40.0 / 30.6   42.6 / 49.0 / 40.3   46.2 / 60.2 / 62.9   90.9 / 95.2 / 107
-//   1024 x 2521         46.2 / 49.4 / 62.8   65.0 / 69.2 / 66.6   98.2 / 98.7 / 114    193 / 198 / 230
+//    256 x  521         19.5 / 27.4 / 21.6   23.4 / 30.6 / 25.0   26.4 / 37.8 / 32.2   27.5 / 42.4 / 38.6
+//    256 x 2521         27.2 / 34.8 / 61.9   33.4 / 41.3 / 64.6   41.2 / 56.8 / 67.0   62.3 / 98.2 / 87.1
+//    512 x  521         22.8 / 27.3 / 21.9   26.3 / 31.0 / 25.1   26.9 / 37.7 / 34.2   30.1 / 44.0 / 49.1
+//    512 x 1024         28.3 / 35.4 / 29.5   34.0 / 44.9 / 37.8   42.6 / 51.3 / 46.0   45.9 / 60.0 / 67.9
+//    512 x 2521         35.0 / 38.0 / 62.0   42.4 / 47.4 / 64.9   62.5 / 74.6 / 70.1   97.1 / 114 / 135
+//   1024 x 1024         35.1 / 38.2 / 30.6   42.0 / 46.5 / 40.3   46.2 / 56.2 / 62.9   88.8 / 92.6 / 107
+//   1024 x 2521         45.2 / 45.0 / 62.8   62.1 / 66.3 / 66.6   97.3 / 97.2 / 114    190 / 195 / 230
 //   D=64
-//    256 x  521         14.1 / 18.9 / 15.4   15.6 / 20.3 / 17.0   18.6 / 24.4 / 21.0   19.2 / 31.4 / 28.4
-//    512 x 1024         18.7 / 26.1 / 21.6   22.3 / 29.9 / 25.5   29.7 / 37.3 / 33.0   31.4 / 45.1 / 47.8
-//   1024 x 1024         24.3 / 26.5 / 21.8   30.4 / 30.7 / 26.1   31.8 / 39.4 / 41.5   49.6 / 58.4 / 61.7
-//   1024 x 2521         33.4 / 42.1 / 42.7   48.5 / 47.5 / 51.8   66.7 / 67.7 / 72.7   108 / 117 / 124
-// (8-bit codes within 7 % of these, D=128 32 pairs 1024 x 2521 64.5 / 70.5 / 63.2.)
+//    256 x  521         12.9 / 18.4 / 15.4   14.9 / 19.8 / 17.0   17.8 / 22.9 / 21.0   18.2 / 31.2 / 28.4
+//    512 x 1024         17.7 / 25.6 / 21.6   21.8 / 28.5 / 25.5   28.6 / 35.6 / 33.0   30.2 / 45.1 / 47.8
+//   1024 x 1024         23.5 / 25.5 / 21.8   28.4 / 28.9 / 26.1   30.4 / 37.7 / 41.5   48.9 / 58.9 / 61.7
+//   1024 x 2521         32.1 / 37.5 / 42.7   47.5 / 45.8 / 51.8   63.6 / 67.8 / 72.7   111 / 118 / 124
+// (8-bit codes within 7 % of these.)
 bool wide_four(int64_t bh, int Lq, int Lk, int D, int cus, bool limits) {
   return limits && Lk <= Lq && Lq > 192 && bh * 26 >= cus && bh * 8 <= cus && bh * ((Lq + 127) / 128) * 4 <= (D == 128 ? 7 : 10) * (int64_t)cus;
 }
