@@ -306,7 +306,9 @@ int varq_quant_step_dequant(const void *x, int x_dtype, int B, int H, int n, int
  *              up to 8 workgroups; their partial results (fp32) pass through the
  *              workspace and a second kernel combines them.  splits = 0: the library
  *              decides, and uses no more shares than the workspace holds (none
- *              without a workspace) -- with at most 16 queries, and up to 128 where the cache is
+ *              without a workspace), and where that is the better way shares the keys out over
+ *              the wavefronts of a workgroup as well, with or without a workspace (with key limits also
+ *              for splits = 1) -- with at most 16 queries, and up to 128 where the cache is
  *              long enough for them, it takes a kernel of its own (at most two scale groups per key;
  *              the default operand form), whose wavefronts all serve the same queries on different
  *              keys, with up to 64 shares; 1: never; 2..8: exactly that many (an error if

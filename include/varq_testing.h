@@ -1,5 +1,5 @@
 /*
- * varq_testing.h -- entry points of libvarq_hip.so that its tests need to reach and to recognise paths of varq_quant_pack.  They are not part
+ * varq_testing.h -- entry points of libvarq_hip.so that its tests need to reach and to recognise paths of varq_quant_pack and of the attention.  They are not part
  * of the interface and may change with any build; the conventions are those of varq.h.
  */
 #ifndef VARQ_TESTING_H
@@ -24,6 +24,12 @@ int varq_quant_pack_wait(const void *x, int x_dtype, const int64_t *host_shape4,
  * block of groups; 1: one workgroup takes each by itself; 0: neither, the input is read twice.  word_bits: bits of the packed codes, 8 for int8 codes.
  */
 int varq_quant_pack_shards(const int64_t *host_shape4, int reduce_mask, int x_dtype, int tensors, int word_bits, int asym);
+
+/*
+ * Over how many wavefronts of a workgroup the attention shares the keys of its queries out on the current device when that is left to it (splits = 0) and
+ * the kernel that widens per workgroup serves the call: 1, 2 or 4; 0: with these key limits K and V are expanded instead. limits: whether there are key limits.
+ */
+int varq_fused_attn_key_waves(int B, int Hkv, int Lq, int Lk, int D, int limits);
 
 #ifdef __cplusplus
 }

@@ -44,6 +44,7 @@ struct AttnParams {
   int k_shift, v_shift;   // log2 of the channels per scale group (fused_attn.hip)
   int f16;   // q, out and the MFMA operands are fp16 (host side only: it selects the instantiation)
   int fq_share_blocks;   // few-queries kernel: 32-key blocks per share of the keys
+  int key_waves;         // fused_attn.hip: wavefronts that share a block of 32 queries, 1, 2 or 4 (host side only)
   int few_waves;         // ... and wavefronts of a workgroup, 4 or 8 (host side only)
   // memory layout, in rows (a row = the D values of one token of one head):
   // q row = b*q_bs + h*q_hs + i*q_ts, out row likewise with o_*, key row = b*kv_bs + slot*kv_hs + j*kv_ts.

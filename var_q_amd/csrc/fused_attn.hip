@@ -18,6 +18,8 @@
 //    16-bit values, which are the MFMA A operands of the first product; those of the second, which runs over keys, are read
 //    from the rows of V with the transposing LDS read.  The tiles are double-buffered, with one workgroup barrier per tile; at head
 //    dim 64 there is also an instantiation with one buffer, for launches of many small workgroups (launch_d64).
+//  * Launches that leave compute units idle have workgroups of 128 or 64 queries, the same eight wavefronts, two or four of which
+//    share the keys of their queries and put their outputs together in LDS at the end (KS, choose_shares).
 //  * Key rows are fed to the first MFMA in a permuted order chosen so that each
 //    lane's accumulator registers hold 8 consecutive keys per 16-key chunk, which is the order of the V^T operand.
 //  * Online softmax in the log2 domain against a reference that is only moved when a logit
@@ -46,9 +48,11 @@
 //      of quantization steps) or with a fractional part are split zp = zp_c + zp_r; the remainder
 //      goes through an fp32 correction term on tiles that have one.
 #include <algorithm>
+#include <cmath>
 #include <type_traits>
 
 #include "attn_common.h"
+#include "../../include/varq_testing.h"
 
 using namespace varq_attn;
 
@@ -717,38 +721,46 @@ template <int BITS> struct Widen {
 // rows each, at D=128 16 banks apart (4 banks apart, as K's, they got in one another's way); at D=64 they are 4 apart too, where 16 measured the same.
 template <int D> constexpr int kKRow = D + 8;
 template <int D> constexpr int kVRow = D + (D == 128 ? 32 : 8);
-template <int D> constexpr int kKBuf = BN * kKRow<D>;   // a tile (elements)
-template <int D> constexpr int kVBuf = BN * kVRow<D>;
+template <int D, int TB = BN> constexpr int kKBuf = TB * kKRow<D>;   // a tile of TB keys (elements)
+template <int D, int TB = BN> constexpr int kVBuf = TB * kVRow<D>;
 // LDS of the kernel (bytes).  ONE: one buffer instead of two, so that more workgroups are resident; a tile is widened and
 // attended before the next one is widened (see launch_d64 for when that is the better way).
-template <int D, bool ONE> struct TileLds {
+// KS: wavefronts that share a block of 32 queries, each with a block of 32 keys of every tile (of 64 keys, 128 with four of them).  Where a launch has fewer
+// workgroups than the device has compute units the chain through a tile is what it takes, and with half the work of a tile in each of twice the workgroups, which all
+// widen it, that chain is two thirds as long (D=128 2.1 us a tile of 64 keys alone, 1.35 with two, 0.95 with four; D=64 1.4, 0.85, 0.55): see choose_shares.
+template <int KS> constexpr int kTileKeys = KS <= 2 ? BN : KS * 32;
+template <int D, bool ONE, int KS = 1> struct TileLds {
   static constexpr int kBufs = ONE ? 1 : 2;
-  static constexpr int kTables = kBufs * (kKBuf<D> + kVBuf<D>) * 2;   // behind K's and V's buffers: the per-channel tables of the launch
+  static constexpr int kTables = kBufs * (kKBuf<D, kTileKeys<KS>> + kVBuf<D, kTileKeys<KS>>) * 2;   // behind K's and V's buffers: the per-channel tables of the launch
+  // ... and, in the place of all of them when the last tile is attended, what the wavefronts of a block of queries tell one another (see join_shares)
+  static constexpr int kStats = 8 * 32 * 8, kJoin = KS == 1 ? 0 : kStats + 8 / KS * (KS - 1) * (D / 8) * 1024;
 };
 
 // CHAN: scales and zero-points per (head, channel) instead of per (key, channel group), in up to 16 tables that change along the
 // keys (a cache quantized step by step has one per step): K[l,d] = (code[l,d] - zk_s[d]) * sk_s[d] with s the segment of key l, and
 // likewise V.  The tables of the head sit in LDS; a tile inside one segment reads that segment's rows, a tile that
 // straddles segments looks the segment up per key.
+// KS: see TileLds.
 // F16: q, out and the MFMA operands are fp16 instead of bf16 (dequantized K and V are rounded to fp16, as the reference's fp16
 // attention call sees them: VAR/models/basic_var.py:157-158 under the fp16 autocast of scripts/inference_multi_VAR.py:123).
 // One workgroup's work: query tile qt of packed pair bh (= batch * p.Hkv + packed head), share `split` of its
 // keys; partial results go to the rows of pair `out_pair`.
-template <int D, int BITS, bool CHAN, int NWV, bool F16, bool ONE = false>
+template <int D, int BITS, bool CHAN, int NWV, bool F16, bool ONE = false, int KS = 1>
 __device__ __forceinline__ void attend_tiles(const AttnParams &p, int bh, int out_pair, int qt, int split) {
-  constexpr int NT = NWV * 64, BM = NWV * 32;
+  constexpr int NT = NWV * 64, BM = NWV / KS * 32, TB = kTileKeys<KS>;
   constexpr int WPR = D * BITS / 32;        // packed words per key row
   constexpr int NCH = D / 16;               // contraction chunks of QK^T
   constexpr int NDB = D / 32;               // 32-row blocks of O^T
   constexpr int CH = D / 8, OCT = CH / 8;   // channels and octets of a thread's piece of a row
   constexpr int PB = CH * BITS / 8, PW = PB < 4 ? 1 : PB / 4;   // bytes and words of it
-  constexpr int IT = BN * 8 / NT;           // pieces of a tile per thread
-  using L = TileLds<D, ONE>;
-  constexpr int KS = kKRow<D>, VS = kVRow<D>;
+  constexpr int IT = TB * 8 / NT;           // pieces of a tile per thread
+  constexpr int KBUF = kKBuf<D, TB>, VBUF = kVBuf<D, TB>;
+  using L = TileLds<D, ONE, KS>;
+  constexpr int KR = kKRow<D>, VR = kVRow<D>;
   constexpr float kUnit = Widen<BITS>::kUnit;
   extern __shared__ __attribute__((aligned(16))) unsigned char lds_raw[];
-  uint16_t *const lds_k = reinterpret_cast<uint16_t *>(lds_raw);   // [kBufs][BN][KS]
-  uint16_t *const lds_v = lds_k + L::kBufs * kKBuf<D>;             // [kBufs][BN][VS]
+  uint16_t *const lds_k = reinterpret_cast<uint16_t *>(lds_raw);   // [kBufs][TB][KR]
+  uint16_t *const lds_v = lds_k + L::kBufs * KBUF;                 // [kBufs][TB][VR]
   float *const lds_tab = reinterpret_cast<float *>(lds_raw + L::kTables);   // [nseg][2 or 4][D]: scales of K and V times kUnit, zero-points over kUnit
   const bool has_zp = p.k_chan_zp || p.v_chan_zp;
   const int tab_rows = has_zp ? 4 : 2;
@@ -757,24 +769,25 @@ __device__ __forceinline__ void attend_tiles(const AttnParams &p, int bh, int ou
   const int hq = p.head_map ? p.head_map[hs] : hs;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int col = lane & 31, half = lane >> 5;
+  const int qwave = wave % (NWV / KS), share = wave / (NWV / KS);   // the wavefront's block of queries, and of keys of a tile
 
   // ---- this lane's query ----------------------------------------------------
-  const int qrow = qt * BM + wave * 32 + col;
+  const int qrow = qt * BM + qwave * 32 + col;
   const bool q_live = qrow < p.Lq;
-  const bool wave_live = qt * BM + wave * 32 < p.Lq;   // wave-uniform
+  const bool wave_live = qt * BM + qwave * 32 < p.Lq;   // wave-uniform
   const int qrow_c = q_live ? qrow : p.Lq - 1;
   const __bf16 *const qptr = p.q + (b * p.q_bs + hq * p.q_hs + qrow_c * p.q_ts) * D + half * 8;
   const int limit = p.kv_limit ? max(min(p.kv_limit[qrow_c], p.Lk), 0) : p.Lk;
 
   // ---- tile range: every lane of the workgroup runs the same number of tiles ----
   const int kv_end = p.kv_limit ? block_limit<BM>(p.kv_limit, qt * BM, p.Lq, p.Lk) : p.Lk;   // without limits every query sees all keys
-  int n_tiles = (kv_end + BN - 1) / BN, tbase = 0;   // tbase: this workgroup's first tile in the block's tile sequence
+  int n_tiles = (kv_end + TB - 1) / TB, tbase = 0;   // tbase: this workgroup's first tile in the block's tile sequence
   if (p.nsplit > 1) {
     const int t_begin = n_tiles * split / p.nsplit, t_end = n_tiles * (split + 1) / p.nsplit;
     tbase = t_begin;
     n_tiles = t_end - t_begin;
   }
-  const int tile_base = tbase * BN;   // first key of this workgroup's tiles
+  const int tile_base = tbase * TB;   // first key of this workgroup's tiles
   // the keys that every query of this wavefront sees, and those that some query sees
   int wave_minlim = p.Lk, wave_end = kv_end;
   if (p.kv_limit) {   // (the two halves of the wavefront hold the same queries)
@@ -853,7 +866,7 @@ __device__ __forceinline__ void attend_tiles(const AttnParams &p, int bh, int ou
       }
       asm volatile("");   // (or the compiler makes the loads of both ways one, with 64 bits of an offset)
     }
-    w_tile += BN * word_row; ks_tile += BN * ks_row; vs_tile += BN * vs_row; last -= BN;
+    w_tile += TB * word_row; ks_tile += TB * ks_row; vs_tile += TB * vs_row; last -= TB;
   };
 
   // CHAN: segment of the first key of the next tile to be widened, and where that segment ends
@@ -861,15 +874,15 @@ __device__ __forceinline__ void attend_tiles(const AttnParams &p, int bh, int ou
   int wseg = 0, wseg_end = p.Lk;
   // the requested tile -> rows of K and V
   auto widen = [&](int tile) {
-    uint16_t *const kx = lds_k + tile % L::kBufs * kKBuf<D>, *const vx = lds_v + tile % L::kBufs * kVBuf<D>;
+    uint16_t *const kx = lds_k + tile % L::kBufs * KBUF, *const vx = lds_v + tile % L::kBufs * VBUF;
     bool one_seg = true;
     if constexpr (CHAN) {
-      const int t0w = tile_base + tile * BN;
+      const int t0w = tile_base + tile * TB;
       while (wseg + 1 < p.nseg && t0w >= wseg_end) {
         ++wseg;
         wseg_end = __builtin_amdgcn_readfirstlane(lds_seg_end[wseg]);
       }
-      one_seg = wseg + 1 >= p.nseg || t0w + BN <= wseg_end;
+      one_seg = wseg + 1 >= p.nseg || t0w + TB <= wseg_end;
     }
     auto put = [&](auto zp_tag) __attribute__((always_inline)) {
       constexpr bool ZP = decltype(zp_tag)::value;
@@ -880,7 +893,7 @@ __device__ __forceinline__ void attend_tiles(const AttnParams &p, int bh, int ou
         if constexpr (CHAN) {
           int sg = wseg;
           if (!one_seg) {
-            const int k = min(tile_base + tile * BN + key, p.Lk - 1);
+            const int k = min(tile_base + tile * TB + key, p.Lk - 1);
             while (sg + 1 < p.nseg && k >= lds_seg_end[sg]) ++sg;
           }
           tab += sg * (tab_rows * D) + part * CH;
@@ -910,8 +923,8 @@ __device__ __forceinline__ void attend_tiles(const AttnParams &p, int bh, int ou
             *reinterpret_cast<u32x4_t *>(dst + o * 8) = r;
           }
         };
-        rows(next[i].k, next[i].ks, k_has_zp ? next[i].kz : 0.f, 0, kx + key * KS + part * CH);
-        rows(next[i].v, next[i].vs, v_has_zp ? next[i].vz : 0.f, 1, vx + key * VS + part * CH);
+        rows(next[i].k, next[i].ks, k_has_zp ? next[i].kz : 0.f, 0, kx + key * KR + part * CH);
+        rows(next[i].v, next[i].vs, v_has_zp ? next[i].vz : 0.f, 1, vx + key * VR + part * CH);
       }
     };
     if constexpr (CHAN) {
@@ -987,15 +1000,15 @@ __device__ __forceinline__ void attend_tiles(const AttnParams &p, int bh, int ou
   const uint16_t *kx = nullptr, *vx = nullptr;
   // V^T operand of block kb, chunk c, rows d: the lane's 8 keys of channel d * 32 + col, four of them by each read (16 lanes read 4 keys x 16
   // channels, 8 bytes each, and are handed a channel's four keys)
-  const uint16_t *const v_lane = lds_v + (half * 8 + (lane & 15) / 4) * VS + (lane & 16) + (lane & 3) * 4;
+  const uint16_t *const v_lane = lds_v + (half * 8 + (lane & 15) / 4) * VR + (lane & 16) + (lane & 3) * 4;
   typedef short s16x4_t __attribute__((ext_vector_type(4)));
   typedef __attribute__((address_space(3))) s16x4_t *lds_s16x4;
   auto load_v_operands = [&](int kb, int c) {
 #pragma unroll
     for (int d = 0; d < NDB; ++d) {
-      const uint16_t *at = vx + (kb * 32 + c * 16) * VS + d * 32;
+      const uint16_t *at = vx + (kb * 32 + c * 16) * VR + d * 32;
       const uint2 lo = __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4)(at)));
-      const uint2 hi = __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4)(at + 4 * VS)));
+      const uint2 hi = __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4)(at + 4 * VR)));
       vta[d] = u32x4_t{lo.x, lo.y, hi.x, hi.y};
     }
   };
@@ -1003,7 +1016,7 @@ __device__ __forceinline__ void attend_tiles(const AttnParams &p, int bh, int ou
     if constexpr (MFMA_PRIO) __builtin_amdgcn_s_setprio(1);
 #pragma unroll
     for (int j = 0; j < 16; ++j) sacc[j] = 0.f;
-    const uint16_t *const krow = kx + (kb * 32 + kperm(col)) * KS + half * 8;
+    const uint16_t *const krow = kx + (kb * 32 + kperm(col)) * KR + half * 8;
 #pragma unroll
     for (int ch = 0; ch < NCH; ++ch) sacc = mfma_32x32x16<F16>(*reinterpret_cast<const u32x4_t *>(krow + ch * 16), qb[ch], sacc);
     if constexpr (MFMA_PRIO) __builtin_amdgcn_s_setprio(0);
@@ -1015,7 +1028,7 @@ __device__ __forceinline__ void attend_tiles(const AttnParams &p, int bh, int ou
 #pragma unroll
     for (int i = 0; i < 16; ++i) z[i] = __builtin_fmaf(p.scale_log2e, sacc[i], -m_ref);
     // mask: block-causal key limit and the ragged last tile (register i of this lane <-> key kb*32 + 16*(i/8) + 8*half + i%8 of the tile)
-    if (t0 + BN > wave_minlim) {
+    if (t0 + (KS == 1 ? BN : kb * 32 + 32) > wave_minlim) {
 #pragma unroll
       for (int i = 0; i < 16; ++i) {
         const int key = t0 + kb * 32 + 16 * (i >> 3) + 8 * half + (i & 7);
@@ -1105,7 +1118,8 @@ __device__ __forceinline__ void attend_tiles(const AttnParams &p, int bh, int ou
   // would be exp2(-inf) = 0): the end of the cache and, under a key limit, whatever the workgroup's other
   // wavefronts still need.  A whole sequence of 680 tokens in ten steps, [8,680,16,64] fp16: a quarter of
   // the workgroups' key blocks; with the order of the query tiles (BlockOf) append and attention 47.5 -> 39.7 us.
-  const int wave_tiles = __builtin_amdgcn_readfirstlane(wave_live ? min(n_tiles, (max(wave_end - tile_base, 0) + BN - 1) / BN) : 0);
+  const int block0 = KS == 1 ? 0 : __builtin_amdgcn_readfirstlane(share * 32);   // the first key of a tile that the wavefront attends
+  const int wave_tiles = __builtin_amdgcn_readfirstlane(wave_live ? min(n_tiles, (max(wave_end - tile_base - block0, 0) + TB - 1) / TB) : 0);
   // with the MFMAs of a block in flight: the next tile is widened into the other buffers
   auto widen_next = [&](int tile) {
     if (tile + 1 >= n_tiles) return;
@@ -1113,12 +1127,12 @@ __device__ __forceinline__ void attend_tiles(const AttnParams &p, int bh, int ou
     if (tile + 2 < n_tiles) request();
   };
   auto attend = [&](int tile) {
-    t0 = tile_base + tile * BN;
-    kx = lds_k + tile % L::kBufs * kKBuf<D>;
-    vx = v_lane + tile % L::kBufs * kVBuf<D>;
+    t0 = tile_base + tile * TB + block0;
+    kx = lds_k + tile % L::kBufs * KBUF + block0 * KR;
+    vx = v_lane + tile % L::kBufs * VBUF + block0 * VR;
     const bool half_tile = wave_end - t0 <= 32;
 #pragma unroll
-    for (int kb = 0; kb < 2; ++kb) {
+    for (int kb = 0; kb < (KS == 1 ? 2 : 1); ++kb) {
       if (kb == 1 && half_tile) continue;
       qk(kb);
       load_v_operands(kb, 0);   // used after the softmax arithmetic
@@ -1150,52 +1164,129 @@ __device__ __forceinline__ void attend_tiles(const AttnParams &p, int bh, int ou
       __syncthreads();
     }
   }
-  if (!wave_live) return;
-
   // ---- epilogue -------------------------------------------------------------------
-  const float l_sum = l_part + __shfl_xor(l_part, 32, 64);
-  store_block<D, F16>(p, b, hq, qrow, q_live, half, split, out_pair, m_ref, l_sum, oacc, [](float o) { return o; });
+  if constexpr (KS == 1) {
+    if (!wave_live) return;
+    const float l_sum = l_part + __shfl_xor(l_part, 32, 64);
+    store_block<D, F16>(p, b, hq, qrow, q_live, half, split, out_pair, m_ref, l_sum, oacc, [](float o) { return o; });
+  } else {
+    // The wavefronts of a block of queries: each hands the others the quads of rows of O^T (four registers, u-th of D / 8) that those put together, weighted
+    // by the softmax mass against the largest reference of all (none where it saw no key; a NaN counts, and makes the result one).
+    constexpr int OWN = D / 8 / KS;
+    if constexpr (ONE) __syncthreads();   // (every tile is attended)
+    float2 *const stats = reinterpret_cast<float2 *>(lds_raw);                       // [NWV / KS][KS][32]
+    float4 *const handed = reinterpret_cast<float4 *>(lds_raw + L::kStats);          // [NWV / KS][to: KS][from: KS - 1][OWN][64]
+    const float l_own = l_part + __shfl_xor(l_part, 32, 64);
+    if (half == 0) stats[(qwave * KS + share) * 32 + col] = make_float2(m_ref, l_own);
+    __syncthreads();
+    float M = -INFINITY, l_sum = 0.f, w_own = 0.f;
+    float2 of[KS];
+#pragma unroll
+    for (int i = 0; i < KS; ++i) {
+      of[i] = stats[(qwave * KS + i) * 32 + col];
+      if (of[i].y != 0.f) M = fmaxf(M, of[i].x);
+    }
+#pragma unroll
+    for (int i = 0; i < KS; ++i) {
+      const float w = of[i].y != 0.f ? __builtin_amdgcn_exp2f(of[i].x - M) : 0.f;
+      l_sum = __builtin_fmaf(w, of[i].y, l_sum);
+      if (i == share) w_own = w;
+    }
+    if (wave_live) {
+#pragma unroll
+      for (int to = 0; to < KS; ++to) {
+        if (to == share) continue;
+        float4 *const dst = handed + ((qwave * KS + to) * (KS - 1) + (share < to ? share : share - 1)) * OWN * 64 + lane;
+#pragma unroll
+        for (int u = 0; u < OWN; ++u) {
+          const int r = to * OWN + u;
+          dst[u * 64] = make_float4(oacc[r / 4][r % 4 * 4] * w_own, oacc[r / 4][r % 4 * 4 + 1] * w_own, oacc[r / 4][r % 4 * 4 + 2] * w_own, oacc[r / 4][r % 4 * 4 + 3] * w_own);
+        }
+      }
+    }
+    __syncthreads();
+    if (!q_live) return;
+    const float inv = l_sum > 0.f ? 1.0f / l_sum : 0.f;
+    const bool shared_out = p.nsplit > 1;
+    __bf16 *const optr = p.out + (b * p.o_bs + hq * p.o_hs + qrow * p.o_ts) * D;
+    const int64_t prow = ((int64_t)split * p.bh_total + out_pair) * p.Lq + qrow;
+    float *const wptr = p.ws_o + prow * D;
+    if (shared_out && half == 0 && share == 0) *reinterpret_cast<float2 *>(p.ws_ml + prow * 2) = make_float2(M == -INFINITY ? 0.f : M, l_sum);
+#pragma unroll
+    for (int to = 0; to < KS; ++to) {   // (registers are named at compile time)
+      if (to != share) continue;
+      const float4 *const src = handed + (qwave * KS + to) * (KS - 1) * OWN * 64 + lane;
+#pragma unroll
+      for (int u = 0; u < OWN; ++u) {
+        const int r = to * OWN + u;
+        float4 o = make_float4(oacc[r / 4][r % 4 * 4] * w_own, oacc[r / 4][r % 4 * 4 + 1] * w_own, oacc[r / 4][r % 4 * 4 + 2] * w_own, oacc[r / 4][r % 4 * 4 + 3] * w_own);
+#pragma unroll
+        for (int from = 0; from < KS - 1; ++from) {
+          const float4 x = src[(from * OWN + u) * 64];
+          o.x += x.x; o.y += x.y; o.z += x.z; o.w += x.w;
+        }
+        o.x *= inv; o.y *= inv; o.z *= inv; o.w *= inv;
+        const int at = r / 4 * 32 + 8 * (r % 4) + 4 * half;
+        if (shared_out) *reinterpret_cast<float4 *>(wptr + at) = o;
+        else *reinterpret_cast<uint2 *>(optr + at) = make_uint2(pack_io_rne<F16>(o.x, o.y), pack_io_rne<F16>(o.z, o.w));
+      }
+    }
+  }
 }
 
 // Workgroup -> (pair, query tile, share of the keys).  XCD-aware: consecutive workgroup ids go to different
-// XCDs (8 of them), so ids congruent mod 8 share an L2.  All query tiles of one (batch, head) are given ids
-// of one residue class to keep its packed K/V in that XCD's L2.
+// XCDs (8 of them), so ids congruent mod 8 share an L2.  An XCD takes a run of the pairs' query tiles and shares, pair after pair, an eighth
+// of all: a pair's packed K/V stay in one L2 (or two), as do the cache lines that neighbouring heads of a token-major cache share.  (Whole pairs to an
+// XCD, as before, are one for six of them and none for two where there are six, and four for some where there are 25.)
+// Under key limits the tiles that see the most keys come first: in windows of an XCD's pairs (HeavyFirst), or with fewer than 64 pairs that are no
+// multiple of eight, which whole pairs would spread unevenly, over all pairs.
 struct BlockOf {
   int pair, qt, split;
   __device__ __forceinline__ explicit BlockOf(const AttnParams &p) {
-    const int xcd = blockIdx.x & 7, slot_s = blockIdx.x >> 3;
-    split = p.nsplit > 1 ? slot_s % p.nsplit : 0;
-    const int slot = p.nsplit > 1 ? slot_s / p.nsplit : slot_s;
-    // (a token-major cache: the key rows of neighbouring heads share cache lines, so an XCD takes a
-    // run of consecutive (batch, head) pairs there instead of every eighth)
-    const int groups = (p.bh_total + 7) >> 3;   // pairs of an XCD
-    int grp = slot / p.q_tiles;
-    qt = slot % p.q_tiles;
+    const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3;
     if (p.kv_limit && p.q_tiles > 1) {
+      if (spread_limits(p.bh_total)) {
+        const int unit = blockIdx.x / p.nsplit, back = unit / p.bh_total;
+        split = blockIdx.x - unit * p.nsplit;
+        pair = back < p.q_tiles ? unit - back * p.bh_total : p.bh_total;
+        qt = p.q_tiles - 1 - back;
+        return;
+      }
       // (windows of the pairs whose workgroups are resident together, 64 on an XCD at two per compute unit)
-      const HeavyFirst k(slot, p.q_tiles, groups, max(64 / p.q_tiles, 1));
+      const int groups = (p.bh_total + 7) >> 3, rest = slot / p.nsplit;   // pairs of an XCD
+      const HeavyFirst k(rest, p.q_tiles, groups, max(64 / p.q_tiles, 1));
+      split = slot - rest * p.nsplit;
       qt = k.qt;
-      grp = k.grp;
+      pair = p.kv_hs == 1 && p.kv_ts > 1 ? xcd * groups + k.grp : k.grp * 8 + xcd;
+      return;
     }
-    pair = p.kv_hs == 1 && p.kv_ts > 1 ? xcd * groups + grp : grp * 8 + xcd;
+    const int unit = xcd * ((p.bh_total * p.q_tiles * p.nsplit + 7) >> 3) + slot, tile = unit / p.nsplit;
+    split = unit - tile * p.nsplit;
+    pair = tile / p.q_tiles;
+    qt = tile - pair * p.q_tiles;
+  }
+  __host__ __device__ static bool spread_limits(int pairs) { return pairs < 64 && pairs % 8 != 0; }
+  static dim3 grid(const AttnParams &p) {
+    if (p.kv_limit && p.q_tiles > 1 && !spread_limits(p.bh_total)) return dim3((unsigned)((p.bh_total + 7) / 8 * 8 * p.q_tiles * p.nsplit));
+    return dim3((unsigned)(((int64_t)p.bh_total * p.q_tiles * p.nsplit + 7) / 8 * 8));
   }
 };
 
 // WPS: wavefronts per SIMD the register allocation aims at (2, or 4: two 8-wavefront workgroups
 // per compute unit at 128 registers, which the D=64 kernels afford)
-template <int D, int BITS, bool CHAN, int NWV, int WPS, bool F16, bool ONE>
+template <int D, int BITS, bool CHAN, int NWV, int WPS, bool F16, bool ONE, int KS>
 __global__ __launch_bounds__(NWV * 64, WPS) void fused_attn_kernel(AttnParams p) {
   const BlockOf k(p);
   if (k.pair >= p.bh_total) return;
-  attend_tiles<D, BITS, CHAN, NWV, F16, ONE>(p, k.pair, k.pair, k.qt, k.split);
+  attend_tiles<D, BITS, CHAN, NWV, F16, ONE, KS>(p, k.pair, k.pair, k.qt, k.split);
 }
 
-template <int D, int NWV, int WPS, bool F16>
+template <int D, int NWV, int WPS, bool F16, int KS>
 __global__ __launch_bounds__(NWV * 64, WPS) void fused_attn_classes_kernel(AttnParams p, ClassTable t) {
   const BlockOf k(p);
   if (k.pair >= p.bh_total) return;
   in_class(p, t, k.pair, [&](auto bits, int bh, int out_pair) __attribute__((always_inline)) {
-    attend_tiles<D, decltype(bits)::value, false, NWV, F16>(p, bh, out_pair, k.qt, k.split);
+    attend_tiles<D, decltype(bits)::value, false, NWV, F16, false, KS>(p, bh, out_pair, k.qt, k.split);
   });
 }
 
@@ -1335,28 +1426,30 @@ template <int D, bool F16> void launch_combine(const AttnParams &p, hipStream_t 
     hipLaunchKernelGGL((combine_splits_kernel<D, F16>), dim3((unsigned)((rows + 1) / 2)), dim3(256), 0, st, p);
 }
 
-dim3 tiles_grid(const AttnParams &p) { return dim3((unsigned)((p.bh_total + 7) / 8 * 8 * p.q_tiles * p.nsplit)); }
-template <int D, int BITS, bool CHAN, int NWV, int WPS = 2, bool F16 = false, bool ONE = false>
+template <int D, int BITS, bool CHAN, int NWV, int WPS = 2, bool F16 = false, bool ONE = false, int KS = 1>
 void launch_shape(const AttnParams &p, hipStream_t st) {
   // (the per-channel tables take LDS by the number of segments of the launch, and half of it without zero-points)
-  constexpr int lds_base = TileLds<D, ONE>::kTables, lds_max = lds_base + (CHAN ? kMaxSegments * 4 * D * 4 : 0);
+  using L = TileLds<D, ONE, KS>;
+  constexpr int lds_base = L::kTables, lds_max = std::max(lds_base + (CHAN ? kMaxSegments * 4 * D * 4 : 0), L::kJoin);
   static_assert(lds_max <= 160 * 1024, "LDS budget");
-  const int lds_bytes = lds_base + (CHAN ? p.nseg * (p.k_chan_zp || p.v_chan_zp ? 4 : 2) * D * 4 : 0);
+  const int lds_bytes = std::max(lds_base + (CHAN ? p.nseg * (p.k_chan_zp || p.v_chan_zp ? 4 : 2) * D * 4 : 0), L::kJoin);
   static bool configured[64] = {false};
-  allow_lds(reinterpret_cast<const void *>(&fused_attn_kernel<D, BITS, CHAN, NWV, WPS, F16, ONE>), lds_max, configured);
-  hipLaunchKernelGGL((fused_attn_kernel<D, BITS, CHAN, NWV, WPS, F16, ONE>), tiles_grid(p), dim3(NWV * 64), lds_bytes, st, p);
+  allow_lds(reinterpret_cast<const void *>(&fused_attn_kernel<D, BITS, CHAN, NWV, WPS, F16, ONE, KS>), lds_max, configured);
+  hipLaunchKernelGGL((fused_attn_kernel<D, BITS, CHAN, NWV, WPS, F16, ONE, KS>), BlockOf::grid(p), dim3(NWV * 64), lds_bytes, st, p);
   if (p.nsplit > 1) launch_combine<D, F16>(p, st);
 }
 template <int BITS> void launch_exact(const AttnParams &p, hipStream_t st) {
   constexpr int lds_bytes = ExactLds<BITS>::kBytes;
   static bool configured[64] = {false};
   allow_lds(reinterpret_cast<const void *>(&exact_attn_kernel<BITS>), lds_bytes, configured);
-  hipLaunchKernelGGL((exact_attn_kernel<BITS>), tiles_grid(p), dim3(NW * 64), lds_bytes, st, p);
+  hipLaunchKernelGGL((exact_attn_kernel<BITS>), BlockOf::grid(p), dim3(NW * 64), lds_bytes, st, p);
   if (p.nsplit > 1) launch_combine<128, false>(p, st);
 }
 
 // The workgroups at D=64, F16 or not.
 template <int BITS, bool CHAN, bool F16> void launch_d64(const AttnParams &p, hipStream_t st) {
+  if (p.key_waves == 2) return launch_shape<64, BITS, CHAN, 8, 4, F16, false, 2>(p, st);
+  if (p.key_waves == 4) return launch_shape<64, BITS, CHAN, 8, 4, F16, false, 4>(p, st);
   // More (batch, head) pairs than compute units, at most four wavefronts of queries each:
   // workgroups of four wavefronts (same arithmetic, same results).  Also for one or two
   // wavefronts of queries: the wavefronts without queries share the widening
@@ -1387,6 +1480,10 @@ template <int D, int BITS, bool CHAN> void launch(const AttnParams &p, hipStream
     // fp16 operands (the VAR path; every VAR model has head dim 64) or bf16 ones
     if (p.f16) launch_d64<BITS, CHAN, true>(p, st);
     else launch_d64<BITS, CHAN, false>(p, st);
+  } else if (p.key_waves == 2) {
+    launch_shape<D, BITS, CHAN, 8, 2, false, false, 2>(p, st);
+  } else if (p.key_waves == 4) {
+    launch_shape<D, BITS, CHAN, 8, 2, false, CHAN, 4>(p, st);
   } else {
     launch_shape<D, BITS, CHAN, 8>(p, st);
   }
@@ -1408,20 +1505,26 @@ bool groups_served(int D, int gk, int gv) {
   return ((gk == gv && (gk == 128 || gk == 64 || gk == 32)) || (gk == 32 && gv == 64)) && gk <= D;
 }
 
-template <int D, int NWV, int WPS, bool F16>
+template <int D, int NWV, int WPS, bool F16, int KS = 1>
 void launch_classes_shape(const AttnParams &p, const ClassTable &t, hipStream_t st) {
-  constexpr int lds = TileLds<D, false>::kTables;
+  constexpr int lds = std::max(TileLds<D, false, KS>::kTables, TileLds<D, false, KS>::kJoin);
   static bool configured[64] = {false};
-  allow_lds(reinterpret_cast<const void *>(&fused_attn_classes_kernel<D, NWV, WPS, F16>), lds, configured);
-  hipLaunchKernelGGL((fused_attn_classes_kernel<D, NWV, WPS, F16>), tiles_grid(p), dim3(NWV * 64), lds, st, p, t);
+  allow_lds(reinterpret_cast<const void *>(&fused_attn_classes_kernel<D, NWV, WPS, F16, KS>), lds, configured);
+  hipLaunchKernelGGL((fused_attn_classes_kernel<D, NWV, WPS, F16, KS>), BlockOf::grid(p), dim3(NWV * 64), lds, st, p, t);
   if (p.nsplit > 1) launch_combine<D, F16>(p, st);
 }
 // (the workgroup sizes by the rules of launch())
 template <int D> void launch_classes(const AttnParams &p, const ClassTable &t, hipStream_t st) {
   if constexpr (D == 64) {
     const bool four = p.Lq <= 128 && p.bh_total > device_cus();
+    if (p.key_waves == 2) { if (p.f16) launch_classes_shape<D, 8, 4, true, 2>(p, t, st); else launch_classes_shape<D, 8, 4, false, 2>(p, t, st); return; }
+    if (p.key_waves == 4) { if (p.f16) launch_classes_shape<D, 8, 4, true, 4>(p, t, st); else launch_classes_shape<D, 8, 4, false, 4>(p, t, st); return; }
     if (p.f16) { if (four) launch_classes_shape<D, 4, 3, true>(p, t, st); else launch_classes_shape<D, 8, 4, true>(p, t, st); }
     else { if (four) launch_classes_shape<D, 4, 3, false>(p, t, st); else launch_classes_shape<D, 8, 4, false>(p, t, st); }
+  } else if (p.key_waves == 2) {
+    launch_classes_shape<D, 8, 2, false, 2>(p, t, st);
+  } else if (p.key_waves == 4) {
+    launch_classes_shape<D, 8, 2, false, 4>(p, t, st);
   } else {
     launch_classes_shape<D, 8, 2, false>(p, t, st);
   }
@@ -1449,38 +1552,63 @@ size_t split_workspace_bytes(int splits, int64_t rows, int D) {
   return splits > 1 ? (size_t)splits * (size_t)rows * (size_t)(D + 2) * sizeof(float) : 0;
 }
 
-// The split count that minimizes a launch's modelled time: workgroups run one per compute
-// unit in rounds; a workgroup costs its tiles plus a fixed prologue and epilogue; shares
-// cost a second pass over fp32 partial outputs.  Few query blocks on a long cache gain,
-// a grid that already fills the device in whole rounds does not.
-int choose_splits(int64_t wgs, int tiles, int64_t rows, int D) {
-  const double cus = device_cus();
-  // (No sharing / what this chooses / the best of one to eight, us, 4 bits: D=64, 32 pairs, 256 x 521 17.3 / 14.8 / 14.8, 256 x 1500 38.2 / 19.9 / 18.5, 128 pairs, 256 x 1500
-  // 39.0 / 31.6 / 31.5, 1024 x 2521 110 / 111 / 110, 240 pairs, 256 x 1500 41.1 / 41.2 / 41.1; D=128, 16 pairs, 576 x 1497 56.1 / 32.2 / 32.1, 32 pairs, 256 x 521 25.5 / 22.8 / 21.5, 1024 x 2521
-  // 89.8 / 62.7 / 62.7, 128 pairs, 256 x 2521 90.4 / 62.5 / 62.4, 240 pairs 94.7 / 94.8 / 94.7; 8 bits with tables likewise.  Of 140 forms eight are 6 to 10 % behind the best, for instance few queries x many keys on a
-  // nearly full device, D=64, 128 pairs, 200 x 4096 97.4 / 59.2 / 54.2, 240 pairs 98.8 / 99.1 / 90.5, and D=128, 64 pairs, 512 x 1024 41.8 / 41.8 / 38.5.)
-  const double tile_us = D == 128 ? 2.3 : 1.4, fixed_us = D == 128 ? 9.0 : 6.0, bytes_us = D == 128 ? 4.0e6 : 5.0e6, gain = D == 128 ? 0.9 : 0.92;
-  double base = 0.0, best = 0.0;
-  int best_s = 1;
-  for (int s = 1; s <= kMaxSplits; ++s) {
-    if (s > 1 && tiles / s < 2) break;
-    const double rounds = (double)((wgs * s + (int64_t)cus - 1) / (int64_t)cus);
-    double t = rounds * ((double)((tiles + s - 1) / s) * tile_us + fixed_us);
-    if (s > 1) t += 4.0 + 2.0 * (double)split_workspace_bytes(s, rows, D) / bytes_us;   // written and read
-    if (s == 1) base = best = t;
-    else if (t < gain * base && t < best) { best = t; best_s = s; }   // sharing must gain a tenth or so
-  }
-  return best_s;
-}
+// How the keys of a block of 256 queries are shared out: over `splits` workgroups, whose partial results take a second launch, and with `waves` 2 or 4
+// over that many wavefronts of a workgroup, which then serves a half or a quarter of the queries and widens every tile for them alone.
+struct KeyShares { int waves, splits; };
 
-// Fills the split fields of p from the caller's request.  splits: 0 = as the model above
-// says, reduced to what the workspace holds; 1 = none; 2..8 = exactly that many.
-int set_splits(AttnParams &p, int D, int tiles, int splits, void *workspace, size_t workspace_bytes, const char *who) {
+// The shares that minimize a launch's modelled time: workgroups run one per compute unit in rounds, an eighth of them on each XCD (see
+// BlockOf); a workgroup costs its tiles (of 128 keys where four wavefronts share them) plus a fixed prologue and epilogue, and with shares of wavefronts their
+// joining.  Fitted to 386 random forms (6 to 960 pairs, 16 to 1100 queries, 17 to 4800 keys, groups and tables, 2, 4 and 8 bits), each with every choice: what this
+// takes is 0.5 % behind the best of all on the geometric mean and 9 % ahead of workgroups alone, and in 5 of them behind those by more than 2.5 %.  4 bits in groups,
+// us, workgroups alone / this: D=128, 32 pairs, 256 queries x 521 keys 22.6 / 16.5, 400 x 921 32.4 / 22.8, 64 pairs, 144 x 300 16.8 / 12.0, 256 x 521
+// 27.2 / 17.4, 400 x 921 40.9 / 30.5, 128 pairs, 256 x 521 28.6 / 22.8; D=64, 32 pairs, 256 x 521 15.7 / 11.6, 1024 x 2521 50.1 / 43.4, 128 pairs, 256 x 521 19.1 / 15.1.
+KeyShares choose_shares(int64_t bh, int Lq, int Lk, int D, int most_waves) {
+  static const double tile_us[2][3] = {{1.45, 0.85, 1.1}, {2.07, 1.35, 1.9}};
+  const double per_xcd = device_cus() / 8.0;
+  const bool wide = D == 128;
+  KeyShares best = {1, 1};
+  double best_us = 0.0;
+  for (int waves = 1, i = 0; waves <= most_waves; waves *= 2, ++i) {
+    // (a single tile has nothing to share; and what up to 128 queries, the first steps of a schedule, come to does not go by how many pairs a launch has,
+    // which would gain up to a tenth in tables: 64 queries x 600 keys, 128 pairs, D=64 15.9 / 13.5, D=128 20.8 / 18.7)
+    if (waves > 1 && (Lk <= BN || Lq <= 128)) break;
+    const int64_t tiles = (Lk + (waves == 4 ? 2 * BN : BN) - 1) / (waves == 4 ? 2 * BN : BN), blocks = bh * ((Lq + BM / waves - 1) / (BM / waves));
+    // (up to 128 queries half of the wavefronts have none, and widen only)
+    const double tile = tile_us[wide][i] * (waves == 1 && Lq <= 128 ? 0.7 : 1.0), fixed = (wide ? 2.8 : 2.2) + (waves > 1 ? 1.1 : 0.0);
+    for (int n = 1; n <= kMaxSplits; ++n) {
+      if (n > 1 && (Lk + BN - 1) / BN / n < 2) break;
+      double us = std::ceil((double)((blocks * n + 7) / 8) / per_xcd) * ((double)((tiles + n - 1) / n) * tile + fixed);
+      if (n > 1) us += 2.4 + 2.0 * (double)split_workspace_bytes(n, bh * Lq, D) / 4.4e6;   // written and read
+      if ((waves == 1 && n == 1) || us < best_us) { best_us = us; best = {waves, n}; }
+    }
+  }
+  return best;
+}
+// Fills the fields of the shares of p from the caller's request.  splits: 0 = as the model above
+// says, reduced to what the workspace holds; 1 = none; 2..8 = exactly that many.  limited: what limited_shares says, or null.
+int set_splits(AttnParams &p, int D, int most_waves, const KeyShares *limited, int splits, void *workspace, size_t workspace_bytes, const char *who) {
   p.nsplit = 1; p.ws_o = nullptr; p.ws_ml = nullptr;
+  p.key_waves = 1;
   if (splits < 0 || splits > kMaxSplits)
     return varq_set_error(VARQ_ERR_INVALID, "%s: splits must be 0 (automatic) or 1..%d (got %d)", who, kMaxSplits, splits);
   const int64_t rows = (int64_t)p.bh_total * p.Lq;
-  int n = splits ? splits : choose_splits((int64_t)p.bh_total * p.q_tiles, tiles, rows, D);
+  // (a workspace that cannot be used is an error wherever workgroups alone would use it)
+  if (splits == 0 && workspace && ((uintptr_t)workspace & 15) && workspace_bytes >= split_workspace_bytes(2, rows, D) && choose_shares(p.bh_total, p.Lq, p.Lk, D, 1).splits > 1)
+    return varq_set_error(VARQ_ERR_INVALID, "%s: the workspace must be 16-byte aligned", who);
+  int n = splits;
+  if (limited) {
+    p.key_waves = limited->waves;
+    n = limited->splits;
+  } else if (splits == 0) {
+    KeyShares k = choose_shares(p.bh_total, p.Lq, p.Lk, D, 1);
+    n = k.splits;
+    if (most_waves > 1) k = choose_shares(p.bh_total, p.Lq, p.Lk, D, most_waves);
+    if (k.waves > 1 && (k.splits == 1 || (workspace && workspace_bytes >= split_workspace_bytes(k.splits, rows, D)))) {
+      p.key_waves = k.waves;
+      n = k.splits;
+    }
+  }
+  p.q_tiles = (p.Lq + BM / p.key_waves - 1) / (BM / p.key_waves);
   if (splits > 1 && (!workspace || workspace_bytes < split_workspace_bytes(n, rows, D)))
     return varq_set_error(VARQ_ERR_INVALID, "%s: %d splits need a workspace of %zu bytes (got %zu)", who, n,
                           split_workspace_bytes(n, rows, D), workspace ? workspace_bytes : (size_t)0);
@@ -1589,6 +1717,42 @@ bool wide_eligible(int B, int Hkv, int Lq, int Lk, int D, bool limits) {
   if (limits && D == 64 && Lq < 6144 && blocks > device_cus() * 5 / 4) return false;
   return Lq >= (D == 128 ? 1280 : 1536) && Lk >= 2048 && blocks >= 160 && bh <= 65535;
 }
+// Under key limits, whose blocks end at different keys that only the device knows; taken for a sequence's own, of which a block sees a quarter
+// more than its share.  The time is that of the longest workgroup or of all of them evenly dealt out, and more where both are alike.  Shares of wavefronts also
+// with splits = 1 (most = 1).  waves 0: K and V are expanded instead.  Fitted to 452 forms (2 to 360 pairs, whole sequences of 129 to 6000 tokens) with
+// every choice: 1.2 % behind the best on the geometric mean, 18 % ahead of the rules before, blocks of 128 queries for few pairs (wide_four) and shares as without
+// limits.  4 bits in groups, us, before / this: D=64, 2 pairs x 4500 tokens 52.7 / 31, 16 x 300 12.4 / 9.0, x 680 17.6 / 12.4, x 1500 29.1 / 24.6, 32 x 524 17.2 / 12.9, 48 x 1000 27.3 / 23.0;
+// D=128, 2 x 4500 93 / 46, 16 x 680 24.8 / 17.3, 24 x 600 24.6 / 16.6, x 1000 33.9 / 28.9, 32 x 854 34.0 / 27.1, 90 x 249 16.7 / 13.7.
+KeyShares limited_shares(int B, int Hkv, int Lq, int Lk, int D, int most, bool may_expand) {
+  const int64_t bh = (int64_t)B * Hkv;
+  const bool four = may_expand && wide_four((int64_t)wide_batch(B, Hkv, Lk, D) * Hkv, Lq, Lk, D, device_cus(), true);
+  if (may_expand && !four && wide_eligible(B, Hkv, Lq, Lk, D, true)) return {0, 1};
+  if (Lq <= 128 || Lk <= 128) return {1, most == 1 ? 1 : choose_shares(bh, Lq, Lk, D, 1).splits};
+  struct Cost { double tile, fixed, again, load; };   // us of a tile, of a workgroup, of one that is not the longest; of the whole load
+  static const Cost cost[2][3] = {{{1.32, 5.8, 4.7, 0.9}, {0.87, 6.0, 4.9, 1.03}, {1.15, 5.6, 4.6, 1.03}}, {{2.1, 4.7, 3.8, 1.0}, {1.4, 6.6, 5.4, 1.14}, {1.9, 6.1, 5.0, 1.14}}};
+  static const Cost expanded[2] = {{0.9, 10.0, 4.0, 0.92}, {1.4, 14.0, 4.0, 0.95}};
+  auto us = [&](const Cost &c, int block, int keys, int n) {
+    const double blocks = (Lq + block - 1) / block, part = std::floor(0.8 * blocks), tiles = (double)Lk / keys * (1.25 * part * (part + 1.0) / (2.0 * blocks) + blocks - part) + 0.5 * blocks;
+    const double longest = c.fixed + c.tile * (((Lk + keys - 1) / keys + n - 1) / n), load = c.load * (double)bh * (blocks * n * c.again + tiles * c.tile) / device_cus();
+    const double two = longest * longest, four = load * load;
+    return std::sqrt(std::sqrt(two * two + four * four));
+  };
+  const int d = D == 128;
+  KeyShares best = {1, 1};
+  double best_us = us(cost[d][0], BM, BN, 1);
+  if (four) {
+    const double t = us(expanded[d], 128, BN, 1);
+    if (t < best_us) { best_us = t; best = {0, 1}; }
+  }
+  for (int i = 0; i < 3; ++i)
+    for (int n = 1; n <= most && (n == 1 || (Lk + BN - 1) / BN / n >= 2); ++n) {
+      double t = us(cost[d][i], BM >> i, i == 2 ? 2 * BN : BN, n) * (i ? 1.05 : 1.0);
+      if (n > 1) t += 2.8 + 2.0 * (double)split_workspace_bytes(n, bh * Lq, D) / 4.0e6;
+      if (t < best_us) { best_us = t; best = {1 << i, n}; }
+    }
+  return best;
+}
+constexpr int kLimitedSplits = 6;   // (more gain nothing)
 // The largest workspace of the parts that the call is done in.
 size_t wide_bytes(int B, int Hkv, int Lq, int Lk, int D, bool share, bool limits) {
   const int n = wide_batch(B, Hkv, Lk, D), last = B - (B - 1) / n * n;
@@ -1622,8 +1786,28 @@ void skip_entries(AttnParams &p, int first, int D, int bits, int k_groups, int v
   if (p.k_zp) p.k_zp += rows * k_groups;
   if (p.v_zp) p.v_zp += rows * v_groups;
 }
+// What limited_shares says of a call, if it is asked: once with the expansion, and again without where the workspace does not hold it.
+class Limited {
+  const AttnParams &p;
+  int B, D, most;   // most: 0 without limits, or where the caller says how the keys are shared out
+  KeyShares k = {0, 1};
+
+ public:
+  Limited(const AttnParams &p_, int B_, int D_, int splits) : p(p_), B(B_), D(D_), most(!p_.kv_limit || splits > 1 ? 0 : splits == 1 ? 1 : kLimitedSplits) {
+    if (most) k = limited_shares(B, p.Hkv, p.Lq, p.Lk, D, most, true);
+  }
+  bool expands() const { return k.waves == 0; }   // (or is not asked)
+  const KeyShares *shares() {
+    if (!most) return nullptr;
+    if (k.waves == 0) k = limited_shares(B, p.Hkv, p.Lq, p.Lk, D, most, false);
+    return &k;
+  }
+};
+
 size_t expand_bytes(int B, int Hkv, int Lq, int Lk, int D, bool limits) {
-  if (B <= 0 || Hkv <= 0 || Lq <= 0 || Lk <= 0 || (D != 64 && D != 128) || !wide_eligible(B, Hkv, Lq, Lk, D, limits)) return 0;
+  if (B <= 0 || Hkv <= 0 || Lq <= 0 || Lk <= 0 || (D != 64 && D != 128) || !wide_eligible(B, Hkv, Lq, Lk, D, limits) ||
+      (limits && limited_shares(B, Hkv, Lq, Lk, D, kLimitedSplits, true).waves))
+    return 0;
   return wide_bytes(B, Hkv, Lq, Lk, D, true, limits);
 }
 
@@ -1633,12 +1817,18 @@ extern "C" size_t varq_fused_attn_workspace_bytes(int B, int Hkv, int Lq, int Lk
   if (B <= 0 || Hkv <= 0 || Lq <= 0 || Lk <= 0 || (D != 64 && D != 128) || splits < 0 || splits > kMaxSplits) return 0;
   const int64_t rows = (int64_t)B * Hkv * Lq;
   (void)nseg;   // (the tile count does not depend on the tables)
-  const int tiles = (Lk + BN - 1) / BN;
-  int n = splits ? splits : choose_splits((int64_t)B * Hkv * ((Lq + BM - 1) / BM), tiles, rows, D);
+  const int64_t bh = (int64_t)B * Hkv;
+  // (whether there will be key limits is not known here)
+  int n = splits ? splits : std::max({choose_shares(bh, Lq, Lk, D, 4).splits, choose_shares(bh, Lq, Lk, D, 1).splits, limited_shares(B, Hkv, Lq, Lk, D, kLimitedSplits, false).splits});
   // (the group sizes are not known here: room for the few-queries kernel's shares whenever the
   // other sizes would admit it)
   if (splits == 0 && fewq_eligible(B, Hkv, Lq, Lk, D, D, D)) n = max(n, fewq_shares(B * Hkv, Lq, Lk, D, D, D));
   return split_workspace_bytes(n, rows, D);
+}
+
+extern "C" int varq_fused_attn_key_waves(int B, int Hkv, int Lq, int Lk, int D, int limits) {
+  if (B <= 0 || Hkv <= 0 || Lq <= 0 || Lk <= 0 || (D != 64 && D != 128)) return -1;
+  return limits ? limited_shares(B, Hkv, Lq, Lk, D, kLimitedSplits, true).waves : choose_shares((int64_t)B * Hkv, Lq, Lk, D, 4).waves;
 }
 
 extern "C" size_t varq_fused_attn_expand_bytes(int B, int Hkv, int Lq, int Lk, int D) {
@@ -1649,7 +1839,7 @@ extern "C" size_t varq_fused_attn_expand_bytes_limits(int B, int Hkv, int Lq, in
 extern "C" int varq_fused_attn_key_shares(int B, int Hkv, int Lq, int Lk, int D, int k_group, int v_group) {
   if (B <= 0 || Hkv <= 0 || Lq <= 0 || Lk <= 0 || (D != 64 && D != 128)) return 0;
   if (fewq_eligible(B, Hkv, Lq, Lk, D, k_group, v_group)) return fewq_shares(B * Hkv, Lq, Lk, D, k_group, v_group);
-  return choose_splits((int64_t)B * Hkv * ((Lq + BM - 1) / BM), (Lk + BN - 1) / BN, (int64_t)B * Hkv * Lq, D);
+  return choose_shares((int64_t)B * Hkv, Lq, Lk, D, 4).splits;
 }
 
 extern "C" int varq_fused_attn(const void *q, void *out,
@@ -1709,7 +1899,8 @@ extern "C" int varq_fused_attn(const void *q, void *out,
     VARQ_CHECK_LAUNCH("fused_attn");
     return VARQ_OK;
   }
-  if ((splits == 0 || splits == 1) && !p.exact_codes && groups_served(D, k_group, v_group) && wide_eligible(B, p.Hkv, Lq, Lk, D, kv_limit != nullptr) &&
+  Limited limited(p, B, D, exact_form ? 2 : splits);
+  if ((splits == 0 || splits == 1) && limited.expands() && !p.exact_codes && groups_served(D, k_group, v_group) && wide_eligible(B, p.Hkv, Lq, Lk, D, kv_limit != nullptr) &&
       run_wide(p, D, splits, workspace, workspace_bytes, st, [&](AttnParams c, int first, char *ws) {
         skip_entries(c, first, D, k_bits, D / k_group, D / v_group);
         launch_expand(c, D, k_bits, k_group, v_group, false, ws, st);
@@ -1717,7 +1908,7 @@ extern "C" int varq_fused_attn(const void *q, void *out,
     VARQ_CHECK_LAUNCH("fused_attn");
     return VARQ_OK;
   }
-  if (int e = set_splits(p, D, (Lk + BN - 1) / BN, splits, workspace, workspace_bytes, "fused_attn")) return e;
+  if (int e = set_splits(p, D, exact_form ? 1 : 4, limited.shares(), splits, workspace, workspace_bytes, "fused_attn")) return e;
   if (!groups_served(D, k_group, v_group))
     return varq_set_error(VARQ_ERR_UNSUPPORTED, "fused_attn: no kernel for D=%d bits=%d k_group=%d v_group=%d", D, k_bits,
                           k_group, v_group);
@@ -1791,7 +1982,8 @@ extern "C" int varq_fused_attn_channel(const void *q, void *out,
   p.exact_codes = 0;
   if (int e = set_layout(p, layout, "fused_attn_channel")) return e;
   hipStream_t st = (hipStream_t)stream;
-  if ((splits == 0 || splits == 1) && wide_eligible(B, p.Hkv, Lq, Lk, D, kv_limit != nullptr) &&
+  Limited limited(p, B, D, splits);
+  if ((splits == 0 || splits == 1) && limited.expands() && wide_eligible(B, p.Hkv, Lq, Lk, D, kv_limit != nullptr) &&
       run_wide(p, D, splits, workspace, workspace_bytes, st, [&](AttnParams c, int first, char *ws) {
         skip_entries(c, first, D, bits, 0, 0);
         launch_expand(c, D, bits, D, D, true, ws, st);
@@ -1799,7 +1991,7 @@ extern "C" int varq_fused_attn_channel(const void *q, void *out,
     VARQ_CHECK_LAUNCH("fused_attn_channel");
     return VARQ_OK;
   }
-  if (int e = set_splits(p, D, (Lk + BN - 1) / BN, splits, workspace, workspace_bytes, "fused_attn_channel"))
+  if (int e = set_splits(p, D, 4, limited.shares(), splits, workspace, workspace_bytes, "fused_attn_channel"))
     return e;
   launch_any<true>(p, D, bits, st);
   VARQ_CHECK_LAUNCH("fused_attn_channel");
@@ -1852,11 +2044,12 @@ extern "C" int varq_fused_attn_classes(const void *q, void *out, const varq_kv_c
   p.f16 = io_dtype == VARQ_F16;
   if (int e = set_layout(p, layout, "fused_attn_classes")) return e;
   hipStream_t st = (hipStream_t)stream;
+  Limited limited(p, B, D, splits);
   if (splits == 0 && fewq_eligible(B, H, Lq, Lk, D, group, group)) {
     set_few(p, D, group, group, workspace, workspace_bytes);
     launch_few_classes(p, D, t, group, st);
     combine_few(p, D, st);
-  } else if ((splits == 0 || splits == 1) && wide_eligible(B, p.Hkv, Lq, Lk, D, kv_limit != nullptr) &&
+  } else if ((splits == 0 || splits == 1) && limited.expands() && wide_eligible(B, p.Hkv, Lq, Lk, D, kv_limit != nullptr) &&
              run_wide(p, D, splits, workspace, workspace_bytes, st, [&](const AttnParams &part, int first, char *ws) {
                ClassTable of = t;   // the part's batch entries of every class
                int pairs = 0;
@@ -1874,7 +2067,7 @@ extern "C" int varq_fused_attn_classes(const void *q, void *out, const varq_kv_c
                launch_expand_classes(part, D, of, group, ws, st);
              })) {
   } else {
-    if (int e = set_splits(p, D, (Lk + BN - 1) / BN, splits, workspace, workspace_bytes, "fused_attn_classes")) return e;
+    if (int e = set_splits(p, D, 4, limited.shares(), splits, workspace, workspace_bytes, "fused_attn_classes")) return e;
     p.k_shift = p.v_shift = varq_log2_exact(group);
     if (D == 128) launch_classes<128>(p, t, st);
     else launch_classes<64>(p, t, st);

@@ -592,6 +592,7 @@ namespace varq_attn {
 // device is full: 680 tokens 22.3 / 26.9 / 23.1 and 33.3 / 41.4 / 41.4.  With fewer than ten pairs the shares of the keys do
 // better (8 pairs, widening / 128: D=64 1656 tokens 26.0 / 27.7, 2440 35.5 / 37.8; 10 pairs of 2440 43.8 / 39.0,
 // of 5064 127 / 106; D=128 44.5 / 40.9 at 1656, 178 / 185 at 5064), and 155 tokens are too few (11.3 / 15.0).
+// (The kernel that widens has since got shares of wavefronts, which are ahead of these blocks up to about 2000 tokens: limited_shares has the last word.)
 // Without limits, where the shares of the keys fill the device, a block of 128 gains at most a tenth, and only where it takes exactly the
 // device and the keys are few.  All launches, 4-bit codes, us, widening per workgroup with its shares / blocks of 256 / of 128 (the last
 // measured earlier and on another card than the others, by up to a tenth slower):
