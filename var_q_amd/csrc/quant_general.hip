@@ -48,22 +48,6 @@ __device__ __forceinline__ float dec_ord(u32 e) {
   return u2f((e & 0x80000000u) ? (e & 0x7fffffffu) : ~e);
 }
 
-// n / d for n < 2^31 by a product: with s = ceil(log2 d) - 1 and mul = floor(2^(32 + s) / d) + 1 the product is too large by
-// n e / (2^(32 + s) d) for some e <= d <= 2^(s + 1), less than 1 / d.  (d = 1: mul = 0 and `all` takes n itself.)  A division of the
-// compiler's is some twenty instructions, and the kernels below have two for every octet.
-struct FastDiv {
-  u32 mul, all;
-  int shift;
-  static FastDiv by(int64_t d) {   // (anything from 2^31 on divides to 0)
-    if (d <= 1) return {0u, 0xffffffffu, 0};
-    if (d >= (1ll << 31)) return {0u, 0u, 0};
-    int s = 0;
-    while ((2ll << s) < d) ++s;
-    return {(u32)((1ull << (32 + s)) / (unsigned long long)d + 1), 0u, s};
-  }
-  __device__ __forceinline__ u32 operator()(u32 n) const { return (__umulhi(n, mul) + (n & all)) >> shift; }
-};
-
 // Where the scale of group g goes when it is written once per token that it serves (and the zero-point like it): elements
 // (g / gi) go + (g % gi) ge + off + i + o * s_out, i < r_in, o < r_out.
 struct Spread {

@@ -138,6 +138,22 @@ template <> struct In8<VARQ_F16> {
   }
 };
 
+// n / d for n < 2^31 by a product: with s = ceil(log2 d) - 1 and mul = floor(2^(32 + s) / d) + 1 the product is too large by
+// n e / (2^(32 + s) d) for some e <= d <= 2^(s + 1), less than 1 / d.  (d = 1: mul = 0 and `all` takes n itself.)  A division of the
+// compiler's is some twenty instructions, and the kernels have one or two for every few elements.
+struct FastDiv {
+  u32 mul, all;
+  int shift;
+  static FastDiv by(int64_t d) {   // (anything from 2^31 on divides to 0)
+    if (d <= 1) return {0u, 0xffffffffu, 0};
+    if (d >= (1ll << 31)) return {0u, 0u, 0};
+    int s = 0;
+    while ((2ll << s) < d) ++s;
+    return {(u32)((1ull << (32 + s)) / (unsigned long long)d + 1), 0u, s};
+  }
+  __device__ __forceinline__ u32 operator()(u32 n) const { return (__umulhi(n, mul) + (n & all)) >> shift; }
+};
+
 // Raw 8-element loads (no conversion) so that a kernel can issue the next
 // tile's loads before converting the current one.  Streaming data: marked
 // non-temporal, it is read exactly once.
