@@ -186,6 +186,14 @@ int varq_quant_pack_spread_once(const void *x0, const void *x1, int x_dtype, con
                                 float eps, int32_t *words0, float *scale0, float *zp0, int32_t *words1, float *scale1, float *zp1,
                                 float *once_scale0, float *once_zp0, float *once_scale1, float *once_zp1,
                                 const int64_t *host_out_map, const int64_t *host_scale_map, void *stream);
+/*
+ * varq_quant_pack_spread_once with a workspace as of varq_quant_pack (for x1 twice the bytes): also tensors that varq_quant_pack quantizes in
+ * several launches, where the scales once per group are asked for.  VARQ_ERR_UNSUPPORTED, and nothing done, for shapes off its tiled kernels.
+ */
+int varq_quant_pack_spread_room(const void *x0, const void *x1, int x_dtype, const int64_t *host_shape4, int reduce_mask, int bits, int asym,
+                                float eps, int32_t *words0, float *scale0, float *zp0, int32_t *words1, float *scale1, float *zp1,
+                                float *once_scale0, float *once_zp0, float *once_scale1, float *once_zp1,
+                                const int64_t *host_out_map, const int64_t *host_scale_map, void *workspace, size_t workspace_bytes, void *stream);
 
 /*
  * varq_quant_pack for callers that cannot allocate device memory (code under HIP graph

@@ -32,6 +32,10 @@ SYMBOLS = {
                                             c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p,
                                             c_void_p, c_void_p, c_void_p, c_void_p,
                                             POINTER(c_int64), POINTER(c_int64), c_void_p]),
+    'varq_quant_pack_spread_room': (c_int, [c_void_p, c_void_p, c_int, POINTER(c_int64), c_int, c_int, c_int, c_float,
+                                            c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p,
+                                            c_void_p, c_void_p, c_void_p, c_void_p,
+                                            POINTER(c_int64), POINTER(c_int64), c_void_p, c_size_t, c_void_p]),
     'varq_quant_static_scratch_bytes': (c_size_t, []),
     'varq_quant_pack_static': (c_int, [c_void_p, c_int, POINTER(c_int64), c_int, c_int, c_int, c_float,
                                        c_void_p, c_void_p, c_void_p, c_void_p, POINTER(c_int64), c_void_p]),

@@ -922,8 +922,15 @@ PyObject *quantizer_step(PyObject *const *a) {
   const int rc = status_unlocked([&] {
     if (rows) return pack_rows(k, x1, dt, sh, mask, bits, asym, (float)eps, w0, w1, s, z, map);
     float *const s0 = own[0].data(), *const s1 = two ? own[1].data() : nullptr;
-    return varq_quant_pack_spread_once(k.data_ptr(), x1, dt, sh, mask, bits, asym, (float)eps, w0, s[0], z[0], w1, s[1], z[1], s0, asym ? s0 + own[0].half : nullptr, s1,
-                                       asym && two ? s1 + own[1].half : nullptr, map, spread, stream_of(k));
+    auto step = [&](void *ws, size_t ws_bytes) {
+      return varq_quant_pack_spread_room(k.data_ptr(), x1, dt, sh, mask, bits, asym, (float)eps, w0, s[0], z[0], w1, s[1], z[1], s0, asym ? s0 + own[0].half : nullptr, s1,
+                                         asym && two ? s1 + own[1].half : nullptr, map, spread, ws, ws_bytes, stream_of(k));
+    };
+    const int rc = step(nullptr, 0);   // (most steps take one launch, which needs none)
+    if (rc != VARQ_ERR_UNSUPPORTED) return rc;
+    const size_t ws_bytes = std::max<size_t>(varq_quant_workspace_bytes(sh, mask), 8) * (two ? 2 : 1);
+    const at::Tensor ws = empty({(int64_t)ws_bytes}, at::kByte, k);
+    return step(ws.data_ptr(), ws_bytes);
   });
   if (!rows && rc == VARQ_ERR_UNSUPPORTED) Py_RETURN_FALSE;
   check(rc, "varq_quant_pack");

@@ -97,6 +97,34 @@ __device__ __forceinline__ bool take_second(GenParams &p) {
   return true;
 }
 
+// The parameters of a workgroup's 2^shift groups, in LDS, to all their places, by all `NT` threads; group_of(t): the number of a group (or less
+// than 0: no such group).  Adjacent threads write adjacent places: those of a token, or of a row of a table, unless the groups' own are adjacent.
+// (G_TOKEN in layout BLHc, two tensors of [64,324,16,64] in three launches, 1024 places a group: 65 us with the groups first, in as many workgroups as
+// the fold takes; so 50.)
+template <bool ASYM, int NT, class F>
+__device__ __forceinline__ void spread_parameters(const GenParams &p, int shift, const float *par_s, const float *par_z, F &&group_of) {
+  auto put = [&](int t, int64_t g, u32 rep) __attribute__((always_inline)) {
+    const u32 o = p.spread.by_in(rep), a = p.spread.by_gi((u32)g);
+    const int64_t at = a * p.spread.go + (int64_t)((u32)g - a * p.spread.gi) * p.spread.ge + p.spread.off + (rep - o * p.spread.r_in) + o * p.spread.s_out;
+    p.scale[at] = par_s[t];
+    if (ASYM) p.zp[at] = par_z[t];
+  };
+  if ((p.spread.gi > 1 ? p.spread.ge : p.spread.go) == 1) {
+    for (u32 i = threadIdx.x; i < p.spread.reps << shift; i += NT) {
+      const int t = i & ((1u << shift) - 1);
+      const int64_t g = group_of(t);
+      if (g >= 0) put(t, g, i >> shift);
+    }
+  } else {   // (a wavefront per group, or all threads by as many groups as there are)
+    const int lanes = max(6, __builtin_ctz((unsigned)NT) - shift);
+    for (int t = threadIdx.x >> lanes; t < 1 << shift; t += NT >> lanes) {
+      const int64_t g = group_of(t);
+      if (g < 0) continue;
+      for (u32 rep = threadIdx.x & ((1u << lanes) - 1); rep < p.spread.reps; rep += 1u << lanes) put(t, g, rep);
+    }
+  }
+}
+
 __device__ __forceinline__ int64_t out_row(const GenParams &p, int64_t row) {
   return p.out_mapped ? row + (row / p.out_inner) * p.out_delta + p.out_off : row;
 }
@@ -311,21 +339,29 @@ __global__ __launch_bounds__(256) void finalize_tiled_kernel(GenParams p, int Z,
     }
     __syncthreads();
   }
-  if (zl != 0 || g >= p.n_groups) return;
-  mx = lds_mx[threadIdx.x];
-  mn = lds_mn[threadIdx.x];
-  float s, z = 0.f;
-  if (ASYM) {
-    s = fmaxf((mx - mn) / (float)((1 << p.bits) - 1), p.eps);
-    z = (float)p.qmin - rintf(mn / s);
-    p.zp[g] = z;
-  } else {
-    s = fmaxf(mx / (float)p.qmax, p.eps);
+  const bool spread = p.spread.on;
+  if (zl == 0 && g < p.n_groups) {
+    mx = lds_mx[threadIdx.x];
+    mn = lds_mn[threadIdx.x];
+    float s, z = 0.f;
+    if (ASYM) {
+      s = fmaxf((mx - mn) / (float)((1 << p.bits) - 1), p.eps);
+      z = (float)p.qmin - rintf(mn / s);
+      (spread ? p.spread.zp : p.zp)[g] = z;
+    } else {
+      s = fmaxf(mx / (float)p.qmax, p.eps);
+    }
+    (spread ? p.spread.scale : p.scale)[g] = s;
+    rinv[g] = 1.0f / s;
+    // whether exact_quotient holds (about x/s = -zp: the values of a group may lie far from 0 in a narrow range)
+    plain[g] = (s > 0x1p-96f && s < 0x1p96f && (f2u(s) & 0x7fffffu) != 0x7fffffu && fabsf(z) <= 0x1p120f) ? 1u : 0u;
+    lds_mx[threadIdx.x] = s;
+    lds_mn[threadIdx.x] = z;
   }
-  p.scale[g] = s;
-  rinv[g] = 1.0f / s;
-  // whether exact_quotient holds (about x/s = -zp: the values of a group may lie far from 0 in a narrow range)
-  plain[g] = (s > 0x1p-96f && s < 0x1p96f && (f2u(s) & 0x7fffffu) != 0x7fffffu && fabsf(z) <= 0x1p120f) ? 1u : 0u;
+  if (!spread) return;
+  __syncthreads();
+  spread_parameters<ASYM, 256>(p, __builtin_ctz((u32)gpb), lds_mx, lds_mn,
+                               [&](int t) { const int64_t of = (int64_t)blockIdx.x * gpb + t; return of < p.n_groups ? of : -1; });
 }
 
 // x/s == RN(q0 + (x - q0*s)*r) with q0 = RN(x*r), r = RN(1/s), for every finite x unless the significand of s is all ones, the
@@ -591,18 +627,8 @@ __device__ __forceinline__ void quant_one_block(const GenParams &p, const OnePla
   }
   __syncthreads();
   if constexpr (!KEEPC) {
-    if (p.spread.on) {
-      // all threads, the groups of the workgroup fastest (n_par, one per q, is a power of two)
-      for (u32 i = tid; i < (u32)n_par * p.spread.reps; i += NT) {
-        const int t = i & (n_par - 1), tqi = (tq << pl.lq_shift) + t;
-        const u32 rep = i >> pl.lq_shift, o = p.spread.by_in(rep);
-        if (tqi >= pl.Q) continue;
-        const u32 g = (u32)(ko * pl.ko_gs + tqi * pl.q_gs), a = p.spread.by_gi(g);
-        const int64_t at = a * p.spread.go + (int64_t)(g - a * p.spread.gi) * p.spread.ge + p.spread.off + (rep - o * p.spread.r_in) + o * p.spread.s_out;
-        p.scale[at] = par_s[t];
-        if (ASYM) p.zp[at] = par_z[t];
-      }
-    }
+    auto group_of = [&](int t) { const int q = (tq << pl.lq_shift) + t; return q < pl.Q ? (int64_t)ko * pl.ko_gs + (int64_t)q * pl.q_gs : -1; };
+    if (p.spread.on) spread_parameters<ASYM, NT>(p, pl.lq_shift, par_s, par_z, group_of);
   }
   if (!live) return;   // (2-bit words take two adjacent columns, which are live together: c is a multiple of 16 there)
   const int t0 = lq * gcols + lcol * (KEEPC ? 8 : 0);
@@ -842,12 +868,17 @@ __global__ __launch_bounds__(256, 4) void quant_shared_kernel(GenParams p, OnePl
     par_s[t] = s;
     // (as in quant_one_block)
     par_r[t] = (s > 0x1p-96f && s < 0x1p96f && (f2u(s) & 0x7fffffu) != 0x7fffffu && fabsf(zp) <= 0x1p21f) ? 1.0f / s : 0.f;
-    if (mine && shard == 0) {
-      p.scale[g] = s;
-      if (ASYM) p.zp[g] = zp;
+    float *const once = KEEPC || !p.spread.on ? p.scale : p.spread.scale;
+    if (mine && shard == 0 && once) {
+      once[g] = s;
+      if (ASYM) (KEEPC || !p.spread.on ? p.zp : p.spread.zp)[g] = zp;
     }
   });
   __syncthreads();
+  if constexpr (!KEEPC) {
+    auto group_of = [&](int t) { const int q = (tq << pl.lq_shift) + t; return q < pl.Q ? (int64_t)ko * pl.ko_gs + (int64_t)q * pl.q_gs : -1; };
+    if (p.spread.on && shard == 0) spread_parameters<ASYM, 256>(p, pl.lq_shift, par_s, par_z, group_of);
+  }
   if (!live) return;   // (2-bit words take two adjacent columns, which are live together: c is a multiple of 16 there)
   const int t0 = lq * gcols + col * (KEEPC ? 8 : 0);
   float s[NV], r[NV], z[NV] = {};
@@ -1284,11 +1315,16 @@ int run_tiled(GenParams &p, const Plan &pl, void *workspace, hipStream_t st) {
   // z-lanes per group in the finalize kernel: enough threads in total, no more lanes than partials
   int ZL = 1;
   while (ZL < 256 && ZL < pl.Z && ng * ZL < VARQ_FIN_THREADS) ZL <<= 1;
+  // ... and where each group's parameters have many places, so many workgroups as there are compute units (or groups)
+  if (p.spread.on)
+    while (ZL < 256 && (256 / ZL) * (int64_t)p.spread.reps > 1024 && ng * ZL < 256 * 256) ZL <<= 1;
   dim3 fgrid((unsigned)((ng + 256 / ZL - 1) / (256 / ZL)), nt);
   if (p.asym)
     hipLaunchKernelGGL((finalize_tiled_kernel<true>), fgrid, dim3(256), 0, st, p, pl.Z, ZL, part_max, part_min, rinv, plain);
   else
     hipLaunchKernelGGL((finalize_tiled_kernel<false>), fgrid, dim3(256), 0, st, p, pl.Z, ZL, part_max, part_min, rinv, plain);
+  // the parameters as the last launch reads them, one after the other by group, are where a caller takes them once each
+  if (p.spread.on) { p.scale = p.spread.scale; p.zp = p.spread.zp; p.scale1 = p.spread.scale1; p.zp1 = p.spread.zp1; }
   // phase B walks the same chunks (its per-thread parameters are eight 16-byte loads; chunks of 4 to 8 steps
   // per thread measured alike, longer ones slower)
   const Plan &pb = pl;
@@ -1393,7 +1429,7 @@ int quant_pack_impl(const void *x, const void *x1, int x_dtype, const int64_t *h
   // the tiled kernels pack whole words per octet: c*bits must fill words (always true for 4 and 8 bits)
   const bool tiled = make_plan(s, reduce_mask, ng, pl) && (!words || (s[3] * bits) % 32 == 0);
   const size_t need = tiled ? plan_workspace_bytes(pl, ng) * (x1 ? 2 : 1) : (size_t)ng * 2 * sizeof(u32);
-  if (workspace_bytes < need && !host_scale_map)
+  if (workspace_bytes < need && (!host_scale_map || workspace))
     return varq_set_error(VARQ_ERR_WORKSPACE, "quant_pack: workspace %zu < %zu bytes", workspace_bytes, need);
   VARQ_CHECK_ARG(rows * s[3] < (1ll << 40), "quant_pack: tensor too large");
   // only the tiled kernels that keep the channel dim move scales, zero-points and partials in
@@ -1446,7 +1482,7 @@ int quant_pack_impl(const void *x, const void *x1, int x_dtype, const int64_t *h
   const size_t words_each = tiled ? plan_workspace_bytes(pl, ng) / sizeof(u32) : 0;
   OnePlan by_many;
   Shards sh = {};
-  const Way way = tiled ? choose_way(s, reduce_mask, ng, x_dtype == VARQ_F32 ? 4 : 2, x1 ? 2 : 1, words ? bits : 8, asym != 0, step != nullptr, !host_scale_map,
+  const Way way = tiled ? choose_way(s, reduce_mask, ng, x_dtype == VARQ_F32 ? 4 : 2, x1 ? 2 : 1, words ? bits : 8, asym != 0, step != nullptr, !host_scale_map || workspace,
                                      words_each, large_wgs(pl), one, threads, by_many, sh)
                         : Way::kAnyShape;
   if (way == Way::kOne) {
@@ -1476,8 +1512,8 @@ int quant_pack_impl(const void *x, const void *x1, int x_dtype, const int64_t *h
     if (x_dtype == VARQ_F32) run_shared<VARQ_F32>(p, by_many, sh, st);
     else if (x_dtype == VARQ_BF16) run_shared<VARQ_BF16>(p, by_many, sh, st);
     else run_shared<VARQ_F16>(p, by_many, sh, st);
-  } else if (host_scale_map) {
-    return varq_set_error(VARQ_ERR_UNSUPPORTED, "quant_pack: spread scales come with groups that one launch quantizes");
+  } else if (host_scale_map && (way == Way::kAnyShape || !workspace || !p.spread.scale)) {
+    return varq_set_error(VARQ_ERR_UNSUPPORTED, "quant_pack: spread scales come with groups that one launch quantizes, or with a workspace and the scales once per group");
   } else if (way == Way::kThree) {
     if (x1) { p.x1 = x1; p.scale1 = scale1; p.zp1 = zp1; p.words1 = words1; p.codes1 = codes1; }
     if (x_dtype == VARQ_F32) run_tiled<VARQ_F32>(p, pl, workspace, st);
@@ -1535,14 +1571,22 @@ extern "C" int varq_quant_pack_shards(const int64_t *host_shape4, int reduce_mas
   return way == Way::kShared ? sh.n : way == Way::kOne ? 1 : 0;
 }
 
+extern "C" int varq_quant_pack_spread_room(const void *x0, const void *x1, int x_dtype, const int64_t *host_shape4, int reduce_mask, int bits, int asym,
+                                           float eps, int32_t *words0, float *scale0, float *zp0, int32_t *words1, float *scale1, float *zp1,
+                                           float *once_scale0, float *once_zp0, float *once_scale1, float *once_zp1,
+                                           const int64_t *host_out_map, const int64_t *host_scale_map, void *workspace, size_t workspace_bytes, void *stream) {
+  VARQ_CHECK_ARG(host_scale_map, "quant_pack_spread: null scale map");
+  float *const once[4] = {once_scale0, once_zp0, once_scale1, once_zp1};
+  return quant_pack_impl(x0, x1, x_dtype, host_shape4, reduce_mask, bits, asym, eps, words0, nullptr, scale0, zp0, words1, nullptr, scale1, zp1,
+                         host_out_map, workspace, workspace_bytes, stream, nullptr, 0, host_scale_map, once);
+}
+
 extern "C" int varq_quant_pack_spread_once(const void *x0, const void *x1, int x_dtype, const int64_t *host_shape4, int reduce_mask, int bits, int asym,
                                            float eps, int32_t *words0, float *scale0, float *zp0, int32_t *words1, float *scale1, float *zp1,
                                            float *once_scale0, float *once_zp0, float *once_scale1, float *once_zp1,
                                            const int64_t *host_out_map, const int64_t *host_scale_map, void *stream) {
-  VARQ_CHECK_ARG(host_scale_map, "quant_pack_spread: null scale map");
-  float *const once[4] = {once_scale0, once_zp0, once_scale1, once_zp1};
-  return quant_pack_impl(x0, x1, x_dtype, host_shape4, reduce_mask, bits, asym, eps, words0, nullptr, scale0, zp0, words1, nullptr, scale1, zp1,
-                         host_out_map, nullptr, 0, stream, nullptr, 0, host_scale_map, once);
+  return varq_quant_pack_spread_room(x0, x1, x_dtype, host_shape4, reduce_mask, bits, asym, eps, words0, scale0, zp0, words1, scale1, zp1,
+                                     once_scale0, once_zp0, once_scale1, once_zp1, host_out_map, host_scale_map, nullptr, 0, stream);
 }
 
 extern "C" int varq_quant_pack_spread(const void *x0, const void *x1, int x_dtype, const int64_t *host_shape4, int reduce_mask, int bits, int asym,
