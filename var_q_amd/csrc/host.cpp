@@ -890,21 +890,20 @@ struct Quantizer {
 // quantizer_step(k_quant, k, v_quant | None, v | None) -> whether the step was taken: quant and cache, K and V of a step in the same launches.
 // One call with the scales written where the cache keeps them took a step of the rules with scales per token from 72 us of host work
 // (two quantizers: reductions, expand, copies into the growing buffers) to that of the shipped rule.
-PyObject *quantizer_step(PyObject *const *a) {
+bool take_step(const Quantizer &kq, PyObject *const *a) {
   const bool two = a[2] != Py_None;
-  const Quantizer kq(a[0]);
-  if (!kq.takes(a[1])) Py_RETURN_FALSE;
+  if (!kq.takes(a[1])) return false;
   std::optional<Quantizer> vq;
   const at::Tensor &k = THPVariable_Unpack(a[1]);
   const double eps = real(Ref(attribute(a[0], NAME(eps))).o);
   if (two) {
     vq.emplace(a[2]);
-    if (a[0] == a[2] || !vq->takes(a[3])) Py_RETURN_FALSE;
+    if (a[0] == a[2] || !vq->takes(a[3])) return false;
     const at::Tensor &v = THPVariable_Unpack(a[3]);
     // (one window of two buffers, one row of two tables)
     if (kq.rule != vq->rule || kq.bits != vq->bits || kq.asym != vq->asym || kq.d != vq->d || kq.len != vq->len || kq.k != vq->k || v.sizes() != k.sizes() ||
         v.scalar_type() != k.scalar_type() || v.device() != k.device() || kq.buf->sizes() != vq->buf->sizes() || eps != real(Ref(attribute(a[2], NAME(eps))).o))
-      Py_RETURN_FALSE;
+      return false;
   }
   const int64_t sh[4] = {k.size(0), k.size(1), k.size(2), k.size(3)}, d = kq.d, n = sh[d], per_tok = d == 1 ? sh[2] : 1, row = kq.k * kq.heads() * kq.c;
   const int64_t map[3] = {n * per_tok, (kq.buf->size(d) - n) * per_tok, kq.len * per_tok};
@@ -918,7 +917,7 @@ PyObject *quantizer_step(PyObject *const *a) {
   int64_t spread[7];
   if (!rows) kq.spread(n, spread);
   Quantizer::Own own[2];
-  if (!rows && (!kq.own_place(own[0], n) || (two && !vq->own_place(own[1], n)))) Py_RETURN_FALSE;
+  if (!rows && (!kq.own_place(own[0], n) || (two && !vq->own_place(own[1], n)))) return false;
   const int rc = status_unlocked([&] {
     if (rows) return pack_rows(k, x1, dt, sh, mask, bits, asym, (float)eps, w0, w1, s, z, map);
     float *const s0 = own[0].data(), *const s1 = two ? own[1].data() : nullptr;
@@ -932,20 +931,25 @@ PyObject *quantizer_step(PyObject *const *a) {
     const at::Tensor ws = empty({(int64_t)ws_bytes}, at::kByte, k);
     return step(ws.data_ptr(), ws_bytes);
   });
-  if (!rows && rc == VARQ_ERR_UNSUPPORTED) Py_RETURN_FALSE;
+  if (!rows && rc == VARQ_ERR_UNSUPPORTED) return false;
   check(rc, "varq_quant_pack");
   kq.commit(n, rows ? nullptr : &own[0]);
   if (two) vq->commit(n, rows ? nullptr : &own[1]);
-  Py_RETURN_TRUE;
+  return true;
+}
+PyObject *quantizer_step(PyObject *const *a) {
+  const Quantizer kq(a[0]);
+  return PyBool_FromLong(take_step(kq, a));
 }
 
-// quantizer_use(quantizer, x, out dtype code) -> the dequantized cache with the step behind the earlier ones (the shipped rule), or None
+// quantizer_use(quantizer, x, out dtype code) -> the dequantized cache with the step behind the earlier ones, or None (nothing done)
 PyObject *quantizer_use(PyObject *const *a) {
   const Quantizer z(a[0]);
-  if (z.rule != Rule::kHeadDim || !z.takes(a[1]) || z.c % 8 != 0 || z.last_end() != z.len) Py_RETURN_NONE;
+  const bool tokens = per_token(z.rule), rows = z.rule == Rule::kHeadDim;
+  if (!z.takes(a[1]) || z.c % 8 != 0 || (!tokens && z.last_end() != z.len)) Py_RETURN_NONE;
   const at::Tensor &x = THPVariable_Unpack(a[1]);
-  const int64_t d = z.d, n = x.size(d), B = x.size(0), H = z.heads(), c = z.c, code = integer(a[2]);
-  if ((uintptr_t)x.data_ptr() & 15 || (z.len + n) * (d == 1 ? H : 1) * (c / 8) >= (1ll << 31) - 2048) Py_RETURN_NONE;
+  const int64_t d = z.d, n = x.size(d), B = x.size(0), H = z.heads(), c = z.c, code = integer(a[2]), len = z.len + n;
+  if ((rows && (uintptr_t)x.data_ptr() & 15) || (!tokens && len * (d == 1 ? H : 1) * (c / 8) >= (1ll << 31) - 2048)) Py_RETURN_NONE;
   int32_t ends[16];
   for (int i = 0; i < z.k; ++i) ends[i] = (int32_t)integer(PyList_GET_ITEM(z.ends.o, i));
   ends[z.k] = (int32_t)(z.len + n);
@@ -954,10 +958,27 @@ PyObject *quantizer_use(PyObject *const *a) {
   const c10::DeviceGuard guard(x.device());
   const int dt = dtype_code(x);
   at::Tensor out;
+  auto new_out = [&] { return d == 1 ? empty({B, len, H, c}, dtype_of((int)code), x) : empty({B, H, len, c}, dtype_of((int)code), x); };
+  if (!rows) {   // the rules whose scales are not a row of the tables: the step, and the launch that dequantizes what they read
+    PyObject *const step[4] = {a[0], a[1], Py_None, Py_None};
+    if (!take_step(z, step)) Py_RETURN_NONE;
+    unlocked("varq_dequant", [&] {
+      out = new_out();
+      const int64_t cap = z.buf->size(d);
+      if (!tokens)
+        return varq_dequant_steps(ptr<int32_t>(z.buf), ptr<float>(z.scale), ptr<float>(z.zp), (int)z.k + 1, ends, (int)B, (int)H, cap, (int)c, (int)z.bits, d == 1,
+                                  out.data_ptr(), (int)code, stream_of(x));
+      const int64_t heads = z.rule == Rule::kTokenHead;   // (the scales of batch entry 0, and of head 0, serve the others)
+      const int64_t shape[4] = {B, d == 1 ? len : H, d == 1 ? H : len, c}, ss[4] = {0, d == 1 ? H : heads * cap, d == 1 ? heads : 1, 0};
+      const int64_t in[8] = {shape[0], shape[1], shape[2], H * cap, d == 1 ? H : cap, 1, 0, -1};
+      return varq_dequant(ptr<int32_t>(z.buf), nullptr, ptr<float>(z.scale), ptr<float>(z.zp), shape, ss, (int)c, (int)z.bits, in, out.data_ptr(), (int)code, stream_of(x));
+    });
+    return wrap(out);
+  }
   unlocked("varq_quant_step_dequant", [&] {
     const size_t ws_bytes = std::max<size_t>(varq_quant_workspace_bytes(sh, z.mask()), 8);
     const at::Tensor ws = empty({(int64_t)ws_bytes}, at::kByte, x);
-    out = d == 1 ? empty({B, z.len + n, H, c}, dtype_of((int)code), x) : empty({B, H, z.len + n, c}, dtype_of((int)code), x);
+    out = new_out();
     return varq_quant_step_dequant(x.data_ptr(), dt, (int)B, (int)H, (int)n, (int)c, d == 1, (int)z.bits, z.asym, eps, ptr<int32_t>(z.buf), z.buf->size(d),
                                    ptr<float>(z.scale), ptr<float>(z.zp), (int)z.k + 1, ends, out.data_ptr(), (int)code, ws.data_ptr(), ws_bytes, stream_of(x));
   });

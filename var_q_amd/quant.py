@@ -329,18 +329,23 @@ class VAR_Q:
         self._window, self._current = None, [q, s, z]
 
     def _make_room(self, x: torch.Tensor) -> bool:
-        """Room for a step of the shipped rule in the cache buffer and the step tables, as quant() and cache() make it;
-        nothing launched, no step added.  False when the quantizer or the item is of another kind."""
-        bits = self.quant_bits
-        if self.quant_method != 'G_SCALE_HEAD_DIM' or not self.pack_to_int32 or bits not in (2, 4, 8):
+        """Room for a step that the native call takes, in the cache buffer and the step tables or the scales per token, as
+        quant() and cache() make it; nothing launched but copies into larger buffers, no step added.  False when the quantizer or
+        the item is of another kind.  (The first step of K and V, and one that finds the buffers full, cost 60-90 us of host
+        work through quant() and cache().)"""
+        bits, m = self.quant_bits, self.quant_method
+        if m not in _NATIVE_METHODS or not self.pack_to_int32 or bits not in (2, 4, 8):
             return False
         if not isinstance(x, torch.Tensor) or x.dim() != 4 or not x.is_cuda or not x.is_contiguous() or x.dtype not in ops._DT:
             return False
         item, d = self._c_item, self.dim_cat
         s0, s1, s2, c = x.shape
         vals = 32 // bits
-        if item.dim != d or len(self._seg_ends) >= MAX_TABLE_STEPS or c % vals or s0 * s1 * s2 == 0:
+        if item.dim != d or len(self._seg_ends) >= MAX_TABLE_STEPS or c % vals or x.numel() == 0:
             return False                      # (quant() says why an empty step is refused)
+        tokens = m in _TOKEN_METHODS
+        if m != 'G_SCALE_HEAD_DIM' and c % 8 or tokens and (self._tok_scale.dim != d or self._tok_scale.len != item.len):
+            return False
         meta = self._pack_meta
         if meta is None:
             self._pack_meta = {'orig_c': c, 'vals_per_word': vals, 'pad_len': 0, 'bits': bits}
@@ -348,15 +353,21 @@ class VAR_Q:
             return False                      # (quant() raises the reference's assertion for this)
         if item.reserve([s0, s1, s2, c // vals], torch.int32, x.device) is None:
             return False
-        self._table_rows(x.shape[3 - d], c, x.device)
+        if tokens:
+            for kept in (self._tok_scale,) if self.symmetric else (self._tok_scale, self._tok_zp):
+                if kept.reserve([s0, s1, s2, 1], torch.float32, x.device) is None:
+                    return False
+        else:
+            self._table_rows(x.shape[3 - d], c, x.device)
+        self._own_room(x.shape[3 - d])
         return True
 
     def _step_fast(self, x: torch.Tensor) -> bool:
         """quant(x) followed by cache() with the host work of a generation step cut to one native call: same kernels, same
         state afterwards.  It takes the rules whose codes and scales the kernels can write where the cache keeps them (one
-        scale per (head, channel), per head, per step, per token or per (token, head); packed codes), once there is room:
-        the general methods make it, with the first step and where the buffers have to grow.  False (nothing done) for
-        everything else; the caller then takes the two general calls."""
+        scale per (head, channel), per head, per step, per token or per (token, head); packed codes), once there is room, which
+        _make_room makes for the first step and where the buffers have to grow.  False (no step added) for everything else; the
+        caller then takes the two general calls."""
         return self._takes_native() and (_lib.host().quantizer_step(self, x, None, None)
                                          or self._make_room(x) and _lib.host().quantizer_step(self, x, None, None))
 
@@ -517,13 +528,14 @@ class VAR_Q:
         two to four times an unquantized bf16 cache, resident until the quantizer is deleted --
         172 MB per tensor at [2,16,10521,128].  `dequant_all()` itself always recomputes everything."""
         if not self.keep_dequantized:
-            # the shipped rule: step and dequantized cache from one library call (and where the sizes allow, one launch)
-            use, code = _lib.host().quantizer_use, ops._DT[out_dtype or torch.float32]
-            res = use(self, item, code)
-            if res is None and self.quant_method == 'G_SCALE_HEAD_DIM' and self._make_room(item):
+            # step and dequantized cache from one native call (and under the shipped rule, where the sizes allow, one launch)
+            if self._takes_native():
+                use, code = _lib.host().quantizer_use, ops._DT[out_dtype or torch.float32]
                 res = use(self, item, code)
-            if res is not None:
-                return res
+                if res is None and self._make_room(item):
+                    res = use(self, item, code)
+                if res is not None:
+                    return res
         if not self._step_fast(item):
             self.quant(item)
             self.cache()
@@ -553,6 +565,8 @@ def _dequant_views(q: torch.Tensor, scale: torch.Tensor, zp: Optional[torch.Tens
 _TABLE_METHODS = ('G_SCALE_HEAD_DIM', 'G_HEAD_DIM', 'G_TENSOR', 'G_SCALE', 'G_HEAD')
 # methods with one scale (per channel group) per token
 _TOKEN_METHODS = ('G_TOKEN', 'G_TOKEN_HEAD', 'G_GROUP')
+# methods whose step is one native call (see VAR_Q._step_fast)
+_NATIVE_METHODS = ('G_SCALE_HEAD_DIM', 'G_SCALE', 'G_HEAD', 'G_TOKEN', 'G_TOKEN_HEAD')
 MAX_TABLE_STEPS = 16
 
 
