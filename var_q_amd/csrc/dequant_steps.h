@@ -54,51 +54,66 @@ struct StepParams {
   int64_t pair_words, pair_octs;   // words of a pair in the buffer, octets of a pair that are read
   int64_t out_pair_octs;           // octets of a pair in the output
   int octs, H, c, nseg;
+  FastDiv by_octs;
   int head_in_pair;                // 1: heads first, the pair's head is pair % H
   int64_t row;                     // H * c: floats of a table
   int seg_oct[16];                 // first octet of a pair that is past segment s
 };
 
-// Block `block` of pair `pair`: NT threads, U octets each.
+// Block `block` of pair `pair`: NT threads, U octets each, all of whose loads are under way before the first is used.  (One octet after the other, each
+// with its search for the step in LDS and a trip for its scales, a workgroup was a chain of some 4 us, and what the launches of
+// a schedule took: [8,n,30,64], ten steps to fp32, 173 -> 169 us.)
 template <int ODT, int BITS, int NT, int U>
 __device__ __forceinline__ void dequant_steps_block(const StepParams &p, int64_t pair, int block) {
-  __shared__ int seg_oct[16];
-  if (threadIdx.x < 16) seg_oct[threadIdx.x] = p.seg_oct[threadIdx.x];
-  __syncthreads();
   const u32 *words = p.words + pair * p.pair_words;
   const float *scale = p.scale + (p.head_in_pair ? (pair % p.H) * p.c : 0);
   const float *zp = p.zp ? p.zp + (p.head_in_pair ? (pair % p.H) * p.c : 0) : nullptr;
-  const int o0 = block * (NT * U) + threadIdx.x;
+  const int first = block * (NT * U), last = (int)p.pair_octs - 1, o0 = first + threadIdx.x;
+  auto segment = [&](int o) __attribute__((always_inline)) {   // (those past the last one end where the pair does)
+    int seg = 0;
+#pragma unroll
+    for (int s = 0; s < 15; ++s) seg += o >= p.seg_oct[s] ? 1 : 0;
+    return seg;
+  };
+  // most blocks lie in one step
+  const int seg0 = segment(first);
+  const bool one_seg = seg0 == segment(min(first + NT * U - 1, last));
   u32 w0[U], w1[U];
+  int64_t at[U];
 #pragma unroll
   for (int u = 0; u < U; ++u) {
-    const int o = min(o0 + u * NT, (int)p.pair_octs - 1);
+    const int o = min(o0 + u * NT, last);
     w1[u] = 0;
     if (BITS == 8) { const uint2 t = *reinterpret_cast<const uint2 *>(words + 2 * (int64_t)o); w0[u] = t.x; w1[u] = t.y; }
     else if (BITS == 4) w0[u] = words[o];
     else w0[u] = words[o >> 1] >> ((o & 1) * 16);
+    at[u] = seg0 * p.row + (int)((u32)o - p.by_octs((u32)o) * (u32)p.octs) * 8;
+    if (!one_seg) at[u] += (segment(o) - seg0) * p.row;
   }
+  float4 s[U][2], z[U][2];
+#pragma unroll
+  for (int u = 0; u < U; ++u)
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      s[u][h] = *reinterpret_cast<const float4 *>(scale + at[u] + 4 * h);
+      if (zp) z[u][h] = *reinterpret_cast<const float4 *>(zp + at[u] + 4 * h);
+    }
 #pragma unroll
   for (int u = 0; u < U; ++u) {
     const int o = o0 + u * NT;
-    if (o >= (int)p.pair_octs) return;
-    int seg = 0;
-    while (seg + 1 < p.nseg && o >= seg_oct[seg]) ++seg;
-    const int64_t t = seg * p.row + (int)((u32)o % (u32)p.octs) * 8;
-    const float4 sa = *reinterpret_cast<const float4 *>(scale + t), sb = *reinterpret_cast<const float4 *>(scale + t + 4);
-    const float s[8] = {sa.x, sa.y, sa.z, sa.w, sb.x, sb.y, sb.z, sb.w};
+    if (o > last) return;
+    const float sv[8] = {s[u][0].x, s[u][0].y, s[u][0].z, s[u][0].w, s[u][1].x, s[u][1].y, s[u][1].z, s[u][1].w};
     float f[8];
 #pragma unroll
     for (int j = 0; j < 8; ++j)
       f[j] = (float)(int)(BITS == 8 ? __builtin_amdgcn_sbfe((int)(j < 4 ? w0[u] : w1[u]), 8 * (j & 3), 8) : __builtin_amdgcn_sbfe((int)w0[u], BITS * j, BITS));
     if (zp) {
-      const float4 za = *reinterpret_cast<const float4 *>(zp + t), zb = *reinterpret_cast<const float4 *>(zp + t + 4);
-      const float z[8] = {za.x, za.y, za.z, za.w, zb.x, zb.y, zb.z, zb.w};
+      const float zv[8] = {z[u][0].x, z[u][0].y, z[u][0].z, z[u][0].w, z[u][1].x, z[u][1].y, z[u][1].z, z[u][1].w};
 #pragma unroll
-      for (int j = 0; j < 8; ++j) f[j] = (f[j] - z[j]) * s[j];
+      for (int j = 0; j < 8; ++j) f[j] = (f[j] - zv[j]) * sv[j];
     } else {
 #pragma unroll
-      for (int j = 0; j < 8; ++j) f[j] = f[j] * s[j];
+      for (int j = 0; j < 8; ++j) f[j] = f[j] * sv[j];
     }
     store8<ODT>(p.out, (pair * p.out_pair_octs + o) * 8, f, 8);
   }
@@ -114,6 +129,7 @@ inline bool set_steps(StepParams &p, const int32_t *words, const float *scale, c
   p.H = H; p.c = c; p.nseg = nseg; p.row = (int64_t)H * c;
   p.head_in_pair = tokens_first ? 0 : 1;
   p.octs = (tokens_first ? H * c : c) / 8;
+  p.by_octs = FastDiv::by(p.octs);
   if (tokens * p.octs >= (1ll << 31) - 2048) return false;
   for (int s = 0; s < 16; ++s) p.seg_oct[s] = (s < nseg ? host_seg_end[s] : (int)tokens) * p.octs;
   p.pair_octs = p.out_pair_octs = tokens * p.octs;

@@ -522,6 +522,40 @@ __global__ __launch_bounds__(256) void quant_tiled_kernel(GenParams p, Plan pl, 
 // the columns are cut into slices of c8s octets, one workgroup each, until there are workgroups enough: the
 // steps of one batch have few groups, and narrow slices (64, 32, then 16 bytes of a row, whose cache lines
 // the slices of one XCD share) still read faster than few workgroups do.
+// The extremes over the lanes whose numbers differ in the bits from `from` up to below `to` (powers of two; all lanes are active), in every one of them.  From
+// rows of 16 lanes up by rotations inside the row and swaps of rows, a few cycles each where an exchange through LDS waits for some
+// hundred.  The small launches are one chain of such waits: with this fold, the wavefronts' extremes requested together and no divisions, us: ten steps with the
+// dequantized cache, [8,n,30,64] to fp32, 178 -> 173; with attention, [64,n,16,64] 375 -> 370, thirteen of [2,16,n,128] 1346 -> 1335.  In quant_shared_kernel,
+// whose registers are full, the same fold costs (K of [32,30,680,64] 63.1 -> 64.1, unpacking included), so it keeps the exchange.
+template <bool ASYM, int NV> __device__ __forceinline__ void fold_lanes(float (&mx)[NV], float (&mn)[NV], int from, int to) {
+  auto with = [&](auto &&other) __attribute__((always_inline)) {
+#pragma unroll
+    for (int j = 0; j < NV; ++j) {
+      mx[j] = fmaxf(mx[j], other(mx[j]));
+      if (ASYM) mn[j] = fminf(mn[j], other(mn[j]));
+    }
+  };
+  if (to < 16) {
+    for (int off = from; off < to; off <<= 1) with([&](float v) __attribute__((always_inline)) { return __shfl_xor(v, off, 64); });
+    return;
+  }
+  if (from <= 1) with([](float v) __attribute__((always_inline)) { return dpp_f<0x121>(v); });   // row_ror:1
+  if (from <= 2) with([](float v) __attribute__((always_inline)) { return dpp_f<0x122>(v); });
+  if (from <= 4) with([](float v) __attribute__((always_inline)) { return dpp_f<0x124>(v); });
+  if (from <= 8) with([](float v) __attribute__((always_inline)) { return dpp_f<0x128>(v); });
+  // (of a value swapped with itself one half is the other rows' and the other half the lane's own)
+  auto swapped = [&](auto &&swap) __attribute__((always_inline)) {
+#pragma unroll
+    for (int j = 0; j < NV; ++j) {
+      const auto a = swap(f2u(mx[j]));
+      mx[j] = fmaxf(u2f(a[0]), u2f(a[1]));
+      if (ASYM) { const auto b = swap(f2u(mn[j])); mn[j] = fminf(u2f(b[0]), u2f(b[1])); }
+    }
+  };
+  if (from <= 16 && to > 16) swapped([](u32 v) __attribute__((always_inline)) { return __builtin_amdgcn_permlane16_swap(v, v, false, false); });
+  if (from <= 32 && to > 32) swapped([](u32 v) __attribute__((always_inline)) { return __builtin_amdgcn_permlane32_swap(v, v, false, false); });
+}
+
 struct OnePlan {
   int64_t ko_rs, ro_rs, ko_gs, q_gs;
   int nko, Q, RR, RI;           // kept outer, kept inner; reduced rows, of which RI are contiguous
@@ -529,6 +563,7 @@ struct OnePlan {
   int c8s_shift, sub_shift, lq_shift;
   int slices, tilesQ, steps;
   int blocks;                   // nko * tilesQ
+  FastDiv by_slices, by_tilesQ;
 };
 
 // also(row, col, codes less their zero-points, scales): what else is made of an octet once it is quantized
@@ -540,9 +575,9 @@ __device__ __forceinline__ void quant_one_block(const GenParams &p, const OnePla
   __shared__ float par_s[MAXG], par_r[MAXG];
   __shared__ float par_z[ASYM ? MAXG : 1];
   // the slices of a block on one XCD (ids congruent mod 8 share an L2): they share the rows' cache lines
-  const int bid = blockIdx.x, slice = (bid >> 3) % pl.slices, blk = (bid >> 3) / pl.slices * 8 + (bid & 7);
+  const int bid = blockIdx.x, of_eight = (int)pl.by_slices((u32)bid >> 3), slice = (bid >> 3) - of_eight * pl.slices, blk = of_eight * 8 + (bid & 7);
   if (blk >= pl.blocks) return;
-  const int tq = blk % pl.tilesQ, ko = blk / pl.tilesQ;
+  const int ko = (int)pl.by_tilesQ((u32)blk), tq = blk - ko * pl.tilesQ;
   const int tid = threadIdx.x, c8s = 1 << pl.c8s_shift, sub = 1 << pl.sub_shift;
   const int lcol = tid & (c8s - 1), col = slice * c8s + lcol, f = (tid >> pl.c8s_shift) & (sub - 1), lq = tid >> (pl.c8s_shift + pl.sub_shift);
   const int q = (tq << pl.lq_shift) + lq;
@@ -579,16 +614,10 @@ __device__ __forceinline__ void quant_one_block(const GenParams &p, const OnePla
   // fold over f (and, with the channel dim reduced, over the columns), inside the wavefront first;
   // what is left is one value per wavefront and column, or per q where a q has less than a wavefront
   const int q_lanes = sub << pl.c8s_shift;         // threads of a q
-  for (int off = KEEPC ? c8s : 1; off < 64 && off < q_lanes; off <<= 1) {
-#pragma unroll
-    for (int j = 0; j < NV; ++j) {
-      mx[j] = fmaxf(mx[j], __shfl_xor(mx[j], off, 64));
-      if (ASYM) mn[j] = fminf(mn[j], __shfl_xor(mn[j], off, 64));
-    }
-  }
+  fold_lanes<ASYM>(mx, mn, KEEPC ? c8s : 1, q_lanes);
   const int gcols = KEEPC ? c8s * 8 : 1;           // groups of a q in this workgroup
   const int parts = q_lanes > 64 ? q_lanes >> 6 : 1, lane_in_part = q_lanes > 64 ? tid & 63 : tid & (q_lanes - 1);
-  const int part = q_lanes > 64 ? tid >> 6 : tid / q_lanes;      // = lq * parts + wavefront of the q
+  const int part = q_lanes > 64 ? tid >> 6 : tid >> (pl.sub_shift + pl.c8s_shift);      // = lq * parts + wavefront of the q
   if (lane_in_part < (KEEPC ? c8s : 1)) {
 #pragma unroll
     for (int j = 0; j < NV; ++j) {
@@ -600,11 +629,14 @@ __device__ __forceinline__ void quant_one_block(const GenParams &p, const OnePla
   // one thread per group
   const int n_par = gcols << pl.lq_shift;
   for (int t = tid; t < n_par; t += NT) {
-    const int tl = t / gcols, g8 = t - tl * gcols, tqi = (tq << pl.lq_shift) + tl;
+    const int tl = KEEPC ? t >> (pl.c8s_shift + 3) : t, g8 = t - tl * gcols, tqi = (tq << pl.lq_shift) + tl;
     float m = ASYM ? -INFINITY : 0.f, n = INFINITY;
-    for (int w = 0; w < parts; ++w) {
-      m = fmaxf(m, lds_mx[(tl * parts + w) * gcols + g8]);
-      if (ASYM) n = fminf(n, lds_mn[(tl * parts + w) * gcols + g8]);
+    // (all of them requested at once, the last one again where they are fewer)
+#pragma unroll
+    for (int w = 0; w < NT / 64; ++w) {
+      const int at = (tl * parts + min(w, parts - 1)) * gcols + g8;
+      m = fmaxf(m, lds_mx[at]);
+      if (ASYM) n = fminf(n, lds_mn[at]);
     }
     const bool mine = tqi < pl.Q && (!KEEPC || slice * c8s * 8 + g8 < p.c);
     float s, zp = 0.f;
@@ -691,6 +723,7 @@ __global__ __launch_bounds__(NT) void quant_one_kernel(GenParams p, OnePlan pl) 
 // waits for the others, in ticks of 10 ns.
 struct Shards {
   int n;
+  FastDiv by_n;
   u32 *mx, *mn;                 // per group, `stride` words apart
   u32 *words;                   // per block, `spacing` words apart, four of them a quarter of that from one another: see quant_shared_kernel
   int stride, spacing;
@@ -713,7 +746,7 @@ __global__ __launch_bounds__(256, 4) void quant_shared_kernel(GenParams p, OnePl
   __shared__ float par_z[ASYM ? kSharedGroups : 1];
   __shared__ u32 lds_next;
   if (take_second(p)) { sh.mx += p.ws1; sh.mn += p.ws1; sh.words += p.ws1; }
-  const int blk = blockIdx.x / sh.n, shard = blockIdx.x - blk * sh.n, tq = blk % pl.tilesQ, ko = blk / pl.tilesQ;
+  const int blk = (int)sh.by_n(blockIdx.x), shard = blockIdx.x - blk * sh.n, ko = (int)pl.by_tilesQ((u32)blk), tq = blk - ko * pl.tilesQ;
   const int tid = threadIdx.x, c8s = 1 << pl.c8s_shift, sub = 1 << pl.sub_shift;
   const int col = tid & (c8s - 1), f = (tid >> pl.c8s_shift) & (sub - 1), lq = tid >> (pl.c8s_shift + pl.sub_shift);
   const int f0 = shard * (pl.steps << pl.sub_shift) + f, q = (tq << pl.lq_shift) + lq;   // f0: the thread's first row
@@ -759,7 +792,7 @@ __global__ __launch_bounds__(256, 4) void quant_shared_kernel(GenParams p, OnePl
   // fold over f (and, with the channel dim reduced, over the columns), inside the wavefront first, as in quant_one_block
   const int q_lanes = sub << pl.c8s_shift, gcols = KEEPC ? c8s * 8 : 1;
   const int parts = q_lanes > 64 ? q_lanes >> 6 : 1, lane_in_part = q_lanes > 64 ? tid & 63 : tid & (q_lanes - 1);
-  const int part = q_lanes > 64 ? tid >> 6 : tid / q_lanes;
+  const int part = q_lanes > 64 ? tid >> 6 : tid >> (pl.sub_shift + pl.c8s_shift);
   auto fold = [&]() __attribute__((always_inline)) {
     for (int off = KEEPC ? c8s : 1; off < 64 && off < q_lanes; off <<= 1) {
 #pragma unroll
@@ -781,11 +814,13 @@ __global__ __launch_bounds__(256, 4) void quant_shared_kernel(GenParams p, OnePl
   const int n_par = gcols << pl.lq_shift;
   auto per_group = [&](auto &&body) __attribute__((always_inline)) {
     for (int t = tid; t < n_par; t += 256) {
-      const int tl = t / gcols, g8 = t - tl * gcols, tqi = (tq << pl.lq_shift) + tl;
+      const int tl = KEEPC ? t >> (pl.c8s_shift + 3) : t, g8 = t - tl * gcols, tqi = (tq << pl.lq_shift) + tl;
       float m = ASYM ? -INFINITY : 0.f, n = INFINITY;
-      for (int w = 0; w < parts; ++w) {
-        m = fmaxf(m, lds_mx[(tl * parts + w) * gcols + g8]);
-        if (ASYM) n = fminf(n, lds_mn[(tl * parts + w) * gcols + g8]);
+#pragma unroll
+      for (int w = 0; w < 4; ++w) {
+        const int at = (tl * parts + min(w, parts - 1)) * gcols + g8;
+        m = fmaxf(m, lds_mx[at]);
+        if (ASYM) n = fminf(n, lds_mn[at]);
       }
       body(t, tqi < pl.Q && (!KEEPC || g8 < p.c), (int64_t)ko * pl.ko_gs + (int64_t)tqi * pl.q_gs + (KEEPC ? g8 : 0), m, n);
     }
@@ -1176,6 +1211,7 @@ bool make_one_plan(const int64_t *sh, int reduce_mask, int elem, int tensors, in
     }
     pl.tilesQ = (int)((k.Q + (1 << pl.lq_shift) - 1) >> pl.lq_shift);
     pl.blocks = pl.nko * pl.tilesQ;
+    pl.by_slices = FastDiv::by(pl.slices); pl.by_tilesQ = FastDiv::by(pl.tilesQ);
     const bool fits = pl.steps <= row_steps;
     const int enough = with_values ? 128 : threads == 1024 ? 129 : 160;
     if (fits && ((int64_t)pl.blocks * pl.slices * tensors >= enough || !keepc || pl.c8s_shift <= narrowest)) return one_launch_pays(pl, c8, 1 << c8p_shift, threads, keepc, mib, elem, tensors, asym, with_values, shared);
@@ -1219,6 +1255,7 @@ bool make_shared_plan(const int64_t *sh, int reduce_mask, int64_t n_groups, int 
   pl.tilesQ = (int)((k.Q + (1 << pl.lq_shift) - 1) >> pl.lq_shift);
   if (k.nko * pl.tilesQ > 512) return false;
   pl.blocks = pl.nko * pl.tilesQ;
+  pl.by_slices = FastDiv::by(1); pl.by_tilesQ = FastDiv::by(pl.tilesQ);
   // as many workgroups as the chip holds at once, of at least four steps (groups of whole rows: eight), and no more than meet quickly; of
   // fewer than three per compute unit, or than nearly four where lanes idle, the three launches read faster (two heads: fp32 [1,2,381944,72], one scale per
   // head, 103 -> 128 us, fp16 [2,2,381944,72] 139 -> 261; three: fp16 [2,3,23148,72] 22.3 -> 23.6, but fp32 [5,3,28645,128] 104 -> 87), in 16 bits also of fewer than
@@ -1236,7 +1273,7 @@ bool make_shared_plan(const int64_t *sh, int reduce_mask, int64_t n_groups, int 
   // (lines of their own for the extremes of each group of whole rows and for the words of a block, and as far apart as there is room
   // otherwise: atomics on one line wait for one another.  One scale per head of 30 heads, 60 or 61 chunks of the three launches and thus room for
   // half a line: fp32 [60,30,66,128] affine 36.4 -> 19.7 us (side by side / 16 words apart; three launches 28.1), [3,30,3843,40] 33.7 -> 21.0 (26.4))
-  s.n = (int)n;
+  s.n = (int)n; s.by_n = FastDiv::by(n);
   for (s.stride = keepc ? 1 : 32; s.stride > 1 && 2 * (size_t)s.stride * (size_t)n_groups + 64 * (size_t)pl.blocks > words;) s.stride /= 2;
   const size_t left = words - std::min(words, 2 * s.stride * (size_t)n_groups);
   for (s.spacing = 64; s.spacing >= 8 && (size_t)s.spacing * pl.blocks > left;) s.spacing /= 2;
