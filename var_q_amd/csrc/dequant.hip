@@ -7,6 +7,7 @@
 // One lane produces 8 consecutive channels.  A block stays inside one (i0,i1)
 // pair so the scale base and the input-window row base are block-uniform.
 #include "dequant_steps.h"
+#include <type_traits>
 
 using namespace varq_deq;
 
@@ -24,13 +25,9 @@ struct DeqParams {
   int64_t octets_per_pair;
   int c, c8, wpr, bits, group;
   int c8_shift;            // log2(c8) when c8 is a power of two, else -1
-  int g8_shift;            // log2(group / 8) when group is 8 times a power of two, else -1
 };
 
-// U items (octets) per lane, 256 lanes apart: all of a lane's loads are issued before the first
-// of them is used, so a wavefront keeps U times the bytes in flight and the launch has a U-th of
-// the wavefronts (with one item per lane the kernel is bound by wavefront turnover, not by
-// bandwidth: 54-61 % of the HBM peak on the benchmark shapes against 62-70 % with four).
+// Any codes, groups, strides and alignments; U items (octets) per lane, 256 lanes apart.
 template <int ODT, int U>
 __global__ __launch_bounds__(256) void dequant_kernel(DeqParams p) {
   // grid = (tiles of 256*U octets, i1, i0): no division to find the block's place
@@ -39,91 +36,6 @@ __global__ __launch_bounds__(256) void dequant_kernel(DeqParams p) {
   const int64_t sbase0 = i0 * p.ss0 + i1 * p.ss1;
   const int64_t in_base = i0 * p.in_map.os0 + i1 * p.in_map.os1 + p.in_map.off;
   const int64_t out_base = (i0 * p.n1 + i1) * p.n2;
-  const bool words_ok = (p.c & 7) == 0 && p.words != nullptr &&
-                        (p.bits != 8 || (reinterpret_cast<uintptr_t>(p.words) & 7) == 0);   // (block-uniform)
-  // one scale per channel that does not depend on the token (a per-(head, channel) table), rows of
-  // a power-of-two number of octets: the lane's U items are the same octet column of U tokens
-  // and share one vector of 8 scales and 8 zero-points
-  const bool chan = words_ok && p.group == 1 && p.ss3 == 1 && p.ss2 == 0 && p.c8_shift >= 0 && p.c8 <= 256 &&
-                    ((sbase0 | (int64_t)(reinterpret_cast<uintptr_t>(p.scale) >> 2) |
-                      (int64_t)(reinterpret_cast<uintptr_t>(p.zp) >> 2)) & 3) == 0;
-  const bool fast = words_ok && (p.group & 7) == 0;
-  if (fast || chan) {
-    // packed words: one word (two for 8-bit codes) per item, and one scale and zero-point per
-    // item (groups of whole octets) or the lane's vectors (per-channel tables)
-    int w0[U], w1[U], i2v[U], colv[U];
-    float sv[U], zv[U];
-    bool live[U];
-    float cs[8], cz[8];
-    if (chan) {
-      const int col = o0 & (p.c8 - 1);
-      const float4 *sp = reinterpret_cast<const float4 *>(p.scale + sbase0 + col * 8);
-      const float4 sa = sp[0], sb = sp[1];
-      cs[0] = sa.x; cs[1] = sa.y; cs[2] = sa.z; cs[3] = sa.w; cs[4] = sb.x; cs[5] = sb.y; cs[6] = sb.z; cs[7] = sb.w;
-#pragma unroll
-      for (int j = 0; j < 8; ++j) cz[j] = 0.f;
-      if (p.zp) {
-        const float4 *zq = reinterpret_cast<const float4 *>(p.zp + sbase0 + col * 8);
-        const float4 za = zq[0], zb = zq[1];
-        cz[0] = za.x; cz[1] = za.y; cz[2] = za.z; cz[3] = za.w; cz[4] = zb.x; cz[5] = zb.y; cz[6] = zb.z; cz[7] = zb.w;
-      }
-    }
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const int o = o0 + u * 256;
-      live[u] = o < p.octets_per_pair;
-      const int oc = live[u] ? o : 0;
-      int i2, col;
-      if (p.c8_shift >= 0) { i2 = oc >> p.c8_shift; col = oc & (p.c8 - 1); }
-      else { i2 = oc / p.c8; col = oc - i2 * p.c8; }
-      i2v[u] = i2; colv[u] = col;
-      const int32_t *src = p.words + (in_base + i2 * p.in_map.os2) * p.wpr;
-      if (p.bits == 4) { w0[u] = src[col]; w1[u] = 0; }
-      else if (p.bits == 8) { const int2 t = *reinterpret_cast<const int2 *>(src + col * 2); w0[u] = t.x; w1[u] = t.y; }
-      else { w0[u] = src[col >> 1]; w1[u] = 0; }
-      if (!chan) {
-        const int gi = p.g8_shift >= 0 ? col >> p.g8_shift : col * 8 / p.group;   // (block-uniform choice)
-        const int64_t g = sbase0 + i2 * p.ss2 + gi * p.ss3;
-        sv[u] = p.scale[g];
-        zv[u] = p.zp ? p.zp[g] : 0.f;
-      }
-    }
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      if (!live[u]) continue;
-      int q[8];
-      if (p.bits == 4) {
-#pragma unroll
-        for (int j = 0; j < 8; ++j) q[j] = __builtin_amdgcn_sbfe(w0[u], 4 * j, 4);
-      } else if (p.bits == 8) {
-#pragma unroll
-        for (int j = 0; j < 4; ++j) { q[j] = __builtin_amdgcn_sbfe(w0[u], 8 * j, 8); q[4 + j] = __builtin_amdgcn_sbfe(w1[u], 8 * j, 8); }
-      } else {
-        const int w = w0[u] >> ((colv[u] & 1) * 16);
-#pragma unroll
-        for (int j = 0; j < 8; ++j) q[j] = __builtin_amdgcn_sbfe(w, 2 * j, 2);
-      }
-      float f[8];
-      if (chan) {
-        // (the same two operations as the scalar form below, so the results are the same bits)
-        if (p.zp) {
-#pragma unroll
-          for (int j = 0; j < 8; ++j) f[j] = ((float)q[j] - cz[j]) * cs[j];
-        } else {
-#pragma unroll
-          for (int j = 0; j < 8; ++j) f[j] = (float)q[j] * cs[j];
-        }
-      } else if (p.zp) {
-#pragma unroll
-        for (int j = 0; j < 8; ++j) f[j] = ((float)q[j] - zv[u]) * sv[u];
-      } else {
-#pragma unroll
-        for (int j = 0; j < 8; ++j) f[j] = (float)q[j] * sv[u];
-      }
-      store8<ODT>(p.out, (out_base + i2v[u]) * p.c + colv[u] * 8, f, 8);
-    }
-    return;
-  }
 #pragma unroll 1
   for (int u = 0; u < U; ++u) {
   const int o = o0 + u * 256;
@@ -205,6 +117,103 @@ __global__ __launch_bounds__(256) void dequant_kernel(DeqParams p) {
   }
 }
 
+// Packed words whose scales lie in groups of whole octets (TABLE = 0) or one per channel (1; 2: the tokens of a pair share them, and the
+// lane's pieces are the same channels of U tokens, with one load): everything else takes dequant_kernel.
+// Bound by HBM.  A lane stores U pieces of 16 bytes, a wavefront 1 KiB with each (two stores of 16 bytes, 32 apart, for the octet of 32-bit values: 68 us where this
+// takes 55), and all loads of a lane are under way before the first is used.  Widths, divisors and kind of scales are known when the kernel is compiled or
+// come as multipliers: with branches and integer divisions between the loads a launch took 2 to 3 us more at any size.  In a graph, us, before -> now: groups of
+// 32, 4 bits, [3,7,1511,96] fp32 6.4 -> 4.3, bf16 5.1 -> 3.2; 2 bits [2,16,2048,128] bf16 7.0 -> 5.2; 8 bits [4,30,1000,64] fp32 10.3 -> 7.1; 4 bits [16,16,2000,128]
+// fp32 77 -> 43, [16,16,4000,128] bf16 76 -> 49; a scale per (head, channel) [8,30,100,64] 8 bits fp32 4.4 -> 3.3, [2,8,8000,40] 4 bits bf16 7.2 -> 5.1.
+// One piece per lane: 55 -> 83 us at 262 MB of fp32, four: 57, with the small launches the same.
+// STREAM: an output that does not fit the Infinity Cache with its codes goes past it (262 MB, alone / with a copy that reads it: fp32 55 / 158 -> 43 / 152, bf16 58 / 158 -> 49 / 154); a
+// smaller one would be read from memory by whoever reads it next (98 MB fp32 18.6 / 48.5 -> 16.3 / 54.3, 84 MB bf16 19.0 / 43.7 -> 18.1 / 48.9).
+constexpr int64_t kStreamBytes = 240ll << 20;
+struct WordsParams {
+  const char *words;
+  const float *scale, *zp;
+  void *out;
+  int64_t os0, os1, off;            // input row of pair (i0, i1)
+  int64_t ss0, ss1;
+  int64_t n1;
+  u32 row_bytes, token_bytes;       // bytes of a row of words, and from a token of a pair to the next
+  int ss2, ss3;                     // floats from a token's scales to the next one's, and from a group's to the next
+  int octets;                       // of a pair
+  int c8;
+  FastDiv by_c8, by_g8;             // octets of a row, and of a group
+};
+template <int ODT, int BITS, int TABLE, int U, bool STREAM>
+__global__ __launch_bounds__(256) void dequant_words_kernel(WordsParams p) {
+  // grid = (tiles of 256 * U pieces, i1, i0)
+  constexpr int Q = ODT == VARQ_F32 ? 4 : 8, PER = 8 / Q;   // channels of a piece, pieces of an octet
+  const int64_t i0 = blockIdx.z, i1 = blockIdx.y;
+  const u32 first = blockIdx.x * (256 * U) + threadIdx.x, n = (u32)p.octets * PER;
+  const char *const words = p.words + (i0 * p.os0 + i1 * p.os1 + p.off) * p.row_bytes;
+  const int64_t table = i0 * p.ss0 + i1 * p.ss1;
+  const float *const scale = p.scale + table, *const zp = p.zp ? p.zp + table : nullptr;
+  constexpr int V = TABLE ? Q / 4 : 1, N = TABLE == 2 ? 1 : U;   // vectors of scales of a piece; pieces with scales of their own
+  typedef float f4 __attribute__((ext_vector_type(4)));
+  u32 w0[U], w1[U];
+  f4 s[N][V], z[N][V];
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    const u32 i = min(first + u * 256, n - 1), o = i / PER, i2 = p.by_c8(o), col = o - i2 * p.c8, ch = col * 8 + i % PER * Q;
+    const char *const src = words + (size_t)(i2 * p.token_bytes + ch * BITS / 8);
+    w1[u] = 0;
+    if constexpr (BITS * Q == 64) { const uint2 t = *reinterpret_cast<const uint2 *>(src); w0[u] = t.x; w1[u] = t.y; }
+    else if constexpr (BITS * Q == 32) w0[u] = *reinterpret_cast<const u32 *>(src);
+    else if constexpr (BITS * Q == 16) w0[u] = *reinterpret_cast<const uint16_t *>(src);
+    else w0[u] = *reinterpret_cast<const unsigned char *>(src);
+    if (u < N) {
+      if constexpr (TABLE) {
+#pragma unroll
+        for (int h = 0; h < V; ++h) {
+          const u32 g = (TABLE == 1 ? i2 * (u32)p.ss2 : 0) + ch + 4 * h;
+          s[u][h] = *reinterpret_cast<const f4 *>(scale + g);
+          if (zp) z[u][h] = *reinterpret_cast<const f4 *>(zp + g);
+        }
+      } else {
+        const u32 g = i2 * (u32)p.ss2 + p.by_g8(col) * (u32)p.ss3;
+        s[u][0][0] = scale[g];
+        if (zp) z[u][0][0] = zp[g];
+      }
+    }
+  }
+  const int64_t pair = (i0 * p.n1 + i1) * n;
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    const u32 i = first + u * 256;
+    const int m = TABLE == 2 ? 0 : u;
+    if (i >= n) return;
+    float f[8];
+#pragma unroll
+    for (int j = 0; j < Q; ++j) {
+      f[j] = (float)(int)(BITS == 8 ? __builtin_amdgcn_sbfe((int)(j < 4 ? w0[u] : w1[u]), 8 * (j & 3), 8) : __builtin_amdgcn_sbfe((int)w0[u], BITS * j, BITS));
+      const float sj = TABLE ? s[m][j / 4 % V][j % 4] : s[m][0][0];
+      f[j] = zp ? (f[j] - (TABLE ? z[m][j / 4 % V][j % 4] : z[m][0][0])) * sj : f[j] * sj;
+    }
+    if constexpr (Q == 4) put<STREAM>(reinterpret_cast<f4 *>(p.out) + (pair + i), f4{f[0], f[1], f[2], f[3]});
+    else store8<ODT, STREAM>(p.out, (pair + i) * 8, f, 8);
+  }
+}
+
+template <int ODT> void launch_words(const WordsParams &w, const int64_t *s, int bits, bool table, hipStream_t st) {
+  constexpr int U = 2, PER = ODT == VARQ_F32 ? 2 : 1;
+  dim3 grid((unsigned)(((int64_t)w.octets * PER + 256 * U - 1) / (256 * U)), (unsigned)s[1], (unsigned)s[0]);
+  const bool stream = s[0] * s[1] * (int64_t)w.octets * 16 * PER >= kStreamBytes;
+  auto kind = [&](auto b, auto t) {
+    if (stream) hipLaunchKernelGGL((dequant_words_kernel<ODT, b(), t(), U, true>), grid, dim3(256), 0, st, w);
+    else hipLaunchKernelGGL((dequant_words_kernel<ODT, b(), t(), U, false>), grid, dim3(256), 0, st, w);
+  };
+  auto width = [&](auto b) {
+    if (!table) kind(b, std::integral_constant<int, 0>{});
+    else if (w.ss2 == 0 && 256 % (w.c8 * PER) == 0) kind(b, std::integral_constant<int, 2>{});
+    else kind(b, std::integral_constant<int, 1>{});
+  };
+  if (bits == 4) width(std::integral_constant<int, 4>{});
+  else if (bits == 8) width(std::integral_constant<int, 8>{});
+  else width(std::integral_constant<int, 2>{});
+}
+
 template <int ODT, int BITS>
 __global__ __launch_bounds__(256) void dequant_steps_kernel(StepParams p) {
   dequant_steps_block<ODT, BITS, 256, 4>(p, (int64_t)blockIdx.z * gridDim.y + blockIdx.y, blockIdx.x);
@@ -278,30 +287,34 @@ extern "C" int varq_dequant(const int32_t *words, const int8_t *codes_i8, const 
   }
   p.octets_per_pair = s[2] * p.c8;
   p.c8_shift = -1;
-  p.g8_shift = -1;
-  for (int sh = 0; sh < 20; ++sh) {
+  for (int sh = 0; sh < 20; ++sh)
     if ((1 << sh) == p.c8) p.c8_shift = sh;
-    if ((8 << sh) == group) p.g8_shift = sh;
-  }
-  // four items per lane where a pair has the work for it (the last block's idle lanes weigh less
-  // than the wavefront turnover they save), one otherwise
-  // (two where four would leave more than a twelfth of the last block's lanes idle; not for
-  // per-channel tables, where a lane's pieces share one load of its eight scales and zero-points)
-  int U = p.octets_per_pair >= 2048 ? 4 : 1;
-  if (U == 4 && !(group == 1 && p.ss3 == 1 && p.ss2 == 0)) {
-    const int64_t t4 = (p.octets_per_pair + 1023) / 1024;
-    if ((t4 * 1024 - p.octets_per_pair) * 12 > t4 * 1024) U = 2;
-  }
-  const int64_t tiles = (p.octets_per_pair + 256 * U - 1) / (256 * U);
   // a pair with few rows wastes lanes of its last block only; pairs map to grid.y/z (limit 65535 each)
   VARQ_CHECK_ARG(p.octets_per_pair < (1ll << 31) - 1024 && s[1] <= 65535 && s[0] <= 65535, "dequant: shape exceeds the grid limits");
-  dim3 grid((unsigned)tiles, (unsigned)s[1], (unsigned)s[0]);
   hipStream_t st = (hipStream_t)stream;
-#define VARQ_DEQ(ODT_)                                                                       \
-  do {                                                                                       \
-    if (U == 4) hipLaunchKernelGGL((dequant_kernel<ODT_, 4>), grid, dim3(256), 0, st, p);    \
-    else if (U == 2) hipLaunchKernelGGL((dequant_kernel<ODT_, 2>), grid, dim3(256), 0, st, p); \
-    else hipLaunchKernelGGL((dequant_kernel<ODT_, 1>), grid, dim3(256), 0, st, p);           \
+  const bool table = group == 1 && p.ss3 == 1 && (s[2] == 1 || p.ss2 % 4 == 0) && (s[0] == 1 || p.ss0 % 4 == 0) && (s[1] == 1 || p.ss1 % 4 == 0) && (((uintptr_t)scale | (uintptr_t)zp) & 15) == 0;
+  const int64_t token_bytes = p.in_map.os2 * p.wpr * 4;
+  // (places inside a pair are counted in 32 bits)
+  if (words && s[3] % 8 == 0 && (bits != 8 || ((uintptr_t)words & 7) == 0) && (group % 8 == 0 || table) && ((uintptr_t)out & 15) == 0 && token_bytes >= 0 &&
+      token_bytes <= (1ll << 32) / s[2] - 1 && p.ss2 >= 0 && p.ss3 >= 0 && p.ss2 <= (1ll << 30) / s[2] && p.ss3 <= (1ll << 30) / s[3]) {
+    WordsParams w;
+    w.words = reinterpret_cast<const char *>(words); w.scale = scale; w.zp = zp; w.out = out;
+    w.os0 = p.in_map.os0; w.os1 = p.in_map.os1; w.off = p.in_map.off; w.ss0 = p.ss0; w.ss1 = p.ss1; w.n1 = s[1];
+    w.row_bytes = (u32)p.wpr * 4; w.token_bytes = (u32)token_bytes; w.ss2 = (int)p.ss2; w.ss3 = (int)p.ss3;
+    w.octets = (int)p.octets_per_pair; w.c8 = p.c8; w.by_c8 = FastDiv::by(p.c8); w.by_g8 = FastDiv::by(table ? 1 : group / 8);
+    if (out_dtype == VARQ_F32) launch_words<VARQ_F32>(w, s, bits, table, st);
+    else if (out_dtype == VARQ_BF16) launch_words<VARQ_BF16>(w, s, bits, table, st);
+    else launch_words<VARQ_F16>(w, s, bits, table, st);
+    VARQ_CHECK_LAUNCH("dequant");
+    return VARQ_OK;
+  }
+  const int U = p.octets_per_pair >= 2048 ? 4 : 1;
+  const int64_t tiles = (p.octets_per_pair + 256 * U - 1) / (256 * U);
+  dim3 grid((unsigned)tiles, (unsigned)s[1], (unsigned)s[0]);
+#define VARQ_DEQ(ODT_)                                                                     \
+  do {                                                                                     \
+    if (U == 4) hipLaunchKernelGGL((dequant_kernel<ODT_, 4>), grid, dim3(256), 0, st, p);  \
+    else hipLaunchKernelGGL((dequant_kernel<ODT_, 1>), grid, dim3(256), 0, st, p);         \
   } while (0)
   if (out_dtype == VARQ_F32) VARQ_DEQ(VARQ_F32);
   else if (out_dtype == VARQ_BF16) VARQ_DEQ(VARQ_BF16);

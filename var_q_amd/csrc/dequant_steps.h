@@ -5,7 +5,14 @@
 
 namespace varq_deq {
 
-template <int ODT> __device__ __forceinline__ void store8(void *out, int64_t elem, const float (&f)[8], int n_valid) {
+typedef u32 u32x4 __attribute__((ext_vector_type(4)));
+
+template <bool STREAM, class T> __device__ __forceinline__ void put(T *at, T v) {
+  if constexpr (STREAM) __builtin_nontemporal_store(v, at);
+  else *at = v;
+}
+// STREAM: past the caches (whole octets only)
+template <int ODT, bool STREAM = false> __device__ __forceinline__ void store8(void *out, int64_t elem, const float (&f)[8], int n_valid) {
   if (ODT == VARQ_F32) {
     float *o = reinterpret_cast<float *>(out) + elem;
     if (n_valid == 8) {
@@ -26,15 +33,15 @@ template <int ODT> __device__ __forceinline__ void store8(void *out, int64_t ele
         const f2 v = {f[2 * j], f[2 * j + 1]};
         w[j] = __builtin_bit_cast(u32, __builtin_convertvector(v, bf2));
       }
-      *reinterpret_cast<uint4 *>(o) = make_uint4(w[0], w[1], w[2], w[3]);
+      put<STREAM>(reinterpret_cast<u32x4 *>(o), u32x4{w[0], w[1], w[2], w[3]});
       return;
     }
     uint16_t h[8];
 #pragma unroll
     for (int j = 0; j < 8; ++j) h[j] = (ODT == VARQ_BF16) ? f32_to_bf16_rne(f[j]) : f32_to_f16_rne(f[j]);
     if (n_valid == 8) {
-      *reinterpret_cast<uint4 *>(o) = make_uint4(h[0] | ((u32)h[1] << 16), h[2] | ((u32)h[3] << 16),
-                                                 h[4] | ((u32)h[5] << 16), h[6] | ((u32)h[7] << 16));
+      put<STREAM>(reinterpret_cast<u32x4 *>(o),
+                  u32x4{h[0] | ((u32)h[1] << 16), h[2] | ((u32)h[3] << 16), h[4] | ((u32)h[5] << 16), h[6] | ((u32)h[7] << 16)});
     } else {
       for (int j = 0; j < n_valid; ++j) o[j] = h[j];
     }
