@@ -193,10 +193,18 @@ __global__ __launch_bounds__(256) void quant_pack_rows_kernel(RowsParams p) {
 //
 // Rounding: x/s is needed exactly as an IEEE fp32 division rounds it; see the
 // two routes (fp32 correction step, fp64 product) in the kernel body.
+// The window is one of 16-byte pieces (one to an octet, two in 32 bits), each load instruction's 64 in a row; a lane's own lie 64 to 128 bytes from its neighbour's
+// where a group is 32 channels, on a few of the banks.  place() spreads them (the lowest three bits by the next ones, the
+// fourth by the seventh), which leaves runs of 16 pieces where they are.  (An octet of 32 bits in one lane, two loads of 16 bytes 32 apart, and the window in order,
+// before -> now, in a graph, us: fp32 [3,7,1511,96] in 4 bits, groups of 32, 4.84 -> 4.25, [4,16,2000,128] 15.5 -> 13.8, 8 bits in groups of 64 19.4 -> 16.7, [16,16,2000,128] groups of
+// 128 52.1 -> 49.6, 6.0 TB/s; fp16 [32,16,680,64] 8 bits 16.3 -> 15.8; 4 and 2 bits of 16-bit inputs the same.)
+__device__ __forceinline__ int place(int piece) { return piece ^ ((piece >> 3) & 7) ^ ((piece >> 3) & 8); }
+template <int DT> constexpr int kPieces = DT == VARQ_F32 ? 2 : 1;   // of an octet
+typedef u32 Piece __attribute__((ext_vector_type(4)));
 // Window `tile` of pair (i0, i1) of one tensor; stage: a wavefront-private window of 256 octets (in, then packed words out).
 template <int DT, int BITS, bool ASYM, int LPG4, bool DENSE>
 __device__ __forceinline__ void quant_window(const RowsParams &p, const void *px, int32_t *pwords, float *pscale, float *pzp, int64_t i0,
-                                             int64_t i1, int tile, int64_t out_base, Raw8<DT> *stage) {
+                                             int64_t i1, int tile, int64_t out_base, Piece *stage) {
   const int64_t pair_elem0 = i0 * p.in_s0 + i1 * p.in_s1;
 
   const int n_oct = (int)p.octets_per_pair;
@@ -205,29 +213,28 @@ __device__ __forceinline__ void quant_window(const RowsParams &p, const void *px
   const int w0 = tile * 1024 + wv * 256;             // first octet of this wave's window, inside the pair
 
   // 1 KiB per load instruction: contiguous, or whole rows in_s2 elements apart.  Only the
-  // offsets are formed under the (launch-uniform) branch; the four loads follow it together.
-  int64_t e[4];
+  // offsets are formed under the (launch-uniform) branch; the loads follow it together.
+  constexpr int PER = kPieces<DT>;
+  int64_t e[4 * PER];
   if (!p.strided) {
 #pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      const int o = w0 + k * 64 + lane;
+    for (int k = 0; k < 4 * PER; ++k) {
+      const int o = w0 + (k * 64 + lane) / PER;
       e[k] = (int64_t)(o < n_oct ? o : 0) * 8;          // past the end: re-read octet 0, never stored
     }
   } else {
     const int s2 = (int)p.in_s2;                        // (the pair's extent fits 31 bits: checked on the host)
 #pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      int o = w0 + k * 64 + lane;
+    for (int k = 0; k < 4 * PER; ++k) {
+      int o = w0 + (k * 64 + lane) / PER;
       o = o < n_oct ? o : 0;
       e[k] = (o >> p.c8_shift) * s2 + (o & (p.c8 - 1)) * 8;
     }
   }
+  const char *const first = reinterpret_cast<const char *>(px) + pair_elem0 * (2 * PER) + lane % PER * 16;
 #pragma unroll
-  for (int k = 0; k < 4; ++k) {
-    Raw8<DT> r;
-    r.load(px, pair_elem0 + e[k]);
-    stage[k * 64 + lane] = r;
-  }
+  for (int k = 0; k < 4 * PER; ++k)   // (streaming data, read exactly once)
+    stage[place(k * 64 + lane)] = __builtin_nontemporal_load(reinterpret_cast<const Piece *>(first + e[k] * (2 * PER)));
   __builtin_amdgcn_wave_barrier();
 
   // lane-owned octets inside the wave window
@@ -235,7 +242,12 @@ __device__ __forceinline__ void quant_window(const RowsParams &p, const void *px
   const int loc0 = ((lane - j) << 2) + j;
   float v[4][8];
 #pragma unroll
-  for (int k = 0; k < 4; ++k) stage[loc0 + k * LPG4].widen(v[k]);
+  for (int k = 0; k < 4; ++k) {
+    Piece raw[PER];
+#pragma unroll
+    for (int h = 0; h < PER; ++h) raw[h] = stage[place((loc0 + k * LPG4) * PER + h)];
+    __builtin_bit_cast(Raw8<DT>, raw).widen(v[k]);
+  }
 
   float mn = 0.f, mx;
   if (ASYM) {
@@ -337,17 +349,18 @@ __device__ __forceinline__ void quant_window(const RowsParams &p, const void *px
     // output rows of the pair are consecutive: word, scale and zp indices follow
     // the pair-local octet index directly
     if (BITS == 4) {
-      // packed words back to global order through the same window, 16 B per lane
-      typedef u32 u32x4 __attribute__((ext_vector_type(4)));
-      u32 *wstage = reinterpret_cast<u32 *>(stage);
-      __builtin_amdgcn_wave_barrier();
+      // packed words back to global order through the same window, 16 B per lane (groups of 32 channels are in order as they are)
+      Piece out4 = {w[0][0], w[1][0], w[2][0], w[3][0]};
+      if constexpr (LPG4 > 1) {
+        u32 *wstage = reinterpret_cast<u32 *>(stage);
+        __builtin_amdgcn_wave_barrier();
 #pragma unroll
-      for (int k = 0; k < 4; ++k) wstage[loc0 + k * LPG4] = w[k][0];
-      __builtin_amdgcn_wave_barrier();
-      const u32x4 out4 = reinterpret_cast<const u32x4 *>(wstage)[lane];
+        for (int k = 0; k < 4; ++k) wstage[loc0 + k * LPG4] = w[k][0];
+        __builtin_amdgcn_wave_barrier();
+        out4 = stage[lane];
+      }
       const int o = w0 + 4 * lane;                    // octet == word index for 4-bit codes
-      if (o < n_oct)
-        __builtin_nontemporal_store(out4, reinterpret_cast<u32x4 *>(pwords + out_base * p.c8 + o));
+      if (o < n_oct) __builtin_nontemporal_store(out4, reinterpret_cast<Piece *>(pwords + out_base * p.c8 + o));
     } else if (live) {
       const int64_t wbase = out_base * p.c8 + oct0;   // in octets
       if (BITS == 8) {
@@ -407,7 +420,7 @@ __device__ __forceinline__ void quant_window(const RowsParams &p, const void *px
 
 template <int DT, int BITS, bool ASYM, int LPG4, bool DENSE>
 __global__ __launch_bounds__(256) void quant_pack_rows32_kernel(RowsParams p) {
-  __shared__ Raw8<DT> lds_stage[4][256];
+  __shared__ Piece lds_stage[4][256 * kPieces<DT>];
   const bool second = blockIdx.z >= (unsigned)p.map.n0;   // block-uniform
   const int64_t i0 = blockIdx.z - (second ? (unsigned)p.map.n0 : 0u), i1 = p.strided ? blockIdx.x : blockIdx.y;
   int64_t s0 = i0, s1 = i1;
@@ -426,7 +439,7 @@ __global__ __launch_bounds__(256) void quant_pack_rows32_kernel(RowsParams p) {
 // 4.3 us, [8,16,1024,128] 28.4 -> 20.1, [8,16,4096,128] 79 -> 64.)
 template <int DT, bool ASYM, int LPG4>
 __global__ __launch_bounds__(256) void quant_pack_classes_kernel(RowsParams p, ClassOuts t) {
-  __shared__ Raw8<DT> lds_stage[4][256];
+  __shared__ Piece lds_stage[4][256 * kPieces<DT>];
   const bool second = blockIdx.z >= (unsigned)p.map.n0;   // block-uniform
   const int64_t i0 = blockIdx.z - (second ? (unsigned)p.map.n0 : 0u), i1 = p.strided ? blockIdx.x : blockIdx.y;
   const bool is_v = second || !p.x;
