@@ -1562,9 +1562,9 @@ struct KeyShares { int waves, splits; };
 // takes is 0.5 % behind the best of all on the geometric mean and 9 % ahead of workgroups alone, and in 5 of them behind those by more than 2.5 %.  4 bits in groups,
 // us, workgroups alone / this: D=128, 32 pairs, 256 queries x 521 keys 22.6 / 16.5, 400 x 921 32.4 / 22.8, 64 pairs, 144 x 300 16.8 / 12.0, 256 x 521
 // 27.2 / 17.4, 400 x 921 40.9 / 30.5, 128 pairs, 256 x 521 28.6 / 22.8; D=64, 32 pairs, 256 x 521 15.7 / 11.6, 1024 x 2521 50.1 / 43.4, 128 pairs, 256 x 521 19.1 / 15.1.
-KeyShares choose_shares(int64_t bh, int Lq, int Lk, int D, int most_waves) {
+KeyShares choose_shares(int64_t bh, int Lq, int Lk, int D, int most_waves, int cus = device_cus()) {
   static const double tile_us[2][3] = {{1.45, 0.85, 1.1}, {2.07, 1.35, 1.9}};
-  const double per_xcd = device_cus() / 8.0;
+  const double per_xcd = cus / 8.0;
   const bool wide = D == 128;
   KeyShares best = {1, 1};
   double best_us = 0.0;
@@ -1724,16 +1724,17 @@ bool wide_eligible(int B, int Hkv, int Lq, int Lk, int D, bool limits) {
 // limits.  4 bits in groups, us, before / this: D=64, 2 pairs x 4500 tokens 52.7 / 31, 16 x 300 12.4 / 9.0, x 680 17.6 / 12.4, x 1500 29.1 / 24.6, 32 x 524 17.2 / 12.9, 48 x 1000 27.3 / 23.0;
 // D=128, 2 x 4500 93 / 46, 16 x 680 24.8 / 17.3, 24 x 600 24.6 / 16.6, x 1000 33.9 / 28.9, 32 x 854 34.0 / 27.1, 90 x 249 16.7 / 13.7.
 KeyShares limited_shares(int B, int Hkv, int Lq, int Lk, int D, int most, bool may_expand) {
+  const int cus = device_cus();   // (asked once: it is a call into the runtime)
   const int64_t bh = (int64_t)B * Hkv;
-  const bool four = may_expand && wide_four((int64_t)wide_batch(B, Hkv, Lk, D) * Hkv, Lq, Lk, D, device_cus(), true);
+  const bool four = may_expand && wide_four((int64_t)wide_batch(B, Hkv, Lk, D) * Hkv, Lq, Lk, D, cus, true);
   if (may_expand && !four && wide_eligible(B, Hkv, Lq, Lk, D, true)) return {0, 1};
-  if (Lq <= 128 || Lk <= 128) return {1, most == 1 ? 1 : choose_shares(bh, Lq, Lk, D, 1).splits};
+  if (Lq <= 128 || Lk <= 128) return {1, most == 1 ? 1 : choose_shares(bh, Lq, Lk, D, 1, cus).splits};
   struct Cost { double tile, fixed, again, load; };   // us of a tile, of a workgroup, of one that is not the longest; of the whole load
   static const Cost cost[2][3] = {{{1.32, 5.8, 4.7, 0.9}, {0.87, 6.0, 4.9, 1.03}, {1.15, 5.6, 4.6, 1.03}}, {{2.1, 4.7, 3.8, 1.0}, {1.4, 6.6, 5.4, 1.14}, {1.9, 6.1, 5.0, 1.14}}};
   static const Cost expanded[2] = {{0.9, 10.0, 4.0, 0.92}, {1.4, 14.0, 4.0, 0.95}};
   auto us = [&](const Cost &c, int block, int keys, int n) {
     const double blocks = (Lq + block - 1) / block, part = std::floor(0.8 * blocks), tiles = (double)Lk / keys * (1.25 * part * (part + 1.0) / (2.0 * blocks) + blocks - part) + 0.5 * blocks;
-    const double longest = c.fixed + c.tile * (((Lk + keys - 1) / keys + n - 1) / n), load = c.load * (double)bh * (blocks * n * c.again + tiles * c.tile) / device_cus();
+    const double longest = c.fixed + c.tile * (((Lk + keys - 1) / keys + n - 1) / n), load = c.load * (double)bh * (blocks * n * c.again + tiles * c.tile) / cus;
     const double two = longest * longest, four = load * load;
     return std::sqrt(std::sqrt(two * two + four * four));
   };
@@ -1819,7 +1820,13 @@ extern "C" size_t varq_fused_attn_workspace_bytes(int B, int Hkv, int Lq, int Lk
   (void)nseg;   // (the tile count does not depend on the tables)
   const int64_t bh = (int64_t)B * Hkv;
   // (whether there will be key limits is not known here)
-  int n = splits ? splits : std::max({choose_shares(bh, Lq, Lk, D, 4).splits, choose_shares(bh, Lq, Lk, D, 1).splits, limited_shares(B, Hkv, Lq, Lk, D, kLimitedSplits, false).splits});
+  int n = splits;
+  if (!splits) {   // (every call asks: up to 128 queries or keys what wavefronts share, and what the limits say, come to the same as this)
+    const int cus = device_cus();
+    n = choose_shares(bh, Lq, Lk, D, 1, cus).splits;
+    if (Lq > 128 && Lk > BN) n = std::max(n, choose_shares(bh, Lq, Lk, D, 4, cus).splits);
+    if (Lq > 128 && Lk > 128) n = std::max(n, limited_shares(B, Hkv, Lq, Lk, D, kLimitedSplits, false).splits);
+  }
   // (the group sizes are not known here: room for the few-queries kernel's shares whenever the
   // other sizes would admit it)
   if (splits == 0 && fewq_eligible(B, Hkv, Lq, Lk, D, D, D)) n = max(n, fewq_shares(B * Hkv, Lq, Lk, D, D, D));
