@@ -216,7 +216,8 @@ template <int ODT> void launch_words(const WordsParams &w, const int64_t *s, int
 
 template <int ODT, int BITS>
 __global__ __launch_bounds__(256) void dequant_steps_kernel(StepParams p) {
-  dequant_steps_block<ODT, BITS, 256, 4>(p, (int64_t)blockIdx.z * gridDim.y + blockIdx.y, blockIdx.x);
+  if constexpr (ODT == VARQ_F32) dequant_steps_halves<BITS, 256, 4>(p, (int64_t)blockIdx.z * gridDim.y + blockIdx.y, blockIdx.x);
+  else dequant_steps_block<ODT, BITS, 256, 4>(p, (int64_t)blockIdx.z * gridDim.y + blockIdx.y, blockIdx.x);
 }
 
 }  // namespace

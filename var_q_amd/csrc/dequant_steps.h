@@ -67,6 +67,14 @@ struct StepParams {
   int seg_oct[16];                 // first octet of a pair that is past segment s
 };
 
+// the step that octet o lies in (those past the last one end where the pair does)
+__device__ __forceinline__ int step_of(const StepParams &p, int o) {
+  int seg = 0;
+#pragma unroll
+  for (int s = 0; s < 15; ++s) seg += o >= p.seg_oct[s] ? 1 : 0;
+  return seg;
+}
+
 // Block `block` of pair `pair`: NT threads, U octets each, all of whose loads are under way before the first is used.  (One octet after the other, each
 // with its search for the step in LDS and a trip for its scales, a workgroup was a chain of some 4 us, and what the launches of
 // a schedule took: [8,n,30,64], ten steps to fp32, 173 -> 169 us.)
@@ -76,12 +84,7 @@ __device__ __forceinline__ void dequant_steps_block(const StepParams &p, int64_t
   const float *scale = p.scale + (p.head_in_pair ? (pair % p.H) * p.c : 0);
   const float *zp = p.zp ? p.zp + (p.head_in_pair ? (pair % p.H) * p.c : 0) : nullptr;
   const int first = block * (NT * U), last = (int)p.pair_octs - 1, o0 = first + threadIdx.x;
-  auto segment = [&](int o) __attribute__((always_inline)) {   // (those past the last one end where the pair does)
-    int seg = 0;
-#pragma unroll
-    for (int s = 0; s < 15; ++s) seg += o >= p.seg_oct[s] ? 1 : 0;
-    return seg;
-  };
+  auto segment = [&](int o) __attribute__((always_inline)) { return step_of(p, o); };
   // most blocks lie in one step
   const int seg0 = segment(first);
   const bool one_seg = seg0 == segment(min(first + NT * U - 1, last));
@@ -123,6 +126,51 @@ __device__ __forceinline__ void dequant_steps_block(const StepParams &p, int64_t
       for (int j = 0; j < 8; ++j) f[j] = f[j] * sv[j];
     }
     store8<ODT>(p.out, (pair * p.out_pair_octs + o) * 8, f, 8);
+  }
+}
+
+// The same to 32 bits, by pieces of 16 bytes: a wavefront stores 1 KiB with each, where an octet takes two stores 32 bytes apart.  All tokens of ten steps, in a
+// graph, us, by octets / by pieces: [8,680,30,64] 8 bits 12.3 / 10.0, 4 bits affine 12.7 / 10.5, [32,30,680,64] 37.0 / 34.2, [2,16,680,128] 2 bits affine 6.5 both.  Beside workgroups
+// that quantize, whose stores are octets by their groups, twice the loads cost more (the ten steps of [8,n,30,64] one by one 167.4 / 169.9).
+template <int BITS, int NT, int U>
+__device__ __forceinline__ void dequant_steps_halves(const StepParams &p, int64_t pair, int block) {
+  constexpr int N = 2 * U;   // pieces of a lane
+  typedef float f4 __attribute__((ext_vector_type(4)));
+  const char *const words = reinterpret_cast<const char *>(p.words + pair * p.pair_words);
+  const int64_t head = p.head_in_pair ? (pair % p.H) * p.c : 0;
+  const float *const scale = p.scale + head, *const zp = p.zp ? p.zp + head : nullptr;
+  const int first = block * (NT * U), last = (int)p.pair_octs - 1, o0 = first + (int)threadIdx.x / 2, half = threadIdx.x & 1;
+  const int seg0 = step_of(p, first);
+  const bool one_seg = seg0 == step_of(p, min(first + NT * U - 1, last));
+  u32 w[N];
+  int64_t at[N];
+#pragma unroll
+  for (int u = 0; u < N; ++u) {
+    const int o = min(o0 + u * (NT / 2), last);
+    const char *const src = words + ((int64_t)o * 2 + half) * (BITS / 2);
+    if constexpr (BITS == 8) w[u] = *reinterpret_cast<const u32 *>(src);
+    else if constexpr (BITS == 4) w[u] = *reinterpret_cast<const uint16_t *>(src);
+    else w[u] = *reinterpret_cast<const unsigned char *>(src);
+    at[u] = seg0 * p.row + (int)((u32)o - p.by_octs((u32)o) * (u32)p.octs) * 8 + half * 4;
+    if (!one_seg) at[u] += (step_of(p, o) - seg0) * p.row;
+  }
+  f4 s[N], z[N];
+#pragma unroll
+  for (int u = 0; u < N; ++u) {
+    s[u] = *reinterpret_cast<const f4 *>(scale + at[u]);
+    if (zp) z[u] = *reinterpret_cast<const f4 *>(zp + at[u]);
+  }
+#pragma unroll
+  for (int u = 0; u < N; ++u) {
+    const int o = o0 + u * (NT / 2);
+    if (o > last) return;
+    f4 f;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const float q = (float)(int)__builtin_amdgcn_sbfe((int)w[u], BITS * j, BITS);
+      f[j] = zp ? (q - z[u][j]) * s[u][j] : q * s[u][j];
+    }
+    reinterpret_cast<f4 *>(p.out)[(pair * p.out_pair_octs + o) * 2 + half] = f;
   }
 }
 
