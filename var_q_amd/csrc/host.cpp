@@ -960,10 +960,13 @@ PyObject *quantizer_use(PyObject *const *a) {
   at::Tensor out;
   auto new_out = [&] { return d == 1 ? empty({B, len, H, c}, dtype_of((int)code), x) : empty({B, H, len, c}, dtype_of((int)code), x); };
   if (!rows) {   // the rules whose scales are not a row of the tables: the step, and the launch that dequantizes what they read
+    // (what that launch would refuse, and a result that there is no room for, before the step is in the cache: a caller may try it again)
+    if (B > 65535 || (d == 2 ? H : tokens ? len : 1) > 65535)
+      raise(g_varq_error, "use_var_q: shape [%lld,%lld,%lld,%lld] exceeds the grid limits", (long long)B, (long long)(d == 1 ? len : H), (long long)(d == 1 ? H : len), (long long)c);
+    status_unlocked([&] { out = new_out(); return (int)VARQ_OK; });
     PyObject *const step[4] = {a[0], a[1], Py_None, Py_None};
     if (!take_step(z, step)) Py_RETURN_NONE;
     unlocked("varq_dequant", [&] {
-      out = new_out();
       const int64_t cap = z.buf->size(d);
       if (!tokens)
         return varq_dequant_steps(ptr<int32_t>(z.buf), ptr<float>(z.scale), ptr<float>(z.zp), (int)z.k + 1, ends, (int)B, (int)H, cap, (int)c, (int)z.bits, d == 1,
