@@ -327,6 +327,8 @@ int varq_quant_step_dequant(const void *x, int x_dtype, int B, int H, int n, int
  * dividing D.
  */
 size_t varq_fused_attn_workspace_bytes(int B, int Hkv, int Lq, int Lk, int D, int nseg, int splits);
+/* The same for a call in the default operand form that is known to have a kv_limit (limits != 0) or none: no more than that, and asked faster. */
+size_t varq_fused_attn_workspace_bytes_call(int B, int Hkv, int Lq, int Lk, int D, int nseg, int splits, int limits);
 /* Many queries over a long cache (five or more blocks of 256 per (batch, head); with key limits also a whole
  * sequence of few (batch, head) pairs): given a workspace of
  * this many bytes and splits = 0 or 1, the attention entry points dequantize K and V once into matrix

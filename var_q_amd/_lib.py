@@ -55,6 +55,7 @@ SYMBOLS = {
                                 c_int, c_int, c_int, c_int,
                                 c_void_p, c_float, c_int, c_int, c_int, c_void_p, c_size_t, c_int, c_void_p]),
     'varq_fused_attn_workspace_bytes': (c_size_t, [c_int, c_int, c_int, c_int, c_int, c_int, c_int]),
+    'varq_fused_attn_workspace_bytes_call': (c_size_t, [c_int] * 8),
     'varq_fused_attn_expand_bytes': (c_size_t, [c_int, c_int, c_int, c_int, c_int]),
     'varq_fused_attn_expand_bytes_limits': (c_size_t, [c_int, c_int, c_int, c_int, c_int]),
     'varq_fused_attn_key_shares': (c_int, [c_int, c_int, c_int, c_int, c_int, c_int, c_int]),

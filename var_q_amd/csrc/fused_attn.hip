@@ -1562,7 +1562,8 @@ struct KeyShares { int waves, splits; };
 // takes is 0.5 % behind the best of all on the geometric mean and 9 % ahead of workgroups alone, and in 5 of them behind those by more than 2.5 %.  4 bits in groups,
 // us, workgroups alone / this: D=128, 32 pairs, 256 queries x 521 keys 22.6 / 16.5, 400 x 921 32.4 / 22.8, 64 pairs, 144 x 300 16.8 / 12.0, 256 x 521
 // 27.2 / 17.4, 400 x 921 40.9 / 30.5, 128 pairs, 256 x 521 28.6 / 22.8; D=64, 32 pairs, 256 x 521 15.7 / 11.6, 1024 x 2521 50.1 / 43.4, 128 pairs, 256 x 521 19.1 / 15.1.
-KeyShares choose_shares(int64_t bh, int Lq, int Lk, int D, int most_waves, int cus = device_cus()) {
+// alone: what workgroups alone would be, where that is asked too (it is what the first round of the loop ends with).
+KeyShares choose_shares(int64_t bh, int Lq, int Lk, int D, int most_waves, int cus, KeyShares *alone = nullptr) {
   static const double tile_us[2][3] = {{1.45, 0.85, 1.1}, {2.07, 1.35, 1.9}};
   const double per_xcd = cus / 8.0;
   const bool wide = D == 128;
@@ -1572,7 +1573,8 @@ KeyShares choose_shares(int64_t bh, int Lq, int Lk, int D, int most_waves, int c
     // (a single tile has nothing to share; and what up to 128 queries, the first steps of a schedule, come to does not go by how many pairs a launch has,
     // which would gain up to a tenth in tables: 64 queries x 600 keys, 128 pairs, D=64 15.9 / 13.5, D=128 20.8 / 18.7)
     if (waves > 1 && (Lk <= BN || Lq <= 128)) break;
-    const int64_t tiles = (Lk + (waves == 4 ? 2 * BN : BN) - 1) / (waves == 4 ? 2 * BN : BN), blocks = bh * ((Lq + BM / waves - 1) / (BM / waves));
+    const int tiles = (Lk + (waves == 4 ? 2 * BN : BN) - 1) / (waves == 4 ? 2 * BN : BN);
+    const int64_t blocks = bh * ((Lq + BM / waves - 1) / (BM / waves));
     // (up to 128 queries half of the wavefronts have none, and widen only)
     const double tile = tile_us[wide][i] * (waves == 1 && Lq <= 128 ? 0.7 : 1.0), fixed = (wide ? 2.8 : 2.2) + (waves > 1 ? 1.1 : 0.0);
     for (int n = 1; n <= kMaxSplits; ++n) {
@@ -1581,29 +1583,32 @@ KeyShares choose_shares(int64_t bh, int Lq, int Lk, int D, int most_waves, int c
       if (n > 1) us += 2.4 + 2.0 * (double)split_workspace_bytes(n, bh * Lq, D) / 4.4e6;   // written and read
       if ((waves == 1 && n == 1) || us < best_us) { best_us = us; best = {waves, n}; }
     }
+    if (waves == 1 && alone) *alone = best;
   }
   return best;
 }
 // Fills the fields of the shares of p from the caller's request.  splits: 0 = as the model above
 // says, reduced to what the workspace holds; 1 = none; 2..8 = exactly that many.  limited: what limited_shares says, or null.
+// (The device is asked for once, and the model too: every step of a schedule pays for it.)
 int set_splits(AttnParams &p, int D, int most_waves, const KeyShares *limited, int splits, void *workspace, size_t workspace_bytes, const char *who) {
   p.nsplit = 1; p.ws_o = nullptr; p.ws_ml = nullptr;
   p.key_waves = 1;
   if (splits < 0 || splits > kMaxSplits)
     return varq_set_error(VARQ_ERR_INVALID, "%s: splits must be 0 (automatic) or 1..%d (got %d)", who, kMaxSplits, splits);
   const int64_t rows = (int64_t)p.bh_total * p.Lq;
-  // (a workspace that cannot be used is an error wherever workgroups alone would use it)
-  if (splits == 0 && workspace && ((uintptr_t)workspace & 15) && workspace_bytes >= split_workspace_bytes(2, rows, D) && choose_shares(p.bh_total, p.Lq, p.Lk, D, 1).splits > 1)
-    return varq_set_error(VARQ_ERR_INVALID, "%s: the workspace must be 16-byte aligned", who);
+  const bool unaligned = workspace && ((uintptr_t)workspace & 15);
   int n = splits;
+  KeyShares alone = {1, 1}, k = {1, 1};
+  if (splits == 0 && (!limited || unaligned)) k = choose_shares(p.bh_total, p.Lq, p.Lk, D, limited ? 1 : most_waves, device_cus(), &alone);
+  // (a workspace that cannot be used is an error wherever workgroups alone would use it)
+  if (unaligned && alone.splits > 1 && workspace_bytes >= split_workspace_bytes(2, rows, D))
+    return varq_set_error(VARQ_ERR_INVALID, "%s: the workspace must be 16-byte aligned", who);
   if (limited) {
     p.key_waves = limited->waves;
     n = limited->splits;
   } else if (splits == 0) {
-    KeyShares k = choose_shares(p.bh_total, p.Lq, p.Lk, D, 1);
-    n = k.splits;
-    if (most_waves > 1) k = choose_shares(p.bh_total, p.Lq, p.Lk, D, most_waves);
-    if (k.waves > 1 && (k.splits == 1 || (workspace && workspace_bytes >= split_workspace_bytes(k.splits, rows, D)))) {
+    n = alone.splits;
+    if (k.waves > 1 && (k.splits == 1 || (workspace && !unaligned && workspace_bytes >= split_workspace_bytes(k.splits, rows, D)))) {
       p.key_waves = k.waves;
       n = k.splits;
     }
@@ -1711,10 +1716,10 @@ int wide_batch(int B, int Hkv, int Lk, int D) {
 // a block and a quarter per compute unit, 16 x 2521 62.6 / 56.8, 24 x 3256 84.5 / 76.8 (though 16 x 4121 85.6 / 88.2), and in long sequences,
 // 32 x 6425 322 / 272, 128 x 6425 1142 / 1050; in between it goes either way, 32 x 3256 89.5 / 100, 128 x 4121 513 / 489,
 // 320 x 2952 645 / 683, 48 x 5417 328 / 319.  (Few pairs: wide_four.)
-bool wide_eligible(int B, int Hkv, int Lq, int Lk, int D, bool limits) {
+bool wide_eligible(int B, int Hkv, int Lq, int Lk, int D, bool limits, int cus = device_cus()) {
   const int64_t bh = (int64_t)wide_batch(B, Hkv, Lk, D) * Hkv, blocks = bh * ((Lq + 255) / 256);
-  if (bh > 0 && wide_four(bh, Lq, Lk, D, device_cus(), limits)) return true;
-  if (limits && D == 64 && Lq < 6144 && blocks > device_cus() * 5 / 4) return false;
+  if (bh > 0 && wide_four(bh, Lq, Lk, D, cus, limits)) return true;
+  if (limits && D == 64 && Lq < 6144 && blocks > cus * 5 / 4) return false;
   return Lq >= (D == 128 ? 1280 : 1536) && Lk >= 2048 && blocks >= 160 && bh <= 65535;
 }
 // Under key limits, whose blocks end at different keys that only the device knows; taken for a sequence's own, of which a block sees a quarter
@@ -1723,11 +1728,10 @@ bool wide_eligible(int B, int Hkv, int Lq, int Lk, int D, bool limits) {
 // every choice: 1.2 % behind the best on the geometric mean, 18 % ahead of the rules before, blocks of 128 queries for few pairs (wide_four) and shares as without
 // limits.  4 bits in groups, us, before / this: D=64, 2 pairs x 4500 tokens 52.7 / 31, 16 x 300 12.4 / 9.0, x 680 17.6 / 12.4, x 1500 29.1 / 24.6, 32 x 524 17.2 / 12.9, 48 x 1000 27.3 / 23.0;
 // D=128, 2 x 4500 93 / 46, 16 x 680 24.8 / 17.3, 24 x 600 24.6 / 16.6, x 1000 33.9 / 28.9, 32 x 854 34.0 / 27.1, 90 x 249 16.7 / 13.7.
-KeyShares limited_shares(int B, int Hkv, int Lq, int Lk, int D, int most, bool may_expand) {
-  const int cus = device_cus();   // (asked once: it is a call into the runtime)
+KeyShares limited_shares(int B, int Hkv, int Lq, int Lk, int D, int most, bool may_expand, int cus) {
   const int64_t bh = (int64_t)B * Hkv;
   const bool four = may_expand && wide_four((int64_t)wide_batch(B, Hkv, Lk, D) * Hkv, Lq, Lk, D, cus, true);
-  if (may_expand && !four && wide_eligible(B, Hkv, Lq, Lk, D, true)) return {0, 1};
+  if (may_expand && !four && wide_eligible(B, Hkv, Lq, Lk, D, true, cus)) return {0, 1};
   if (Lq <= 128 || Lk <= 128) return {1, most == 1 ? 1 : choose_shares(bh, Lq, Lk, D, 1, cus).splits};
   struct Cost { double tile, fixed, again, load; };   // us of a tile, of a workgroup, of one that is not the longest; of the whole load
   static const Cost cost[2][3] = {{{1.32, 5.8, 4.7, 0.9}, {0.87, 6.0, 4.9, 1.03}, {1.15, 5.6, 4.6, 1.03}}, {{2.1, 4.7, 3.8, 1.0}, {1.4, 6.6, 5.4, 1.14}, {1.9, 6.1, 5.0, 1.14}}};
@@ -1795,47 +1799,60 @@ class Limited {
 
  public:
   Limited(const AttnParams &p_, int B_, int D_, int splits) : p(p_), B(B_), D(D_), most(!p_.kv_limit || splits > 1 ? 0 : splits == 1 ? 1 : kLimitedSplits) {
-    if (most) k = limited_shares(B, p.Hkv, p.Lq, p.Lk, D, most, true);
+    if (most) k = limited_shares(B, p.Hkv, p.Lq, p.Lk, D, most, true, device_cus());
   }
   bool expands() const { return k.waves == 0; }   // (or is not asked)
   const KeyShares *shares() {
     if (!most) return nullptr;
-    if (k.waves == 0) k = limited_shares(B, p.Hkv, p.Lq, p.Lk, D, most, false);
+    if (k.waves == 0) k = limited_shares(B, p.Hkv, p.Lq, p.Lk, D, most, false, device_cus());
     return &k;
   }
 };
 
 size_t expand_bytes(int B, int Hkv, int Lq, int Lk, int D, bool limits) {
-  if (B <= 0 || Hkv <= 0 || Lq <= 0 || Lk <= 0 || (D != 64 && D != 128) || !wide_eligible(B, Hkv, Lq, Lk, D, limits) ||
-      (limits && limited_shares(B, Hkv, Lq, Lk, D, kLimitedSplits, true).waves))
-    return 0;
+  if (B <= 0 || Hkv <= 0 || Lq <= 0 || Lk <= 0 || (D != 64 && D != 128)) return 0;
+  const int cus = device_cus();   // (a call into the runtime)
+  if (!wide_eligible(B, Hkv, Lq, Lk, D, limits, cus) || (limits && limited_shares(B, Hkv, Lq, Lk, D, kLimitedSplits, true, cus).waves)) return 0;
   return wide_bytes(B, Hkv, Lq, Lk, D, true, limits);
 }
 
 }  // namespace
 
-extern "C" size_t varq_fused_attn_workspace_bytes(int B, int Hkv, int Lq, int Lk, int D, int nseg, int splits) {
+namespace {
+// Bytes for the shares of a call without key limits, with them, or either and in any operand form.
+enum { kPlain = 1, kLimits = 2 };
+size_t shares_bytes(int B, int Hkv, int Lq, int Lk, int D, int splits, int of) {
   if (B <= 0 || Hkv <= 0 || Lq <= 0 || Lk <= 0 || (D != 64 && D != 128) || splits < 0 || splits > kMaxSplits) return 0;
-  const int64_t rows = (int64_t)B * Hkv * Lq;
-  (void)nseg;   // (the tile count does not depend on the tables)
-  const int64_t bh = (int64_t)B * Hkv;
-  // (whether there will be key limits is not known here)
+  const int64_t bh = (int64_t)B * Hkv, rows = bh * Lq;
   int n = splits;
-  if (!splits) {   // (every call asks: up to 128 queries or keys what wavefronts share, and what the limits say, come to the same as this)
+  if (!splits) {   // (every call asks: up to 128 queries or keys what wavefronts share, and what the limits say, come to the same as workgroups alone)
     const int cus = device_cus();
-    n = choose_shares(bh, Lq, Lk, D, 1, cus).splits;
-    if (Lq > 128 && Lk > BN) n = std::max(n, choose_shares(bh, Lq, Lk, D, 4, cus).splits);
-    if (Lq > 128 && Lk > 128) n = std::max(n, limited_shares(B, Hkv, Lq, Lk, D, kLimitedSplits, false).splits);
+    const bool waves = of & kPlain && Lq > 128 && Lk > BN, limits = of & kLimits && Lq > 128 && Lk > 128;
+    KeyShares alone = {1, 1};
+    if (limits) n = limited_shares(B, Hkv, Lq, Lk, D, kLimitedSplits, false, cus).splits;
+    if (!limits || of & kPlain) n = std::max(n, choose_shares(bh, Lq, Lk, D, waves ? 4 : 1, cus, &alone).splits);
+    if (of == (kPlain | kLimits)) n = std::max(n, alone.splits);   // (the form with exact codes has no shares of wavefronts)
+    // (the group sizes are not known here: room for the few-queries kernel's shares whenever the
+    // other sizes would admit it)
+    if (fewq_eligible(B, Hkv, Lq, Lk, D, D, D)) n = std::max(n, fewq_shares(B * Hkv, Lq, Lk, D, D, D));
   }
-  // (the group sizes are not known here: room for the few-queries kernel's shares whenever the
-  // other sizes would admit it)
-  if (splits == 0 && fewq_eligible(B, Hkv, Lq, Lk, D, D, D)) n = max(n, fewq_shares(B * Hkv, Lq, Lk, D, D, D));
   return split_workspace_bytes(n, rows, D);
+}
+}  // namespace
+
+extern "C" size_t varq_fused_attn_workspace_bytes(int B, int Hkv, int Lq, int Lk, int D, int nseg, int splits) {
+  (void)nseg;   // (the tile count does not depend on the tables)
+  return shares_bytes(B, Hkv, Lq, Lk, D, splits, kPlain | kLimits);
+}
+extern "C" size_t varq_fused_attn_workspace_bytes_call(int B, int Hkv, int Lq, int Lk, int D, int nseg, int splits, int limits) {
+  (void)nseg;
+  return shares_bytes(B, Hkv, Lq, Lk, D, splits, limits ? kLimits : kPlain);
 }
 
 extern "C" int varq_fused_attn_key_waves(int B, int Hkv, int Lq, int Lk, int D, int limits) {
   if (B <= 0 || Hkv <= 0 || Lq <= 0 || Lk <= 0 || (D != 64 && D != 128)) return -1;
-  return limits ? limited_shares(B, Hkv, Lq, Lk, D, kLimitedSplits, true).waves : choose_shares((int64_t)B * Hkv, Lq, Lk, D, 4).waves;
+  const int cus = device_cus();
+  return limits ? limited_shares(B, Hkv, Lq, Lk, D, kLimitedSplits, true, cus).waves : choose_shares((int64_t)B * Hkv, Lq, Lk, D, 4, cus).waves;
 }
 
 extern "C" size_t varq_fused_attn_expand_bytes(int B, int Hkv, int Lq, int Lk, int D) {
@@ -1846,7 +1863,7 @@ extern "C" size_t varq_fused_attn_expand_bytes_limits(int B, int Hkv, int Lq, in
 extern "C" int varq_fused_attn_key_shares(int B, int Hkv, int Lq, int Lk, int D, int k_group, int v_group) {
   if (B <= 0 || Hkv <= 0 || Lq <= 0 || Lk <= 0 || (D != 64 && D != 128)) return 0;
   if (fewq_eligible(B, Hkv, Lq, Lk, D, k_group, v_group)) return fewq_shares(B * Hkv, Lq, Lk, D, k_group, v_group);
-  return choose_shares((int64_t)B * Hkv, Lq, Lk, D, 4).splits;
+  return choose_shares((int64_t)B * Hkv, Lq, Lk, D, 4, device_cus()).splits;
 }
 
 extern "C" int varq_fused_attn(const void *q, void *out,

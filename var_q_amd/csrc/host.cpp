@@ -367,9 +367,10 @@ void check_limit_and_map(const at::Tensor *limit, const at::Tensor *map, const A
 int io_code(const at::Tensor &q) { return q.scalar_type() == at::kHalf ? VARQ_F16 : VARQ_BF16; }
 
 // Device memory for a launch that shares keys out or expands them (undefined: neither).  Expanding takes more the longer the
-// cache is; where the device has no room for it the call does without.
+// cache is; where the device has no room for it the call does without.  expands: the default operand form.
 at::Tensor workspace(const AttnShape &s, const at::Tensor &q, int64_t Lk, int nseg, int64_t splits, bool limits, bool expands = true) {
-  const size_t shared = varq_fused_attn_workspace_bytes((int)s.B, (int)s.Hkv, (int)s.Lq, (int)Lk, (int)s.D, nseg, (int)splits);
+  const size_t shared = expands ? varq_fused_attn_workspace_bytes_call((int)s.B, (int)s.Hkv, (int)s.Lq, (int)Lk, (int)s.D, nseg, (int)splits, limits)
+                                : varq_fused_attn_workspace_bytes((int)s.B, (int)s.Hkv, (int)s.Lq, (int)Lk, (int)s.D, nseg, (int)splits);
   const auto bytes = limits ? varq_fused_attn_expand_bytes_limits : varq_fused_attn_expand_bytes;
   const size_t expanded = expands && splits <= 1 ? bytes((int)s.B, (int)s.Hkv, (int)s.Lq, (int)Lk, (int)s.D) : 0;
   if (expanded > shared) {
