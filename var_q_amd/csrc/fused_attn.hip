@@ -1600,12 +1600,12 @@ int set_splits(AttnParams &p, int D, int most_waves, const KeyShares *limited, i
   int n = splits;
   KeyShares alone = {1, 1}, k = {1, 1};
   if (splits == 0 && (!limited || unaligned)) k = choose_shares(p.bh_total, p.Lq, p.Lk, D, limited ? 1 : most_waves, device_cus(), &alone);
-  // (a workspace that cannot be used is an error wherever workgroups alone would use it)
+  // (a workspace that cannot be used is an error wherever workgroups alone would use it, and is not used otherwise)
   if (unaligned && alone.splits > 1 && workspace_bytes >= split_workspace_bytes(2, rows, D))
     return varq_set_error(VARQ_ERR_INVALID, "%s: the workspace must be 16-byte aligned", who);
   if (limited) {
     p.key_waves = limited->waves;
-    n = limited->splits;
+    n = unaligned ? 1 : limited->splits;
   } else if (splits == 0) {
     n = alone.splits;
     if (k.waves > 1 && (k.splits == 1 || (workspace && !unaligned && workspace_bytes >= split_workspace_bytes(k.splits, rows, D)))) {
