@@ -1,5 +1,5 @@
 /*
- * varq_testing.h -- entry points of libvarq_hip.so that its tests need to reach and to recognise paths of varq_quant_pack and of the attention.  They are not part
+ * varq_testing.h -- entry points of libvarq_hip.so that its tests need to reach and to recognise paths of varq_quant_pack, of the attention and of packing.  They are not part
  * of the interface and may change with any build; the conventions are those of varq.h.
  */
 #ifndef VARQ_TESTING_H
@@ -30,6 +30,13 @@ int varq_quant_pack_shards(const int64_t *host_shape4, int reduce_mask, int x_dt
  * the kernel that widens per workgroup serves the call: 1, 2 or 4; 0: with these key limits K and V are expanded instead. limits: whether there are key limits.
  */
 int varq_fused_attn_key_waves(int B, int Hkv, int Lq, int Lk, int D, int limits);
+
+/*
+ * varq_pack and varq_unpack with rows that do not fill their last word, or codes off 16 bytes, in launches of at most `stretch` codes each, padding included
+ * (they count them in 32 bits).  by_pieces: 16 codes per thread (1, rows of 15 codes or more) or a word per thread (0).
+ */
+int varq_pack_stretches(const int8_t *codes, int64_t rows, int c, int bits, int32_t *words, int64_t stretch, void *stream);
+int varq_unpack_stretches(const int32_t *words, int64_t rows, int c, int bits, int8_t *codes, int64_t stretch, int by_pieces, void *stream);
 
 #ifdef __cplusplus
 }

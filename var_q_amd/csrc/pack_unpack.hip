@@ -3,10 +3,12 @@
 // definition).  Pure byte shuffling, HBM-bound: one thread per four 32-bit words
 // (16 bytes of words, 16 to 64 bytes of codes, all in 16-byte accesses) when a row is a
 // whole number of words and both buffers are 16-byte aligned; otherwise one thread per word
-// (packing, and the words that are left over) or per 16 codes (unpacking rows that do not fill their last word).
+// (packing, the words that are left over, and unpacking short rows or few words) or per 16 codes (unpacking other rows that do not fill their last word).
 #include <algorithm>
+#include <type_traits>
 
 #include "varq_common.h"
+#include "../../include/varq_testing.h"
 
 namespace {
 
@@ -134,22 +136,26 @@ __global__ __launch_bounds__(256) void pack_ragged_kernel(const int8_t *codes, i
 }
 
 // Unpacking writes most of the bytes: one piece of 16 codes per thread, stored whole, whichever rows
-// they belong to.  The words of a row hold its codes as one run of bits, so the piece's part of a row
-// is BITS / 2 words of that run, shifted into place from one word more; where the piece goes on
+// they belong to (two at most: rows are of 15 codes or more).  The words of a row hold its codes as one run of bits, so the piece's
+// part of a row is BITS / 2 words of that run, shifted into place from one word more; where the piece goes on
 // in the next row, the same window is taken so far before that row's first word that its codes
-// land in their places, and the two are joined by a mask.  (Rows shorter than a piece: as often as it takes.)
-// The pieces whose window would read past the last word go by bytes.  400000 rows of 255 4-bit codes
-// take 25.0 us where a word per thread, stored by bytes, took 67.4; 40009 rows of 100 2.9 where it took 4.9.
-template <int BITS> struct Window {
-  u32 w[BITS / 2];
-  __device__ __forceinline__ void take(const u32 *words, u32 code0, u32 sub) {   // 16 codes from code0 - sub on, counted in fields
-    constexpr u32 VALS = 32 / BITS;
-    const u32 field = code0 - sub;
-    u32 x[BITS / 2 + 1];
-    __builtin_memcpy(x, words + field / VALS, sizeof x);
+// land in their places, and the two are joined by a mask.
+// Bound by memory: 400000 rows of 255 4-bit codes take 28.3 us where a word per thread, stored by bytes, takes 68.0; of 100 11.8 / 29.5.
+// The pieces whose windows would end behind the last word take them word by word, and store what there is of the last one by bytes.
+template <int BITS> struct Window {   // 16 codes
+  static constexpr u32 VALS = 32 / BITS, WIN = BITS / 2;
+  u32 x[WIN + 1], shift;
+  template <bool INSIDE> __device__ __forceinline__ void take(const u32 *words, u32 n_words, u32 field) {   // from `field` on, counted in fields
+    const u32 w = field / VALS;
+    shift = field % VALS * BITS;
+    if constexpr (INSIDE) {
+      __builtin_memcpy(x, words + w, sizeof x);
+    } else {
 #pragma unroll
-    for (int k = 0; k < BITS / 2; ++k) w[k] = __builtin_amdgcn_alignbit(x[k + 1], x[k], field % VALS * BITS);
+      for (u32 k = 0; k <= WIN; ++k) x[k] = words[min(w + k, n_words - 1)];   // (the codes that are there lie in words that are there)
+    }
   }
+  __device__ __forceinline__ u32 word(u32 k) const { return __builtin_amdgcn_alignbit(x[k + 1], x[k], shift); }
 };
 template <int BITS>
 __global__ __launch_bounds__(256) void unpack_ragged_kernel(const int32_t *words, int8_t *codes, u32 n_codes, u32 n_words, u32 c, u32 wpr, FastDiv by_c) {
@@ -157,38 +163,57 @@ __global__ __launch_bounds__(256) void unpack_ragged_kernel(const int32_t *words
   if (at >= n_codes) return;
   constexpr u32 VALS = 32 / BITS, WIN = BITS / 2, DPW = 8 / BITS;
   const u32 *const src = reinterpret_cast<const u32 *>(words);
-  const u32 r = by_c(at), ch = at - r * c, row0 = r * wpr * VALS;
-  const u32 rows_on = by_c(ch + 15);                       // rows that the piece reaches into behind the first
-  if (at + 16 <= n_codes && (row0 + rows_on * wpr * VALS + 16) / VALS + 1 < n_words && (row0 + ch) / VALS + WIN < n_words) {
-    Window<BITS> a;
-    a.take(src, row0 + ch, 0);
-    u32 got = c - ch;                                      // codes of the piece in the window so far
-    for (u32 row = row0 + wpr * VALS; got < 16; row += wpr * VALS, got += c) {
-      Window<BITS> b;
-      b.take(src, row, got);
+  const u32 r = by_c(at), ch = at - r * c, first = r * wpr * VALS + ch, got = c - ch;   // got: codes of the piece in the first row
+  const u32 second = first - ch + wpr * VALS - got;   // (a field that is there: c <= wpr * VALS)
+  u32 q[4];
+  auto piece = [&](auto inside) __attribute__((always_inline)) {
+    Window<BITS> a, b;
+    a.template take<inside()>(src, n_words, first);
+    u32 w[WIN];
+#pragma unroll
+    for (u32 k = 0; k < WIN; ++k) w[k] = a.word(k);
+    if (got < 16) {
+      b.template take<inside()>(src, n_words, second);
 #pragma unroll
       for (u32 k = 0; k < WIN; ++k) {
-        const u32 in = got > k * VALS ? min(got - k * VALS, VALS) : 0u;   // fields of this word that are there
+        const u32 in = got > k * VALS ? min(got - k * VALS, VALS) : 0u;   // fields of this word that are the first row's
         const u32 m = in ? 0xffffffffu >> ((VALS - in) * BITS) : 0u;
-        a.w[k] = (a.w[k] & m) | (b.w[k] & ~m);
+        w[k] = (w[k] & m) | (b.word(k) & ~m);
       }
     }
-    u32 q[4];
 #pragma unroll
-    for (u32 k = 0; k < WIN; ++k) unpack_word<BITS>(a.w[k], q + k * DPW);
+    for (u32 k = 0; k < WIN; ++k) unpack_word<BITS>(w[k], q + k * DPW);
+  };
+  if (at + 16 <= n_codes && (got < 16 ? second : first) / VALS + WIN < n_words) {
+    piece(std::true_type{});
     __builtin_memcpy(codes + at, q, 16);
   } else {
-    u32 row = r, i = ch;
-    for (u32 j = at; j < min(at + 16, n_codes); ++j) {
-      codes[j] = (int8_t)__builtin_amdgcn_sbfe(words[row * wpr + i / VALS], i % VALS * BITS, BITS);
-      if (++i == c) { i = 0; ++row; }
-    }
+    piece(std::false_type{});
+#pragma unroll
+    for (u32 j = 0; j < 16; ++j)
+      if (at + j < n_codes) codes[at + j] = (int8_t)(q[j / 4] >> (8 * (j % 4)));
   }
 }
+// A word per thread, its codes stored by bytes: rows of less than 15 codes (by pieces of 16 and a window per row, 1.8-2.2 us where it takes 1.75-2.1
+// had become 3.1-4.9), and 4 and 8 bits up to 2^19 codes, whose pieces at the end are a longer chain (us, pieces / this: 300 rows of
+// 201 codes, 8 bits, 2.44 / 2.11, 4 bits 2.47 / 2.04, but 30000 rows of 145 2.97 / 4.5 and 2.95 / 5.4; 2 bits, 16 stores of a byte, 300 x 201 2.33 / 2.57).
+template <int BITS>
+__global__ __launch_bounds__(256) void unpack_short_kernel(const int32_t *words, int8_t *codes, u32 n_words, u32 c, u32 wpr, FastDiv by_wpr) {
+  const u32 t = blockIdx.x * 256 + threadIdx.x;
+  if (t >= n_words) return;
+  constexpr u32 VALS = 32 / BITS;
+  const u32 r = by_wpr(t), ch = (t - r * wpr) * VALS, at = r * c + ch, n = min(VALS, c - ch);
+  u32 q[8 / BITS];
+  unpack_word<BITS>((u32)words[t], q);
+#pragma unroll
+  for (u32 j = 0; j < VALS; ++j)
+    if (j < n) codes[at + j] = (int8_t)(q[j / 4] >> (8 * (j % 4)));
+}
 
-// Launches f(first row, rows) over stretches of rows that the ragged kernels can count.
-template <class F> void row_chunks(int64_t rows, int wpr, int vals, F f) {
-  const int64_t most = std::max<int64_t>(1, ((1ll << 31) - 4096) / ((int64_t)wpr * vals));
+// Launches f(first row, rows) over stretches of rows that the ragged kernels can count: `fields` codes at most, padding included.
+constexpr int64_t kStretch = (1ll << 31) - 4096;
+template <class F> void row_chunks(int64_t rows, int wpr, int vals, int64_t fields, F f) {
+  const int64_t most = std::max<int64_t>(1, fields / ((int64_t)wpr * vals));
   for (int64_t r0 = 0; r0 < rows; r0 += most) f(r0, std::min(most, rows - r0));
 }
 
@@ -202,9 +227,7 @@ int check_common(const void *a, const void *b, int64_t rows, int c, int bits, co
   return 0;
 }
 
-}  // namespace
-
-extern "C" int varq_pack(const int8_t *codes, int64_t rows, int c, int bits, int32_t *words, void *stream) {
+int pack_codes(const int8_t *codes, int64_t rows, int c, int bits, int32_t *words, int64_t stretch, void *stream) {
   if (int rc = check_common(codes, words, rows, c, bits, "pack")) return rc;
   if (rows == 0) return VARQ_OK;
   hipStream_t st = (hipStream_t)stream;
@@ -225,7 +248,7 @@ extern "C" int varq_pack(const int8_t *codes, int64_t rows, int c, int bits, int
     if (bits == 8) VARQ_PACK(8) else if (bits == 4) VARQ_PACK(4) else VARQ_PACK(2)
 #undef VARQ_PACK
   } else {
-    row_chunks(rows, wpr, vals, [&](int64_t r0, int64_t n) {
+    row_chunks(rows, wpr, vals, stretch, [&](int64_t r0, int64_t n) {
       const u32 nc = (u32)(n * c), nw = (u32)(n * wpr);
       auto *const kernel = bits == 8 ? pack_ragged_kernel<8> : bits == 4 ? pack_ragged_kernel<4> : pack_ragged_kernel<2>;
       hipLaunchKernelGGL(kernel, dim3((nw + 255) / 256), dim3(256), 0, st, codes + r0 * c, words + r0 * wpr, nc, nw, (u32)c, (u32)wpr, FastDiv::by(wpr));
@@ -235,7 +258,8 @@ extern "C" int varq_pack(const int8_t *codes, int64_t rows, int c, int bits, int
   return VARQ_OK;
 }
 
-extern "C" int varq_unpack(const int32_t *words, int64_t rows, int c, int bits, int8_t *codes, void *stream) {
+// by_pieces: 0 or 1 for the tests, which reach both kernels at sizes of their own (rows of 15 codes or more), or -1
+int unpack_words(const int32_t *words, int64_t rows, int c, int bits, int8_t *codes, int64_t stretch, int by_pieces, void *stream) {
   if (int rc = check_common(words, codes, rows, c, bits, "unpack")) return rc;
   if (rows == 0) return VARQ_OK;
   hipStream_t st = (hipStream_t)stream;
@@ -255,12 +279,32 @@ extern "C" int varq_unpack(const int32_t *words, int64_t rows, int c, int bits, 
     if (bits == 8) VARQ_UNPACK(8) else if (bits == 4) VARQ_UNPACK(4) else VARQ_UNPACK(2)
 #undef VARQ_UNPACK
   } else {
-    row_chunks(rows, wpr, vals, [&](int64_t r0, int64_t n) {
+    row_chunks(rows, wpr, vals, stretch, [&](int64_t r0, int64_t n) {
       const u32 nc = (u32)(n * c), nw = (u32)(n * wpr);
+      if (c < 15 || (by_pieces < 0 ? bits > 2 && (int64_t)nw * vals <= 1 << 19 : !by_pieces)) {
+        auto *const kernel = bits == 8 ? unpack_short_kernel<8> : bits == 4 ? unpack_short_kernel<4> : unpack_short_kernel<2>;
+        hipLaunchKernelGGL(kernel, dim3((nw + 255) / 256), dim3(256), 0, st, words + r0 * wpr, codes + r0 * c, nw, (u32)c, (u32)wpr, FastDiv::by(wpr));
+        return;
+      }
       auto *const kernel = bits == 8 ? unpack_ragged_kernel<8> : bits == 4 ? unpack_ragged_kernel<4> : unpack_ragged_kernel<2>;
       hipLaunchKernelGGL(kernel, dim3((nc + 4095) / 4096), dim3(256), 0, st, words + r0 * wpr, codes + r0 * c, nc, nw, (u32)c, (u32)wpr, FastDiv::by(c));
     });
   }
   VARQ_CHECK_LAUNCH("unpack");
   return VARQ_OK;
+}
+
+}  // namespace
+
+extern "C" int varq_pack(const int8_t *codes, int64_t rows, int c, int bits, int32_t *words, void *stream) {
+  return pack_codes(codes, rows, c, bits, words, kStretch, stream);
+}
+extern "C" int varq_unpack(const int32_t *words, int64_t rows, int c, int bits, int8_t *codes, void *stream) {
+  return unpack_words(words, rows, c, bits, codes, kStretch, -1, stream);
+}
+extern "C" int varq_pack_stretches(const int8_t *codes, int64_t rows, int c, int bits, int32_t *words, int64_t stretch, void *stream) {
+  return pack_codes(codes, rows, c, bits, words, std::min(std::max<int64_t>(stretch, 1), kStretch), stream);
+}
+extern "C" int varq_unpack_stretches(const int32_t *words, int64_t rows, int c, int bits, int8_t *codes, int64_t stretch, int by_pieces, void *stream) {
+  return unpack_words(words, rows, c, bits, codes, std::min(std::max<int64_t>(stretch, 1), kStretch), by_pieces, stream);
 }
