@@ -40,10 +40,15 @@ def test_no_room_for_the_result(dev, method, layout):
     torch.cuda.empty_cache()
     before, total = _state(z), torch.cuda.get_device_properties(dev).total_memory
     torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + 100e6) / total, dev)
+    held = []
     try:
+        with pytest.raises(torch.OutOfMemoryError):     # (what other tests have left of their allocations is taken)
+            while True:
+                held.append(torch.empty(64 << 20, dtype=torch.uint8, device=dev))
         with pytest.raises(torch.OutOfMemoryError):
             z.use_var_q(x)
     finally:
         torch.cuda.set_per_process_memory_fraction(1.0, dev)
+    del held
     assert _state(z) == before
     assert z.use_var_q(x).shape == shape(8193)
