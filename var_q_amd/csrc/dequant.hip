@@ -214,10 +214,10 @@ template <int ODT> void launch_words(const WordsParams &w, const int64_t *s, int
   else width(std::integral_constant<int, 2>{});
 }
 
-template <int ODT, int BITS>
+template <int ODT, int BITS, int U>
 __global__ __launch_bounds__(256) void dequant_steps_kernel(StepParams p) {
-  if constexpr (ODT == VARQ_F32) dequant_steps_halves<BITS, 256, 4>(p, (int64_t)blockIdx.z * gridDim.y + blockIdx.y, blockIdx.x);
-  else dequant_steps_block<ODT, BITS, 256, 4>(p, (int64_t)blockIdx.z * gridDim.y + blockIdx.y, blockIdx.x);
+  if constexpr (ODT == VARQ_F32) dequant_steps_halves<BITS, 256, U>(p, (int64_t)blockIdx.z * gridDim.y + blockIdx.y, blockIdx.x);
+  else dequant_steps_block<ODT, BITS, 256, U>(p, (int64_t)blockIdx.z * gridDim.y + blockIdx.y, blockIdx.x);
 }
 
 }  // namespace
@@ -236,14 +236,26 @@ extern "C" int varq_dequant_steps(const int32_t *words, const float *scale, cons
   VARQ_CHECK_ARG(tokens <= capacity && set_steps(p, words, scale, zp, nseg, host_seg_end, B, H, capacity, c, bits, tokens_first, out),
                  "dequant_steps: more tokens than the buffer or the grid holds");
   if (tokens <= 0) return VARQ_OK;
-  // (pair b * H + h is block (h, b): the grid's limit holds for each dim, as in varq_dequant)
-  dim3 grid((unsigned)((p.pair_octs + 1023) / 1024), (unsigned)(tokens_first ? 1 : H), (unsigned)B);
   hipStream_t st = (hipStream_t)stream;
-#define VARQ_STEPS(ODT_)                                                                                        \
-  do {                                                                                                          \
-    if (bits == 8) hipLaunchKernelGGL((dequant_steps_kernel<ODT_, 8>), grid, dim3(256), 0, st, p);              \
-    else if (bits == 4) hipLaunchKernelGGL((dequant_steps_kernel<ODT_, 4>), grid, dim3(256), 0, st, p);         \
-    else hipLaunchKernelGGL((dequant_steps_kernel<ODT_, 2>), grid, dim3(256), 0, st, p);                        \
+  auto launch = [&](auto odt, auto width, auto per) {
+    // (pair b * H + h is block (h, b): the grid's limit holds for each dim, as in varq_dequant)
+    dim3 grid((unsigned)((p.pair_octs + 256 * per() - 1) / (256 * per())), (unsigned)(tokens_first ? 1 : H), (unsigned)B);
+    hipLaunchKernelGGL((dequant_steps_kernel<odt(), width(), per()>), grid, dim3(256), 0, st, p);
+  };
+  // An octet per lane up to four workgroups per compute unit: a chain of one, where four cost the small launches their idle rounds and the search for the
+  // block's steps.  All tokens of the first 1, 2 and 5 of ten steps, five forms of [1..32,n,6..30,64..128], in a graph, us, four / one: to fp32 2.73 / 2.24, 3.66 / 2.32,
+  // 4.15 / 3.04, to 16 bits 2.59 / 2.13, 3.05 / 2.15, 3.36 / 2.71; from 2^18 octets on it goes either way, one up to 15 % behind.
+  const bool few = (int64_t)B * (tokens_first ? 1 : H) * p.pair_octs <= 1 << 18;
+  auto of = [&](auto odt, auto width) {
+    if (few) launch(odt, width, std::integral_constant<int, 1>{});
+    else launch(odt, width, std::integral_constant<int, 4>{});
+  };
+#define VARQ_STEPS(ODT_)                                        \
+  do {                                                          \
+    std::integral_constant<int, ODT_> odt;                      \
+    if (bits == 8) of(odt, std::integral_constant<int, 8>{});   \
+    else if (bits == 4) of(odt, std::integral_constant<int, 4>{}); \
+    else of(odt, std::integral_constant<int, 2>{});             \
   } while (0)
   if (out_dtype == VARQ_F32) VARQ_STEPS(VARQ_F32);
   else if (out_dtype == VARQ_BF16) VARQ_STEPS(VARQ_BF16);

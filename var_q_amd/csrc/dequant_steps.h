@@ -85,9 +85,9 @@ __device__ __forceinline__ void dequant_steps_block(const StepParams &p, int64_t
   const float *zp = p.zp ? p.zp + (p.head_in_pair ? (pair % p.H) * p.c : 0) : nullptr;
   const int first = block * (NT * U), last = (int)p.pair_octs - 1, o0 = first + threadIdx.x;
   auto segment = [&](int o) __attribute__((always_inline)) { return step_of(p, o); };
-  // most blocks lie in one step
-  const int seg0 = segment(first);
-  const bool one_seg = seg0 == segment(min(first + NT * U - 1, last));
+  // most blocks lie in one step (with an octet per lane, looking for it comes to as much as for the octets')
+  const int seg0 = U > 1 ? segment(first) : 0;
+  const bool one_seg = U > 1 && seg0 == segment(min(first + NT * U - 1, last));
   u32 w0[U], w1[U];
   int64_t at[U];
 #pragma unroll
@@ -140,8 +140,8 @@ __device__ __forceinline__ void dequant_steps_halves(const StepParams &p, int64_
   const int64_t head = p.head_in_pair ? (pair % p.H) * p.c : 0;
   const float *const scale = p.scale + head, *const zp = p.zp ? p.zp + head : nullptr;
   const int first = block * (NT * U), last = (int)p.pair_octs - 1, o0 = first + (int)threadIdx.x / 2, half = threadIdx.x & 1;
-  const int seg0 = step_of(p, first);
-  const bool one_seg = seg0 == step_of(p, min(first + NT * U - 1, last));
+  const int seg0 = U > 1 ? step_of(p, first) : 0;
+  const bool one_seg = U > 1 && seg0 == step_of(p, min(first + NT * U - 1, last));
   u32 w[N];
   int64_t at[N];
 #pragma unroll
