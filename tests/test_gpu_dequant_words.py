@@ -77,3 +77,20 @@ def test_past_the_caches(dev, dt):
         w, s = words[:, :, :n].contiguous(), scale[:, :, :n].contiguous()
         q = ((w.unsqueeze(-1) >> nibble & 15) ^ 8) - 8
         assert torch.equal(ops.dequant(w, s, None, c, 4, dt), (q.view(1, 2, n, c).float() * s).to(dt))
+
+
+@pytest.mark.parametrize('bits', [2, 4, 8])
+@pytest.mark.parametrize('n,c', [(1, 8), (63, 8), (64, 8), (127, 8), (128, 8), (255, 8), (256, 8), (257, 8), (30, 64), (16, 128)])
+@pytest.mark.parametrize('kind', ['row', 'shared_table', 'token_table'])
+def test_pairs_of_one_workgroup(dev, bits, n, c, kind):
+    """Pairs of up to 256 pieces of 16 bytes (an octet in 16 bits, half of one in 32), one per lane, and just more."""
+    from var_q_amd import ops
+    note('pairs of one workgroup', bits, n, c, kind)
+    q = _codes((5, 7, n, c), bits, n + c)
+    words, _ = O.pack_last_dim(q, bits)
+    shape = {'row': (5, 7, n, 1), 'shared_table': (1, 7, 1, c), 'token_table': (1, 1, n, c)}[kind]
+    g = torch.Generator().manual_seed(c)
+    scale, zp = torch.rand(shape, generator=g) + 0.1, torch.randint(-200, 200, shape, generator=g).float()
+    for dt in DTYPES:
+        got = ops.dequant(words.to(dev), scale.to(dev), zp.to(dev), c, bits, dt)
+        assert torch.equal(got.cpu(), _values(q, scale, zp, dt))

@@ -124,7 +124,9 @@ __global__ __launch_bounds__(256) void dequant_kernel(DeqParams p) {
 // come as multipliers: with branches and integer divisions between the loads a launch took 2 to 3 us more at any size.  In a graph, us, before -> now: groups of
 // 32, 4 bits, [3,7,1511,96] fp32 6.4 -> 4.3, bf16 5.1 -> 3.2; 2 bits [2,16,2048,128] bf16 7.0 -> 5.2; 8 bits [4,30,1000,64] fp32 10.3 -> 7.1; 4 bits [16,16,2000,128]
 // fp32 77 -> 43, [16,16,4000,128] bf16 76 -> 49; a scale per (head, channel) [8,30,100,64] 8 bits fp32 4.4 -> 3.3, [2,8,8000,40] 4 bits bf16 7.2 -> 5.1.
-// One piece per lane: 55 -> 83 us at 262 MB of fp32, four: 57, with the small launches the same.
+// One piece per lane: 55 -> 83 us at 262 MB of fp32, four: 57, with the small launches the same.  But pairs of up to 256 pieces, whose second round would load and
+// store nothing, have one, and their wavefronts without any end at once: a scale per (row, channel), 8 bits to bf16, 30 rows of 64 channels, 4096 pairs 8.5 -> 6.5 us (the general
+// kernel 7.6), 20000 28.3 -> 19.0 (22.6), one row 24.9 -> 10.5 (15.5); groups of whole rows 1.06 times as fast, a table per head 1.12.
 // STREAM: an output that does not fit the Infinity Cache with its codes goes past it (262 MB, alone / with a copy that reads it: fp32 55 / 158 -> 43 / 152, bf16 58 / 158 -> 49 / 154); a
 // smaller one would be read from memory by whoever reads it next (98 MB fp32 18.6 / 48.5 -> 16.3 / 54.3, 84 MB bf16 19.0 / 43.7 -> 18.1 / 48.9).
 constexpr int64_t kStreamBytes = 240ll << 20;
@@ -147,6 +149,7 @@ __global__ __launch_bounds__(256) void dequant_words_kernel(WordsParams p) {
   constexpr int Q = ODT == VARQ_F32 ? 4 : 8, PER = 8 / Q;   // channels of a piece, pieces of an octet
   const int64_t i0 = blockIdx.z, i1 = blockIdx.y;
   const u32 first = blockIdx.x * (256 * U) + threadIdx.x, n = (u32)p.octets * PER;
+  if (U == 1 && first >= n) return;
   const char *const words = p.words + (i0 * p.os0 + i1 * p.os1 + p.off) * p.row_bytes;
   const int64_t table = i0 * p.ss0 + i1 * p.ss1;
   const float *const scale = p.scale + table, *const zp = p.zp ? p.zp + table : nullptr;
@@ -197,12 +200,16 @@ __global__ __launch_bounds__(256) void dequant_words_kernel(WordsParams p) {
 }
 
 template <int ODT> void launch_words(const WordsParams &w, const int64_t *s, int bits, bool table, hipStream_t st) {
-  constexpr int U = 2, PER = ODT == VARQ_F32 ? 2 : 1;
-  dim3 grid((unsigned)(((int64_t)w.octets * PER + 256 * U - 1) / (256 * U)), (unsigned)s[1], (unsigned)s[0]);
+  constexpr int PER = ODT == VARQ_F32 ? 2 : 1;
   const bool stream = s[0] * s[1] * (int64_t)w.octets * 16 * PER >= kStreamBytes;
+  auto pieces = [&](auto b, auto t, auto u) {
+    dim3 grid((unsigned)(((int64_t)w.octets * PER + 256 * u() - 1) / (256 * u())), (unsigned)s[1], (unsigned)s[0]);
+    if (stream) hipLaunchKernelGGL((dequant_words_kernel<ODT, b(), t(), u(), true>), grid, dim3(256), 0, st, w);
+    else hipLaunchKernelGGL((dequant_words_kernel<ODT, b(), t(), u(), false>), grid, dim3(256), 0, st, w);
+  };
   auto kind = [&](auto b, auto t) {
-    if (stream) hipLaunchKernelGGL((dequant_words_kernel<ODT, b(), t(), U, true>), grid, dim3(256), 0, st, w);
-    else hipLaunchKernelGGL((dequant_words_kernel<ODT, b(), t(), U, false>), grid, dim3(256), 0, st, w);
+    if ((int64_t)w.octets * PER <= 256) pieces(b, t, std::integral_constant<int, 1>{});
+    else pieces(b, t, std::integral_constant<int, 2>{});
   };
   auto width = [&](auto b) {
     if (!table) kind(b, std::integral_constant<int, 0>{});
