@@ -94,3 +94,18 @@ def test_pairs_of_one_workgroup(dev, bits, n, c, kind):
     for dt in DTYPES:
         got = ops.dequant(words.to(dev), scale.to(dev), zp.to(dev), c, bits, dt)
         assert torch.equal(got.cpu(), _values(q, scale, zp, dt))
+
+
+@pytest.mark.parametrize('octets', [2047, 2048, 2049, 3070, 3072, 4096, 4100])
+@pytest.mark.parametrize('c', [96, 100])
+def test_general_kernel_octets_of_a_lane(dev, octets, c):
+    """One, two and four octets of a lane one after the other: int8 codes, and packed rows that are no whole octets."""
+    from var_q_amd import ops
+    note('general dequantizing', octets, c)
+    n = -(-octets // (-(-c // 8)))
+    q = _codes((2, 3, n, c), 4, octets)
+    g = torch.Generator().manual_seed(octets)
+    scale, zp = torch.rand((2, 3, n, 1), generator=g) + 0.1, torch.randint(-20, 20, (2, 3, n, 1), generator=g).float()
+    for codes in ([q] if c == 96 else [q, O.pack_last_dim(q, 4)[0]]):
+        for dt in DTYPES:
+            assert torch.equal(ops.dequant(codes.to(dev), scale.to(dev), zp.to(dev), c, 4, dt).cpu(), _values(q, scale, zp, dt))

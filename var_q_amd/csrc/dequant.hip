@@ -328,12 +328,19 @@ extern "C" int varq_dequant(const int32_t *words, const int8_t *codes_i8, const 
     VARQ_CHECK_LAUNCH("dequant");
     return VARQ_OK;
   }
-  const int U = p.octets_per_pair >= 2048 ? 4 : 1;
+  // The octets of a lane follow one another: four where a pair has the work for it, two where four would leave more than a twelfth of the last block's lanes idle
+  // (four / two, us: int8 codes [3,6,173,128] fp16 4.0 / 3.1, [8,6,662,64] fp32 6.0 / 5.1, packed rows of 100 channels [12,30,177,100] fp16 15.4 / 12.3).
+  int U = p.octets_per_pair >= 2048 ? 4 : 1;
+  if (U == 4 && !(group == 1 && p.ss3 == 1 && p.ss2 == 0)) {
+    const int64_t t4 = (p.octets_per_pair + 1023) / 1024;
+    if ((t4 * 1024 - p.octets_per_pair) * 12 > t4 * 1024) U = 2;
+  }
   const int64_t tiles = (p.octets_per_pair + 256 * U - 1) / (256 * U);
   dim3 grid((unsigned)tiles, (unsigned)s[1], (unsigned)s[0]);
 #define VARQ_DEQ(ODT_)                                                                     \
   do {                                                                                     \
     if (U == 4) hipLaunchKernelGGL((dequant_kernel<ODT_, 4>), grid, dim3(256), 0, st, p);  \
+    else if (U == 2) hipLaunchKernelGGL((dequant_kernel<ODT_, 2>), grid, dim3(256), 0, st, p);  \
     else hipLaunchKernelGGL((dequant_kernel<ODT_, 1>), grid, dim3(256), 0, st, p);         \
   } while (0)
   if (out_dtype == VARQ_F32) VARQ_DEQ(VARQ_F32);
