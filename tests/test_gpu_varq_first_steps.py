@@ -22,18 +22,30 @@ class General(VAR_Q):
 @pytest.mark.parametrize('use', [None, torch.float32, torch.float16])
 @pytest.mark.parametrize('steps', [(1, 1), (64, 1, 150), (70, 60)])      # room for 64 tokens at first: exactly full, and beyond
 def test_first_and_growing_steps(dev, monkeypatch, method, layout, symmetric, use, steps):
-    note('first steps', method, layout, symmetric, use, steps)
+    _steps(dev, monkeypatch, method, layout, symmetric, use, steps, 8, 64)
+
+
+@pytest.mark.parametrize('method', ['G_SCALE_HEAD_DIM', 'G_SCALE', 'G_HEAD', 'G_TOKEN', 'G_TOKEN_HEAD'])
+@pytest.mark.parametrize('layout', ['BLHc', 'BHLc'])
+@pytest.mark.parametrize('use', [None, torch.bfloat16])
+@pytest.mark.parametrize('bits,c', [(8, 24), (4, 40), (4, 128), (2, 48), (2, 128)])
+def test_other_rows(dev, monkeypatch, method, layout, use, bits, c):
+    _steps(dev, monkeypatch, method, layout, bits != 4, use, (1, 63, 1, 80), bits, c)
+
+
+def _steps(dev, monkeypatch, method, layout, symmetric, use, steps, bits, c):
+    note('first steps', method, layout, symmetric, use, steps, bits, c)
     d, g = 1 if layout == 'BLHc' else 2, torch.Generator().manual_seed(sum(steps))
-    a, b = [cls(8, layout, method, symmetric=symmetric) for cls in (VAR_Q, General)]
+    a, b = [cls(bits, layout, method, symmetric=symmetric) for cls in (VAR_Q, General)]
     with pytest.raises(RuntimeError):
-        a.use_var_q(torch.empty((2, 0, 3, 64) if d == 1 else (2, 3, 0, 64), device=dev))
+        a.use_var_q(torch.empty((2, 0, 3, c) if d == 1 else (2, 3, 0, c), device=dev))
     assert a._pack_meta is None and a._c_item.buf is None
 
     def refuse(self, item):
         raise AssertionError('the general method of a quantizer that has a native step')
     monkeypatch.setattr(VAR_Q, 'quant', refuse)
     for n in steps:
-        x = torch.randn(*((2, n, 3, 64) if d == 1 else (2, 3, n, 64)), generator=g).to(dev, torch.bfloat16)
+        x = torch.randn(*((2, n, 3, c) if d == 1 else (2, 3, n, c)), generator=g).to(dev, torch.bfloat16)
         if use is None:
             assert a._step_fast(x)
             General.general(b, x)
