@@ -132,3 +132,24 @@ def test_a_nan_in_one_share(dev, at, waves):
     out = ops.fused_attn(q, kw, ks, kz, *vq, 8, 8, Lk, 1 / math.sqrt(D))
     bad = torch.isnan(out).all(-1)
     assert bool(bad[0, 3].all()) and not bool(torch.isnan(out[0, [h for h in range(H) if h != 3]]).any())
+
+
+@pytest.mark.parametrize('waves', [2, 4])
+@pytest.mark.parametrize('D,bits,group,dtype', [(128, 4, 128, 'bf16'), (64, 8, 64, 'fp16')])
+@pytest.mark.parametrize('bad', [math.nan, math.inf])
+def test_a_nan_behind_the_limit_in_another_share(dev, D, bits, group, dtype, bad, waves):
+    """Queries that see the first share's keys alone, among others that see all: what the other shares hold of V is not theirs."""
+    dt = torch.float16 if dtype == 'fp16' else torch.bfloat16
+    Lq = Lk = 449
+    B, H = 1, _pairs(waves, Lq, Lk, D, 1)
+    q, k, v = _inputs(dev, B, H, Lq, Lk, D, dt)
+    kq, (vw, vs, vz) = ops.quant_pack_rows(k, group, bits, True), ops.quant_pack_rows(v, group, bits, True)
+    few = torch.arange(Lq, device=dev) % 2 == 0
+    lim = torch.where(few, 32, Lk).int().contiguous()
+    run = lambda: ops.fused_attn(q, *kq, vw, vs, vz, bits, bits, Lk, 1 / math.sqrt(D), kv_limit=lim)
+    note('key waves, NaN behind the limit', D, bad, waves)
+    want = run()
+    vs[:, :, 40] = bad
+    out = run()
+    assert torch.equal(out[:, :, few], want[:, :, few])
+    assert not bool(torch.isfinite(out[:, :, ~few]).all(-1).any())

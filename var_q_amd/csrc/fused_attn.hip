@@ -1177,6 +1177,12 @@ __device__ __forceinline__ void attend_tiles(const AttnParams &p, int bh, int ou
     float2 *const stats = reinterpret_cast<float2 *>(lds_raw);                       // [NWV / KS][KS][32]
     float4 *const handed = reinterpret_cast<float4 *>(lds_raw + L::kStats);          // [NWV / KS][to: KS][from: KS - 1][OWN][64]
     const float l_own = l_part + __shfl_xor(l_part, 32, 64);
+    if (l_own == 0.f) {   // (the query sees none of the share's keys: an infinity or NaN among them, times 0, has no say either)
+#pragma unroll
+      for (int d = 0; d < NDB; ++d)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) oacc[d][i] = 0.f;
+    }
     if (half == 0) stats[(qwave * KS + share) * 32 + col] = make_float2(m_ref, l_own);
     __syncthreads();
     float M = -INFINITY, l_sum = 0.f, w_own = 0.f;
