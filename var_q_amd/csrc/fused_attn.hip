@@ -1292,6 +1292,7 @@ template <int D, int NWV, int WPS, bool F16, int KS>
 __global__ __launch_bounds__(NWV * 64, WPS) void fused_attn_classes_kernel(AttnParams p, ClassTable t) {
   const BlockOf k(p);
   if (k.pair >= p.bh_total) return;
+  p.kv_ts = 1;   // (heads first, which a constant tells the compiler: rows as far apart as they are long)
   in_class(p, t, k.pair, [&](auto bits, int bh, int out_pair) __attribute__((always_inline)) {
     attend_tiles<D, decltype(bits)::value, false, NWV, F16, false, KS>(p, bh, out_pair, k.qt, k.split);
   });
