@@ -821,8 +821,10 @@ __device__ __forceinline__ void attend_tiles(const AttnParams &p, int bh, int ou
   const char *const vsc = reinterpret_cast<const char *>(p.v_scale) + kv_row0 * (4 * v_groups);
   const char *const vzp = reinterpret_cast<const char *>(v_has_zp ? p.v_zp : p.v_scale) + kv_row0 * (4 * v_groups);
   const int k_g4 = CHAN ? 0 : (part * CH >> p.k_shift) * 4, v_g4 = CHAN ? 0 : (part * CH >> p.v_shift) * 4;
-  struct Piece { u32 k[PW], v[PW]; float ks, kz, vs, vz; } next[IT];
-  auto load_piece = [](const char *src, u32 (&dst)[PW]) __attribute__((always_inline)) {
+  // (two bytes stay two until they are used: widened where the two ways of request() meet, they would be waited for there)
+  using Raw = std::conditional_t<PB == 2, uint16_t, u32>;
+  struct Piece { Raw k[PW], v[PW]; float ks, kz, vs, vz; } next[IT];
+  auto load_piece = [](const char *src, Raw (&dst)[PW]) __attribute__((always_inline)) {
     if constexpr (PB == 16) {
       const u32x4_t t = *reinterpret_cast<const u32x4_t *>(src);
 #pragma unroll
@@ -898,7 +900,10 @@ __device__ __forceinline__ void attend_tiles(const AttnParams &p, int bh, int ou
           }
           tab += sg * (tab_rows * D) + part * CH;
         }
-        auto rows = [&](const u32 (&w)[PW], float s, float z, int row, uint16_t *dst) __attribute__((always_inline)) {
+        auto rows = [&](const Raw (&raw)[PW], float s, float z, int row, uint16_t *dst) __attribute__((always_inline)) {
+          u32 w[PW];
+#pragma unroll
+          for (int j = 0; j < PW; ++j) w[j] = raw[j];
           const float s1 = s * kUnit, z1 = z * (1.f / kUnit);
 #pragma unroll
           for (int o = 0; o < OCT; ++o) {
