@@ -27,9 +27,9 @@ int varq_quant_pack_shards(const int64_t *host_shape4, int reduce_mask, int x_dt
 
 /*
  * Over how many wavefronts of a workgroup the attention shares the keys of its queries out on the current device when that is left to it (splits = 0) and
- * the kernel that widens per workgroup serves the call: 1, 2 or 4; 0: with these key limits K and V are expanded instead. limits: whether there are key limits.
+ * the kernel that widens per workgroup serves the call: 1, 2 or 4; 0: with these key limits K and V are expanded instead. nseg: tables (1 for scales per key); limits: whether there are key limits.
  */
-int varq_fused_attn_key_waves(int B, int Hkv, int Lq, int Lk, int D, int limits);
+int varq_fused_attn_key_waves(int B, int Hkv, int Lq, int Lk, int D, int nseg, int limits);
 
 /*
  * varq_pack and varq_unpack with rows that do not fill their last word, or codes off 16 bytes, in launches of at most `stretch` codes each, padding included

@@ -17,14 +17,14 @@ EDGES = [(129, 65), (192, 96), (193, 97), (256, 128), (257, 129), (130, 161), (3
 LIMIT_EDGES = [(193, 193), (256, 256), (257, 257), (385, 385), (449, 449), (400, 1025)]
 
 
-def _waves(B, H, Lq, Lk, D, limits):
-    return _lib.load().varq_fused_attn_key_waves(B, H, Lq, Lk, D, limits)
+def _waves(B, H, Lq, Lk, D, limits, nseg=1):
+    return _lib.load().varq_fused_attn_key_waves(B, H, Lq, Lk, D, nseg, limits)
 
 
-def _pairs(waves, Lq, Lk, D, limits=0):
+def _pairs(waves, Lq, Lk, D, limits=0, nseg=1):
     """The fewest pairs (five at least) whose keys that many wavefronts share."""
-    found = [n for n in range(5, 129) if _waves(1, n, Lq, Lk, D, limits) == waves]
-    assert found, (waves, Lq, Lk, D, limits)
+    found = [n for n in range(5, 129) if _waves(1, n, Lq, Lk, D, limits, nseg) == waves]
+    assert found, (waves, Lq, Lk, D, limits, nseg)
     return found[0]
 
 
@@ -84,10 +84,10 @@ def test_few_pairs_under_limits(dev, D, bits, group, dtype, Lq, Lk):
 @pytest.mark.parametrize('Lq,Lk,limits', [e + (0,) for e in EDGES] + [(257, 257, 1), (449, 449, 1)])
 @pytest.mark.parametrize('D,bits,asym', [(128, 8, False), (128, 4, True), (64, 8, False), (64, 2, True)])
 def test_tables(dev, D, bits, asym, Lq, Lk, limits, waves):
-    B, H = 1, _pairs(waves, Lq, Lk, D, limits)
+    ends = sorted({1, 5, Lk // 3, Lk // 2 + 7, Lk})
+    B, H = 1, _pairs(waves, Lq, Lk, D, limits, len(ends))
     dt = torch.float16 if D == 64 else torch.bfloat16
     q, k, v = _inputs(dev, B, H, Lq, Lk, D, dt)
-    ends = sorted({1, 5, Lk // 3, Lk // 2 + 7, Lk})
     cuts = list(zip([0] + ends[:-1], ends))
     def quant(x):
         parts = [ops.quant_pack(x[:, :, a:b].contiguous(), (0, 2), bits, asym=asym) for a, b in cuts]

@@ -20,7 +20,7 @@ def test_allocates_what_the_call_uses(dev, D, limits, B, H, Lq, Lk):
     want = lib.varq_fused_attn_workspace_bytes_call(B, H, Lq, Lk, D, 1, 0, int(limits))
     assert want <= lib.varq_fused_attn_workspace_bytes(B, H, Lq, Lk, D, 1, 0)
     if (D, Lk, limits) == (64, 400, False):
-        assert want == 0 and lib.varq_fused_attn_key_waves(B, H, Lq, Lk, D, int(limits)) > 1
+        assert want == 0 and lib.varq_fused_attn_key_waves(B, H, Lq, Lk, D, 1, int(limits)) > 1
     k, v = (ops.quant_pack_rows(torch.randn(B, H, Lk, D, device=dev), 64, 4, True) for _ in range(2))
     q, out = (torch.randn(B, H, Lq, D, device=dev).bfloat16() for _ in range(2))
     lim = torch.full((Lq,), Lk, dtype=torch.int32, device=dev) if limits else None

@@ -87,7 +87,7 @@ TESTING = {
     'varq_quant_pack_wait': (c_int, [c_void_p, c_int, POINTER(c_int64), c_int, c_int, c_int, c_float, c_void_p, c_void_p, c_void_p, c_void_p,
                                      POINTER(c_int64), c_uint32, c_void_p, c_size_t, c_void_p]),
     'varq_quant_pack_shards': (c_int, [POINTER(c_int64), c_int, c_int, c_int, c_int, c_int]),
-    'varq_fused_attn_key_waves': (c_int, [c_int] * 6),
+    'varq_fused_attn_key_waves': (c_int, [c_int] * 7),
     'varq_pack_stretches': (c_int, [c_void_p, c_int64, c_int, c_int, c_void_p, c_int64, c_void_p]),
     'varq_unpack_stretches': (c_int, [c_void_p, c_int64, c_int, c_int, c_void_p, c_int64, c_int, c_void_p]),
 }

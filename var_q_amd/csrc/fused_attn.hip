@@ -1575,8 +1575,11 @@ struct KeyShares { int waves, splits; };
 // takes is 0.5 % behind the best of all on the geometric mean and 9 % ahead of workgroups alone, and in 5 of them behind those by more than 2.5 %.  4 bits in groups,
 // us, workgroups alone / this: D=128, 32 pairs, 256 queries x 521 keys 22.6 / 16.5, 400 x 921 32.4 / 22.8, 64 pairs, 144 x 300 16.8 / 12.0, 256 x 521
 // 27.2 / 17.4, 400 x 921 40.9 / 30.5, 128 pairs, 256 x 521 28.6 / 22.8; D=64, 32 pairs, 256 x 521 15.7 / 11.6, 1024 x 2521 50.1 / 43.4, 128 pairs, 256 x 521 19.1 / 15.1.
+// Tables take a workgroup 0.1 us per KiB beyond the first one (their LDS, at D=64 with four wavefronts beyond 80 KiB one workgroup per compute unit instead of two): of 600 forms with 1, 5, 10 and
+// 16 tables without that 31 were more than 3 % behind workgroups alone, by up to 28 %, with it 19, by up to 11 %, and 9.7 -> 10.1 % ahead of them on the geometric mean.
+double tables_us(int nseg, int D) { return 0.1 * (nseg - 1) * (4 * D * 4) / 1024.0; }
 // alone: what workgroups alone would be, where that is asked too (it is what the first round of the loop ends with).
-KeyShares choose_shares(int64_t bh, int Lq, int Lk, int D, int most_waves, int cus, KeyShares *alone = nullptr) {
+KeyShares choose_shares(int64_t bh, int Lq, int Lk, int D, int nseg, int most_waves, int cus, KeyShares *alone = nullptr) {
   static const double tile_us[2][3] = {{1.45, 0.85, 1.1}, {2.07, 1.35, 1.9}};
   const double per_xcd = cus / 8.0;
   const bool wide = D == 128;
@@ -1589,7 +1592,7 @@ KeyShares choose_shares(int64_t bh, int Lq, int Lk, int D, int most_waves, int c
     const int tiles = (Lk + (waves == 4 ? 2 * BN : BN) - 1) / (waves == 4 ? 2 * BN : BN);
     const int64_t blocks = bh * ((Lq + BM / waves - 1) / (BM / waves));
     // (up to 128 queries half of the wavefronts have none, and widen only)
-    const double tile = tile_us[wide][i] * (waves == 1 && Lq <= 128 ? 0.7 : 1.0), fixed = (wide ? 2.8 : 2.2) + (waves > 1 ? 1.1 : 0.0);
+    const double tile = tile_us[wide][i] * (waves == 1 && Lq <= 128 ? 0.7 : 1.0), fixed = (wide ? 2.8 : 2.2) + (waves > 1 ? 1.1 : 0.0) + tables_us(nseg, D);
     for (int n = 1; n <= kMaxSplits; ++n) {
       if (n > 1 && (Lk + BN - 1) / BN / n < 2) break;
       double us = std::ceil((double)((blocks * n + 7) / 8) / per_xcd) * ((double)((tiles + n - 1) / n) * tile + fixed);
@@ -1612,7 +1615,7 @@ int set_splits(AttnParams &p, int D, int most_waves, const KeyShares *limited, i
   const bool unaligned = workspace && ((uintptr_t)workspace & 15);
   int n = splits;
   KeyShares alone = {1, 1}, k = {1, 1};
-  if (splits == 0 && (!limited || unaligned)) k = choose_shares(p.bh_total, p.Lq, p.Lk, D, limited ? 1 : most_waves, device_cus(), &alone);
+  if (splits == 0 && (!limited || unaligned)) k = choose_shares(p.bh_total, p.Lq, p.Lk, D, p.nseg, limited ? 1 : most_waves, device_cus(), &alone);
   // (a workspace that cannot be used is an error wherever workgroups alone would use it, and is not used otherwise)
   if (unaligned && alone.splits > 1 && workspace_bytes >= split_workspace_bytes(2, rows, D))
     return varq_set_error(VARQ_ERR_INVALID, "%s: the workspace must be 16-byte aligned", who);
@@ -1741,36 +1744,42 @@ bool wide_eligible(int B, int Hkv, int Lq, int Lk, int D, bool limits, int cus =
 // every choice: 1.2 % behind the best on the geometric mean, 18 % ahead of the rules before, blocks of 128 queries for few pairs (wide_four) and shares as without
 // limits.  4 bits in groups, us, before / this: D=64, 2 pairs x 4500 tokens 52.7 / 31, 16 x 300 12.4 / 9.0, x 680 17.6 / 12.4, x 1500 29.1 / 24.6, 32 x 524 17.2 / 12.9, 48 x 1000 27.3 / 23.0;
 // D=128, 2 x 4500 93 / 46, 16 x 680 24.8 / 17.3, 24 x 600 24.6 / 16.6, x 1000 33.9 / 28.9, 32 x 854 34.0 / 27.1, 90 x 249 16.7 / 13.7.
-KeyShares limited_shares(int B, int Hkv, int Lq, int Lk, int D, int most, bool may_expand, int cus) {
+KeyShares limited_shares(int B, int Hkv, int Lq, int Lk, int D, int nseg, int most, bool may_expand, int cus) {
   const int64_t bh = (int64_t)B * Hkv;
   const bool four = may_expand && wide_four((int64_t)wide_batch(B, Hkv, Lk, D) * Hkv, Lq, Lk, D, cus, true);
   if (may_expand && !four && wide_eligible(B, Hkv, Lq, Lk, D, true, cus)) return {0, 1};
-  if (Lq <= 128 || Lk <= 128) return {1, most == 1 ? 1 : choose_shares(bh, Lq, Lk, D, 1, cus).splits};
+  if (Lq <= 128 || Lk <= 128) return {1, most == 1 ? 1 : choose_shares(bh, Lq, Lk, D, nseg, 1, cus).splits};
   struct Cost { double tile, fixed, again, load; };   // us of a tile, of a workgroup, of one that is not the longest; of the whole load
   static const Cost cost[2][3] = {{{1.32, 5.8, 4.7, 0.9}, {0.87, 6.0, 4.9, 1.03}, {1.15, 5.6, 4.6, 1.03}}, {{2.1, 4.7, 3.8, 1.0}, {1.4, 6.6, 5.4, 1.14}, {1.9, 6.1, 5.0, 1.14}}};
   static const Cost expanded[2] = {{0.9, 10.0, 4.0, 0.92}, {1.4, 14.0, 4.0, 0.95}};
-  auto us = [&](const Cost &c, int block, int keys, int n) {
+  const double tables = tables_us(nseg, D);
+  auto us = [&](const Cost &c, int block, int keys, int n, double tables = 0.0) {
     const double blocks = (Lq + block - 1) / block, part = std::floor(0.8 * blocks), tiles = (double)Lk / keys * (1.25 * part * (part + 1.0) / (2.0 * blocks) + blocks - part) + 0.5 * blocks;
-    const double longest = c.fixed + c.tile * (((Lk + keys - 1) / keys + n - 1) / n), load = c.load * (double)bh * (blocks * n * c.again + tiles * c.tile) / cus;
+    const double longest = c.fixed + tables + c.tile * (((Lk + keys - 1) / keys + n - 1) / n), load = c.load * (double)bh * (blocks * n * (c.again + tables) + tiles * c.tile) / cus;
     const double two = longest * longest, four = load * load;
     return std::sqrt(std::sqrt(two * two + four * four));
   };
   const int d = D == 128;
   KeyShares best = {1, 1};
-  double best_us = us(cost[d][0], BM, BN, 1);
+  double best_us = us(cost[d][0], BM, BN, 1, tables);
   if (four) {
     const double t = us(expanded[d], 128, BN, 1);
     if (t < best_us) { best_us = t; best = {0, 1}; }
   }
   for (int i = 0; i < 3; ++i)
     for (int n = 1; n <= most && (n == 1 || (Lk + BN - 1) / BN / n >= 2); ++n) {
-      double t = us(cost[d][i], BM >> i, i == 2 ? 2 * BN : BN, n) * (i ? 1.05 : 1.0);
+      double t = us(cost[d][i], BM >> i, i == 2 ? 2 * BN : BN, n, tables) * (i ? 1.05 : 1.0);
       if (n > 1) t += 2.8 + 2.0 * (double)split_workspace_bytes(n, bh * Lq, D) / 4.0e6;
       if (t < best_us) { best_us = t; best = {1 << i, n}; }
     }
   return best;
 }
 constexpr int kLimitedSplits = 6;   // (more gain nothing)
+// What a call does, whose caller asks expand_bytes, which knows of no tables, whether it expands.
+KeyShares limited_call(int B, int Hkv, int Lq, int Lk, int D, int nseg, int most, int cus) {
+  const KeyShares k = limited_shares(B, Hkv, Lq, Lk, D, 1, most, true, cus);
+  return k.waves && nseg > 1 ? limited_shares(B, Hkv, Lq, Lk, D, nseg, most, false, cus) : k;
+}
 // The largest workspace of the parts that the call is done in.
 size_t wide_bytes(int B, int Hkv, int Lq, int Lk, int D, bool share, bool limits) {
   const int n = wide_batch(B, Hkv, Lk, D), last = B - (B - 1) / n * n;
@@ -1812,12 +1821,12 @@ class Limited {
 
  public:
   Limited(const AttnParams &p_, int B_, int D_, int splits) : p(p_), B(B_), D(D_), most(!p_.kv_limit || splits > 1 ? 0 : splits == 1 ? 1 : kLimitedSplits) {
-    if (most) k = limited_shares(B, p.Hkv, p.Lq, p.Lk, D, most, true, device_cus());
+    if (most) k = limited_call(B, p.Hkv, p.Lq, p.Lk, D, p.nseg, most, device_cus());
   }
   bool expands() const { return k.waves == 0; }   // (or is not asked)
   const KeyShares *shares() {
     if (!most) return nullptr;
-    if (k.waves == 0) k = limited_shares(B, p.Hkv, p.Lq, p.Lk, D, most, false, device_cus());
+    if (k.waves == 0) k = limited_shares(B, p.Hkv, p.Lq, p.Lk, D, p.nseg, most, false, device_cus());
     return &k;
   }
 };
@@ -1825,7 +1834,7 @@ class Limited {
 size_t expand_bytes(int B, int Hkv, int Lq, int Lk, int D, bool limits) {
   if (B <= 0 || Hkv <= 0 || Lq <= 0 || Lk <= 0 || (D != 64 && D != 128)) return 0;
   const int cus = device_cus();   // (a call into the runtime)
-  if (!wide_eligible(B, Hkv, Lq, Lk, D, limits, cus) || (limits && limited_shares(B, Hkv, Lq, Lk, D, kLimitedSplits, true, cus).waves)) return 0;
+  if (!wide_eligible(B, Hkv, Lq, Lk, D, limits, cus) || (limits && limited_shares(B, Hkv, Lq, Lk, D, 1, kLimitedSplits, true, cus).waves)) return 0;
   return wide_bytes(B, Hkv, Lq, Lk, D, true, limits);
 }
 
@@ -1834,16 +1843,17 @@ size_t expand_bytes(int B, int Hkv, int Lq, int Lk, int D, bool limits) {
 namespace {
 // Bytes for the shares of a call without key limits, with them, or either and in any operand form.
 enum { kPlain = 1, kLimits = 2 };
-size_t shares_bytes(int B, int Hkv, int Lq, int Lk, int D, int splits, int of) {
+size_t shares_bytes(int B, int Hkv, int Lq, int Lk, int D, int nseg, int splits, int of) {
   if (B <= 0 || Hkv <= 0 || Lq <= 0 || Lk <= 0 || (D != 64 && D != 128) || splits < 0 || splits > kMaxSplits) return 0;
+  nseg = std::min(std::max(nseg, 1), kMaxSegments);
   const int64_t bh = (int64_t)B * Hkv, rows = bh * Lq;
   int n = splits;
   if (!splits) {   // (every call asks: up to 128 queries or keys what wavefronts share, and what the limits say, come to the same as workgroups alone)
     const int cus = device_cus();
     const bool waves = of & kPlain && Lq > 128 && Lk > BN, limits = of & kLimits && Lq > 128 && Lk > 128;
     KeyShares alone = {1, 1};
-    if (limits) n = limited_shares(B, Hkv, Lq, Lk, D, kLimitedSplits, false, cus).splits;
-    if (!limits || of & kPlain) n = std::max(n, choose_shares(bh, Lq, Lk, D, waves ? 4 : 1, cus, &alone).splits);
+    if (limits) n = limited_shares(B, Hkv, Lq, Lk, D, nseg, kLimitedSplits, false, cus).splits;
+    if (!limits || of & kPlain) n = std::max(n, choose_shares(bh, Lq, Lk, D, nseg, waves ? 4 : 1, cus, &alone).splits);
     if (of == (kPlain | kLimits)) n = std::max(n, alone.splits);   // (the form with exact codes has no shares of wavefronts)
     // (the group sizes are not known here: room for the few-queries kernel's shares whenever the
     // other sizes would admit it)
@@ -1854,18 +1864,16 @@ size_t shares_bytes(int B, int Hkv, int Lq, int Lk, int D, int splits, int of) {
 }  // namespace
 
 extern "C" size_t varq_fused_attn_workspace_bytes(int B, int Hkv, int Lq, int Lk, int D, int nseg, int splits) {
-  (void)nseg;   // (the tile count does not depend on the tables)
-  return shares_bytes(B, Hkv, Lq, Lk, D, splits, kPlain | kLimits);
+  return shares_bytes(B, Hkv, Lq, Lk, D, nseg, splits, kPlain | kLimits);
 }
 extern "C" size_t varq_fused_attn_workspace_bytes_call(int B, int Hkv, int Lq, int Lk, int D, int nseg, int splits, int limits) {
-  (void)nseg;
-  return shares_bytes(B, Hkv, Lq, Lk, D, splits, limits ? kLimits : kPlain);
+  return shares_bytes(B, Hkv, Lq, Lk, D, nseg, splits, limits ? kLimits : kPlain);
 }
 
-extern "C" int varq_fused_attn_key_waves(int B, int Hkv, int Lq, int Lk, int D, int limits) {
-  if (B <= 0 || Hkv <= 0 || Lq <= 0 || Lk <= 0 || (D != 64 && D != 128)) return -1;
+extern "C" int varq_fused_attn_key_waves(int B, int Hkv, int Lq, int Lk, int D, int nseg, int limits) {
+  if (B <= 0 || Hkv <= 0 || Lq <= 0 || Lk <= 0 || (D != 64 && D != 128) || nseg < 1) return -1;
   const int cus = device_cus();
-  return limits ? limited_shares(B, Hkv, Lq, Lk, D, kLimitedSplits, true, cus).waves : choose_shares((int64_t)B * Hkv, Lq, Lk, D, 4, cus).waves;
+  return limits ? limited_call(B, Hkv, Lq, Lk, D, nseg, kLimitedSplits, cus).waves : choose_shares((int64_t)B * Hkv, Lq, Lk, D, nseg, 4, cus).waves;
 }
 
 extern "C" size_t varq_fused_attn_expand_bytes(int B, int Hkv, int Lq, int Lk, int D) {
@@ -1876,7 +1884,7 @@ extern "C" size_t varq_fused_attn_expand_bytes_limits(int B, int Hkv, int Lq, in
 extern "C" int varq_fused_attn_key_shares(int B, int Hkv, int Lq, int Lk, int D, int k_group, int v_group) {
   if (B <= 0 || Hkv <= 0 || Lq <= 0 || Lk <= 0 || (D != 64 && D != 128)) return 0;
   if (fewq_eligible(B, Hkv, Lq, Lk, D, k_group, v_group)) return fewq_shares(B * Hkv, Lq, Lk, D, k_group, v_group);
-  return choose_shares((int64_t)B * Hkv, Lq, Lk, D, 4, device_cus()).splits;
+  return choose_shares((int64_t)B * Hkv, Lq, Lk, D, 1, 4, device_cus()).splits;
 }
 
 extern "C" int varq_fused_attn(const void *q, void *out,

@@ -525,7 +525,7 @@ __global__ __launch_bounds__(256) void quant_tiled_kernel(GenParams p, Plan pl, 
 // The extremes over the lanes whose numbers differ in the bits from `from` up to below `to` (powers of two; all lanes are active), in every one of them.  From
 // rows of 16 lanes up by rotations inside the row and swaps of rows, a few cycles each where an exchange through LDS waits for some
 // hundred.  The small launches are one chain of such waits: with this fold, the wavefronts' extremes requested together and no divisions, us: ten steps with the
-// dequantized cache, [8,n,30,64] to fp32, 178 -> 173; with attention, [64,n,16,64] 375 -> 370, thirteen of [2,16,n,128] 1346 -> 1335.  In quant_shared_kernel,
+// dequantized cache, [8,n,30,64] to fp32, 178 -> 173; with attention, [64,n,16,64] 375 -> 370.  In quant_shared_kernel,
 // whose registers are full, the same fold costs (K of [32,30,680,64] 63.1 -> 64.1, unpacking included), so it keeps the exchange.
 template <bool ASYM, int NV> __device__ __forceinline__ void fold_lanes(float (&mx)[NV], float (&mn)[NV], int from, int to) {
   auto with = [&](auto &&other) __attribute__((always_inline)) {
