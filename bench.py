@@ -861,7 +861,7 @@ def main():
                           'timing': '40 back-to-back launches over the %d cycled input sets between one HIP event pair, median '
                                     'of 5 (inside the timed steps, one launch between its own events: '
                                     'pack_us_per_tensor_in_step)' % NBUF},
-        'roofline_dequant': {'kernel': 'dequant_kernel<int4 words, group 128, bf16 out>', 'bound': 'hbm',
+        'roofline_dequant': {'kernel': 'dequant_words_kernel<bf16 out, int4 words, group 128>', 'bound': 'hbm',
                              'achieved': round(deq_bytes / t_deq / 1e9, 2), 'peak': HBM_PEAK_GBPS, 'unit': 'GB/s',
                              'frac': round(deq_bytes / t_deq / 1e9 / HBM_PEAK_GBPS, 4),
                              'traffic': None if not traffic else traffic.get('dequant'),
